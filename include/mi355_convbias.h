@@ -224,6 +224,20 @@ int mi355_convbias_s8_exec_preprocessed(void* stream, const mi355_conv_desc* d, 
                                         const void* preprocessed, size_t preprocessed_bytes, const int32_t* bias,
                                         const int8_t* z, void* dst, void* workspace, size_t workspace_bytes);
 
+/* A bound call: one exec with its arguments -- descriptor, algorithm, tensors, workspace -- fixed, for a program that
+ * issues the same launches many times (an inference plan over a static activation arena).  _bind validates and chooses
+ * exactly as exec does and keeps the resulting kernel launches; _launch issues them on a stream, which costs the host no
+ * more than the launches themselves (exec walks validation, tile choice and argument set-up each time: about 0.6 us).
+ * preprocessed_bytes != 0: `filter` is the tensor of mi355_convbias_s8_preprocess, otherwise the reference layout.
+ * Belongs to the device that is current at _bind; the tensors must outlive the call object.  Launching one bound call
+ * from several threads is safe (it is not modified); destroy it when no thread uses it any more. */
+typedef struct mi355_bound_call mi355_bound_call;
+int mi355_convbias_s8_bind(const mi355_conv_desc* d, const mi355_algo* algo, const int8_t* src, const void* filter,
+                           size_t preprocessed_bytes, const int32_t* bias, const int8_t* z, void* dst, void* workspace,
+                           size_t workspace_bytes, mi355_bound_call** out);
+int mi355_bound_call_launch(void* stream, const mi355_bound_call* call);
+void mi355_bound_call_destroy(mi355_bound_call* call);
+
 /* Profiling primitive of a fast-run chooser (the role of rdnn::AlgoChooser's timed trial runs over
  * get_all_algorithms_info_safe, src/rdnn/impl/algo_chooser.cpp; dnn/include/megdnn/oprs/base.h:545-615): `warmup`
  * untimed and `iters` timed launches of ONE algorithm, bracketed by HIP events on `stream`; *avg_usec receives the

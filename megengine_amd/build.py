@@ -1,4 +1,4 @@
-"""Compiles the HIP extension (C-ABI shared library) for gfx950, in-tree.
+"""Compiles the HIP extension (C-ABI shared library) for gfx950 and the Python module over it, in-tree.
 
     python -m megengine_amd.build
 
@@ -14,10 +14,12 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmi355_convbias.so")
+NATIVE = os.path.join(HERE, "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
 SOURCES = ["capi.hip", "conv_direct.hip", "conv_igemm.hip", "conv_igemm_dma.hip", "conv_igemm2.hip", "conv_igemm3.hip", "conv_igemm4.hip", "conv_pw4.hip", "conv_c4.hip", "conv_dw.hip", "conv_nchw.hip", "relayout.hip", "requant.hip", "elemwise_q.hip", "pooling.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -50,7 +52,24 @@ def build(verbose=False, jobs=5):
     subprocess.check_call(cmd)
     with open(RESOURCES, "w") as f:
         json.dump(_resources, f, indent=0, sort_keys=True)
+    build_native(verbose)
     return LIB
+
+
+def build_native(verbose=False):
+    """The Python operators over the C ABI (csrc/native.cpp), linked against the library beside it and against torch."""
+    import torch
+    from torch.utils import cpp_extension
+    libs = cpp_extension.library_paths("cuda")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           *["-isystem" + p for p in cpp_extension.include_paths("cuda")], "-isystem" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "native.cpp"), "-o", NATIVE, "-L" + HERE, "-lmi355_convbias", *["-L" + p for p in libs],
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    return NATIVE
 
 
 _resources = {}

@@ -7,6 +7,7 @@
 #include <string.h>
 
 #include <mutex>
+#include <new>
 #include <shared_mutex>
 #include <unordered_map>
 #include <vector>
@@ -561,6 +562,8 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 }  // namespace
 
 namespace mi355 {
+thread_local LaunchList* t_binding = nullptr;
+
 bool epi_residual_table(const EpiParams& e, float* c, const float** tab) {
     if (!e.fast || !e.has_z || (e.nonline != MI355_NL_IDENTITY && e.nonline != MI355_NL_RELU)) return false;
     const TableEntry* t = epi_table_cached(e.s_b, e.s_z, e.s_d, e.nonline == MI355_NL_RELU);
@@ -849,6 +852,43 @@ int mi355_convbias_s8_exec_preprocessed(void* stream, const mi355_conv_desc* d, 
     return exec_impl(stream, d, algo, src, reinterpret_cast<const int8_t*>(preprocessed), true, bias, z, dst, workspace,
                      workspace_bytes);
 }
+
+// ---- bound calls ----
+struct mi355_bound_call {
+    LaunchList launches;
+};
+
+int mi355_convbias_s8_bind(const mi355_conv_desc* d, const mi355_algo* algo, const int8_t* src, const void* filter,
+                           size_t preprocessed_bytes, const int32_t* bias, const int8_t* z, void* dst, void* workspace,
+                           size_t workspace_bytes, mi355_bound_call** out) {
+    if (!out) return fail(MI355_ERR_BAD_ARG, "null argument");
+    *out = nullptr;
+    mi355_bound_call* b = new (std::nothrow) mi355_bound_call;
+    if (!b) return fail(MI355_ERR_BAD_ARG, "out of host memory");
+    t_binding = &b->launches;
+    const int st = preprocessed_bytes
+                           ? mi355_convbias_s8_exec_preprocessed(nullptr, d, algo, src, filter, preprocessed_bytes, bias, z, dst,
+                                                                 workspace, workspace_bytes)
+                           : mi355_convbias_s8_exec(nullptr, d, algo, src, static_cast<const int8_t*>(filter), bias, z, dst,
+                                                    workspace, workspace_bytes);
+    t_binding = nullptr;
+    if (st) {
+        delete b;
+        return st;
+    }
+    b->launches.seal();
+    *out = b;
+    return MI355_OK;
+}
+
+int mi355_bound_call_launch(void* stream, const mi355_bound_call* call) {
+    if (!call) return fail(MI355_ERR_BAD_ARG, "null bound call");
+    const hipError_t e = call->launches.replay(reinterpret_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(MI355_ERR_LAUNCH, "bound call: %s", hipGetErrorString(e));
+    return MI355_OK;
+}
+
+void mi355_bound_call_destroy(mi355_bound_call* call) { delete call; }
 
 int mi355_convbias_s8_profile(void* stream, const mi355_conv_desc* d, const mi355_algo* algo, const int8_t* src,
                               const int8_t* filter, const int32_t* bias, const int8_t* z, void* dst, void* workspace,

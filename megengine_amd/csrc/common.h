@@ -6,6 +6,7 @@
 
 #include "../../include/mi355_convbias.h"
 #include "epilogue.h"
+#include "launch.h"
 
 namespace mi355 {
 

@@ -373,8 +373,7 @@ int launch_conv_c4(hipStream_t st, const ConvProblem& p, int cu_count, const int
     }
     int64_t grid = (int64_t)occ[si].load(std::memory_order_relaxed) * cu_count;
     if (grid > a.tiles) grid = a.tiles;
-    hipLaunchKernelGGL(kerns[si], dim3((unsigned)grid), dim3(C4_THREADS), 0, st, a);
-    return (int)hipGetLastError();
+    return launch_kernel(kerns[si], dim3((unsigned)grid), dim3(C4_THREADS), 0, st, a);
 }
 
 }  // namespace mi355

@@ -178,8 +178,7 @@ int launch_conv_direct(hipStream_t st, const ConvProblem& p, const int8_t* src, 
     if (total == 0) return 0;
     const int64_t blocks = (total + 255) / 256;
     if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL(conv_direct_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a);
-    return (int)hipGetLastError();
+    return launch_kernel(conv_direct_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a);
 }
 
 }  // namespace mi355

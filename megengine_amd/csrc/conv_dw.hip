@@ -434,17 +434,16 @@ __global__ __launch_bounds__(256) void dw3x3_kernel(Dw3Args a) {
 }
 
 template <int S, int R>
-void launch_dw3(hipStream_t st, dim3 grid, const Dw3Args& b) {
+int launch_dw3(hipStream_t st, dim3 grid, const Dw3Args& b) {
     const bool buf = b.src_bytes != 0 && b.pw <= 1;
     const int epi = !b.epi.fast ? 2 : b.epi.lin ? 0 : (!b.epi.has_z && b.epi.nonline == NL_RELU) ? 1 : 2;
     const dim3 block(256);
     if (buf) {
-        if (epi == 0) hipLaunchKernelGGL((dw3x3_kernel<S, R, 0, true>), grid, block, 0, st, b);
-        else if (epi == 1) hipLaunchKernelGGL((dw3x3_kernel<S, R, 1, true>), grid, block, 0, st, b);
-        else hipLaunchKernelGGL((dw3x3_kernel<S, R, 2, true>), grid, block, 0, st, b);
-    } else {
-        hipLaunchKernelGGL((dw3x3_kernel<S, R, 2, false>), grid, block, 0, st, b);
+        if (epi == 0) return launch_kernel((dw3x3_kernel<S, R, 0, true>), grid, block, 0, st, b);
+        if (epi == 1) return launch_kernel((dw3x3_kernel<S, R, 1, true>), grid, block, 0, st, b);
+        return launch_kernel((dw3x3_kernel<S, R, 2, true>), grid, block, 0, st, b);
     }
+    return launch_kernel((dw3x3_kernel<S, R, 2, false>), grid, block, 0, st, b);
 }
 
 }  // namespace
@@ -487,22 +486,14 @@ int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, const int8_t* sr
             b.src_bytes = src_total < ((int64_t)1 << 31) ? (uint32_t)src_total : 0u;
             b.div_qw = make_fastdiv(b.QW); b.div_ohs = make_fastdiv(b.OHS); b.div_cg = make_fastdiv(b.CG);
             const dim3 grid((unsigned)((items + 255) / 256));
-            if (d.stride_h == 1 && R == 4)
-                launch_dw3<1, 4>(st, grid, b);
-            else if (d.stride_h == 1)
-                launch_dw3<1, 2>(st, grid, b);
-            else if (R == 2)
-                launch_dw3<2, 2>(st, grid, b);
-            else
-                launch_dw3<2, 1>(st, grid, b);
-            return (int)hipGetLastError();
+            if (d.stride_h == 1) return R == 4 ? launch_dw3<1, 4>(st, grid, b) : launch_dw3<1, 2>(st, grid, b);
+            return R == 2 ? launch_dw3<2, 2>(st, grid, b) : launch_dw3<2, 1>(st, grid, b);
         }
     }
     const int quads = a.OH * a.QW;
     const int threads = quads >= 192 ? 256 : (quads > 64 ? 128 : 64);
     dim3 grid((quads + threads - 1) / threads, d.n * a.CG), block(threads);
-    hipLaunchKernelGGL((dw4_kernel<0, 0>), grid, block, 0, st, a);
-    return (int)hipGetLastError();
+    return launch_kernel((dw4_kernel<0, 0>), grid, block, 0, st, a);
 }
 
 }  // namespace mi355

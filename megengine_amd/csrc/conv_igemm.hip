@@ -453,8 +453,7 @@ int launch_pw(hipStream_t st, IgemmArgs& a, int cu_count) {
     // a second tile and double the launch's duration; otherwise down, inside what the device holds at once.
     if (grid > tiles) grid = tiles;
     if (grid >= 8) grid = grid == tiles ? (grid + 7) & ~(int64_t)7 : grid & ~(int64_t)7;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(IG_THREADS), lds, st, a);
-    return (int)hipGetLastError();
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(IG_THREADS), lds, st, a);
 }
 
 template <int PIN, int POUT, int BM, int BN, int WM, int WN, int KCH, int MINW>

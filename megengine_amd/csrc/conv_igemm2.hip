@@ -775,8 +775,7 @@ int launch_k(hipStream_t st, IgemmArgs& a, int cu_count) {
     if (grid > tiles) grid = tiles;
     if (grid >= 8) grid = grid == tiles ? (grid + 7) & ~(int64_t)7 : grid & ~(int64_t)7;
     a.div_step = make_fastdiv((uint32_t)((grid & 7) == 0 ? grid >> 3 : grid));  // the kernel's tile stride
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(K::THREADS), lds, st, a);
-    return (int)hipGetLastError();
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(K::THREADS), lds, st, a);
 }
 
 template <int POUT, int BM, int BN, int WM, int WN, int KCH, int NS, int MINW, bool GEN, int KS = 1>
@@ -868,9 +867,8 @@ int launch_igemm2_preprocess(hipStream_t st, const int8_t* flt, int8_t* out, int
     const int ocp = (oc + 31) / 32 * 32, kc = (kbytes + 31) / 32;
     const int64_t units = (int64_t)kc * ocp * 2;
     if (units == 0) return 0;
-    hipLaunchKernelGGL(igemm2_preprocess_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, flt, out, oc, ocp,
+    return launch_kernel(igemm2_preprocess_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, flt, out, oc, ocp,
                        kbytes, units);
-    return (int)hipGetLastError();
 }
 
 // A tile that cannot run the problem (no instantiation with the general epilogue, or ring + residual slot beyond the

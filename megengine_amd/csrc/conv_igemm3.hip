@@ -460,8 +460,7 @@ int launch_k(hipStream_t st, IgemmArgs& a) {
         max_lds_set.store(kLdsPerCu, std::memory_order_relaxed);
     }
     const int64_t grid = (tiles + 7) / 8 * 8;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(K::THREADS), lds, st, a);
-    return (int)hipGetLastError();
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(K::THREADS), lds, st, a);
 }
 
 int launch_cfg(hipStream_t st, IgemmArgs& a, int cfg) {

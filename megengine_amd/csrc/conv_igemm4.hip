@@ -269,8 +269,7 @@ int launch_k(hipStream_t st, IgemmArgs& a, const R4Geom& g, int lds, int cu_coun
     // persistent grid: as many workgroups as are resident at once (two per CU)
     int64_t grid = (int64_t)occ.load(std::memory_order_relaxed) * cu_count;
     if (grid > a.tiles) grid = a.tiles;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(R4_THREADS), lds, st, a, g);
-    return (int)hipGetLastError();
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(R4_THREADS), lds, st, a, g);
 }
 
 }  // namespace

@@ -488,8 +488,7 @@ int launch_pw(hipStream_t st, IgemmArgs& a, int cu_count) {
     if (grid > tiles) grid = tiles;
     if (grid >= 8) grid = grid == tiles ? (grid + 7) & ~(int64_t)7 : grid & ~(int64_t)7;
     a.div_step = make_fastdiv((uint32_t)((grid & 7) == 0 ? grid >> 3 : grid));  // the kernel's tile stride
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(K::THREADS), lds, st, a);
-    return (int)hipGetLastError();
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(K::THREADS), lds, st, a);
 }
 
 template <int POUT, int BM, int BN, int WM, int WN, int KCH, int NS, int MINW>

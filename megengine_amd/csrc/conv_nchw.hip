@@ -131,16 +131,14 @@ int launch_conv_nchw_mfma(hipStream_t st, const ConvProblem& p, int cu_count, co
         // filter rows of the padded output channels (dense convolutions only: groups are whole blocks)
         const size_t row = (size_t)icpg32 * d.fh * d.fw;  // a multiple of 32 bytes
         const uint64_t vecs = (uint64_t)(L.oc32 - d.oc) * row / 16;
-        hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, st,
+        rc = launch_kernel(zero_fill_kernel, dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, st,
                            reinterpret_cast<v4i*>(flt32 + (size_t)d.oc * row), vecs);
-        rc = (int)hipGetLastError();
         if (rc) return rc;
     }
     const int32_t* bias32 = bias;
     if (d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL && L.oc32 != d.oc) {
         int32_t* b = reinterpret_cast<int32_t*>(ws + L.off_bias);
-        hipLaunchKernelGGL(bias_pad_kernel, dim3((L.oc32 + 255) / 256), dim3(256), 0, st, bias, b, d.oc, L.oc32);
-        rc = (int)hipGetLastError();
+        rc = launch_kernel(bias_pad_kernel, dim3((L.oc32 + 255) / 256), dim3(256), 0, st, bias, b, d.oc, L.oc32);
         if (rc) return rc;
         bias32 = b;
     }

@@ -206,11 +206,9 @@ int launch32_mt(hipStream_t st, const IgemmArgs& a, int cu_count) {
     if (a.epi.has_z) {
         ResidualTable tab;
         if (a.epi.zlin) memcpy(tab.v, a.ztab, sizeof(tab.v)); else memset(tab.v, 0, sizeof(tab.v));
-        hipLaunchKernelGGL((pw32s_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, tab);
-    } else {
-        hipLaunchKernelGGL((pw32s_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, NoResidualTable{});
+        return launch_kernel((pw32s_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, tab);
     }
-    return (int)hipGetLastError();
+    return launch_kernel((pw32s_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, NoResidualTable{});
 }
 
 template <int MT, int KC>
@@ -224,10 +222,8 @@ int launch_mt(hipStream_t st, const IgemmArgs& a, int cu_count) {
     if (blocks > cap) blocks = cap;
     blocks = (blocks + n_ocg - 1) / n_ocg * n_ocg;  // waves of one pixel block stay together; 4 * blocks % n_ocg == 0
     if (a.epi.has_z)
-        hipLaunchKernelGGL((pw4s_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb);
-    else
-        hipLaunchKernelGGL((pw4s_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb);
-    return (int)hipGetLastError();
+        return launch_kernel((pw4s_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb);
+    return launch_kernel((pw4s_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb);
 }
 
 }  // namespace

@@ -129,14 +129,10 @@ __global__ __launch_bounds__(256) void elemwise_q_kernel(EwArgs a) {
 
 template <int ARITY>
 int launch_arity(hipStream_t st, const EwArgs& a, bool src32, bool dst32, unsigned blocks) {
-    if (src32) {
-        if (dst32) hipLaunchKernelGGL((elemwise_q_kernel<ARITY, true, true>), dim3(blocks), dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((elemwise_q_kernel<ARITY, true, false>), dim3(blocks), dim3(256), 0, st, a);
-    } else {
-        if (dst32) hipLaunchKernelGGL((elemwise_q_kernel<ARITY, false, true>), dim3(blocks), dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((elemwise_q_kernel<ARITY, false, false>), dim3(blocks), dim3(256), 0, st, a);
-    }
-    return (int)hipGetLastError();
+    if (src32 && dst32) return launch_kernel(elemwise_q_kernel<ARITY, true, true>, dim3(blocks), dim3(256), 0, st, a);
+    if (src32) return launch_kernel(elemwise_q_kernel<ARITY, true, false>, dim3(blocks), dim3(256), 0, st, a);
+    if (dst32) return launch_kernel(elemwise_q_kernel<ARITY, false, true>, dim3(blocks), dim3(256), 0, st, a);
+    return launch_kernel(elemwise_q_kernel<ARITY, false, false>, dim3(blocks), dim3(256), 0, st, a);
 }
 
 }  // namespace

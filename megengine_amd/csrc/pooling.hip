@@ -249,22 +249,19 @@ __global__ __launch_bounds__(256) void pooling_kernel(PoolArgs a) {
 }
 
 template <int PACK, int VB, int FH, int FW>
-void launch_static(hipStream_t st, const PoolArgs& a, int mode, unsigned blocks) {
+int launch_static(hipStream_t st, const PoolArgs& a, int mode, unsigned blocks) {
     switch (mode) {
         case POOL_MAX:
-            hipLaunchKernelGGL((pooling_static_kernel<PACK, VB, POOL_MAX, FH, FW>), dim3(blocks), dim3(256), 0, st, a);
-            break;
+            return launch_kernel((pooling_static_kernel<PACK, VB, POOL_MAX, FH, FW>), dim3(blocks), dim3(256), 0, st, a);
         case POOL_AVG:
-            hipLaunchKernelGGL((pooling_static_kernel<PACK, VB, POOL_AVG, FH, FW>), dim3(blocks), dim3(256), 0, st, a);
-            break;
+            return launch_kernel((pooling_static_kernel<PACK, VB, POOL_AVG, FH, FW>), dim3(blocks), dim3(256), 0, st, a);
         default:
-            hipLaunchKernelGGL((pooling_static_kernel<PACK, VB, POOL_AVG_EXCL, FH, FW>), dim3(blocks), dim3(256), 0, st, a);
-            break;
+            return launch_kernel((pooling_static_kernel<PACK, VB, POOL_AVG_EXCL, FH, FW>), dim3(blocks), dim3(256), 0, st, a);
     }
 }
 
 template <int PACK, int VB>
-void launch_mode(hipStream_t st, const PoolArgs& a, int mode, unsigned blocks) {
+int launch_mode(hipStream_t st, const PoolArgs& a, int mode, unsigned blocks) {
     if constexpr (VB >= 4) {
         // the static kernels address a plane with 32-bit offsets
         if ((uint64_t)a.IH * (uint64_t)a.IW * PACK >= (1ull << 31)) goto generic;
@@ -274,14 +271,11 @@ void launch_mode(hipStream_t st, const PoolArgs& a, int mode, unsigned blocks) {
 generic:
     switch (mode) {
         case POOL_MAX:
-            hipLaunchKernelGGL((pooling_kernel<PACK, VB, POOL_MAX>), dim3(blocks), dim3(256), 0, st, a);
-            break;
+            return launch_kernel((pooling_kernel<PACK, VB, POOL_MAX>), dim3(blocks), dim3(256), 0, st, a);
         case POOL_AVG:
-            hipLaunchKernelGGL((pooling_kernel<PACK, VB, POOL_AVG>), dim3(blocks), dim3(256), 0, st, a);
-            break;
+            return launch_kernel((pooling_kernel<PACK, VB, POOL_AVG>), dim3(blocks), dim3(256), 0, st, a);
         default:
-            hipLaunchKernelGGL((pooling_kernel<PACK, VB, POOL_AVG_EXCL>), dim3(blocks), dim3(256), 0, st, a);
-            break;
+            return launch_kernel((pooling_kernel<PACK, VB, POOL_AVG_EXCL>), dim3(blocks), dim3(256), 0, st, a);
     }
 }
 
@@ -307,13 +301,9 @@ int launch_pooling(hipStream_t st, const mi355_pooling_desc& d, int pack, uint32
     uint64_t blocks = (units + 255) / 256;
     const uint64_t cap = (uint64_t)cu_count * 64;
     if (blocks > cap) blocks = cap;
-    if (pack == 32)
-        launch_mode<32, 16>(st, a, (int)d.mode, (unsigned)blocks);
-    else if (pack == 4)
-        launch_mode<4, 4>(st, a, (int)d.mode, (unsigned)blocks);
-    else
-        launch_mode<1, 1>(st, a, (int)d.mode, (unsigned)blocks);
-    return (int)hipGetLastError();
+    if (pack == 32) return launch_mode<32, 16>(st, a, (int)d.mode, (unsigned)blocks);
+    if (pack == 4) return launch_mode<4, 4>(st, a, (int)d.mode, (unsigned)blocks);
+    return launch_mode<1, 1>(st, a, (int)d.mode, (unsigned)blocks);
 }
 
 }  // namespace mi355

@@ -279,14 +279,13 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
             if (C % p == 0 && HW % 16 == 0 && (uint64_t)C * HW < (1ull << 31)) {
                 if (p == 4) {
                     uint32_t items = (C / 4) * (HW / 16);
-                    hipLaunchKernelGGL(nchw_to_nchw4_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st,
+                    return launch_kernel(nchw_to_nchw4_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st,
                                        (const int8_t*)src, (int8_t*)dst, C, HW);
                 } else {
                     uint32_t ptiles = (HW + RL_TP - 1) / RL_TP;
-                    hipLaunchKernelGGL(nchw_to_nchw32_kernel, dim3((C / 32) * ptiles, N), dim3(256), 0, st,
+                    return launch_kernel(nchw_to_nchw32_kernel, dim3((C / 32) * ptiles, N), dim3(256), 0, st,
                                        (const int8_t*)src, (int8_t*)dst, C / 32, HW);
                 }
-                return (int)hipGetLastError();
             }
         } else if ((d.mode == MI355_RL_NCHW4_NCHW || d.mode == MI355_RL_NCHW32_NCHW) &&
                    (d.oc == 0 || d.oc == d.shape[1] * d.shape[4])) {
@@ -294,14 +293,13 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
             if (HW % 16 == 0 && (uint64_t)C * HW < (1ull << 31)) {
                 if (p == 4) {
                     uint32_t items = (C / 4) * (HW / 16);
-                    hipLaunchKernelGGL(nchw4_to_nchw_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st,
+                    return launch_kernel(nchw4_to_nchw_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st,
                                        (const int8_t*)src, (int8_t*)dst, C, HW);
                 } else {
                     uint32_t ptiles = (HW + RL_TP - 1) / RL_TP;
-                    hipLaunchKernelGGL(nchw32_to_nchw_kernel, dim3((C / 32) * ptiles, N), dim3(256), 0, st,
+                    return launch_kernel(nchw32_to_nchw_kernel, dim3((C / 32) * ptiles, N), dim3(256), 0, st,
                                        (const int8_t*)src, (int8_t*)dst, C / 32, HW);
                 }
-                return (int)hipGetLastError();
             }
         }
     }
@@ -318,8 +316,7 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
     a.total = total;
     int64_t blocks = (total + 255) / 256;
     if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL(relayout_generic_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a);
-    return (int)hipGetLastError();
+    return launch_kernel(relayout_generic_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a);
 }
 
 }  // namespace mi355

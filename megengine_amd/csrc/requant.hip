@@ -99,16 +99,14 @@ unsigned stream_blocks(uint64_t steps, int cu_count) {
 
 int launch_cvt_f32_s8(hipStream_t st, float scale, const float* src, int8_t* dst, uint64_t count, int cu_count) {
     if (count == 0) return 0;
-    hipLaunchKernelGGL(cvt_f32_s8_kernel, dim3(stream_blocks(count / 4, cu_count)), dim3(256), 0, st, src, dst, count / 4,
+    return launch_kernel(cvt_f32_s8_kernel, dim3(stream_blocks(count / 4, cu_count)), dim3(256), 0, st, src, dst, count / 4,
                        count, scale);
-    return (int)hipGetLastError();
 }
 
 int launch_cvt_s8_f32(hipStream_t st, float scale, const int8_t* src, float* dst, uint64_t count, int cu_count) {
     if (count == 0) return 0;
-    hipLaunchKernelGGL(cvt_s8_f32_kernel, dim3(stream_blocks(count / 4, cu_count)), dim3(256), 0, st, src, dst, count / 4,
+    return launch_kernel(cvt_s8_f32_kernel, dim3(stream_blocks(count / 4, cu_count)), dim3(256), 0, st, src, dst, count / 4,
                        count, scale);
-    return (int)hipGetLastError();
 }
 
 int launch_requant8(hipStream_t st, const EpiParams& e, const int8_t* src, const int8_t* z, int8_t* dst, uint64_t count,
@@ -120,8 +118,7 @@ int launch_requant8(hipStream_t st, const EpiParams& e, const int8_t* src, const
     const uint64_t cap = (uint64_t)cu_count * 16;
     if (blocks > cap) blocks = cap;
     if (blocks == 0) blocks = 1;
-    hipLaunchKernelGGL(requant8_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, blocks16, count, e);
-    return (int)hipGetLastError();
+    return launch_kernel(requant8_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, blocks16, count, e);
 }
 
 int launch_requant(hipStream_t st, const EpiParams& e, const int32_t* src, const int8_t* z, int8_t* dst, uint64_t count,
@@ -133,8 +130,7 @@ int launch_requant(hipStream_t st, const EpiParams& e, const int32_t* src, const
     const uint64_t cap = (uint64_t)cu_count * 16;
     if (blocks > cap) blocks = cap;
     if (blocks == 0) blocks = 1;
-    hipLaunchKernelGGL(requant_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, quads, count, e);
-    return (int)hipGetLastError();
+    return launch_kernel(requant_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, quads, count, e);
 }
 
 // ---- streaming probe: what a launch that only moves bytes costs on this device ----------------------------------
@@ -161,9 +157,8 @@ int launch_stream_probe(hipStream_t st, const void* src, uint64_t read_bytes, vo
     const uint64_t units = nr > nw ? nr : nw;
     uint64_t blocks = (units + 255) / 256;
     if (blocks > (uint64_t)cu_count * 8) blocks = (uint64_t)cu_count * 8;
-    hipLaunchKernelGGL(stream_probe_kernel, dim3((unsigned)blocks), dim3(256), 0, st, reinterpret_cast<const u32x4p*>(src),
+    return launch_kernel(stream_probe_kernel, dim3((unsigned)blocks), dim3(256), 0, st, reinterpret_cast<const u32x4p*>(src),
                        reinterpret_cast<u32x4p*>(dst), nr, nw);
-    return (int)hipGetLastError();
 }
 
 }  // namespace mi355

@@ -19,7 +19,7 @@ EXPORTS = [
     "mi355_convbias_algo_usable", "mi355_convbias_s8_query", "mi355_convbias_s8_exec",
     "mi355_igemm_tile_count", "mi355_igemm_tile_name", "mi355_igemm_tile_usable", "mi355_epilogue_linear_form", "mi355_epilogue_residual_table",
     "mi355_relayout_deduce", "mi355_relayout_exec", "mi355_requant_s32_s8_exec", "mi355_requant_s8_s8_exec", "mi355_elemwise_q_exec",
-    "mi355_convbias_s8_profile",
+    "mi355_convbias_s8_profile", "mi355_convbias_s8_bind", "mi355_bound_call_launch", "mi355_bound_call_destroy",
     "mi355_pooling_deduce_out", "mi355_pooling_s8_exec", "mi355_typecvt_f32_s8_exec", "mi355_typecvt_s8_f32_exec",
     "mi355_static_workspace_bytes", "mi355_convbias_s8_exec_static_workspace",
     "mi355_epilogue_quotient_form", "mi355_convbias_s8_preprocess_size", "mi355_convbias_s8_preprocess", "mi355_convbias_s8_exec_preprocessed",
