@@ -5,8 +5,8 @@
 //
 // Two tiers:
 //   * relayout_generic_kernel: one thread per destination element, any mode / element size.
-//   * byte-transposing fast kernels for the int8 pure-permutation cases the conv path uses;
-//     all global traffic is 16-byte vectors, fully coalesced on both sides (HBM bound).
+//   * byte-transposing kernels for the int8 pure permutations, any channel count and image size;
+//     16-byte vectors, coalesced on both sides (HBM bound).
 #include "common.h"
 
 namespace mi355 {
@@ -126,78 +126,146 @@ __device__ __forceinline__ void transpose4x4(uint32_t r0, uint32_t r1, uint32_t 
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// NCHW -> NCHW4, int8, C % 4 == 0, HW % 16 == 0.  Thread: 4 channels x 16 pixels.
-// grid.x covers (C/4) * (HW/16) work items per image, grid.y = N.
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(1)));  // 16 bytes at any address
+typedef uint32_t u32u __attribute__((aligned(1)));
+
+__device__ __forceinline__ u32x4 load16u(const int8_t* p) { return *reinterpret_cast<const u32x4u*>(p); }
+__device__ __forceinline__ void store16u(int8_t* p, u32x4 v) { *reinterpret_cast<u32x4u*>(p) = v; }
+
+// `have` (>= 1) bytes from p, the rest zero
+__device__ __forceinline__ u32x4 load16_tail(const int8_t* p, uint32_t have) {
+    if (have >= 16) return load16u(p);
+    u32x4 x = {0, 0, 0, 0};
+#pragma unroll
+    for (uint32_t k = 0; k < 16; ++k)
+        if (k < have) x[k / 4] |= (uint32_t)(uint8_t)p[k] << (8 * (k % 4));
+    return x;
+}
+__device__ __forceinline__ void store16_tail(int8_t* p, u32x4 v, uint32_t have) {
+    if (have >= 16) return store16u(p, v);
+#pragma unroll
+    for (uint32_t k = 0; k < 16; ++k)
+        if (k < have) p[k] = (int8_t)(v[k / 4] >> (8 * (k % 4)));
+}
+
+// Planes of a plain tensor start at any byte when the image has an odd size: their 16-byte accesses are unaligned ones
+// (the memory pipe takes them at full rate as long as a wave's run is contiguous).  The last 16 pixels of a plane start
+// at HW - 16, so they overlap the run before them and both write the same bytes: no tail code, every lane does the same.
+//
+// NCHW -> NCHW4 (C any: missing channels are zero), HW >= 16.  Thread: 4 channels x 16 pixels.
+// grid.x covers CB * ceil(HW / 16) work items per image, grid.y = N.  3 x 224 x 224, batch 64 (the image of a first
+// layer): 53 us one byte per thread, 8.4 here.
 __global__ __launch_bounds__(256) void nchw_to_nchw4_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
-                                                            uint32_t C, uint32_t HW) {
-    const uint32_t pq = HW / 16;
-    const uint32_t items = (C / 4) * pq;
-    uint32_t it = blockIdx.x * 256 + threadIdx.x;
+                                                            uint32_t C, uint32_t HW, uint32_t items, FastDiv pq) {
+    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
     if (it >= items) return;
-    const uint32_t cg = it / pq, pb = it % pq;
-    const int64_t img = (int64_t)blockIdx.y * C * HW;
-    const int8_t* s = src + img + (int64_t)cg * 4 * HW + pb * 16;
-    u32x4 r0 = *reinterpret_cast<const u32x4*>(s);
-    u32x4 r1 = *reinterpret_cast<const u32x4*>(s + HW);
-    u32x4 r2 = *reinterpret_cast<const u32x4*>(s + 2 * (int64_t)HW);
-    u32x4 r3 = *reinterpret_cast<const u32x4*>(s + 3 * (int64_t)HW);
-    int8_t* d = dst + img + ((int64_t)cg * HW + pb * 16) * 4;
+    const uint32_t cg = fdiv(it, pq), pb = it - cg * pq.d;
+    const uint32_t px = pb * 16 + 16 <= HW ? pb * 16 : HW - 16;
+    const uint32_t CB = (C + 3) / 4;
+    const int8_t* s = src + ((int64_t)blockIdx.y * C + cg * 4) * HW + px;
+    const uint32_t have = C - cg * 4;
+    u32x4 r[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        r[k] = u32x4{0, 0, 0, 0};
+        if (k < have) r[k] = load16u(s + (int64_t)k * HW);
+    }
+    int8_t* d = dst + (((int64_t)blockIdx.y * CB + cg) * HW + px) * 4;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        u32x4 o;
         uint32_t c0, c1, c2, c3;
-        transpose4x4(r0[j], r1[j], r2[j], r3[j], c0, c1, c2, c3);
-        o[0] = c0; o[1] = c1; o[2] = c2; o[3] = c3;
-        *reinterpret_cast<u32x4*>(d + j * 16) = o;
+        transpose4x4(r[0][j], r[1][j], r[2][j], r[3][j], c0, c1, c2, c3);
+        store16u(d + j * 16, u32x4{c0, c1, c2, c3});
     }
 }
 
-// NCHW4 -> NCHW, int8, same constraints.
+// NCHW4 -> NCHW (the first C channels), HW >= 16.
 __global__ __launch_bounds__(256) void nchw4_to_nchw_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
-                                                            uint32_t C, uint32_t HW) {
-    const uint32_t pq = HW / 16;
-    const uint32_t items = (C / 4) * pq;
-    uint32_t it = blockIdx.x * 256 + threadIdx.x;
+                                                            uint32_t C, uint32_t HW, uint32_t items, FastDiv pq) {
+    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
     if (it >= items) return;
-    const uint32_t cg = it / pq, pb = it % pq;
-    const int64_t img = (int64_t)blockIdx.y * C * HW;
-    const int8_t* s = src + img + ((int64_t)cg * HW + pb * 16) * 4;
-    u32x4 o0, o1, o2, o3;
+    const uint32_t cg = fdiv(it, pq), pb = it - cg * pq.d;
+    const uint32_t px = pb * 16 + 16 <= HW ? pb * 16 : HW - 16;
+    const uint32_t CB = (C + 3) / 4;
+    const int8_t* s = src + (((int64_t)blockIdx.y * CB + cg) * HW + px) * 4;
+    u32x4 o[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        u32x4 v = *reinterpret_cast<const u32x4*>(s + j * 16);  // 4 pixels x 4 channels
+        const u32x4 v = load16u(s + j * 16);  // 4 pixels x 4 channels
         uint32_t c0, c1, c2, c3;
         transpose4x4(v[0], v[1], v[2], v[3], c0, c1, c2, c3);
-        o0[j] = c0; o1[j] = c1; o2[j] = c2; o3[j] = c3;
+        o[0][j] = c0; o[1][j] = c1; o[2][j] = c2; o[3][j] = c3;
     }
-    int8_t* d = dst + img + (int64_t)cg * 4 * HW + pb * 16;
-    *reinterpret_cast<u32x4*>(d) = o0;
-    *reinterpret_cast<u32x4*>(d + HW) = o1;
-    *reinterpret_cast<u32x4*>(d + 2 * (int64_t)HW) = o2;
-    *reinterpret_cast<u32x4*>(d + 3 * (int64_t)HW) = o3;
+    int8_t* d = dst + ((int64_t)blockIdx.y * C + cg * 4) * HW + px;
+    const uint32_t have = C - cg * 4;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        if (k < have) store16u(d + (int64_t)k * HW, o[k]);
+}
+
+// NCHW4 <-> NCHW32: dwords change places.  Two threads per pixel of a 32-channel block, each moves 16 channels: on the
+// NCHW32 side a wave covers one contiguous kilobyte, on the other side two runs of 128 bytes per access.
+// 16 blocks of 4 at 56 x 56, batch 64: 53 us one byte per thread, 5.8 here.
+template <bool TO32>
+__global__ __launch_bounds__(256) void nchw4_nchw32_kernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst,
+                                                           uint32_t HW, uint32_t items, FastDiv hw) {
+    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
+    if (it >= items) return;
+    const uint32_t half = it & 1, t = it >> 1;
+    const uint32_t blk = fdiv(t, hw), px = t - blk * HW;      // blk = image * channel blocks of 32 + block
+    const int64_t at4 = ((int64_t)blk * 8 + half * 4) * HW + px;
+    const int64_t at32 = (int64_t)it * 4;
+    if (TO32) {
+        u32x4 v;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = src[at4 + (int64_t)k * HW];
+        *reinterpret_cast<u32x4*>(dst + at32) = v;
+    } else {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(src + at32);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) dst[at4 + (int64_t)k * HW] = v[k];
+    }
+}
+
+// NCHW -> NCHW4 / NCHW32 for small planes (filters, 7 x 7 images): one thread per 4 output channels of a pixel.
+__global__ __launch_bounds__(256) void nchw_to_packed_small_kernel(const int8_t* __restrict__ src, uint32_t* __restrict__ dst,
+                                                                   uint32_t C, uint32_t CB, uint32_t HW,
+                                                                   uint32_t log_quads, uint32_t items, FastDiv hw, FastDiv cb) {
+    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
+    if (it >= items) return;
+    const uint32_t k = it & ((1u << log_quads) - 1), t = it >> log_quads;  // 1 or 8 quads per pixel
+    const uint32_t b = fdiv(t, hw), px = t - b * HW;
+    const uint32_t n = fdiv(b, cb), c0 = ((b - n * CB) << (log_quads + 2)) + k * 4;
+    const int8_t* s = src + ((int64_t)n * C + c0) * HW + px;
+    uint32_t w = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q)
+        if (c0 + q < C) w |= (uint32_t)(uint8_t)s[(int64_t)q * HW] << (8 * q);
+    dst[it] = w;
 }
 
 // NCHW <-> NCHW32 through LDS.  Tile = 32 channels x 512 pixels (16 KiB).  The LDS image keeps
 // the NCHW order (channel rows of 512 bytes, padded to 520 so that rows c and c+16 are 32 banks
-// apart); global accesses on both sides are 16-byte vectors over contiguous runs.
+// apart); global accesses on both sides are 16-byte vectors over contiguous runs, unaligned ones on the plain side when
+// the image has an odd size.  C any: missing channels are zero on the way in and dropped on the way out.
 constexpr int RL_TP = 512;           // pixels per tile
 constexpr int RL_ROW = RL_TP + 8;    // padded channel row (bytes): 16 rows = 8320 = 32*256 + 128
 
 __global__ __launch_bounds__(256) void nchw_to_nchw32_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
-                                                             uint32_t CB, uint32_t HW) {
+                                                             uint32_t C, uint32_t CB, uint32_t HW) {
     __shared__ __attribute__((aligned(16))) int8_t sm[32 * RL_ROW];
     const uint32_t t = threadIdx.x;
     const uint32_t ptiles = (HW + RL_TP - 1) / RL_TP;
     const uint32_t cb = blockIdx.x / ptiles, pt = blockIdx.x % ptiles;
     const uint32_t p0 = pt * RL_TP;
-    const int64_t img = (int64_t)blockIdx.y * CB * 32 * HW;
+    const int64_t n = blockIdx.y;
     // load: 32 rows x 32 vectors; thread t -> vector (t % 32), rows t/32 + 8*i
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t row = t / 32 + 8 * i, v = t % 32;
         uint32_t px = p0 + v * 16;
         u32x4 x = {0, 0, 0, 0};
-        if (px < HW) x = *reinterpret_cast<const u32x4*>(src + img + ((int64_t)cb * 32 + row) * HW + px);
+        if (px < HW && cb * 32 + row < C) x = load16_tail(src + (n * C + cb * 32 + row) * HW + px, HW - px);
         *reinterpret_cast<u32x4*>(sm + row * RL_ROW + v * 16) = x;
     }
     __syncthreads();
@@ -215,28 +283,27 @@ __global__ __launch_bounds__(256) void nchw_to_nchw32_kernel(const int8_t* __res
         out[0][q] = c0; out[1][q] = c1; out[2][q] = c2; out[3][q] = c3;
     }
     const uint32_t px = p0 + pq * 4;
-    if (px < HW) {
-        int8_t* d = dst + img + ((int64_t)cb * HW + px) * 32 + half * 16;
+    int8_t* d = dst + ((n * CB + cb) * HW + px) * 32 + half * 16;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(d + i * 32) = out[i];
-    }
+    for (int i = 0; i < 4; ++i)
+        if (px + i < HW) *reinterpret_cast<u32x4*>(d + i * 32) = out[i];
 }
 
 __global__ __launch_bounds__(256) void nchw32_to_nchw_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
-                                                             uint32_t CB, uint32_t HW) {
+                                                             uint32_t C, uint32_t CB, uint32_t HW) {
     __shared__ __attribute__((aligned(16))) int8_t sm[32 * RL_ROW];
     const uint32_t t = threadIdx.x;
     const uint32_t ptiles = (HW + RL_TP - 1) / RL_TP;
     const uint32_t cb = blockIdx.x / ptiles, pt = blockIdx.x % ptiles;
     const uint32_t p0 = pt * RL_TP;
-    const int64_t img = (int64_t)blockIdx.y * CB * 32 * HW;
+    const int64_t n = blockIdx.y;
     const uint32_t pq = t >> 1, half = t & 1;
     const uint32_t px = p0 + pq * 4;
     u32x4 in[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         in[i] = u32x4{0, 0, 0, 0};
-        if (px < HW) in[i] = *reinterpret_cast<const u32x4*>(src + img + ((int64_t)cb * HW + px + i) * 32 + half * 16);
+        if (px + i < HW) in[i] = *reinterpret_cast<const u32x4*>(src + ((n * CB + cb) * HW + px + i) * 32 + half * 16);
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -254,9 +321,9 @@ __global__ __launch_bounds__(256) void nchw32_to_nchw_kernel(const int8_t* __res
     for (int i = 0; i < 4; ++i) {
         uint32_t row = t / 32 + 8 * i, v = t % 32;
         uint32_t p = p0 + v * 16;
-        if (p < HW) {
+        if (p < HW && cb * 32 + row < C) {
             u32x4 x = *reinterpret_cast<const u32x4*>(sm + row * RL_ROW + v * 16);
-            *reinterpret_cast<u32x4*>(dst + img + ((int64_t)cb * 32 + row) * HW + p) = x;
+            store16_tail(dst + (n * C + cb * 32 + row) * HW + p, x, HW - p);
         }
     }
 }
@@ -270,37 +337,55 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
     if (total == 0) return 0;
     const bool requant = d.elem_bytes == 1 && d.scale_src != d.scale_dst;
     const uint32_t g = d.group ? d.group : 1;
-    // fast byte-permutation paths
-    if (allow_fast && d.elem_bytes == 1 && !requant && g == 1 && d.shape[0] <= 65535) {
-        const uint32_t N = d.shape[0];
-        if (d.mode == MI355_RL_NCHW_NCHW4 || d.mode == MI355_RL_NCHW_NCHW32) {
-            const uint32_t C = d.shape[1], HW = d.shape[2] * d.shape[3];
-            const uint32_t p = d.mode == MI355_RL_NCHW_NCHW4 ? 4 : 32;
-            if (C % p == 0 && HW % 16 == 0 && (uint64_t)C * HW < (1ull << 31)) {
-                if (p == 4) {
-                    uint32_t items = (C / 4) * (HW / 16);
-                    return launch_kernel(nchw_to_nchw4_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st,
-                                       (const int8_t*)src, (int8_t*)dst, C, HW);
-                } else {
-                    uint32_t ptiles = (HW + RL_TP - 1) / RL_TP;
-                    return launch_kernel(nchw_to_nchw32_kernel, dim3((C / 32) * ptiles, N), dim3(256), 0, st,
-                                       (const int8_t*)src, (int8_t*)dst, C / 32, HW);
+    // byte permutations without channel groups: kernels that move vectors.  What is left to the generic kernel -- rescaling
+    // conversions, group padding, 32-bit elements, weights with padded output channels -- runs once per model or not at all.
+    const uint64_t HW64 = d.ndim >= 4 ? (uint64_t)d.shape[2] * d.shape[3] : 0;
+    if (allow_fast && d.elem_bytes == 1 && !requant && g == 1 && d.shape[0] <= 65535 && HW64 < (1ull << 31) &&
+        total < ((int64_t)1 << 31)) {
+        const uint32_t N = d.shape[0], HW = (uint32_t)HW64;
+        const int8_t* s8 = (const int8_t*)src;
+        int8_t* d8 = (int8_t*)dst;
+        const uint32_t ptiles = (HW + RL_TP - 1) / RL_TP;
+        switch (d.mode) {
+            case MI355_RL_NCHW_NCHW4:
+            case MI355_RL_NCHW_NCHW4_IC_SMALL:
+            case MI355_RL_NCHW_NCHW32: {
+                const uint32_t C = d.shape[1], CB = oshape[1];
+                if (oshape[4] == 4 && HW >= 16) {
+                    const uint32_t pq = (HW + 15) / 16, items = CB * pq;
+                    return launch_kernel(nchw_to_nchw4_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, items,
+                                         make_fastdiv(pq));
                 }
+                // planes of a quarter of the LDS tile and more: below, most of a tile's threads would find no pixel
+                if (oshape[4] == 32 && HW >= RL_TP / 4)
+                    return launch_kernel(nchw_to_nchw32_kernel, dim3(CB * ptiles, N), dim3(256), 0, st, s8, d8, C, CB, HW);
+                const uint32_t log_quads = oshape[4] == 32 ? 3 : 0, items = (uint32_t)(total / 4);
+                return launch_kernel(nchw_to_packed_small_kernel, dim3((items + 255) / 256), dim3(256), 0, st, s8,
+                                     reinterpret_cast<uint32_t*>(dst), C, CB, HW, log_quads, items, make_fastdiv(HW), make_fastdiv(CB));
             }
-        } else if ((d.mode == MI355_RL_NCHW4_NCHW || d.mode == MI355_RL_NCHW32_NCHW) &&
-                   (d.oc == 0 || d.oc == d.shape[1] * d.shape[4])) {
-            const uint32_t p = d.shape[4], C = d.shape[1] * p, HW = d.shape[2] * d.shape[3];
-            if (HW % 16 == 0 && (uint64_t)C * HW < (1ull << 31)) {
-                if (p == 4) {
-                    uint32_t items = (C / 4) * (HW / 16);
-                    return launch_kernel(nchw4_to_nchw_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st,
-                                       (const int8_t*)src, (int8_t*)dst, C, HW);
-                } else {
-                    uint32_t ptiles = (HW + RL_TP - 1) / RL_TP;
-                    return launch_kernel(nchw32_to_nchw_kernel, dim3((C / 32) * ptiles, N), dim3(256), 0, st,
-                                       (const int8_t*)src, (int8_t*)dst, C / 32, HW);
+            case MI355_RL_NCHW4_NCHW:
+                if (HW >= 16) {
+                    const uint32_t C = oshape[1], pq = (HW + 15) / 16, items = d.shape[1] * pq;
+                    return launch_kernel(nchw4_to_nchw_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, items,
+                                         make_fastdiv(pq));
                 }
+                break;
+            case MI355_RL_NCHW32_NCHW:
+                return launch_kernel(nchw32_to_nchw_kernel, dim3(d.shape[1] * ptiles, N), dim3(256), 0, st, s8, d8, oshape[1],
+                                     d.shape[1], HW);
+            case MI355_RL_NCHW4_NCHW32:
+            case MI355_RL_NCHW32_NCHW4: {
+                const uint32_t items = (uint32_t)(total / 16);
+                const uint32_t* sw = (const uint32_t*)src;
+                uint32_t* dw = (uint32_t*)dst;
+                if (d.mode == MI355_RL_NCHW4_NCHW32)
+                    return launch_kernel(nchw4_nchw32_kernel<true>, dim3((items + 255) / 256), dim3(256), 0, st, sw, dw, HW, items,
+                                         make_fastdiv(HW));
+                return launch_kernel(nchw4_nchw32_kernel<false>, dim3((items + 255) / 256), dim3(256), 0, st, sw, dw, HW, items,
+                                     make_fastdiv(HW));
             }
+            default:
+                break;
         }
     }
     RelayoutArgs a;
