@@ -482,8 +482,8 @@ int launch_fmt(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
 }  // namespace
 
 // tile_cfg numbering: register-staged tiles, LDS-direct tiles, second-generation tiles, patch-staged tiles, weight-resident
-// tiles, the 32-packed streaming kernel
-int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1; }
+// tiles, the 32-packed streaming kernel, the tiles that split the reduction over the waves of a workgroup
+int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1 + igemm5_num_cfgs(); }
 int igemm_first_v2_cfg() { return kNumCfgs + igemm_dma_num_cfgs(); }
 // planar destination (NCHW4_NCHW): two of the register-staged tiles
 static int launch_planar(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
@@ -497,13 +497,15 @@ static int launch_planar(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
 static int igemm_first_v3_cfg() { return igemm_first_v2_cfg() + igemm2_num_cfgs(); }
 static int igemm_first_v4_cfg() { return igemm_first_v3_cfg() + igemm3_num_cfgs(); }
 static int igemm_pw32s_cfg() { return igemm_first_v4_cfg() + igemm4_num_cfgs(); }
+static int igemm_first_ks_cfg() { return igemm_pw32s_cfg() + 1; }
 const char* igemm_cfg_name(int cfg) {
     if (cfg >= 0 && cfg < kNumCfgs) return kCfgs[cfg].name;
     if (cfg < igemm_first_v2_cfg()) return igemm_dma_cfg_name(cfg - kNumCfgs);
     if (cfg < igemm_first_v3_cfg()) return igemm2_cfg_name(cfg - igemm_first_v2_cfg());
     if (cfg < igemm_first_v4_cfg()) return igemm3_cfg_name(cfg - igemm_first_v3_cfg());
     if (cfg < igemm_pw32s_cfg()) return igemm4_cfg_name(cfg - igemm_first_v4_cfg());
-    return "pw32_stream";
+    if (cfg == igemm_pw32s_cfg()) return "pw32_stream";
+    return igemm5_cfg_name(cfg - igemm_first_ks_cfg());
 }
 
 static bool igemm_needs_general(const ConvProblem& p) {
@@ -570,12 +572,31 @@ bool igemm_usable(const ConvProblem& p) {
     return true;
 }
 
+static void igemm_fill_args(const ConvProblem& p, IgemmArgs& a);
+
+// a pointwise layer with a residual over at most 128 channels whose scales have the residual table form
+static bool igemm_takes_table(const ConvProblem& p) {
+    const mi355_conv_desc& d = p.d;
+    float c;
+    const float* tab;
+    return d.has_z && p.pin == 32 && p.pout == 32 && d.group == 1 && d.fh == 1 && d.fw == 1 && d.pad_h == 0 && d.pad_w == 0 &&
+           d.ic <= 128 && epi_residual_table(p.epi, &c, &tab);
+}
+
 static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_preprocess) {
     const mi355_conv_desc& d = p.d;
     if (p.pout == 1) {
         // planar destination: 128 x 128 tiles once they fill the device, else 64 x 64
         const int64_t t128 = (int64_t)((d.oc + 127) / 128) * (((int64_t)d.n * p.oh * p.ow + 127) / 128);
         return d.oc > 64 && t128 >= (cu_count > 0 ? cu_count : 256) ? 0 : 3;
+    }
+    if (d.group == 1 && !igemm_needs_general(p) && !igemm_takes_table(p)) {
+        // few output pixels: the reduction split over the waves of a workgroup (a residual layer whose requantisation has
+        // the table form stays on the streaming kernel, which has it)
+        IgemmArgs a;
+        igemm_fill_args(p, a);
+        const int ks = igemm5_pick(a, p.pin, p.pout);
+        if (ks >= 0) return igemm_first_ks_cfg() + ks;
     }
     if (p.pin == 32 && p.pout == 32 && d.group == 1 && !igemm_needs_general(p) && d.fh == 3 && d.fw == 3 &&
         d.stride_h == 1 && d.stride_w == 1 && d.pad_h == 1 && d.pad_w == 1 && (d.ic == 32 || d.ic == 64)) {
@@ -602,10 +623,8 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         // 128 -> 512 at 28 x 28: 14.6 against 16.1)
         // Over at most 64 channels the streaming kernel wins without a table too (64 -> 256 at 56 x 56 with the
         // multi-step form, inside the ResNet-50 stack: -4 us per step against the tiled kernel, alternating bench runs).
-        float c;
-        const float* tab;
         const int s = igemm_pw32s_cfg();
-        if ((d.ic <= 64 || epi_residual_table(p.epi, &c, &tab)) && igemm_resolve_cfg(p, s) == s) return s;
+        if ((d.ic <= 64 || igemm_takes_table(p)) && igemm_resolve_cfg(p, s) == s) return s;
     }
     if (will_preprocess && p.pin == 32 && p.pout == 32 && d.group == 1 && !igemm_needs_general(p)) {
         // The caller re-tiles the filter for the chosen algorithm (weight pre-processing): the second-generation tiles
@@ -712,7 +731,8 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
 
 size_t igemm_preprocessed_bytes(const ConvProblem& p, int cfg) {
     // the weight-resident tiles read the reference layout (once per workgroup: nothing to gain from re-tiling)
-    if (p.pin != 32 || cfg < igemm_first_v2_cfg() || cfg >= igemm_first_v4_cfg()) return 0;
+    const bool ks = cfg >= igemm_first_ks_cfg() && cfg < igemm_num_cfgs();
+    if (p.pin != 32 || !(ks || (cfg >= igemm_first_v2_cfg() && cfg < igemm_first_v4_cfg()))) return 0;
     return igemm2_preprocessed_bytes((int)p.d.oc, (int)(p.icpg * p.d.fh * p.d.fw));
 }
 
@@ -787,6 +807,10 @@ int igemm_resolve_cfg(const ConvProblem& p, int cfg) {
     const int first_v2 = igemm_first_v2_cfg();
     // group convolutions and the general epilogue exist on the second-generation tiles only
     if ((d.group != 1 || a.general) && cfg < first_v2) cfg = first_v2 + (p.ocpg <= 64 ? 3 : 0);
+    if (cfg >= igemm_first_ks_cfg()) {
+        if (igemm5_can_run(a, p.pin, p.pout, cfg - igemm_first_ks_cfg())) return cfg;
+        cfg = first_v2;
+    }
     if (cfg == igemm_pw32s_cfg()) {
         // the 32-packed streaming kernel: pointwise over at most 128 channels; otherwise as above
         if (pw32s_usable(a, p.pin, p.pout)) return cfg;
@@ -886,6 +910,7 @@ int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_coun
             a.ztab = tab;
         }
     }
+    if (cfg >= igemm_first_ks_cfg()) return launch_igemm5(st, a, p.pin, p.pout, cfg - igemm_first_ks_cfg());
     if (cfg == igemm_pw32s_cfg()) return launch_pw32s(st, a, cu_count);
     if (cfg >= igemm_first_v4_cfg()) return launch_igemm4(st, a, p.pin, p.pout, cfg - igemm_first_v4_cfg(), cu_count);
     if (cfg >= igemm_first_v3_cfg()) return launch_igemm3(st, a, p.pin, p.pout, cfg - igemm_first_v3_cfg());

@@ -1,0 +1,373 @@
+// Implicit GEMM for convolutions with few output pixels (tiles "v2_ks_*" for 32-packed
+// inputs, "ks4_*" for 4-packed ones): the reduction of one small output tile is split
+// over the waves of a workgroup, and operands go from global memory straight into registers.
+//
+// A layer of one image leaves a tiled kernel two bad choices: its tiles are too few for the chip, and one tile is a serial
+// chain of LDS stages (copy, barrier, multiply) as long as the reduction -- 3x3 over 512 channels at 7 x 7 took 11 us on
+// 16 workgroups, 36 stages of 0.3 us each, whatever the tile.  What bounds such a layer is latency, so this kernel has
+// next to none of its own:
+//   * tile = 16 to 64 channels x 16 to 64 pixels, so that the tiles of a layer reach more of the 256 CUs;
+//   * the waves of a workgroup take contiguous pieces of the reduction.  An MFMA operand of a 32-byte k-chunk is one
+//     16-byte load per lane (32 filter rows, or 32 pixels of a 32-packed tensor: one contiguous kilobyte); a wave keeps
+//     several chunks of both operands in flight, sixteen waves therefore most of the tile's operands, and memory is
+//     waited for about once instead of once per stage;
+//   * no staging, no barrier before the partial sums meet in LDS; there the quads of an accumulator block are dealt out
+//     over the waves again, each adds up its quad, adds the bias, requantises and stores.
+// The price is operand traffic (2 KB per MFMA of a 32 x 32 tile, through a path of 64 bytes per clock and CU): with enough
+// pixels to fill the chip the staged tiles win, see the chooser.
+//
+// 4-packed inputs: a lane's 16 k-bytes are four dwords of its pixel, one per (channel block, tap) unit of the filter's own
+// order; a table in LDS says where each unit lies.
+#include <atomic>
+
+#include "igemm_shared.h"
+
+namespace mi355 {
+namespace {
+
+// MFMA steps whose operands a wave keeps in flight
+constexpr int ks_ahead(int s, int mt, int nt) { return s == 16 ? 6 : mt * nt == 1 ? 8 : 4; }
+// 16-byte vectors between the rows of partial sums in LDS (a row: 4 channels of the S pixels of a block): both ways of
+// reading them back -- a row by consecutive lanes, or all rows of a pixel by consecutive lanes -- then meet every bank once
+// per pass
+constexpr int ks_row(int s) { return s == 32 ? 34 : 20; }
+
+struct KsArgs {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    uint32_t src_bytes, flt_bytes, z_bytes, dst_bytes;
+    int IH, IW, OHW, OW, FW, T;
+    int sh, sw, ph, pw;
+    int OC, M, KC, entries;
+    int src_sn, src_scb, dst_sn, dst_scb, z_sn;
+    int flt_rstride, flt_kstride;
+    int tiles_m, tiles_n, by_m;
+    int log_pout, has_bias;
+    FastDiv div_ohw, div_ow, div_t, div_fw;
+    EpiParams epi;
+};
+
+// S = 32: v_mfma_i32_32x32x32_i8, a step is one 32-byte k-chunk; S = 16: v_mfma_i32_16x16x64_i8, a step is two of them.
+// Lane l holds filter row (pixel) l % S and 16 bytes at 16 (l / S) of the step.
+template <int S>
+struct KsAcc;
+template <>
+struct KsAcc<32> {
+    v16i v;
+    __device__ __forceinline__ void clear() { v = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}; }
+    __device__ __forceinline__ void mfma(v4i a, v4i b) { v = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, v, 0, 0, 0); }
+    // quad q: channels 8 q + 4 (lane / 32) .. + 3, a row of its own in LDS
+    __device__ __forceinline__ v4i quad(int q) const { return v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]}; }
+};
+template <>
+struct KsAcc<16> {
+    v4i v;
+    __device__ __forceinline__ void clear() { v = v4i{0, 0, 0, 0}; }
+    __device__ __forceinline__ void mfma(v4i a, v4i b) { v = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, v, 0, 0, 0); }
+    __device__ __forceinline__ v4i quad(int) const { return v; }  // channels 4 (lane / 16) .. + 3
+};
+
+template <int PIN, int S, int MT, int NT, bool PW>
+__global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
+    constexpr int BL = MT * NT;           // S x S blocks of the tile
+    constexpr int ROWS = S / 4;           // channel quads of a block
+    constexpr int PARTS = S == 32 ? 4 : 1;  // a block's quads over its pixels, 64 at a time
+    constexpr int ROWP = ks_row(S), WP = BL * ROWS * ROWP;  // vectors per row, per wave
+    constexpr int CH = S == 32 ? 1 : 2;   // 32-byte chunks per step
+    constexpr int AHEAD = ks_ahead(S, MT, NT);
+    extern __shared__ __attribute__((aligned(16))) v4i red[];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), W = blockDim.x >> 6;
+    const int ls = lane & (S - 1), lk = lane / S;
+
+    // Workgroup b runs on XCD b % 8.  Layers with eight and more channel tiles give each XCD channel tiles of its own (the
+    // filter, the larger operand there, enters one L2 only); the others give each XCD a contiguous run of pixels.
+    int tm, tn;
+    {
+        const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
+        if (a.by_m) {
+            const int r = i / a.tiles_n;
+            tm = r * 8 + x;
+            tn = i - r * a.tiles_n;
+            if (tm >= a.tiles_m) return;
+        } else {
+            const int per = (a.tiles_n + 7) >> 3, r = i / a.tiles_m;
+            tm = i - r * a.tiles_m;
+            tn = x * per + r;
+            if (tn >= a.tiles_n) return;
+        }
+    }
+    const int oc0 = tm * MT * S, px0 = tn * NT * S;
+    const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes);
+    const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, a.flt_bytes);
+
+    // this wave's piece of the reduction, in steps
+    const int steps = (a.KC + CH - 1) / CH;
+    const int per = steps / W, extra = steps - per * W;
+    const int k0 = wave * per + (wave < extra ? wave : extra), k1 = k0 + per + (wave < extra ? 1 : 0);
+
+    KEntry* tab = reinterpret_cast<KEntry*>(red + W * WP);
+    if (PIN == 4 && !PW) {
+        for (int u = t; u < steps * CH * 8; u += blockDim.x) {
+            const uint32_t cb = fdiv(u, a.div_t), tap = u - cb * a.T, fh = fdiv(tap, a.div_fw), fw = tap - fh * a.FW;
+            tab[u] = u < a.entries ? KEntry{(int)cb * a.src_scb + ((int)fh * a.IW + (int)fw) * 4, (int)(fh | fw << 16)}
+                                   : KEntry{0, 0x4000};
+        }
+    }
+
+    int arow[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int row = oc0 + i * S + ls;
+        arow[i] = row < a.OC ? row * a.flt_rstride + (S == 32 ? lk * 16 : (lk >> 1) * a.flt_kstride + (lk & 1) * 16) : SENT;
+    }
+    int pix[NT], ih0[NT], iw0[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int m = px0 + j * S + ls;
+        const bool ok = m < a.M;
+        const uint32_t mm = ok ? m : 0;
+        const uint32_t n = fdiv(mm, a.div_ohw), rem = mm - n * a.OHW;
+        const uint32_t oh = fdiv(rem, a.div_ow), ow = rem - oh * a.OW;
+        ih0[j] = ok ? (int)oh * a.sh - a.ph : -0x10000;  // no tap of a pixel past the last one lies inside
+        iw0[j] = (int)ow * a.sw - a.pw;
+        pix[j] = (int)n * a.src_sn + ((int)oh * a.sh - a.ph) * a.IW * PIN + iw0[j] * PIN + (PIN == 32 ? (lk & 1) * 16 : 0);
+        if (PW && !ok) pix[j] = SENT;
+    }
+    if (PIN == 4 && !PW) __syncthreads();
+
+    // load cursor: step kc; for 32-packed inputs and one chunk per step its channel block and tap (wave-uniform)
+    int kc = k0, cb = 0, fh = 0, fw = 0;
+    if (PIN == 32 && !PW && S == 32) {
+        cb = (int)fdiv(k0, a.div_t);
+        const int tap = k0 - cb * a.T;
+        fh = (int)fdiv(tap, a.div_fw);
+        fw = tap - fh * a.FW;
+    }
+    const int FH = PW ? 1 : a.T / a.FW;
+    // Operands of the next step.  Past the wave's piece every lane is out of the buffers' range: zeros, no memory access
+    // (an unconditional load keeps the number of loads in flight known to the compiler, and with it the waits short).
+    // A 4-packed row may end inside its last chunk, so there the whole offset stands where the descriptor checks it.
+    auto load = [&](v4i (&fa)[MT], v4i (&fb)[NT]) __attribute__((always_inline)) {
+        const bool in = kc < k1;
+        const int kf = kc * CH * a.flt_kstride;
+        const bool half_in = S == 32 || kc * 2 + (lk >> 1) < a.KC;  // an odd number of chunks: no second one in the last step
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const bool ok = in && half_in && arow[i] != SENT;
+            fa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, ok ? arow[i] + kf : SENT, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            if (PIN == 32 && PW) {
+                const int c = S == 32 ? 0 : (lk >> 1) * a.src_scb;
+                fb[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, in && half_in && pix[j] != SENT ? pix[j] + c : SENT, kc * CH * a.src_scb, 0);
+            } else if (PIN == 32 && S == 32) {
+                const bool ok = in && (unsigned)(ih0[j] + fh) < (unsigned)a.IH && (unsigned)(iw0[j] + fw) < (unsigned)a.IW;
+                fb[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, ok ? pix[j] + (fh * a.IW + fw) * 32 : SENT, cb * a.src_scb, 0);
+            } else if (PIN == 32) {
+                const uint32_t c = kc * 2 + (lk >> 1), b = fdiv(c, a.div_t), tap = c - b * a.T, h = fdiv(tap, a.div_fw), w = tap - h * a.FW;
+                const bool ok = in && half_in && (unsigned)(ih0[j] + (int)h) < (unsigned)a.IH && (unsigned)(iw0[j] + (int)w) < (unsigned)a.IW;
+                fb[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, ok ? pix[j] + ((int)h * a.IW + (int)w) * 32 + (int)b * a.src_scb : SENT, 0, 0);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int u = kc * CH * 8 + lk * 4 + i;
+                    if (PW) {
+                        fb[j][i] = __builtin_amdgcn_raw_buffer_load_b32(rs_src, in && u < a.entries && pix[j] != SENT ? pix[j] + u * a.src_scb : SENT, 0, 0);
+                    } else {
+                        const KEntry e = tab[in ? u : 0];
+                        const bool ok = in && (unsigned)(ih0[j] + (e.fhfw & 0xffff)) < (unsigned)a.IH &&
+                                        (unsigned)(iw0[j] + (e.fhfw >> 16)) < (unsigned)a.IW;
+                        fb[j][i] = __builtin_amdgcn_raw_buffer_load_b32(rs_src, ok ? pix[j] + e.off : SENT, 0, 0);
+                    }
+                }
+            }
+        }
+        ++kc;
+        if (PIN == 32 && !PW && S == 32) {
+            if (++fw == a.FW) {
+                fw = 0;
+                if (++fh == FH) {
+                    fh = 0;
+                    ++cb;
+                }
+            }
+        }
+    };
+
+    KsAcc<S> acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j].clear();
+
+    // The partial sums of a block are dealt out over the waves in parts of 64 quads: by rows where the destination keeps
+    // four channels of a pixel together (consecutive pixels are contiguous), by pixels where it keeps 32.
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.z_bytes);
+    const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
+    const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes);
+    int d_off = SENT, at_red = 0;
+    v4i bv = {0, 0, 0, 0};
+    uint32_t zw = 0;
+    auto fetch = [&](int u) __attribute__((always_inline)) {
+        const int blk = u / PARTS, part = u % PARTS, i = blk / NT, j = blk % NT;
+        const int row = a.log_pout == 5 ? lane % ROWS : part * (64 / S) + lk;  // channels 4 row .. + 3 of the block
+        const int px = a.log_pout == 5 ? part * (64 / ROWS) + lane / ROWS : ls;
+        at_red = (blk * ROWS + row) * ROWP + px;
+        const int oc4 = oc0 + i * S + row * 4, m = px0 + j * S + px;
+        const bool ok = m < a.M && oc4 < a.OC;
+        const uint32_t mm = m < a.M ? m : 0;
+        const uint32_t n = fdiv(mm, a.div_ohw), rem = mm - n * a.OHW;
+        const int at = (oc4 >> a.log_pout) * a.dst_scb + ((int)rem << a.log_pout) + (oc4 & ((1 << a.log_pout) - 1));
+        d_off = ok ? (int)n * a.dst_sn + at : SENT;
+        bv = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, oc4 * 4, 0, 0);
+        zw = 0;
+        if (a.epi.has_z) zw = __builtin_amdgcn_raw_buffer_load_b32(rs_z, ok ? (int)n * a.z_sn + at : SENT, 0, 0);
+    };
+
+    if (k0 < k1) {  // (waves beyond the number of steps have nothing to add)
+        v4i fa[AHEAD][MT], fb[AHEAD][NT];
+#pragma unroll
+        for (int g = 0; g < AHEAD; ++g) load(fa[g], fb[g]);
+        auto multiply = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j].mfma(fa[g][i], fb[g][j]);
+        };
+        int left = k1 - k0;
+        for (; left > AHEAD; left -= AHEAD) {
+#pragma unroll
+            for (int g = 0; g < AHEAD; ++g) {
+                multiply(g);
+                load(fa[g], fb[g]);
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < AHEAD; ++g)
+            if (g < left) multiply(g);
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int q = 0; q < PARTS; ++q)
+                red[wave * WP + ((i * NT + j) * ROWS + q * (64 / S) + lk) * ROWP + ls] = acc[i][j].quad(q);
+    if (wave < BL * PARTS) fetch(wave);  // lands while the partial sums meet
+    __syncthreads();
+    for (int u = wave; u < BL * PARTS; u += W) {
+        if (u != wave) fetch(u);
+        v4i s = bv;
+#pragma unroll 4
+        for (int w = 0; w < W; ++w) s += red[w * WP + at_red];
+        const uint32_t o = requant4(s[0], s[1], s[2], s[3], zw, a.epi);
+        __builtin_amdgcn_raw_buffer_store_b32(o, rs_dst, d_off, 0, 0);
+    }
+}
+
+struct KsCfg {
+    int pin, s, mt, nt, waves;
+    const char* name;
+};
+constexpr KsCfg kKs[] = {
+        {32, 16, 1, 1, 8, "v2_ks_16x16w8"}, {32, 16, 1, 1, 4, "v2_ks_16x16w4"}, {32, 32, 1, 1, 8, "v2_ks_32x32w8"},
+        {32, 32, 1, 1, 4, "v2_ks_32x32w4"}, {32, 32, 2, 1, 8, "v2_ks_64x32w8"}, {32, 32, 2, 1, 4, "v2_ks_64x32w4"},
+        {4, 16, 1, 1, 8, "ks4_16x16w8"},    {4, 16, 1, 1, 4, "ks4_16x16w4"},    {4, 32, 1, 1, 8, "ks4_32x32w8"},
+        {4, 32, 1, 1, 4, "ks4_32x32w4"},    {4, 32, 2, 1, 8, "ks4_64x32w8"},    {4, 32, 2, 1, 4, "ks4_64x32w4"}};
+constexpr int kKsCount = sizeof(kKs) / sizeof(kKs[0]);
+
+int ks_lds(const IgemmArgs& a, const KsCfg& c, bool pw) {
+    return c.waves * c.mt * c.nt * (c.s / 4) * ks_row(c.s) * 16 + (c.pin == 4 && !pw ? (a.KC + 1) * 8 * 8 : 0);
+}
+
+template <int PIN, int S, int MT, int NT, bool PW>
+int launch_ks(hipStream_t st, const KsArgs& k, int waves, int lds) {
+    auto kern = ks_kernel<PIN, S, MT, NT, PW>;
+    static std::atomic<int> max_lds_set{0};
+    if (lds > max_lds_set.load(std::memory_order_relaxed)) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return (int)e;
+        max_lds_set.store(160 * 1024, std::memory_order_relaxed);
+    }
+    const int64_t grid = k.by_m ? (int64_t)((k.tiles_m + 7) / 8) * k.tiles_n * 8 : (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
+    if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(waves * 64), lds, st, k);
+}
+
+}  // namespace
+
+int igemm5_num_cfgs() { return kKsCount; }
+const char* igemm5_cfg_name(int cfg) { return kKs[cfg].name; }
+
+// The tile for a problem, or -1 where the staged tiles are the better ones.  The line between them is the number of
+// workgroups a tile would make: up to about one per CU this kernel hides what the staged tiles wait for, beyond that its
+// operand traffic costs more.  Drawn from the ResNet-50 and MobileNetV2 layers at batch 1 to 64 (sizes 128 to 263), each on
+// every tile: the choice is within 2 % of the best tile over each network's layers.  At batch 1 its layers sum to 178 us
+// instead of 255 (3x3 over 512 channels at 7 x 7: 11.0 -> 4.2 us; over 256 at 14 x 14: 7.2 -> 3.4; 1024 -> 256 at 14 x 14:
+// 4.3 -> 3.0), the pointwise layers of MobileNetV2 to 115 instead of 140.
+static int ks_id(int pin, int s, int mt, int waves) {
+    for (int i = 0; i < kKsCount; ++i)
+        if (kKs[i].pin == pin && kKs[i].s == s && kKs[i].mt == mt && kKs[i].waves == waves) return i;
+    return -1;
+}
+int igemm5_pick(const IgemmArgs& a, int pin, int pout) {
+    auto tiles = [&](int bm, int bn) { return (int64_t)((a.OC + bm - 1) / bm) * ((a.M + bn - 1) / bn); };
+    const int64_t g16 = tiles(16, 16), g32 = tiles(32, 32), g64 = tiles(64, 32);
+    const int K = a.kbytes;
+    const bool window = a.T > 1;
+    int id = -1;
+    if (pin == 32) {
+        if (K >= 512 && g16 <= 256) id = ks_id(32, 16, 1, K >= 2048 ? 8 : 4);
+        else if (K >= 512 && window && g16 <= 600) id = ks_id(32, 16, 1, 4);
+        else if (g32 <= 256 && (K < 1024 || g16 <= 600)) id = ks_id(32, 32, 1, K >= 2048 && !window ? 8 : 4);
+        else if (g32 <= 200 && window && K >= 1024) id = ks_id(32, 32, 1, 4);
+        else if (g64 <= 256) id = ks_id(32, 32, 2, K >= 512 || K <= 128 ? 8 : 4);
+    } else {
+        if (K >= 128 && g16 <= 300) id = ks_id(4, 16, 1, K >= 1024 ? 8 : 4);
+        else if (g64 <= 256) id = ks_id(4, 32, 2, K <= 192 ? 8 : 4);
+    }
+    return id >= 0 && igemm5_can_run(a, pin, pout, id) ? id : -1;
+}
+
+bool igemm5_can_run(const IgemmArgs& a, int pin, int pout, int cfg) {
+    if (cfg < 0 || cfg >= kKsCount || kKs[cfg].pin != pin || a.groups != 1 || a.general || (pout != 4 && pout != 32)) return false;
+    const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0;
+    return ks_lds(a, kKs[cfg], pw) <= 160 * 1024;
+}
+
+int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg) {
+    if (!igemm5_can_run(a, pin, pout, cfg)) return (int)hipErrorInvalidConfiguration;
+    const KsCfg& c = kKs[cfg];
+    KsArgs k;
+    k.src = a.src; k.flt = a.flt; k.bias = a.bias; k.z = a.z; k.dst = a.dst;
+    k.src_bytes = a.src_bytes; k.flt_bytes = a.flt_bytes; k.z_bytes = a.z_bytes; k.dst_bytes = a.dst_bytes;
+    k.IH = a.IH; k.IW = a.IW; k.OHW = a.OHW; k.OW = a.OW; k.FW = a.FW; k.T = a.T;
+    k.sh = a.sh; k.sw = a.sw; k.ph = a.ph; k.pw = a.pw;
+    k.OC = a.OC; k.M = a.M; k.KC = a.KC; k.entries = a.entries;
+    k.src_sn = a.src_sn; k.src_scb = a.src_scb; k.dst_sn = a.dst_sn; k.dst_scb = a.dst_scb; k.z_sn = a.z_sn;
+    k.flt_rstride = a.flt_rstride; k.flt_kstride = a.flt_kstride;
+    k.tiles_m = (a.OC + c.s * c.mt - 1) / (c.s * c.mt);
+    k.tiles_n = (a.M + c.s * c.nt - 1) / (c.s * c.nt);
+    k.by_m = k.tiles_m >= 8;
+    k.log_pout = pout == 32 ? 5 : 2;
+    k.has_bias = a.has_bias;
+    k.div_ohw = a.div_ohw; k.div_ow = a.div_ow; k.div_t = a.div_t; k.div_fw = a.div_fw;
+    k.epi = a.epi;
+    const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0;
+    const int lds = ks_lds(a, c, pw);
+#define MI355_KS(PIN, S, MT, NT) \
+    (pw ? launch_ks<PIN, S, MT, NT, true>(st, k, c.waves, lds) : launch_ks<PIN, S, MT, NT, false>(st, k, c.waves, lds))
+    if (pin == 32) {
+        if (c.s == 16) return MI355_KS(32, 16, 1, 1);
+        return c.mt == 1 ? MI355_KS(32, 32, 1, 1) : MI355_KS(32, 32, 2, 1);
+    }
+    if (c.s == 16) return MI355_KS(4, 16, 1, 1);
+    return c.mt == 1 ? MI355_KS(4, 32, 1, 1) : MI355_KS(4, 32, 2, 1);
+#undef MI355_KS
+}
+
+}  // namespace mi355

@@ -421,6 +421,14 @@ const char* igemm4_cfg_name(int cfg);
 bool igemm4_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
 int launch_igemm4(hipStream_t st, IgemmArgs& a, int pin, int pout, int cfg, int cu_count);
 
+// few output pixels: the reduction split over the waves of a workgroup, operands straight into registers
+// (conv_igemm5.hip); reads the reference filter layout or the pre-processed one
+int igemm5_num_cfgs();
+const char* igemm5_cfg_name(int cfg);
+bool igemm5_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
+int igemm5_pick(const IgemmArgs& a, int pin, int pout);  // the tile for few output pixels, -1 where there are too many
+int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg);
+
 // streaming kernel for 4-packed pointwise layers with few input or few output channels (conv_pw4.hip)
 bool pw4s_usable(const IgemmArgs& a);
 int launch_pw4s(hipStream_t st, const IgemmArgs& a, int cu_count);
