@@ -485,24 +485,54 @@ int canonize_checked(const mi355_conv_desc* d, ConvProblem* p) {
     return MI355_OK;
 }
 
-// An operator call canonizes the same descriptor several times in a row (get_workspace_in_bytes, the algorithm
-// choice, exec): each thread remembers the last descriptor that passed and its canonical form.  Equal bytes mean an
-// equal descriptor; different padding bytes only cost the full path.
+// What follows from a descriptor alone is kept per thread: its canonical form and what the heuristic answers for it.  An
+// operator call needs them several times in a row (get_workspace_in_bytes, the algorithm choice, exec), a network of some
+// fifty layers once per layer and pass.  A direct-mapped table of kMemo entries, so bounded; equal bytes mean an equal
+// descriptor, different padding bytes only cost the full path.  (A call on a small layer spends 2.7 us in its launch; the
+// full path costs another 0.9 us, an answer from here 0.1 us.)
+struct Memo {
+    bool have = false;
+    mi355_conv_desc key;
+    ConvProblem p;
+    bool have_heuristic[2] = {false, false};  // [for a caller that pre-processes the filter]
+    mi355_algo heuristic[2];
+    int heuristic_cu[2];
+    size_t workspace[2];
+};
+constexpr uint32_t kMemo = 64;
+
+// the entry of a valid descriptor, or null and the error status; valid until the thread's next call of find_memo
+Memo* find_memo(const mi355_conv_desc* d, int* status) {
+    if (!d) {
+        *status = fail(MI355_ERR_BAD_ARG, "null descriptor");
+        return nullptr;
+    }
+    thread_local Memo table[kMemo];
+    static_assert(sizeof(mi355_conv_desc) % 8 == 0, "hashed as 64-bit words");
+    uint64_t h = 0, w;
+    for (size_t i = 0; i < sizeof(*d); i += 8) {
+        memcpy(&w, reinterpret_cast<const char*>(d) + i, 8);
+        h = (h ^ w) * 0x9e3779b97f4a7c15ull;
+        h ^= h >> 29;
+    }
+    Memo* m = &table[h % kMemo];
+    if (m->have && memcmp(d, &m->key, sizeof(*d)) == 0) return m;
+    ConvProblem p;
+    *status = canonize_checked(d, &p);
+    if (*status != MI355_OK) return nullptr;
+    m->p = p;
+    memcpy(&m->key, d, sizeof(*d));
+    m->have = true;
+    m->have_heuristic[0] = m->have_heuristic[1] = false;
+    return m;
+}
+
 int canonize(const mi355_conv_desc* d, ConvProblem* p) {
-    if (!d) return fail(MI355_ERR_BAD_ARG, "null descriptor");
-    thread_local bool have = false;
-    thread_local ConvProblem last;
-    if (have && memcmp(d, &last.d, sizeof(*d)) == 0) {
-        *p = last;
-        return MI355_OK;
-    }
-    const int st = canonize_checked(d, p);
-    if (st == MI355_OK) {
-        last = *p;
-        memcpy(&last.d, d, sizeof(*d));  // padding bytes included, so that the comparison above can hit
-        have = true;
-    }
-    return st;
+    int st = MI355_OK;
+    const Memo* m = find_memo(d, &st);
+    if (!m) return st;
+    *p = m->p;
+    return MI355_OK;
 }
 
 struct DevInfo {
@@ -638,24 +668,35 @@ int mi355_convbias_algo_usable(const mi355_conv_desc* d, int id) {
 
 int mi355_convbias_s8_query(const mi355_conv_desc* d, int algo_request, mi355_algo* algo_out,
                             size_t* workspace_bytes) {
-    ConvProblem p;
-    int st = canonize(d, &p);
-    if (st) return st;
+    int st = MI355_OK;
+    Memo* m = find_memo(d, &st);
+    if (!m) return st;
+    const ConvProblem& p = m->p;
     int id = algo_request;
     const bool pre = algo_request == MI355_ALGO_HEURISTIC_PREPROCESS;
     if (id == MI355_ALGO_HEURISTIC || pre) {
-        id = pick_algo(p);
-    } else if (id < 0 || id >= ALGO_COUNT) {
-        return fail(MI355_ERR_ALGO, "unknown algorithm id %d", id);
-    } else if (!algo_usable(p, id)) {
-        return fail(MI355_ERR_ALGO, "%s cannot run this problem", kAlgoNames[id]);
+        const int cu = cu_count();
+        if (!m->have_heuristic[pre] || m->heuristic_cu[pre] != cu) {
+            mi355_algo& a = m->heuristic[pre];
+            a.id = pick_algo(p);
+            a.tile_cfg = a.id == ALGO_IGEMM_MFMA ? igemm_pick_cfg(p, cu, pre) : 0;
+            // an algorithm the heuristic chose may be replaced by the generic kernel at exec time (misaligned tensors);
+            // one the caller asked for by id may not
+            a.reserved = MI355_ALGO_FLAG_HEURISTIC;
+            m->workspace[pre] = algo_workspace(p, a.id);
+            m->heuristic_cu[pre] = cu;
+            m->have_heuristic[pre] = true;
+        }
+        if (algo_out) *algo_out = m->heuristic[pre];
+        if (workspace_bytes) *workspace_bytes = m->workspace[pre];
+        return MI355_OK;
     }
+    if (id < 0 || id >= ALGO_COUNT) return fail(MI355_ERR_ALGO, "unknown algorithm id %d", id);
+    if (!algo_usable(p, id)) return fail(MI355_ERR_ALGO, "%s cannot run this problem", kAlgoNames[id]);
     if (algo_out) {
         algo_out->id = id;
-        algo_out->tile_cfg = id == ALGO_IGEMM_MFMA ? igemm_pick_cfg(p, cu_count(), pre) : 0;
-        // an algorithm the heuristic chose may be replaced by the generic kernel at exec time (misaligned tensors);
-        // one the caller asked for by id may not
-        algo_out->reserved = algo_request == MI355_ALGO_HEURISTIC || pre ? MI355_ALGO_FLAG_HEURISTIC : 0;
+        algo_out->tile_cfg = id == ALGO_IGEMM_MFMA ? igemm_pick_cfg(p, cu_count()) : 0;
+        algo_out->reserved = 0;
     }
     // the packed-format kernels read the reference layouts in place (no filter repack, no float staging): 0 bytes;
     // the plain-NCHW algorithm keeps its packed intermediates in the workspace
@@ -666,9 +707,10 @@ int mi355_convbias_s8_query(const mi355_conv_desc* d, int algo_request, mi355_al
 // filter: the reference layout, or (preprocessed) the artefact of mi355_convbias_s8_preprocess for this algorithm
 static int exec_impl(void* stream, const mi355_conv_desc* d, const mi355_algo* algo, const int8_t* src, const int8_t* filter,
                      bool preprocessed, const int32_t* bias, const int8_t* z, void* dst, void* workspace, size_t workspace_bytes) {
-    ConvProblem p;
-    int st = canonize(d, &p);
-    if (st) return st;
+    int st = MI355_OK;
+    const Memo* m = find_memo(d, &st);
+    if (!m) return st;
+    const ConvProblem& p = m->p;
     if (!src || !filter || !dst) return fail(MI355_ERR_BAD_ARG, "null tensor pointer");
     if (d->bias_mode != MI355_BIAS_NONE && !bias) return fail(MI355_ERR_BAD_ARG, "bias_mode set but bias is null");
     if (d->has_z && !z) return fail(MI355_ERR_BAD_ARG, "has_z set but z is null");
@@ -678,10 +720,20 @@ static int exec_impl(void* stream, const mi355_conv_desc* d, const mi355_algo* a
         id = pick_algo(p, workspace ? workspace_bytes : 0);  // whatever fits the workspace the caller brought
         cfg = -1;
     }
-    if (id < 0 || id >= ALGO_COUNT) return fail(MI355_ERR_ALGO, "unknown algorithm id %d", id);
-    if (!algo_usable(p, id)) return fail(MI355_ERR_ALGO, "%s cannot run this problem", kAlgoNames[id]);
+    // the heuristic's own answer for this descriptor: usable, resolved to the tile that runs, its workspace known
+    const mi355_algo* known = nullptr;
+    size_t ws_need = 0;
+    for (int k = 0; k < 2 && !known; ++k)
+        if (m->have_heuristic[k] && m->heuristic[k].id == id && m->heuristic[k].tile_cfg == cfg) {
+            known = &m->heuristic[k];
+            ws_need = m->workspace[k];
+        }
+    if (!known) {
+        if (id < 0 || id >= ALGO_COUNT) return fail(MI355_ERR_ALGO, "unknown algorithm id %d", id);
+        if (!algo_usable(p, id)) return fail(MI355_ERR_ALGO, "%s cannot run this problem", kAlgoNames[id]);
+        ws_need = algo_workspace(p, id);
+    }
     // check_exec's workspace rule (dnn/src/common/conv_bias.cpp:32-37)
-    const size_t ws_need = algo_workspace(p, id);
     if (ws_need) {
         if (!workspace || workspace_bytes < ws_need)
             return fail(MI355_ERR_WORKSPACE, "workspace of %zu bytes, %s needs %zu", workspace ? workspace_bytes : (size_t)0,
@@ -689,7 +741,7 @@ static int exec_impl(void* stream, const mi355_conv_desc* d, const mi355_algo* a
         if (!aligned16(workspace)) return fail(MI355_ERR_BAD_ARG, "the workspace needs 16-byte alignment");
     }
     const bool by_heuristic = !algo || algo->id == MI355_ALGO_HEURISTIC || (algo->reserved & MI355_ALGO_FLAG_HEURISTIC);
-    if (id == ALGO_IGEMM_MFMA) {
+    if (id == ALGO_IGEMM_MFMA && !known) {
         if (cfg < 0 || cfg >= igemm_num_cfgs()) {
             cfg = igemm_pick_cfg(p, cu_count());
         } else {

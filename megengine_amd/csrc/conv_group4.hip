@@ -1,0 +1,294 @@
+// NCHW4 group convolutions with few channels per group, in one launch (tile "grp4_dot4").
+//
+// Such a layer is G small convolutions.  As G launches of the dense tiles it costs G launch latencies, and a matrix tile of
+// 32 channels is mostly empty when a group has 4, 8 or 16: 32 groups of 4 channels, 3x3 at 56 x 56, batch 16, took 165 us.
+// Here a thread computes 4 or 8 channels of one group for two rows (3x3 filters; otherwise one) of one output column, one
+// byte dot product per 4 input channels and tap:
+//   * a wave's lanes are consecutive output columns of one group of one image: its loads and stores are contiguous runs of
+//     4-byte pixels, and its filter words are the same for all lanes, so they are scalar loads and cost no vector memory;
+//   * two output rows share the input rows between them (12 loads for 8 or 16 outputs at stride 1);
+//   * what lies outside the image is an out-of-range offset of a buffer descriptor that spans the group's planes.
+// Bound by the dot products (9 per 4 channels in and output) and the instructions around its loads.
+//
+// The usual grouped bottleneck -- 3x3, as many channels out of a group as into it, 4, 8 or 16 -- goes to the matrix cores
+// all the same, sixteen channels at a time (one group of 16, two of 8, four of 4): the filter of the slab is a 16 x 16
+// matrix per tap, block-diagonal where several groups share it, and sixteen channels of a pixel are exactly the 16 bytes
+// a lane of v_mfma_i32_16x16x64_i8 holds, so a step is four taps and 3x3 is three steps, zeros of the block diagonal
+// included a third of the time of the dot products.  A workgroup stages a band of input rows in LDS as [pixel][16
+// channels] (NCHW4 keeps them in four planes), so every operand is one conflict-free ds_read_b128; the filter stays in
+// twelve registers; the next band is in flight while this one is multiplied.
+// 32 groups of 4 at 56 x 56, batch 16 (13 MB): 165 us as 32 launches, 9.8 with dot products, 6.8 here; 32 groups of 16
+// (51 MB): 50 us with dot products, 17 here.
+#include "igemm_shared.h"
+
+namespace mi355 {
+namespace {
+
+constexpr int GRP4_MAX_IC = 16;  // beyond, a group is worth a matrix tile of its own
+
+struct Grp4Args {
+    const int8_t* src;
+    const int* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    int IH, IW, OH, OW, FH, FW, sh, sw, ph, pw;
+    int icb, ocpg, src_scb, dst_scb, has_bias;
+    int64_t src_sn, dst_sn, z_sn;
+    uint32_t items;
+    FastDiv div_ow;
+    EpiParams epi;
+};
+
+// OQ: output channel quads per thread; F = 3: 3x3 filter, stride ST, two output rows per thread; F = 0: any filter, one row
+template <int OQ, int F, int ST>
+__global__ __launch_bounds__(256) void grp4_kernel(Grp4Args a) {
+    constexpr int R = F == 3 ? 2 : 1;
+    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
+    const bool live = it < a.items;
+    const uint32_t ohs = fdiv(live ? it : 0, a.div_ow), ow = (live ? it : 0) - ohs * a.OW;
+    const int oh0 = (int)ohs * R, oc0 = blockIdx.y * OQ * 4, g = oc0 / a.ocpg;
+    const int64_t n = blockIdx.z;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.src + n * a.src_sn + (int64_t)g * a.icb * a.src_scb, (uint32_t)(a.icb * a.src_scb));
+    const int ih0 = oh0 * a.sh - a.ph, iw0 = (int)ow * a.sw - a.pw;
+    const int T = F == 3 ? 9 : a.FH * a.FW;
+    const int* __restrict__ w = a.flt + (int64_t)oc0 * a.icb * T;
+
+    int acc[R][OQ * 4];
+#pragma unroll
+    for (int o = 0; o < OQ * 4; ++o)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r][o] = a.has_bias ? a.bias[oc0 + o] : 0;
+
+    // the residual is in flight while the sums are made
+    const int64_t plane = n * a.dst_sn + (int64_t)(oc0 / 4) * a.dst_scb, zplane = n * a.z_sn + (int64_t)(oc0 / 4) * a.dst_scb;
+    uint32_t zw[R][OQ] = {};
+    if (a.epi.has_z) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int q = 0; q < OQ; ++q)
+                if (live && oh0 + r < a.OH)
+                    zw[r][q] = *reinterpret_cast<const uint32_t*>(a.z + zplane + (int64_t)q * a.dst_scb + ((oh0 + r) * a.OW + (int)ow) * 4);
+    }
+
+    for (int ib = 0; ib < a.icb; ++ib) {
+        const int base = ib * a.src_scb;
+        if constexpr (F == 3) {
+            constexpr int ROWS = (R - 1) * ST + 3;
+            int x[ROWS][3];
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                const int row = live && (unsigned)(ih0 + r) < (unsigned)a.IH ? ((ih0 + r) * a.IW + iw0) * 4 : SENT;
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    x[r][c] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (unsigned)(iw0 + c) < (unsigned)a.IW ? row + c * 4 : SENT, base, 0);
+            }
+#pragma unroll
+            for (int o = 0; o < OQ * 4; ++o)
+#pragma unroll
+                for (int t = 0; t < 9; ++t) {
+                    const int f = w[(o * a.icb + ib) * 9 + t];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) acc[r][o] = __builtin_amdgcn_sdot4(x[r * ST + t / 3][t % 3], f, acc[r][o], false);
+                }
+        } else {
+            for (int fh = 0; fh < a.FH; ++fh)
+                for (int fw = 0; fw < a.FW; ++fw) {
+                    const bool ok = live && (unsigned)(ih0 + fh) < (unsigned)a.IH && (unsigned)(iw0 + fw) < (unsigned)a.IW;
+                    const int x = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, ok ? base + ((ih0 + fh) * a.IW + iw0 + fw) * 4 : SENT, 0, 0);
+#pragma unroll
+                    for (int o = 0; o < OQ * 4; ++o)
+                        acc[0][o] = __builtin_amdgcn_sdot4(x, w[(o * a.icb + ib) * T + fh * a.FW + fw], acc[0][o], false);
+                }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int q = 0; q < OQ; ++q) {
+            const uint32_t o = requant4(acc[r][4 * q], acc[r][4 * q + 1], acc[r][4 * q + 2], acc[r][4 * q + 3], zw[r][q], a.epi);
+            if (live && oh0 + r < a.OH)
+                *reinterpret_cast<uint32_t*>(a.dst + plane + (int64_t)q * a.dst_scb + ((oh0 + r) * a.OW + (int)ow) * 4) = o;
+        }
+}
+
+constexpr int G16_PX = 1024;  // pixels of a staged band (16 KiB), four per thread
+
+struct G16Args {
+    const int8_t* src;
+    const int* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    int IH, IW, OH, OW, s, ph, pw;
+    int TH, PW, bands, items;  // output rows of a band, padded input columns, bands per image, bands of the batch
+    int icpg, src_scb, dst_scb, has_bias;
+    int64_t src_sn, dst_sn, z_sn;
+    FastDiv div_pw, div_ow, div_bands;
+    EpiParams epi;
+};
+
+// both dwords through one choice of the requantisation form; the results replace the residual words
+__device__ __forceinline__ void requant8(v4i x, v4i y, uint32_t (&w)[2], const EpiParams& e) {
+#define MI355_BOTH(F)                                  \
+    do {                                               \
+        w[0] = F(x[0], x[1], x[2], x[3], w[0], e);     \
+        w[1] = F(y[0], y[1], y[2], y[3], w[1], e);     \
+    } while (0)
+    if (e.lin) MI355_BOTH((requant4_fast<NL_LIN, false>));
+    else if (e.nonline == NL_RELU && !e.has_z) MI355_BOTH((requant4_fast<NL_RELU, false>));
+    else MI355_BOTH(requant4);
+#undef MI355_BOTH
+}
+
+template <bool HZ>
+__global__ __launch_bounds__(256) void grp16_kernel(G16Args a) {
+    __shared__ __attribute__((aligned(16))) v4i sm[G16_PX];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int l16 = lane & 15, kq = lane >> 4, slab = blockIdx.y, oc = slab * 16 + l16;
+    const int PH = (a.TH - 1) * a.s + 3, patch = PH * a.PW;
+
+    // filter rows: lane = output channel, 16 bytes of tap 4 step + kq = its 16 input channels, zero outside its group
+    v4i fa[3];
+    int tap_off[3];
+    const int icb = a.icpg / 4, first = l16 / a.icpg * icb;  // channel blocks of a group, first one of the lane's group
+#pragma unroll
+    for (int st = 0; st < 3; ++st) {
+        const int tap = st * 4 + kq;
+        tap_off[st] = tap < 9 ? tap / 3 * a.PW + tap % 3 : 0;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            fa[st][b] = tap < 9 && b >= first && b < first + icb ? a.flt[(oc * icb + b - first) * 9 + tap] : 0;
+    }
+    v4i bv = {0, 0, 0, 0};
+    if (a.has_bias) bv = *reinterpret_cast<const v4i*>(a.bias + slab * 16 + kq * 4);
+
+    v4i x[G16_PX / 256];
+    auto fetch = [&](int item) __attribute__((always_inline)) {
+        const int n = (int)fdiv(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.src + n * a.src_sn + (int64_t)slab * 4 * a.src_scb, (uint32_t)a.src_scb * 4);
+#pragma unroll
+        for (int k = 0; k < G16_PX / 256; ++k) {
+            const uint32_t p = t + k * 256, pr = fdiv(p, a.div_pw), pc = p - pr * a.PW;
+            const int ih = oh0 * a.s - a.ph + (int)pr, iw = (int)pc - a.pw;
+            const bool ok = (int)p < patch && (unsigned)ih < (unsigned)a.IH && (unsigned)iw < (unsigned)a.IW;
+            const int off = ok ? (ih * a.IW + iw) * 4 : SENT;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) x[k][b] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, off, b * a.src_scb, 0);
+        }
+    };
+
+    int item = blockIdx.x;
+    fetch(item);
+    while (item < a.items) {
+#pragma unroll
+        for (int k = 0; k < G16_PX / 256; ++k) sm[t + k * 256] = x[k];
+        __syncthreads();
+        const int next = item + gridDim.x;
+        if (next < a.items) fetch(next);  // lands during the multiplies
+        const int n = (int)fdiv(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
+        const int pixels = (a.OH - oh0 < a.TH ? a.OH - oh0 : a.TH) * a.OW;
+        const int64_t at = (int64_t)(slab * 4 + kq) * a.dst_scb + (int64_t)oh0 * a.OW * 4;
+        int8_t* dst = a.dst + n * a.dst_sn + at;
+        const int8_t* z = a.z + n * a.z_sn + at;
+        // two units of 16 pixels at a time: their LDS reads and multiplies overlap
+        for (int u = wave * 32; u < pixels; u += 128) {
+            uint32_t zw[2] = {0, 0};
+            v4i acc[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int p = u + k * 16 + l16, pp = p < pixels ? p : 0;
+                const int oh = (int)fdiv(pp, a.div_ow), ow = pp - oh * a.OW;
+                if (HZ) zw[k] = *reinterpret_cast<const uint32_t*>(z + pp * 4);
+                const v4i* px = sm + (oh * a.PW + ow) * a.s;
+                acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[0], px[tap_off[0]], bv, 0, 0, 0);
+                acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[1], px[tap_off[1]], acc[k], 0, 0, 0);
+                acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[2], px[tap_off[2]], acc[k], 0, 0, 0);
+            }
+            requant8(acc[0], acc[1], zw, a.epi);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int p = u + k * 16 + l16;
+                if (p < pixels) *reinterpret_cast<uint32_t*>(dst + p * 4) = zw[k];
+            }
+        }
+        __syncthreads();
+        item = next;
+    }
+}
+
+// output rows of a band: the largest number whose input patch fits; 0: not even one row fits
+int g16_rows(const ConvProblem& p) {
+    const int s = p.d.stride_h, pw = ((int)p.ow - 1) * s + 3;
+    const int rows = (int)(G16_PX / pw);
+    return rows < 3 ? 0 : (rows - 3) / s + 1;
+}
+
+bool g16_usable(const ConvProblem& p) {
+    const mi355_conv_desc& d = p.d;
+    return d.fh == 3 && d.fw == 3 && d.stride_h == d.stride_w && d.stride_h <= 2 && p.icpg == p.ocpg &&
+           (p.icpg == 4 || p.icpg == 8 || p.icpg == 16) && d.oc % 16 == 0 && p.ow < G16_PX && g16_rows(p) > 0 &&
+           (int64_t)d.ih * d.iw * 16 < (1ll << 31);
+}
+
+int launch_g16(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+               int8_t* dst) {
+    const mi355_conv_desc& d = p.d;
+    G16Args a;
+    a.src = src; a.flt = reinterpret_cast<const int*>(flt); a.bias = bias; a.z = z; a.dst = dst;
+    a.IH = d.ih; a.IW = d.iw; a.OH = p.oh; a.OW = p.ow; a.s = d.stride_h; a.ph = d.pad_h; a.pw = d.pad_w;
+    const int slabs = d.oc / 16;
+    a.TH = g16_rows(p);
+    if (a.TH > (int)p.oh) a.TH = p.oh;
+    // fewer rows per band while that leaves CUs without one
+    while (a.TH > 1 && (int64_t)slabs * d.n * ((p.oh + a.TH - 1) / a.TH) < 512) a.TH = (a.TH + 1) / 2;
+    a.PW = ((int)p.ow - 1) * a.s + 3;
+    a.bands = ((int)p.oh + a.TH - 1) / a.TH;
+    const int64_t items = (int64_t)d.n * a.bands;
+    if (items > 0x3fffffff) return (int)hipErrorInvalidValue;
+    a.items = (int)items;
+    a.icpg = p.icpg; a.src_scb = d.ih * d.iw * 4; a.dst_scb = p.oh * p.ow * 4;
+    a.has_bias = d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL;
+    a.src_sn = p.src_sn; a.dst_sn = p.dst_sn; a.z_sn = p.z_sn;
+    a.div_pw = make_fastdiv(a.PW); a.div_ow = make_fastdiv(p.ow); a.div_bands = make_fastdiv(a.bands);
+    a.epi = p.epi;
+    int64_t per_slab = (2048 + slabs - 1) / slabs;  // eight workgroups per CU over all slabs
+    if (per_slab > items) per_slab = items;
+    const dim3 grid((unsigned)per_slab, slabs);
+    return d.has_z ? launch_kernel(grp16_kernel<true>, grid, dim3(256), 0, st, a) : launch_kernel(grp16_kernel<false>, grid, dim3(256), 0, st, a);
+}
+
+}  // namespace
+
+bool grp4_usable(const ConvProblem& p) {
+    const mi355_conv_desc& d = p.d;
+    return d.format == MI355_FMT_NCHW4 && d.group > 1 && !p.dw4 && p.icpg % 4 == 0 && p.ocpg % 4 == 0 && p.icpg <= GRP4_MAX_IC &&
+           d.n <= 65535 && d.oc / 4 <= 65535 && (uint64_t)p.oh * p.ow < (1u << 28);
+}
+
+int launch_grp4(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+                int8_t* dst) {
+    const mi355_conv_desc& d = p.d;
+    if (d.n == 0 || p.oh == 0 || p.ow == 0) return 0;
+    if (g16_usable(p)) return launch_g16(st, p, src, flt, bias, z, dst);
+    Grp4Args a;
+    a.src = src; a.flt = reinterpret_cast<const int*>(flt); a.bias = bias; a.z = z; a.dst = dst;
+    a.IH = d.ih; a.IW = d.iw; a.OH = p.oh; a.OW = p.ow; a.FH = d.fh; a.FW = d.fw;
+    a.sh = d.stride_h; a.sw = d.stride_w; a.ph = d.pad_h; a.pw = d.pad_w;
+    a.icb = p.icpg / 4; a.ocpg = p.ocpg;
+    a.src_scb = d.ih * d.iw * 4; a.dst_scb = p.oh * p.ow * 4;
+    a.has_bias = d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL;
+    a.src_sn = p.src_sn; a.dst_sn = p.dst_sn; a.z_sn = p.z_sn;
+    a.div_ow = make_fastdiv(p.ow);
+    a.epi = p.epi;
+    const bool f3 = d.fh == 3 && d.fw == 3 && d.stride_h == d.stride_w && d.stride_h <= 2;
+    const bool wide = p.ocpg % 8 == 0;  // 8 channels per thread halve the loads per output
+    a.items = (f3 ? (p.oh + 1) / 2 : p.oh) * p.ow;
+    const dim3 grid((a.items + 255) / 256, d.oc / (wide ? 8 : 4), d.n);
+    if (f3 && d.stride_h == 1) return wide ? launch_kernel(grp4_kernel<2, 3, 1>, grid, dim3(256), 0, st, a) : launch_kernel(grp4_kernel<1, 3, 1>, grid, dim3(256), 0, st, a);
+    if (f3) return wide ? launch_kernel(grp4_kernel<2, 3, 2>, grid, dim3(256), 0, st, a) : launch_kernel(grp4_kernel<1, 3, 2>, grid, dim3(256), 0, st, a);
+    return wide ? launch_kernel(grp4_kernel<2, 0, 1>, grid, dim3(256), 0, st, a) : launch_kernel(grp4_kernel<1, 0, 1>, grid, dim3(256), 0, st, a);
+}
+
+}  // namespace mi355

@@ -482,8 +482,9 @@ int launch_fmt(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
 }  // namespace
 
 // tile_cfg numbering: register-staged tiles, LDS-direct tiles, second-generation tiles, patch-staged tiles, weight-resident
-// tiles, the 32-packed streaming kernel, the tiles that split the reduction over the waves of a workgroup
-int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1 + igemm5_num_cfgs(); }
+// tiles, the 32-packed streaming kernel, the tiles that split the reduction over the waves of a
+// workgroup, the one-launch NCHW4 group kernel
+int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1 + igemm5_num_cfgs() + 1; }
 int igemm_first_v2_cfg() { return kNumCfgs + igemm_dma_num_cfgs(); }
 // planar destination (NCHW4_NCHW): two of the register-staged tiles
 static int launch_planar(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
@@ -498,6 +499,7 @@ static int igemm_first_v3_cfg() { return igemm_first_v2_cfg() + igemm2_num_cfgs(
 static int igemm_first_v4_cfg() { return igemm_first_v3_cfg() + igemm3_num_cfgs(); }
 static int igemm_pw32s_cfg() { return igemm_first_v4_cfg() + igemm4_num_cfgs(); }
 static int igemm_first_ks_cfg() { return igemm_pw32s_cfg() + 1; }
+static int igemm_grp4_cfg() { return igemm_first_ks_cfg() + igemm5_num_cfgs(); }
 const char* igemm_cfg_name(int cfg) {
     if (cfg >= 0 && cfg < kNumCfgs) return kCfgs[cfg].name;
     if (cfg < igemm_first_v2_cfg()) return igemm_dma_cfg_name(cfg - kNumCfgs);
@@ -505,7 +507,8 @@ const char* igemm_cfg_name(int cfg) {
     if (cfg < igemm_first_v4_cfg()) return igemm3_cfg_name(cfg - igemm_first_v3_cfg());
     if (cfg < igemm_pw32s_cfg()) return igemm4_cfg_name(cfg - igemm_first_v4_cfg());
     if (cfg == igemm_pw32s_cfg()) return "pw32_stream";
-    return igemm5_cfg_name(cfg - igemm_first_ks_cfg());
+    if (cfg < igemm_grp4_cfg()) return igemm5_cfg_name(cfg - igemm_first_ks_cfg());
+    return "grp4_dot4";
 }
 
 static bool igemm_needs_general(const ConvProblem& p) {
@@ -731,7 +734,7 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
 
 size_t igemm_preprocessed_bytes(const ConvProblem& p, int cfg) {
     // the weight-resident tiles read the reference layout (once per workgroup: nothing to gain from re-tiling)
-    const bool ks = cfg >= igemm_first_ks_cfg() && cfg < igemm_num_cfgs();
+    const bool ks = cfg >= igemm_first_ks_cfg() && cfg < igemm_grp4_cfg();
     if (p.pin != 32 || !(ks || (cfg >= igemm_first_v2_cfg() && cfg < igemm_first_v4_cfg()))) return 0;
     return igemm2_preprocessed_bytes((int)p.d.oc, (int)(p.icpg * p.d.fh * p.d.fw));
 }
@@ -742,6 +745,9 @@ int launch_igemm_preprocess(hipStream_t st, const ConvProblem& p, const int8_t* 
 
 // The chooser's tile, as the launch code will run it: what query() hands out names the kernel that executes.
 int igemm_pick_cfg(const ConvProblem& p, int cu_count, bool will_preprocess) {
+    // few channels per group: one launch for all groups, always (32 groups of 4 channels, 3x3 at 56 x 56, batch 16: 165 us as
+    // 32 launches; two groups of 16 at 7 x 7: two launches cost more than one, whatever runs in them)
+    if (igemm_group_by_launch(p) && grp4_usable(p)) return igemm_grp4_cfg();
     if (igemm_group_by_launch(p)) return igemm_pick_cfg(igemm_group_view(p), cu_count, will_preprocess);
     const int c = pick_cfg_by_shape(p, cu_count, will_preprocess);
     const int r = igemm_resolve_cfg(p, c);
@@ -796,17 +802,16 @@ static int staged_tile_of_shape(int bm, int bn, int kch) {
     return cfg;
 }
 
-int igemm_resolve_cfg(const ConvProblem& p, int cfg) {
+// `a`: the filled arguments of `p`
+static int resolve_filled(const ConvProblem& p, const IgemmArgs& a, int cfg) {
     if (cfg < 0 || cfg >= igemm_num_cfgs()) return -1;
-    if (igemm_group_by_launch(p)) return igemm_resolve_cfg(igemm_group_view(p), cfg);
     const mi355_conv_desc& d = p.d;
-    IgemmArgs a;
-    igemm_fill_args(p, a);
     if (a.M == 0 || a.OC == 0) return cfg;  // nothing is launched
     if (p.pout == 1) return cfg == 3 ? 3 : 0;  // planar destination: two register-staged tiles
     const int first_v2 = igemm_first_v2_cfg();
     // group convolutions and the general epilogue exist on the second-generation tiles only
     if ((d.group != 1 || a.general) && cfg < first_v2) cfg = first_v2 + (p.ocpg <= 64 ? 3 : 0);
+    if (cfg == igemm_grp4_cfg()) cfg = first_v2;  // (a problem it can run never gets here)
     if (cfg >= igemm_first_ks_cfg()) {
         if (igemm5_can_run(a, p.pin, p.pout, cfg - igemm_first_ks_cfg())) return cfg;
         cfg = first_v2;
@@ -861,10 +866,19 @@ int igemm_resolve_cfg(const ConvProblem& p, int cfg) {
     return cfg;
 }
 
+int igemm_resolve_cfg(const ConvProblem& p, int cfg) {
+    if (cfg == igemm_grp4_cfg() && igemm_group_by_launch(p) && grp4_usable(p)) return cfg;
+    if (igemm_group_by_launch(p)) return igemm_resolve_cfg(igemm_group_view(p), cfg);
+    IgemmArgs a;
+    igemm_fill_args(p, a);
+    return resolve_filled(p, a, cfg);
+}
+
 int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_count, const int8_t* src,
                       const int8_t* flt, const int32_t* bias, const int8_t* z, int8_t* dst, bool flt_preprocessed) {
     if (igemm_group_by_launch(p)) {
         if (flt_preprocessed) return (int)hipErrorInvalidValue;
+        if (cfg == igemm_grp4_cfg() && grp4_usable(p)) return launch_grp4(st, p, src, flt, bias, z, dst);
         const ConvProblem q = igemm_group_view(p);
         const mi355_conv_desc& d = p.d;
         const int64_t src_g = (int64_t)p.icpg * d.ih * d.iw, dst_g = (int64_t)p.ocpg * p.oh * p.ow;
@@ -882,7 +896,7 @@ int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_coun
     igemm_fill_args(p, a);
     a.src = src; a.flt = flt; a.bias = bias; a.z = z; a.dst = dst;
     if (a.M == 0 || a.OC == 0) return 0;
-    cfg = igemm_resolve_cfg(p, cfg);
+    cfg = resolve_filled(p, a, cfg);
     if (cfg < 0) return (int)hipErrorInvalidValue;
     if (flt_preprocessed) {
         if (igemm_preprocessed_bytes(p, cfg) == 0) return (int)hipErrorInvalidValue;

@@ -421,6 +421,11 @@ const char* igemm4_cfg_name(int cfg);
 bool igemm4_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
 int launch_igemm4(hipStream_t st, IgemmArgs& a, int pin, int pout, int cfg, int cu_count);
 
+// NCHW4 group convolutions with few channels per group in one launch (conv_group4.hip, tile "grp4_dot4")
+bool grp4_usable(const ConvProblem& p);
+int launch_grp4(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+                int8_t* dst);
+
 // few output pixels: the reduction split over the waves of a workgroup, operands straight into registers
 // (conv_igemm5.hip); reads the reference filter layout or the pre-processed one
 int igemm5_num_cfgs();
