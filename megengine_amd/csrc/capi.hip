@@ -594,6 +594,12 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 namespace mi355 {
 thread_local LaunchList* t_binding = nullptr;
 
+bool epi_quotient(float scale_dst, float* y_hi, float* y_lo) {
+    *y_hi = 1.0f / scale_dst;
+    *y_lo = epi_recip_lo(scale_dst);
+    return epi_fast_ok(1.f, 1.f, scale_dst, false) && epi_quotient_proved(scale_dst);
+}
+
 bool epi_residual_table(const EpiParams& e, float* c, const float** tab) {
     if (!e.fast || !e.has_z || (e.nonline != MI355_NL_IDENTITY && e.nonline != MI355_NL_RELU)) return false;
     const TableEntry* t = epi_table_cached(e.s_b, e.s_z, e.s_d, e.nonline == MI355_NL_RELU);
@@ -1129,10 +1135,7 @@ int mi355_igemm_tile_usable(const mi355_conv_desc* d, int tile_cfg) {
 
 int mi355_epilogue_quotient_form(float scale_dst, float* y_hi, float* y_lo) {
     if (!y_hi || !y_lo) return -fail(MI355_ERR_BAD_ARG, "null argument");
-    *y_hi = 1.0f / scale_dst;
-    *y_lo = epi_recip_lo(scale_dst);
-    if (!epi_fast_ok(1.f, 1.f, scale_dst, false)) return 0;
-    return epi_quotient_proved(scale_dst) ? 1 : 0;
+    return epi_quotient(scale_dst, y_hi, y_lo) ? 1 : 0;
 }
 
 int mi355_epilogue_linear_form(float scale_bias, float scale_dst, uint32_t nonline, float* c, float* d) {

@@ -36,6 +36,9 @@ struct ConvProblem {
 // for these scales and this activation.  A hash lookup after the first call for a scale triple.
 bool epi_residual_table(const EpiParams& e, float* c, const float** tab);
 
+// The divide-free quotient by scale_dst (epilogue.h): true and the two parts of the reciprocal when it is proved
+bool epi_quotient(float scale_dst, float* y_hi, float* y_lo);
+
 // ---- launchers (each returns a hipError_t-compatible int; 0 = success) ----
 int launch_conv_direct(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt,
                        const int32_t* bias, const void* z, void* dst);

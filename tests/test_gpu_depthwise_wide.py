@@ -1,0 +1,36 @@
+"""Channel-wise 5x5 and 7x7 convolutions at the edges of a thread's work: widths around the blocks of four pixels, odd
+heights (two output rows per thread), images smaller than the filter, both strides, every activation with and without a
+residual; paddings other than F / 2 and odd strides stay on the kernel that takes anything."""
+import pytest
+
+from megengine_amd import _abi, lib, ops
+from tests.gpu_util import check_case
+
+pytestmark = pytest.mark.gpu
+
+S = dict(scale_bias=2e-4, scale_z=0.05, scale_dst=0.05)
+
+
+@pytest.mark.parametrize("f", [5, 7])
+@pytest.mark.parametrize("stride", [1, 2])
+@pytest.mark.parametrize("ih,iw", [(1, 1), (3, 2), (5, 4), (6, 5), (8, 7), (9, 8), (7, 13), (12, 16), (11, 33)])
+def test_same_padding(oracle, f, stride, ih, iw):
+    for k, (nl, z, c) in enumerate((("RELU", False, 8), ("IDENTITY", True, 4), ("H_SWISH", False, 12))):
+        d = _abi.make_conv_desc("NCHW4", 3, c, ih, iw, c, f, pad=f // 2, stride=stride, group=c, nonline=nl, has_z=z, **S)
+        assert lib.algo_names()[ops.conv_bias_query(d)[0].id] == "MI355_DEPTHWISE_DOT4"
+        check_case(oracle, d, seed=10 * f + stride + k, tag="dw%d" % f)
+    # scales for which the one-instruction requantisation is proved
+    d = _abi.make_conv_desc("NCHW44", 2, 8, ih, iw, 8, f, pad=f // 2, stride=stride, group=8, nonline="RELU", scale_bias=1.3e-3,
+                            scale_dst=0.0271)
+    check_case(oracle, d, seed=f, tag="dw%d linear" % f)
+
+
+@pytest.mark.parametrize("f,pad,stride", [(5, 0, 1), (5, (2, 1), 1), (7, 4, 2), (5, 2, 3)])
+def test_other_paddings_and_strides(oracle, f, pad, stride):
+    d = _abi.make_conv_desc("NCHW4", 2, 8, 11, 13, 8, f, pad=pad, stride=stride, group=8, nonline="RELU", has_z=True, **S)
+    check_case(oracle, d, seed=5, tag="dw other")
+
+
+def test_height_padding_may_differ(oracle):
+    d = _abi.make_conv_desc("NCHW4", 2, 8, 11, 13, 8, 5, pad=(1, 2), stride=1, group=8, nonline="RELU", **S)
+    check_case(oracle, d, seed=6, tag="dw pad_h 1")
