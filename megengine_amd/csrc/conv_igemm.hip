@@ -586,6 +586,11 @@ static bool igemm_takes_table(const ConvProblem& p) {
            d.ic <= 128 && epi_residual_table(p.epi, &c, &tab);
 }
 
+// a QuantizedS32 dst and nothing else that needs the general epilogue
+static bool igemm_plain_s32(const ConvProblem& p) {
+    return p.d.dst_dtype == MI355_DT_QS32 && p.d.bias_mode != MI355_BIAS_FULL;
+}
+
 static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_preprocess) {
     const mi355_conv_desc& d = p.d;
     if (p.pout == 1) {
@@ -593,7 +598,7 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         const int64_t t128 = (int64_t)((d.oc + 127) / 128) * (((int64_t)d.n * p.oh * p.ow + 127) / 128);
         return d.oc > 64 && t128 >= (cu_count > 0 ? cu_count : 256) ? 0 : 3;
     }
-    if (d.group == 1 && !igemm_needs_general(p) && !igemm_takes_table(p)) {
+    if (d.group == 1 && (!igemm_needs_general(p) || igemm_plain_s32(p)) && !igemm_takes_table(p)) {
         // few output pixels: the reduction split over the waves of a workgroup (a residual layer whose requantisation has
         // the table form stays on the streaming kernel, which has it)
         IgemmArgs a;
@@ -675,7 +680,12 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
     const int OC = d.oc;
     if (cu_count <= 0) cu_count = 256;
     // group convolution and the general epilogue: second-generation tiles only; a channel tile never spans two groups
-    if (d.group != 1 || igemm_needs_general(p)) return igemm_first_v2_cfg() + (p.ocpg <= 64 ? 3 : 0);
+    // (the 64-channel tile too where 128 x 128 tiles would leave CUs without one: an int32 result 128 -> 256 at 28 x 28, batch 1
+    // to 8: 5.1 .. 6.2 us against 6.5 .. 7.6; 3x3 128 -> 128, batch 16: 8.8 against 11.9; at batch 32 the two are equal)
+    if (d.group != 1 || igemm_needs_general(p)) {
+        const int64_t t128 = (int64_t)d.group * ((p.ocpg + 127) / 128) * ((M + 127) / 128);
+        return igemm_first_v2_cfg() + (p.ocpg <= 64 || (2 * t128 < 3 * (int64_t)cu_count) ? 3 : 0);
+    }
     auto tiles = [&](int cfg) { return ((OC + kCfgs[cfg].bm - 1) / kCfgs[cfg].bm) * ((M + kCfgs[cfg].bn - 1) / kCfgs[cfg].bn); };
     const int kbytes = d.ic * d.fh * d.fw;
     if (p.pin == 4 && p.pout == 4 && d.fh == 1 && d.fw == 1 && d.pad_h == 0 && d.pad_w == 0) {

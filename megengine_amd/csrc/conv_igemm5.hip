@@ -45,7 +45,7 @@ struct KsArgs {
     int src_sn, src_scb, dst_sn, dst_scb, z_sn;
     int flt_rstride, flt_kstride;
     int tiles_m, tiles_n, by_m;
-    int log_pout, has_bias;
+    int log_pout, has_bias, dst_s32;
     FastDiv div_ohw, div_ow, div_t, div_fw;
     EpiParams epi;
 };
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
     const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.z_bytes);
     const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
     const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes);
-    int d_off = SENT, at_red = 0;
+    int d_off = SENT, z_off = SENT, at_red = 0;
     v4i bv = {0, 0, 0, 0};
     uint32_t zw = 0;
     auto fetch = [&](int u) __attribute__((always_inline)) {
@@ -223,9 +223,10 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
         const uint32_t n = fdiv(mm, a.div_ohw), rem = mm - n * a.OHW;
         const int at = (oc4 >> a.log_pout) * a.dst_scb + ((int)rem << a.log_pout) + (oc4 & ((1 << a.log_pout) - 1));
         d_off = ok ? (int)n * a.dst_sn + at : SENT;
+        z_off = ok ? (int)n * a.z_sn + at : SENT;
         bv = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, oc4 * 4, 0, 0);
         zw = 0;
-        if (a.epi.has_z) zw = __builtin_amdgcn_raw_buffer_load_b32(rs_z, ok ? (int)n * a.z_sn + at : SENT, 0, 0);
+        if (a.epi.has_z && !a.dst_s32) zw = __builtin_amdgcn_raw_buffer_load_b32(rs_z, z_off, 0, 0);
     };
 
     if (k0 < k1) {  // (waves beyond the number of steps have nothing to add)
@@ -264,8 +265,19 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
         v4i s = bv;
 #pragma unroll 4
         for (int w = 0; w < W; ++w) s += red[w * WP + at_red];
-        const uint32_t o = requant4(s[0], s[1], s[2], s[3], zw, a.epi);
-        __builtin_amdgcn_raw_buffer_store_b32(o, rs_dst, d_off, 0, 0);
+        if (a.dst_s32) {
+            // four elements of an int32 dst: element offset d_off, a residual of the same type and its own batch stride
+            if (a.epi.has_z || a.epi.nonline != NL_IDENTITY) {
+                v4i zv = {0, 0, 0, 0};
+                if (a.epi.has_z) zv = __builtin_amdgcn_raw_buffer_load_b128(rs_z, z_off != SENT ? z_off * 4 : SENT, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[r] = requant_s32_exact(s[r], a.epi.has_z != 0, zv[r], a.epi);
+            }
+            __builtin_amdgcn_raw_buffer_store_b128(s, rs_dst, d_off != SENT ? d_off * 4 : SENT, 0, 0);
+        } else {
+            const uint32_t o = requant4(s[0], s[1], s[2], s[3], zw, a.epi);
+            __builtin_amdgcn_raw_buffer_store_b32(o, rs_dst, d_off, 0, 0);
+        }
     }
 }
 
@@ -334,7 +346,9 @@ int igemm5_pick(const IgemmArgs& a, int pin, int pout) {
 }
 
 bool igemm5_can_run(const IgemmArgs& a, int pin, int pout, int cfg) {
-    if (cfg < 0 || cfg >= kKsCount || kKs[cfg].pin != pin || a.groups != 1 || a.general || (pout != 4 && pout != 32)) return false;
+    if (cfg < 0 || cfg >= kKsCount || kKs[cfg].pin != pin || a.groups != 1 || (pout != 4 && pout != 32)) return false;
+    // of the general epilogue only the int32 result, below 2 GiB
+    if (a.general && !(a.dst_s32 && !a.bias_full && a.dst_bytes < (1u << 29) && a.z_bytes < (1u << 29))) return false;
     const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0;
     return ks_lds(a, kKs[cfg], pw) <= 160 * 1024;
 }
@@ -355,6 +369,11 @@ int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg
     k.by_m = k.tiles_m >= 8;
     k.log_pout = pout == 32 ? 5 : 2;
     k.has_bias = a.has_bias;
+    k.dst_s32 = a.dst_s32;
+    if (a.dst_s32) {  // bytes of int32 tensors
+        k.dst_bytes = a.dst_bytes * 4;
+        k.z_bytes = a.z_bytes * 4;
+    }
     k.div_ohw = a.div_ohw; k.div_ow = a.div_ow; k.div_t = a.div_t; k.div_fw = a.div_fw;
     k.epi = a.epi;
     const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0;

@@ -248,6 +248,30 @@ template <int POUT, int MT, int NT>
 __device__ __forceinline__ void igemm_epilogue_general(const IgemmArgs& a, v16i (&acc)[MT][NT], int oc_w, int pix_w, int l32,
                                                        int lh, int oc_end) {
     const bool hz = a.epi.has_z != 0;
+    if (POUT == 32 && a.dst_s32 && !hz && a.epi.nonline == NL_IDENTITY && !a.bias_full && a.dst_bytes < (1u << 29)) {
+        // the bare sums (a graph that keeps its activation apart): stores through a descriptor as in the fast epilogue,
+        // with no 64-bit address arithmetic and no branch around each of them
+        const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes * 4);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int m = pix_w + j * 32 + l32;
+            const bool pok = m < a.M;
+            const uint32_t mm = pok ? m : 0;
+            const uint32_t n = fdiv(mm, a.div_ohw), rem = mm - n * a.OHW;
+            const int at = pok ? ((int)n * a.dst_sn + (int)rem * 32) * 4 + lh * 16 : SENT;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const int ocb = oc_w + i * 32;
+                if (ocb >= oc_end) continue;  // wave-uniform; whole blocks of 32 channels
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const v4i o = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                    __builtin_amdgcn_raw_buffer_store_b128(o, rs_dst, at, (ocb >> 5) * a.dst_scb * 4 + q * 32, 0);
+                }
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         const int m = pix_w + j * 32 + l32;
