@@ -20,6 +20,10 @@ enum AlgoId {
     ALGO_COUNT = 5
 };
 
+// Packed input, planar output, the inner problems of a plain-NCHW convolution (conv_nchw.hip): no formats of the interface
+// (whose NCHW4_NCHW promises its two tiles and no others)
+constexpr uint32_t FMT_INNER_NCHW32_NCHW = 0x100, FMT_INNER_NCHW4_NCHW = 0x101;
+
 // Canonical problem description used by every launcher (derived from mi355_conv_desc)
 struct ConvProblem {
     mi355_conv_desc d;

@@ -540,6 +540,8 @@ static ConvProblem igemm_group_view(const ConvProblem& p) {
     return q;  // batch strides stay those of the whole tensors
 }
 
+static bool inner_planar(const ConvProblem& p) { return p.d.format == FMT_INNER_NCHW32_NCHW || p.d.format == FMT_INNER_NCHW4_NCHW; }
+
 bool igemm_usable(const ConvProblem& p) {
     const mi355_conv_desc& d = p.d;
     if (p.dw4) return false;
@@ -548,8 +550,8 @@ bool igemm_usable(const ConvProblem& p) {
     if (d.group != 1 && !(p.pin == 32 && p.icpg % 32 == 0 && p.ocpg % 32 == 0) && !igemm_group_by_launch(p)) return false;
     // planar destination (NCHW4_NCHW: QuantizedS8 or Float32 dst, any bias shape, any scales): dense, on two of the
     // register-staged tiles, whose planar epilogue covers all of it
-    const bool planar = d.format == MI355_FMT_NCHW4_NCHW;
-    if (planar && ((d.group != 1 && !igemm_group_by_launch(p)) || d.dst_dtype == MI355_DT_QS32)) return false;
+    const bool planar = p.pout == 1 && (d.format == MI355_FMT_NCHW4_NCHW || inner_planar(p));
+    if (planar && ((d.group != 1 && !igemm_group_by_launch(p) && p.pin == 4) || d.dst_dtype == MI355_DT_QS32)) return false;
     if (d.format != MI355_FMT_NCHW4 && d.format != MI355_FMT_NCHW32 && d.format != MI355_FMT_NCHW4_NCHW32 &&
         d.format != MI355_FMT_NCHW32_NCHW4 && !planar)
         return false;
@@ -594,8 +596,16 @@ static bool igemm_plain_s32(const ConvProblem& p) {
 static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_preprocess) {
     const mi355_conv_desc& d = p.d;
     if (p.pout == 1) {
-        // planar destination: 128 x 128 tiles once they fill the device, else 64 x 64
+        // planar destination: few pixels as everywhere, else 128 x 128 tiles once they fill the device, else smaller ones
         const int64_t t128 = (int64_t)((d.oc + 127) / 128) * (((int64_t)d.n * p.oh * p.ow + 127) / 128);
+        if (d.group == 1 && inner_planar(p)) {
+            IgemmArgs a;
+            igemm_fill_args(p, a);
+            const int ks = igemm5_pick(a, p.pin, p.pout);
+            if (ks >= 0) return igemm_first_ks_cfg() + ks;
+        }
+        if (p.pin == 32)
+            return igemm_first_v2_cfg() + (p.ocpg <= 64 || 2 * t128 < 3 * (int64_t)(cu_count > 0 ? cu_count : 256) ? 3 : 0);
         return d.oc > 64 && t128 >= (cu_count > 0 ? cu_count : 256) ? 0 : 3;
     }
     if (d.group == 1 && (!igemm_needs_general(p) || igemm_plain_s32(p)) && !igemm_takes_table(p)) {
@@ -797,7 +807,7 @@ static void igemm_fill_args(const ConvProblem& p, IgemmArgs& a) {
     a.groups = d.group;
     a.ocpg = p.ocpg;
     a.src_sg = (p.icpg / p.pin) * a.src_scb;
-    a.general = igemm_needs_general(p) && p.pout != 1 ? 1 : 0;
+    a.general = igemm_needs_general(p) && p.pout != 1 ? 1 : 0;  // (the planar epilogue covers everything itself)
     a.dst_f32 = d.dst_dtype == MI355_DT_F32;
     if (a.dst_f32) a.has_bias = 0;  // a Float32 bias is added by the planar epilogue, not to the int32 accumulators
     a.dst_s32 = d.dst_dtype == MI355_DT_QS32;
@@ -817,8 +827,15 @@ static int resolve_filled(const ConvProblem& p, const IgemmArgs& a, int cfg) {
     if (cfg < 0 || cfg >= igemm_num_cfgs()) return -1;
     const mi355_conv_desc& d = p.d;
     if (a.M == 0 || a.OC == 0) return cfg;  // nothing is launched
-    if (p.pout == 1) return cfg == 3 ? 3 : 0;  // planar destination: two register-staged tiles
     const int first_v2 = igemm_first_v2_cfg();
+    if (p.pout == 1) {
+        // planar destination: the split-reduction tiles, and two register-staged (4-packed inputs) or two
+        // second-generation tiles (32-packed ones)
+        if (cfg >= igemm_first_ks_cfg() && cfg < igemm_grp4_cfg() && inner_planar(p) && d.group == 1 && igemm5_can_run(a, p.pin, 1, cfg - igemm_first_ks_cfg()))
+            return cfg;
+        if (p.pin == 32) return cfg == first_v2 ? cfg : first_v2 + 3;
+        return cfg == 3 ? 3 : 0;
+    }
     // group convolutions and the general epilogue exist on the second-generation tiles only
     if ((d.group != 1 || a.general) && cfg < first_v2) cfg = first_v2 + (p.ocpg <= 64 ? 3 : 0);
     if (cfg == igemm_grp4_cfg()) cfg = first_v2;  // (a problem it can run never gets here)
@@ -917,6 +934,8 @@ int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_coun
     }
     if (p.pout == 1) {
         if (p.d.bias_mode == MI355_BIAS_NONE) a.bias = nullptr;  // the planar epilogue tests the pointer
+        if (cfg >= igemm_first_ks_cfg()) return launch_igemm5(st, a, p.pin, 1, cfg - igemm_first_ks_cfg());
+        if (p.pin == 32) return launch_igemm2(st, a, 1, cfg - igemm_first_v2_cfg(), cu_count);
         return launch_planar(st, a, cfg, cu_count);
     }
     const int first_v2 = igemm_first_v2_cfg();

@@ -658,7 +658,9 @@ struct Igemm2 {
                 read_z(zr, zbuf + zslot * ZSLOT, lane);
                 if (zslots == 2) zslot ^= 1;
             }
-            if constexpr (GEN)
+            if constexpr (POUT == 1)
+                igemm_epilogue_planar<MT, NT>(a, acc, cur.oc0 + wm * WTM, cur.pix0 + wn * WTN, l32, lh, cur.oc_end);
+            else if constexpr (GEN)
                 igemm_epilogue_general<POUT, MT, NT>(a, acc, cur.oc0 + wm * WTM, cur.pix0 + wn * WTN, l32, lh, cur.oc_end);
             else if constexpr (KS > 1)  // the blocks this wave finishes
                 igemm_run_epilogue<POUT, MT, NT, false>(a, acc, cur.oc0 + wm * WTM, cur.pix0 + wn * WTN, l32, lh, nullptr, cur.oc_end, KS, kg);
@@ -738,7 +740,7 @@ int launch_k(hipStream_t st, IgemmArgs& a, int cu_count) {
     // tile to hide it behind (one slot, and room for a second workgroup per CU)
     const int fixed = K::RING_BYTES + tab_entries * 8;
     a.zslots = 0;
-    if (a.epi.has_z && !a.general && !K::ZD) {
+    if (a.epi.has_z && !a.general && !K::ZD && POUT != 1) {
         a.zslots = a.nstages <= 2 ? 2 : 1;
         if (fixed + a.zslots * K::ZSLOT > kLdsPerCu) a.zslots = 1;
     }
@@ -834,6 +836,20 @@ int launch_fmt(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
     }
 }
 
+// planar destination: two tiles, with the planar epilogue in the place of the general one
+template <>
+int launch_fmt<1>(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
+    switch (cfg) {
+        case 0: return launch_gen<1, 128, 128, 2, 2, 2, 4, 2, true>(st, a, cu);
+        case 3: return launch_gen<1, 64, 128, 2, 2, 4, 3, 2, true>(st, a, cu);
+        default: return kNoGen;
+    }
+}
+
+int launch_pout(hipStream_t st, IgemmArgs& a, int pout, int cfg, int cu) {
+    return pout == 32 ? launch_fmt<32>(st, a, cfg, cu) : pout == 4 ? launch_fmt<4>(st, a, cfg, cu) : launch_fmt<1>(st, a, cfg, cu);
+}
+
 }  // namespace
 
 int igemm2_num_cfgs() { return kNumCfg2; }
@@ -874,14 +890,14 @@ int launch_igemm2_preprocess(hipStream_t st, const int8_t* flt, int8_t* out, int
 // A tile that cannot run the problem (no instantiation with the general epilogue, or ring + residual slot beyond the
 // LDS of a CU) is an error here: igemm_resolve_cfg (conv_igemm.hip) names the tile that runs before anything is launched.
 int launch_igemm2(hipStream_t st, IgemmArgs& a, int pout, int cfg, int cu_count) {
-    const int rc = pout == 32 ? launch_fmt<32>(st, a, cfg, cu_count) : launch_fmt<4>(st, a, cfg, cu_count);
+    const int rc = launch_pout(st, a, pout, cfg, cu_count);
     return rc == kNoFit || rc == kNoGen ? (int)hipErrorInvalidConfiguration : rc;
 }
 
 bool igemm2_can_run(const IgemmArgs& a, int pout, int cfg) {
     IgemmArgs t = a;
     t.dry_run = 1;
-    return (pout == 32 ? launch_fmt<32>(nullptr, t, cfg, 256) : launch_fmt<4>(nullptr, t, cfg, 256)) == 0;
+    return launch_pout(nullptr, t, pout, cfg, 256) == 0;
 }
 
 }  // namespace mi355

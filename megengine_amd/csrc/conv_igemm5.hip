@@ -209,7 +209,7 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
     const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.z_bytes);
     const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
     const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes);
-    int d_off = SENT, z_off = SENT, at_red = 0;
+    int d_off = SENT, z_off = SENT, at_red = 0, left = 0;
     v4i bv = {0, 0, 0, 0};
     uint32_t zw = 0;
     auto fetch = [&](int u) __attribute__((always_inline)) {
@@ -226,7 +226,14 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
         z_off = ok ? (int)n * a.z_sn + at : SENT;
         bv = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, oc4 * 4, 0, 0);
         zw = 0;
-        if (a.epi.has_z && !a.dst_s32) zw = __builtin_amdgcn_raw_buffer_load_b32(rs_z, z_off, 0, 0);
+        if (a.log_pout == 0) {
+            // planar: four channels of a pixel lie OHW apart
+            left = ok ? a.OC - oc4 : 0;
+            if (a.epi.has_z)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (r < left) zw |= (uint32_t)(uint8_t)a.z[z_off + r * a.OHW] << (8 * r);
+        } else if (a.epi.has_z && !a.dst_s32) zw = __builtin_amdgcn_raw_buffer_load_b32(rs_z, z_off, 0, 0);
     };
 
     if (k0 < k1) {  // (waves beyond the number of steps have nothing to add)
@@ -276,7 +283,13 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
             __builtin_amdgcn_raw_buffer_store_b128(s, rs_dst, d_off != SENT ? d_off * 4 : SENT, 0, 0);
         } else {
             const uint32_t o = requant4(s[0], s[1], s[2], s[3], zw, a.epi);
-            __builtin_amdgcn_raw_buffer_store_b32(o, rs_dst, d_off, 0, 0);
+            if (a.log_pout == 0) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (r < left) a.dst[d_off + r * a.OHW] = (int8_t)(o >> (8 * r));
+            } else {
+                __builtin_amdgcn_raw_buffer_store_b32(o, rs_dst, d_off, 0, 0);
+            }
         }
     }
 }
@@ -346,7 +359,8 @@ int igemm5_pick(const IgemmArgs& a, int pin, int pout) {
 }
 
 bool igemm5_can_run(const IgemmArgs& a, int pin, int pout, int cfg) {
-    if (cfg < 0 || cfg >= kKsCount || kKs[cfg].pin != pin || a.groups != 1 || (pout != 4 && pout != 32)) return false;
+    if (cfg < 0 || cfg >= kKsCount || kKs[cfg].pin != pin || a.groups != 1 || (pout != 1 && pout != 4 && pout != 32)) return false;
+    if (pout == 1 && (a.dst_f32 || a.bias_full || !a.epi.fast)) return false;  // planar: the fast int8 forms
     // of the general epilogue only the int32 result, below 2 GiB
     if (a.general && !(a.dst_s32 && !a.bias_full && a.dst_bytes < (1u << 29) && a.z_bytes < (1u << 29))) return false;
     const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0;
@@ -367,7 +381,7 @@ int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg
     k.tiles_m = (a.OC + c.s * c.mt - 1) / (c.s * c.mt);
     k.tiles_n = (a.M + c.s * c.nt - 1) / (c.s * c.nt);
     k.by_m = k.tiles_m >= 8;
-    k.log_pout = pout == 32 ? 5 : 2;
+    k.log_pout = pout == 32 ? 5 : pout == 4 ? 2 : 0;
     k.has_bias = a.has_bias;
     k.dst_s32 = a.dst_s32;
     if (a.dst_s32) {  // bytes of int32 tensors

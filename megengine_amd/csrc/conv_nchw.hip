@@ -2,42 +2,33 @@
 //
 // Format::NCHW is what the reference's own x86 int8 algorithms accept (dnn/src/x86/conv_bias/int8/
 // algo_usable_preferred.cpp:19-37,88-108; shape rule dnn/src/common/convolution.cpp:774-801), and the CUDA backend runs
-// it the same way this file does: relayout into the packed format of its tensor-core kernels, convolve, relayout back
-// (dnn/src/cuda/conv_bias/conv_nchwqs8.cpp).  All intermediates live in the caller's workspace -- the first algorithm
-// of this backend that reports a non-zero get_workspace_in_bytes (dnn/include/megdnn/oprs/nn.h:419-422):
+// it by way of the packed format of its tensor-core kernels (dnn/src/cuda/conv_bias/conv_nchwqs8.cpp).  Here two launches
+// do: one brings src and filter into the packed layout, in the caller's workspace -- the first algorithm of this backend
+// that reports a non-zero get_workspace_in_bytes (dnn/include/megdnn/oprs/nn.h:419-422) --
 //
-//     [src as NCHW32, channels padded to 32][filter as (OC32, IC32/32, FH, FW, 32)][dst as NCHW32][z as NCHW32][bias, OC32]
+//     [src packed by 4 or 32 channels][filter as (OC, IC/pack, FH, FW, pack)]
 //
-// Padded input channels are zero bytes (they add nothing to a sum); padded output channels have zero filter rows and
-// zero bias and are cropped by the relayout back.  The arithmetic is that of the NCHW32 kernel, which is bit-exact to
-// the reference's naive path; a permutation of the operands changes no integer sum.
+// and the implicit GEMM reads those, and bias, residual and destination as they are: its planar epilogue knows NCHW.
+// Padded input channels are zero bytes (they add nothing to a sum).  The arithmetic is that of the packed kernels, which
+// is bit-exact to the reference's naive path; a permutation of the operands changes no integer sum.
+// 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual (3.3 Gop): 48.8 us as four conversions, two fills and a
+// convolution, 17 us as two launches.
 #include <string.h>
 
 #include "igemm_shared.h"
+#include "relayout_parts.h"
 
 namespace mi355 {
 namespace {
 
 constexpr size_t kAlign = 256;
 size_t up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }  // the vector paths of the relayouts
 
 struct NchwLayout {
-    uint32_t ic32, oc32;                              // channel counts padded to whole blocks of 32
-    size_t off_src, off_flt, off_dst, off_z, off_bias, total;
-    ConvProblem inner;                                // the NCHW32 problem the MFMA kernel runs
+    int pack;                       // channel pack of the inner problem
+    size_t off_flt, total;          // (src stands at the front)
+    ConvProblem inner;              // packed src and filter, planar bias, z and dst
 };
-
-// 16 bytes per thread
-__global__ __launch_bounds__(256) void zero_fill_kernel(v4i* dst, uint64_t vecs) {
-    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < vecs) dst[i] = v4i{0, 0, 0, 0};
-}
-
-__global__ __launch_bounds__(256) void bias_pad_kernel(const int32_t* src, int32_t* dst, uint32_t oc, uint32_t oc32) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < oc32) dst[i] = i < oc ? src[i] : 0;
-}
 
 bool make_layout(const ConvProblem& p, NchwLayout* L) {
     const mi355_conv_desc& d = p.d;
@@ -45,57 +36,77 @@ bool make_layout(const ConvProblem& p, NchwLayout* L) {
     if (d.dst_dtype != MI355_DT_QS8 || d.bias_mode == MI355_BIAS_FULL || !p.epi.fast) return false;
     if (d.mode != MI355_MODE_CROSS_CORRELATION || d.dilate_h != 1 || d.dilate_w != 1) return false;
     // groups must be whole channel blocks on both sides: then the packed tensors of the groups are contiguous pieces of
-    // the packed tensors, as the NCHW32 group kernel expects them
+    // the packed tensors, as the 32-packed group kernel expects them
     if (d.group != 1 && (p.icpg % 32 || p.ocpg % 32)) return false;
-    // dense batches only (a strided view would need strided relayouts)
+    // dense batches only (a strided view would need strided conversions)
     const int64_t src_img = (int64_t)d.ic * d.ih * d.iw, dst_img = (int64_t)d.oc * p.oh * p.ow;
     if (p.src_sn != src_img || p.dst_sn != dst_img || (d.has_z && p.z_sn != dst_img)) return false;
     if (d.n > 65535) return false;
-    L->ic32 = (d.ic + 31) / 32 * 32;
-    L->oc32 = (d.oc + 31) / 32 * 32;
-    const size_t src_b = (size_t)d.n * L->ic32 * d.ih * d.iw, flt_b = (size_t)L->oc32 * (L->ic32 / d.group) * d.fh * d.fw;
-    const size_t dst_b = (size_t)d.n * L->oc32 * p.oh * p.ow;
-    size_t o = 0;
-    L->off_src = o; o += up(src_b);
-    L->off_flt = o; o += up(flt_b);
-    L->off_dst = o; o += up(dst_b);
-    L->off_z = o; o += d.has_z ? up(dst_b) : 0;
-    L->off_bias = o; o += d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL && L->oc32 != d.oc ? up((size_t)L->oc32 * 4) : 0;
-    L->total = o;
+    // The size reported for the workspace is what callers have planned memory with: that of src, filter, dst, z and bias all
+    // packed by 32.  The first two are what is used.
+    const uint32_t ic32 = (d.ic + 31) / 32 * 32, oc32 = (d.oc + 31) / 32 * 32;
+    const size_t src32 = (size_t)d.n * ic32 * d.ih * d.iw, dst32 = (size_t)d.n * oc32 * p.oh * p.ow;
+    L->total = up(src32) + up((size_t)oc32 * (ic32 / d.group) * d.fh * d.fw) + up(dst32) + (d.has_z ? up(dst32) : 0) +
+               (d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL && oc32 != d.oc ? up((size_t)oc32 * 4) : 0);
+    // up to 16 channels a block of 32 would be half and more padding
+    L->pack = d.ic <= 16 ? 4 : 32;
+    const uint32_t icp = (d.ic + L->pack - 1) / L->pack * L->pack;
+    if ((uint64_t)d.n * icp * d.ih * d.iw >= (1ull << 31) || (uint64_t)d.oc * (icp / d.group) * d.fh * d.fw >= (1ull << 31)) return false;
+    L->off_flt = up((size_t)d.n * icp * d.ih * d.iw);
     ConvProblem& q = L->inner;
     q = p;
-    q.d.format = MI355_FMT_NCHW32;
-    q.d.ic = L->ic32;
-    q.d.oc = L->oc32;
+    q.d.format = L->pack == 4 ? FMT_INNER_NCHW4_NCHW : FMT_INNER_NCHW32_NCHW;
+    q.d.ic = icp;
     q.d.src_stride_n = q.d.dst_stride_n = q.d.z_stride_n = 0;
-    q.icpg = L->ic32 / d.group;
-    q.ocpg = L->oc32 / d.group;
-    q.pin = q.pout = 32;
+    q.icpg = icp / d.group;
+    q.pin = L->pack;
+    q.pout = 1;
     q.dw4 = false;
-    q.src_sn = (int64_t)L->ic32 * d.ih * d.iw;
-    q.dst_sn = q.z_sn = (int64_t)L->oc32 * p.oh * p.ow;
+    q.src_sn = (int64_t)icp * d.ih * d.iw;
     return igemm_usable(q);
 }
 
-mi355_relayout_desc rl_desc(uint32_t mode, uint32_t ndim, uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3, uint32_t s4,
-                            uint32_t oc) {
-    mi355_relayout_desc r;
-    memset(&r, 0, sizeof(r));
-    r.mode = mode;
-    r.ndim = ndim;
-    r.shape[0] = s0; r.shape[1] = s1; r.shape[2] = s2; r.shape[3] = s3; r.shape[4] = s4;
-    r.group = 1;
-    r.oc = oc;
-    r.elem_bytes = 1;
-    r.scale_src = r.scale_dst = 1.f;
-    return r;
-}
+// src and filter into their packed layouts, one launch: the first blocks convert src -- 32 channels x 128 pixels through
+// LDS, or quads of a pixel where the planes are smaller than that -- the others the filter, an NCHW tensor of oc images.
+constexpr int NP_TP = 128, NP_ROW = NP_TP + 4;  // pixels per tile; padded LDS row (33 dwords: channel rows on other banks)
+struct PrepArgs {
+    const int8_t* src;
+    int8_t* src_p;
+    const int8_t* flt;
+    int8_t* flt_p;
+    uint32_t C, CB, HW, ptiles;    // tiled src
+    uint32_t src_blocks, tiled;
+    FastDiv div_ptiles, div_cb;
+    SmallPlanes src_small, flt_small;
+};
 
-// (n, c, h, w) -> (n, ceil(c / 32), h, w, 32), zero padding past c
-int to_nchw32(hipStream_t st, const void* src, void* dst, uint32_t n, uint32_t c, uint32_t h, uint32_t w) {
-    const mi355_relayout_desc r = rl_desc(MI355_RL_NCHW_NCHW32, 4, n, c, h, w, 0, 0);
-    const uint32_t oshape[7] = {n, (c + 31) / 32, h, w, 32, 0, 0};
-    return launch_relayout(st, r, oshape, 5, src, dst, aligned16(src) && aligned16(dst));
+__global__ __launch_bounds__(256) void nchw_prep_kernel(PrepArgs a) {
+    __shared__ __attribute__((aligned(16))) int8_t sm[32 * NP_ROW];
+    const uint32_t t = threadIdx.x;
+    if (blockIdx.x >= a.src_blocks)
+        return small_planes_quad(a.flt, reinterpret_cast<uint32_t*>(a.flt_p), a.flt_small, (blockIdx.x - a.src_blocks) * 256 + t);
+    if (!a.tiled) return small_planes_quad(a.src, reinterpret_cast<uint32_t*>(a.src_p), a.src_small, blockIdx.x * 256 + t);
+    const uint32_t b = fdiv(blockIdx.x, a.div_ptiles), p0 = (blockIdx.x - b * a.ptiles) * NP_TP;  // b = image * CB + block
+    const uint32_t n = fdiv(b, a.div_cb), cb = b - n * a.CB;
+    {
+        const uint32_t row = t >> 3, v = t & 7, px = p0 + v * 16, c = cb * 32 + row;
+        u32x4 x = {0, 0, 0, 0};
+        if (px < a.HW && c < a.C) x = load16_tail(a.src + ((int64_t)n * a.C + c) * a.HW + px, a.HW - px);
+        uint32_t* d = reinterpret_cast<uint32_t*>(sm + row * NP_ROW + v * 16);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d[k] = x[k];
+    }
+    __syncthreads();
+    // 4 channels x 4 pixels per thread; eight neighbouring lanes are the 32 channels of a pixel
+    const uint32_t cq = t & 7, pq = t >> 3;
+    uint32_t r[4], o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r[k] = *reinterpret_cast<const uint32_t*>(sm + (cq * 4 + k) * NP_ROW + pq * 4);
+    transpose4x4(r[0], r[1], r[2], r[3], o[0], o[1], o[2], o[3]);
+    uint32_t* d = reinterpret_cast<uint32_t*>(a.src_p) + ((int64_t)b * a.HW + p0 + pq * 4) * 8 + cq;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        if (p0 + pq * 4 + k < a.HW) d[k * 8] = o[k];
 }
 
 }  // namespace
@@ -117,41 +128,21 @@ int launch_conv_nchw_mfma(hipStream_t st, const ConvProblem& p, int cu_count, co
     const mi355_conv_desc& d = p.d;
     if ((uint64_t)d.n * d.oc * p.oh * p.ow == 0) return 0;
     int8_t* ws = reinterpret_cast<int8_t*>(workspace);
-    int8_t* src32 = ws + L.off_src;
-    int8_t* flt32 = ws + L.off_flt;
-    int8_t* dst32 = ws + L.off_dst;
-    int8_t* z32 = d.has_z ? ws + L.off_z : nullptr;
-    int rc = to_nchw32(st, src, src32, d.n, d.ic, d.ih, d.iw);
+    const uint32_t HW = d.ih * d.iw;
+    PrepArgs a;
+    a.src = src; a.src_p = ws; a.flt = flt; a.flt_p = ws + L.off_flt;
+    a.C = d.ic; a.CB = (d.ic + 31) / 32; a.HW = HW;
+    a.ptiles = (HW + NP_TP - 1) / NP_TP;
+    a.div_ptiles = make_fastdiv(a.ptiles);
+    a.div_cb = make_fastdiv(a.CB);
+    a.tiled = L.pack == 32 && HW >= NP_TP / 2;
+    a.src_small = make_small_planes(d.n, d.ic, HW, L.pack);
+    a.flt_small = make_small_planes(d.oc, p.icpg, d.fh * d.fw, L.pack);
+    a.src_blocks = a.tiled ? d.n * a.CB * a.ptiles : (a.src_small.items + 255) / 256;
+    const uint32_t blocks = a.src_blocks + (a.flt_small.items + 255) / 256;
+    const int rc = launch_kernel(nchw_prep_kernel, dim3(blocks), dim3(256), 0, st, a);
     if (rc) return rc;
-    // the filter (oc, icpg, fh, fw) is an "NCHW tensor" of oc images; with groups icpg is a multiple of 32 already
-    const uint32_t icpg32 = L.ic32 / d.group;
-    rc = to_nchw32(st, flt, flt32, d.oc, p.icpg, d.fh, d.fw);
-    if (rc) return rc;
-    if (L.oc32 != d.oc) {
-        // filter rows of the padded output channels (dense convolutions only: groups are whole blocks)
-        const size_t row = (size_t)icpg32 * d.fh * d.fw;  // a multiple of 32 bytes
-        const uint64_t vecs = (uint64_t)(L.oc32 - d.oc) * row / 16;
-        rc = launch_kernel(zero_fill_kernel, dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, st,
-                           reinterpret_cast<v4i*>(flt32 + (size_t)d.oc * row), vecs);
-        if (rc) return rc;
-    }
-    const int32_t* bias32 = bias;
-    if (d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL && L.oc32 != d.oc) {
-        int32_t* b = reinterpret_cast<int32_t*>(ws + L.off_bias);
-        rc = launch_kernel(bias_pad_kernel, dim3((L.oc32 + 255) / 256), dim3(256), 0, st, bias, b, d.oc, L.oc32);
-        if (rc) return rc;
-        bias32 = b;
-    }
-    if (d.has_z) {
-        rc = to_nchw32(st, z, z32, d.n, d.oc, p.oh, p.ow);
-        if (rc) return rc;
-    }
-    const int cfg = igemm_pick_cfg(L.inner, cu_count, false);
-    rc = launch_conv_igemm(st, L.inner, cfg, cu_count, src32, flt32, bias32, z32, dst32, false);
-    if (rc) return rc;
-    const mi355_relayout_desc back = rl_desc(MI355_RL_NCHW32_NCHW, 5, d.n, L.oc32 / 32, p.oh, p.ow, 32, d.oc);
-    const uint32_t oshape[7] = {d.n, d.oc, p.oh, p.ow, 0, 0, 0};
-    return launch_relayout(st, back, oshape, 4, dst32, dst, aligned16(dst32) && aligned16(dst));
+    return launch_conv_igemm(st, L.inner, igemm_pick_cfg(L.inner, cu_count, false), cu_count, a.src_p, a.flt_p, bias, z, dst, false);
 }
 
 }  // namespace mi355

@@ -321,9 +321,21 @@ __device__ __forceinline__ void igemm_epilogue_general(const IgemmArgs& a, v16i 
 // chain in whichever form the scales allow; Float32 dst: the exact sum dequantised once, then bias, z and activation in
 // float (forward_bias and handle_z_inp_and_activation_naive on float tensors, dnn/src/naive/conv_bias/opr_impl.cpp:21-98).
 enum { PLANAR_F32 = 0, PLANAR_S8_EXACT = 1, PLANAR_S8_FAST = 2 };
+// Four pixels at a time for the fast int8 forms: a dword holds four channels of a lane's pixel; two exchanges with the
+// neighbouring lanes (DPP, no LDS) turn the dwords of four lanes into four pixels of one channel each, so that lane j stores
+// (and loads the residual of) four consecutive pixels of channel j with one access instead of four.  A wave that holds a
+// group of four pixels across the end of an image, or of the batch, writes element by element.
+__device__ __forceinline__ uint32_t quad_transpose(uint32_t x, int lane) {
+    const uint32_t n1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xf, 0xf, true);  // lane ^ 1
+    x = __builtin_amdgcn_perm(n1, x, lane & 1 ? 0x03070105u : 0x06020400u);
+    const uint32_t n2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xf, 0xf, true);  // lane ^ 2
+    return __builtin_amdgcn_perm(n2, x, lane & 2 ? 0x03020706u : 0x05040100u);
+}
+typedef uint32_t u32_any __attribute__((aligned(1)));
+
 template <int MT, int NT, int KIND, int NL, bool HZ>
 __device__ __forceinline__ void igemm_epilogue_planar_as(const IgemmArgs& a, v16i (&acc)[MT][NT], int oc_w, int pix_w, int l32,
-                                                         int lh) {
+                                                         int lh, int oc_end) {
     const bool hz = KIND == PLANAR_S8_FAST ? HZ : a.epi.has_z != 0;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
@@ -331,6 +343,35 @@ __device__ __forceinline__ void igemm_epilogue_planar_as(const IgemmArgs& a, v16
         const bool pok = m < a.M;
         const uint32_t mm = pok ? m : 0;
         const uint32_t n = fdiv(mm, a.div_ohw), rem = mm - n * a.OHW;
+        if (KIND == PLANAR_S8_FAST && !a.bias_full) {
+            const int m4 = m & ~3, lane4 = l32 & 3;
+            const uint32_t mm4 = m4 < a.M ? m4 : 0;
+            const uint32_t n4 = fdiv(mm4, a.div_ohw), rem4 = mm4 - n4 * a.OHW;
+            const bool whole = m4 >= a.M || (m4 + 3 < a.M && rem4 + 3 < (uint32_t)a.OHW);
+            if (__builtin_amdgcn_ballot_w64(!whole) == 0) {
+                const uint32_t px = rem4 + (uint32_t)(4 * lh + lane4) * (uint32_t)a.OHW;
+                const uint32_t d0 = n4 * (uint32_t)a.dst_sn + px, z0 = n4 * (uint32_t)a.z_sn + px;
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    const v16i& c = acc[i][j];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int oc8 = oc_w + i * 32 + 8 * q;  // wave-uniform
+                        if (oc8 >= oc_end) continue;
+                        const int64_t at = (int64_t)oc8 * a.OHW;
+                        const bool ok = m4 < a.M && oc8 + 4 * lh + lane4 < oc_end;
+                        uint32_t zw = 0;
+                        if (HZ) {
+                            if (ok) zw = *reinterpret_cast<const u32_any*>(a.z + at + z0);
+                            zw = quad_transpose(zw, lane4);
+                        }
+                        const uint32_t o = quad_transpose(requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], zw, a.epi), lane4);
+                        if (ok) *reinterpret_cast<u32_any*>(a.dst + at + d0) = o;
+                    }
+                }
+                continue;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
             const int ocb = oc_w + i * 32;
@@ -338,7 +379,7 @@ __device__ __forceinline__ void igemm_epilogue_planar_as(const IgemmArgs& a, v16
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int oc4 = ocb + 8 * q + 4 * lh;
-                const int left = pok ? a.OC - oc4 : 0;              // channels of this quad that exist (<= 0: none)
+                const int left = pok ? oc_end - oc4 : 0;              // channels of this quad that exist (<= 0: none)
                 const int64_t in_img = (int64_t)oc4 * a.OHW + rem;  // element of channel oc4 inside one image
                 const int64_t full = (int64_t)n * ((int64_t)a.OC * a.OHW) + in_img;
                 if (KIND == PLANAR_F32) {
@@ -386,8 +427,9 @@ __device__ __forceinline__ void igemm_epilogue_planar_as(const IgemmArgs& a, v16
 
 template <int MT, int NT>
 __device__ __forceinline__ void igemm_epilogue_planar(const IgemmArgs& a, v16i (&acc)[MT][NT], int oc_w, int pix_w, int l32,
-                                                      int lh) {
-#define MI355_PLANAR(KIND, NL, HZ) igemm_epilogue_planar_as<MT, NT, KIND, NL, HZ>(a, acc, oc_w, pix_w, l32, lh)
+                                                      int lh, int oc_end = -1) {
+    if (oc_end < 0) oc_end = a.OC;
+#define MI355_PLANAR(KIND, NL, HZ) igemm_epilogue_planar_as<MT, NT, KIND, NL, HZ>(a, acc, oc_w, pix_w, l32, lh, oc_end)
     if (a.dst_f32) {
         MI355_PLANAR(PLANAR_F32, NL_IDENTITY, false);
     } else if (!a.epi.fast) {

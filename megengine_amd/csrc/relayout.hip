@@ -7,7 +7,7 @@
 //   * relayout_generic_kernel: one thread per destination element, any mode / element size.
 //   * byte-transposing kernels for the int8 pure permutations, any channel count and image size;
 //     16-byte vectors, coalesced on both sides (HBM bound).
-#include "common.h"
+#include "relayout_parts.h"
 
 namespace mi355 {
 namespace {
@@ -110,44 +110,6 @@ __global__ __launch_bounds__(256) void relayout_generic_kernel(RelayoutArgs a) {
     }
 }
 
-// ---- 4x4 byte transpose in registers: rows r0..r3 (4 bytes each) -> columns ----
-__device__ __forceinline__ void transpose4x4(uint32_t r0, uint32_t r1, uint32_t r2, uint32_t r3, uint32_t& c0,
-                                             uint32_t& c1, uint32_t& c2, uint32_t& c3) {
-    // t01_lo = r0.b0 r1.b0 r0.b1 r1.b1 ; t01_hi = r0.b2 r1.b2 r0.b3 r1.b3
-    uint32_t t01_lo = __builtin_amdgcn_perm(r1, r0, 0x05010400u);
-    uint32_t t01_hi = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
-    uint32_t t23_lo = __builtin_amdgcn_perm(r3, r2, 0x05010400u);
-    uint32_t t23_hi = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
-    c0 = __builtin_amdgcn_perm(t23_lo, t01_lo, 0x05040100u);
-    c1 = __builtin_amdgcn_perm(t23_lo, t01_lo, 0x07060302u);
-    c2 = __builtin_amdgcn_perm(t23_hi, t01_hi, 0x05040100u);
-    c3 = __builtin_amdgcn_perm(t23_hi, t01_hi, 0x07060302u);
-}
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(1)));  // 16 bytes at any address
-typedef uint32_t u32u __attribute__((aligned(1)));
-
-__device__ __forceinline__ u32x4 load16u(const int8_t* p) { return *reinterpret_cast<const u32x4u*>(p); }
-__device__ __forceinline__ void store16u(int8_t* p, u32x4 v) { *reinterpret_cast<u32x4u*>(p) = v; }
-
-// `have` (>= 1) bytes from p, the rest zero
-__device__ __forceinline__ u32x4 load16_tail(const int8_t* p, uint32_t have) {
-    if (have >= 16) return load16u(p);
-    u32x4 x = {0, 0, 0, 0};
-#pragma unroll
-    for (uint32_t k = 0; k < 16; ++k)
-        if (k < have) x[k / 4] |= (uint32_t)(uint8_t)p[k] << (8 * (k % 4));
-    return x;
-}
-__device__ __forceinline__ void store16_tail(int8_t* p, u32x4 v, uint32_t have) {
-    if (have >= 16) return store16u(p, v);
-#pragma unroll
-    for (uint32_t k = 0; k < 16; ++k)
-        if (k < have) p[k] = (int8_t)(v[k / 4] >> (8 * (k % 4)));
-}
-
 // Planes of a plain tensor start at any byte when the image has an odd size: their 16-byte accesses are unaligned ones
 // (the memory pipe takes them at full rate as long as a wave's run is contiguous).  The last 16 pixels of a plane start
 // at HW - 16, so they overlap the run before them and both write the same bytes: no tail code, every lane does the same.
@@ -227,21 +189,9 @@ __global__ __launch_bounds__(256) void nchw4_nchw32_kernel(const uint32_t* __res
     }
 }
 
-// NCHW -> NCHW4 / NCHW32 for small planes (filters, 7 x 7 images): one thread per 4 output channels of a pixel.
 __global__ __launch_bounds__(256) void nchw_to_packed_small_kernel(const int8_t* __restrict__ src, uint32_t* __restrict__ dst,
-                                                                   uint32_t C, uint32_t CB, uint32_t HW,
-                                                                   uint32_t log_quads, uint32_t items, FastDiv hw, FastDiv cb) {
-    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
-    if (it >= items) return;
-    const uint32_t k = it & ((1u << log_quads) - 1), t = it >> log_quads;  // 1 or 8 quads per pixel
-    const uint32_t b = fdiv(t, hw), px = t - b * HW;
-    const uint32_t n = fdiv(b, cb), c0 = ((b - n * CB) << (log_quads + 2)) + k * 4;
-    const int8_t* s = src + ((int64_t)n * C + c0) * HW + px;
-    uint32_t w = 0;
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q)
-        if (c0 + q < C) w |= (uint32_t)(uint8_t)s[(int64_t)q * HW] << (8 * q);
-    dst[it] = w;
+                                                                   SmallPlanes g) {
+    small_planes_quad(src, dst, g, blockIdx.x * 256 + threadIdx.x);
 }
 
 // NCHW <-> NCHW32 through LDS.  Tile = 32 channels x 512 pixels (16 KiB).  The LDS image keeps
@@ -359,9 +309,9 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
                 // planes of a quarter of the LDS tile and more: below, most of a tile's threads would find no pixel
                 if (oshape[4] == 32 && HW >= RL_TP / 4)
                     return launch_kernel(nchw_to_nchw32_kernel, dim3(CB * ptiles, N), dim3(256), 0, st, s8, d8, C, CB, HW);
-                const uint32_t log_quads = oshape[4] == 32 ? 3 : 0, items = (uint32_t)(total / 4);
-                return launch_kernel(nchw_to_packed_small_kernel, dim3((items + 255) / 256), dim3(256), 0, st, s8,
-                                     reinterpret_cast<uint32_t*>(dst), C, CB, HW, log_quads, items, make_fastdiv(HW), make_fastdiv(CB));
+                const SmallPlanes g = make_small_planes(N, C, HW, oshape[4]);
+                return launch_kernel(nchw_to_packed_small_kernel, dim3((g.items + 255) / 256), dim3(256), 0, st, s8,
+                                     reinterpret_cast<uint32_t*>(dst), g);
             }
             case MI355_RL_NCHW4_NCHW:
                 if (HW >= 16) {
