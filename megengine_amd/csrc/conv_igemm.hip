@@ -483,8 +483,8 @@ int launch_fmt(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
 
 // tile_cfg numbering: register-staged tiles, LDS-direct tiles, second-generation tiles, patch-staged tiles, weight-resident
 // tiles, the 32-packed streaming kernel, the tiles that split the reduction over the waves of a
-// workgroup, the one-launch NCHW4 group kernel
-int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1 + igemm5_num_cfgs() + 1; }
+// workgroup, the one-launch NCHW4 group kernel, the 4-packed patch tiles
+int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1 + igemm5_num_cfgs() + 1 + patch4_num_cfgs(); }
 int igemm_first_v2_cfg() { return kNumCfgs + igemm_dma_num_cfgs(); }
 // planar destination (NCHW4_NCHW): two of the register-staged tiles
 static int launch_planar(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
@@ -500,6 +500,7 @@ static int igemm_first_v4_cfg() { return igemm_first_v3_cfg() + igemm3_num_cfgs(
 static int igemm_pw32s_cfg() { return igemm_first_v4_cfg() + igemm4_num_cfgs(); }
 static int igemm_first_ks_cfg() { return igemm_pw32s_cfg() + 1; }
 static int igemm_grp4_cfg() { return igemm_first_ks_cfg() + igemm5_num_cfgs(); }
+static int igemm_first_p4_cfg() { return igemm_grp4_cfg() + 1; }
 const char* igemm_cfg_name(int cfg) {
     if (cfg >= 0 && cfg < kNumCfgs) return kCfgs[cfg].name;
     if (cfg < igemm_first_v2_cfg()) return igemm_dma_cfg_name(cfg - kNumCfgs);
@@ -508,7 +509,8 @@ const char* igemm_cfg_name(int cfg) {
     if (cfg < igemm_pw32s_cfg()) return igemm4_cfg_name(cfg - igemm_first_v4_cfg());
     if (cfg == igemm_pw32s_cfg()) return "pw32_stream";
     if (cfg < igemm_grp4_cfg()) return igemm5_cfg_name(cfg - igemm_first_ks_cfg());
-    return "grp4_dot4";
+    if (cfg == igemm_grp4_cfg()) return "grp4_dot4";
+    return patch4_cfg_name(cfg - igemm_first_p4_cfg());
 }
 
 static bool igemm_needs_general(const ConvProblem& p) {
@@ -615,6 +617,8 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         igemm_fill_args(p, a);
         const int ks = igemm5_pick(a, p.pin, p.pout);
         if (ks >= 0) return igemm_first_ks_cfg() + ks;
+        const int p4 = patch4_pick(a, p.pin, p.pout);
+        if (p4 >= 0) return igemm_first_p4_cfg() + p4;
     }
     if (p.pin == 32 && p.pout == 32 && d.group == 1 && !igemm_needs_general(p) && d.fh == 3 && d.fw == 3 &&
         d.stride_h == 1 && d.stride_w == 1 && d.pad_h == 1 && d.pad_w == 1 && (d.ic == 32 || d.ic == 64)) {
@@ -743,6 +747,9 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         return kbytes >= 2048 && 4 * tiles(6) >= 3 * cu_count ? D64x128x128w8 : D64x64x128;
     }
     if (OC <= 64) return tiles(1) >= cu_count ? 1 : 3;
+    // 4-packed windowed layers that are not on the patch tiles: the gather of their operands bounds them, which a 128 x 128 tile
+    // does least of (3x3 128 -> 128 at 28 x 28, batch 32, 196 tiles: 13.7 us against 19.2 on 64 x 128)
+    if (d.fh * d.fw > 1 && tiles(0) >= 150 && kbytes >= 512) return 5;
     // 128x128 tiles as soon as they give every CU 1.5 tiles; the deeper k stage pays once the
     // reduction is long enough to amortise its larger prologue
     if (tiles(0) >= 2 * cu_count) return kbytes >= 512 ? 5 : 0;
@@ -838,6 +845,10 @@ static int resolve_filled(const ConvProblem& p, const IgemmArgs& a, int cfg) {
     }
     // group convolutions and the general epilogue exist on the second-generation tiles only
     if ((d.group != 1 || a.general) && cfg < first_v2) cfg = first_v2 + (p.ocpg <= 64 ? 3 : 0);
+    if (cfg >= igemm_first_p4_cfg()) {
+        if (patch4_can_run(a, p.pin, p.pout, cfg - igemm_first_p4_cfg())) return cfg;
+        cfg = first_v2;
+    }
     if (cfg == igemm_grp4_cfg()) cfg = first_v2;  // (a problem it can run never gets here)
     if (cfg >= igemm_first_ks_cfg()) {
         if (igemm5_can_run(a, p.pin, p.pout, cfg - igemm_first_ks_cfg())) return cfg;
@@ -953,6 +964,7 @@ int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_coun
             a.ztab = tab;
         }
     }
+    if (cfg >= igemm_first_p4_cfg()) return launch_patch4(st, a, cfg - igemm_first_p4_cfg());
     if (cfg >= igemm_first_ks_cfg()) return launch_igemm5(st, a, p.pin, p.pout, cfg - igemm_first_ks_cfg());
     if (cfg == igemm_pw32s_cfg()) return launch_pw32s(st, a, cu_count);
     if (cfg >= igemm_first_v4_cfg()) return launch_igemm4(st, a, p.pin, p.pout, cfg - igemm_first_v4_cfg(), cu_count);

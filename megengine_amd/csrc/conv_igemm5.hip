@@ -351,6 +351,16 @@ int igemm5_pick(const IgemmArgs& a, int pin, int pout) {
         else if (g32 <= 256 && (K < 1024 || g16 <= 600)) id = ks_id(32, 32, 1, K >= 2048 && !window ? 8 : 4);
         else if (g32 <= 200 && window && K >= 1024) id = ks_id(32, 32, 1, 4);
         else if (g64 <= 256) id = ks_id(32, 32, 2, K >= 512 || K <= 128 ? 8 : 4);
+    } else if (window) {
+        // Against the 4-packed patch tiles: they pay a fixed price per 32 input channels, this kernel one per pixel and tap.
+        // Graph replays of every tile, us, ks against patch: 128 -> 128 at 28 x 28, batch 1 (g16 = 392): 5.4 / 5.9, batch 4:
+        // 6.8 / 6.0; 232 -> 72 at 40 x 16, stride 2, batch 12: 8.9 / 10.8; 5x5 64 -> 64 at 32 x 32, batch 8: 8.0 / 8.9;
+        // 512 -> 512 at 7 x 7, batch 16: 16.1 / 17.9.
+        const bool patch = patch4_can_run(a, pin, pout, 0), few_taps = a.T <= 9 && a.sh == 1 && a.sw == 1;
+        if (K >= 128 && g16 <= 300) id = ks_id(4, 16, 1, K >= 1024 ? 8 : 4);
+        else if (K >= 1024 && g16 <= 450) id = ks_id(4, 16, 1, 4);
+        else if (K >= 1024 && g32 <= (patch && few_taps && K < 4096 ? 200 : 256)) id = ks_id(4, 32, 1, 8);
+        else if (g64 <= 256 && (!patch || a.T > 9 || K >= 4096)) id = ks_id(4, 32, 2, 8);
     } else {
         if (K >= 128 && g16 <= 300) id = ks_id(4, 16, 1, K >= 1024 ? 8 : 4);
         else if (g64 <= 256) id = ks_id(4, 32, 2, K <= 192 ? 8 : 4);

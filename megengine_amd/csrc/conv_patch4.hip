@@ -1,0 +1,432 @@
+// Windowed convolutions on 4-packed tensors (NCHW4 in and out), tiles "patch4_*".
+//
+// An im2col operand of a 4-packed tensor comes in pieces of 4 bytes -- the channels of a pixel lie in planes -- so a tiled
+// implicit GEMM loads every byte of a 3x3 layer nine times, a dword at a time, through a per-unit table of offsets: 3x3
+// 64 -> 64 at 56 x 56, batch 16, took 11.6 us where its bytes and products allow 1.5, and the vector-memory path was what
+// it waited for.  Here the input patch of a tile is loaded once and turned on its way into LDS: sixteen channels of a pixel
+// side by side, [group of 16 channels][patch pixel][16 bytes], so that every tap's operand is one ds_read_b128 at a shifted
+// pixel, consecutive lanes consecutive pixels, free of bank conflicts.  The filter is turned with it: entry (channel group,
+// tap) of a stage holds 16 bytes per output channel, [entry][channel][16 bytes]; a step of v_mfma_i32_32x32x32_i8 is two
+// entries, one per half wave.
+//   * A workgroup is four waves side by side over the pixels; each multiplies all BM = 32 or 64 channels of the tile by its
+//     32 or 64 pixels.  A stage is GS channel groups (two for 3x3, one for larger filters); two stages are in LDS, the
+//     next one's global loads are in registers while the current one is multiplied, one barrier per stage.
+//   * Tiles are TH x TW pixels of one image, or of NI whole images where one is small; sizes chosen on the host so that the
+//     last tiles of a row and column are as full as the others.
+//   * Channel blocks past the last one meet zero filter bytes.
+//   * What bounds it: LDS, which a wave of 32 x 64 outputs reads three times for two matrix instructions, and the latency of a
+//     stage where tiles are few.  A wave of 64 x 64 (four reads for four) is ahead only where it still fills the chip twice: it
+//     costs a third of the occupancy.  Loads two stages ahead, tried, cost more occupancy than they hid (7.5 us against 6.9 at
+//     56 x 56 below); reading one step's operands ahead instead of two, or computing a descriptor per channel block instead of
+//     a scalar offset (157 scalar instructions per stage instead of 64), cost up to a quarter of the time.
+// Graph replays: 3x3 64 -> 64 at 56 x 56, batch 16: 12.5 -> 6.9 us, batch 64: 32.7 -> 17.1; 256 -> 256 at 14 x 14, batch 16:
+// 15.6 -> 8.8; 32 -> 32 at 112 x 112, batch 64: 54 -> 26; 5x5 100 -> 132 at 33 x 35, batch 20: 50 -> 22.8.
+#include <atomic>
+
+#include "igemm_shared.h"
+
+namespace mi355 {
+namespace {
+
+constexpr int P4_NPK = 4;   // patch vectors per thread and stage
+constexpr int P4_NKA = 7;   // filter vectors per thread and stage
+
+struct P4Args {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    uint32_t src_bytes, flt_bytes;
+    int IH, IW, OH, OW, FW, T, sh, sw, ph, pw;
+    int OC, N, icb, GS, nstages, kbytes;
+    int src_sn, src_scb, dst_sn, dst_scb, z_sn, has_bias;
+    int NI, TH, TW, PWC, PXI, PX;     // images, rows, columns of a tile; patch columns, pixels per image, pixels
+    int pkn, rpi, kan;                // patch pixels per thread; filter rows per pass of the workgroup, passes
+    int tiles_m, tiles_n, vr;         // vr: filter vectors per output channel and stage
+    FastDiv div_tiles_m, div_tiles_img, div_tiles_w, div_tw, div_tile_px, div_pxi, div_pwc, div_vr, div_t;
+    int tiles_img, tiles_w;           // tiles per image group, tiles per row
+    EpiParams epi;
+};
+
+template <int MT, int NT, int NL, bool HZ>
+__device__ __forceinline__ void p4_epilogue(const P4Args& a, v16i (&acc)[MT][NT], int oc0, const int (&d_px)[NT], const int (&z_px)[NT], int lh) {
+    uint32_t zw[NT][MT][4];
+    if (HZ) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int oc4 = oc0 + i * 32 + 8 * q + 4 * lh;
+                    zw[j][i][q] = d_px[j] >= 0 && oc4 < a.OC ? *reinterpret_cast<const uint32_t*>(a.z + z_px[j] + (int64_t)(oc4 >> 2) * a.dst_scb) : 0u;
+                }
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int oc4 = oc0 + i * 32 + 8 * q + 4 * lh;
+                const v16i& c = acc[i][j];
+                const uint32_t o = requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], HZ ? zw[j][i][q] : 0u, a.epi);
+                if (d_px[j] >= 0 && oc4 < a.OC) *reinterpret_cast<uint32_t*>(a.dst + d_px[j] + (int64_t)(oc4 >> 2) * a.dst_scb) = o;
+            }
+}
+
+// STEPS: MFMA steps of a stage when known (9: 3x3 filters, two groups), 0: from the arguments
+template <int MT, int NT, int STEPS>
+__global__ __launch_bounds__(256, 2) void patch4_kernel(P4Args a) {
+    constexpr int BM = MT * 32, KAN = (BM + 13) / 14;
+    // vectors from one entry to the next: the rows its passes store, made odd so that the stores of a row spread over the banks
+    const int kan = STEPS ? KAN : a.kan, rpi = STEPS ? 14 : a.rpi, BMP = (kan * rpi) | 1;
+    extern __shared__ __attribute__((aligned(16))) v4i lds[];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l32 = lane & 31, lh = lane >> 5;
+    const int E = a.GS * a.T, EP = (E + 1) & ~1;              // entries of a stage, of a whole number of steps
+    const int a_vecs = EP * BMP, stage_vecs = a_vecs + a.GS * a.PX;
+
+    // tile: contiguous pixel tiles per XCD (workgroup b runs on XCD b % 8), channel tiles of a pixel tile side by side
+    int tm, tn;
+    {
+        const int per = (a.tiles_n + 7) >> 3, x = blockIdx.x & 7, i = blockIdx.x >> 3;
+        const int r = (int)fdiv(i, a.div_tiles_m);
+        tm = i - r * a.tiles_m;
+        tn = x * per + r;
+        if (r >= per || tn >= a.tiles_n) return;
+    }
+    const int ig = (int)fdiv(tn, a.div_tiles_img), ti = tn - ig * a.tiles_img;
+    const int th = (int)fdiv(ti, a.div_tiles_w), tw = ti - th * a.tiles_w;
+    const int n0 = ig * a.NI, oh0 = th * a.TH, ow0 = tw * a.TW, oc0 = tm * BM;
+
+    // patch pixels of this thread: source offset of the first channel block, SENT outside the image
+    int p_off[P4_NPK];
+#pragma unroll
+    for (int k = 0; k < P4_NPK; ++k) {
+        if (k >= a.pkn) break;
+        const uint32_t px = t + k * 256, im = fdiv(px, a.div_pxi), r = px - im * a.PXI, pr = fdiv(r, a.div_pwc), pc = r - pr * a.PWC;
+        const int ih = oh0 * a.sh - a.ph + (int)pr, iw = ow0 * a.sw - a.pw + (int)pc, n = n0 + (int)im;
+        const bool ok = (int)px < a.PX && n < a.N && (unsigned)ih < (unsigned)a.IH && (unsigned)iw < (unsigned)a.IW;
+        p_off[k] = ok ? n * a.src_sn + (ih * a.IW + iw) * 4 : SENT;
+    }
+    // filter vectors of this thread: the same 16 bytes of every rpi-th row; dword d of a row is tap d % T of channel block
+    // d / T (rows past the last channel lie past the end of the buffer: zero)
+    const int T = STEPS ? 9 : a.T, vr = STEPS ? 18 : a.vr;
+    const int f_row = STEPS ? t / 18 : (int)fdiv(t, a.div_vr), f_first = (t - f_row * vr) * 4;
+    int f_off[P4_NKA];
+#pragma unroll
+    for (int k = 0; k < P4_NKA; ++k) {
+        if (k >= kan) break;
+        f_off[k] = f_row < rpi ? (oc0 + f_row + k * rpi) * a.kbytes + f_first * 4 : SENT;
+    }
+    const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes), rs_flt = make_rsrc(a.flt, a.flt_bytes);
+    v4i xp[P4_NPK], xf[P4_NKA];
+    const int row_words = a.icb * T, GS = STEPS ? 2 : a.GS;
+    // The patch's channel blocks are a scalar offset: those past the last one are the last one's again (they meet zero filter
+    // bytes), so that the scalar offset never leads out of the image.  The filter's stage is part of the lane's offset, which
+    // the descriptor's bounds check covers.
+    const uint32_t last_cb = (uint32_t)(a.icb - 1) * a.src_scb;
+    auto fetch = [&](int st) __attribute__((always_inline)) {
+        const int cb0 = st * GS * 4, left = row_words - cb0 * T;  // filter words left in a row
+        const int fo = cb0 * T * 4;
+#pragma unroll
+        for (int k = 0; k < P4_NKA; ++k) {
+            if (k >= kan) break;
+            xf[k] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, f_off[k] + fo, 0, 0);
+        }
+        int so[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) so[i] = (int)min((uint32_t)(cb0 + i) * a.src_scb, last_cb);
+#pragma unroll
+        for (int k = 0; k < P4_NPK; ++k) {
+            if (k >= a.pkn) break;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) xp[k][i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_src, p_off[k], so[i], 0);
+            if (k < P4_NPK / 2 && GS == 2) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) xp[P4_NPK / 2 + k][i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_src, p_off[k], so[4 + i], 0);
+            }
+        }
+        if (left < vr * 4) {  // the last stage, incomplete: words past the row's end are the next row's
+#pragma unroll
+            for (int k = 0; k < P4_NKA; ++k)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) xf[k][i] = f_first + i < left ? xf[k][i] : 0;
+        }
+    };
+    fetch(0);
+
+    int f_lds[4];
+    {
+        uint32_t cb = STEPS ? f_first / 9 : fdiv(f_first, a.div_t), tap = f_first - cb * T;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            f_lds[i] = (int)((((cb >> 2) * T + tap) * BMP + f_row) * 4 + (cb & 3));
+            if (++tap == (uint32_t)T) {
+                tap = 0;
+                ++cb;
+            }
+        }
+    }
+    auto store = [&](int buf) __attribute__((always_inline)) {
+        v4i* s = lds + buf * stage_vecs;
+        int* sw = reinterpret_cast<int*>(s);
+        if (f_row < rpi) {
+#pragma unroll
+            for (int k = 0; k < P4_NKA; ++k) {
+                if (k >= kan) break;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sw[f_lds[i] + k * rpi * 4] = xf[k][i];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < P4_NPK; ++k) {
+            if (k >= a.pkn) break;
+            if (t + k * 256 < a.PX) {
+                s[a_vecs + t + k * 256] = xp[k];
+                if (k < P4_NPK / 2 && GS == 2) s[a_vecs + a.PX + t + k * 256] = xp[P4_NPK / 2 + k];
+            }
+        }
+    };
+
+    // B operands: patch vector of each of this lane's pixels, and of each entry relative to it
+    int b_px[NT], d_px[NT], z_px[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const uint32_t p = (wave * NT + j) * 32 + l32;
+        const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)(a.TH * a.TW), oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
+        const bool ok = (int)im < a.NI && n0 + (int)im < a.N && oh0 + (int)oh < a.OH && ow0 + (int)ow < a.OW;
+        b_px[j] = (int)im < a.NI ? (int)(im * a.PXI + oh * a.sh * a.PWC + ow * a.sw) : 0;
+        const int at = ((oh0 + (int)oh) * a.OW + ow0 + (int)ow) * 4;
+        d_px[j] = ok ? (n0 + (int)im) * a.dst_sn + at : -1;
+        z_px[j] = (n0 + (int)im) * a.z_sn + at;
+    }
+    int* tab = reinterpret_cast<int*>(lds + 2 * stage_vecs);
+    for (int e = t; e < EP; e += 256) {
+        const int g = (int)fdiv(e, a.div_t), tap = e - g * a.T, fh = tap / a.FW, fw = tap - fh * a.FW;
+        tab[e] = e < E ? a_vecs + g * a.PX + fh * a.PWC + fw : a_vecs;
+    }
+    // the filter entry that fills up an odd number stays zero
+    if (EP != E && t < 2 * BM) lds[(t / BM) * stage_vecs + E * BMP + t % BM] = v4i{0, 0, 0, 0};
+    v16i acc[MT][NT];
+    {
+        const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            v16i b;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const v4i v = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, (oc0 + i * 32 + 8 * q + 4 * lh) * 4, 0, 0);
+                b[4 * q] = v[0]; b[4 * q + 1] = v[1]; b[4 * q + 2] = v[2]; b[4 * q + 3] = v[3];
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] = b;
+        }
+    }
+    store(0);
+    __syncthreads();
+    const int steps = EP / 2;
+    int offs[STEPS ? STEPS : 1];
+    if constexpr (STEPS != 0) {
+#pragma unroll
+        for (int k = 0; k < STEPS; ++k) offs[k] = tab[2 * k + lh];
+    }
+    for (int st = 0; st < a.nstages; ++st) {
+        if (st + 1 < a.nstages) fetch(st + 1);
+        const v4i* s = lds + (st & 1) * stage_vecs;
+        const v4i* pa = s + lh * BMP + l32;
+        auto load = [&](int k, int off, v4i (&fa)[MT], v4i (&fb)[NT]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) fa[i] = pa[k * 2 * BMP + i * 32];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) fb[j] = s[off + b_px[j]];
+        };
+        auto mult = [&](const v4i (&fa)[MT], const v4i (&fb)[NT]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
+        };
+        if constexpr (STEPS != 0) {
+            constexpr int AHEAD = 2;  // steps whose operands are read ahead
+            v4i fa[AHEAD + 1][MT], fb[AHEAD + 1][NT];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) load(k, offs[k], fa[k], fb[k]);
+#pragma unroll
+            for (int k = 0; k < STEPS; ++k) {
+                if (k + AHEAD < STEPS) load(k + AHEAD, offs[k + AHEAD], fa[(k + AHEAD) % (AHEAD + 1)], fb[(k + AHEAD) % (AHEAD + 1)]);
+                __builtin_amdgcn_sched_barrier(0);
+                mult(fa[k % (AHEAD + 1)], fb[k % (AHEAD + 1)]);
+            }
+        } else {
+            // two steps' operands, and the table entries of the two after them, are read ahead (past the last step: its own)
+            v4i fa[3][MT], fb[3][NT];
+            const int last = steps - 1;
+            load(0, tab[lh], fa[0], fb[0]);
+            load(min(1, last), tab[2 * min(1, last) + lh], fa[1], fb[1]);
+            int o0 = tab[2 * min(2, last) + lh], o1 = tab[2 * min(3, last) + lh], o2 = tab[2 * min(4, last) + lh];
+            for (int k = 0; k < steps; k += 3) {
+                load(min(k + 2, last), o0, fa[2], fb[2]);
+                o0 = tab[2 * min(k + 5, last) + lh];
+                mult(fa[0], fb[0]);
+                if (k + 1 >= steps) break;
+                load(min(k + 3, last), o1, fa[0], fb[0]);
+                o1 = tab[2 * min(k + 6, last) + lh];
+                mult(fa[1], fb[1]);
+                if (k + 2 >= steps) break;
+                load(min(k + 4, last), o2, fa[1], fb[1]);
+                o2 = tab[2 * min(k + 7, last) + lh];
+                mult(fa[2], fb[2]);
+            }
+        }
+        if (st + 1 < a.nstages) store((st + 1) & 1);
+        __syncthreads();
+    }
+
+#define MI355_P4(NL, HZ) p4_epilogue<MT, NT, NL, HZ>(a, acc, oc0, d_px, z_px, lh)
+    if (a.epi.lin) {
+        MI355_P4(NL_LIN, false);
+    } else if (a.epi.has_z) {
+        switch (a.epi.nonline) {
+            case NL_RELU: MI355_P4(NL_RELU, true); break;
+            case NL_H_SWISH: MI355_P4(NL_H_SWISH, true); break;
+            default: MI355_P4(NL_IDENTITY, true); break;
+        }
+    } else {
+        switch (a.epi.nonline) {
+            case NL_RELU: MI355_P4(NL_RELU, false); break;
+            case NL_H_SWISH: MI355_P4(NL_H_SWISH, false); break;
+            default: MI355_P4(NL_IDENTITY, false); break;
+        }
+    }
+#undef MI355_P4
+}
+
+struct P4Cfg {
+    int mt, nt;
+    const char* name;
+};
+constexpr P4Cfg kP4[] = {{1, 1, "patch4_32x128"}, {1, 2, "patch4_32x256"}, {2, 2, "patch4_64x256"}};
+constexpr int kP4Count = sizeof(kP4) / sizeof(kP4[0]);
+
+// geometry of a tile; false where no patch fits
+bool p4_plan(const IgemmArgs& a, int cfg, P4Args* k, int* lds_bytes) {
+    const int bm = kP4[cfg].mt * 32, bn = kP4[cfg].nt * 128;
+    const int FH = a.FH, FW = a.FW;
+    k->icb = a.kbytes / (4 * a.T);
+    const int G = (k->icb + 3) / 4;
+    k->GS = a.T <= 9 && G > 1 ? 2 : 1;
+    k->nstages = (G + k->GS - 1) / k->GS;
+    k->vr = k->GS * a.T;
+    if (k->vr > 256) return false;
+    k->rpi = 256 / k->vr;
+    k->kan = (bm + k->rpi - 1) / k->rpi;
+    if (k->kan > P4_NKA) return false;
+    const int max_px = P4_NPK / k->GS * 256;
+    // whole images while they fit several times, else rows; a wide image is split into equal columns
+    int tiles_w = 1;
+    for (;; ++tiles_w) {
+        k->TW = (a.OW + tiles_w - 1) / tiles_w;
+        if (k->TW > bn) continue;
+        int th = bn / k->TW;
+        k->NI = 1;
+        if (th >= a.OH) {
+            k->NI = tiles_w == 1 ? th / a.OH : 1;
+            th = a.OH;
+        }
+        for (;;) {
+            const int bands = (a.OH + th - 1) / th;
+            k->TH = (a.OH + bands - 1) / bands;
+            k->PWC = (k->TW - 1) * a.sw + FW;
+            k->PXI = ((k->TH - 1) * a.sh + FH) * k->PWC;
+            while (k->NI > 1 && k->NI * k->PXI > max_px) --k->NI;
+            k->PX = k->NI * k->PXI;
+            if (k->PX <= max_px || th == 1) break;
+            th = k->TH - 1;
+        }
+        if (k->PX <= max_px) break;
+        if (k->TW == 1) return false;
+    }
+    k->pkn = (k->PX + 255) / 256;
+    k->tiles_w = (a.OW + k->TW - 1) / k->TW;
+    k->tiles_img = k->tiles_w * ((a.OH + k->TH - 1) / k->TH);
+    const int64_t tn = (int64_t)((a.NB + k->NI - 1) / k->NI) * k->tiles_img;
+    k->tiles_m = (a.OC + bm - 1) / bm;
+    if (tn * k->tiles_m > 0x3ffffff0) return false;
+    k->tiles_n = (int)tn;
+    const int E = k->GS * a.T, EP = (E + 1) & ~1;
+    *lds_bytes = 2 * (EP * ((k->kan * k->rpi) | 1) + k->GS * k->PX) * 16 + EP * 4;
+    return *lds_bytes <= 160 * 1024;
+}
+
+template <int MT, int NT>
+int launch_p4(hipStream_t st, const P4Args& k, int lds) {
+    auto kern = k.GS * k.T == 18 ? patch4_kernel<MT, NT, 9> : patch4_kernel<MT, NT, 0>;
+    static std::atomic<int> max_lds_set{0};
+    if (max_lds_set.load(std::memory_order_relaxed) == 0) {
+        for (auto f : {patch4_kernel<MT, NT, 9>, patch4_kernel<MT, NT, 0>}) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if (e != hipSuccess) return (int)e;
+        }
+        max_lds_set.store(1, std::memory_order_relaxed);
+    }
+    const int64_t grid = (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(256), lds, st, k);
+}
+
+}  // namespace
+
+int patch4_num_cfgs() { return kP4Count; }
+const char* patch4_cfg_name(int cfg) { return kP4[cfg].name; }
+
+bool patch4_can_run(const IgemmArgs& a, int pin, int pout, int cfg) {
+    if (cfg < 0 || cfg >= kP4Count || pin != 4 || pout != 4 || a.groups != 1 || a.general || a.T < 2) return false;
+    P4Args k;
+    int lds;
+    return p4_plan(a, cfg, &k, &lds);
+}
+
+// Which tile: a workgroup of 32 x 256 once those are more than one per CU (64 -> 64 at 56 x 56, batch 16, 448 of them: 6.8 us
+// against 7.3 on 32 x 128; 100 -> 132 at 33 x 35 with a 5x5 filter: 22.8 against 30), or 64 x 256 once those are two (128 -> 128
+// at 28 x 28, batch 64: 14.4 us against 16.8); below, the smallest tile, because a stage's latency is all there is (256 -> 256 at
+// 14 x 14, batch 16, 128 workgroups of 32 x 256: 10.0 us against 8.8).  At strides a tile's patch is several times its pixels:
+// the smallest tile (64 -> 128 at 56 x 56, stride 2, batch 16: 7.1 us against 7.8 on 32 x 256), and with many output channels
+// and pixels the 128 x 128 tiles of the general kernel, whose operand traffic shrinks with the stride (the same at batch 64:
+// 14.5 us against 18.3; 128 -> 128, batch 32: 14.6 against 16.3).
+int patch4_pick(const IgemmArgs& a, int pin, int pout) {
+    if (!patch4_can_run(a, pin, pout, 0)) return -1;
+    if (a.sh > 1 || a.sw > 1) return a.OC > 64 && (int64_t)((a.OC + 127) / 128) * ((a.M + 127) / 128) >= 150 ? -1 : 0;
+    auto wgs = [&](int cfg) {
+        P4Args k;
+        int lds;
+        return p4_plan(a, cfg, &k, &lds) ? (int64_t)k.tiles_n * k.tiles_m : 0;
+    };
+    if (a.OC > 64 && wgs(2) >= 512) return 2;
+    return wgs(1) >= 300 ? 1 : 0;
+}
+
+int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg) {
+    P4Args k;
+    int lds;
+    if (!p4_plan(a, cfg, &k, &lds)) return (int)hipErrorInvalidConfiguration;
+    k.src = a.src; k.flt = a.flt; k.bias = a.bias; k.z = a.z; k.dst = a.dst;
+    k.src_bytes = a.src_bytes; k.flt_bytes = a.flt_bytes;
+    k.IH = a.IH; k.IW = a.IW; k.OH = a.OH; k.OW = a.OW; k.FW = a.FW; k.T = a.T;
+    k.sh = a.sh; k.sw = a.sw; k.ph = a.ph; k.pw = a.pw;
+    k.OC = a.OC; k.N = a.NB; k.kbytes = a.kbytes;
+    k.src_sn = a.src_sn; k.src_scb = a.src_scb; k.dst_sn = a.dst_sn; k.dst_scb = a.dst_scb; k.z_sn = a.z_sn;
+    k.has_bias = a.has_bias;
+    k.div_tiles_m = make_fastdiv(k.tiles_m); k.div_tiles_img = make_fastdiv(k.tiles_img); k.div_tiles_w = make_fastdiv(k.tiles_w);
+    k.div_tw = make_fastdiv(k.TW); k.div_tile_px = make_fastdiv(k.TH * k.TW);
+    k.div_pxi = make_fastdiv(k.PXI); k.div_pwc = make_fastdiv(k.PWC);
+    k.div_vr = make_fastdiv(k.vr); k.div_t = make_fastdiv(a.T);
+    k.epi = a.epi;
+    switch (cfg) {
+        case 0: return launch_p4<1, 1>(st, k, lds);
+        case 1: return launch_p4<1, 2>(st, k, lds);
+        default: return launch_p4<2, 2>(st, k, lds);
+    }
+}
+
+}  // namespace mi355

@@ -500,6 +500,13 @@ bool igemm5_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
 int igemm5_pick(const IgemmArgs& a, int pin, int pout);  // the tile for few output pixels, -1 where there are too many
 int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg);
 
+// windowed layers on 4-packed tensors: the input patch of a tile turned to 16 channels per pixel in LDS (conv_patch4.hip)
+int patch4_num_cfgs();
+const char* patch4_cfg_name(int cfg);
+bool patch4_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
+int patch4_pick(const IgemmArgs& a, int pin, int pout);  // its tile for this problem, -1 where another kernel is ahead
+int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg);
+
 // streaming kernel for 4-packed pointwise layers with few input or few output channels (conv_pw4.hip)
 bool pw4s_usable(const IgemmArgs& a);
 int launch_pw4s(hipStream_t st, const IgemmArgs& a, int cu_count);
