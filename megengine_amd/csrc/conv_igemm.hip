@@ -484,7 +484,7 @@ int launch_fmt(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
 // tile_cfg numbering: register-staged tiles, LDS-direct tiles, second-generation tiles, patch-staged tiles, weight-resident
 // tiles, the 32-packed streaming kernel, the tiles that split the reduction over the waves of a
 // workgroup, the one-launch NCHW4 group kernel, the 4-packed patch tiles
-int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1 + igemm5_num_cfgs() + 1 + patch4_num_cfgs(); }
+int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1 + igemm5_num_cfgs() + 1 + patch4_num_cfgs() + 1; }
 int igemm_first_v2_cfg() { return kNumCfgs + igemm_dma_num_cfgs(); }
 // planar destination (NCHW4_NCHW): two of the register-staged tiles
 static int launch_planar(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
@@ -501,6 +501,7 @@ static int igemm_pw32s_cfg() { return igemm_first_v4_cfg() + igemm4_num_cfgs(); 
 static int igemm_first_ks_cfg() { return igemm_pw32s_cfg() + 1; }
 static int igemm_grp4_cfg() { return igemm_first_ks_cfg() + igemm5_num_cfgs(); }
 static int igemm_first_p4_cfg() { return igemm_grp4_cfg() + 1; }
+static int igemm_pw4_split_cfg() { return igemm_first_p4_cfg() + patch4_num_cfgs(); }
 const char* igemm_cfg_name(int cfg) {
     if (cfg >= 0 && cfg < kNumCfgs) return kCfgs[cfg].name;
     if (cfg < igemm_first_v2_cfg()) return igemm_dma_cfg_name(cfg - kNumCfgs);
@@ -510,6 +511,7 @@ const char* igemm_cfg_name(int cfg) {
     if (cfg == igemm_pw32s_cfg()) return "pw32_stream";
     if (cfg < igemm_grp4_cfg()) return igemm5_cfg_name(cfg - igemm_first_ks_cfg());
     if (cfg == igemm_grp4_cfg()) return "grp4_dot4";
+    if (cfg == igemm_pw4_split_cfg()) return "pw4_split";
     return patch4_cfg_name(cfg - igemm_first_p4_cfg());
 }
 
@@ -615,6 +617,8 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         // the table form stays on the streaming kernel, which has it)
         IgemmArgs a;
         igemm_fill_args(p, a);
+        // NCHW4 pointwise at stride 1: four pixels per lane, at any number of pixels
+        if (pw4_quad_pick(a, p.pin, p.pout)) return pw4s_usable(a) ? kNumCfgs + igemm_dma_num_cfgs() - 1 : igemm_pw4_split_cfg();
         const int ks = igemm5_pick(a, p.pin, p.pout);
         if (ks >= 0) return igemm_first_ks_cfg() + ks;
         const int p4 = patch4_pick(a, p.pin, p.pout);
@@ -706,7 +710,8 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         // 4-packed pointwise layers (per-tile sweep of the MobileNetV2 1x1 layers): the LDS-direct tiles win wherever the
         // register-staged loop is latency-bound -- narrow outputs, and few tiles with a long reduction
         enum { D4_128x128x64 = kNumCfgs + 19, D4_64x64x128 = kNumCfgs + 20, D4_128x64x128 = kNumCfgs + 21, PW4_STREAM = kNumCfgs + 23 };
-        // at most 64 channels in, many out (the expansions): the streaming kernel, which has no per-tile pipeline
+        // strided (stride 1 is decided above).  At most 64 channels in, many out: the streaming kernel, which has no per-tile
+        // pipeline
         if (kbytes <= 64 && OC >= 64 && OC <= 1024) return PW4_STREAM;
         // one channel block out (the narrow projections): the same kernel, up to six k-steps
         if (OC <= 32 && kbytes <= 192) return PW4_STREAM;
@@ -845,6 +850,10 @@ static int resolve_filled(const ConvProblem& p, const IgemmArgs& a, int cfg) {
     }
     // group convolutions and the general epilogue exist on the second-generation tiles only
     if ((d.group != 1 || a.general) && cfg < first_v2) cfg = first_v2 + (p.ocpg <= 64 ? 3 : 0);
+    if (cfg == igemm_pw4_split_cfg()) {
+        if (pw4_split_usable(a, p.pin, p.pout)) return cfg;
+        cfg = first_v2;
+    }
     if (cfg >= igemm_first_p4_cfg()) {
         if (patch4_can_run(a, p.pin, p.pout, cfg - igemm_first_p4_cfg())) return cfg;
         cfg = first_v2;
@@ -964,6 +973,7 @@ int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_coun
             a.ztab = tab;
         }
     }
+    if (cfg == igemm_pw4_split_cfg()) return launch_pw4_split(st, a);
     if (cfg >= igemm_first_p4_cfg()) return launch_patch4(st, a, cfg - igemm_first_p4_cfg());
     if (cfg >= igemm_first_ks_cfg()) return launch_igemm5(st, a, p.pin, p.pout, cfg - igemm_first_ks_cfg());
     if (cfg == igemm_pw32s_cfg()) return launch_pw32s(st, a, cu_count);

@@ -1,5 +1,5 @@
-// Pointwise (1x1) int8 ConvBias on 4-packed activations, NCHW4 in and out, for the two kinds of layer that a tiled
-// kernel serves badly: at most 64 input channels and many output channels (the expansion layers of the MobileNet
+// Pointwise (1x1) int8 ConvBias on 4-packed activations, NCHW4 in and out.  At stride 1 pw4q_kernel and pw4k_kernel below;
+// pw4s_kernel serves strided layers of the two kinds that a tiled kernel serves badly: at most 64 input channels and many output channels (the expansion layers of the MobileNet
 // family: one or two MFMA k-steps, the cost is the output), and at most 32 output channels with up to 192 input
 // channels (its narrow projections: a tile of 128 filter rows would be three quarters empty).
 //
@@ -93,6 +93,274 @@ __global__ __launch_bounds__(256) void pw4s_kernel(IgemmArgs a, int n_ocg, int n
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) fb[kc] = nb[kc];
         if constexpr (HZ) zr = nz;
+    }
+}
+
+// Stride 1, at most 64 input channels and many tiles: the same with four consecutive pixels per lane.  pw4s_kernel's cost is its memory instructions -- a dword per lane,
+// four loads and four stores for every 32 x 32 block, 256 bytes each -- and an NCHW4 plane is contiguous over its pixels.  The
+// 32 columns of an MFMA need not be 32 neighbouring pixels: column l of product j is pixel 4 l + j here, so that a lane's operands
+// of four products are 16-byte loads, its results 16-byte stores, and a wave's access is a contiguous half kilobyte per channel
+// block.  The last group of an image whose plane is no multiple of four holds 1 to 3 pixels: its surplus columns multiply
+// whatever follows (the descriptor answers zeros past the tensor) and are not stored.  Bound by the output stream and the
+// four vector instructions per output: 16 -> 96 at 112 x 112, batch 64, 18.9 us for 90 MB (4.8 TB/s) against 22.2.
+template <int MT, int KC, bool HZ>
+__global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, int n_ocg, int n_pb, int groups, FastDiv div_g) {
+    __shared__ __attribute__((aligned(16))) int sBias[PW4_MAX_OC + 96];
+    const int t = threadIdx.x;
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    const int gw = blockIdx.x * 4 + wave, GW = gridDim.x * 4;  // GW is a multiple of n_ocg
+    const int pb0 = gw / n_ocg, ocg = gw - pb0 * n_ocg, step = GW / n_ocg;
+    const int oc_w = ocg * MT * 32;
+    const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes);
+    const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, a.flt_bytes);
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, HZ ? a.z_bytes : 0);
+    const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes);
+
+    v4i fa[MT][KC];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int row = oc_w + i * 32 + l32;
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc)
+            fa[i][kc] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, row < a.OC ? row * a.kbytes + kc * 32 + lh * 16 : SENT, 0, 0);
+    }
+    const int icb = a.kbytes >> 2, total = a.NB * groups;
+    // x[kc][i]: four pixels of channel block kc * 8 + lh * 4 + i (zeros past the last one)
+    auto load_b = [&](int pb, v4i (&x)[KC][4]) __attribute__((always_inline)) {
+        const int m = pb * 32 + l32;
+        const bool ok = m < total;  // also false for every block past the last one
+        const uint32_t mm = ok ? m : 0, n = fdiv(mm, div_g), g = mm - n * groups;
+        const int pix = (int)n * a.src_sn + (int)g * 16 + lh * 4 * a.src_scb;
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                x[kc][i] = __builtin_amdgcn_raw_buffer_load_b128(
+                        rs_src, ok && kc * 8 + lh * 4 + i < icb ? pix + (kc * 8 + i) * a.src_scb : SENT, 0, 0);
+    };
+    v4i x[KC][4];
+    load_b(pb0, x);
+    // the bias goes to LDS after the filter rows and the first block are requested
+    for (int i = t; i < PW4_MAX_OC + 96; i += 256) sBias[i] = (a.has_bias && i < a.OC) ? a.bias[i] : 0;
+    __syncthreads();
+    const int tail = a.OHW & 3;
+    auto blocks = [&](auto nl) __attribute__((always_inline)) {
+        constexpr int NL = decltype(nl)::value;
+        for (int pb = pb0; pb < n_pb; pb += step) {
+            v4i fb[KC][4];
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) fb[kc][j] = v4i{x[kc][0][j], x[kc][1][j], x[kc][2][j], x[kc][3][j]};
+            load_b(pb + step, x);  // in flight during the products and the epilogue of this block
+            const int m = pb * 32 + l32;
+            const bool ok = m < total;
+            const uint32_t mm = ok ? m : 0, n = fdiv(mm, div_g), g = mm - n * groups;
+            const bool part = tail != 0 && (int)g == groups - 1;
+            const int d0 = (int)n * a.dst_sn + (int)g * 16 + ((oc_w >> 2) + lh) * a.dst_scb;
+            const int z0 = (int)n * a.z_sn + (int)g * 16 + ((oc_w >> 2) + lh) * a.dst_scb;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                if (oc_w + i * 32 >= a.OC) break;  // wave-uniform
+                v4i zv[4];
+                if constexpr (HZ)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        zv[q] = __builtin_amdgcn_raw_buffer_load_b128(
+                                rs_z, ok && oc_w + i * 32 + 8 * q + 4 * lh < a.OC ? z0 + (i * 8 + q * 2) * a.dst_scb : SENT, 0, 0);
+                v16i bv;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const v4i b = *reinterpret_cast<const v4i*>(sBias + oc_w + i * 32 + 8 * q + 4 * lh);
+                    bv[4 * q + 0] = b[0]; bv[4 * q + 1] = b[1]; bv[4 * q + 2] = b[2]; bv[4 * q + 3] = b[3];
+                }
+                v4i o[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v16i c = bv;
+#pragma unroll
+                    for (int kc = 0; kc < KC; ++kc) c = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i][kc], fb[kc][j], c, 0, 0, 0);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        o[q][j] = (int)requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], HZ ? (uint32_t)zv[q][j] : 0u, a.epi);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const bool in = ok && oc_w + i * 32 + 8 * q + 4 * lh < a.OC;
+                    const int at = d0 + (i * 8 + q * 2) * a.dst_scb;
+                    __builtin_amdgcn_raw_buffer_store_b128(o[q], rs_dst, in && !part ? at : SENT, 0, 0);
+                    // (see igemm_epilogue: the data registers of a wide store are read after it issues, and inline
+                    // assembly packs the next results)
+                    asm volatile("s_nop 1" ::"v"(o[q]) : "memory");
+                    if (tail != 0)
+#pragma unroll
+                        for (int r = 0; r < 3; ++r)
+                            if (r < tail) __builtin_amdgcn_raw_buffer_store_b32(o[q][r], rs_dst, in && part ? at + r * 4 : SENT, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // one channel block's accumulators and residual at a time
+            }
+        }
+    };
+    if (!HZ && a.epi.lin) {
+        blocks(std::integral_constant<int, NL_LIN>{});
+    } else {
+        switch (a.epi.nonline) {
+            case NL_RELU: blocks(std::integral_constant<int, NL_RELU>{}); break;
+            case NL_H_SWISH: blocks(std::integral_constant<int, NL_H_SWISH>{}); break;
+            default: blocks(std::integral_constant<int, NL_IDENTITY>{}); break;
+        }
+    }
+}
+
+// Longer reductions at stride 1: four pixels per lane as above, tiles of 16 MT channels x 64 pixels, and the reduction split
+// over the W waves of a workgroup, operands straight into registers (v_mfma_i32_16x16x64_i8: lane l holds filter row l % 16
+// and, of pixels 4 (l % 16) .. + 3, the 16 k-bytes at 16 (l / 16)).  What bounds these layers is latency -- a few megabytes and a
+// few hundred products per CU -- so a wave asks for all (or four steps) of its operands at once, and the partial sums meet
+// in LDS once.
+template <int MT>
+__global__ __launch_bounds__(512) void pw4k_kernel(IgemmArgs a, int tiles_m, int tiles_n, int groups, FastDiv div_g, FastDiv div_tm) {
+    constexpr int AHEAD = MT <= 2 ? 4 : 3;
+    extern __shared__ __attribute__((aligned(16))) v4i part[];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), W = blockDim.x >> 6;
+    const int ls = lane & 15, lk = lane >> 4;
+    // workgroup b runs on XCD b % 8: each XCD takes a contiguous run of pixels with all their channels
+    const uint32_t at = blockIdx.x >> 3, r0 = fdiv(at, div_tm);
+    const int tm = (int)(at - r0 * tiles_m), tn = (int)(blockIdx.x & 7) * ((tiles_n + 7) >> 3) + (int)r0;
+    if (tn >= tiles_n) return;
+    const int oc0 = tm * MT * 16;
+    const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes);
+    const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, a.flt_bytes);
+    const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.z_bytes);
+    const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes);
+
+    const int m = tn * 16 + ls;
+    const bool ok = m < a.NB * groups;
+    const uint32_t mm = ok ? m : 0, n = fdiv(mm, div_g), g = mm - n * groups;
+    const int pix = (int)n * a.src_sn + (int)g * 16 + lk * 4 * a.src_scb, icb = ok ? a.kbytes >> 2 : 0;
+    int row[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) row[i] = oc0 + i * 16 + ls < a.OC ? (oc0 + i * 16 + ls) * a.kbytes + lk * 16 : SENT;
+
+    // this wave's piece of the reduction, in steps of 64 bytes
+    const int steps = (a.kbytes + 63) >> 6, per = steps / W, extra = steps - per * W;
+    int kc = wave * per + (wave < extra ? wave : extra);
+    const int k1 = kc + per + (wave < extra ? 1 : 0);
+    int left = k1 - kc;
+    // operands of the next step; past the wave's piece every lane is out of range: zeros, no memory access
+    auto load = [&](v4i (&fa)[MT], v4i (&x)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            fa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, kc < k1 && row[i] != SENT ? row[i] + kc * 64 : SENT, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int cb = kc * 16 + i;
+            x[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, kc < k1 && cb + lk * 4 < icb ? pix + cb * a.src_scb : SENT, 0, 0);
+        }
+        ++kc;
+    };
+    v4i acc[MT][4];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+    auto multiply = [&](const v4i (&fa)[MT], const v4i (&x)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const v4i fb = {x[0][j], x[1][j], x[2][j], x[3][j]};
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb, acc[i][j], 0, 0, 0);
+        }
+    };
+    const int tail = a.OHW & 3;
+    const bool cut = tail != 0 && (int)g == groups - 1;  // 1 to 3 pixels: the last group of an image
+    v4i bz[MT], zv[MT];
+    auto bias_z = [&](int i, v4i& b, v4i& z) __attribute__((always_inline)) {
+        const int oc4 = oc0 + i * 16 + lk * 4;
+        b = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, oc4 * 4, 0, 0);
+        z = v4i{0, 0, 0, 0};
+        if (a.epi.has_z)
+            z = __builtin_amdgcn_raw_buffer_load_b128(rs_z, ok && oc4 < a.OC ? (int)n * a.z_sn + (int)g * 16 + (oc4 >> 2) * a.dst_scb : SENT, 0, 0);
+    };
+    {
+        v4i fa[AHEAD][MT], x[AHEAD][4];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) load(fa[u], x[u]);
+        if (W == 1) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) bias_z(i, bz[i], zv[i]);
+        } else if (wave < MT) {
+            bias_z(wave, bz[0], zv[0]);
+        }
+        for (; left > AHEAD; left -= AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                multiply(fa[u], x[u]);
+                load(fa[u], x[u]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (u < left) multiply(fa[u], x[u]);
+    }
+    if (W > 1) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) part[((wave * MT + i) * 4 + j) * 64 + lane] = acc[i][j];
+        __syncthreads();
+        if (wave >= MT) return;
+    }
+    auto finish = [&](auto nl, auto hz) __attribute__((always_inline)) {
+        constexpr int NL = decltype(nl)::value;
+        constexpr bool HZ = decltype(hz)::value;
+        auto write = [&](int i, const v4i (&s)[4], const v4i& z) __attribute__((always_inline)) {
+            const int oc4 = oc0 + i * 16 + lk * 4;
+            const bool in = ok && oc4 < a.OC;
+            const int d = (int)n * a.dst_sn + (int)g * 16 + (oc4 >> 2) * a.dst_scb;
+            v4i o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = (int)requant4_fast<NL, HZ>(s[j][0], s[j][1], s[j][2], s[j][3], (uint32_t)z[j], a.epi);
+            __builtin_amdgcn_raw_buffer_store_b128(o, rs_dst, in && !cut ? d : SENT, 0, 0);
+            asm volatile("s_nop 1" ::"v"(o) : "memory");  // (see igemm_epilogue)
+            if (tail != 0)
+#pragma unroll
+                for (int r = 0; r < 3; ++r)
+                    if (r < tail) __builtin_amdgcn_raw_buffer_store_b32(o[r], rs_dst, in && cut ? d + r * 4 : SENT, 0, 0);
+        };
+        if (W == 1) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const v4i s[4] = {acc[i][0] + bz[i], acc[i][1] + bz[i], acc[i][2] + bz[i], acc[i][3] + bz[i]};
+                write(i, s, zv[i]);
+            }
+            return;
+        }
+        for (int i = wave; i < MT; i += W) {
+            if (i != wave) bias_z(i, bz[0], zv[0]);
+            v4i s[4] = {bz[0], bz[0], bz[0], bz[0]};
+            for (int w = 0; w < W; ++w)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s[j] += part[((w * MT + i) * 4 + j) * 64 + lane];
+            write(i, s, zv[0]);
+        }
+    };
+    using std::integral_constant;
+    if (a.epi.lin) {
+        finish(integral_constant<int, NL_LIN>{}, integral_constant<bool, false>{});
+    } else if (a.epi.has_z) {
+        switch (a.epi.nonline) {
+            case NL_RELU: finish(integral_constant<int, NL_RELU>{}, integral_constant<bool, true>{}); break;
+            case NL_H_SWISH: finish(integral_constant<int, NL_H_SWISH>{}, integral_constant<bool, true>{}); break;
+            default: finish(integral_constant<int, NL_IDENTITY>{}, integral_constant<bool, true>{}); break;
+        }
+    } else {
+        switch (a.epi.nonline) {
+            case NL_RELU: finish(integral_constant<int, NL_RELU>{}, integral_constant<bool, false>{}); break;
+            case NL_H_SWISH: finish(integral_constant<int, NL_H_SWISH>{}, integral_constant<bool, false>{}); break;
+            default: finish(integral_constant<int, NL_IDENTITY>{}, integral_constant<bool, false>{}); break;
+        }
     }
 }
 
@@ -212,6 +480,34 @@ int launch32_mt(hipStream_t st, const IgemmArgs& a, int cu_count) {
 }
 
 template <int MT, int KC>
+int launch_quad(hipStream_t st, const IgemmArgs& a, int cu_count) {
+    const int ocb = (a.OC + 31) / 32;
+    const int n_ocg = (ocb + MT - 1) / MT;
+    const int groups = (a.OHW + 3) / 4;
+    const int n_pb = (int)(((int64_t)a.NB * groups + 31) / 32);
+    if (cu_count <= 0) cu_count = 256;
+    int64_t blocks = ((int64_t)n_pb * n_ocg + 3) / 4;
+    const int64_t cap = (int64_t)cu_count * 3;  // 12 waves per CU
+    if (blocks > cap) blocks = cap;
+    blocks = (blocks + n_ocg - 1) / n_ocg * n_ocg;  // waves of one pixel block stay together; 4 * blocks % n_ocg == 0
+    const FastDiv div_g = make_fastdiv(groups);
+    if (a.epi.has_z)
+        return launch_kernel((pw4q_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, groups, div_g);
+    return launch_kernel((pw4q_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, groups, div_g);
+}
+
+template <int MT>
+int launch_split(hipStream_t st, const IgemmArgs& a, int waves) {
+    const int tiles_m = (a.OC + MT * 16 - 1) / (MT * 16);
+    const int groups = (a.OHW + 3) / 4;
+    const int tiles_n = (int)(((int64_t)a.NB * groups + 15) / 16);
+    const int64_t grid = (int64_t)((tiles_n + 7) / 8) * 8 * tiles_m;
+    if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
+    return launch_kernel(pw4k_kernel<MT>, dim3((unsigned)grid), dim3(waves * 64), waves > 1 ? waves * MT * 4096 : 0, st, a, tiles_m, tiles_n,
+                         groups, make_fastdiv(groups), make_fastdiv(tiles_m));
+}
+
+template <int MT, int KC>
 int launch_mt(hipStream_t st, const IgemmArgs& a, int cu_count) {
     const int ocb = (a.OC + 31) / 32;
     const int n_ocg = (ocb + MT - 1) / MT;
@@ -228,9 +524,60 @@ int launch_mt(hipStream_t st, const IgemmArgs& a, int cu_count) {
 
 }  // namespace
 
+// Stride 1, where the planes of src and dst match pixel for pixel: which kernel with four pixels per lane, and its tile.
+// Tiles of 16 channels x 64 pixels (T) and steps of 64 input channels decide.  Every variant was timed as graph replays on the
+// layers of MobileNetV2 at batch 1 to 64 and on 70 sizes drawn over 16 to 960 channels on both sides, planes of 7 x 7 to
+// 112 x 112 and batch 1 to 64, against the kernels that served them before; us, this rule against those:
+//   at most 64 channels, streaming: 16 -> 96 at 112 x 112, batch 64: 18.9 / 22.2; 24 -> 144 at 56 x 56: 11.2 / 13.6; batch 16:
+//     5.0 / 6.6; 32 -> 192 at 28 x 28, batch 64: 5.9 / 7.2.  (96 channels per wave instead of 32 with very many tiles: less of the
+//     input again, 18.9 / 19.4.)
+//   one wave per tile while a wave can ask for all its operands at once (up to five steps): 96 -> 576 at 14 x 14, batch 64:
+//     6.4 / 7.2; 160 -> 960 at 7 x 7: 5.3 / 6.1; 192 -> 32 at 28 x 28: 4.3 / 5.7; 68 -> 76 at 10 x 70, batch 13: 3.6 / 4.8.
+//   longer reductions over the waves of a workgroup: 576 -> 96 at 14 x 14, batch 64: 6.0 / 7.0; 960 -> 160 at 7 x 7: 5.5 / 6.8,
+//     batch 16: 4.0 / 5.2, batch 1: 3.7 / 3.7.
+// The tiled kernels keep what they are better at (pw4_quad_pick), large products without a residual: 88 -> 448 at 42 x 19,
+// batch 30: 9.2 / 8.4; 956 -> 524 at 105 x 25, batch 7: 28.2 / 23.9; 960 -> 320 at 7 x 7, batch 64: 7.1 / 6.7 (with a residual
+// they are behind: 156 -> 628 at 43 x 58, batch 23: 27.5 / 34.9).  Between T = 3000 and 9000 without a residual, and for six
+// steps, the two are close and the tiled kernels keep their layers: 384 -> 64 at 14 x 14, batch 64: 4.7 / 5.0; 96 -> 576: 6.4 /
+// 7.2; 108 -> 384 at 11 x 12, batch 62: 4.6 / 5.1.
+struct QuadPlan {
+    int mt;      // 0: none
+    int waves;   // 0: the streaming kernel
+};
+static bool quad_stride(const IgemmArgs& a) { return a.sh == 1 && a.sw == 1; }
+static int64_t quad_tiles(const IgemmArgs& a) {
+    return (int64_t)((a.OC + 15) / 16) * (((int64_t)a.NB * ((a.OHW + 3) / 4) + 15) / 16);
+}
+static QuadPlan quad_plan(const IgemmArgs& a) {
+    const int64_t T = quad_tiles(a);
+    const int steps = (a.kbytes + 63) / 64;
+    const auto most = [&](int mt) { return mt > 2 && a.OC <= 32 ? 2 : mt; };  // no rows for channels that are not there
+    if (steps == 1 && T > 2000 && a.OC <= PW4_MAX_OC) return {T >= 30000 && a.kbytes <= 32 && a.OC > 64 && a.OC <= 512 ? 3 : 1, 0};
+    if (steps <= 5) return {T <= 1300 ? 1 : T <= 3000 ? 2 : most(4), 1};
+    if (T <= 250) return {1, 4};
+    if (T <= 450) return {2, 4};
+    if (T <= 2000) return steps > 6 ? QuadPlan{most(4), 4} : QuadPlan{2, 2};
+    return {most(4), 1};
+}
+// The streaming tile (pw4_stream) runs where a wave holds its channels' whole filter rows or, narrow, at most three steps; the
+// split tile (pw4_split) runs every pointwise layer at stride 1.
 bool pw4s_usable(const IgemmArgs& a) {
     if (a.T != 1 || a.ph != 0 || a.pw != 0 || a.OC > PW4_MAX_OC) return false;
     return a.kbytes <= 64 || (a.OC <= 32 && a.kbytes <= 192);
+}
+bool pw4_split_usable(const IgemmArgs& a, int pin, int pout) {
+    return pin == 4 && pout == 4 && a.groups == 1 && !a.general && a.T == 1 && a.ph == 0 && a.pw == 0 && quad_stride(a);
+}
+// whether one of the two is ahead of the tiled kernels
+bool pw4_quad_pick(const IgemmArgs& a, int pin, int pout) {
+    if (!pw4_split_usable(a, pin, pout)) return false;
+    if (pw4s_usable(a)) return true;
+    const int64_t T = quad_tiles(a);
+    const int steps = (a.kbytes + 63) / 64;
+    if (steps > 6 && T > 450 && T <= 2000 && a.OC > 256) return false;
+    if (a.epi.has_z) return T * steps <= 200000;
+    if (T * steps > 100000) return false;
+    return a.OC <= 64 ? T <= 750 || steps != 6 : T <= (steps == 6 ? 750 : steps > 6 ? 9000 : 3000);
 }
 
 // 32-packed: pointwise without padding, dense, the fast epilogue, 32 to 128 input channels, at most 1024 output channels
@@ -250,9 +597,22 @@ int launch_pw32s(hipStream_t st, const IgemmArgs& a, int cu_count) {
     }
 }
 
+int launch_pw4_split(hipStream_t st, const IgemmArgs& a) {
+    if (a.M == 0 || a.OC == 0) return 0;
+    QuadPlan q = quad_plan(a);
+    if (q.waves == 0) q = {4, 1};
+    return q.mt == 1 ? launch_split<1>(st, a, q.waves) : q.mt == 2 ? launch_split<2>(st, a, q.waves) : launch_split<4>(st, a, q.waves);
+}
+
 int launch_pw4s(hipStream_t st, const IgemmArgs& a, int cu_count) {
     if (a.M == 0 || a.OC == 0) return 0;
     const int ocb = (a.OC + 31) / 32;
+    if (quad_stride(a)) {
+        const QuadPlan q = quad_plan(a);
+        if (q.waves != 0) return launch_pw4_split(st, a);
+        if (a.kbytes > 32) return launch_quad<1, 2>(st, a, cu_count);
+        return q.mt == 3 ? launch_quad<3, 1>(st, a, cu_count) : launch_quad<1, 1>(st, a, cu_count);
+    }
     if (ocb == 1) {  // narrow outputs (the projections): one channel block per wave, up to six k-steps
         switch ((a.kbytes + 31) / 32) {
             case 1: return launch_mt<1, 1>(st, a, cu_count);

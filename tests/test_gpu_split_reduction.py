@@ -44,7 +44,7 @@ def test_every_tile(oracle, i):
 
 
 def test_the_chooser_takes_them_for_few_pixels_only():
-    for fmt, ic, hw, oc, f in (("NCHW32", 512, 7, 512, 3), ("NCHW32", 1024, 14, 256, 1), ("NCHW4", 384, 14, 64, 1)):
+    for fmt, ic, hw, oc, f in (("NCHW32", 512, 7, 512, 3), ("NCHW32", 1024, 14, 256, 1), ("NCHW4", 128, 28, 128, 3)):
         names = [lib.tile_names()[ops.conv_bias_query(_abi.make_conv_desc(fmt, n, ic, hw, hw, oc, f, pad=f // 2, **S))[0].tile_cfg]
                  for n in (1, 64)]
         assert "ks" in names[0] and "ks" not in names[1], names
