@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void dw3x3_kernel(Dw3Args a) {
     asm volatile("" ::"s"(a.div_qw.m), "s"(a.div_qw.s1), "s"(a.div_qw.s2), "s"(a.div_ohs.m), "s"(a.div_ohs.s1),
                  "s"(a.div_ohs.s2), "s"(a.div_cg.m), "s"(a.div_cg.s1), "s"(a.div_cg.s2), "s"(a.epi.fast), "s"(a.epi.lin),
                  "s"(a.epi.has_z), "s"(a.epi.nonline), "s"(a.epi.lin_c), "s"(a.epi.lin_d), "s"(a.epi.lin_lo));
-    const uint32_t item = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t item = xcd_block() * 256u + threadIdx.x;
     if (item >= a.items) return;
     // item = ((n * CG + cg) * OHS + strip) * QW + quad
     const uint32_t i1 = fdiv(item, a.div_qw), q = item - i1 * a.QW;
@@ -431,7 +431,7 @@ __global__ __launch_bounds__(256) void dwf_kernel(Dw3Args a) {
     constexpr int R = 2, P = F / 2, ROWS = (R - 1) * S + F;
     constexpr int FIRST = 4 - P;                       // pixel of the loaded blocks at which output 0's window starts
     constexpr int NB = (FIRST + 3 * S + F + 3) / 4;    // blocks a thread loads per row
-    const uint32_t item = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t item = xcd_block() * 256u + threadIdx.x;
     if (item >= a.items) return;
     const uint32_t i1 = fdiv(item, a.div_qw), q = item - i1 * a.QW;
     const uint32_t i2 = fdiv(i1, a.div_ohs), strip = i1 - i2 * a.OHS;

@@ -109,8 +109,17 @@ __global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, int n_ocg, in
     const int t = threadIdx.x;
     const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
-    const int gw = blockIdx.x * 4 + wave, GW = gridDim.x * 4;  // GW is a multiple of n_ocg
-    const int pb0 = gw / n_ocg, ocg = gw - pb0 * n_ocg, step = GW / n_ocg;
+    // pixel blocks by XCD, as in pw32s_kernel below
+    int pb_lo = 0, pb_hi = n_pb, gw = blockIdx.x * 4 + wave, GW = gridDim.x * 4;  // GW is a multiple of n_ocg
+    if ((gridDim.x & 7) == 0 && ((gridDim.x >> 3) * 4) % n_ocg == 0) {
+        const int xc = blockIdx.x & 7, per = n_pb >> 3, rem = n_pb & 7;
+        pb_lo = xc * per + (xc < rem ? xc : rem);
+        pb_hi = pb_lo + per + (xc < rem ? 1 : 0);
+        gw = (blockIdx.x >> 3) * 4 + wave;
+        GW = (gridDim.x >> 3) * 4;
+    }
+    const int q0 = gw / n_ocg, ocg = gw - q0 * n_ocg, step = GW / n_ocg;
+    const int pb0 = pb_lo + q0;
     const int oc_w = ocg * MT * 32;
     const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes);
     const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, a.flt_bytes);
@@ -140,20 +149,20 @@ __global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, int n_ocg, in
                         rs_src, ok && kc * 8 + lh * 4 + i < icb ? pix + (kc * 8 + i) * a.src_scb : SENT, 0, 0);
     };
     v4i x[KC][4];
-    load_b(pb0, x);
+    load_b(pb0 < pb_hi ? pb0 : n_pb, x);
     // the bias goes to LDS after the filter rows and the first block are requested
     for (int i = t; i < PW4_MAX_OC + 96; i += 256) sBias[i] = (a.has_bias && i < a.OC) ? a.bias[i] : 0;
     __syncthreads();
     const int tail = a.OHW & 3;
     auto blocks = [&](auto nl) __attribute__((always_inline)) {
         constexpr int NL = decltype(nl)::value;
-        for (int pb = pb0; pb < n_pb; pb += step) {
+        for (int pb = pb0; pb < pb_hi; pb += step) {
             v4i fb[KC][4];
 #pragma unroll
             for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) fb[kc][j] = v4i{x[kc][0][j], x[kc][1][j], x[kc][2][j], x[kc][3][j]};
-            load_b(pb + step, x);  // in flight during the products and the epilogue of this block
+            load_b(pb + step < pb_hi ? pb + step : n_pb, x);  // in flight during the products and the epilogue of this block
             const int m = pb * 32 + l32;
             const bool ok = m < total;
             const uint32_t mm = ok ? m : 0, n = fdiv(mm, div_g), g = mm - n * groups;
@@ -490,6 +499,9 @@ int launch_quad(hipStream_t st, const IgemmArgs& a, int cu_count) {
     const int64_t cap = (int64_t)cu_count * 3;  // 12 waves per CU
     if (blocks > cap) blocks = cap;
     blocks = (blocks + n_ocg - 1) / n_ocg * n_ocg;  // waves of one pixel block stay together; 4 * blocks % n_ocg == 0
+    // a multiple of the workgroups that deal out whole pixel blocks on every XCD (see the kernel)
+    const int unit = 8 * (n_ocg % 4 == 0 ? n_ocg / 4 : n_ocg % 2 == 0 ? n_ocg / 2 : n_ocg);
+    if (2 * blocks >= unit) blocks = (blocks + unit - 1) / unit * unit;
     const FastDiv div_g = make_fastdiv(groups);
     if (a.epi.has_z)
         return launch_kernel((pw4q_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, groups, div_g);

@@ -101,8 +101,8 @@ template <int PACK, int VB, int MODE, int FH, int FW>
 __global__ __launch_bounds__(256) void pooling_static_kernel(PoolArgs a) {
     constexpr int UPP = PACK / VB;
     constexpr int W = VB / 4;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t u = blockIdx.x * blockDim.x + threadIdx.x; u < a.units; u += stride) {
+    const XcdRun<uint32_t> run = xcd_run<uint32_t>(a.units);
+    for (uint32_t u = run.at; u < run.end; u += run.step) {
         const uint32_t sub = UPP == 1 ? 0 : u % UPP, pix = UPP == 1 ? u : u / UPP;
         const uint32_t t = fdiv(pix, a.div_ow), ow = pix - t * a.OW;
         const uint32_t plane = fdiv(t, a.div_oh), oh = t - plane * a.OH;
@@ -177,8 +177,8 @@ template <int PACK, int VB, int MODE>
 __global__ __launch_bounds__(256) void pooling_kernel(PoolArgs a) {
     constexpr int UPP = PACK / VB;  // threads per pixel
     constexpr int W = VB >= 4 ? VB / 4 : 1;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t u = blockIdx.x * blockDim.x + threadIdx.x; u < a.units; u += stride) {
+    const XcdRun<uint32_t> run = xcd_run<uint32_t>(a.units);
+    for (uint32_t u = run.at; u < run.end; u += run.step) {
         const uint32_t sub = UPP == 1 ? 0 : u % UPP, pix = UPP == 1 ? u : u / UPP;
         const uint32_t t = fdiv(pix, a.div_ow), ow = pix - t * a.OW;
         const uint32_t plane = fdiv(t, a.div_oh), oh = t - plane * a.OH;
@@ -401,6 +401,7 @@ int launch_pooling(hipStream_t st, const mi355_pooling_desc& d, int pack, uint32
     uint64_t blocks = (units + 255) / 256;
     const uint64_t cap = (uint64_t)cu_count * 64;
     if (blocks > cap) blocks = cap;
+    blocks = xcd_grid(blocks);
     if (pack == 32) return launch_mode<32, 16>(st, a, (int)d.mode, (unsigned)blocks);
     if (pack == 4) return launch_mode<4, 4>(st, a, (int)d.mode, (unsigned)blocks);
     return launch_mode<1, 1>(st, a, (int)d.mode, (unsigned)blocks);

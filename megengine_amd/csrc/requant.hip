@@ -12,8 +12,8 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(256) void requant_kernel(const int32_t* __restrict__ src, const int8_t* __restrict__ z,
                                                       int8_t* __restrict__ dst, uint64_t quads, uint64_t count, EpiParams e) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads; i += stride) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads);
+    for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4i a = reinterpret_cast<const v4i*>(src)[i];
         const uint32_t zw = e.has_z ? reinterpret_cast<const uint32_t*>(z)[i] : 0u;
         reinterpret_cast<uint32_t*>(dst)[i] = requant4(a[0], a[1], a[2], a[3], zw, e);
@@ -28,8 +28,8 @@ __global__ __launch_bounds__(256) void requant_kernel(const int32_t* __restrict_
 // QuantizedS8 first operand: 16 elements per thread step (16 + 16 bytes in, 16 out; 2-3 bytes per element)
 __global__ __launch_bounds__(256) void requant8_kernel(const int8_t* __restrict__ src, const int8_t* __restrict__ z,
                                                        int8_t* __restrict__ dst, uint64_t blocks16, uint64_t count, EpiParams e) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < blocks16; i += stride) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(blocks16);
+    for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4i a = reinterpret_cast<const v4i*>(src)[i];
         v4i zv = {0, 0, 0, 0};
         if (e.has_z) zv = reinterpret_cast<const v4i*>(z)[i];
@@ -60,8 +60,8 @@ __device__ __forceinline__ int quantize_s8(float x, float scale) {
 
 __global__ __launch_bounds__(256) void cvt_f32_s8_kernel(const float* __restrict__ src, int8_t* __restrict__ dst,
                                                          uint64_t quads, uint64_t count, float scale) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads; i += stride) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads);
+    for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4f x = reinterpret_cast<const v4f*>(src)[i];
         reinterpret_cast<uint32_t*>(dst)[i] =
                 pack4(quantize_s8(x[0], scale), quantize_s8(x[1], scale), quantize_s8(x[2], scale), quantize_s8(x[3], scale));
@@ -73,8 +73,8 @@ __global__ __launch_bounds__(256) void cvt_f32_s8_kernel(const float* __restrict
 // TypeCvt QuantizedS8 -> Float32: dequantize = float(x) * scale
 __global__ __launch_bounds__(256) void cvt_s8_f32_kernel(const int8_t* __restrict__ src, float* __restrict__ dst,
                                                          uint64_t quads, uint64_t count, float scale) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads; i += stride) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads);
+    for (uint64_t i = run.at; i < run.end; i += run.step) {
         const int w = reinterpret_cast<const int*>(src)[i];
         v4f o;
         o[0] = (float)((w << 24) >> 24) * scale;
@@ -92,7 +92,7 @@ unsigned stream_blocks(uint64_t steps, int cu_count) {
     uint64_t blocks = (steps + 255) / 256;
     const uint64_t cap = (uint64_t)cu_count * 16;
     if (blocks > cap) blocks = cap;
-    return blocks ? (unsigned)blocks : 1u;
+    return blocks ? (unsigned)xcd_grid(blocks) : 1u;
 }
 
 }  // namespace
@@ -118,6 +118,7 @@ int launch_requant8(hipStream_t st, const EpiParams& e, const int8_t* src, const
     const uint64_t cap = (uint64_t)cu_count * 16;
     if (blocks > cap) blocks = cap;
     if (blocks == 0) blocks = 1;
+    blocks = xcd_grid(blocks);
     return launch_kernel(requant8_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, blocks16, count, e);
 }
 
@@ -130,6 +131,7 @@ int launch_requant(hipStream_t st, const EpiParams& e, const int32_t* src, const
     const uint64_t cap = (uint64_t)cu_count * 16;
     if (blocks > cap) blocks = cap;
     if (blocks == 0) blocks = 1;
+    blocks = xcd_grid(blocks);
     return launch_kernel(requant_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, quads, count, e);
 }
 
