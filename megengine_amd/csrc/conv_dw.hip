@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void dw3x3_kernel(Dw3Args a) {
     asm volatile("" ::"s"(a.div_qw.m), "s"(a.div_qw.s1), "s"(a.div_qw.s2), "s"(a.div_ohs.m), "s"(a.div_ohs.s1),
                  "s"(a.div_ohs.s2), "s"(a.div_cg.m), "s"(a.div_cg.s1), "s"(a.div_cg.s2), "s"(a.epi.fast), "s"(a.epi.lin),
                  "s"(a.epi.has_z), "s"(a.epi.nonline), "s"(a.epi.lin_c), "s"(a.epi.lin_d), "s"(a.epi.lin_lo));
-    const uint32_t item = xcd_block() * 256u + threadIdx.x;
+    const uint32_t item = xcd_block() * 64u + threadIdx.x;
     if (item >= a.items) return;
     // item = ((n * CG + cg) * OHS + strip) * QW + quad
     const uint32_t i1 = fdiv(item, a.div_qw), q = item - i1 * a.QW;
@@ -403,10 +403,9 @@ __global__ __launch_bounds__(256) void dw3x3_kernel(Dw3Args a) {
 }
 
 template <int S, int R>
-int launch_dw3(hipStream_t st, dim3 grid, const Dw3Args& b) {
+int launch_dw3(hipStream_t st, dim3 grid, dim3 block, const Dw3Args& b) {
     const bool buf = b.src_bytes != 0 && b.pw <= 1;
     const int epi = !b.epi.fast ? 2 : b.epi.lin ? 0 : (!b.epi.has_z && b.epi.nonline == NL_RELU) ? 1 : 2;
-    const dim3 block(256);
     if (buf) {
         if (epi == 0) return launch_kernel((dw3x3_kernel<S, R, 0, true>), grid, block, 0, st, b);
         if (epi == 1) return launch_kernel((dw3x3_kernel<S, R, 1, true>), grid, block, 0, st, b);
@@ -416,7 +415,7 @@ int launch_dw3(hipStream_t st, dim3 grid, const Dw3Args& b) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// 5x5 and 7x7 with "same" padding (pad_w = F / 2), stride S in {1, 2}: the same work item as above, two output rows.
+// 5x5 and 7x7 with "same" padding (pad_w = F / 2), stride S in {1, 2}: the same work item as above, one or two output rows.
 //
 // A window row is two groups of four taps (the second one filled up with zero weights), so an output costs two dot products
 // per filter row.  Input rows arrive in blocks of four pixels that start at column ow0 * S - 4: a multiple of four, so the
@@ -425,13 +424,14 @@ int launch_dw3(hipStream_t st, dim3 grid, const Dw3Args& b) {
 // windows of the four outputs are byte-aligned pieces of neighbouring blocks (one v_alignbyte each, shared by the two
 // output rows).  What it replaces walks the taps one at a time, four scattered dword loads and sixteen dot products each.
 // 240 channels, 5x5 stride 2 at 57 x 57, batch 16 (16 MB): 22.5 -> 8.6 us; 96 channels, stride 1 at 56 x 56: 36.7 -> 9.2 us.
+// (launch bounds of 256 although workgroups hold one wave: with 64 the compiler spends twice the registers on these kernels)
 // ---------------------------------------------------------------------------------------------
-template <int F, int S>
+template <int F, int S, int R>
 __global__ __launch_bounds__(256) void dwf_kernel(Dw3Args a) {
-    constexpr int R = 2, P = F / 2, ROWS = (R - 1) * S + F;
+    constexpr int P = F / 2, ROWS = (R - 1) * S + F;
     constexpr int FIRST = 4 - P;                       // pixel of the loaded blocks at which output 0's window starts
     constexpr int NB = (FIRST + 3 * S + F + 3) / 4;    // blocks a thread loads per row
-    const uint32_t item = xcd_block() * 256u + threadIdx.x;
+    const uint32_t item = xcd_block() * 64u + threadIdx.x;
     if (item >= a.items) return;
     const uint32_t i1 = fdiv(item, a.div_qw), q = item - i1 * a.QW;
     const uint32_t i2 = fdiv(i1, a.div_ohs), strip = i1 - i2 * a.OHS;
@@ -567,7 +567,16 @@ int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, const int8_t* sr
     const bool wide = sq && (d.fh == 5 || d.fh == 7) && d.pad_w == d.fw / 2;
     const int64_t src_total = (int64_t)(d.n - 1) * p.src_sn + (int64_t)d.ic * d.ih * d.iw;
     if (sq && (d.fh == 3 || (wide && src_total < ((int64_t)1 << 31)))) {
-        const int R = wide ? 2 : d.stride_h == 1 ? (p.oh % 4 == 0 ? 4 : 2) : (p.oh % 2 == 0 ? 2 : 1);
+        // Output rows per thread.  Few work items: one, because a thread's own chain -- its rows' loads, products and stores -- is
+        // all there is to wait for; at stride 2 always, where rows share little.  With enough threads to fill the device two
+        // rows at stride 1 read a third less, and four a sixth less again once there are a million rows of four pixels.
+        // 3x3, us with 1 / 2 / 4 rows: 192 channels at 28 x 28, batch 1: 2.5 / 2.9 / 3.6, batch 16 (150528 rows of four):
+        // 4.0 / 4.1 / 4.1, batch 64: 8.5 / 7.2 / 7.8; 144 at 56 x 56, batch 64: 19.9 / 15.4 / 14.4; stride 2, 192 at 28 x 28,
+        // batch 64: 4.2 / 4.8, 96 at 112 x 112: 16.6 / 16.4.  Planes of few, odd rows leave strips of two half empty: 960 at
+        // 7 x 7, batch 64 (215040): 4.6 / 5.1.
+        const int64_t rows = (int64_t)d.n * a.CG * a.OH * a.QW;
+        const bool few = rows <= (a.OH % 2 && a.OH <= 7 ? 262144 : 131072);
+        const int R = few || (!wide && d.stride_h == 2) ? 1 : !wide && p.oh % 4 == 0 && rows >= 1000000 ? 4 : 2;
         Dw3Args b;
         b.src = src; b.flt = flt; b.bias = bias; b.z = z; b.dst = dst;
         b.CG = a.CG; b.IH = a.IH; b.IW = a.IW; b.OH = a.OH; b.OW = a.OW; b.QW = a.QW; b.OHS = (a.OH + R - 1) / R;
@@ -578,14 +587,18 @@ int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, const int8_t* sr
             b.items = (uint32_t)items;
             b.src_bytes = src_total < ((int64_t)1 << 31) ? (uint32_t)src_total : 0u;
             b.div_qw = make_fastdiv(b.QW); b.div_ohs = make_fastdiv(b.OHS); b.div_cg = make_fastdiv(b.CG);
-            const dim3 grid((unsigned)((items + 255) / 256));
+            // workgroups of one wave: waves share nothing, and a layer of a few hundred of them spreads over as many CUs
+            // (7 x 7 x 960, batch 1: 2.64 us against 2.97 with four waves; batch 64: 4.6 against 4.8)
+            const dim3 grid((unsigned)((items + 63) / 64)), block(64);
             if (wide) {
-                auto kern = d.fh == 5 ? (d.stride_h == 1 ? dwf_kernel<5, 1> : dwf_kernel<5, 2>)
-                                      : (d.stride_h == 1 ? dwf_kernel<7, 1> : dwf_kernel<7, 2>);
-                return launch_kernel(kern, grid, dim3(256), 0, st, b);
+                auto kern = d.fh == 5 ? (d.stride_h == 1 ? (R == 1 ? dwf_kernel<5, 1, 1> : dwf_kernel<5, 1, 2>)
+                                                          : (R == 1 ? dwf_kernel<5, 2, 1> : dwf_kernel<5, 2, 2>))
+                                      : (d.stride_h == 1 ? (R == 1 ? dwf_kernel<7, 1, 1> : dwf_kernel<7, 1, 2>)
+                                                          : (R == 1 ? dwf_kernel<7, 2, 1> : dwf_kernel<7, 2, 2>));
+                return launch_kernel(kern, grid, block, 0, st, b);
             }
-            if (d.stride_h == 1) return R == 4 ? launch_dw3<1, 4>(st, grid, b) : launch_dw3<1, 2>(st, grid, b);
-            return R == 2 ? launch_dw3<2, 2>(st, grid, b) : launch_dw3<2, 1>(st, grid, b);
+            if (d.stride_h == 1) return R == 4 ? launch_dw3<1, 4>(st, grid, block, b) : R == 2 ? launch_dw3<1, 2>(st, grid, block, b) : launch_dw3<1, 1>(st, grid, block, b);
+            return launch_dw3<2, 1>(st, grid, block, b);
         }
     }
     const int quads = a.OH * a.QW;

@@ -34,3 +34,19 @@ def test_other_paddings_and_strides(oracle, f, pad, stride):
 def test_height_padding_may_differ(oracle):
     d = _abi.make_conv_desc("NCHW4", 2, 8, 11, 13, 8, 5, pad=(1, 2), stride=1, group=8, nonline="RELU", **S)
     check_case(oracle, d, seed=6, tag="dw pad_h 1")
+
+
+@pytest.mark.parametrize("n,c,ih,iw,f,stride", [
+    (40, 64, 41, 37, 3, 1),   # two output rows per thread, an odd number of them
+    (40, 64, 41, 37, 5, 1),
+    (40, 64, 81, 73, 5, 2),
+    (41, 64, 43, 33, 7, 1),
+    (64, 96, 44, 59, 3, 1),   # four
+    (40, 64, 81, 75, 3, 2),   # one at any size
+    (64, 640, 7, 7, 3, 1),    # planes of seven rows, around the line between one and two
+    (64, 736, 7, 6, 3, 1),
+])
+def test_rows_per_thread(oracle, n, c, ih, iw, f, stride):
+    for nl, z in (("RELU", False), ("IDENTITY", True)):
+        d = _abi.make_conv_desc("NCHW4", n, c, ih, iw, c, f, pad=f // 2, stride=stride, group=c, nonline=nl, has_z=z, **S)
+        check_case(oracle, d, seed=70 + f, tag="dw rows")
