@@ -76,7 +76,7 @@ __device__ __forceinline__ void p4_epilogue(const P4Args& a, v16i (&acc)[MT][NT]
             }
 }
 
-// STEPS: MFMA steps of a stage when known (9: 3x3 filters, two groups), 0: from the arguments
+// STEPS: MFMA steps of a stage when known (9: nine taps, two channel groups), 0: from the arguments
 template <int MT, int NT, int STEPS>
 __global__ __launch_bounds__(256, 2) void patch4_kernel(P4Args a) {
     constexpr int BM = MT * 32, KAN = (BM + 13) / 14;
@@ -362,7 +362,9 @@ bool p4_plan(const IgemmArgs& a, int cfg, P4Args* k, int* lds_bytes) {
 
 template <int MT, int NT>
 int launch_p4(hipStream_t st, const P4Args& k, int lds) {
-    auto kern = k.GS * k.T == 18 ? patch4_kernel<MT, NT, 9> : patch4_kernel<MT, NT, 0>;
+    // two groups of nine taps, and not one group of eighteen (3x6, 2x9, ...): the stage has as many entries, the filter rows
+    // and the patch of the two differ
+    auto kern = k.GS == 2 && k.T == 9 ? patch4_kernel<MT, NT, 9> : patch4_kernel<MT, NT, 0>;
     static std::atomic<int> max_lds_set{0};
     if (max_lds_set.load(std::memory_order_relaxed) == 0) {
         for (auto f : {patch4_kernel<MT, NT, 9>, patch4_kernel<MT, NT, 0>}) {

@@ -37,3 +37,31 @@ def test_every_tile(oracle, i):
             if check_case(oracle, d, seed=90 + i, algo=IGEMM, tile=t, tag=lib.tile_names()[t]) is not None:
                 ran += 1
     assert ran >= 6
+
+
+# filters that are not square: as many taps as the 3x3 kernel has entries per stage (18: one group of eighteen taps, not two of
+# nine), as many as its taps in another arrangement (9), and windows of a single row or column
+TAPS = [(3, 6), (6, 3), (2, 9), (9, 2), (1, 18), (18, 1), (1, 9), (9, 1), (1, 7), (2, 5)]
+
+
+@pytest.mark.parametrize("ic", [8, 16, 20, 52, 100])
+@pytest.mark.parametrize("fh,fw", TAPS)
+def test_filters_that_are_not_square(oracle, fh, fw, ic):
+    tiles = [t for t, name in enumerate(lib.tile_names()) if name.startswith("patch4_")]
+    ran = 0
+    for oc, stride, z in ((36, 1, True), (68, 2, False)):
+        d = _abi.make_conv_desc("NCHW4", 2, ic, 19, 23, oc, fh, fw, pad=(fh // 2, fw // 2), stride=stride, nonline="RELU", has_z=z, **S)
+        for t in tiles:
+            if check_case(oracle, d, seed=fh * 100 + fw + ic, algo=IGEMM, tile=t, tag=lib.tile_names()[t]) is not None:
+                ran += 1
+    assert ran >= 4
+
+
+@pytest.mark.parametrize("fh,fw", [(3, 6), (9, 2), (1, 9)])
+def test_filters_that_are_not_square_group_by_group(oracle, fh, fw):
+    """Groups of more than sixteen channels run as one dense launch each, on views with the batch strides of the whole."""
+    for t, name in enumerate(lib.tile_names()):
+        if not name.startswith("patch4_"):
+            continue
+        d = _abi.make_conv_desc("NCHW4", 3, 40, 13, 18, 72, fh, fw, pad=(fh // 2, fw // 2), group=2, nonline="RELU", has_z=True, **S)
+        assert check_case(oracle, d, seed=fh + fw, algo=IGEMM, tile=t, tag=name) is not None
