@@ -47,3 +47,29 @@ def test_large_windows(oracle, mode, fmt, c, window, stride, pad, size):
     got = ops.pooling_exec(d, to_dev(x))
     torch.cuda.synchronize()
     assert np.array_equal(got.cpu().numpy(), oracle.pooling(d, x))
+
+
+# Tensors beyond 2 GiB (offsets in 64 bits) and beyond 4 GiB (one thread per byte would be more threads than a launch can
+# number): planes of whole and of broken 16-byte vectors, and planes too small for either kernel of vectors
+@pytest.mark.parametrize("shape", [(9, 64, 2048, 2048), (9, 63, 1999, 2003), (33000, 97, 26, 27), (44000, 1030, 7, 7),
+                                   (17, 64, 2048, 2048)])
+def test_large_tensors(shape):
+    n, c, h, w = shape
+    x = torch.randint(-128, 128, shape, dtype=torch.int8, device="cuda")
+    assert x.numel() >= 1 << 31
+    for to, back, p in ((_abi.RL_NCHW_NCHW4, _abi.RL_NCHW4_NCHW, 4), (_abi.RL_NCHW_NCHW32, _abi.RL_NCHW32_NCHW, 32)):
+        y = ops.relayout_exec(ops.relayout_desc(to, shape), x)
+        assert y.shape == (n, -(-c // p), h, w, p)
+        for lo in range(0, n, max(1, n // 8)):
+            part = y[lo:lo + max(1, n // 8)].permute(0, 1, 4, 2, 3).reshape(-1, y.shape[1] * p, h, w)
+            assert torch.equal(part[:, :c], x[lo:lo + part.shape[0]]), (p, lo)
+            assert not part[:, c:].any(), (p, lo)
+        z = ops.relayout_exec(ops.relayout_desc(back, tuple(y.shape), oc=c), y)
+        assert torch.equal(z, x), p
+        del y, z
+    if c % 32 == 0:
+        y = x.view(n, c // 4, h, w, 4)
+        z = ops.relayout_exec(ops.relayout_desc(_abi.RL_NCHW4_NCHW32, tuple(y.shape)), y)
+        for lo in range(n):
+            assert torch.equal(z[lo].view(c // 32, h * w, 8, 4).permute(0, 2, 1, 3).reshape(c // 4, h, w, 4), y[lo]), lo
+        assert torch.equal(ops.relayout_exec(ops.relayout_desc(_abi.RL_NCHW32_NCHW4, tuple(z.shape)), z), y)
