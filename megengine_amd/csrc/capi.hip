@@ -6,6 +6,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <memory>
 #include <mutex>
 #include <new>
 #include <shared_mutex>
@@ -921,22 +922,29 @@ int mi355_convbias_s8_bind(const mi355_conv_desc* d, const mi355_algo* algo, con
                            size_t workspace_bytes, mi355_bound_call** out) {
     if (!out) return fail(MI355_ERR_BAD_ARG, "null argument");
     *out = nullptr;
-    mi355_bound_call* b = new (std::nothrow) mi355_bound_call;
-    if (!b) return fail(MI355_ERR_BAD_ARG, "out of host memory");
-    t_binding = &b->launches;
-    const int st = preprocessed_bytes
-                           ? mi355_convbias_s8_exec_preprocessed(nullptr, d, algo, src, filter, preprocessed_bytes, bias, z, dst,
-                                                                 workspace, workspace_bytes)
-                           : mi355_convbias_s8_exec(nullptr, d, algo, src, static_cast<const int8_t*>(filter), bias, z, dst,
-                                                    workspace, workspace_bytes);
-    t_binding = nullptr;
-    if (st) {
-        delete b;
-        return st;
+    // Noting the launches down allocates.  However exec is left, the thread stops binding: its later calls would otherwise
+    // be noted down too instead of launched.
+    struct Binding {
+        ~Binding() { t_binding = nullptr; }
+    };
+    try {
+        std::unique_ptr<mi355_bound_call> b(new mi355_bound_call);
+        {
+            const Binding binding;
+            t_binding = &b->launches;
+            const int st = preprocessed_bytes
+                                   ? mi355_convbias_s8_exec_preprocessed(nullptr, d, algo, src, filter, preprocessed_bytes, bias, z,
+                                                                         dst, workspace, workspace_bytes)
+                                   : mi355_convbias_s8_exec(nullptr, d, algo, src, static_cast<const int8_t*>(filter), bias, z, dst,
+                                                            workspace, workspace_bytes);
+            if (st) return st;
+        }
+        b->launches.seal();
+        *out = b.release();
+        return MI355_OK;
+    } catch (const std::bad_alloc&) {
+        return fail(MI355_ERR_BAD_ARG, "out of host memory");
     }
-    b->launches.seal();
-    *out = b;
-    return MI355_OK;
 }
 
 int mi355_bound_call_launch(void* stream, const mi355_bound_call* call) {

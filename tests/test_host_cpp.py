@@ -41,6 +41,17 @@ def test_abi_calls_from_many_threads():
     assert r.returncode == 0 and "ALL OK" in r.stdout, r.stdout[-4000:]
 
 
+def test_bind_without_host_memory():
+    """tests/host/bind_oom.cpp: every allocation of mi355_convbias_s8_bind fails in turn"""
+    _binary(allow_build=True)
+    exe = os.path.join(ROOT, "tests", "host", "bind_oom")
+    if not os.path.exists(exe):
+        subprocess.check_call(["make", "-C", os.path.dirname(exe), "-s", exe])
+    r = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120,
+                       env=dict(os.environ, HIP_VISIBLE_DEVICES="-1"))
+    assert r.returncode == 0 and "ALL OK" in r.stdout, r.stdout[-4000:]
+
+
 @pytest.mark.gpu
 def test_host_classes_gpu():
     """exec of every listed algorithm through the C++ classes, bit-exact against the CPU checker"""
