@@ -133,13 +133,16 @@ at::Tensor empty_like_device(at::IntArrayRef shape, at::ScalarType dt, const at:
     return at::empty(shape, at::TensorOptions().dtype(dt).device(like.device()));
 }
 
-// Runs a C-ABI call without the GIL (a full queue blocks it).
+// Runs a C-ABI call without the GIL (a full queue blocks it).  Taken back also when the call ends in an exception (the host
+// caches behind it allocate), which guarded() then turns into a Python one.
 template <class F>
 int without_gil(F f) {
-    PyThreadState* s = PyEval_SaveThread();
-    const int st = f();
-    PyEval_RestoreThread(s);
-    return st;
+    struct Released {
+        PyThreadState* s = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(s); }
+    };
+    const Released released;
+    return f();
 }
 
 // dst as given, or a new tensor
@@ -482,10 +485,12 @@ PyObject* bound_run(PyObject* self, PyObject* const*, size_t nargsf, PyObject* k
         PyErr_SetObject(g_error, b->error);
         return nullptr;
     }
-    void* stream = b->has_stream ? b->stream : current_stream();
-    const int st = without_gil([&] { return mi355_bound_call_launch(stream, b->call); });
-    if (st) return raise_status(st);
-    Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        void* stream = b->has_stream ? b->stream : current_stream();
+        const int st = without_gil([&] { return mi355_bound_call_launch(stream, b->call); });
+        if (st) return raise_status(st);
+        Py_RETURN_NONE;
+    });
 }
 
 void bound_dealloc(PyObject* self) {
