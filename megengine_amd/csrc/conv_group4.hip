@@ -1,4 +1,5 @@
-// NCHW4 group convolutions with few channels per group, in one launch (tile "grp4_dot4").
+// NCHW4 group convolutions with few channels per group, in one launch (tile "grp4_dot4": dot products in general, the matrix
+// cores for the usual grouped bottleneck).
 //
 // Such a layer is G small convolutions.  As G launches of the dense tiles it costs G launch latencies, and a matrix tile of
 // 32 channels is mostly empty when a group has 4, 8 or 16: 32 groups of 4 channels, 3x3 at 56 x 56, batch 16, took 165 us.
@@ -260,6 +261,34 @@ int launch_g16(hipStream_t st, const ConvProblem& p, const int8_t* src, const in
 }
 
 }  // namespace
+
+// Whether one launch is ahead of a dense launch per group.  The matrix form always is (165 sizes of 2 to 64 groups, batch 1 to
+// 64, 7 x 7 to 112 x 112), and 3x3 dot products at stride 2 almost always.  The others lose where a group is large -- the
+// dense patch tiles run on the matrix cores -- or has many taps: without the unrolled 3x3 form a thread loads and waits for
+// one tap after the other.  The two sides in us, fitted to graph replays of 1775 sizes of 4 to 16 channels into a group and
+// 4 to 128 out of it, filters 1x1 to 7x7, 1x7 and 3x6, with outputs, dot products and matrix steps in millions:
+//   one launch      3x3: 4 + 0.5 outputs + 0.04 dot products
+//                   others: 3 + 0.145 per tap and channel block (in a row, for any size) + 1 outputs + 0.22 dot products
+//   each group      3.6 + 0.05 matrix steps (pixels x taps x output channels in 32s x input channels in 16s)
+//   all groups      0.1 outputs, with a residual 0.5
+// One launch is kept up to a quarter more, which G submissions cost the host.  Of the 1775, 422 go group by group for it, one
+// launch against those: 2.7 times faster on average (2 groups 16 -> 116, 7x7 at 33 x 39, batch 51: 590 us / 46; 4 groups 16 ->
+// 120, 3x3 at 90 x 67, batch 38: 173 / 81; 6 groups 16 -> 76, 7x7 at 8 x 14, batch 12: 77 / 29; 3 groups 12 -> 100, 1x1 at 57 x
+// 79, batch 44: 114 / 42), none of them more than a quarter slower; of what stays, 26 are behind by more than that, at most by
+// 2.2 times (34 groups 8 -> 108, 7x7 stride 2 at 31 x 8).  On 250 other sizes 44 change sides and are 2.2 times faster on average.
+bool grp4_pick(const ConvProblem& p) {
+    const mi355_conv_desc& d = p.d;
+    if (!grp4_usable(p)) return false;
+    if (g16_usable(p)) return true;
+    const bool f3 = d.fh == 3 && d.fw == 3 && d.stride_h == d.stride_w;
+    if (f3 && d.stride_h == 2) return true;
+    const double pixels = (double)d.n * p.oh * p.ow * 1e-6, outputs = pixels * d.oc;
+    const double taps = (double)d.fh * d.fw, serial = taps * (p.icpg / 4), dots = outputs * serial;
+    const double steps = pixels * taps * ((p.ocpg + 31) / 32 * 32) * ((p.icpg + 15) / 16);
+    const double one = f3 && d.stride_h == 1 ? 4 + 0.5 * outputs + 0.04 * dots : 3 + 0.145 * serial + outputs + 0.22 * dots;
+    const double groups = d.group * (3.6 + 0.05 * steps) + (d.has_z ? 0.5 : 0.1) * outputs;
+    return one <= 1.25 * groups;
+}
 
 bool grp4_usable(const ConvProblem& p) {
     const mi355_conv_desc& d = p.d;

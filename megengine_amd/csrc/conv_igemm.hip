@@ -777,9 +777,9 @@ int launch_igemm_preprocess(hipStream_t st, const ConvProblem& p, const int8_t* 
 
 // The chooser's tile, as the launch code will run it: what query() hands out names the kernel that executes.
 int igemm_pick_cfg(const ConvProblem& p, int cu_count, bool will_preprocess) {
-    // few channels per group: one launch for all groups, always (32 groups of 4 channels, 3x3 at 56 x 56, batch 16: 165 us as
-    // 32 launches; two groups of 16 at 7 x 7: two launches cost more than one, whatever runs in them)
-    if (igemm_group_by_launch(p) && grp4_usable(p)) return igemm_grp4_cfg();
+    // few channels per group: one launch for all groups (32 groups of 4 channels, 3x3 at 56 x 56, batch 16: 165 us as 32
+    // launches), unless the groups are worth a launch each
+    if (igemm_group_by_launch(p) && grp4_pick(p)) return igemm_grp4_cfg();
     if (igemm_group_by_launch(p)) return igemm_pick_cfg(igemm_group_view(p), cu_count, will_preprocess);
     const int c = pick_cfg_by_shape(p, cu_count, will_preprocess);
     const int r = igemm_resolve_cfg(p, c);

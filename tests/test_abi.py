@@ -213,3 +213,20 @@ def test_plain_nchw_reports_a_workspace():
     d = _abi.make_conv_desc("NCHW", 2, 64, 14, 14, 128, 3, pad=1, group=2, scale_bias=2e-4, scale_dst=0.05)
     assert ops.conv_bias_query(d)[0].id == nchw
     assert lib.lib().mi355_convbias_algo_usable(C.byref(_abi.make_conv_desc("NCHW32", 2, 64, 14, 14, 128, 1)), nchw) == _abi.ERR_ALGO
+
+
+def test_groups_that_are_worth_a_launch_each():
+    """NCHW4 groups of at most 16 input channels run in one launch (tile grp4_dot4) only while their products are small:
+    dot products against matrix tiles, taps one after the other against a patch in LDS."""
+    names = lib.tile_names()
+
+    def tile(n, group, icpg, ocpg, hw, f, **kw):
+        d = _abi.make_conv_desc("NCHW4", n, group * icpg, hw, hw, group * ocpg, f, pad=f // 2, group=group, scale_bias=2e-4, scale_dst=0.05, **kw)
+        return names[ops.conv_bias_query(d)[0].tile_cfg]
+
+    assert tile(64, 2, 16, 128, 56, 3).startswith("patch4_")
+    assert tile(51, 2, 12, 116, 36, 7).startswith("patch4_")
+    assert tile(12, 6, 16, 76, 12, 7) != "grp4_dot4"
+    assert tile(44, 3, 12, 100, 68, 1).startswith("pw4_")
+    for args in ((16, 32, 4, 4, 56, 3), (64, 32, 16, 16, 56, 3), (64, 2, 16, 16, 112, 3), (1, 4, 16, 8, 6, 5), (1, 2, 4, 8, 9, 3), (8, 16, 8, 16, 28, 3)):
+        assert tile(*args) == "grp4_dot4", args

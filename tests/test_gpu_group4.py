@@ -54,3 +54,22 @@ def test_wide_groups_keep_a_launch_of_matrix_tiles_each():
     d = _abi.make_conv_desc("NCHW4", 1, 64, 8, 8, 64, 3, pad=1, group=2, **S)
     algo, _ = ops.conv_bias_query(d)
     assert algo.id == IGEMM and lib.tile_names()[algo.tile_cfg] != "grp4_dot4"
+
+
+@pytest.mark.parametrize("case", [(1, 2, 16, 32, 20, 20, (7, 7), 1), (3, 2, 16, 20, 19, 33, (5, 5), 2), (6, 2, 8, 36, 30, 36, (3, 6), 1),
+                                  (2, 2, 16, 8, 40, 11, (18, 1), 1)])
+def test_groups_with_many_taps_run_group_by_group(oracle, case):
+    """Where the default is a dense launch per group: its results, residuals and batch strides."""
+    n, g, icpg, ocpg, ih, iw, f, stride = case
+    names = lib.tile_names()
+    for nl, z in (("RELU", True), ("IDENTITY", False), ("H_SWISH", True)):
+        kw = dict(pad=(f[0] // 2, f[1] // 2), stride=stride, group=g, nonline=nl, has_z=z, **S)
+        d = _abi.make_conv_desc("NCHW4", n, g * icpg, ih, iw, g * ocpg, *f, **kw)
+        algo, _ = ops.conv_bias_query(d)
+        assert algo.id == IGEMM and names[algo.tile_cfg] != "grp4_dot4"
+        check_case(oracle, d, seed=60 + icpg, tag="default " + names[algo.tile_cfg])
+        check_case(oracle, d, seed=60 + icpg, algo=IGEMM, tile=names.index("grp4_dot4"), tag="one launch")
+        ss, _, _, ds = _abi.conv_shapes(d)
+        d = _abi.make_conv_desc("NCHW4", n, g * icpg, ih, iw, g * ocpg, *f, src_stride_n=int(np.prod(ss[1:])) + 32,
+                                dst_stride_n=int(np.prod(ds[1:])) + 16, z_stride_n=int(np.prod(ds[1:])) + 48, **kw)
+        check_case(oracle, d, seed=80 + icpg, tag="default strided")
