@@ -572,16 +572,22 @@ bool algo_usable(const ConvProblem& p, int id) {
 
 // Heuristic order (cf. the reference's per-backend get_algorithm_heuristic, e.g.
 // dnn/src/cuda/conv_bias/opr_impl.cpp:44-238): channel-wise kernel, the 4-channel first-layer kernel,
-// then the MFMA implicit GEMM, then the generic direct kernel.  Plain NCHW takes the relayout + MFMA algorithm once
-// the problem is large enough to pay for its five extra launches (the generic kernel runs ~4 M multiply-adds in the time
-// those take); workspace_limit is get_algorithm_heuristic's (dnn/include/megdnn/oprs/base.h:595-614).
-int pick_algo(const ConvProblem& p, size_t workspace_limit = SIZE_MAX) {
+// then the MFMA implicit GEMM, then the generic direct kernel.  workspace, bytes: what the caller brought (the workspace
+// limit of get_algorithm_heuristic, dnn/include/megdnn/oprs/base.h:595-614).
+// Plain NCHW takes its MFMA algorithm, a packing launch ahead of the convolution, from 2^22 multiply-adds on.  The line is
+// not where the two meet: graph replays of 500 sizes of 2^13 to 2^25 multiply-adds put the generic kernel, whose threads walk
+// their reductions alone, at 13 to 183 us and this one at 6 to 8, and reductions of 32 and more ahead of it from 2^16 on.  It
+// is the line below which a call needs no workspace, which callers may rely on.
+constexpr uint64_t kNchwMfmaMacs = 1ull << 22;
+int pick_algo(const ConvProblem& p, const void* workspace, size_t bytes) {
     if (depthwise_usable(p)) return ALGO_DEPTHWISE;
     if (c4_usable(p)) return ALGO_C4_MFMA;
     if (igemm_usable(p)) return ALGO_IGEMM_MFMA;
     if (p.d.format == MI355_FMT_NCHW) {
         const uint64_t macs = (uint64_t)p.d.n * p.d.oc * p.oh * p.ow * p.icpg * p.d.fh * p.d.fw;
-        if (macs >= (1ull << 22) && nchw_mfma_usable(p) && nchw_mfma_workspace(p) <= workspace_limit) return ALGO_NCHW_MFMA;
+        // (a misaligned workspace of the reported size is an error of exec, not a reason to pass the algorithm by)
+        const bool al = (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
+        if (macs >= kNchwMfmaMacs && nchw_mfma_usable(p) && (al ? nchw_mfma_workspace_used(p) : nchw_mfma_workspace(p)) <= bytes) return ALGO_NCHW_MFMA;
     }
     return ALGO_DIRECT;
 }
@@ -685,7 +691,7 @@ int mi355_convbias_s8_query(const mi355_conv_desc* d, int algo_request, mi355_al
         const int cu = cu_count();
         if (!m->have_heuristic[pre] || m->heuristic_cu[pre] != cu) {
             mi355_algo& a = m->heuristic[pre];
-            a.id = pick_algo(p);
+            a.id = pick_algo(p, nullptr, SIZE_MAX);
             a.tile_cfg = a.id == ALGO_IGEMM_MFMA ? igemm_pick_cfg(p, cu, pre) : 0;
             // an algorithm the heuristic chose may be replaced by the generic kernel at exec time (misaligned tensors);
             // one the caller asked for by id may not
@@ -723,8 +729,9 @@ static int exec_impl(void* stream, const mi355_conv_desc* d, const mi355_algo* a
     if (d->has_z && !z) return fail(MI355_ERR_BAD_ARG, "has_z set but z is null");
     int id = algo ? algo->id : MI355_ALGO_HEURISTIC;
     int cfg = algo ? algo->tile_cfg : -1;
-    if (id == MI355_ALGO_HEURISTIC) {
-        id = pick_algo(p, workspace ? workspace_bytes : 0);  // whatever fits the workspace the caller brought
+    const bool own_choice = id == MI355_ALGO_HEURISTIC;
+    if (own_choice) {
+        id = pick_algo(p, workspace, workspace ? workspace_bytes : 0);  // whatever fits the workspace the caller brought
         cfg = -1;
     }
     // the heuristic's own answer for this descriptor: usable, resolved to the tile that runs, its workspace known
@@ -738,7 +745,7 @@ static int exec_impl(void* stream, const mi355_conv_desc* d, const mi355_algo* a
     if (!known) {
         if (id < 0 || id >= ALGO_COUNT) return fail(MI355_ERR_ALGO, "unknown algorithm id %d", id);
         if (!algo_usable(p, id)) return fail(MI355_ERR_ALGO, "%s cannot run this problem", kAlgoNames[id]);
-        ws_need = algo_workspace(p, id);
+        ws_need = own_choice && id == ALGO_NCHW_MFMA ? nchw_mfma_workspace_used(p) : algo_workspace(p, id);
     }
     // check_exec's workspace rule (dnn/src/common/conv_bias.cpp:32-37)
     if (ws_need) {

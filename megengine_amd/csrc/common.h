@@ -73,9 +73,11 @@ bool c4_usable(const ConvProblem& p);
 int launch_conv_c4(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt,
                    const int32_t* bias, const int8_t* z, int8_t* dst);
 
-// plain NCHW through the caller's workspace (conv_nchw.hip); nchw_mfma_workspace is 0 when the algorithm cannot run
+// plain NCHW through the caller's workspace (conv_nchw.hip): the size reported for it and the part that is written, 0 when
+// the algorithm cannot run
 bool nchw_mfma_usable(const ConvProblem& p);
 size_t nchw_mfma_workspace(const ConvProblem& p);
+size_t nchw_mfma_workspace_used(const ConvProblem& p);
 int launch_conv_nchw_mfma(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt,
                           const int32_t* bias, const int8_t* z, int8_t* dst, void* workspace);
 

@@ -26,7 +26,8 @@ size_t up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 
 struct NchwLayout {
     int pack;                       // channel pack of the inner problem
-    size_t off_flt, total;          // (src stands at the front)
+    size_t off_flt, used;           // (src stands at the front)
+    size_t reported;                // what query answers
     ConvProblem inner;              // packed src and filter, planar bias, z and dst
 };
 
@@ -42,17 +43,19 @@ bool make_layout(const ConvProblem& p, NchwLayout* L) {
     const int64_t src_img = (int64_t)d.ic * d.ih * d.iw, dst_img = (int64_t)d.oc * p.oh * p.ow;
     if (p.src_sn != src_img || p.dst_sn != dst_img || (d.has_z && p.z_sn != dst_img)) return false;
     if (d.n > 65535) return false;
-    // The size reported for the workspace is what callers have planned memory with: that of src, filter, dst, z and bias all
-    // packed by 32.  The first two are what is used.
+    // The size that query reports, and that exec asks of a caller who names this algorithm, is part of the interface and fixed
+    // by its tests: src, filter, dst, z and bias all packed by 32, the tensors this algorithm once kept.  The first two, `used`,
+    // are what it writes, and what an exec that chooses for itself goes by.
     const uint32_t ic32 = (d.ic + 31) / 32 * 32, oc32 = (d.oc + 31) / 32 * 32;
     const size_t src32 = (size_t)d.n * ic32 * d.ih * d.iw, dst32 = (size_t)d.n * oc32 * p.oh * p.ow;
-    L->total = up(src32) + up((size_t)oc32 * (ic32 / d.group) * d.fh * d.fw) + up(dst32) + (d.has_z ? up(dst32) : 0) +
+    L->reported = up(src32) + up((size_t)oc32 * (ic32 / d.group) * d.fh * d.fw) + up(dst32) + (d.has_z ? up(dst32) : 0) +
                (d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL && oc32 != d.oc ? up((size_t)oc32 * 4) : 0);
     // up to 16 channels a block of 32 would be half and more padding
     L->pack = d.ic <= 16 ? 4 : 32;
     const uint32_t icp = (d.ic + L->pack - 1) / L->pack * L->pack;
     if ((uint64_t)d.n * icp * d.ih * d.iw >= (1ull << 31) || (uint64_t)d.oc * (icp / d.group) * d.fh * d.fw >= (1ull << 31)) return false;
     L->off_flt = up((size_t)d.n * icp * d.ih * d.iw);
+    L->used = L->off_flt + up((size_t)d.oc * (icp / d.group) * d.fh * d.fw);
     ConvProblem& q = L->inner;
     q = p;
     q.d.format = L->pack == 4 ? FMT_INNER_NCHW4_NCHW : FMT_INNER_NCHW32_NCHW;
@@ -118,7 +121,12 @@ bool nchw_mfma_usable(const ConvProblem& p) {
 
 size_t nchw_mfma_workspace(const ConvProblem& p) {
     NchwLayout L;
-    return make_layout(p, &L) ? L.total : 0;
+    return make_layout(p, &L) ? L.reported : 0;
+}
+
+size_t nchw_mfma_workspace_used(const ConvProblem& p) {
+    NchwLayout L;
+    return make_layout(p, &L) ? L.used : 0;
 }
 
 int launch_conv_nchw_mfma(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt,

@@ -85,3 +85,26 @@ def test_static_workspace_exec_refuses_what_does_not_fit():
     assert "static workspace" in lib.lib().mi355_last_error().decode()
     torch.cuda.synchronize()
     assert int((dst != 77).sum()) == 0
+
+
+def test_exec_that_chooses_for_itself_goes_by_what_is_written():
+    """Without an algorithm, a workspace that holds the packed src and filter is enough for the plain-NCHW algorithm, although
+    query reports more and exec asks a caller who names it for that; with less the generic kernel leaves it alone."""
+    L, names = lib.lib(), lib.algo_names()
+    up = lambda x: (x + 255) // 256 * 256
+    d = _abi.make_conv_desc("NCHW", 4, 24, 28, 28, 40, 3, pad=1, nonline="RELU", has_z=True, **S)
+    used = up(4 * 32 * 28 * 28) + up(40 * 32 * 9)
+    t = [torch.from_numpy(x).cuda() for x in util.make_tensors(d, seed=5)]
+    algo, ws = ops.conv_bias_query(d)
+    assert names[algo.id] == "MI355_NCHW_RELAYOUT_MFMA_I8" and ws > used
+    want = ops.conv_bias_exec(d, *t)
+    for size, shift, written in ((used, 0, True), (used - 1, 0, False), (ws - 16, 4, False)):
+        buf = torch.full((used + ws + 256,), 113, dtype=torch.uint8, device="cuda")
+        dst = torch.zeros_like(want)
+        args = [ops._ptr(x) for x in t] + [ops._ptr(dst), ops._ptr(buf[shift:]), size]
+        assert L.mi355_convbias_s8_exec(ops._stream(), d, None, *args) == 0, L.mi355_last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(dst, want)
+        assert bool((buf != 113).any()) == written
+        assert bool((buf[shift + size:] == 113).all())
+        assert L.mi355_convbias_s8_exec(ops._stream(), d, algo, *args) == _abi.ERR_WORKSPACE
