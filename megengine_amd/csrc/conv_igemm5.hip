@@ -6,7 +6,7 @@
 // chain of LDS stages (copy, barrier, multiply) as long as the reduction -- 3x3 over 512 channels at 7 x 7 took 11 us on
 // 16 workgroups, 36 stages of 0.3 us each, whatever the tile.  What bounds such a layer is latency, so this kernel has
 // next to none of its own:
-//   * tile = 16 to 64 channels x 16 to 64 pixels, so that the tiles of a layer reach more of the 256 CUs;
+//   * tile = 16 to 64 channels x 16 or 32 pixels, so that the tiles of a layer reach more of the 256 CUs;
 //   * the waves of a workgroup take contiguous pieces of the reduction.  An MFMA operand of a 32-byte k-chunk is one
 //     16-byte load per lane (32 filter rows, or 32 pixels of a 32-packed tensor: one contiguous kilobyte); a wave keeps
 //     several chunks of both operands in flight, sixteen waves therefore most of the tile's operands, and memory is
@@ -26,7 +26,7 @@ namespace mi355 {
 namespace {
 
 // MFMA steps whose operands a wave keeps in flight
-constexpr int ks_ahead(int s, int mt, int nt) { return s == 16 ? 6 : mt * nt == 1 ? 8 : 4; }
+constexpr int ks_ahead(int s, int mt) { return s == 16 ? 6 : mt == 1 ? 8 : 4; }
 // 16-byte vectors between the rows of partial sums in LDS (a row: 4 channels of the S pixels of a block): both ways of
 // reading them back -- a row by consecutive lanes, or all rows of a pixel by consecutive lanes -- then meet every bank once
 // per pass
@@ -70,14 +70,13 @@ struct KsAcc<16> {
     __device__ __forceinline__ v4i quad(int) const { return v; }  // channels 4 (lane / 16) .. + 3
 };
 
-template <int PIN, int S, int MT, int NT, bool PW>
-__global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
-    constexpr int BL = MT * NT;           // S x S blocks of the tile
+template <int PIN, int S, int MT, bool PW>
+__global__ __launch_bounds__(MT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
     constexpr int ROWS = S / 4;           // channel quads of a block
     constexpr int PARTS = S == 32 ? 4 : 1;  // a block's quads over its pixels, 64 at a time
-    constexpr int ROWP = ks_row(S), WP = BL * ROWS * ROWP;  // vectors per row, per wave
+    constexpr int ROWP = ks_row(S), WP = MT * ROWS * ROWP;  // vectors per row, per wave
     constexpr int CH = S == 32 ? 1 : 2;   // 32-byte chunks per step
-    constexpr int AHEAD = ks_ahead(S, MT, NT);
+    constexpr int AHEAD = ks_ahead(S, MT);
     extern __shared__ __attribute__((aligned(16))) v4i red[];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), W = blockDim.x >> 6;
     const int ls = lane & (S - 1), lk = lane / S;
@@ -99,7 +98,7 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
             if (tn >= a.tiles_n) return;
         }
     }
-    const int oc0 = tm * MT * S, px0 = tn * NT * S;
+    const int oc0 = tm * MT * S, px0 = tn * S;
     const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes);
     const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, a.flt_bytes);
 
@@ -123,18 +122,17 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
         const int row = oc0 + i * S + ls;
         arow[i] = row < a.OC ? row * a.flt_rstride + (S == 32 ? lk * 16 : (lk >> 1) * a.flt_kstride + (lk & 1) * 16) : SENT;
     }
-    int pix[NT], ih0[NT], iw0[NT];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const int m = px0 + j * S + ls;
+    int pix, ih0, iw0;
+    {
+        const int m = px0 + ls;
         const bool ok = m < a.M;
         const uint32_t mm = ok ? m : 0;
         const uint32_t n = fdiv(mm, a.div_ohw), rem = mm - n * a.OHW;
         const uint32_t oh = fdiv(rem, a.div_ow), ow = rem - oh * a.OW;
-        ih0[j] = ok ? (int)oh * a.sh - a.ph : -0x10000;  // no tap of a pixel past the last one lies inside
-        iw0[j] = (int)ow * a.sw - a.pw;
-        pix[j] = (int)n * a.src_sn + ((int)oh * a.sh - a.ph) * a.IW * PIN + iw0[j] * PIN + (PIN == 32 ? (lk & 1) * 16 : 0);
-        if (PW && !ok) pix[j] = SENT;
+        ih0 = ok ? (int)oh * a.sh - a.ph : -0x10000;  // no tap of a pixel past the last one lies inside
+        iw0 = (int)ow * a.sw - a.pw;
+        pix = (int)n * a.src_sn + ((int)oh * a.sh - a.ph) * a.IW * PIN + iw0 * PIN + (PIN == 32 ? (lk & 1) * 16 : 0);
+        if (PW && !ok) pix = SENT;
     }
     if (PIN == 4 && !PW) __syncthreads();
 
@@ -150,7 +148,7 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
     // Operands of the next step.  Past the wave's piece every lane is out of the buffers' range: zeros, no memory access
     // (an unconditional load keeps the number of loads in flight known to the compiler, and with it the waits short).
     // A 4-packed row may end inside its last chunk, so there the whole offset stands where the descriptor checks it.
-    auto load = [&](v4i (&fa)[MT], v4i (&fb)[NT]) __attribute__((always_inline)) {
+    auto load = [&](v4i (&fa)[MT], v4i& fb) __attribute__((always_inline)) {
         const bool in = kc < k1;
         const int kf = kc * CH * a.flt_kstride;
         const bool half_in = S == 32 || kc * 2 + (lk >> 1) < a.KC;  // an odd number of chunks: no second one in the last step
@@ -159,30 +157,27 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
             const bool ok = in && half_in && arow[i] != SENT;
             fa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, ok ? arow[i] + kf : SENT, 0, 0);
         }
+        if (PIN == 32 && PW) {
+            const int c = S == 32 ? 0 : (lk >> 1) * a.src_scb;
+            fb = __builtin_amdgcn_raw_buffer_load_b128(rs_src, in && half_in && pix != SENT ? pix + c : SENT, kc * CH * a.src_scb, 0);
+        } else if (PIN == 32 && S == 32) {
+            const bool ok = in && (unsigned)(ih0 + fh) < (unsigned)a.IH && (unsigned)(iw0 + fw) < (unsigned)a.IW;
+            fb = __builtin_amdgcn_raw_buffer_load_b128(rs_src, ok ? pix + (fh * a.IW + fw) * 32 : SENT, cb * a.src_scb, 0);
+        } else if (PIN == 32) {
+            const uint32_t c = kc * 2 + (lk >> 1), b = fdiv(c, a.div_t), tap = c - b * a.T, h = fdiv(tap, a.div_fw), w = tap - h * a.FW;
+            const bool ok = in && half_in && (unsigned)(ih0 + (int)h) < (unsigned)a.IH && (unsigned)(iw0 + (int)w) < (unsigned)a.IW;
+            fb = __builtin_amdgcn_raw_buffer_load_b128(rs_src, ok ? pix + ((int)h * a.IW + (int)w) * 32 + (int)b * a.src_scb : SENT, 0, 0);
+        } else {
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            if (PIN == 32 && PW) {
-                const int c = S == 32 ? 0 : (lk >> 1) * a.src_scb;
-                fb[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, in && half_in && pix[j] != SENT ? pix[j] + c : SENT, kc * CH * a.src_scb, 0);
-            } else if (PIN == 32 && S == 32) {
-                const bool ok = in && (unsigned)(ih0[j] + fh) < (unsigned)a.IH && (unsigned)(iw0[j] + fw) < (unsigned)a.IW;
-                fb[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, ok ? pix[j] + (fh * a.IW + fw) * 32 : SENT, cb * a.src_scb, 0);
-            } else if (PIN == 32) {
-                const uint32_t c = kc * 2 + (lk >> 1), b = fdiv(c, a.div_t), tap = c - b * a.T, h = fdiv(tap, a.div_fw), w = tap - h * a.FW;
-                const bool ok = in && half_in && (unsigned)(ih0[j] + (int)h) < (unsigned)a.IH && (unsigned)(iw0[j] + (int)w) < (unsigned)a.IW;
-                fb[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, ok ? pix[j] + ((int)h * a.IW + (int)w) * 32 + (int)b * a.src_scb : SENT, 0, 0);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int u = kc * CH * 8 + lk * 4 + i;
-                    if (PW) {
-                        fb[j][i] = __builtin_amdgcn_raw_buffer_load_b32(rs_src, in && u < a.entries && pix[j] != SENT ? pix[j] + u * a.src_scb : SENT, 0, 0);
-                    } else {
-                        const KEntry e = tab[in ? u : 0];
-                        const bool ok = in && (unsigned)(ih0[j] + (e.fhfw & 0xffff)) < (unsigned)a.IH &&
-                                        (unsigned)(iw0[j] + (e.fhfw >> 16)) < (unsigned)a.IW;
-                        fb[j][i] = __builtin_amdgcn_raw_buffer_load_b32(rs_src, ok ? pix[j] + e.off : SENT, 0, 0);
-                    }
+            for (int i = 0; i < 4; ++i) {
+                const int u = kc * CH * 8 + lk * 4 + i;
+                if (PW) {
+                    fb[i] = __builtin_amdgcn_raw_buffer_load_b32(rs_src, in && u < a.entries && pix != SENT ? pix + u * a.src_scb : SENT, 0, 0);
+                } else {
+                    const KEntry e = tab[in ? u : 0];
+                    const bool ok = in && (unsigned)(ih0 + (e.fhfw & 0xffff)) < (unsigned)a.IH &&
+                                    (unsigned)(iw0 + (e.fhfw >> 16)) < (unsigned)a.IW;
+                    fb[i] = __builtin_amdgcn_raw_buffer_load_b32(rs_src, ok ? pix + e.off : SENT, 0, 0);
                 }
             }
         }
@@ -198,11 +193,9 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
         }
     };
 
-    KsAcc<S> acc[MT][NT];
+    KsAcc<S> acc[MT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j].clear();
+    for (int i = 0; i < MT; ++i) acc[i].clear();
 
     // The partial sums of a block are dealt out over the waves in parts of 64 quads: by rows where the destination keeps
     // four channels of a pixel together (consecutive pixels are contiguous), by pixels where it keeps 32.
@@ -213,11 +206,11 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
     v4i bv = {0, 0, 0, 0};
     uint32_t zw = 0;
     auto fetch = [&](int u) __attribute__((always_inline)) {
-        const int blk = u / PARTS, part = u % PARTS, i = blk / NT, j = blk % NT;
+        const int i = u / PARTS, part = u % PARTS;
         const int row = a.log_pout == 5 ? lane % ROWS : part * (64 / S) + lk;  // channels 4 row .. + 3 of the block
         const int px = a.log_pout == 5 ? part * (64 / ROWS) + lane / ROWS : ls;
-        at_red = (blk * ROWS + row) * ROWP + px;
-        const int oc4 = oc0 + i * S + row * 4, m = px0 + j * S + px;
+        at_red = (i * ROWS + row) * ROWP + px;
+        const int oc4 = oc0 + i * S + row * 4, m = px0 + px;
         const bool ok = m < a.M && oc4 < a.OC;
         const uint32_t mm = m < a.M ? m : 0;
         const uint32_t n = fdiv(mm, a.div_ohw), rem = mm - n * a.OHW;
@@ -237,14 +230,12 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
     };
 
     if (k0 < k1) {  // (waves beyond the number of steps have nothing to add)
-        v4i fa[AHEAD][MT], fb[AHEAD][NT];
+        v4i fa[AHEAD][MT], fb[AHEAD];
 #pragma unroll
         for (int g = 0; g < AHEAD; ++g) load(fa[g], fb[g]);
         auto multiply = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j].mfma(fa[g][i], fb[g][j]);
+            for (int i = 0; i < MT; ++i) acc[i].mfma(fa[g][i], fb[g]);
         };
         int left = k1 - k0;
         for (; left > AHEAD; left -= AHEAD) {
@@ -261,13 +252,10 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int q = 0; q < PARTS; ++q)
-                red[wave * WP + ((i * NT + j) * ROWS + q * (64 / S) + lk) * ROWP + ls] = acc[i][j].quad(q);
-    if (wave < BL * PARTS) fetch(wave);  // lands while the partial sums meet
+        for (int q = 0; q < PARTS; ++q) red[wave * WP + (i * ROWS + q * (64 / S) + lk) * ROWP + ls] = acc[i].quad(q);
+    if (wave < MT * PARTS) fetch(wave);  // lands while the partial sums meet
     __syncthreads();
-    for (int u = wave; u < BL * PARTS; u += W) {
+    for (int u = wave; u < MT * PARTS; u += W) {
         if (u != wave) fetch(u);
         v4i s = bv;
 #pragma unroll 4
@@ -295,23 +283,23 @@ __global__ __launch_bounds__(MT* NT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) 
 }
 
 struct KsCfg {
-    int pin, s, mt, nt, waves;
+    int pin, s, mt, waves;
     const char* name;
 };
 constexpr KsCfg kKs[] = {
-        {32, 16, 1, 1, 8, "v2_ks_16x16w8"}, {32, 16, 1, 1, 4, "v2_ks_16x16w4"}, {32, 32, 1, 1, 8, "v2_ks_32x32w8"},
-        {32, 32, 1, 1, 4, "v2_ks_32x32w4"}, {32, 32, 2, 1, 8, "v2_ks_64x32w8"}, {32, 32, 2, 1, 4, "v2_ks_64x32w4"},
-        {4, 16, 1, 1, 8, "ks4_16x16w8"},    {4, 16, 1, 1, 4, "ks4_16x16w4"},    {4, 32, 1, 1, 8, "ks4_32x32w8"},
-        {4, 32, 1, 1, 4, "ks4_32x32w4"},    {4, 32, 2, 1, 8, "ks4_64x32w8"},    {4, 32, 2, 1, 4, "ks4_64x32w4"}};
+        {32, 16, 1, 8, "v2_ks_16x16w8"}, {32, 16, 1, 4, "v2_ks_16x16w4"}, {32, 32, 1, 8, "v2_ks_32x32w8"},
+        {32, 32, 1, 4, "v2_ks_32x32w4"}, {32, 32, 2, 8, "v2_ks_64x32w8"}, {32, 32, 2, 4, "v2_ks_64x32w4"},
+        {4, 16, 1, 8, "ks4_16x16w8"},    {4, 16, 1, 4, "ks4_16x16w4"},    {4, 32, 1, 8, "ks4_32x32w8"},
+        {4, 32, 1, 4, "ks4_32x32w4"},    {4, 32, 2, 8, "ks4_64x32w8"},    {4, 32, 2, 4, "ks4_64x32w4"}};
 constexpr int kKsCount = sizeof(kKs) / sizeof(kKs[0]);
 
 int ks_lds(const IgemmArgs& a, const KsCfg& c, bool pw) {
-    return c.waves * c.mt * c.nt * (c.s / 4) * ks_row(c.s) * 16 + (c.pin == 4 && !pw ? (a.KC + 1) * 8 * 8 : 0);
+    return c.waves * c.mt * (c.s / 4) * ks_row(c.s) * 16 + (c.pin == 4 && !pw ? (a.KC + 1) * 8 * 8 : 0);
 }
 
-template <int PIN, int S, int MT, int NT, bool PW>
+template <int PIN, int S, int MT, bool PW>
 int launch_ks(hipStream_t st, const KsArgs& k, int waves, int lds) {
-    auto kern = ks_kernel<PIN, S, MT, NT, PW>;
+    auto kern = ks_kernel<PIN, S, MT, PW>;
     static std::atomic<int> max_lds_set{0};
     if (lds > max_lds_set.load(std::memory_order_relaxed)) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -389,7 +377,7 @@ int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg
     k.src_sn = a.src_sn; k.src_scb = a.src_scb; k.dst_sn = a.dst_sn; k.dst_scb = a.dst_scb; k.z_sn = a.z_sn;
     k.flt_rstride = a.flt_rstride; k.flt_kstride = a.flt_kstride;
     k.tiles_m = (a.OC + c.s * c.mt - 1) / (c.s * c.mt);
-    k.tiles_n = (a.M + c.s * c.nt - 1) / (c.s * c.nt);
+    k.tiles_n = (a.M + c.s - 1) / c.s;
     k.by_m = k.tiles_m >= 8;
     k.log_pout = pout == 32 ? 5 : pout == 4 ? 2 : 0;
     k.has_bias = a.has_bias;
@@ -402,14 +390,14 @@ int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg
     k.epi = a.epi;
     const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0;
     const int lds = ks_lds(a, c, pw);
-#define MI355_KS(PIN, S, MT, NT) \
-    (pw ? launch_ks<PIN, S, MT, NT, true>(st, k, c.waves, lds) : launch_ks<PIN, S, MT, NT, false>(st, k, c.waves, lds))
+#define MI355_KS(PIN, S, MT) \
+    (pw ? launch_ks<PIN, S, MT, true>(st, k, c.waves, lds) : launch_ks<PIN, S, MT, false>(st, k, c.waves, lds))
     if (pin == 32) {
-        if (c.s == 16) return MI355_KS(32, 16, 1, 1);
-        return c.mt == 1 ? MI355_KS(32, 32, 1, 1) : MI355_KS(32, 32, 2, 1);
+        if (c.s == 16) return MI355_KS(32, 16, 1);
+        return c.mt == 1 ? MI355_KS(32, 32, 1) : MI355_KS(32, 32, 2);
     }
-    if (c.s == 16) return MI355_KS(4, 16, 1, 1);
-    return c.mt == 1 ? MI355_KS(4, 32, 1, 1) : MI355_KS(4, 32, 2, 1);
+    if (c.s == 16) return MI355_KS(4, 16, 1);
+    return c.mt == 1 ? MI355_KS(4, 32, 1) : MI355_KS(4, 32, 2);
 #undef MI355_KS
 }
 
