@@ -489,8 +489,8 @@ int canonize_checked(const mi355_conv_desc* d, ConvProblem* p) {
 // What follows from a descriptor alone is kept per thread: its canonical form and what the heuristic answers for it.  An
 // operator call needs them several times in a row (get_workspace_in_bytes, the algorithm choice, exec), a network of some
 // fifty layers once per layer and pass.  A direct-mapped table of kMemo entries, so bounded; equal bytes mean an equal
-// descriptor, different padding bytes only cost the full path.  (A call on a small layer spends 2.7 us in its launch; the
-// full path costs another 0.9 us, an answer from here 0.1 us.)
+// descriptor, different padding bytes only cost the full path.  (A query: 0.20 us by the full path, 0.07 from here, where a call on
+// a small layer takes 3.8 us, most of it the launch: 64 -> 64 at 28 x 28, pointwise.)
 struct Memo {
     bool have = false;
     mi355_conv_desc key;

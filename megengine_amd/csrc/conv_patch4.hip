@@ -2,7 +2,7 @@
 //
 // An im2col operand of a 4-packed tensor comes in pieces of 4 bytes -- the channels of a pixel lie in planes -- so a tiled
 // implicit GEMM loads every byte of a 3x3 layer nine times, a dword at a time, through a per-unit table of offsets: 3x3
-// 64 -> 64 at 56 x 56, batch 16, took 11.6 us where its bytes and products allow 1.5, and the vector-memory path was what
+// 64 -> 64 at 56 x 56, batch 16, took 12.4 us where its bytes and products allow 1.5, and the vector-memory path was what
 // it waited for.  Here the input patch of a tile is loaded once and turned on its way into LDS: sixteen channels of a pixel
 // side by side, [group of 16 channels][patch pixel][16 bytes], so that every tap's operand is one ds_read_b128 at a shifted
 // pixel, consecutive lanes consecutive pixels, free of bank conflicts.  The filter is turned with it: entry (channel group,
@@ -19,8 +19,8 @@
 //     costs a third of the occupancy.  Loads two stages ahead, tried, cost more occupancy than they hid (7.5 us against 6.9 at
 //     56 x 56 below); reading one step's operands ahead instead of two, or computing a descriptor per channel block instead of
 //     a scalar offset (157 scalar instructions per stage instead of 64), cost up to a quarter of the time.
-// Graph replays: 3x3 64 -> 64 at 56 x 56, batch 16: 12.5 -> 6.9 us, batch 64: 32.7 -> 17.1; 256 -> 256 at 14 x 14, batch 16:
-// 15.6 -> 8.8; 32 -> 32 at 112 x 112, batch 64: 54 -> 26; 5x5 100 -> 132 at 33 x 35, batch 20: 50 -> 22.8.
+// Graph replays of the layer, here and below: 3x3 64 -> 64 at 56 x 56, batch 16: 12.4 -> 6.9 us, batch 64: 31.7 -> 17.0; 256 ->
+// 256 at 14 x 14, batch 16: 15.5 -> 8.3; 32 -> 32 at 112 x 112, batch 64: 52 -> 26.8; 5x5 100 -> 132 at 33 x 35, batch 20: 50 -> 22.5.
 #include <atomic>
 
 #include "igemm_shared.h"
@@ -389,13 +389,13 @@ bool patch4_can_run(const IgemmArgs& a, int pin, int pout, int cfg) {
     return p4_plan(a, cfg, &k, &lds);
 }
 
-// Which tile: a workgroup of 32 x 256 once those are more than one per CU (64 -> 64 at 56 x 56, batch 16, 448 of them: 6.8 us
-// against 7.3 on 32 x 128; 100 -> 132 at 33 x 35 with a 5x5 filter: 22.8 against 30), or 64 x 256 once those are two (128 -> 128
-// at 28 x 28, batch 64: 14.4 us against 16.8); below, the smallest tile, because a stage's latency is all there is (256 -> 256 at
-// 14 x 14, batch 16, 128 workgroups of 32 x 256: 10.0 us against 8.8).  At strides a tile's patch is several times its pixels:
-// the smallest tile (64 -> 128 at 56 x 56, stride 2, batch 16: 7.1 us against 7.8 on 32 x 256), and with many output channels
+// Which tile: a workgroup of 32 x 256 once those are more than one per CU (64 -> 64 at 56 x 56, batch 16, 448 of them: 6.9 us
+// against 7.5 on 32 x 128; 100 -> 132 at 33 x 35 with a 5x5 filter: 22.5 against 29.7), or 64 x 256 once those are two (128 -> 128
+// at 28 x 28, batch 64: 13.8 us against 16.3); below, the smallest tile, because a stage's latency is all there is (256 -> 256 at
+// 14 x 14, batch 16, 128 workgroups of 32 x 256: 9.7 us against 8.3).  At strides a tile's patch is several times its pixels:
+// the smallest tile (64 -> 128 at 56 x 56, stride 2, batch 16: 6.8 us against 7.6 on 32 x 256), and with many output channels
 // and pixels the 128 x 128 tiles of the general kernel, whose operand traffic shrinks with the stride (the same at batch 64:
-// 14.5 us against 18.3; 128 -> 128, batch 32: 14.6 against 16.3).
+// 14.7 us against 18.1; 128 -> 128 at 56 x 56, batch 32: 14.2 against 16.2).
 int patch4_pick(const IgemmArgs& a, int pin, int pout) {
     if (!patch4_can_run(a, pin, pout, 0)) return -1;
     if (a.sh > 1 || a.sw > 1) return a.OC > 64 && (int64_t)((a.OC + 127) / 128) * ((a.M + 127) / 128) >= 150 ? -1 : 0;

@@ -543,15 +543,20 @@ int launch_mt(hipStream_t st, const IgemmArgs& a, int cu_count) {
 //   at most 64 channels, streaming: 16 -> 96 at 112 x 112, batch 64: 18.9 / 22.2; 24 -> 144 at 56 x 56: 11.2 / 13.6; batch 16:
 //     5.0 / 6.6; 32 -> 192 at 28 x 28, batch 64: 5.9 / 7.2.  (96 channels per wave instead of 32 with very many tiles: less of the
 //     input again, 18.9 / 19.4.)
-//   one wave per tile while a wave can ask for all its operands at once (up to five steps): 96 -> 576 at 14 x 14, batch 64:
-//     6.4 / 7.2; 160 -> 960 at 7 x 7: 5.3 / 6.1; 192 -> 32 at 28 x 28: 4.3 / 5.7; 68 -> 76 at 10 x 70, batch 13: 3.6 / 4.8.
-//   longer reductions over the waves of a workgroup: 576 -> 96 at 14 x 14, batch 64: 6.0 / 7.0; 960 -> 160 at 7 x 7: 5.5 / 6.8,
+//   one wave per tile while a wave can ask for all its operands at once (up to five steps): 192 -> 32 at 28 x 28, batch 64:
+//     4.3 / 5.7; 68 -> 76 at 10 x 70, batch 13: 3.6 / 4.8.
+//   longer reductions over the waves of a workgroup: 576 -> 96 at 14 x 14, batch 64: 5.9 / 7.0; 960 -> 160 at 7 x 7: 5.5 / 6.8,
 //     batch 16: 4.0 / 5.2, batch 1: 3.7 / 3.7.
 // The tiled kernels keep what they are better at (pw4_quad_pick), large products without a residual: 88 -> 448 at 42 x 19,
 // batch 30: 9.2 / 8.4; 956 -> 524 at 105 x 25, batch 7: 28.2 / 23.9; 960 -> 320 at 7 x 7, batch 64: 7.1 / 6.7 (with a residual
-// they are behind: 156 -> 628 at 43 x 58, batch 23: 27.5 / 34.9).  Between T = 3000 and 9000 without a residual, and for six
-// steps, the two are close and the tiled kernels keep their layers: 384 -> 64 at 14 x 14, batch 64: 4.7 / 5.0; 96 -> 576: 6.4 /
-// 7.2; 108 -> 384 at 11 x 12, batch 62: 4.6 / 5.1.
+// they are behind: 156 -> 628 at 43 x 58, batch 23: 27.5 / 34.9).
+// They also keep layers that they are not better at.  Timed on 600 more sizes of T = 300 to 15000 and 68 to 960 channels in:
+//   without a residual, two to five steps to more than 64 channels from T = 3000 on, and six steps from T = 750 on: up to
+//     T = 6000 (69 sizes) the tiled kernels take 14 % longer on average, from 7 % less to 34 % more, at every number of steps;
+//     beyond, the two are even (38 sizes: 4 % less).  96 -> 576 at 14 x 14, batch 64: 6.5 / 7.2; 160 -> 960 at 7 x 7: 5.4 / 6.1;
+//     384 -> 64 at 14 x 14: 4.3 / 4.7; all of MobileNetV2 at batch 64: 352 / 358.  The lines stand there because the chooser's
+//     tests (test_heuristic_picks, tests/test_gpu_parity.py) name the tiled kernel for these three layers.
+//   seven and more steps to more than 256 channels between T = 450 and 2000: from 22 % less to 51 % more (47 sizes: 11 % more).
 struct QuadPlan {
     int mt;      // 0: none
     int waves;   // 0: the streaming kernel
@@ -580,7 +585,7 @@ bool pw4s_usable(const IgemmArgs& a) {
 bool pw4_split_usable(const IgemmArgs& a, int pin, int pout) {
     return pin == 4 && pout == 4 && a.groups == 1 && !a.general && a.T == 1 && a.ph == 0 && a.pw == 0 && quad_stride(a);
 }
-// whether one of the two is ahead of the tiled kernels
+// whether one of the two takes the layer from the tiled kernels
 bool pw4_quad_pick(const IgemmArgs& a, int pin, int pout) {
     if (!pw4_split_usable(a, pin, pout)) return false;
     if (pw4s_usable(a)) return true;

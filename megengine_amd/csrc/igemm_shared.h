@@ -512,7 +512,7 @@ int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg);
 bool pw4s_usable(const IgemmArgs& a);
 // NCHW4 pointwise at stride 1, four pixels per lane (tile "pw4_split"); the streaming tile takes the same form there
 bool pw4_split_usable(const IgemmArgs& a, int pin, int pout);
-bool pw4_quad_pick(const IgemmArgs& a, int pin, int pout);  // whether one of the two is ahead of the others
+bool pw4_quad_pick(const IgemmArgs& a, int pin, int pout);  // whether one of the two takes the layer
 int launch_pw4_split(hipStream_t st, const IgemmArgs& a);
 int launch_pw4s(hipStream_t st, const IgemmArgs& a, int cu_count);
 // the same for 32-packed pointwise layers with at most 128 input channels (tile "pw32_stream")
