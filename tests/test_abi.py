@@ -185,8 +185,9 @@ def test_tile_usable_names_the_kernel_that_runs():
 
 
 def test_plain_nchw_reports_a_workspace():
-    """Format::NCHW runs relayout -> NCHW32 MFMA kernel -> relayout through the caller's workspace: query reports its
-    size (get_workspace_in_bytes, dnn/include/megdnn/oprs/nn.h:419-422), the packed-format algorithms report 0."""
+    """Format::NCHW runs on the MFMA kernel with src and filter packed in the caller's workspace: query reports a size
+    (get_workspace_in_bytes, dnn/include/megdnn/oprs/nn.h:419-422) that holds every tensor packed by 32, the packed-format
+    algorithms report 0."""
     names = lib.algo_names()
     nchw = names.index("MI355_NCHW_RELAYOUT_MFMA_I8")
     up = lambda x: (x + 255) // 256 * 256

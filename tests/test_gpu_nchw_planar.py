@@ -38,6 +38,13 @@ def test_edges(oracle, i):
         check_case(oracle, d, seed=30 + i, algo=NCHW, tag="nchw planar %d" % i)
 
 
+@pytest.mark.parametrize("fh,fw", [(3, 6), (2, 9), (18, 1), (1, 9)])
+@pytest.mark.parametrize("n,ic,oc", [(2, 12, 45), (2, 75, 70), (24, 40, 66)])   # packed by 4, by 32; pixels for the tiled kernel
+def test_filters_that_are_not_square(oracle, n, ic, oc, fh, fw):
+    d = _abi.make_conv_desc("NCHW", n, ic, 21, 23, oc, fh, fw, pad=(fh // 2, fw // 2), stride=(1, 2), nonline="RELU", has_z=True, **S)
+    check_case(oracle, d, seed=fh * fw + n, algo=NCHW, tag="nchw planar %dx%d" % (fh, fw))
+
+
 def test_tensors_at_any_address(oracle):
     d = _abi.make_conv_desc("NCHW", 3, 37, 19, 21, 45, 3, pad=1, nonline="RELU", has_z=True, **S)
     src, flt, bias, z = util.make_tensors(d, seed=9)

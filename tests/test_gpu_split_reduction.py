@@ -48,3 +48,15 @@ def test_the_chooser_takes_them_for_few_pixels_only():
         names = [lib.tile_names()[ops.conv_bias_query(_abi.make_conv_desc(fmt, n, ic, hw, hw, oc, f, pad=f // 2, **S))[0].tile_cfg]
                  for n in (1, 64)]
         assert "ks" in names[0] and "ks" not in names[1], names
+
+
+@pytest.mark.parametrize("fh,fw", [(3, 6), (9, 2), (1, 18), (1, 9), (5, 1)])
+@pytest.mark.parametrize("fmt,ic,oc", [("NCHW32", 96, 64), ("NCHW4", 20, 36), ("NCHW4_NCHW32", 12, 32), ("NCHW32_NCHW4", 32, 20)])
+def test_filters_that_are_not_square(oracle, fmt, ic, oc, fh, fw):
+    ran = 0
+    for stride in ((1, 1), (2, 1)):
+        d = _abi.make_conv_desc(fmt, 2, ic, 11, 19, oc, fh, fw, pad=(fh // 2, fw // 2), stride=stride, nonline="RELU", has_z="_" not in fmt, **S)
+        for t, name in enumerate(lib.tile_names()):
+            if name.startswith(("v2_ks_", "ks4_")) and check_case(oracle, d, seed=fh + fw, algo=IGEMM, tile=t, tag=name) is not None:
+                ran += 1
+    assert ran >= 8
