@@ -271,10 +271,10 @@ int launch_g16(hipStream_t st, const ConvProblem& p, const int8_t* src, const in
 //                   others: 3 + 0.145 per tap and channel block (in a row, for any size) + 1 outputs + 0.22 dot products
 //   each group      3.6 + 0.05 matrix steps (pixels x taps x output channels in 32s x input channels in 16s)
 //   all groups      0.1 outputs, with a residual 0.5
-// One launch is kept up to a quarter more, which G submissions cost the host.  Of the 1775, 422 go group by group for it, one
-// launch against those: 2.7 times faster on average (2 groups 16 -> 116, 7x7 at 33 x 39, batch 51: 590 us / 46; 4 groups 16 ->
+// One launch is kept up to a quarter more, which G submissions cost the host.  Of the 1775, 435 go group by group for it, one
+// launch against those: 2.6 times faster on average (2 groups 16 -> 116, 7x7 at 33 x 39, batch 51: 590 us / 46; 4 groups 16 ->
 // 120, 3x3 at 90 x 67, batch 38: 173 / 81; 6 groups 16 -> 76, 7x7 at 8 x 14, batch 12: 77 / 29; 3 groups 12 -> 100, 1x1 at 57 x
-// 79, batch 44: 114 / 42), none of them more than a quarter slower; of what stays, 26 are behind by more than that, at most by
+// 79, batch 44: 114 / 42), none of them more than a fifth slower; of what stays, 29 are behind by more than a quarter, at most by
 // 2.2 times (34 groups 8 -> 108, 7x7 stride 2 at 31 x 8).  On 250 other sizes 44 change sides and are 2.2 times faster on average.
 bool grp4_pick(const ConvProblem& p) {
     const mi355_conv_desc& d = p.d;
