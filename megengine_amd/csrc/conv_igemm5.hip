@@ -45,6 +45,8 @@ struct KsArgs {
     int src_sn, src_scb, dst_sn, dst_scb, z_sn;
     int flt_rstride, flt_kstride;
     int tiles_m, tiles_n, by_m;
+    int FH, steps, per_wave, extra;  // steps of the reduction: per_wave for every wave, one more for the first `extra`
+    FastDiv div_tile;                // by tiles_n (by_m) or tiles_m
     int log_pout, has_bias, dst_s32;
     FastDiv div_ohw, div_ow, div_t, div_fw;
     EpiParams epi;
@@ -70,15 +72,26 @@ struct KsAcc<16> {
     __device__ __forceinline__ v4i quad(int) const { return v; }  // channels 4 (lane / 16) .. + 3
 };
 
-template <int PIN, int S, int MT, bool PW>
-__global__ __launch_bounds__(MT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
+template <int PIN, int S, int MT, int W, bool PW>
+__global__ __launch_bounds__(W * 64) void ks_kernel(KsArgs a) {
     constexpr int ROWS = S / 4;           // channel quads of a block
     constexpr int PARTS = S == 32 ? 4 : 1;  // a block's quads over its pixels, 64 at a time
     constexpr int ROWP = ks_row(S), WP = MT * ROWS * ROWP;  // vectors per row, per wave
     constexpr int CH = S == 32 ? 1 : 2;   // 32-byte chunks per step
     constexpr int AHEAD = ks_ahead(S, MT);
     extern __shared__ __attribute__((aligned(16))) v4i red[];
-    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), W = blockDim.x >> 6;
+    // Every argument on the way to the operands in one batch of scalar loads (left alone, the compiler asks for them where they
+    // are first used, behind the early exit: a second round trip), and one word of each line that the epilogue reads.
+    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.OHW), "s"(a.OW), "s"(a.IW),
+                 "s"(a.IH), "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.OC), "s"(a.M), "s"(a.src_sn), "s"(a.src_scb),
+                 "s"(a.flt_rstride), "s"(a.flt_kstride), "s"(a.tiles_m), "s"(a.tiles_n), "s"(a.by_m), "s"(a.KC));
+    asm volatile("" ::"s"(a.steps), "s"(a.per_wave), "s"(a.extra), "s"(a.div_tile.m), "s"(a.div_tile.s1), "s"(a.div_tile.s2),
+                 "s"(a.div_ohw.m), "s"(a.div_ohw.s1), "s"(a.div_ohw.s2), "s"(a.div_ow.m), "s"(a.div_ow.s1), "s"(a.div_ow.s2),
+                 "s"(a.log_pout), "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo));
+    if (!PW)
+        asm volatile("" ::"s"(a.div_t.m), "s"(a.div_t.s1), "s"(a.div_t.s2), "s"(a.div_fw.m), "s"(a.div_fw.s1), "s"(a.div_fw.s2), "s"(a.T),
+                     "s"(a.FW), "s"(a.FH));
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int ls = lane & (S - 1), lk = lane / S;
 
     // Workgroup b runs on XCD b % 8.  Layers with eight and more channel tiles give each XCD channel tiles of its own (the
@@ -87,12 +100,12 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
     {
         const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
         if (a.by_m) {
-            const int r = i / a.tiles_n;
+            const int r = (int)fdiv(i, a.div_tile);
             tm = r * 8 + x;
             tn = i - r * a.tiles_n;
             if (tm >= a.tiles_m) return;
         } else {
-            const int per = (a.tiles_n + 7) >> 3, r = i / a.tiles_m;
+            const int per = (a.tiles_n + 7) >> 3, r = (int)fdiv(i, a.div_tile);
             tm = i - r * a.tiles_m;
             tn = x * per + r;
             if (tn >= a.tiles_n) return;
@@ -103,13 +116,11 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
     const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, a.flt_bytes);
 
     // this wave's piece of the reduction, in steps
-    const int steps = (a.KC + CH - 1) / CH;
-    const int per = steps / W, extra = steps - per * W;
-    const int k0 = wave * per + (wave < extra ? wave : extra), k1 = k0 + per + (wave < extra ? 1 : 0);
+    const int k0 = wave * a.per_wave + (wave < a.extra ? wave : a.extra), k1 = k0 + a.per_wave + (wave < a.extra ? 1 : 0);
 
     KEntry* tab = reinterpret_cast<KEntry*>(red + W * WP);
     if (PIN == 4 && !PW) {
-        for (int u = t; u < steps * CH * 8; u += blockDim.x) {
+        for (int u = t; u < a.steps * CH * 8; u += W * 64) {
             const uint32_t cb = fdiv(u, a.div_t), tap = u - cb * a.T, fh = fdiv(tap, a.div_fw), fw = tap - fh * a.FW;
             tab[u] = u < a.entries ? KEntry{(int)cb * a.src_scb + ((int)fh * a.IW + (int)fw) * 4, (int)(fh | fw << 16)}
                                    : KEntry{0, 0x4000};
@@ -144,7 +155,6 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
         fh = (int)fdiv(tap, a.div_fw);
         fw = tap - fh * a.FW;
     }
-    const int FH = PW ? 1 : a.T / a.FW;
     // Operands of the next step.  Past the wave's piece every lane is out of the buffers' range: zeros, no memory access
     // (an unconditional load keeps the number of loads in flight known to the compiler, and with it the waits short).
     // A 4-packed row may end inside its last chunk, so there the whole offset stands where the descriptor checks it.
@@ -185,7 +195,7 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
         if (PIN == 32 && !PW && S == 32) {
             if (++fw == a.FW) {
                 fw = 0;
-                if (++fh == FH) {
+                if (++fh == a.FH) {
                     fh = 0;
                     ++cb;
                 }
@@ -211,13 +221,13 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
         const int px = a.log_pout == 5 ? part * (64 / ROWS) + lane / ROWS : ls;
         at_red = (i * ROWS + row) * ROWP + px;
         const int oc4 = oc0 + i * S + row * 4, m = px0 + px;
-        const bool ok = m < a.M && oc4 < a.OC;
+        const bool ok = m < a.M && oc4 < a.OC && u < MT * PARTS;
         const uint32_t mm = m < a.M ? m : 0;
         const uint32_t n = fdiv(mm, a.div_ohw), rem = mm - n * a.OHW;
         const int at = (oc4 >> a.log_pout) * a.dst_scb + ((int)rem << a.log_pout) + (oc4 & ((1 << a.log_pout) - 1));
         d_off = ok ? (int)n * a.dst_sn + at : SENT;
         z_off = ok ? (int)n * a.z_sn + at : SENT;
-        bv = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, oc4 * 4, 0, 0);
+        bv = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, ok ? oc4 * 4 : SENT, 0, 0);
         zw = 0;
         if (a.log_pout == 0) {
             // planar: four channels of a pixel lie OHW apart
@@ -229,10 +239,12 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
         } else if (a.epi.has_z && !a.dst_s32) zw = __builtin_amdgcn_raw_buffer_load_b32(rs_z, z_off, 0, 0);
     };
 
-    if (k0 < k1) {  // (waves beyond the number of steps have nothing to add)
+    {
         v4i fa[AHEAD][MT], fb[AHEAD];
+        if (k0 < k1)  // (waves beyond the number of steps have nothing to add)
 #pragma unroll
-        for (int g = 0; g < AHEAD; ++g) load(fa[g], fb[g]);
+            for (int g = 0; g < AHEAD; ++g) load(fa[g], fb[g]);
+        fetch(wave);  // behind the first operands, so that bias and residual cost no round trip of their own
         auto multiply = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) acc[i].mfma(fa[g][i], fb[g]);
@@ -253,12 +265,11 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void ks_kernel(KsArgs a) {
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int q = 0; q < PARTS; ++q) red[wave * WP + (i * ROWS + q * (64 / S) + lk) * ROWP + ls] = acc[i].quad(q);
-    if (wave < MT * PARTS) fetch(wave);  // lands while the partial sums meet
     __syncthreads();
     for (int u = wave; u < MT * PARTS; u += W) {
         if (u != wave) fetch(u);
         v4i s = bv;
-#pragma unroll 4
+#pragma unroll
         for (int w = 0; w < W; ++w) s += red[w * WP + at_red];
         if (a.dst_s32) {
             // four elements of an int32 dst: element offset d_off, a residual of the same type and its own batch stride
@@ -297,9 +308,9 @@ int ks_lds(const IgemmArgs& a, const KsCfg& c, bool pw) {
     return c.waves * c.mt * (c.s / 4) * ks_row(c.s) * 16 + (c.pin == 4 && !pw ? (a.KC + 1) * 8 * 8 : 0);
 }
 
-template <int PIN, int S, int MT, bool PW>
-int launch_ks(hipStream_t st, const KsArgs& k, int waves, int lds) {
-    auto kern = ks_kernel<PIN, S, MT, PW>;
+template <int PIN, int S, int MT, int W, bool PW>
+int launch_ks(hipStream_t st, const KsArgs& k, int lds) {
+    auto kern = ks_kernel<PIN, S, MT, W, PW>;
     static std::atomic<int> max_lds_set{0};
     if (lds > max_lds_set.load(std::memory_order_relaxed)) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -308,7 +319,7 @@ int launch_ks(hipStream_t st, const KsArgs& k, int waves, int lds) {
     }
     const int64_t grid = k.by_m ? (int64_t)((k.tiles_m + 7) / 8) * k.tiles_n * 8 : (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
-    return launch_kernel(kern, dim3((unsigned)grid), dim3(waves * 64), lds, st, k);
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(W * 64), lds, st, k);
 }
 
 }  // namespace
@@ -379,6 +390,11 @@ int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg
     k.tiles_m = (a.OC + c.s * c.mt - 1) / (c.s * c.mt);
     k.tiles_n = (a.M + c.s - 1) / c.s;
     k.by_m = k.tiles_m >= 8;
+    k.div_tile = make_fastdiv(k.by_m ? k.tiles_n : k.tiles_m);
+    k.FH = a.FH;
+    k.steps = c.s == 32 ? a.KC : (a.KC + 1) / 2;
+    k.per_wave = k.steps / c.waves;
+    k.extra = k.steps % c.waves;
     k.log_pout = pout == 32 ? 5 : pout == 4 ? 2 : 0;
     k.has_bias = a.has_bias;
     k.dst_s32 = a.dst_s32;
@@ -391,7 +407,8 @@ int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg
     const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0;
     const int lds = ks_lds(a, c, pw);
 #define MI355_KS(PIN, S, MT) \
-    (pw ? launch_ks<PIN, S, MT, true>(st, k, c.waves, lds) : launch_ks<PIN, S, MT, false>(st, k, c.waves, lds))
+    (pw ? c.waves == 8 ? launch_ks<PIN, S, MT, 8, true>(st, k, lds) : launch_ks<PIN, S, MT, 4, true>(st, k, lds) \
+        : c.waves == 8 ? launch_ks<PIN, S, MT, 8, false>(st, k, lds) : launch_ks<PIN, S, MT, 4, false>(st, k, lds))
     if (pin == 32) {
         if (c.s == 16) return MI355_KS(32, 16, 1);
         return c.mt == 1 ? MI355_KS(32, 32, 1) : MI355_KS(32, 32, 2);

@@ -22,6 +22,35 @@ namespace {
 
 constexpr int PW4_MAX_OC = 1024;
 
+// How the waves of a streaming launch walk the pixel blocks: wave g of the launch (of its XCD's share of the launch) takes the
+// channel group g % n_ocg of the blocks g / n_ocg, + step, ...  With slabs the XCDs take one contiguous eighth of the blocks
+// each.  The divisions are the host's: a run-time integer division is 0.1 us on the way to the first load.
+struct PwWalk {
+    int n_ocg, step, slabs;
+    FastDiv div_ocg;
+};
+PwWalk make_walk(int64_t blocks, int n_ocg) {
+    PwWalk w;
+    w.n_ocg = n_ocg;
+    w.slabs = blocks % 8 == 0 && blocks / 8 * 4 % n_ocg == 0;
+    w.step = (int)((w.slabs ? blocks / 8 : blocks) * 4 / n_ocg);
+    w.div_ocg = make_fastdiv(n_ocg);
+    return w;
+}
+__device__ __forceinline__ void pw_walk(const PwWalk& w, int n_pb, int wave, int* pb0, int* pb_hi, int* ocg) {
+    int lo = 0, hi = n_pb, g = (int)blockIdx.x * 4 + wave;
+    if (w.slabs) {
+        const int xc = blockIdx.x & 7, per = n_pb >> 3, rem = n_pb & 7;
+        lo = xc * per + (xc < rem ? xc : rem);
+        hi = lo + per + (xc < rem ? 1 : 0);
+        g = (int)(blockIdx.x >> 3) * 4 + wave;
+    }
+    const int q = (int)fdiv(g, w.div_ocg);
+    *ocg = g - q * w.n_ocg;
+    *pb0 = lo + q;
+    *pb_hi = hi;
+}
+
 // HZ: the launch has a residual (its registers exist only in that instantiation)
 template <int MT, int KC, bool HZ>
 __global__ __launch_bounds__(256) void pw4s_kernel(IgemmArgs a, int n_ocg, int n_pb) {
@@ -104,23 +133,20 @@ __global__ __launch_bounds__(256) void pw4s_kernel(IgemmArgs a, int n_ocg, int n
 // whatever follows (the descriptor answers zeros past the tensor) and are not stored.  Bound by the output stream and the
 // four vector instructions per output: 16 -> 96 at 112 x 112, batch 64, 18.9 us for 90 MB (4.8 TB/s) against 22.2.
 template <int MT, int KC, bool HZ>
-__global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, int n_ocg, int n_pb, int groups, FastDiv div_g) {
-    __shared__ __attribute__((aligned(16))) int sBias[PW4_MAX_OC + 96];
+__global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, PwWalk w, int n_pb, int groups, FastDiv div_g) {
+    __shared__ __attribute__((aligned(16))) int sBias[4][MT * 32];
     const int t = threadIdx.x;
     const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
-    // pixel blocks by XCD, as in pw32s_kernel below
-    int pb_lo = 0, pb_hi = n_pb, gw = blockIdx.x * 4 + wave, GW = gridDim.x * 4;  // GW is a multiple of n_ocg
-    if ((gridDim.x & 7) == 0 && ((gridDim.x >> 3) * 4) % n_ocg == 0) {
-        const int xc = blockIdx.x & 7, per = n_pb >> 3, rem = n_pb & 7;
-        pb_lo = xc * per + (xc < rem ? xc : rem);
-        pb_hi = pb_lo + per + (xc < rem ? 1 : 0);
-        gw = (blockIdx.x >> 3) * 4 + wave;
-        GW = (gridDim.x >> 3) * 4;
-    }
-    const int q0 = gw / n_ocg, ocg = gw - q0 * n_ocg, step = GW / n_ocg;
-    const int pb0 = pb_lo + q0;
-    const int oc_w = ocg * MT * 32;
+    // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
+    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.OHW), "s"(a.OC), "s"(a.NB),
+                 "s"(a.kbytes), "s"(a.src_sn), "s"(a.src_scb), "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(w.div_ocg.m),
+                 "s"(w.div_ocg.s1), "s"(w.div_ocg.s2), "s"(w.n_ocg), "s"(w.step), "s"(w.slabs), "s"(n_pb), "s"(groups), "s"(div_g.m),
+                 "s"(div_g.s1), "s"(div_g.s2));
+    int pb0, pb_hi, ocg;
+    pw_walk(w, n_pb, wave, &pb0, &pb_hi, &ocg);
+    const int oc_w = ocg * MT * 32, step = w.step;
+    int* bias_w = sBias[wave];
     const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes);
     const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, a.flt_bytes);
     const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, HZ ? a.z_bytes : 0);
@@ -134,6 +160,10 @@ __global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, int n_ocg, in
         for (int kc = 0; kc < KC; ++kc)
             fa[i][kc] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, row < a.OC ? row * a.kbytes + kc * 32 + lh * 16 : SENT, 0, 0);
     }
+    const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
+    int bias_v[(MT + 1) / 2];
+#pragma unroll
+    for (int i = 0; i < MT * 32; i += 64) bias_v[i / 64] = __builtin_amdgcn_raw_buffer_load_b32(rs_bias, (oc_w + i + lane) * 4, 0, 0);
     const int icb = a.kbytes >> 2, total = a.NB * groups;
     // x[kc][i]: four pixels of channel block kc * 8 + lh * 4 + i (zeros past the last one)
     auto load_b = [&](int pb, v4i (&x)[KC][4]) __attribute__((always_inline)) {
@@ -150,9 +180,12 @@ __global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, int n_ocg, in
     };
     v4i x[KC][4];
     load_b(pb0 < pb_hi ? pb0 : n_pb, x);
-    // the bias goes to LDS after the filter rows and the first block are requested
-    for (int i = t; i < PW4_MAX_OC + 96; i += 256) sBias[i] = (a.has_bias && i < a.OC) ? a.bias[i] : 0;
-    __syncthreads();
+    // The bias of the wave's channels in accumulator order lies in LDS that only this wave reads: no barrier, and no round trip
+    // beside that of the operands.
+#pragma unroll
+    for (int i = 0; i < MT * 32; i += 64)
+        if (i + lane < MT * 32) bias_w[i + lane] = bias_v[i / 64];
+    __builtin_amdgcn_wave_barrier();
     const int tail = a.OHW & 3;
     auto blocks = [&](auto nl) __attribute__((always_inline)) {
         constexpr int NL = decltype(nl)::value;
@@ -181,7 +214,7 @@ __global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, int n_ocg, in
                 v16i bv;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const v4i b = *reinterpret_cast<const v4i*>(sBias + oc_w + i * 32 + 8 * q + 4 * lh);
+                    const v4i b = *reinterpret_cast<const v4i*>(bias_w + i * 32 + 8 * q + 4 * lh);
                     bv[4 * q + 0] = b[0]; bv[4 * q + 1] = b[1]; bv[4 * q + 2] = b[2]; bv[4 * q + 3] = b[3];
                 }
                 v4i o[4];
@@ -227,11 +260,15 @@ __global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, int n_ocg, in
 // and, of pixels 4 (l % 16) .. + 3, the 16 k-bytes at 16 (l / 16)).  What bounds these layers is latency -- a few megabytes and a
 // few hundred products per CU -- so a wave asks for all (or four steps) of its operands at once, and the partial sums meet
 // in LDS once.
-template <int MT>
-__global__ __launch_bounds__(512) void pw4k_kernel(IgemmArgs a, int tiles_m, int tiles_n, int groups, FastDiv div_g, FastDiv div_tm) {
+template <int MT, int W>
+__global__ __launch_bounds__(W * 64, 2) void pw4k_kernel(IgemmArgs a, int tiles_m, int tiles_n, int groups, FastDiv div_g, FastDiv div_tm) {
     constexpr int AHEAD = MT <= 2 ? 4 : 3;
     extern __shared__ __attribute__((aligned(16))) v4i part[];
-    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), W = blockDim.x >> 6;
+    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.z), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.z_bytes),
+                 "s"(a.OHW), "s"(a.OC), "s"(a.NB), "s"(a.kbytes), "s"(a.src_sn), "s"(a.src_scb), "s"(a.dst_scb), "s"(a.z_sn),
+                 "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(tiles_m), "s"(tiles_n), "s"(groups), "s"(div_g.m), "s"(div_g.s1),
+                 "s"(div_g.s2), "s"(div_tm.m), "s"(div_tm.s1), "s"(div_tm.s2));
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int ls = lane & 15, lk = lane >> 4;
     // workgroup b runs on XCD b % 8: each XCD takes a contiguous run of pixels with all their channels
     const uint32_t at = blockIdx.x >> 3, r0 = fdiv(at, div_tm);
@@ -253,19 +290,20 @@ __global__ __launch_bounds__(512) void pw4k_kernel(IgemmArgs a, int tiles_m, int
     for (int i = 0; i < MT; ++i) row[i] = oc0 + i * 16 + ls < a.OC ? (oc0 + i * 16 + ls) * a.kbytes + lk * 16 : SENT;
 
     // this wave's piece of the reduction, in steps of 64 bytes
-    const int steps = (a.kbytes + 63) >> 6, per = steps / W, extra = steps - per * W;
+    const int steps = (a.kbytes + 63) >> 6, per = steps / W, extra = steps % W;  // (W is a power of two)
     int kc = wave * per + (wave < extra ? wave : extra);
     const int k1 = kc + per + (wave < extra ? 1 : 0);
     int left = k1 - kc;
-    // operands of the next step; past the wave's piece every lane is out of range: zeros, no memory access
+    // operands of the next step; past the wave's piece every lane is out of range: zeros, no memory access.  (No && here: the
+    // compiler makes a branch of a wave-uniform one, with the load behind it, and waits for everything at each of them.)
     auto load = [&](v4i (&fa)[MT], v4i (&x)[4]) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
-            fa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, kc < k1 && row[i] != SENT ? row[i] + kc * 64 : SENT, 0, 0);
+            fa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, ((kc < k1) & (row[i] != SENT)) ? row[i] + kc * 64 : SENT, 0, 0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int cb = kc * 16 + i;
-            x[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, kc < k1 && cb + lk * 4 < icb ? pix + cb * a.src_scb : SENT, 0, 0);
+            x[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, ((kc < k1) & (cb + lk * 4 < icb)) ? pix + cb * a.src_scb : SENT, 0, 0);
         }
         ++kc;
     };
@@ -283,25 +321,43 @@ __global__ __launch_bounds__(512) void pw4k_kernel(IgemmArgs a, int tiles_m, int
         }
     };
     const int tail = a.OHW & 3;
-    const bool cut = tail != 0 && (int)g == groups - 1;  // 1 to 3 pixels: the last group of an image
-    v4i bz[MT], zv[MT];
-    auto bias_z = [&](int i, v4i& b, v4i& z) __attribute__((always_inline)) {
-        const int oc4 = oc0 + i * 16 + lk * 4;
-        b = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, oc4 * 4, 0, 0);
-        z = v4i{0, 0, 0, 0};
-        if (a.epi.has_z)
-            z = __builtin_amdgcn_raw_buffer_load_b128(rs_z, ok && oc4 < a.OC ? (int)n * a.z_sn + (int)g * 16 + (oc4 >> 2) * a.dst_scb : SENT, 0, 0);
+    // What a thread finishes.  Tiles of at least one block of 16 channels per wave: whole blocks, 4 pixels x 4 channels of each.
+    // Tiles of fewer blocks than waves: their dwords are dealt out again, so that no wave adds up and requantises for all -- unit
+    // u = wave, + W, ... is the channel quad u % 4 of block u / 4, and a lane takes pixel `lane` of the 64 (64 consecutive
+    // dwords of the plane; 960 -> 160 at 7 x 7, one image, with a residual: 3.7 -> 3.3 us).
+    constexpr bool DEAL = MT < W;
+    constexpr int ITEMS = DEAL ? MT * 4 / W : MT / W;
+    const int mf = tn * 16 + (lane >> 2);
+    const bool okf = DEAL ? mf < a.NB * groups : ok;
+    const uint32_t mmf = okf ? mf : 0, nf = DEAL ? fdiv(mmf, div_g) : n, gf = DEAL ? mmf - nf * groups : g;
+    const bool cut = tail != 0 && (int)gf == groups - 1;  // 1 to 3 pixels: the last group of an image
+    const bool px_ok = okf && !(DEAL && cut && (lane & 3) >= tail);
+    const int z_px = (int)nf * a.z_sn + (int)gf * 16 + (DEAL ? (lane & 3) * 4 : 0), d_px = (int)nf * a.dst_sn + (int)gf * 16 + (DEAL ? (lane & 3) * 4 : 0);
+    auto quad_of = [&](int r) __attribute__((always_inline)) { return DEAL ? oc0 + (wave + W * r) * 4 : oc0 + (wave + W * r) * 16 + lk * 4; };
+    v4i bz[ITEMS], zv[ITEMS];
+    auto bias_z = [&](int r) __attribute__((always_inline)) {
+        const int oc4 = quad_of(r), at = px_ok && oc4 < a.OC ? z_px + (oc4 >> 2) * a.dst_scb : SENT;
+        if (W > 1) bz[r] = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, oc4 * 4, 0, 0);
+        zv[r] = v4i{0, 0, 0, 0};
+        if (a.epi.has_z) {
+            if (DEAL) zv[r][0] = __builtin_amdgcn_raw_buffer_load_b32(rs_z, at, 0, 0);
+            else zv[r] = __builtin_amdgcn_raw_buffer_load_b128(rs_z, at, 0, 0);
+        }
     };
+    if (W == 1)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) bz[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, quad_of(i) * 4, 0, 0);
     {
         v4i fa[AHEAD][MT], x[AHEAD][4];
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) load(fa[u], x[u]);
-        if (W == 1) {
 #pragma unroll
-            for (int i = 0; i < MT; ++i) bias_z(i, bz[i], zv[i]);
-        } else if (wave < MT) {
-            bias_z(wave, bz[0], zv[0]);
-        }
+        for (int r = 0; r < ITEMS; ++r) bias_z(r);
+        if (W == 1)  // one wave: the sums start from the bias (asked for before the operands)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = bz[i];
         for (; left > AHEAD; left -= AHEAD) {
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u) {
@@ -317,42 +373,45 @@ __global__ __launch_bounds__(512) void pw4k_kernel(IgemmArgs a, int tiles_m, int
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) part[((wave * MT + i) * 4 + j) * 64 + lane] = acc[i][j];
+            // (the slots of a lane's four pixels are turned by its number: no two lanes of a write meet on a bank)
+            for (int j = 0; j < 4; ++j)
+                part[DEAL ? (wave * MT + i) * 256 + lane * 4 + (j ^ ((lane >> 1) & 3)) : ((wave * MT + i) * 4 + j) * 64 + lane] = acc[i][j];
         __syncthreads();
-        if (wave >= MT) return;
     }
     auto finish = [&](auto nl, auto hz) __attribute__((always_inline)) {
         constexpr int NL = decltype(nl)::value;
         constexpr bool HZ = decltype(hz)::value;
-        auto write = [&](int i, const v4i (&s)[4], const v4i& z) __attribute__((always_inline)) {
-            const int oc4 = oc0 + i * 16 + lk * 4;
-            const bool in = ok && oc4 < a.OC;
-            const int d = (int)n * a.dst_sn + (int)g * 16 + (oc4 >> 2) * a.dst_scb;
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const int oc4 = quad_of(r);
+            const bool in = px_ok && oc4 < a.OC;
+            const int at = d_px + (oc4 >> 2) * a.dst_scb;
+            if (DEAL) {
+                const int u = wave + W * r, owner = (u & 3) * 16 + (lane >> 2);
+                v4i s = bz[r];
+#pragma unroll
+                for (int w = 0; w < W; ++w) s += part[(w * MT + (u >> 2)) * 256 + owner * 4 + ((lane & 3) ^ ((owner >> 1) & 3))];
+                const uint32_t o = requant4_fast<NL, HZ>(s[0], s[1], s[2], s[3], (uint32_t)zv[r][0], a.epi);
+                __builtin_amdgcn_raw_buffer_store_b32(o, rs_dst, in ? at : SENT, 0, 0);
+                continue;
+            }
+            v4i s[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] = W == 1 ? acc[r][j] : bz[r];
+            if (W > 1)
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) s[j] += part[((w * MT + wave + W * r) * 4 + j) * 64 + lane];
             v4i o;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) o[j] = (int)requant4_fast<NL, HZ>(s[j][0], s[j][1], s[j][2], s[j][3], (uint32_t)z[j], a.epi);
-            __builtin_amdgcn_raw_buffer_store_b128(o, rs_dst, in && !cut ? d : SENT, 0, 0);
+            for (int j = 0; j < 4; ++j) o[j] = (int)requant4_fast<NL, HZ>(s[j][0], s[j][1], s[j][2], s[j][3], (uint32_t)zv[r][j], a.epi);
+            __builtin_amdgcn_raw_buffer_store_b128(o, rs_dst, in && !cut ? at : SENT, 0, 0);
             asm volatile("s_nop 1" ::"v"(o) : "memory");  // (see igemm_epilogue)
             if (tail != 0)
 #pragma unroll
-                for (int r = 0; r < 3; ++r)
-                    if (r < tail) __builtin_amdgcn_raw_buffer_store_b32(o[r], rs_dst, in && cut ? d + r * 4 : SENT, 0, 0);
-        };
-        if (W == 1) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i) {
-                const v4i s[4] = {acc[i][0] + bz[i], acc[i][1] + bz[i], acc[i][2] + bz[i], acc[i][3] + bz[i]};
-                write(i, s, zv[i]);
-            }
-            return;
-        }
-        for (int i = wave; i < MT; i += W) {
-            if (i != wave) bias_z(i, bz[0], zv[0]);
-            v4i s[4] = {bz[0], bz[0], bz[0], bz[0]};
-            for (int w = 0; w < W; ++w)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) s[j] += part[((w * MT + i) * 4 + j) * 64 + lane];
-            write(i, s, zv[0]);
+                for (int k = 0; k < 3; ++k)
+                    if (k < tail) __builtin_amdgcn_raw_buffer_store_b32(o[k], rs_dst, in && cut ? at + k * 4 : SENT, 0, 0);
         }
     };
     using std::integral_constant;
@@ -378,27 +437,24 @@ __global__ __launch_bounds__(512) void pw4k_kernel(IgemmArgs a, int tiles_m, int
 // of k-step kc is one 16-byte load -- half of its pixel's 32-byte block kc; 32 consecutive pixels are one contiguous
 // kilobyte -- and the stores are the 16-byte stores of the tiled kernels.
 template <int MT, int KC, bool HZ>
-__global__ __launch_bounds__(256, 2) void pw32s_kernel(IgemmArgs a, int n_ocg, int n_pb,
+__global__ __launch_bounds__(256, 2) void pw32s_kernel(IgemmArgs a, PwWalk w, int n_pb,
                                                        std::conditional_t<HZ, ResidualTable, NoResidualTable> tab) {
     const int t = threadIdx.x;
     const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
 
+    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.z), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.z_bytes),
+                 "s"(a.OHW), "s"(a.OC), "s"(a.M), "s"(a.OW), "s"(a.IW), "s"(a.sh), "s"(a.sw), "s"(a.kbytes), "s"(a.src_sn), "s"(a.src_scb),
+                 "s"(a.dst_scb), "s"(a.z_sn), "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(w.div_ocg.m));
+    asm volatile("" ::"s"(a.div_ohw.m), "s"(a.div_ohw.s1), "s"(a.div_ohw.s2), "s"(a.div_ow.m), "s"(a.div_ow.s1), "s"(a.div_ow.s2),
+                 "s"(w.div_ocg.s1), "s"(w.div_ocg.s2), "s"(w.n_ocg), "s"(w.step), "s"(w.slabs), "s"(n_pb));
     // Pixel blocks by XCD, as the tiled kernels deal out their tiles: workgroup b runs on XCD b % 8 (round-robin
     // dispatch) and each XCD takes one contiguous eighth of the pixel blocks, so that this layer finds its inputs in the
     // L2 of the XCD that wrote them and leaves its outputs where the next layer's workgroups will look for them.
     // (Grids that are no multiple of 8 n_ocg / 4 workgroups -- small problems -- interleave the blocks instead.)
-    int pb_lo = 0, pb_hi = n_pb, gw = blockIdx.x * 4 + wave, GW = gridDim.x * 4;  // GW is a multiple of n_ocg
-    if ((gridDim.x & 7) == 0 && ((gridDim.x >> 3) * 4) % n_ocg == 0) {
-        const int x = blockIdx.x & 7, per = n_pb >> 3, rem = n_pb & 7;
-        pb_lo = x * per + (x < rem ? x : rem);
-        pb_hi = pb_lo + per + (x < rem ? 1 : 0);
-        gw = (blockIdx.x >> 3) * 4 + wave;
-        GW = (gridDim.x >> 3) * 4;
-    }
-    const int q0 = gw / n_ocg, ocg = gw - q0 * n_ocg, step = GW / n_ocg;
-    const int pb0 = pb_lo + q0;
-    const int oc_w = ocg * MT * 32;
+    int pb0, pb_hi, ocg;
+    pw_walk(w, n_pb, wave, &pb0, &pb_hi, &ocg);
+    const int oc_w = ocg * MT * 32, step = w.step;
     const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes);
     const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, a.flt_bytes);
     const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
@@ -483,9 +539,9 @@ int launch32_mt(hipStream_t st, const IgemmArgs& a, int cu_count) {
     if (a.epi.has_z) {
         ResidualTable tab;
         if (a.epi.zlin) memcpy(tab.v, a.ztab, sizeof(tab.v)); else memset(tab.v, 0, sizeof(tab.v));
-        return launch_kernel((pw32s_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, tab);
+        return launch_kernel((pw32s_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, make_walk(blocks, n_ocg), n_pb, tab);
     }
-    return launch_kernel((pw32s_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, NoResidualTable{});
+    return launch_kernel((pw32s_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, make_walk(blocks, n_ocg), n_pb, NoResidualTable{});
 }
 
 template <int MT, int KC>
@@ -504,18 +560,18 @@ int launch_quad(hipStream_t st, const IgemmArgs& a, int cu_count) {
     if (2 * blocks >= unit) blocks = (blocks + unit - 1) / unit * unit;
     const FastDiv div_g = make_fastdiv(groups);
     if (a.epi.has_z)
-        return launch_kernel((pw4q_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, groups, div_g);
-    return launch_kernel((pw4q_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, n_ocg, n_pb, groups, div_g);
+        return launch_kernel((pw4q_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, make_walk(blocks, n_ocg), n_pb, groups, div_g);
+    return launch_kernel((pw4q_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, make_walk(blocks, n_ocg), n_pb, groups, div_g);
 }
 
-template <int MT>
-int launch_split(hipStream_t st, const IgemmArgs& a, int waves) {
+template <int MT, int W>
+int launch_split(hipStream_t st, const IgemmArgs& a) {
     const int tiles_m = (a.OC + MT * 16 - 1) / (MT * 16);
     const int groups = (a.OHW + 3) / 4;
     const int tiles_n = (int)(((int64_t)a.NB * groups + 15) / 16);
     const int64_t grid = (int64_t)((tiles_n + 7) / 8) * 8 * tiles_m;
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
-    return launch_kernel(pw4k_kernel<MT>, dim3((unsigned)grid), dim3(waves * 64), waves > 1 ? waves * MT * 4096 : 0, st, a, tiles_m, tiles_n,
+    return launch_kernel(pw4k_kernel<MT, W>, dim3((unsigned)grid), dim3(W * 64), W > 1 ? W * MT * 4096 : 0, st, a, tiles_m, tiles_n,
                          groups, make_fastdiv(groups), make_fastdiv(tiles_m));
 }
 
@@ -618,7 +674,9 @@ int launch_pw4_split(hipStream_t st, const IgemmArgs& a) {
     if (a.M == 0 || a.OC == 0) return 0;
     QuadPlan q = quad_plan(a);
     if (q.waves == 0) q = {4, 1};
-    return q.mt == 1 ? launch_split<1>(st, a, q.waves) : q.mt == 2 ? launch_split<2>(st, a, q.waves) : launch_split<4>(st, a, q.waves);
+    if (q.waves == 1) return q.mt == 1 ? launch_split<1, 1>(st, a) : q.mt == 2 ? launch_split<2, 1>(st, a) : launch_split<4, 1>(st, a);
+    if (q.waves == 2) return launch_split<2, 2>(st, a);
+    return q.mt == 1 ? launch_split<1, 4>(st, a) : q.mt == 2 ? launch_split<2, 4>(st, a) : launch_split<4, 4>(st, a);
 }
 
 int launch_pw4s(hipStream_t st, const IgemmArgs& a, int cu_count) {
