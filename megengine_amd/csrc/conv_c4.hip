@@ -41,7 +41,8 @@ struct C4Args {
     uint32_t src_bytes, dst_bytes, dst_bytes_z;  // extents for the buffer descriptors
     int has_bias;
     int tiles_w, tiles_h, tiles_m, tiles;  // tile = ((mt * N + n) * tiles_h + th) * tiles_w + tw
-    FastDiv div_tw, div_th, div_n;
+    int step;  // the number of workgroups
+    FastDiv div_tw, div_th, div_n, div_step;
     EpiParams epi;
 };
 
@@ -122,7 +123,7 @@ template <int S, bool HZ, int FHT>
 __global__ __launch_bounds__(C4_THREADS, FHT ? 3 : 2) void c4_kernel(C4Args a) {
     using G = C4Geom<S>;
     __shared__ __attribute__((aligned(16))) uint32_t sP[G::NSLOT * G::SLOT_DW];
-    __shared__ __attribute__((aligned(16))) uint32_t sW[C4_BM * (C4_MAXF * 8 + 4)];
+    __shared__ __attribute__((aligned(16))) uint32_t sW[C4_BM * C4_MAXF * C4_MAXF + 8];  // (+ 8: the last row is read in whole fragments)
     __shared__ __attribute__((aligned(16))) int sBias[C4_BM];
 
     const int t = threadIdx.x;
@@ -132,9 +133,13 @@ __global__ __launch_bounds__(C4_THREADS, FHT ? 3 : 2) void c4_kernel(C4Args a) {
     const int FH = FHT ? FHT : a.FH;
     const int rows = (C4_TH - 1) * S + FH;
 
-    const int first = blockIdx.x, step = gridDim.x;
+    // what the copies and the weights need in one batch of scalar loads, and a word of each line that the epilogue reads
+    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.N), "s"(a.IH), "s"(a.IW), "s"(a.OH), "s"(a.OW), "s"(a.OC),
+                 "s"(a.FH), "s"(a.FW), "s"(a.ph), "s"(a.pw), "s"(a.src_sn), "s"(a.src_bytes), "s"(a.has_bias), "s"(a.tiles), "s"(a.tiles_w),
+                 "s"(a.tiles_h), "s"(a.div_tw.m), "s"(a.div_th.m), "s"(a.div_n.m), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(a.step));
+    const int first = blockIdx.x, step = a.step;
     if (first >= a.tiles) return;
-    const int count = (a.tiles - 1 - first) / step + 1;  // tiles of this workgroup
+    const int count = (int)fdiv(a.tiles - 1 - first, a.div_step) + 1;  // tiles of this workgroup
 
     const uint32_t lds_p = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)sP);
     const v4i rs_src = uniform_rsrc(a.src, a.src_bytes);
@@ -163,50 +168,49 @@ __global__ __launch_bounds__(C4_THREADS, FHT ? 3 : 2) void c4_kernel(C4Args a) {
     };
 
     // A fragments of every filter row: lane (l32, lh) holds taps 4 * lh .. 4 * lh + 3 of channel i * 32 + l32, zeros for
-    // taps >= FW and channels >= OC.  The filter is read once per channel tile with consecutive threads on consecutive
-    // dwords, re-blocked in LDS to 8 taps per row (16 bytes of padding per channel: conflict-free 128-bit reads), and
-    // from there each lane takes its fragments.
+    // taps >= FW and channels >= OC.  The filter rows of a channel tile are one contiguous piece of memory: it is copied to LDS
+    // as it is, 16 bytes per thread and load, all loads of a thread in flight at once (past the end of the filter the
+    // descriptor answers zeros), and from there each lane takes its fragments; FH * FW dwords per channel are an odd number for
+    // the usual filters, so the 32 channels of a read lie on 32 banks.  (Dword by dword under a condition the compiler put a
+    // branch and a wait around every load, fourteen round trips in a row: 2 us of the 5.3 of a layer of one image.)
+    const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, (uint32_t)(a.OC * FH * a.FW * 4));
+    const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
     v4i wr[C4_MAXF][2];
-    const int wrow_dw = FH * 8 + 4;
     auto stage_weights = [&](int mt) __attribute__((always_inline)) {
-        const uint32_t* fp = reinterpret_cast<const uint32_t*>(a.flt);
-        const int per_oc = FH * 8, total = C4_BM * per_oc;
-        // thread indices through an opaque copy: nothing of this rarely run block is kept in registers across the tile loop
+        const int bytes = C4_BM * FH * a.FW * 4;
+        // the thread index through an opaque copy: nothing of this rarely run block is kept in registers across the tile loop
         int tid = t;
         asm volatile("" : "+v"(tid));
-        constexpr int HALF = C4_BM * C4_MAXF * 8 / C4_THREADS / 2;
+        constexpr int VECS = (C4_BM * (FHT ? FHT : C4_MAXF) * C4_MAXF * 4 + C4_THREADS * 16 - 1) / (C4_THREADS * 16);
+        v4i v[VECS];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            uint32_t v[HALF];
-#pragma unroll
-            for (int j = 0; j < HALF; ++j) {  // a batch of loads before the first LDS write
-                const int idx = tid + C4_THREADS * (h * HALF + j);
-                const int oc = idx / per_oc, rem = idx - oc * per_oc;
-                const int fh = rem >> 3, tap = rem & 7;
-                const int goc = mt * C4_BM + oc;
-                v[j] = (idx < total && goc < a.OC && tap < a.FW) ? fp[(goc * FH + fh) * a.FW + tap] : 0u;
-            }
-#pragma unroll
-            for (int j = 0; j < HALF; ++j) {
-                const int idx = tid + C4_THREADS * (h * HALF + j);
-                const int oc = idx / per_oc, rem = idx - oc * per_oc;
-                if (idx < total) sW[oc * wrow_dw + rem] = v[j];
-            }
+        for (int j = 0; j < VECS; ++j) {
+            const int at = (tid + C4_THREADS * j) * 16;
+            v[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, at < bytes ? mt * bytes + at : SENT, 0, 0);
         }
+        const int b = __builtin_amdgcn_raw_buffer_load_b32(rs_bias, tid < C4_BM ? (mt * C4_BM + tid) * 4 : SENT, 0, 0);
+#pragma unroll
+        for (int j = 0; j < VECS; ++j) {
+            const int at = (tid + C4_THREADS * j) * 16;
+            if (at < bytes) *reinterpret_cast<v4i*>(reinterpret_cast<char*>(sW) + at) = v[j];
+        }
+        if (tid < C4_BM) sBias[tid] = b;
     };
     auto read_weights = [&]() __attribute__((always_inline)) {
+        int ln = lane;
+        asm volatile("" : "+v"(ln));  // (as above)
+        const uint32_t* p = sW + (ln & 31) * FH * a.FW + 4 * (ln >> 5);
+        int keep[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) keep[k] = 4 * (ln >> 5) + k < a.FW ? -1 : 0;
 #pragma unroll
         for (int fh = 0; fh < C4_MAXF; ++fh) {
             if (fh < FH) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) wr[fh][i] = *reinterpret_cast<const v4i*>(sW + (i * 32 + l32) * wrow_dw + fh * 8 + lh * 4);
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) wr[fh][i][k] = (int)p[i * 32 * FH * a.FW + fh * a.FW + k] & keep[k];
             }
-        }
-    };
-    auto load_bias = [&](int mt) __attribute__((always_inline)) {
-        if (t < C4_BM) {
-            const int goc = mt * C4_BM + t;
-            sBias[t] = (a.has_bias && goc < a.OC) ? a.bias[goc] : 0;
         }
     };
 
@@ -221,7 +225,6 @@ __global__ __launch_bounds__(C4_THREADS, FHT ? 3 : 2) void c4_kernel(C4Args a) {
     if (count > 2) { issued += copy_patch(2); mk2 = issued; }
     C4Tile tl = c4_decode(a, first);
     stage_weights(tl.mt);
-    load_bias(tl.mt);
     __builtin_amdgcn_s_waitcnt(C4_VMCNT0);  // the first patches have landed (this wave's copies; the barrier covers the rest)
     __syncthreads();
     read_weights();
@@ -288,7 +291,6 @@ __global__ __launch_bounds__(C4_THREADS, FHT ? 3 : 2) void c4_kernel(C4Args a) {
             __syncthreads();
             if (tn.mt != tl.mt) {  // every wave has read the old bias; the old weights are dead
                 stage_weights(tn.mt);
-                load_bias(tn.mt);
                 __syncthreads();
                 read_weights();
             }
@@ -373,6 +375,8 @@ int launch_conv_c4(hipStream_t st, const ConvProblem& p, int cu_count, const int
     }
     int64_t grid = (int64_t)occ[si].load(std::memory_order_relaxed) * cu_count;
     if (grid > a.tiles) grid = a.tiles;
+    a.step = (int)grid;
+    a.div_step = make_fastdiv((uint32_t)grid);
     return launch_kernel(kerns[si], dim3((unsigned)grid), dim3(C4_THREADS), 0, st, a);
 }
 
