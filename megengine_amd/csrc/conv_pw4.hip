@@ -22,6 +22,11 @@ namespace {
 
 constexpr int PW4_MAX_OC = 1024;
 
+// All loads so far have landed, and the compiler knows.  Ahead of a loop whose loads run a step ahead: with the first step's
+// loads possibly pending at the loop's head, the wait that the compiler puts there is for everything, the stores of the step
+// before included.
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+
 // How the waves of a streaming launch walk the pixel blocks: wave g of the launch (of its XCD's share of the launch) takes the
 // channel group g % n_ocg of the blocks g / n_ocg, + step, ...  With slabs the XCDs take one contiguous eighth of the blocks
 // each.  The divisions are the host's: a run-time integer division is 0.1 us on the way to the first load.
@@ -186,6 +191,7 @@ __global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, PwWalk w, int
     for (int i = 0; i < MT * 32; i += 64)
         if (i + lane < MT * 32) bias_w[i + lane] = bias_v[i / 64];
     __builtin_amdgcn_wave_barrier();
+    wait_loads();
     const int tail = a.OHW & 3;
     auto blocks = [&](auto nl) __attribute__((always_inline)) {
         constexpr int NL = decltype(nl)::value;
@@ -204,7 +210,7 @@ __global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, PwWalk w, int
             const int z0 = (int)n * a.z_sn + (int)g * 16 + ((oc_w >> 2) + lh) * a.dst_scb;
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                if (oc_w + i * 32 >= a.OC) break;  // wave-uniform
+                if (i > 0 && oc_w + i * 32 >= a.OC) break;  // wave-uniform (a wave's first block always holds channels)
                 v4i zv[4];
                 if constexpr (HZ)
 #pragma unroll
@@ -363,6 +369,7 @@ __global__ __launch_bounds__(W * 64, 2) void pw4k_kernel(IgemmArgs a, int tiles_
             for (int u = 0; u < AHEAD; ++u) {
                 multiply(fa[u], x[u]);
                 load(fa[u], x[u]);
+                __builtin_amdgcn_sched_barrier(0);  // (or the loads of all steps end up behind the last product)
             }
         }
 #pragma unroll
@@ -501,26 +508,47 @@ __global__ __launch_bounds__(256, 2) void pw32s_kernel(IgemmArgs a, PwWalk w, in
     ZRegs<HZ ? MT : 1, 1> zr, nz;
     load_b(pb0 < pb_hi ? pb0 : n_pb, fb);
     if constexpr (HZ) igemm_load_z<32, MT, 1>(a, zr, oc_w, (pb0 < pb_hi ? pb0 : n_pb) * 32, l32, lh);
-    for (int pb = pb0; pb < pb_hi; pb += step) {
-        // the next block's pixels and residual are in flight during the multiply and the epilogue (past the end of this
-        // XCD's blocks: the block past the last one, whose lanes are all masked)
-        const int nx = pb + step < pb_hi ? pb + step : n_pb;
-        load_b(nx, nb);
-        if constexpr (HZ) igemm_load_z<32, MT, 1>(a, nz, oc_w, nx * 32, l32, lh);
-        v16i acc[MT][1];
+    wait_loads();
+    // one loop per form of the epilogue: a choice inside the loop, and a branch around a wave's first block, which always
+    // holds channels, leave the compiler unable to count the stores of a step, and it waits for them at the next one
+    auto blocks = [&](auto nl) __attribute__((always_inline)) {
+        constexpr int NL = decltype(nl)::value;
+        for (int pb = pb0; pb < pb_hi; pb += step) {
+            // the next block's pixels and residual are in flight during the multiply and the epilogue (past the end of this
+            // XCD's blocks: the block past the last one, whose lanes are all masked)
+            const int nx = pb + step < pb_hi ? pb + step : n_pb;
+            load_b(nx, nb);
+            if constexpr (HZ) igemm_load_z<32, MT, 1>(a, nz, oc_w, nx * 32, l32, lh);
+            v16i acc[MT][1][1];
 #pragma unroll
-        for (int i = 0; i < MT; ++i) acc[i][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i][0], fb[0], bv[i], 0, 0, 0);
+            for (int i = 0; i < MT; ++i) acc[i][0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i][0], fb[0], bv[i], 0, 0, 0);
 #pragma unroll
-        for (int kc = 1; kc < KC; ++kc)
+            for (int kc = 1; kc < KC; ++kc)
 #pragma unroll
-            for (int i = 0; i < MT; ++i) acc[i][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i][kc], fb[kc], acc[i][0], 0, 0, 0);
-        if constexpr (HZ)
-            igemm_run_epilogue<32, MT, 1, true>(a, acc, oc_w, pb * 32, l32, lh, &zr, -1, 1, 0, -1, zt);
-        else
-            igemm_run_epilogue<32, MT, 1>(a, acc, oc_w, pb * 32, l32, lh);
+                for (int i = 0; i < MT; ++i) acc[i][0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i][kc], fb[kc], acc[i][0][0], 0, 0, 0);
 #pragma unroll
-        for (int kc = 0; kc < KC; ++kc) fb[kc] = nb[kc];
-        if constexpr (HZ) zr = nz;
+            for (int i = 0; i < MT; ++i) {
+                if (i > 0 && oc_w + i * 32 >= a.OC) break;  // wave-uniform
+                ZRegs<1, 1> z1;
+                if constexpr (HZ) z1.v[0][0] = zr.v[i][0];
+                igemm_epilogue<32, 1, 1, NL, HZ, HZ>(a, acc[i], &z1, oc_w + i * 32, pb * 32, l32, lh, 0x7fffffff, 1, 0, a.M, zt);
+            }
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc) fb[kc] = nb[kc];
+            if constexpr (HZ) zr = nz;
+        }
+    };
+    using std::integral_constant;
+    if (HZ && a.epi.zlin) {
+        if constexpr (HZ) blocks(integral_constant<int, NL_ZLIN>{});
+    } else if (!HZ && a.epi.lin) {
+        if constexpr (!HZ) blocks(integral_constant<int, NL_LIN>{});
+    } else {
+        switch (a.epi.nonline) {
+            case NL_RELU: blocks(integral_constant<int, NL_RELU>{}); break;
+            case NL_H_SWISH: blocks(integral_constant<int, NL_H_SWISH>{}); break;
+            default: blocks(integral_constant<int, NL_IDENTITY>{}); break;
+        }
     }
 }
 
