@@ -791,9 +791,17 @@ static int exec_impl(void* stream, const mi355_conv_desc* d, const mi355_algo* a
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     int rc = 0;
     switch (id) {
-        case ALGO_DIRECT:
-            rc = launch_conv_direct(hs, p, src, filter, bias, z, dst);
+        case ALGO_DIRECT: {
+            // Plain NCHW without a workspace, chosen by the library itself: the planar patch kernel wherever it runs.  A thread of
+            // the generic kernel walks its reduction alone, 0.27 us per 32-bit word of it: from five bytes on it is behind (1x1
+            // over 6 channels, 101 x 7 pixels: 5.1 us / 4.6; 3x3 over 256, 6 x 6: 617 / 15).  Named by the caller it runs as itself.
+            const bool planar = by_heuristic && d->format == MI355_FMT_NCHW && p.icpg * d->fh * d->fw >= 5 &&
+                                (reinterpret_cast<uintptr_t>(bias) & 3) == 0;
+            const int tile = planar ? patch1_pick(p, false) : -1;
+            rc = tile >= 0 ? launch_patch1(hs, p, tile, src, filter, bias, z, reinterpret_cast<int8_t*>(dst))
+                           : launch_conv_direct(hs, p, src, filter, bias, z, dst);
             break;
+        }
         case ALGO_IGEMM_MFMA:
             rc = launch_conv_igemm(hs, p, cfg, cu_count(), src, filter, bias, z, reinterpret_cast<int8_t*>(dst), preprocessed);
             break;

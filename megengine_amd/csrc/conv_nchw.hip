@@ -11,8 +11,8 @@
 // and the implicit GEMM reads those, and bias, residual and destination as they are: its planar epilogue knows NCHW.
 // Padded input channels are zero bytes (they add nothing to a sum).  The arithmetic is that of the packed kernels, which
 // is bit-exact to the reference's naive path; a permutation of the operands changes no integer sum.
-// 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual (3.3 Gop): 48.8 us as four conversions, two fills and a
-// convolution, 16.3 us as two launches.
+// Most sizes with filters of 1x1, 3x3 and 5x5 need neither the packing nor the workspace: conv_patch1.hip reads the planes
+// themselves, and patch1_pick says where it is ahead.
 #include <string.h>
 
 #include "igemm_shared.h"
@@ -135,6 +135,8 @@ int launch_conv_nchw_mfma(hipStream_t st, const ConvProblem& p, int cu_count, co
     if (!make_layout(p, &L)) return (int)hipErrorInvalidValue;
     const mi355_conv_desc& d = p.d;
     if ((uint64_t)d.n * d.oc * p.oh * p.ow == 0) return 0;
+    const int tile = patch1_pick(p, true);  // no packing where the kernel that reads the planes is ahead
+    if (tile >= 0) return launch_patch1(st, p, tile, src, flt, bias, z, dst);
     int8_t* ws = reinterpret_cast<int8_t*>(workspace);
     const uint32_t HW = d.ih * d.iw;
     PrepArgs a;

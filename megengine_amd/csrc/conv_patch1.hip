@@ -1,0 +1,505 @@
+// Plain NCHW convolutions in one launch, no workspace: the input patch and the filter are turned on their way into LDS.
+//
+// The matrix cores want sixteen reduction bytes side by side, and an NCHW tensor keeps every channel in a plane of its own.
+// Packing it in a launch ahead of the convolution (conv_nchw.hip) costs that launch, the gap behind it, a round trip through
+// memory and the padding of 75 channels to 96.  Here a workgroup stages the patch of its tile -- rows and columns with their halo, sixteen
+// channels at a time -- as [group of 16 channels][patch pixel][16 bytes], as the 4-packed patch kernel does (conv_patch4.hip),
+// so that the operand of a tap is one ds_read_b128 at a shifted pixel:
+//   * A thread takes four neighbouring pixels of sixteen channels: sixteen dword loads at any address, consecutive lanes
+//     consecutive dwords of a row, and turns them with v_perm into four 16-byte vectors.  The selectors of v_perm are per lane
+//     and made once per tile: they put zeros where a column lies outside the image, move the bytes of a dword that was loaded
+//     further left because the row ends inside it, and turn the order of the four pixels by lane, so that the 16-byte writes of
+//     eight lanes meet eight different bank groups.
+//   * The filter's rows are [channel][tap] bytes: a thread takes four channels of a row, 4 T contiguous bytes, and T times three
+//     v_perm with constant selectors make the T dwords (four channels of one tap) that an operand is made of.
+//   * Two stages in LDS, the next one's loads in registers while the current one is multiplied, one barrier per stage.
+//   * Bound by LDS, as the 4-packed patch tiles are, and by the latency of a stage where tiles are few.
+// Filters of 1x1, 3x3 and 5x5; others go through the
+// workspace.  Graph replays: 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual: 17.3 us packed, 13.2 here (four waves of
+// 1200 vector instructions for 23 products each, a third of their time waiting for a stage's loads); more at patch1_pick.
+#include <algorithm>
+#include <atomic>
+
+#include "igemm_shared.h"
+#include "relayout_parts.h"
+
+namespace mi355 {
+namespace {
+
+constexpr int P1_NPI = 2;          // pixel quads per thread and stage
+constexpr int P1_VMCNT0 = 0x0f70;  // s_waitcnt vmcnt(0), the other counters at their maxima
+
+constexpr int p1_gs(int t) { return t == 1 ? 4 : t == 9 ? 2 : 1; }  // channel groups of a stage
+constexpr int p1_f(int t) { return t == 1 ? 1 : t == 9 ? 3 : 5; }
+constexpr int p1_bmp(int mt) { return mt * 32 + 1; }  // odd: the dword writes of a filter row spread over the banks
+
+struct P1Args {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    int IC, IH, IW, IHW, OC, OH, OW, OHW, N, sh, sw, ph, pw;
+    int src_sn, dst_sn, z_sn, kbytes, flt_bytes, has_bias, nstages;
+    uint32_t src_bytes, dst_bytes, z_bytes;
+    int NI, TH, TW, PWC, PXI, PX, PXQ;  // images, rows, columns of a tile; patch columns (a multiple of 4), pixels per image, pixels, quads
+    int tiles_m, tiles_n, tiles_img, tiles_w;
+    FastDiv div_tiles_m, div_tiles_img, div_tiles_w, div_tw, div_tile_px, div_pqi, div_pqw;
+    EpiParams epi;
+};
+
+typedef uint32_t u32_at __attribute__((aligned(1)));
+
+// byte b of 4 T contiguous bytes
+template <int T>
+__device__ __forceinline__ uint32_t p1_tap(const uint32_t (&x)[T], int tap) {
+    const int b0 = tap, b1 = T + tap, b2 = 2 * T + tap, b3 = 3 * T + tap;
+    const uint32_t lo = __builtin_amdgcn_perm(x[b1 >> 2], x[b0 >> 2], (uint32_t)(0x0c0c0400 | (b0 & 3) | (b1 & 3) << 8));
+    const uint32_t hi = __builtin_amdgcn_perm(x[b3 >> 2], x[b2 >> 2], (uint32_t)(0x04000c0c | (b2 & 3) << 16 | (b3 & 3) << 24));
+    return lo | hi;
+}
+
+// where four neighbouring lanes put (and find the residual of) their four columns: offset of channel ch = 4 lh + l32 % 4 of the
+// first eight channels, and the columns from there to the row's end (0: nothing)
+struct P1Out {
+    int d0, z0, cols;
+};
+__device__ __forceinline__ P1Out p1_out(const P1Args& a, int p, int n0, int oh0, int ow0, int ch) {
+    const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)(a.TH * a.TW), oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
+    const bool in = ((int)im < a.NI) & (n0 + (int)im < a.N) & (oh0 + (int)oh < a.OH);
+    const int px = (oh0 + (int)oh) * a.OW + ow0 + (int)ow + ch * a.OHW;
+    return {(n0 + (int)im) * a.dst_sn + px, (n0 + (int)im) * a.z_sn + px, in ? a.OW - (ow0 + (int)ow) : 0};
+}
+
+template <int MT, int NT, int NL, bool HZ>
+__device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT], const uint32_t (&zq)[NT][MT][4], int n0, int oh0, int ow0, int oc0,
+                                            int wave, int l32, int lh) {
+    const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes), rs_z = make_rsrc(a.z, HZ ? a.z_bytes : 0);
+    const int lane4 = l32 & 3, ch = 4 * lh + lane4;  // after the exchange a lane holds four columns of channel ch of every eight
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const P1Out w = p1_out(a, (wave * NT + j) * 32 + (l32 & ~3), n0, oh0, ow0, ch);
+        const int d0 = w.d0, z0 = w.z0, cols = w.cols;
+        const bool part = (cols > 0) & (cols < 4), split = __builtin_amdgcn_ballot_w64(part) != 0;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int oc8 = oc0 + i * 32 + 8 * q, at = oc8 * a.OHW;  // wave-uniform
+                const bool ok = oc8 + ch < a.OC;
+                uint32_t zw = 0;
+                if (HZ) {
+                    zw = MT * NT <= 2 ? zq[j][i][q] : (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, (ok & (cols >= 4)) ? z0 : SENT, at, 0);
+                    if (split) {
+#pragma unroll
+                        for (int k = 0; k < 3; ++k)
+                            zw |= (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rs_z, (ok & part & (k < cols)) ? z0 + k : SENT, at, 0) << (8 * k);
+                    }
+                    zw = quad_transpose(zw, lane4);
+                }
+                const v16i& c = acc[i][j];
+                const uint32_t o = quad_transpose(requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], zw, a.epi), lane4);
+                __builtin_amdgcn_raw_buffer_store_b32((int)o, rs_dst, (ok & (cols >= 4)) ? d0 : SENT, at, 0);
+                if (split) {
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(o >> (8 * k)), rs_dst, (ok & part & (k < cols)) ? d0 + k : SENT, at, 0);
+                }
+            }
+    }
+}
+
+template <int MT, int NT, int T>
+__global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
+    constexpr int NPI = P1_NPI;
+    constexpr bool ZPRE = MT * NT <= 2;  // the residual is asked for ahead of the products (the largest tile has no registers for it)
+    constexpr int BM = MT * 32, GS = p1_gs(T), F = p1_f(T), E = GS * T, EP = (E + 1) & ~1, STEPS = EP / 2, BMP = p1_bmp(MT);
+    constexpr int TPG = 256 / GS;                          // threads per channel group of the patch
+    constexpr int QPR = 4 * GS;                            // channel quads of a filter row and stage
+    constexpr int FI = (BM * QPR + 255) / 256;             // filter items per thread and stage
+    constexpr int A_VECS = EP * BMP;
+    extern __shared__ __attribute__((aligned(16))) v4i lds[];
+    __shared__ __attribute__((aligned(16))) int sBias[BM];
+    // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
+    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.IC), "s"(a.IH), "s"(a.IW), "s"(a.IHW), "s"(a.OC), "s"(a.N),
+                 "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.src_sn), "s"(a.kbytes), "s"(a.flt_bytes), "s"(a.has_bias), "s"(a.nstages),
+                 "s"(a.NI), "s"(a.TH), "s"(a.TW), "s"(a.PWC), "s"(a.PX), "s"(a.PXQ), "s"(a.tiles_m));
+    asm volatile("" ::"s"(a.tiles_n), "s"(a.tiles_img), "s"(a.tiles_w), "s"(a.div_tiles_m.m), "s"(a.div_tiles_img.m), "s"(a.div_tiles_w.m),
+                 "s"(a.div_pqi.m), "s"(a.div_pqi.s2), "s"(a.div_pqw.m), "s"(a.div_pqw.s2), "s"(a.div_tile_px.m), "s"(a.div_tw.m), "s"(a.epi.s_b),
+                 "s"(a.epi.lin_lo));
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l32 = lane & 31, lh = lane >> 5;
+    const int stage_vecs = A_VECS + GS * a.PX;
+
+    // tile: contiguous pixel tiles per XCD (workgroup b runs on XCD b % 8), channel tiles of a pixel tile side by side
+    int tm, tn;
+    {
+        const int per = (a.tiles_n + 7) >> 3, x = blockIdx.x & 7, i = blockIdx.x >> 3;
+        const int r = (int)fdiv(i, a.div_tiles_m);
+        tm = i - r * a.tiles_m;
+        tn = x * per + r;
+        if (r >= per || tn >= a.tiles_n) return;
+    }
+    const int ig = (int)fdiv(tn, a.div_tiles_img), ti = tn - ig * a.tiles_img;
+    const int th = (int)fdiv(ti, a.div_tiles_w), tw = ti - th * a.tiles_w;
+    const int n0 = ig * a.NI, oh0 = th * a.TH, ow0 = tw * a.TW, oc0 = tm * BM;
+    const int iw_lo = (ow0 * a.sw - a.pw) & ~3;  // the patch starts at a column that is a multiple of four: a quad that starts
+                                                 // inside a row starts at one of its columns
+
+    // Patch quads of this thread.  Waves of a group of TPG threads share a channel group, so a channel's plane is a scalar base.
+    const int g = GS == 1 ? 0 : wave / (TPG / 64), tg = t & (TPG - 1);
+    uint32_t p_sel[NPI][4];
+    int p_off[NPI], p_lds[NPI];
+    const int turn = (tg >> 1) & 3;
+#pragma unroll
+    for (int k = 0; k < NPI; ++k) {
+        const uint32_t pq = tg + k * TPG, im = fdiv(pq, a.div_pqi), r = pq - im * (uint32_t)(a.PXI >> 2);
+        const uint32_t pr = fdiv(r, a.div_pqw), pc = (r - pr * (uint32_t)(a.PWC >> 2)) * 4;
+        const int ih = oh0 * a.sh - a.ph + (int)pr, iw = iw_lo + (int)pc, n = n0 + (int)im;
+        const bool ok = ((int)pq < a.PXQ) & (n < a.N) & ((unsigned)ih < (unsigned)a.IH) & ((unsigned)iw < (unsigned)a.IW);
+        const int back = iw + 4 > a.IW ? iw + 4 - a.IW : 0;  // the row ends inside the quad: loaded `back` columns further left
+        p_off[k] = ok ? n * a.src_sn + ih * a.IW + iw - back : SENT;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int p = ((j + turn) & 3) + back;  // byte of the loaded dword that is this pixel
+            p_sel[k][j] = ok && p < 4 ? 0x00000400u | (uint32_t)(p | p << 8) : 0x0c0cu;
+            p_sel[k][j] |= 0x0c0c0000u;
+        }
+        p_lds[k] = (int)pq < a.PXQ ? A_VECS + g * a.PX + (int)pq * 4 : -1;
+    }
+    // filter items of this thread: four channels of a row
+    const int f_quad = t & (QPR - 1), f_row = t / QPR;
+    constexpr int ROWS_PER_PASS = 256 / QPR;
+    int f_off[FI];
+#pragma unroll
+    for (int k = 0; k < FI; ++k) {
+        const int row = f_row + k * ROWS_PER_PASS;
+        f_off[k] = row < BM && oc0 + row < a.OC ? (oc0 + row) * a.kbytes + f_quad * 4 * T : -1;
+    }
+
+    const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes), rs_flt = make_rsrc(a.flt, (uint32_t)a.flt_bytes);
+    const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
+    uint32_t xp[NPI][16], xf[FI][T];
+    const bool two = a.PXQ > TPG;  // a second quad per thread
+    auto fetch = [&](int st) __attribute__((always_inline)) {
+        const int c0 = (st * GS + g) * 16;
+#pragma unroll
+        for (int k = 0; k < FI; ++k) {
+            // (a quad past the last channel, or whose bytes pass the end of the filter, is not loaded here, see store)
+            const int at = f_off[k] + st * GS * 16 * T;
+            const bool in = (f_off[k] >= 0) & (st * GS * 16 + f_quad * 4 < a.IC) & (at + 4 * T <= a.flt_bytes);
+            const int v0 = in ? at : SENT;
+#pragma unroll
+            for (int v = 0; v + 4 <= T; v += 4) {
+                const v4i y = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, v0 + 4 * v, 0, 0);
+                xf[k][v] = y[0]; xf[k][v + 1] = y[1]; xf[k][v + 2] = y[2]; xf[k][v + 3] = y[3];
+            }
+            if constexpr (T % 4 != 0) xf[k][T - 1] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_flt, v0 + 4 * (T - 1), 0, 0);
+        }
+        // (channels past the last one meet zero filter bytes; the scalar offset never leads out of the image)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            xp[0][i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_src, p_off[0], min(c0 + i, a.IC - 1) * a.IHW, 0);
+        if (two)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                xp[NPI - 1][i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_src, p_off[NPI - 1], min(c0 + i, a.IC - 1) * a.IHW, 0);
+    };
+    auto store = [&](int st) __attribute__((always_inline)) {
+        v4i* s = lds + (st & 1) * stage_vecs;
+        uint32_t* sw = reinterpret_cast<uint32_t*>(s);
+#pragma unroll
+        for (int k = 0; k < FI; ++k) {
+            const int row = f_row + k * ROWS_PER_PASS, left = a.IC - (st * GS * 16 + f_quad * 4);  // channels from here on
+            uint32_t keep = left >= 4 ? 0xffffffffu : left > 0 ? (1u << (8 * left)) - 1 : 0u;
+            const int at = f_off[k] + st * GS * 16 * T;
+            if (f_off[k] < 0) keep = 0;
+            if (keep != 0 && at + 4 * T > a.flt_bytes) {  // the last quad of the last row
+#pragma unroll
+                for (int v = 0; v < T; ++v) {
+                    uint32_t w = 0;
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+                        w |= (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rs_flt, 4 * v + b < left * T ? at + 4 * v + b : SENT, 0, 0) << (8 * b);
+                    xf[k][v] = w;
+                }
+            }
+            if (BM * QPR >= 256 || row < BM)
+#pragma unroll
+                for (int tap = 0; tap < T; ++tap)
+                    sw[(((f_quad >> 2) * T + tap) * BMP + row) * 4 + (f_quad & 3)] = p1_tap<T>(xf[k], tap) & keep;
+        }
+#pragma unroll
+        for (int k = 0; k < NPI; ++k) {
+            if (k == 1 && !two) break;
+            if (p_lds[k] >= 0)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v4i o;
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const uint32_t lo = __builtin_amdgcn_perm(xp[k][4 * c + 1], xp[k][4 * c], p_sel[k][j]);
+                        const uint32_t hi = __builtin_amdgcn_perm(xp[k][4 * c + 3], xp[k][4 * c + 2], p_sel[k][j]);
+                        o[c] = (int)(lo | hi << 16);
+                    }
+                    s[p_lds[k] + ((j + turn) & 3)] = o;
+                }
+        }
+    };
+    const int bias_v = __builtin_amdgcn_raw_buffer_load_b32(rs_bias, (oc0 + (t & (BM - 1))) * 4, 0, 0);
+    fetch(0);
+
+    // the filter entry that fills up an odd number stays zero, and the bias
+    if (EP != E)
+        for (int u = t; u < 2 * BM; u += 256) lds[(u / BM) * stage_vecs + E * BMP + u % BM] = v4i{0, 0, 0, 0};
+    if (t < BM) sBias[t] = bias_v;
+
+    // B operands: patch vector of each of this lane's pixels, and of each step's entry relative to it
+    int b_px[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const uint32_t p = (wave * NT + j) * 32 + l32;
+        const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)(a.TH * a.TW), oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
+        b_px[j] = (int)im < a.NI ? (int)(im * a.PXI + oh * a.sh * a.PWC) + ((int)ow + ow0) * a.sw - a.pw - iw_lo : 0;
+    }
+    int offs[STEPS];
+#pragma unroll
+    for (int k = 0; k < STEPS; ++k) {
+        const int e0 = 2 * k, e1 = 2 * k + 1 < E ? 2 * k + 1 : 0;  // (the filling entry multiplies any vector by zero)
+        const int o0 = (e0 / T) * a.PX + ((e0 % T) / F) * a.PWC + (e0 % T) % F, o1 = (e1 / T) * a.PX + ((e1 % T) / F) * a.PWC + (e1 % T) % F;
+        offs[k] = A_VECS + (lh ? o1 : o0);
+    }
+    store(0);
+    __builtin_amdgcn_s_waitcnt(P1_VMCNT0);  // (the compiler knows: a stage's products do not wait for the next stage's loads)
+    if (a.nstages > 1) fetch(1);
+    // the residual of whole groups of four columns (a launch without one: a descriptor of no bytes)
+    uint32_t zq[NT][MT][4];
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.epi.has_z ? a.z_bytes : 0);
+    if constexpr (ZPRE)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const P1Out w = p1_out(a, (wave * NT + j) * 32 + (l32 & ~3), n0, oh0, ow0, 4 * lh + (l32 & 3));
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int oc8 = oc0 + i * 32 + 8 * q;
+                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(
+                        rs_z, ((oc8 + 4 * lh + (l32 & 3) < a.OC) & (w.cols >= 4)) ? w.z0 : SENT, oc8 * a.OHW, 0);
+            }
+    }
+    __syncthreads();
+    v16i acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const v4i b = *reinterpret_cast<const v4i*>(sBias + i * 32 + 8 * q + 4 * lh);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                acc[i][j][4 * q] = b[0]; acc[i][j][4 * q + 1] = b[1]; acc[i][j][4 * q + 2] = b[2]; acc[i][j][4 * q + 3] = b[3];
+            }
+        }
+    const int groups = (a.IC + 15) >> 4;
+    auto products = [&](int st) __attribute__((always_inline)) {
+        const v4i* s = lds + (st & 1) * stage_vecs;
+        const v4i* pa = s + lh * BMP + l32;
+        auto load = [&](int k, v4i (&fa)[MT], v4i (&fb)[NT]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) fa[i] = pa[k * 2 * BMP + i * 32];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) fb[j] = s[offs[k] + b_px[j]];
+        };
+        constexpr int AHEAD = 2;  // steps whose operands are read ahead
+        v4i fa[AHEAD + 1][MT], fb[AHEAD + 1][NT];
+#pragma unroll
+        for (int k = 0; k < AHEAD && k < STEPS; ++k) load(k, fa[k], fb[k]);
+#pragma unroll
+        for (int k = 0; k < STEPS; ++k) {
+            // (an incomplete last stage: nothing of the groups past the last one; wave-uniform)
+            if (k > 0 && (2 * k) % T < 2 && st * GS + (2 * k) / T >= groups) break;
+            if (k + AHEAD < STEPS) load(k + AHEAD, fa[(k + AHEAD) % (AHEAD + 1)], fb[(k + AHEAD) % (AHEAD + 1)]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[k % (AHEAD + 1)][i], fb[k % (AHEAD + 1)][j], acc[i][j], 0, 0, 0);
+        }
+    };
+    for (int st = 0;; ++st) {
+        products(st);
+        if (st + 1 >= a.nstages) break;
+        store(st + 1);
+        if (st + 2 < a.nstages) fetch(st + 2);
+        __syncthreads();
+    }
+
+#define MI355_P1(NL, HZ) p1_epilogue<MT, NT, NL, HZ>(a, acc, zq, n0, oh0, ow0, oc0, wave, l32, lh)
+    if (a.epi.lin) {
+        MI355_P1(NL_LIN, false);
+    } else if (a.epi.has_z) {
+        switch (a.epi.nonline) {
+            case NL_RELU: MI355_P1(NL_RELU, true); break;
+            case NL_H_SWISH: MI355_P1(NL_H_SWISH, true); break;
+            default: MI355_P1(NL_IDENTITY, true); break;
+        }
+    } else {
+        switch (a.epi.nonline) {
+            case NL_RELU: MI355_P1(NL_RELU, false); break;
+            case NL_H_SWISH: MI355_P1(NL_H_SWISH, false); break;
+            default: MI355_P1(NL_IDENTITY, false); break;
+        }
+    }
+#undef MI355_P1
+}
+
+constexpr int kP1Tiles[][2] = {{1, 1}, {1, 2}, {2, 2}, {2, 1}};  // 32 x 128, 32 x 256, 64 x 256, 64 x 128
+
+// geometry of a tile; false where no patch fits
+bool p1_plan(const ConvProblem& p, int tile, P1Args* k, int* lds_bytes) {
+    const mi355_conv_desc& d = p.d;
+    const int T = (int)(d.fh * d.fw), F = (int)d.fw, GS = p1_gs(T), mt = kP1Tiles[tile][0], bm = mt * 32, bn = kP1Tiles[tile][1] * 128;
+    const int OH = (int)p.oh, OW = (int)p.ow, sh = (int)d.stride_h, sw = (int)d.stride_w, max_q = P1_NPI * (256 / GS);
+    const int G = ((int)d.ic + 15) / 16;
+    k->nstages = (G + GS - 1) / GS;
+    int64_t best = -1;
+    // equal columns of whole quads, as wide as the tile or narrower; rows (of whole images where one is small) as they fit
+    const int ow4 = (OW + 3) & ~3;
+    for (int most = std::min(bn, ow4), last = 0; most >= std::min(16, ow4); most -= 4) {
+        const int cols = (OW + most - 1) / most, TW = ((OW + cols - 1) / cols + 3) & ~3;
+        if (TW == last) continue;
+        last = TW;
+        // patch columns: the first is rounded down to a multiple of four, whatever the tile's position
+        const int PWC = ((TW - 1) * sw + F + 3 + 3) & ~3;
+        int th = bn / TW, NI = 1;
+        if (th >= OH) {
+            NI = TW >= OW ? th / OH : 1;
+            th = OH;
+        }
+        int TH, PXI, PXQ;
+        for (;;) {
+            const int bands = (OH + th - 1) / th;
+            TH = (OH + bands - 1) / bands;
+            PXI = ((TH - 1) * sh + F) * PWC;
+            while (NI > 1 && NI * PXI / 4 > max_q) --NI;
+            PXQ = NI * PXI / 4;
+            if (PXQ <= max_q || th == 1) break;
+            th = TH - 1;
+        }
+        if (PXQ <= max_q) {
+            const int64_t tiles = ((int64_t)d.n + NI - 1) / NI * cols * ((OH + TH - 1) / TH);
+            // fewest tiles; among those the smallest patch
+            const int64_t cost = tiles * 4096 + PXQ;
+            if (best < 0 || cost < best) {
+                best = cost;
+                k->NI = NI; k->TH = TH; k->TW = TW; k->PWC = PWC; k->PXI = PXI; k->PX = PXQ * 4; k->PXQ = PXQ;
+                k->tiles_w = cols;
+                k->tiles_img = cols * ((OH + TH - 1) / TH);
+                if (tiles > 0x3fffffff) return false;
+                k->tiles_n = (int)tiles;
+            }
+        }
+    }
+    if (best < 0) return false;
+    k->tiles_m = ((int)d.oc + bm - 1) / bm;
+    if ((int64_t)k->tiles_n * k->tiles_m > 0x3ffffff0) return false;
+    const int E = GS * T, EP = (E + 1) & ~1;
+    *lds_bytes = 2 * (EP * p1_bmp(mt) + GS * k->PX) * 16;
+    return *lds_bytes <= 150 * 1024;
+}
+
+template <int MT, int NT, int T>
+int launch_p1(hipStream_t st, const P1Args& k, int lds) {
+    auto kern = patch1_kernel<MT, NT, T>;
+    static std::atomic<int> max_lds_set{0};
+    if (max_lds_set.load(std::memory_order_relaxed) == 0) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024);
+        if (e != hipSuccess) return (int)e;
+        max_lds_set.store(1, std::memory_order_relaxed);
+    }
+    const int64_t grid = (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(256), lds, st, k);
+}
+
+template <int T>
+int launch_p1_tile(hipStream_t st, const P1Args& k, int tile, int lds) {
+    switch (tile) {
+        case 0: return launch_p1<1, 1, T>(st, k, lds);
+        case 1: return launch_p1<1, 2, T>(st, k, lds);
+        case 2: return launch_p1<2, 2, T>(st, k, lds);
+        default: return launch_p1<2, 1, T>(st, k, lds);
+    }
+}
+
+}  // namespace
+
+bool patch1_usable(const ConvProblem& p) {
+    const mi355_conv_desc& d = p.d;
+    if (d.format != MI355_FMT_NCHW || p.dw4 || d.group != 1) return false;
+    if (d.dst_dtype != MI355_DT_QS8 || d.bias_mode == MI355_BIAS_FULL || !p.epi.fast) return false;
+    if (d.mode != MI355_MODE_CROSS_CORRELATION || d.dilate_h != 1 || d.dilate_w != 1) return false;
+    if (d.fh != d.fw || (d.fh != 1 && d.fh != 3 && d.fh != 5)) return false;
+    // a row holds a quad; the filter holds one item; paddings and strides that keep a tile's coordinates small
+    if (d.iw < 4 || (uint64_t)d.oc * d.ic < 4 || d.pad_h > 0xfff || d.pad_w > 0xfff || d.stride_h > 64 || d.stride_w > 64) return false;
+    const int64_t lim = (int64_t)1 << 31, n1 = (int64_t)d.n - 1;
+    const int64_t src_b = n1 * p.src_sn + (int64_t)d.ic * d.ih * d.iw, out = (int64_t)d.oc * p.oh * p.ow;
+    if (src_b >= lim || n1 * p.dst_sn + out >= lim || n1 * p.z_sn + out >= lim || (int64_t)d.oc * d.ic * d.fh * d.fw >= lim / 2) return false;
+    return d.n > 0 && out > 0;
+}
+
+// The tile, or -1 where packing in a launch of its own is ahead.  Graph replays of every tile and of the packed path on 220
+// sizes drawn over 3 to 256 channels in, 8 to 256 out, planes of 7 x 7 to 112 x 112 and batch 1 to 64; w0: workgroups of 32 x 128.
+//   The packed path takes 6 to 9 us however few the tiles -- two launches, but its few-pixel kernel splits the reduction -- where
+// this kernel walks the stages one after the other at 0.9 us each (1.7 with 25 taps): up to half a workgroup per CU a long
+// reduction goes there (3x3 130 -> 44 at 12 x 12, five stages: 8.6 us here, 6.9 there; 48 -> 12, two: 5.0 / 6.4).  With more tiles
+// it is the other way round: 3x3 45 -> 12 at 22 x 22, batch 47: 5.9 / 11.5; 1x1 20 -> 149 at 96 x 78: 24.1 / 34.3; 5x5 46 -> 45,
+// 168640 pixels: 25.4 / 41.4.  A caller without a workspace has no packed path (packed = false).
+//   Below 64 workgroups and from 2^24 multiply-adds on the packed path stays, 5 to 25 % behind on one or two stages: a workspace of
+// the size that it needs is written there, which the interface's tests hold (24 -> 40 at 28 x 28, batch 4, among them).
+//   Tiles: the smallest up to 400 workgroups of it (5x5: 256), where a stage's latency is all there is; beyond that 32 x 256 (3x3
+// 14 -> 19, 202800 pixels: 15.6 us against 18.5), and 64 x 256, which turns a patch for twice the channels, once those are two per
+// CU (3x3 8 -> 189, 61950 pixels: 15.6 against 18.9 and 20.1).  At strides a patch is several times its pixels: 64 x 128 (3x3 38 ->
+// 97, stride 2, 588 workgroups: 14.0 against 18.3).
+int patch1_pick(const ConvProblem& p, bool packed) {
+    if (!patch1_usable(p)) return -1;
+    P1Args k;
+    int lds;
+    auto wgs = [&](int tile) { return p1_plan(p, tile, &k, &lds) ? (int64_t)k.tiles_n * k.tiles_m : (int64_t)-1; };
+    const int64_t w0 = wgs(0);
+    const int T = (int)(p.d.fh * p.d.fw);
+    if (w0 < 0) return -1;
+    const uint64_t macs = (uint64_t)p.d.n * p.d.oc * p.oh * p.ow * p.icpg * p.d.fh * p.d.fw;
+    if (packed && w0 < 64 && macs >= (1u << 24)) return -1;
+    if (packed && w0 < 128 && k.nstages >= (T == 1 ? 4 : T == 9 ? 3 : 2)) return -1;
+    if (w0 <= (T == 25 ? 256 : 400)) return 0;
+    if (p.d.stride_h > 1 || p.d.stride_w > 1) return p.d.oc > 32 && wgs(3) > 0 ? 3 : 0;
+    if (p.d.oc > 32 && wgs(2) >= 512) return 2;
+    return wgs(1) > 0 ? 1 : 0;
+}
+
+int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+                  int8_t* dst) {
+    const mi355_conv_desc& d = p.d;
+    P1Args k;
+    int lds;
+    if (!p1_plan(p, tile, &k, &lds)) return (int)hipErrorInvalidConfiguration;
+    k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
+    k.IC = d.ic; k.IH = d.ih; k.IW = d.iw; k.IHW = d.ih * d.iw;
+    k.OC = d.oc; k.OH = p.oh; k.OW = p.ow; k.OHW = p.oh * p.ow; k.N = d.n;
+    k.sh = d.stride_h; k.sw = d.stride_w; k.ph = d.pad_h; k.pw = d.pad_w;
+    k.src_sn = (int)p.src_sn; k.dst_sn = (int)p.dst_sn; k.z_sn = (int)p.z_sn;
+    k.src_bytes = (uint32_t)((d.n - 1) * p.src_sn + (int64_t)d.ic * k.IHW);
+    k.dst_bytes = (uint32_t)((d.n - 1) * p.dst_sn + (int64_t)d.oc * k.OHW);
+    k.z_bytes = (uint32_t)((d.n - 1) * p.z_sn + (int64_t)d.oc * k.OHW);
+    k.kbytes = d.ic * d.fh * d.fw;
+    k.flt_bytes = k.kbytes * d.oc;
+    k.has_bias = d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL;
+    k.div_tiles_m = make_fastdiv(k.tiles_m); k.div_tiles_img = make_fastdiv(k.tiles_img); k.div_tiles_w = make_fastdiv(k.tiles_w);
+    k.div_tw = make_fastdiv(k.TW); k.div_tile_px = make_fastdiv(k.TH * k.TW);
+    k.div_pqi = make_fastdiv(k.PXI >> 2); k.div_pqw = make_fastdiv(k.PWC >> 2);
+    k.epi = p.epi;
+    const int T = (int)(d.fh * d.fw);
+    return T == 1 ? launch_p1_tile<1>(st, k, tile, lds) : T == 9 ? launch_p1_tile<9>(st, k, tile, lds) : launch_p1_tile<25>(st, k, tile, lds);
+}
+
+}  // namespace mi355
