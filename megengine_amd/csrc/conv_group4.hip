@@ -18,8 +18,10 @@
 // included a third of the time of the dot products.  A workgroup stages a band of input rows in LDS as [pixel][16
 // channels] (NCHW4 keeps them in four planes), so every operand is one conflict-free ds_read_b128; the filter stays in
 // twelve registers; the next band is in flight while this one is multiplied.
-// 32 groups of 4 at 56 x 56, batch 16 (13 MB): 165 us as 32 launches, 9.8 with dot products, 6.8 here; 32 groups of 16
-// (51 MB): 50 us with dot products, 17 here.
+// 32 groups of 4 at 56 x 56, batch 16 (13 MB): 165 us as 32 launches, 9.8 with dot products, 6.6 here; 32 groups of 16
+// (51 MB): 50 us with dot products, 17 here.  Small layers are a chain: with the filter staged beside the first band instead of
+// gathered dword by dword ahead of it, and the next operands read while results are requantised, 55 groups of 16 at 8 x 47,
+// stride 2, batch 4 went from 6.2 to 4.2 us, 5 groups of 16 at 33 x 100, stride 2, batch 64 from 9.8 to 8.4.
 #include "igemm_shared.h"
 
 namespace mi355 {
@@ -124,7 +126,8 @@ struct G16Args {
     int8_t* dst;
     int IH, IW, OH, OW, s, ph, pw;
     int TH, PW, bands, items;  // output rows of a band, padded input columns, bands per image, bands of the batch
-    int icpg, src_scb, dst_scb, has_bias;
+    int log_icpg, src_scb, dst_scb, has_bias;
+    int slabs, step;  // blocks of 16 channels; workgroups per slab
     int64_t src_sn, dst_sn, z_sn;
     FastDiv div_pw, div_ow, div_bands;
     EpiParams epi;
@@ -145,25 +148,14 @@ __device__ __forceinline__ void requant8(v4i x, v4i y, uint32_t (&w)[2], const E
 
 template <bool HZ>
 __global__ __launch_bounds__(256) void grp16_kernel(G16Args a) {
-    __shared__ __attribute__((aligned(16))) v4i sm[G16_PX];
+    __shared__ __attribute__((aligned(16))) v4i sm[G16_PX], sf[144];
+    // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
+    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.IH), "s"(a.IW), "s"(a.OH), "s"(a.OW), "s"(a.s), "s"(a.ph),
+                 "s"(a.pw), "s"(a.TH), "s"(a.PW), "s"(a.bands), "s"(a.items), "s"(a.log_icpg), "s"(a.src_scb), "s"(a.dst_scb), "s"(a.has_bias),
+                 "s"(a.slabs), "s"(a.src_sn), "s"(a.div_pw.m), "s"(a.div_bands.m), "s"(a.div_ow.m), "s"(a.epi.s_b), "s"(a.epi.lin_lo));
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int l16 = lane & 15, kq = lane >> 4, slab = blockIdx.y, oc = slab * 16 + l16;
+    const int l16 = lane & 15, kq = lane >> 4, slab = blockIdx.y;
     const int PH = (a.TH - 1) * a.s + 3, patch = PH * a.PW;
-
-    // filter rows: lane = output channel, 16 bytes of tap 4 step + kq = its 16 input channels, zero outside its group
-    v4i fa[3];
-    int tap_off[3];
-    const int icb = a.icpg / 4, first = l16 / a.icpg * icb;  // channel blocks of a group, first one of the lane's group
-#pragma unroll
-    for (int st = 0; st < 3; ++st) {
-        const int tap = st * 4 + kq;
-        tap_off[st] = tap < 9 ? tap / 3 * a.PW + tap % 3 : 0;
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-            fa[st][b] = tap < 9 && b >= first && b < first + icb ? a.flt[(oc * icb + b - first) * 9 + tap] : 0;
-    }
-    v4i bv = {0, 0, 0, 0};
-    if (a.has_bias) bv = *reinterpret_cast<const v4i*>(a.bias + slab * 16 + kq * 4);
 
     v4i x[G16_PX / 256];
     auto fetch = [&](int item) __attribute__((always_inline)) {
@@ -180,33 +172,70 @@ __global__ __launch_bounds__(256) void grp16_kernel(G16Args a) {
         }
     };
 
+    // The slab's filter is one contiguous piece, at most 2304 bytes: 16 bytes per thread into LDS, ahead of the band's pixels, and
+    // from there each lane takes its dwords.  (Taken from memory, 48 gathers of 64 scattered dwords per workgroup cost more of the
+    // vector-memory path than everything else.)
+    const int icb = 1 << (a.log_icpg - 2), f_vecs = 36 * icb;
+    const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, (uint32_t)(a.slabs * f_vecs) * 16);
+    const v4i f_vec = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, t < f_vecs ? (slab * f_vecs + t) * 16 : SENT, 0, 0);
+    const v4i bv = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(a.bias, a.has_bias ? a.slabs * 64 : 0), (slab * 16 + kq * 4) * 4, 0, 0);
     int item = blockIdx.x;
     fetch(item);
-    while (item < a.items) {
+    if (t < f_vecs) sf[t] = f_vec;
 #pragma unroll
-        for (int k = 0; k < G16_PX / 256; ++k) sm[t + k * 256] = x[k];
-        __syncthreads();
-        const int next = item + gridDim.x;
+    for (int k = 0; k < G16_PX / 256; ++k) sm[t + k * 256] = x[k];
+    __syncthreads();
+    // filter rows: lane = output channel, 16 bytes of tap 4 step + kq = its 16 input channels, zero outside its group
+    v4i fa[3];
+    int tap_off[3];
+    const int first = (l16 >> a.log_icpg) * icb;  // first channel block of the lane's group
+#pragma unroll
+    for (int st = 0; st < 3; ++st) {
+        const int tap = st * 4 + kq;
+        tap_off[st] = tap < 9 ? tap / 3 * a.PW + tap % 3 : 0;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const bool in = (tap < 9) & (b >= first) & (b < first + icb);
+            const int w = reinterpret_cast<const int*>(sf)[in ? (l16 * icb + b - first) * 9 + tap : 0];
+            fa[st][b] = in ? w : 0;
+        }
+    }
+    for (;;) {
+        const int next = item + a.step;
         if (next < a.items) fetch(next);  // lands during the multiplies
         const int n = (int)fdiv(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
         const int pixels = (a.OH - oh0 < a.TH ? a.OH - oh0 : a.TH) * a.OW;
         const int64_t at = (int64_t)(slab * 4 + kq) * a.dst_scb + (int64_t)oh0 * a.OW * 4;
         int8_t* dst = a.dst + n * a.dst_sn + at;
         const int8_t* z = a.z + n * a.z_sn + at;
-        // two units of 16 pixels at a time: their LDS reads and multiplies overlap
-        for (int u = wave * 32; u < pixels; u += 128) {
-            uint32_t zw[2] = {0, 0};
-            v4i acc[2];
+        // two units of 16 pixels at a time; the operands of the next two are read while these are requantised
+        v4i fb[2][3];
+        auto operands = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
                 const int p = u + k * 16 + l16, pp = p < pixels ? p : 0;
                 const int oh = (int)fdiv(pp, a.div_ow), ow = pp - oh * a.OW;
-                if (HZ) zw[k] = *reinterpret_cast<const uint32_t*>(z + pp * 4);
                 const v4i* px = sm + (oh * a.PW + ow) * a.s;
-                acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[0], px[tap_off[0]], bv, 0, 0, 0);
-                acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[1], px[tap_off[1]], acc[k], 0, 0, 0);
-                acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[2], px[tap_off[2]], acc[k], 0, 0, 0);
+#pragma unroll
+                for (int st = 0; st < 3; ++st) fb[k][st] = px[tap_off[st]];
             }
+        };
+        operands(wave * 32);
+        for (int u = wave * 32; u < pixels; u += 128) {
+            uint32_t zw[2] = {0, 0};
+            v4i acc[2] = {bv, bv};
+            if (HZ)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const int p = u + k * 16 + l16;
+                    zw[k] = *reinterpret_cast<const uint32_t*>(z + (p < pixels ? p : 0) * 4);
+                }
+#pragma unroll
+            for (int st = 0; st < 3; ++st)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[st], fb[k][st], acc[k], 0, 0, 0);
+            operands(u + 128);
+            __builtin_amdgcn_sched_barrier(0);
             requant8(acc[0], acc[1], zw, a.epi);
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
@@ -214,6 +243,10 @@ __global__ __launch_bounds__(256) void grp16_kernel(G16Args a) {
                 if (p < pixels) *reinterpret_cast<uint32_t*>(dst + p * 4) = zw[k];
             }
         }
+        if (next >= a.items) break;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < G16_PX / 256; ++k) sm[t + k * 256] = x[k];
         __syncthreads();
         item = next;
     }
@@ -242,20 +275,27 @@ int launch_g16(hipStream_t st, const ConvProblem& p, const int8_t* src, const in
     const int slabs = d.oc / 16;
     a.TH = g16_rows(p);
     if (a.TH > (int)p.oh) a.TH = p.oh;
-    // fewer rows per band while that leaves CUs without one
-    while (a.TH > 1 && (int64_t)slabs * d.n * ((p.oh + a.TH - 1) / a.TH) < 512) a.TH = (a.TH + 1) / 2;
+    // Fewer rows per band while that leaves CUs without one, or with one long one: a workgroup's fixed part is worth about 200
+    // pixels (8 groups of 16 at 11 x 10, batch 30, 240 workgroups: 4.3 us, 5.0 with twice as many; 6 groups of 16 at 20 x 70, batch
+    // 18, H_SWISH and a residual: 7.8 with bands of 420 pixels, 6.9 with 210).
+    while (a.TH > 1) {
+        const int64_t wgs = (int64_t)slabs * d.n * ((p.oh + a.TH - 1) / a.TH);
+        if (wgs >= (a.TH * (int)p.ow > 400 ? 512 : 240)) break;
+        a.TH = (a.TH + 1) / 2;
+    }
     a.PW = ((int)p.ow - 1) * a.s + 3;
     a.bands = ((int)p.oh + a.TH - 1) / a.TH;
     const int64_t items = (int64_t)d.n * a.bands;
     if (items > 0x3fffffff) return (int)hipErrorInvalidValue;
     a.items = (int)items;
-    a.icpg = p.icpg; a.src_scb = d.ih * d.iw * 4; a.dst_scb = p.oh * p.ow * 4;
+    a.log_icpg = p.icpg == 4 ? 2 : p.icpg == 8 ? 3 : 4; a.src_scb = d.ih * d.iw * 4; a.dst_scb = p.oh * p.ow * 4;
     a.has_bias = d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL;
     a.src_sn = p.src_sn; a.dst_sn = p.dst_sn; a.z_sn = p.z_sn;
     a.div_pw = make_fastdiv(a.PW); a.div_ow = make_fastdiv(p.ow); a.div_bands = make_fastdiv(a.bands);
     a.epi = p.epi;
     int64_t per_slab = (2048 + slabs - 1) / slabs;  // eight workgroups per CU over all slabs
     if (per_slab > items) per_slab = items;
+    a.slabs = slabs; a.step = (int)per_slab;
     const dim3 grid((unsigned)per_slab, slabs);
     return d.has_z ? launch_kernel(grp16_kernel<true>, grid, dim3(256), 0, st, a) : launch_kernel(grp16_kernel<false>, grid, dim3(256), 0, st, a);
 }
