@@ -17,7 +17,6 @@
 // Filters of 1x1, 3x3 and 5x5; others go through the
 // workspace.  Graph replays: 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual: 17.3 us packed, 13.2 here (four waves of
 // 1200 vector instructions for 23 products each, a third of their time waiting for a stage's loads); more at patch1_pick.
-#include <algorithm>
 #include <atomic>
 
 #include "igemm_shared.h"
@@ -364,9 +363,10 @@ bool p1_plan(const ConvProblem& p, int tile, P1Args* k, int* lds_bytes) {
     k->nstages = (G + GS - 1) / GS;
     int64_t best = -1;
     // equal columns of whole quads, as wide as the tile or narrower; rows (of whole images where one is small) as they fit
-    const int ow4 = (OW + 3) & ~3;
-    for (int most = std::min(bn, ow4), last = 0; most >= std::min(16, ow4); most -= 4) {
-        const int cols = (OW + most - 1) / most, TW = ((OW + cols - 1) / cols + 3) & ~3;
+    const int cols0 = (OW + bn - 1) / bn;
+    for (int parts = cols0, last = 0;; ++parts) {
+        const int TW = ((OW + parts - 1) / parts + 3) & ~3, cols = (OW + TW - 1) / TW;
+        if (TW < 16 && parts > cols0) break;
         if (TW == last) continue;
         last = TW;
         // patch columns: the first is rounded down to a multiple of four, whatever the tile's position
