@@ -483,8 +483,8 @@ int launch_fmt(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
 
 // tile_cfg numbering: register-staged tiles, LDS-direct tiles, second-generation tiles, patch-staged tiles, weight-resident
 // tiles, the 32-packed streaming kernel, the tiles that split the reduction over the waves of a
-// workgroup, the one-launch NCHW4 group kernel, the 4-packed patch tiles
-int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1 + igemm5_num_cfgs() + 1 + patch4_num_cfgs() + 1; }
+// workgroup, the one-launch NCHW4 group kernel, the 4-packed patch tiles, the split pointwise tile, the 32-packed group tiles
+int igemm_num_cfgs() { return kNumCfgs + igemm_dma_num_cfgs() + igemm2_num_cfgs() + igemm3_num_cfgs() + igemm4_num_cfgs() + 1 + igemm5_num_cfgs() + 1 + patch4_num_cfgs() + 1 + grp32_num_cfgs(); }
 int igemm_first_v2_cfg() { return kNumCfgs + igemm_dma_num_cfgs(); }
 // planar destination (NCHW4_NCHW): two of the register-staged tiles
 static int launch_planar(hipStream_t st, IgemmArgs& a, int cfg, int cu) {
@@ -502,6 +502,7 @@ static int igemm_first_ks_cfg() { return igemm_pw32s_cfg() + 1; }
 static int igemm_grp4_cfg() { return igemm_first_ks_cfg() + igemm5_num_cfgs(); }
 static int igemm_first_p4_cfg() { return igemm_grp4_cfg() + 1; }
 static int igemm_pw4_split_cfg() { return igemm_first_p4_cfg() + patch4_num_cfgs(); }
+static int igemm_first_g32_cfg() { return igemm_pw4_split_cfg() + 1; }
 const char* igemm_cfg_name(int cfg) {
     if (cfg >= 0 && cfg < kNumCfgs) return kCfgs[cfg].name;
     if (cfg < igemm_first_v2_cfg()) return igemm_dma_cfg_name(cfg - kNumCfgs);
@@ -512,6 +513,7 @@ const char* igemm_cfg_name(int cfg) {
     if (cfg < igemm_grp4_cfg()) return igemm5_cfg_name(cfg - igemm_first_ks_cfg());
     if (cfg == igemm_grp4_cfg()) return "grp4_dot4";
     if (cfg == igemm_pw4_split_cfg()) return "pw4_split";
+    if (cfg >= igemm_first_g32_cfg()) return grp32_cfg_name(cfg - igemm_first_g32_cfg());
     return patch4_cfg_name(cfg - igemm_first_p4_cfg());
 }
 
@@ -623,6 +625,8 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         if (ks >= 0) return igemm_first_ks_cfg() + ks;
         const int p4 = patch4_pick(a, p.pin, p.pout);
         if (p4 >= 0) return igemm_first_p4_cfg() + p4;
+        const int g32 = igemm_needs_general(p) ? -1 : grp32_pick(a, p.pin, p.pout, will_preprocess);
+        if (g32 >= 0) return igemm_first_g32_cfg() + g32;
     }
     if (p.pin == 32 && p.pout == 32 && d.group == 1 && !igemm_needs_general(p) && d.fh == 3 && d.fw == 3 &&
         d.stride_h == 1 && d.stride_w == 1 && d.pad_h == 1 && d.pad_w == 1 && (d.ic == 32 || d.ic == 64)) {
@@ -700,6 +704,12 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
     // group convolution and the general epilogue: second-generation tiles only; a channel tile never spans two groups
     // (the 64-channel tile too where 128 x 128 tiles would leave CUs without one: an int32 result 128 -> 256 at 28 x 28, batch 1
     // to 8: 5.1 .. 6.2 us against 6.5 .. 7.6; 3x3 128 -> 128, batch 16: 8.8 against 11.9; at batch 32 the two are equal)
+    if (d.group != 1 && !igemm_needs_general(p)) {
+        IgemmArgs a;
+        igemm_fill_args(p, a);
+        const int g32 = grp32_pick(a, p.pin, p.pout, will_preprocess);
+        if (g32 >= 0) return igemm_first_g32_cfg() + g32;
+    }
     if (d.group != 1 || igemm_needs_general(p)) {
         const int64_t t128 = (int64_t)d.group * ((p.ocpg + 127) / 128) * ((M + 127) / 128);
         return igemm_first_v2_cfg() + (p.ocpg <= 64 || (2 * t128 < 3 * (int64_t)cu_count) ? 3 : 0);
@@ -766,7 +776,7 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
 
 size_t igemm_preprocessed_bytes(const ConvProblem& p, int cfg) {
     // the weight-resident tiles read the reference layout (once per workgroup: nothing to gain from re-tiling)
-    const bool ks = cfg >= igemm_first_ks_cfg() && cfg < igemm_grp4_cfg();
+    const bool ks = (cfg >= igemm_first_ks_cfg() && cfg < igemm_grp4_cfg()) || cfg >= igemm_first_g32_cfg();
     if (p.pin != 32 || !(ks || (cfg >= igemm_first_v2_cfg() && cfg < igemm_first_v4_cfg()))) return 0;
     return igemm2_preprocessed_bytes((int)p.d.oc, (int)(p.icpg * p.d.fh * p.d.fw));
 }
@@ -847,6 +857,10 @@ static int resolve_filled(const ConvProblem& p, const IgemmArgs& a, int cfg) {
             return cfg;
         if (p.pin == 32) return cfg == first_v2 ? cfg : first_v2 + 3;
         return cfg == 3 ? 3 : 0;
+    }
+    if (cfg >= igemm_first_g32_cfg()) {
+        if (grp32_can_run(a, p.pin, p.pout, cfg - igemm_first_g32_cfg())) return cfg;
+        cfg = first_v2;
     }
     // group convolutions and the general epilogue exist on the second-generation tiles only
     if ((d.group != 1 || a.general) && cfg < first_v2) cfg = first_v2 + (p.ocpg <= 64 ? 3 : 0);
@@ -973,6 +987,7 @@ int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_coun
             a.ztab = tab;
         }
     }
+    if (cfg >= igemm_first_g32_cfg()) return launch_grp32(st, a, cfg - igemm_first_g32_cfg());
     if (cfg == igemm_pw4_split_cfg()) return launch_pw4_split(st, a);
     if (cfg >= igemm_first_p4_cfg()) return launch_patch4(st, a, cfg - igemm_first_p4_cfg());
     if (cfg >= igemm_first_ks_cfg()) return launch_igemm5(st, a, p.pin, p.pout, cfg - igemm_first_ks_cfg());

@@ -508,6 +508,13 @@ bool patch4_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
 int patch4_pick(const IgemmArgs& a, int pin, int pout);  // its tile for this problem, -1 where another kernel is ahead
 int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg);
 
+// 3x3 over 32 or 64 channels per group, 32-packed, the whole reduction in one stage (conv_group32.hip, tiles "v2_patch_*")
+int grp32_num_cfgs();
+const char* grp32_cfg_name(int cfg);
+bool grp32_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
+int grp32_pick(const IgemmArgs& a, int pin, int pout, bool will_preprocess);  // its tile, -1 where another kernel is ahead
+int launch_grp32(hipStream_t st, const IgemmArgs& a, int cfg);
+
 // streaming kernel for 4-packed pointwise layers with few input or few output channels (conv_pw4.hip)
 bool pw4s_usable(const IgemmArgs& a);
 // NCHW4 pointwise at stride 1, four pixels per lane (tile "pw4_split"); the streaming tile takes the same form there
