@@ -66,6 +66,9 @@ size_t igemm_preprocessed_bytes(const ConvProblem& p, int tile_cfg);
 int launch_igemm_preprocess(hipStream_t st, const ConvProblem& p, const int8_t* flt, int8_t* out);
 
 bool depthwise_usable(const ConvProblem& p);
+bool dwm_usable(const ConvProblem& p);
+int launch_dwm(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+               int8_t* dst);
 int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt,
                           const int32_t* bias, const int8_t* z, int8_t* dst);
 

@@ -2,8 +2,7 @@
 //
 // Layouts: src/dst (n, c/4, h, w, 4), filter (c/4, 1, 1, fh, fw, 4) -- the reference's NCHW44
 // channel-wise filter (dnn/src/naive/convolution/helper.h:251-256, :419-424).  Every output
-// needs fh*fw multiply-adds per channel and moves ~2 bytes, so the kernel is bandwidth bound:
-// no matrix cores.  One thread produces 4 consecutive output pixels x 4 channels:
+// needs fh*fw multiply-adds per channel and moves ~2 bytes.  One thread produces 4 consecutive output pixels x 4 channels:
 //   * a pixel's 4 channels arrive as one dword; the 4 per-channel products of a tap are 4
 //     v_dot4_i32_i8 against the filter dword masked to one byte each (the masks are wave-uniform
 //     and live in scalar registers), so no byte unpacking is needed;
@@ -12,7 +11,7 @@
 //   * all threads of a workgroup share (n, c/4), so filter and bias loads are scalar.
 // That form (dw4_kernel) serves every filter size / stride.  The 3x3, stride 1 or 2 case -- every
 // channel-wise layer of the MobileNet family -- has its own kernel, dw3x3_kernel, and so have 5x5 and 7x7 with "same"
-// padding, dwf_kernel, below.
+// padding, dwf_kernel, below.  Where the dot products bound them, the matrix cores take over (conv_dwm.hip).
 #include "common.h"
 
 namespace mi355 {
@@ -565,6 +564,17 @@ int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, const int8_t* sr
     if (d.n == 0 || p.oh == 0 || p.ow == 0) return 0;
     const bool sq = d.fh == d.fw && d.stride_h == d.stride_w && (d.stride_h == 1 || d.stride_h == 2);
     const bool wide = sq && (d.fh == 5 || d.fh == 7) && d.pad_w == d.fw / 2;
+    // The matrix-core form against the vector forms (us, graph replays):
+    //   5x5 and 7x7 "same", against dwf_kernel: 560 channels, 5x5 at 30 x 55, batch 14: 14.3 / 20.1; 240, 5x5 stride 2 at 57 x 57,
+    //     batch 16: 8.4 / 9.4; 136, 7x7 at 42 x 37, batch 7: 6.1 / 7.8; 68, 5x5 stride 2 at 24 x 10, batch 3: 3.6 / 4.3.  Its workgroups
+    //     set themselves up for one plane each, so many small planes stay behind: 740, 5x5 stride 2 at 10 x 14, batch 16 (10 quads a
+    //     plane): 5.7 / 4.8; 604 at 14 x 78, batch 17 (70 quads): 10 / 8.2; from about 100 quads it is ahead at any number of planes.
+    //   other filters, against dw4_kernel: 4x4 at 35 x 38, 112 channels, batch 45: 8.8 / 29.9; 6x6 at 101 x 14, 256, batch 1: 4.2 / 12.8;
+    //     2x2 at 71 x 26, 108, batch 63: 12.6 / 15.7.  At strides of 3 and 4 a filter of few taps leaves most of the patch unused: 7x1,
+    //     stride 3, 448 at 44 x 82, batch 2: 6.3 / 5.6.
+    const bool small_planes = (int64_t)d.n * a.CG >= 512 && (int64_t)a.OH * a.QW < 100;
+    const bool matrix = wide ? !small_planes : !(sq && d.fh == 3) && (d.stride_w <= 2 || d.fh * d.fw >= 9);
+    if (matrix && dwm_usable(p)) return launch_dwm(st, p, src, flt, bias, z, dst);
     const int64_t src_total = (int64_t)(d.n - 1) * p.src_sn + (int64_t)d.ic * d.ih * d.iw;
     if (sq && (d.fh == 3 || (wide && src_total < ((int64_t)1 << 31)))) {
         // Output rows per thread.  Few work items: one, because a thread's own chain -- its rows' loads, products and stores -- is

@@ -1,0 +1,251 @@
+// Channel-wise convolution on the matrix cores (4-packed activations, filters up to 32 blocks of a window, any stride).
+//
+// A channel-wise layer has no contraction over channels, but it has one over the pixels of a window, and the layout
+// (n, c/4, h, w, 4) lays that out for the matrix cores as it stands: 16 bytes in memory are four pixels of four channels.
+// v_mfma_i32_16x16x64_i8 takes four such blocks of a window as its K dimension,
+//   B (64 x 16): column = a quad of four output pixels, its K = blocks of four input pixels, read from LDS as they lie;
+//   A (16 x 64): row = (output pixel j of the quad, channel c), K = (input pixel, channel): the filter tap that connects input
+//                pixel and output pixel where the channels agree, zero elsewhere,
+// so the transposes, byte alignments and dot products of the vector form (conv_dw.hip) all fall away: a wave's 64 pixels of four
+// channels take ceil(rows x blocks / 4) matrix instructions -- 2 for 3x3, 3 for 5x5, 6 for 7x7 at stride 1 -- of which a sixth to
+// a third is useful, still several times the rate of byte dot products.  A lane ends with the four channels of one pixel.
+//
+// A workgroup computes a band of output rows of one channel block: the padded input rows go to LDS in one pass (a row, or several
+// narrow ones, per wave instruction, no register stage), so a pixel is read from memory once, and everything outside the image
+// is zero there.  Bound by the vector instructions: the requantisation of 8 values per lane and iteration and the set-up of
+// a workgroup (350 instructions per wave), not by the matrix instructions (5x5 stride 2, 240 channels at 57 x 57, batch 16:
+// 8.4 us, of which the copy rate accounts for 3.2; the byte dot products took 9.4).
+#include "lds_copy.h"
+
+namespace mi355 {
+namespace {
+
+constexpr int DWM_LDS_PX = 8192;  // most pixels of a band's patch
+
+// division of 24-bit numbers up to a known bound by one full-rate multiplication and a shift
+struct SmallDiv {
+    uint32_t m, s;
+};
+SmallDiv small_div(uint32_t d, uint32_t most) {  // most < 32768
+    SmallDiv v = {0, 0};
+    while (((uint64_t)1 << v.s) <= (uint64_t)most * d) ++v.s;
+    v.m = (uint32_t)(((uint64_t)1 << v.s) / d + 1);
+    return v;
+}
+__device__ __forceinline__ int sdiv(int x, const SmallDiv& d) { return (int)(__umul24((uint32_t)x, d.m) >> d.s); }
+__device__ __forceinline__ int mad24(int a, int b, int c) { return (int)(__umul24((uint32_t)a, (uint32_t)b) + (uint32_t)c); }
+
+struct DwmArgs {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    int IH, IW, OH, OW, FH, FW, sh, sw, ph, pw;
+    int TH, PH, PW, NB;  // output rows of a band, patch rows of an image, patch columns, 4-pixel blocks of a quad's window
+    int rpw, waves;      // patch rows of one copy instruction, waves of the workgroup
+    int part;            // blocks of a patch row that lie together
+    int QW, tab_w, tab, tab_at;  // quads of an output row; columns of the filter table and its entries (whole runs of 64), and where it starts
+    int CG, bands, taps, has_bias;
+    int64_t src_sn, dst_sn, z_sn;
+    FastDiv div_bands, div_cg, div_tab;
+    SmallDiv div_qw, div_pw, div_nb, div_part, div_sw;
+    EpiParams epi;
+};
+
+__device__ __forceinline__ void dwm_requant(v4i x, v4i y, uint32_t (&w)[2], const EpiParams& e) {
+#define MI355_BOTH(F)                                  \
+    do {                                               \
+        w[0] = F(x[0], x[1], x[2], x[3], w[0], e);     \
+        w[1] = F(y[0], y[1], y[2], y[3], w[1], e);     \
+    } while (0)
+    if (e.lin) MI355_BOTH((requant4_fast<NL_LIN, false>));
+    else if (e.nonline == NL_RELU && !e.has_z) MI355_BOTH((requant4_fast<NL_RELU, false>));
+    else MI355_BOTH(requant4);
+#undef MI355_BOTH
+}
+
+template <int STEPS, bool HZ>
+__global__ __launch_bounds__(256) void dwm_kernel(DwmArgs a) {
+    extern __shared__ __attribute__((aligned(16))) v4i lds_dwm[];  // patch, filter table
+    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.IH), "s"(a.IW), "s"(a.OH), "s"(a.OW), "s"(a.FH), "s"(a.FW),
+                 "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.TH), "s"(a.PH), "s"(a.PW), "s"(a.NB), "s"(a.rpw), "s"(a.waves), "s"(a.part),
+                 "s"(a.CG), "s"(a.bands));
+    asm volatile("" ::"s"(a.taps), "s"(a.has_bias), "s"(a.src_sn), "s"(a.dst_sn), "s"(a.z_sn), "s"(a.QW), "s"(a.tab_w), "s"(a.tab), "s"(a.tab_at),
+                 "s"(a.div_bands.m), "s"(a.div_cg.m), "s"(a.div_tab.m), "s"(a.div_qw.m), "s"(a.div_pw.m), "s"(a.div_nb.m), "s"(a.epi.s_b),
+                 "s"(a.epi.lin_lo));
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int l16 = lane & 15, kq = lane >> 4;
+    const uint32_t item = xcd_block();
+    const uint32_t i1 = fdiv(item, a.div_bands), band = item - i1 * a.bands;
+    const uint32_t n = fdiv(i1, a.div_cg), cg = i1 - n * a.CG;
+    const int oh0 = (int)band * a.TH, th = a.OH - oh0 < a.TH ? a.OH - oh0 : a.TH;
+    const int plane = a.IH * a.IW * 4, oplane = a.OH * a.OW * 4;
+    const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)lds_dwm);
+
+    // Filter table: row by row, with 3 sw zeros in front (the later pixels of a quad start further on) and zeros behind
+    {
+        const v4i rs = uniform_rsrc(a.flt, (uint32_t)(a.CG * a.taps) * 4);
+        for (int e = wave * 64; e < a.tab; e += a.waves * 64) {
+            const int r = (int)fdiv(e + lane, a.div_tab), tap = e + lane - r * a.tab_w - 3 * a.sw;
+            const bool ok = (r < a.FH) & ((unsigned)tap < (unsigned)a.FW);
+            lds_copy64x4(lds0 + (uint32_t)(a.tab_at + e) * 4, ok ? ((int)cg * a.taps + r * a.FW + tap) * 4 : SENT, rs);
+        }
+    }
+    const v4i bv = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(a.bias, a.has_bias ? a.CG * 16 : 0), (int)cg * 16, 0, 0);
+    // the patch: lanes are the columns of `rpw` rows, or of 64 columns of one row
+    {
+        const v4i rs = uniform_rsrc(a.src + n * a.src_sn + (int64_t)cg * plane, (uint32_t)plane);
+        const int r0 = a.PW < 64 ? sdiv(lane, a.div_pw) : 0, rows = a.PH;
+        const int ih0 = oh0 * a.sh - a.ph, rstep = a.waves * a.rpw;
+        for (int c = lane - r0 * a.PW, cb = 0; cb < a.PW; cb += 64, c += 64) {
+            // every sw-th block of a row lies together: the windows of consecutive quads start at consecutive blocks, at any stride
+            const int blk = c >> 2, part = sdiv(blk, a.div_part), iw = ((blk - part * a.part) * a.sw + part) * 4 + (c & 3) - a.pw;
+            const bool in = (r0 < a.rpw) & (c < a.PW);
+            // an invalid column is an invalid row from the start
+            const int r_in = in ? r0 : 0x40000000;
+            int ih = (unsigned)iw < (unsigned)a.IW ? ih0 + wave * a.rpw + r0 : 0x40000000;
+            int off = ((ih0 + wave * a.rpw + r0) * a.IW + iw) * 4;
+            for (int r = wave * a.rpw; r < rows; r += rstep) {
+                if (r_in < rows - r) lds_copy64x4(lds0 + (uint32_t)(r * a.PW + cb) * 4, (unsigned)ih < (unsigned)a.IH ? off : SENT, rs);
+                ih += rstep;
+                off += rstep * a.IW * 4;
+            }
+        }
+    }
+    // while the copies run: where this lane finds its operands, and its first two units
+    int boff[STEPS], woff[STEPS];
+    const int mask = 0xff << (8 * (l16 & 3));
+    {
+        const int at = a.tab_at + (3 - (l16 >> 2)) * a.sw;
+#pragma unroll
+        for (int st = 0; st < STEPS; ++st) {
+            const int b = st * 4 + kq, row = sdiv(b, a.div_nb), q = b - mad24(row, a.NB, 0), turn = sdiv(q, a.div_sw);
+            boff[st] = row < a.FH ? mad24(row, a.PW >> 2, mad24(q - mad24(turn, a.sw, 0), a.part, turn)) : 0;
+            woff[st] = mad24(row, a.tab_w, q * 4) + at;
+        }
+    }
+    const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst + n * a.dst_sn + (int64_t)cg * oplane, (uint32_t)oplane);
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z + n * a.z_sn + (int64_t)cg * oplane, HZ ? (uint32_t)oplane : 0u);
+    const int quads = th * a.QW, out0 = oh0 * a.OW * 4, kq4 = out0 + kq * 4, x_end = a.OW - kq;
+    struct Unit {
+        int src, dst;  // first block of the window in LDS; byte offset of this lane's pixel, out of range if it has none
+    };
+    const int row_blk = a.sh * a.PW >> 2, row_b = a.OW * 4;
+    auto unit = [&](int u) __attribute__((always_inline)) {
+        const int qi = u + l16, qc = qi < quads ? qi : quads - 1;
+        const int r = sdiv(qc, a.div_qw), q = qc - mad24(r, a.QW, 0);
+        Unit o;
+        o.src = mad24(r, row_blk, q);
+        o.dst = ((qi < quads) & (q * 4 < x_end)) ? mad24(r, row_b, q * 16 + kq4) : SENT;
+        return o;
+    };
+    const int step = a.waves * 32;
+    Unit un[2];
+    uint32_t zn[2] = {0, 0};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        un[k] = unit(wave * 32 + k * 16);
+        if (HZ) zn[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, un[k].dst, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<0>();
+    __syncthreads();
+    v4i fa[STEPS];
+#pragma unroll
+    for (int st = 0; st < STEPS; ++st)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) fa[st][p] = reinterpret_cast<const int*>(lds_dwm)[woff[st] + p] & mask;
+    for (int u = wave * 32; u < quads; u += step) {
+        v4i fb[2][STEPS];
+        uint32_t zw[2] = {zn[0], zn[1]};
+        int d[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+#pragma unroll
+            for (int st = 0; st < STEPS; ++st) fb[k][st] = lds_dwm[un[k].src + boff[st]];
+            d[k] = un[k].dst;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            un[k] = unit(u + step + k * 16);
+            if (HZ) zn[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, un[k].dst, 0, 0);
+        }
+        v4i acc[2] = {bv, bv};
+#pragma unroll
+        for (int st = 0; st < STEPS; ++st)
+#pragma unroll
+            for (int k = 0; k < 2; ++k) acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[st], fb[k][st], acc[k], 0, 0, 0);
+        dwm_requant(acc[0], acc[1], zw, a.epi);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) __builtin_amdgcn_raw_buffer_store_b32(zw[k], rs_dst, d[k], 0, 0);
+    }
+}
+
+template <int STEPS>
+int launch_steps(hipStream_t st, dim3 grid, dim3 block, int lds, const DwmArgs& a, bool hz) {
+    return hz ? launch_kernel((dwm_kernel<STEPS, true>), grid, block, lds, st, a) : launch_kernel((dwm_kernel<STEPS, false>), grid, block, lds, st, a);
+}
+
+int dwm_blocks(const ConvProblem& p) { return (3 * p.d.stride_w + (int)p.d.fw + 3) / 4; }
+
+// whole blocks, as many for each of the sw parts
+int dwm_columns(const ConvProblem& p) {
+    const int sw = p.d.stride_w, cols = ((int)p.ow - 1) * sw + (int)p.d.fw;
+    return (cols + 4 * sw - 1) / (4 * sw) * (4 * sw);
+}
+
+}  // namespace
+
+bool dwm_usable(const ConvProblem& p) {
+    const mi355_conv_desc& d = p.d;
+    if (!depthwise_usable(p) || d.stride_w > 4 || d.stride_h > 64) return false;
+    // matrix instructions of a quad, one output row's patch, and 24-bit products of rows and bytes
+    return (int)d.fh * dwm_blocks(p) <= 32 && p.ow < 65536 && (int64_t)dwm_columns(p) * d.fh <= DWM_LDS_PX;
+}
+
+// Bands: as much of the patch as 16 KiB hold, so that eight workgroups share a CU; fewer rows where that leaves CUs without one.
+int launch_dwm(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+               int8_t* dst) {
+    const mi355_conv_desc& d = p.d;
+    DwmArgs a;
+    a.src = src; a.flt = flt; a.bias = bias; a.z = z; a.dst = dst;
+    a.IH = d.ih; a.IW = d.iw; a.OH = p.oh; a.OW = p.ow; a.FH = d.fh; a.FW = d.fw; a.sh = d.stride_h; a.sw = d.stride_w;
+    a.ph = d.pad_h; a.pw = d.pad_w;
+    a.NB = dwm_blocks(p); a.PW = dwm_columns(p); a.part = a.PW / 4 / a.sw;
+    a.CG = d.ic / 4; a.taps = d.fh * d.fw; a.QW = ((int)p.ow + 3) / 4;
+    a.has_bias = d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL;
+    const int64_t most = (4096 / a.PW - a.FH) / a.sh + 1;
+    a.TH = most < 1 ? 1 : most < (int64_t)p.oh ? (int)most : (int)p.oh;
+    while (a.TH > 1 && a.TH * a.QW > 64 && (int64_t)d.n * a.CG * ((p.oh + a.TH - 1) / a.TH) < 256) a.TH = (a.TH + 1) / 2;
+    a.bands = ((int)p.oh + a.TH - 1) / a.TH;
+    a.TH = ((int)p.oh + a.bands - 1) / a.bands;  // even bands
+    a.PH = (a.TH - 1) * a.sh + a.FH;
+    a.rpw = a.PW < 64 ? 64 / a.PW : 1;
+    const int units = (a.TH * a.QW + 15) / 16, steps = (a.FH * a.NB + 3) / 4;
+    a.waves = units > 4 ? 4 : units > 2 ? 2 : 1;
+    a.tab_w = a.NB * 4 + 3 * a.sw;
+    a.tab = (((steps * 4 - 1) / a.NB + 1) * a.tab_w + 63) / 64 * 64;
+    a.tab_at = a.PH * a.PW + a.NB * 4;  // the window of a row's last quad may end past its columns
+    a.src_sn = p.src_sn; a.dst_sn = p.dst_sn; a.z_sn = p.z_sn;
+    a.div_bands = make_fastdiv(a.bands); a.div_cg = make_fastdiv(a.CG); a.div_tab = make_fastdiv(a.tab_w);
+    a.div_qw = small_div(a.QW, a.TH * a.QW); a.div_pw = small_div(a.PW, 64); a.div_nb = small_div(a.NB, 32);
+    a.div_part = small_div(a.part, a.PW / 4 + 16); a.div_sw = small_div(a.sw, 32);
+    a.epi = p.epi;
+    const int64_t items = (int64_t)d.n * a.CG * a.bands;
+    if (items > 0x7fffffff) return (int)hipErrorInvalidValue;
+    const int lds = (a.tab_at + a.tab) * 4;
+    const dim3 grid((unsigned)items), block(64 * a.waves);
+    switch (steps) {
+        case 1: return launch_steps<1>(st, grid, block, lds, a, d.has_z);
+        case 2: return launch_steps<2>(st, grid, block, lds, a, d.has_z);
+        case 3: return launch_steps<3>(st, grid, block, lds, a, d.has_z);
+        case 4: return launch_steps<4>(st, grid, block, lds, a, d.has_z);
+        case 5: return launch_steps<5>(st, grid, block, lds, a, d.has_z);
+        case 6: return launch_steps<6>(st, grid, block, lds, a, d.has_z);
+        case 7: return launch_steps<7>(st, grid, block, lds, a, d.has_z);
+        default: return launch_steps<8>(st, grid, block, lds, a, d.has_z);
+    }
+}
+
+}  // namespace mi355
