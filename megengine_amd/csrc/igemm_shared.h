@@ -239,6 +239,20 @@ __device__ __forceinline__ void igemm_run_epilogue(const IgemmArgs& a, v16i (&ac
     }
 }
 
+// the value of lane L of a group of four lanes
+template <int L>
+__device__ __forceinline__ int quad_lane(int x) {
+    return __builtin_amdgcn_mov_dpp(x, L * 0x55, 0xf, 0xf, true);
+}
+// one step of the transposition of a square of values over neighbouring lanes: the lanes that PERM pairs keep one of (a, b) and
+// exchange the other
+template <int PERM>
+__device__ __forceinline__ void quad_swap(int& a, int& b, bool upper) {
+    const int from_a = __builtin_amdgcn_mov_dpp(a, PERM, 0xf, 0xf, true), from_b = __builtin_amdgcn_mov_dpp(b, PERM, 0xf, 0xf, true);
+    a = upper ? from_b : a;
+    b = upper ? b : from_a;
+}
+
 // General epilogue of one wave tile: every dst dtype / bias shape / scale the operator accepts, with the literal
 // requantisation chain where the fast forms do not apply.  Register quad q of a 32x32 block holds channels
 // ocb + 8q + 4 (lane / 32) .. + 3 of pixel lane % 32: one dword of int8 results, or 16 bytes of int32 results.
@@ -259,14 +273,28 @@ __device__ __forceinline__ void igemm_epilogue_general(const IgemmArgs& a, v16i 
             const uint32_t mm = pok ? m : 0;
             const uint32_t n = fdiv(mm, a.div_ohw), rem = mm - n * a.OHW;
             const int at = pok ? ((int)n * a.dst_sn + (int)rem * 32) * 4 + lh * 16 : SENT;
+            // Four neighbouring lanes exchange their quads, so that a store writes whole 128-byte lines (a pixel's 32 sums) of
+            // eight pixels and not 32 bytes of each of thirty-two.
+            const int at4[4] = {quad_lane<0>(at), quad_lane<1>(at), quad_lane<2>(at), quad_lane<3>(at)};
+            const int l4 = (l32 & 3) * 32;
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
                 const int ocb = oc_w + i * 32;
                 if (ocb >= oc_end) continue;  // wave-uniform; whole blocks of 32 channels
+                int x[4][4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) x[q][r] = acc[i][j][4 * q + r];
+#pragma unroll
+                    for (int q = 0; q < 4; q += 2) quad_swap<0xB1>(x[q][r], x[q + 1][r], (l32 & 1) != 0);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) quad_swap<0x4E>(x[q][r], x[q + 2][r], (l32 & 2) != 0);
+                }
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const v4i o = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                    __builtin_amdgcn_raw_buffer_store_b128(o, rs_dst, at, (ocb >> 5) * a.dst_scb * 4 + q * 32, 0);
+                    const v4i o = {x[q][0], x[q][1], x[q][2], x[q][3]};
+                    __builtin_amdgcn_raw_buffer_store_b128(o, rs_dst, at4[q] + l4, (ocb >> 5) * a.dst_scb * 4, 0);
                 }
             }
         }
