@@ -599,6 +599,43 @@ static bool igemm_plain_s32(const ConvProblem& p) {
     return p.d.dst_dtype == MI355_DT_QS32 && p.d.bias_mode != MI355_BIAS_FULL;
 }
 
+// 32-packed dense layers with the filter in the reference layout.  What such a layer takes on a tile is a price per launch (a chain of
+// copies as long as the reduction), one per round of tiles over the device's CUs and one per tile and CU, each with a part that grows
+// with the reduction.  The prices, in us and us per 1024 reduction bytes, are fitted to graph replays of 600 layers of 32 to 1024
+// channels, 1x1 to 5x5, stride 1 and 2, batch 1 to 64, each on nineteen tiles (two halves of them predict each other as well as
+// themselves); the five tiles here hold the best of the nineteen to 3.5 % on average, where the thresholds that they replace lost 15 %:
+// 1.11 times as fast over the 600, and 3x3 288 -> 672 at 45 x 37, batch 10: 48.8 -> 34.4 us; 5x5 32 -> 992 at 51 x 64, stride 2, batch
+// 59: 70.8 -> 63.4; 3x3 320 -> 192 at 17 x 57, batch 53: 47.7 -> 36.8; 1x1 320 -> 672 at 60 x 34, batch 49: 63.7 -> 47.8.
+// (600 layers: 61 are more than 3 % slower on the new choice.)
+static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool strided, bool has_z) {
+    struct Price {
+        int cfg, bm, bn;
+        float launch, launch_k, round, round_k, tile, tile_k, tile_strided_k, tile_z;
+    };
+    const int dma = kNumCfgs, v2 = igemm_first_v2_cfg();
+    const Price prices[] = {
+            {dma + 18, 64, 128, 4.11f, 0.62f, 0.57f, 1.37f, 0.57f, 0.52f, 0.20f, 0.28f},   // dma64x128x128w8
+            {v2 + 10, 128, 256, 4.35f, 0.14f, 0.31f, 4.79f, 1.74f, 0.52f, 2.85f, 1.96f},   // v2_128x256x64r3w8
+            {v2 + 8, 64, 64, 3.88f, 0.49f, 0.00f, 1.61f, 0.52f, 0.00f, 0.29f, 0.18f},      // v2_64x64x128r4
+            {dma + 17, 128, 128, 3.31f, 1.75f, 0.88f, 1.91f, 0.86f, 0.59f, 0.39f, 0.65f},  // dma128x128x128r2w8
+            {v2 + 4, 64, 128, 3.95f, 1.12f, 0.02f, 1.94f, 0.67f, 0.18f, 0.65f, 0.47f},     // v2_64x128x64r4
+    };
+    const float k = kbytes / 1024.0f;
+    float best = 0;
+    int cfg = -1;
+    for (const Price& c : prices) {
+        const int64_t tiles = (int64_t)((OC + c.bm - 1) / c.bm) * ((M + c.bn - 1) / c.bn);
+        const float rounds = (float)((tiles + 255) / 256), share = tiles / 256.0f;
+        const float us = c.launch + c.launch_k * k + rounds * (c.round + c.round_k * k) +
+                         share * (c.tile + c.tile_k * k + (strided ? c.tile_strided_k * k : 0) + (has_z ? c.tile_z : 0));
+        if (cfg < 0 || us < best) {
+            best = us;
+            cfg = c.cfg;
+        }
+    }
+    return cfg;
+}
+
 static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_preprocess) {
     const mi355_conv_desc& d = p.d;
     if (p.pout == 1) {
@@ -633,9 +670,10 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         // 3x3 over 32 or 64 channels with five and more 64 x 128 tiles for each of the two workgroups of a CU: the
         // weight-resident tile, whose workgroups load the filter once (64 -> 64 at 56 x 56, batch 128: 24.4 against 26.7 us
         // on the second-generation tile; at batch 64, three tiles per workgroup, its longer prologue loses: 15.7 against 14.8)
+        // (up to 128 output channels: every 64 more read the whole input again, 32 -> 832 at 71 x 102, batch 6: 29.1 against 20.5)
         const int64_t t = (int64_t)((d.oc + 63) / 64) * d.n * ((p.oh * p.ow + 127) / 128);
         const int v4 = igemm_first_v4_cfg();
-        if (t >= 10 * (int64_t)(cu_count > 0 ? cu_count : 256) && igemm_resolve_cfg(p, v4) == v4) return v4;
+        if (d.oc <= 128 && t >= 10 * (int64_t)(cu_count > 0 ? cu_count : 256) && igemm_resolve_cfg(p, v4) == v4) return v4;
     }
     if (p.pin == 32 && p.pout == 32 && d.group == 1 && !igemm_needs_general(p) && d.fh == 1 && d.fw == 1 && d.pad_h == 0 &&
         d.pad_w == 0 && d.ic <= 64 && d.oc <= 64) {
@@ -743,6 +781,7 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
             D128x64x128w8 = kNumCfgs + 15, D256x128x64w8 = kNumCfgs + 16, D128x128x128r2w8 = kNumCfgs + 17,
             D64x64x128r2 = kNumCfgs + 6, D64x128x128w8 = kNumCfgs + 18, D64x64x128r4 = kNumCfgs + 12
         };
+        if (!will_preprocess && (d.fh * d.fw > 1 || kbytes >= 256)) return pick_plain_cfg(M, OC, kbytes, d.stride_h * d.stride_w > 1, d.has_z != 0);
         if (OC <= 64) return kbytes <= 64 ? D128x128x64w8 : kbytes <= 256 ? D64x64x128r2 : D64x128x128r2;
         const int64_t t128 = tiles(0);
         // layers with a residual and a short reduction (the expanding 1x1 of a bottleneck block) are bound by their
