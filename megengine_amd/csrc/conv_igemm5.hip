@@ -355,6 +355,9 @@ int igemm5_pick(const IgemmArgs& a, int pin, int pout) {
         // Graph replays of every tile, us, ks against patch: 128 -> 128 at 28 x 28, batch 1 (g16 = 392): 5.4 / 5.9, batch 4:
         // 6.8 / 6.0; 232 -> 72 at 40 x 16, stride 2, batch 12: 8.9 / 10.8; 5x5 64 -> 64 at 32 x 32, batch 8: 8.0 / 8.9;
         // 512 -> 512 at 7 x 7, batch 16: 16.1 / 17.9.
+        // 3x3 over at most 32 channels: the patch tile that has one stage too is ahead at any number of pixels (32 -> 20, 1980 pixels:
+        // 3.75 us / 4.5; 24 -> 12, 112 pixels: 3.5 / 4.1); over 64 the two meet at about 200 tiles of 16 x 16.
+        if (K <= 288 && patch4_one_stage(a, pin, pout)) return -1;
         const bool patch = patch4_can_run(a, pin, pout, 0), few_taps = a.T <= 9 && a.sh == 1 && a.sw == 1;
         if (K >= 128 && g16 <= 300) id = ks_id(4, 16, 1, K >= 1024 ? 8 : 4);
         else if (K >= 1024 && g16 <= 450) id = ks_id(4, 16, 1, 4);

@@ -533,6 +533,7 @@ int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg
 int patch4_num_cfgs();
 const char* patch4_cfg_name(int cfg);
 bool patch4_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
+bool patch4_one_stage(const IgemmArgs& a, int pin, int pout);
 int patch4_pick(const IgemmArgs& a, int pin, int pout);  // its tile for this problem, -1 where another kernel is ahead
 int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg);
 
