@@ -574,10 +574,10 @@ bool algo_usable(const ConvProblem& p, int id) {
 // dnn/src/cuda/conv_bias/opr_impl.cpp:44-238): channel-wise kernel, the 4-channel first-layer kernel,
 // then the MFMA implicit GEMM, then the generic direct kernel.  workspace, bytes: what the caller brought (the workspace
 // limit of get_algorithm_heuristic, dnn/include/megdnn/oprs/base.h:595-614).
-// Plain NCHW takes its MFMA algorithm, a packing launch ahead of the convolution, from 2^22 multiply-adds on.  The line is
-// not where the two meet: graph replays of 500 sizes of 2^13 to 2^25 multiply-adds put the generic kernel, whose threads walk
-// their reductions alone, at 13 to 183 us and this one at 6 to 8, and reductions of 32 and more ahead of it from 2^16 on.  It
-// is the line below which a call needs no workspace, which callers may rely on.
+// Plain NCHW takes its MFMA algorithm from 2^22 multiply-adds on.  It is the line below which a call needs no workspace, which
+// callers may rely on, and not where two kernels meet: on either side most sizes run on the one-launch patch kernel
+// (conv_patch1.hip), which packs nothing; what it does not take is packed by a launch of its own above the line (6 to 8 us
+// up to 2^25 multiply-adds) and left to the generic kernel below it.
 constexpr uint64_t kNchwMfmaMacs = 1ull << 22;
 int pick_algo(const ConvProblem& p, const void* workspace, size_t bytes) {
     if (depthwise_usable(p)) return ALGO_DEPTHWISE;
