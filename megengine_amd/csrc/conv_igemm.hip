@@ -684,6 +684,17 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         if (igemm_resolve_cfg(p, s) == s) return s;
     }
     if (p.pin == 32 && p.pout == 32 && d.group == 1 && !igemm_needs_general(p) && d.fh == 1 && d.fw == 1 && d.pad_h == 0 &&
+        d.pad_w == 0 && !d.has_z) {
+        // pointwise without a residual over at most 96 channels, any number out, from about a million outputs on: the same
+        // kernel, whose waves have no ring to fill, with the filter pre-processed or not (us; tiled plain, tiled pre-processed,
+        // streaming: 64 -> 256, 200704 pixels: 21.5 / 23.1 / 18.9; 96 -> 160, 136512: 16.4 / 15.5 / 11.2; 32 -> 800, 12384: 8.9 /
+        // 7.4 / 6.3; below, 96 -> 480, 1600: 4.3 / 4.2 / 4.7).  Over 128 only into one block of channels (128 -> 32, 12000: 4.8 /
+        // 4.0 / 3.8; 128 -> 704, 8528: 7.9 / 7.9 / 8.8).
+        const int64_t M = (int64_t)d.n * p.oh * p.ow;
+        const int s = igemm_pw32s_cfg();
+        if ((d.ic <= 96 ? M * (int64_t)d.oc >= 1100000 : d.ic <= 128 && d.oc <= 32 && M >= 8192) && igemm_resolve_cfg(p, s) == s) return s;
+    }
+    if (p.pin == 32 && p.pout == 32 && d.group == 1 && !igemm_needs_general(p) && d.fh == 1 && d.fw == 1 && d.pad_h == 0 &&
         d.pad_w == 0 && d.has_z && d.ic <= 128) {
         // pointwise with a residual over at most 128 channels (the expanding 1x1 of a bottleneck block): bound by the
         // vector instructions of the requantisation, which the residual table form halves -- the streaming kernel where

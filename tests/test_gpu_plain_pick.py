@@ -14,6 +14,8 @@ pytestmark = pytest.mark.gpu
     (12, 64, 31, 45, 96, 5, 1, True, None),
     (9, 96, 47, 46, 320, 3, 1, False, {"v2_128x256x64r3w8", "dma128x128x128r2w8"}),   # many tiles: the large ones
     (33, 64, 30, 31, 64, 5, 1, False, {"dma64x128x128w8", "v2_64x128x64r4"}),         # 64 channels: no tile of 128
+    (9, 96, 31, 33, 160, 1, 1, False, {"pw32_stream"}),                               # pointwise, at most 96 channels, no residual
+    (3, 96, 40, 41, 224, 1, 2, False, None),                                          # the same with fewer outputs
 ])
 def test_plain_pick(oracle, n, ic, h, w, oc, f, stride, z, names):
     d = _abi.make_conv_desc("NCHW32", n, ic, h, w, oc, f, pad=f // 2, stride=stride, nonline="RELU", has_z=z, scale_bias=2e-4, scale_z=0.05,
