@@ -53,18 +53,6 @@ struct DwmArgs {
     EpiParams epi;
 };
 
-__device__ __forceinline__ void dwm_requant(v4i x, v4i y, uint32_t (&w)[2], const EpiParams& e) {
-#define MI355_BOTH(F)                                  \
-    do {                                               \
-        w[0] = F(x[0], x[1], x[2], x[3], w[0], e);     \
-        w[1] = F(y[0], y[1], y[2], y[3], w[1], e);     \
-    } while (0)
-    if (e.lin) MI355_BOTH((requant4_fast<NL_LIN, false>));
-    else if (e.nonline == NL_RELU && !e.has_z) MI355_BOTH((requant4_fast<NL_RELU, false>));
-    else MI355_BOTH(requant4);
-#undef MI355_BOTH
-}
-
 template <int STEPS, bool HZ>
 __global__ __launch_bounds__(256) void dwm_kernel(DwmArgs a) {
     extern __shared__ __attribute__((aligned(16))) v4i lds_dwm[];  // patch, filter table
@@ -176,7 +164,7 @@ __global__ __launch_bounds__(256) void dwm_kernel(DwmArgs a) {
         for (int st = 0; st < STEPS; ++st)
 #pragma unroll
             for (int k = 0; k < 2; ++k) acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[st], fb[k][st], acc[k], 0, 0, 0);
-        dwm_requant(acc[0], acc[1], zw, a.epi);
+        requant8(acc[0], acc[1], zw, a.epi);
 #pragma unroll
         for (int k = 0; k < 2; ++k) __builtin_amdgcn_raw_buffer_store_b32(zw[k], rs_dst, d[k], 0, 0);
     }

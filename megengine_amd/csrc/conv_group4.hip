@@ -133,19 +133,6 @@ struct G16Args {
     EpiParams epi;
 };
 
-// both dwords through one choice of the requantisation form; the results replace the residual words
-__device__ __forceinline__ void requant8(v4i x, v4i y, uint32_t (&w)[2], const EpiParams& e) {
-#define MI355_BOTH(F)                                  \
-    do {                                               \
-        w[0] = F(x[0], x[1], x[2], x[3], w[0], e);     \
-        w[1] = F(y[0], y[1], y[2], y[3], w[1], e);     \
-    } while (0)
-    if (e.lin) MI355_BOTH((requant4_fast<NL_LIN, false>));
-    else if (e.nonline == NL_RELU && !e.has_z) MI355_BOTH((requant4_fast<NL_RELU, false>));
-    else MI355_BOTH(requant4);
-#undef MI355_BOTH
-}
-
 template <bool HZ>
 __global__ __launch_bounds__(256) void grp16_kernel(G16Args a) {
     __shared__ __attribute__((aligned(16))) v4i sm[G16_PX], sf[144];

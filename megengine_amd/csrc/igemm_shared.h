@@ -93,6 +93,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint3
 
 constexpr int SENT = (int)0x80000000;  // byte offset that is out of range for every buffer (< 2 GiB)
 
+// both dwords through one choice of the requantisation form; the results replace the residual words
+__device__ __forceinline__ void requant8(v4i x, v4i y, uint32_t (&w)[2], const EpiParams& e) {
+#define MI355_BOTH(F)                                  \
+    do {                                               \
+        w[0] = F(x[0], x[1], x[2], x[3], w[0], e);     \
+        w[1] = F(y[0], y[1], y[2], y[3], w[1], e);     \
+    } while (0)
+    if (e.lin) MI355_BOTH((requant4_fast<NL_LIN, false>));
+    else if (e.nonline == NL_RELU && !e.has_z) MI355_BOTH((requant4_fast<NL_RELU, false>));
+    else MI355_BOTH(requant4);
+#undef MI355_BOTH
+}
+
 // Residual (z) of one wave tile in the order the epilogue consumes it: POUT = 32: one 16-byte vector per 32x32 block
 // (16 consecutive channels of the lane's pixel); POUT = 4: four dwords per block.
 template <int MT, int NT>
