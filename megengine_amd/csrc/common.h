@@ -126,8 +126,7 @@ static inline FastDiv make_fastdiv(uint32_t d) {
         f.m = 0; f.s1 = 0; f.s2 = 0;
         return f;
     }
-    uint32_t l = 0;
-    while ((1ull << l) < d) ++l;
+    const uint32_t l = 32 - (uint32_t)__builtin_clz(d - 1);  // smallest l with 2^l >= d (1 < d)
     f.m = (uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1);
     f.s1 = 1;
     f.s2 = l - 1;
