@@ -52,6 +52,14 @@ def test_bind_without_host_memory():
     assert r.returncode == 0 and "ALL OK" in r.stdout, r.stdout[-4000:]
 
 
+def test_sanitizer_builds_cover_every_source():
+    """a library that the sanitizer targets link without one of its sources has undefined references and never runs"""
+    from megengine_amd import build
+    out = subprocess.run(["make", "-s", "--no-print-directory", "-C", os.path.join(ROOT, "tests", "host"), "sources"],
+                         capture_output=True, text=True, check=True).stdout
+    assert sorted(out.split()) == sorted(s[:-len(".hip")] for s in build.SOURCES)
+
+
 @pytest.mark.gpu
 def test_host_classes_gpu():
     """exec of every listed algorithm through the C++ classes, bit-exact against the CPU checker"""
