@@ -601,13 +601,14 @@ static bool igemm_plain_s32(const ConvProblem& p) {
 
 // 32-packed dense layers with the filter in the reference layout.  What such a layer takes on a tile is a price per launch (a chain of
 // copies as long as the reduction), one per round of tiles over the device's CUs and one per tile and CU, each with a part that grows
-// with the reduction.  The prices, in us and us per 1024 reduction bytes, are fitted to graph replays of 600 layers of 32 to 1024
-// channels, 1x1 to 5x5, stride 1 and 2, batch 1 to 64, each on nineteen tiles (two halves of them predict each other as well as
-// themselves); the five tiles here hold the best of the nineteen to 3.5 % on average, where the thresholds that they replace lost 15 %:
+// with the reduction.  The prices, in us and us per 1024 reduction bytes, are fitted to graph replays on 256 CUs of 600 layers of 32
+// to 1024 channels, 1x1 to 5x5, stride 1 and 2, batch 1 to 64, each on nineteen tiles (two halves of them predict each other as well
+// as themselves); the five tiles here hold the best of the nineteen to 3.5 % on average, where the thresholds that they replace lost
+// 15 %:
 // 1.11 times as fast over the 600, and 3x3 288 -> 672 at 45 x 37, batch 10: 48.8 -> 34.4 us; 5x5 32 -> 992 at 51 x 64, stride 2, batch
 // 59: 70.8 -> 63.4; 3x3 320 -> 192 at 17 x 57, batch 53: 47.7 -> 36.8; 1x1 320 -> 672 at 60 x 34, batch 49: 63.7 -> 47.8.
 // (600 layers: 61 are more than 3 % slower on the new choice.)
-static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool strided, bool has_z) {
+static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool strided, bool has_z, int cu_count) {
     struct Price {
         int cfg, bm, bn;
         float launch, launch_k, round, round_k, tile, tile_k, tile_strided_k, tile_z;
@@ -625,7 +626,7 @@ static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool strided, bool has_
     int cfg = -1;
     for (const Price& c : prices) {
         const int64_t tiles = (int64_t)((OC + c.bm - 1) / c.bm) * ((M + c.bn - 1) / c.bn);
-        const float rounds = (float)((tiles + 255) / 256), share = tiles / 256.0f;
+        const float rounds = (float)((tiles + cu_count - 1) / cu_count), share = tiles / (float)cu_count;
         const float us = c.launch + c.launch_k * k + rounds * (c.round + c.round_k * k) +
                          share * (c.tile + c.tile_k * k + (strided ? c.tile_strided_k * k : 0) + (has_z ? c.tile_z : 0));
         if (cfg < 0 || us < best) {
@@ -792,7 +793,7 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
             D128x64x128w8 = kNumCfgs + 15, D256x128x64w8 = kNumCfgs + 16, D128x128x128r2w8 = kNumCfgs + 17,
             D64x64x128r2 = kNumCfgs + 6, D64x128x128w8 = kNumCfgs + 18, D64x64x128r4 = kNumCfgs + 12
         };
-        if (!will_preprocess && (d.fh * d.fw > 1 || kbytes >= 256)) return pick_plain_cfg(M, OC, kbytes, d.stride_h * d.stride_w > 1, d.has_z != 0);
+        if (!will_preprocess && (d.fh * d.fw > 1 || kbytes >= 256)) return pick_plain_cfg(M, OC, kbytes, d.stride_h * d.stride_w > 1, d.has_z != 0, cu_count);
         if (OC <= 64) return kbytes <= 64 ? D128x128x64w8 : kbytes <= 256 ? D64x64x128r2 : D64x128x128r2;
         const int64_t t128 = tiles(0);
         // layers with a residual and a short reduction (the expanding 1x1 of a bottleneck block) are bound by their

@@ -52,6 +52,16 @@ def test_bind_without_host_memory():
     assert r.returncode == 0 and "ALL OK" in r.stdout, r.stdout[-4000:]
 
 
+def test_tiles_follow_the_size_of_the_device():
+    """tests/host/pick_cu.cpp: n images on half a device take the tile of 2n images on a whole one"""
+    _binary(allow_build=True)
+    exe = os.path.join(ROOT, "tests", "host", "pick_cu")
+    if not os.path.exists(exe):
+        subprocess.check_call(["make", "-C", os.path.dirname(exe), "-s", exe])
+    r = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert r.returncode == 0 and "ALL OK" in r.stdout, r.stdout[-4000:]
+
+
 def test_sanitizer_builds_cover_every_source():
     """a library that the sanitizer targets link without one of its sources has undefined references and never runs"""
     from megengine_amd import build
