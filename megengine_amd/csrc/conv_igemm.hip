@@ -601,34 +601,44 @@ static bool igemm_plain_s32(const ConvProblem& p) {
 
 // 32-packed dense layers with the filter in the reference layout.  What such a layer takes on a tile is a price per launch (a chain of
 // copies as long as the reduction), one per round of tiles over the device's CUs and one per tile and CU, each with a part that grows
-// with the reduction.  The prices, in us and us per 1024 reduction bytes, are fitted to graph replays on 256 CUs of 600 layers of 32
-// to 1024 channels, 1x1 to 5x5, stride 1 and 2, batch 1 to 64, each on nineteen tiles (two halves of them predict each other as well
-// as themselves); the five tiles here hold the best of the nineteen to 3.5 % on average, where the thresholds that they replace lost
-// 15 %:
-// 1.11 times as fast over the 600, and 3x3 288 -> 672 at 45 x 37, batch 10: 48.8 -> 34.4 us; 5x5 32 -> 992 at 51 x 64, stride 2, batch
-// 59: 70.8 -> 63.4; 3x3 320 -> 192 at 17 x 57, batch 53: 47.7 -> 36.8; 1x1 320 -> 672 at 60 x 34, batch 49: 63.7 -> 47.8.
-// (600 layers: 61 are more than 3 % slower on the new choice.)
-static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool strided, bool has_z, int cu_count) {
+// with the reduction.  Four terms separate what those leave together:
+//   line_k: filter rows of whole 128-byte lines.  The second-generation tiles read a plain filter 32 bytes of every row at a time, all
+//     of them at the same place of a line then: 10 to 20 % longer than one channel block more or less (3x3 over 384 channels, stride 2,
+//     165 tiles of 64 x 64: 13.8 us; over 416, 168 of them: 12.2).  The first-generation tiles read whole rows and hardly have it.
+//   alone_k: no more tiles than CUs, so that no second workgroup covers a stage's copies.
+//   pair_k: a round of two workgroups to a CU, which the tiles with small rings go by.
+//   window: the table of offsets that a workgroup of a windowed layer begins with.
+// The prices, in us and us per 1024 reduction bytes, are fitted to graph replays on 256 CUs of 2640 layers of 32 to 2048 channels, 1x1 to
+// 5x5, stride 1 and 2, batch 1 to 64 (two halves of them predict each other as well as themselves).  The six tiles here hold the best of
+// eleven to nineteen to 1.9 % on average and are 1.13 times as fast as thresholds on tile counts: 3x3 288 -> 672 at 45 x 37, batch 10:
+// 48.8 -> 34.4 us; 5x5 32 -> 992 at 51 x 64, stride 2, batch 59: 70.8 -> 63.4; 1x1 320 -> 672 at 60 x 34, batch 49: 63.7 -> 47.8.
+// Without the four terms and the last tile it was 1.11, and 306 of the 2640 were more than 3 % slower than by thresholds (97 more than
+// 10 %); 79 are with them (9), at most 1.19.
+static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool window, bool strided, bool has_z, int cu_count) {
     struct Price {
         int cfg, bm, bn;
-        float launch, launch_k, round, round_k, tile, tile_k, tile_strided_k, tile_z;
+        float launch, window, launch_k, round, round_k, pair_k, tile, tile_k, strided_k, z, line_k, alone_k;
     };
     const int dma = kNumCfgs, v2 = igemm_first_v2_cfg();
     const Price prices[] = {
-            {dma + 18, 64, 128, 4.11f, 0.62f, 0.57f, 1.37f, 0.57f, 0.52f, 0.20f, 0.28f},   // dma64x128x128w8
-            {v2 + 10, 128, 256, 4.35f, 0.14f, 0.31f, 4.79f, 1.74f, 0.52f, 2.85f, 1.96f},   // v2_128x256x64r3w8
-            {v2 + 8, 64, 64, 3.88f, 0.49f, 0.00f, 1.61f, 0.52f, 0.00f, 0.29f, 0.18f},      // v2_64x64x128r4
-            {dma + 17, 128, 128, 3.31f, 1.75f, 0.88f, 1.91f, 0.86f, 0.59f, 0.39f, 0.65f},  // dma128x128x128r2w8
-            {v2 + 4, 64, 128, 3.95f, 1.12f, 0.02f, 1.94f, 0.67f, 0.18f, 0.65f, 0.47f},     // v2_64x128x64r4
+            {dma + 18, 64, 128, 3.61f, 0.25f, 0.00f, 0.70f, 1.53f, 0.18f, 0.30f, 0.50f, 0.18f, 0.28f, 0.02f, 0.31f},   // dma64x128x128w8
+            {v2 + 10, 128, 256, 3.78f, 0.01f, 0.03f, 0.96f, 4.89f, 0.03f, 1.01f, 0.14f, 2.61f, 2.21f, 1.64f, 0.00f},   // v2_128x256x64r3w8
+            {v2 + 8, 64, 64, 3.44f, 0.22f, 0.32f, 0.47f, 1.62f, 0.01f, 0.00f, 0.00f, 0.36f, 0.19f, 0.39f, 0.00f},      // v2_64x64x128r4
+            {dma + 17, 128, 128, 3.30f, 0.21f, 0.00f, 0.84f, 1.64f, 1.83f, 0.50f, 0.79f, 0.38f, 0.79f, 0.00f, 0.09f},  // dma128x128x128r2w8
+            {v2 + 4, 64, 128, 3.46f, 0.64f, 0.04f, 0.32f, 2.30f, 0.18f, 0.21f, 0.00f, 0.48f, 0.55f, 0.60f, 0.31f},     // v2_64x128x64r4
+            {dma + 12, 64, 64, 3.37f, 0.53f, 0.00f, 0.69f, 0.23f, 1.41f, 0.00f, 0.41f, 0.11f, 0.19f, 0.00f, 0.21f},    // dma64x64x128r4
     };
     const float k = kbytes / 1024.0f;
+    const bool lines = kbytes % 128 == 0;
     float best = 0;
     int cfg = -1;
     for (const Price& c : prices) {
         const int64_t tiles = (int64_t)((OC + c.bm - 1) / c.bm) * ((M + c.bn - 1) / c.bn);
         const float rounds = (float)((tiles + cu_count - 1) / cu_count), share = tiles / (float)cu_count;
-        const float us = c.launch + c.launch_k * k + rounds * (c.round + c.round_k * k) +
-                         share * (c.tile + c.tile_k * k + (strided ? c.tile_strided_k * k : 0) + (has_z ? c.tile_z : 0));
+        const float pairs = (float)((tiles + 2 * cu_count - 1) / (2 * cu_count));
+        const float tile = c.tile + k * (c.tile_k + (strided ? c.strided_k : 0) + (lines ? c.line_k : 0)) + (has_z ? c.z : 0);
+        const float us = c.launch + (window ? c.window : 0) + k * (c.launch_k + (tiles <= cu_count ? c.alone_k : 0) + pairs * c.pair_k) +
+                         rounds * (c.round + c.round_k * k) + share * tile;
         if (cfg < 0 || us < best) {
             best = us;
             cfg = c.cfg;
@@ -793,7 +803,7 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
             D128x64x128w8 = kNumCfgs + 15, D256x128x64w8 = kNumCfgs + 16, D128x128x128r2w8 = kNumCfgs + 17,
             D64x64x128r2 = kNumCfgs + 6, D64x128x128w8 = kNumCfgs + 18, D64x64x128r4 = kNumCfgs + 12
         };
-        if (!will_preprocess && (d.fh * d.fw > 1 || kbytes >= 256)) return pick_plain_cfg(M, OC, kbytes, d.stride_h * d.stride_w > 1, d.has_z != 0, cu_count);
+        if (!will_preprocess && (d.fh * d.fw > 1 || kbytes >= 256)) return pick_plain_cfg(M, OC, kbytes, d.fh * d.fw > 1, d.stride_h * d.stride_w > 1, d.has_z != 0, cu_count);
         if (OC <= 64) return kbytes <= 64 ? D128x128x64w8 : kbytes <= 256 ? D64x64x128r2 : D64x128x128r2;
         const int64_t t128 = tiles(0);
         // layers with a residual and a short reduction (the expanding 1x1 of a bottleneck block) are bound by their
