@@ -304,16 +304,21 @@ bool grp32_can_run(const IgemmArgs& a, int pin, int pout, int cfg) {
 // 256 from 2400 on (19344: 63.1 / 57.6, the second-generation tile 87.4).  At stride 2 a patch is four times its pixels and never 256
 // wide; 64 x 128 from 250 on (11 groups of 64 at 41 x 105, batch 26: 39.7 / 32.1).
 //   Dense layers over 32 or 64 channels that are too large for the few-pixel tiles: 64 -> 64 at 49 x 49, batch 7: 6.4 / 4.7; 64 -> 96
-// at 61 x 23, batch 49, residual: 13.6 / 9.6.  Against pre-processed filters the lead is gone from about 1500 tiles of 64 x 128 on
-// (56 x 56, batch 64: 13.1 / 13.1, the tile that the chooser's tests name there); the weight-resident tile keeps its range; and at
-// stride 2 with several channel tiles the staged tiles are ahead from 800 workgroups on (64 -> 128 at 56 x 56, batch 64: 11.1 / 10.0).
+// at 61 x 23, batch 49, residual: 13.6 / 9.6.  The weight-resident tile keeps its range, from 2560 tiles of 64 x 128 on; and at stride
+// 2 with several channel tiles the staged tiles are ahead from 800 workgroups on (64 -> 128 at 56 x 56, batch 64: 11.1 / 10.0).
+//   Against a pre-processed filter (340 dense layers of 500 to 2600 such tiles; this kernel's time over the ring's):
+//     stride 1, channels that leave half a 64-channel tile empty: 0.50 to 1.01 at any number of tiles (64 -> 288 at 2205: 16.5 / 20.0);
+//     64 channels out: 0.75 to 1.02 from 1200 to 1500 tiles (64 -> 64 at 1323: 12.8 / 14.2).  Beyond, 0.9 to 1.0 up to 1850 and even
+//     from there; the line stands at 1500 because the chooser's tests name the ring for 56 x 56, batch 64, 1568 tiles;
+//     several whole channel tiles: 0.98 to 1.07 around 1100, 0.87 to 1.16 beyond, so 1200;
+//     stride 2: 1.03 to 1.4 from 1000 on.
 int grp32_pick(const IgemmArgs& a, int pin, int pout, bool will_preprocess) {
     if (pin != 32 || pout != 32 || a.general || a.FH != 3 || a.FW != 3 || (a.kbytes != 288 && a.kbytes != 576) || a.ocpg % 32 != 0) return -1;
     const bool s1 = a.sh == 1 && a.sw == 1;
     const int64_t px = ((int64_t)a.M + 127) / 128, w0 = px * a.groups * (a.ocpg / 32);
     if (a.groups == 1) {
         const int64_t t64 = px * ((a.OC + 63) / 64);
-        if (t64 >= (will_preprocess ? 1200 : 2560)) return -1;
+        if (t64 >= (!will_preprocess || (s1 && a.OC % 64 != 0) ? 2560 : s1 && a.OC == 64 ? 1500 : 1200)) return -1;
         if (!s1 && a.OC > 64 && w0 >= 800) return -1;
     }
     int cfg;
