@@ -241,7 +241,7 @@ bool g32_plan(const IgemmArgs& a, int cfg, G32Args* k, int* lds_bytes) {
         }
         if (PX > max_px) continue;
         const int tiles_img = cols * ((a.OH + TH - 1) / TH);
-        const int64_t tiles = ((int64_t)a.NB + NI - 1) / NI * tiles_img, cost = tiles * 4096 + PX;  // fewest tiles, then the smallest patch
+        const int64_t tiles = (int64_t)(((uint32_t)a.NB + NI - 1) / NI) * tiles_img, cost = tiles * 4096 + PX;  // fewest tiles, then the smallest patch
         if (best < 0 || cost < best) {
             if (tiles > 0x3fffffff) return false;
             best = cost;

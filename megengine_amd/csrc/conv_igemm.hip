@@ -616,28 +616,29 @@ static bool igemm_plain_s32(const ConvProblem& p) {
 // 10 %); 79 are with them (9), at most 1.19.
 static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool window, bool strided, bool has_z, int cu_count) {
     struct Price {
-        int cfg, bm, bn;
+        int cfg, bm, bn;  // tile: 2^bm channels x 2^bn pixels
         float launch, window, launch_k, round, round_k, pair_k, tile, tile_k, strided_k, z, line_k, alone_k;
     };
     const int dma = kNumCfgs, v2 = igemm_first_v2_cfg();
     const Price prices[] = {
-            {dma + 18, 64, 128, 3.61f, 0.25f, 0.00f, 0.70f, 1.53f, 0.18f, 0.30f, 0.50f, 0.18f, 0.28f, 0.02f, 0.31f},   // dma64x128x128w8
-            {v2 + 10, 128, 256, 3.78f, 0.01f, 0.03f, 0.96f, 4.89f, 0.03f, 1.01f, 0.14f, 2.61f, 2.21f, 1.64f, 0.00f},   // v2_128x256x64r3w8
-            {v2 + 8, 64, 64, 3.44f, 0.22f, 0.32f, 0.47f, 1.62f, 0.01f, 0.00f, 0.00f, 0.36f, 0.19f, 0.39f, 0.00f},      // v2_64x64x128r4
-            {dma + 17, 128, 128, 3.30f, 0.21f, 0.00f, 0.84f, 1.64f, 1.83f, 0.50f, 0.79f, 0.38f, 0.79f, 0.00f, 0.09f},  // dma128x128x128r2w8
-            {v2 + 4, 64, 128, 3.46f, 0.64f, 0.04f, 0.32f, 2.30f, 0.18f, 0.21f, 0.00f, 0.48f, 0.55f, 0.60f, 0.31f},     // v2_64x128x64r4
-            {dma + 12, 64, 64, 3.37f, 0.53f, 0.00f, 0.69f, 0.23f, 1.41f, 0.00f, 0.41f, 0.11f, 0.19f, 0.00f, 0.21f},    // dma64x64x128r4
+            {dma + 18, 6, 7, 3.61f, 0.25f, 0.00f, 0.70f, 1.53f, 0.18f, 0.30f, 0.50f, 0.18f, 0.28f, 0.02f, 0.31f},  // dma64x128x128w8
+            {v2 + 10, 7, 8, 3.78f, 0.01f, 0.03f, 0.96f, 4.89f, 0.03f, 1.01f, 0.14f, 2.61f, 2.21f, 1.64f, 0.00f},   // v2_128x256x64r3w8
+            {v2 + 8, 6, 6, 3.44f, 0.22f, 0.32f, 0.47f, 1.62f, 0.01f, 0.00f, 0.00f, 0.36f, 0.19f, 0.39f, 0.00f},    // v2_64x64x128r4
+            {dma + 17, 7, 7, 3.30f, 0.21f, 0.00f, 0.84f, 1.64f, 1.83f, 0.50f, 0.79f, 0.38f, 0.79f, 0.00f, 0.09f},  // dma128x128x128r2w8
+            {v2 + 4, 6, 7, 3.46f, 0.64f, 0.04f, 0.32f, 2.30f, 0.18f, 0.21f, 0.00f, 0.48f, 0.55f, 0.60f, 0.31f},    // v2_64x128x64r4
+            {dma + 12, 6, 6, 3.37f, 0.53f, 0.00f, 0.69f, 0.23f, 1.41f, 0.00f, 0.41f, 0.11f, 0.19f, 0.00f, 0.21f},  // dma64x64x128r4
     };
     const float k = kbytes / 1024.0f;
     const bool lines = kbytes % 128 == 0;
+    const uint32_t cu = cu_count;
     float best = 0;
     int cfg = -1;
     for (const Price& c : prices) {
-        const int64_t tiles = (int64_t)((OC + c.bm - 1) / c.bm) * ((M + c.bn - 1) / c.bn);
-        const float rounds = (float)((tiles + cu_count - 1) / cu_count), share = tiles / (float)cu_count;
-        const float pairs = (float)((tiles + 2 * cu_count - 1) / (2 * cu_count));
+        const uint32_t tiles = (uint32_t)((OC + (1 << c.bm) - 1) >> c.bm) * (uint32_t)((M + (1 << c.bn) - 1) >> c.bn);  // (OC * M < 2^31)
+        const uint32_t full = (tiles + cu - 1) / cu;
+        const float rounds = (float)full, pairs = (float)((full + 1) / 2), share = (float)tiles / (float)cu;
         const float tile = c.tile + k * (c.tile_k + (strided ? c.strided_k : 0) + (lines ? c.line_k : 0)) + (has_z ? c.z : 0);
-        const float us = c.launch + (window ? c.window : 0) + k * (c.launch_k + (tiles <= cu_count ? c.alone_k : 0) + pairs * c.pair_k) +
+        const float us = c.launch + (window ? c.window : 0) + k * (c.launch_k + (full <= 1 ? c.alone_k : 0) + pairs * c.pair_k) +
                          rounds * (c.round + c.round_k * k) + share * tile;
         if (cfg < 0 || us < best) {
             best = us;
@@ -853,6 +854,7 @@ int igemm_pick_cfg(const ConvProblem& p, int cu_count, bool will_preprocess) {
     if (igemm_group_by_launch(p) && grp4_pick(p)) return igemm_grp4_cfg();
     if (igemm_group_by_launch(p)) return igemm_pick_cfg(igemm_group_view(p), cu_count, will_preprocess);
     const int c = pick_cfg_by_shape(p, cu_count, will_preprocess);
+    if (c >= igemm_first_g32_cfg()) return c;  // (its plan, which grp32_pick has made, is all that there is to resolve)
     const int r = igemm_resolve_cfg(p, c);
     return r >= 0 ? r : c;
 }
