@@ -460,6 +460,10 @@ bool patch1_usable(const ConvProblem& p) {
 // 14 -> 19, 202800 pixels: 15.6 us against 18.5), and 64 x 256, which turns a patch for twice the channels, once those are two per
 // CU (3x3 8 -> 189, 61950 pixels: 15.6 against 18.9 and 20.1).  At strides a patch is several times its pixels: 64 x 128 (3x3 38 ->
 // 97, stride 2, 588 workgroups: 14.0 against 18.3).
+//   At strides every tile of 64 channels turns that patch again, so from three of them on, at 2000 workgroups and more, packing once is
+// ahead on filters of 1x1 and 3x3 (23 layers, this kernel over the packed path: 0.84 to 1.83, 1.19 on average; 3x3 6 -> 194 at 59 x 107,
+// batch 57: 51.4 / 28.1; 1x1 7 -> 197 at 89 x 27, batch 51: 19.6 / 13.9).  Not with a residual (1.00 on 10 layers), not where rows out
+// are whole quads (0.95 on 5), not with 25 taps (1.0 on 4), whose products outweigh the turning.
 int patch1_pick(const ConvProblem& p, bool packed) {
     if (!patch1_usable(p)) return -1;
     P1Args k;
@@ -472,7 +476,10 @@ int patch1_pick(const ConvProblem& p, bool packed) {
     if (packed && w0 < 64 && macs >= (1u << 24)) return -1;
     if (packed && w0 < 128 && k.nstages >= (T == 1 ? 4 : T == 9 ? 3 : 2)) return -1;
     if (w0 <= (T == 25 ? 256 : 400)) return 0;
-    if (p.d.stride_h > 1 || p.d.stride_w > 1) return p.d.oc > 32 && wgs(3) > 0 ? 3 : 0;
+    if (p.d.stride_h > 1 || p.d.stride_w > 1) {
+        if (packed && w0 >= 2000 && p.d.oc > 128 && T <= 9 && !p.d.has_z && p.ow % 4 != 0) return -1;
+        return p.d.oc > 32 && wgs(3) > 0 ? 3 : 0;
+    }
     if (p.d.oc > 32 && wgs(2) >= 512) return 2;
     return wgs(1) > 0 ? 1 : 0;
 }
