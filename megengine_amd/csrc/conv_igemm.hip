@@ -796,8 +796,11 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         return tiles(0) >= cu_count ? 0 : 3;
     }
     if (p.pin == 32) {
-        // 32-packed inputs: LDS-direct tiles (ids after the register-staged ones), chosen from a sweep of every
-        // tile over the ResNet-50 / large-convolution shapes.  t128 = number of 128x128 tiles.
+        // 32-packed inputs: LDS-direct tiles (ids after the register-staged ones).  t128 = number of 128x128 tiles.
+        // A plain filter over 256 bytes and more, or with a window, goes by prices.  What is left to the lines below reads the
+        // reference layout too: callers that pre-process the filter, for layers with a residual (which costs these tiles no LDS;
+        // chosen from a sweep of every tile over the ResNet-50 and large-convolution shapes inside their networks, where weights
+        // are cold), for strided windows on few tiles, and for 4-packed outputs; and pointwise layers over at most 224 channels.
         enum {
             D128x128x64 = kNumCfgs + 0, D64x64x128 = kNumCfgs + 1, D128x128x128r2 = kNumCfgs + 7, D64x64x64r4 = kNumCfgs + 10,
             D128x64x128r2 = kNumCfgs + 11, D64x128x128r2 = kNumCfgs + 13, D128x128x64w8 = kNumCfgs + 14,
@@ -815,11 +818,11 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         if (t128 >= 2 * cu_count) return D128x64x128r2;
         if (2 * t128 >= 3 * cu_count) return kbytes >= 512 ? D128x128x128r2w8 : D128x128x64;
         // few tiles, long reductions: the deeper ring hides the cold first touch of every weight byte; the longest
-        // ones (3x3 over 256 channels) run best with more pixels than channels per tile
+        // ones (strided 3x3 over 256 channels) run best with more pixels than channels per tile
         if (kbytes >= 2304 && tiles(6) >= cu_count) return D64x128x128w8;
         if (tiles(7) >= cu_count) return D128x64x128w8;
-        // fewer tiles than CUs: the longest reductions (3x3 over 512 channels) take the deepest ring, 2048-channel
-        // pointwise layers the 8-wave tile with more pixels than channels
+        // fewer tiles than CUs: the longest reductions take the deepest ring, those of 2048 to 4607 bytes with a 64 x 128 tile for
+        // three CUs of four the 8-wave tile with more pixels than channels
         if (kbytes >= 4608) return D64x64x128r4;
         return kbytes >= 2048 && 4 * tiles(6) >= 3 * cu_count ? D64x128x128w8 : D64x64x128;
     }
