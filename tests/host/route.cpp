@@ -1,15 +1,32 @@
-// Which launches an exec of the heuristic's choice makes (no GPU: the runtime's calls that would need one are answered here, and
-// a launch is only noted).  One layer per line of the input: format (0 NCHW, else as in the interface), n, ic, ih, iw, oc, filter,
-// stride, group, residual; one line of the output for each: the number of launches, and dynamic LDS and threads of the last one.
+// Which kernels an exec launches (no GPU: the runtime's calls that would need one are answered here, and a launch is only noted).
+// One exec per line of the input: the descriptor's bytes in hexadecimal, an algorithm (a number: by that name; -1: the heuristic's
+// choice, named; -2: none, exec chooses for itself), its tile (-1: the query's), and whether there is a workspace.  One line of the
+// output for each: the number of launches, dynamic LDS and threads of the last one, and the kernels, separated by tabs.
+#include <cxxabi.h>
 #include <hip/hip_runtime.h>
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
+
+#include <map>
+#include <string>
 
 #include "../../include/mi355_convbias.h"
 
+static std::map<const void*, std::string>& kernels() {  // (filled by the library's constructors, ahead of this file's)
+    static std::map<const void*, std::string> m;
+    return m;
+}
+static std::string g_names;
 static int g_launches;
 static unsigned g_lds, g_threads;
 extern "C" {
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) {
+    int st;
+    char* s = abi::__cxa_demangle(name, nullptr, nullptr, &st);
+    kernels()[host] = s ? s : name;
+    free(s);
+}
 hipError_t hipGetDevice(int* d) {
     *d = 0;
     return hipSuccess;
@@ -24,43 +41,47 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int
     *n = 2;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void*, dim3, dim3 block, void**, size_t lds, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3, dim3 block, void**, size_t lds, hipStream_t) {
     ++g_launches;
     g_lds = (unsigned)lds;
     g_threads = block.x;
+    g_names += "\t" + (kernels().count(f) ? kernels()[f] : "?");
     return hipSuccess;
 }
 }
 
 int main() {
-    unsigned fmt, n, ic, ih, iw, oc, f, stride, group, z;
-    while (scanf("%u %u %u %u %u %u %u %u %u %u", &fmt, &n, &ic, &ih, &iw, &oc, &f, &stride, &group, &z) == 10) {
+    static char hex[2 * sizeof(mi355_conv_desc) + 2];
+    char format[32];
+    snprintf(format, sizeof(format), "%%%zus %%d %%d %%d", sizeof(hex) - 1);
+    int algo, tile, room;
+    while (scanf(format, hex, &algo, &tile, &room) == 4) {
         mi355_conv_desc d;
-        memset(&d, 0, sizeof(d));
-        d.format = fmt;
-        d.sparse = group > 1 ? MI355_SPARSE_GROUP : MI355_SPARSE_DENSE;
-        d.n = n; d.ic = ic; d.oc = oc; d.ih = ih; d.iw = iw; d.group = group;
-        d.fh = d.fw = f;
-        d.pad_h = d.pad_w = f / 2;
-        d.stride_h = d.stride_w = stride;
-        d.dilate_h = d.dilate_w = 1;
-        d.bias_mode = MI355_BIAS_BROADCAST_CHANNEL;
-        d.nonline = MI355_NL_RELU;
-        d.has_z = z;
-        d.dst_dtype = MI355_DT_QS8;
-        d.scale_bias = 2e-4f;
-        d.scale_z = d.scale_dst = 0.05f;
+        unsigned char* bytes = reinterpret_cast<unsigned char*>(&d);
+        unsigned b;
+        if (strlen(hex) != 2 * sizeof(d)) {
+            printf("a descriptor of %zu characters\n", strlen(hex));
+            return 1;
+        }
+        for (size_t i = 0; i < sizeof(d); ++i) {
+            if (sscanf(hex + 2 * i, "%2x", &b) != 1) return 1;
+            bytes[i] = (unsigned char)b;
+        }
         mi355_algo a;
         size_t ws = 0;
         int8_t* const t = reinterpret_cast<int8_t*>(0x1000000);  // device addresses that nothing on the host reads
         g_launches = 0;
-        int st = mi355_convbias_s8_query(&d, MI355_ALGO_HEURISTIC, &a, &ws);
-        if (!st) st = mi355_convbias_s8_exec(nullptr, &d, &a, t, t, reinterpret_cast<int32_t*>(t), z ? t : nullptr, t, t, ws);
+        g_names.clear();
+        int st = mi355_convbias_s8_query(&d, algo < 0 ? MI355_ALGO_HEURISTIC : algo, &a, &ws);
+        if (tile >= 0) a.tile_cfg = tile;
+        if (!st)
+            st = mi355_convbias_s8_exec(nullptr, &d, algo == -2 ? nullptr : &a, t, t, reinterpret_cast<int32_t*>(t), d.has_z ? t : nullptr, t,
+                                        room ? t : nullptr, room ? ws : 0);
         if (st) {
             printf("status %d: %s\n", st, mi355_last_error());
             return 1;
         }
-        printf("%d %u %u\n", g_launches, g_lds, g_threads);
+        printf("%d %u %u%s\n", g_launches, g_lds, g_threads, g_names.c_str());
     }
     return 0;
 }

@@ -1,22 +1,9 @@
-"""Which kernels an exec of the heuristic's choice launches (tests/host/route.cpp, no GPU), for layers where two ways were timed as graph
-replays: the faster one, to 5 %, which a rule over sizes may miss where both are close."""
-import os
-import subprocess
+"""Which kernels an exec of the heuristic's choice launches (tests/host/route.cpp, no GPU): layers where two ways were timed as graph
+replays take the faster one, to 5 %, which a rule over sizes may miss where both are close."""
+from megengine_amd import _abi
+from tests.routes import UNNAMED, routes
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-EXE = os.path.join(ROOT, "tests", "host", "route")
-NCHW, NCHW4 = 0, 3
-
-
-def _routes(layers):
-    """layers: (format, n, ic, ih, iw, oc, f, stride, group, residual) -> (launches, dynamic LDS and threads of the last) each"""
-    if not os.path.exists(EXE):
-        subprocess.check_call(["make", "-C", os.path.dirname(EXE), "-s", EXE])
-    r = subprocess.run([EXE], input="".join(" ".join(str(int(v)) for v in l) + "\n" for l in layers), capture_output=True, text=True, timeout=120)
-    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
-    out = [tuple(int(v) for v in line.split()) for line in r.stdout.splitlines()]
-    assert len(out) == len(layers)
-    return out
+S = dict(scale_bias=2e-4, scale_z=0.05, scale_dst=0.05)
 
 
 # n, ic, ih, iw, oc, f, stride, residual; us packed (two launches) and in one launch
@@ -37,9 +24,78 @@ PLAIN_NCHW = [
 ]
 
 
+def _nchw(n, ic, ih, iw, oc, f, stride=1, z=0, **kw):
+    return _abi.make_conv_desc("NCHW", n, ic, ih, iw, oc, f, pad=f // 2, stride=stride, nonline="RELU", has_z=bool(z), **dict(S, **kw))
+
+
 def test_plain_nchw_strides():
-    got = _routes([(NCHW, n, ic, ih, iw, oc, f, s, 1, z) for n, ic, ih, iw, oc, f, s, z, _, _ in PLAIN_NCHW])
-    for (launches, _, _), layer in zip(got, PLAIN_NCHW):
+    got = routes([_nchw(n, ic, ih, iw, oc, f, s, z) for n, ic, ih, iw, oc, f, s, z, _, _ in PLAIN_NCHW])
+    for r, layer in zip(got, PLAIN_NCHW):
         packed, one = layer[-2:]
-        assert launches in (1, 2)
-        assert (packed if launches == 2 else one) <= 1.05 * min(packed, one), layer
+        assert r.launches in (1, 2)
+        assert (packed if r.launches == 2 else one) <= 1.05 * min(packed, one), layer
+
+
+def _kernels(execs):
+    return [r.kernels for r in routes(execs)]
+
+
+def test_plain_nchw_lines():
+    """Both sides of every line of patch1_pick, with a workspace; planes out of 8 x 16 are one tile of 128 pixels, 32 channels out one of 32"""
+    plane = lambda n, ic, oc, f, stride=1: _nchw(n, ic, 8 * stride, 16 * stride, oc, f, stride)  # noqa: E731
+    k = lambda mt, nt, taps: ("patch1_kernel<%d, %d, %d>" % (mt, nt, taps),)  # noqa: E731
+    table = [
+        (plane(63, 64, 32, 3), None), (plane(64, 64, 32, 3), k(1, 1, 9)),     # 64 workgroups,
+        (plane(63, 14, 32, 3), None), (plane(63, 7, 32, 3), k(1, 1, 9)),      # or 2^24 multiply-adds
+        (plane(127, 65, 32, 3), None), (plane(128, 65, 32, 3), k(1, 1, 9)), (plane(127, 64, 32, 3), k(1, 1, 9)),        # stages
+        (plane(127, 193, 32, 1), None), (plane(128, 193, 32, 1), k(1, 1, 1)), (plane(127, 192, 32, 1), k(1, 1, 1)),
+        (plane(127, 17, 32, 5), None), (plane(128, 17, 32, 5), k(1, 1, 25)), (plane(127, 16, 32, 5), k(1, 1, 25)),
+        (plane(400, 8, 32, 3), k(1, 1, 9)), (plane(401, 8, 32, 3), k(1, 2, 9)),                                         # tiles
+        (plane(256, 8, 32, 5), k(1, 1, 25)), (plane(257, 8, 32, 5), k(1, 2, 25)),
+        (plane(1022, 8, 64, 3), k(1, 2, 9)), (plane(1023, 8, 64, 3), k(2, 2, 9)), (plane(1023, 8, 32, 3), k(1, 2, 9)),
+        (plane(200, 8, 64, 3, 2), k(1, 1, 9)), (plane(201, 8, 64, 3, 2), k(2, 1, 9)), (plane(402, 8, 32, 3, 2), k(1, 1, 9)),
+    ]
+    for got, (d, want) in zip(_kernels([d for d, _ in table]), table):
+        if want is None:
+            assert got[0] == "nchw_prep_kernel" and len(got) == 2, (d.key(), got)
+        else:
+            assert got == want, (d.key(), got)
+    # without a workspace: reductions of five bytes and more, if the caller names nothing
+    one = lambda ic, algo: (plane(2, ic, 32, 1), algo, -1, False)  # noqa: E731
+    assert _kernels([one(4, UNNAMED), one(5, UNNAMED), one(5, 0)]) == [("conv_direct_kernel",), k(1, 1, 1), ("conv_direct_kernel",)]
+
+
+def _dw(n, c, ih, iw, fh, fw, pad, stride):
+    return _abi.make_conv_desc("NCHW4", n, c, ih, iw, c, fh, fw, group=c, pad=pad, stride=stride, nonline="RELU", has_z=True, **S)
+
+
+def test_channel_wise_lines():
+    """Both sides of every line between the matrix form (dwm) and the vector forms (dwf, dw4)"""
+    table = [
+        # 5x5 and 7x7 with their own padding: 512 planes, 100 quads of a plane
+        (_dw(7, 292, 24, 16, 5, 5, 2, 1), "dwm_kernel<3, true>"), (_dw(8, 256, 24, 16, 5, 5, 2, 1), "dwf_kernel<5, 1, 1>"),
+        (_dw(8, 256, 25, 16, 5, 5, 2, 1), "dwm_kernel<3, true>"), (_dw(8, 256, 50, 32, 7, 7, 3, 2), "dwm_kernel<7, true>"),
+        (_dw(8, 256, 48, 32, 7, 7, 3, 2), "dwf_kernel<7, 2, 1>"), (_dw(32, 256, 24, 16, 5, 5, 2, 1), "dwf_kernel<5, 1, 2>"),
+        (_dw(1, 8, 5, 1632, 5, 5, 2, 1), "dwm_kernel<3, true>"), (_dw(1, 8, 5, 1633, 5, 5, 2, 1), "dwf_kernel<5, 1, 1>"),   # one row's patch
+        # other filters: strides, taps, the window's blocks, one row's patch
+        (_dw(1, 8, 24, 24, 7, 1, 0, 2), "dwm_kernel<4, true>"), (_dw(1, 8, 24, 24, 7, 1, 0, 3), "dw4_kernel"),
+        (_dw(1, 8, 24, 24, 9, 1, 0, 3), "dwm_kernel<7, true>"), (_dw(1, 8, 24, 24, 5, 5, 2, 4), "dwm_kernel<7, true>"),
+        (_dw(1, 8, 24, 24, 5, 5, 2, 5), "dw4_kernel"), (_dw(1, 8, 24, 24, 8, 8, 0, 1), "dwm_kernel<6, true>"),
+        (_dw(1, 8, 24, 24, 11, 11, 0, 1), "dw4_kernel"), (_dw(1, 8, 5, 1634, 5, 5, (2, 1), 1), "dwm_kernel<3, true>"),
+        (_dw(1, 8, 5, 1635, 5, 5, (2, 1), 1), "dw4_kernel"), (_dw(1, 8, 70, 9, 5, 5, 0, (65, 1)), "dw4_kernel"),
+    ]
+    for got, (d, want) in zip(_kernels([d for d, _ in table]), table):
+        assert got == (want,), (d.key(), got)
+
+
+def test_one_stage_line():
+    """4-packed 3x3 layers: at most 64 channels are one stage, on every tile"""
+    from megengine_amd import lib
+    tiles = [t for t, name in enumerate(lib.tile_names()) if name.startswith("patch4_")]
+    execs = [(_abi.make_conv_desc("NCHW4", 4, ic, 28, 28, 64, f, pad=f // 2, nonline="RELU", **S), 1, t, False)
+             for ic, f in ((32, 3), (36, 3), (64, 3), (68, 3), (64, 5)) for t in tiles]
+    want = []
+    for form in ("patch4_one_kernel<1, %d, %d>", "patch4_one_kernel<2, %d, %d>", "patch4_one_kernel<2, %d, %d>", "patch4_kernel<%d, %d, 9>",
+                 "patch4_kernel<%d, %d, 0>"):
+        want += [(form % tile,) for tile in ((1, 1), (1, 2), (2, 2))]
+    assert _kernels(execs) == want
