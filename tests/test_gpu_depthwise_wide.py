@@ -1,6 +1,7 @@
-"""Channel-wise 5x5 and 7x7 convolutions at the edges of a thread's work: widths around the blocks of four pixels, odd
-heights (two output rows per thread), images smaller than the filter, both strides, every activation with and without a
-residual; paddings other than F / 2 and odd strides stay on the kernel that takes anything."""
+"""Channel-wise 5x5 and 7x7 convolutions at widths around the blocks of four pixels, odd heights, images smaller than the filter,
+both strides, every activation with and without a residual, and other paddings and strides: on these few or large planes all of them
+run the matrix form (test_gpu_dw_matrix.py); the vector forms have their cases in test_gpu_dw_vector.py.  3x3 layers with one,
+two and four output rows per thread."""
 import pytest
 
 from megengine_amd import _abi, lib, ops
@@ -47,6 +48,7 @@ def test_height_padding_may_differ(oracle):
     (64, 736, 7, 6, 3, 1),
 ])
 def test_rows_per_thread(oracle, n, c, ih, iw, f, stride):
+    """(the lines of 5x5 and 7x7 are the matrix form's now: large planes, several bands)"""
     for nl, z in (("RELU", False), ("IDENTITY", True)):
         d = _abi.make_conv_desc("NCHW4", n, c, ih, iw, c, f, pad=f // 2, stride=stride, group=c, nonline=nl, has_z=z, **S)
         check_case(oracle, d, seed=70 + f, tag="dw rows")

@@ -4,6 +4,7 @@ import pytest
 
 from megengine_amd import _abi, ops
 from tests.gpu_util import check_case
+from tests.routes import routes
 
 pytestmark = pytest.mark.gpu
 
@@ -40,7 +41,7 @@ def test_depthwise_matrix(oracle, i):
                                 dst_stride_n=do + 8, z_stride_n=do + 12 if "has_z" in kw else 0, **kw, **S)
         for desc in (d0, d):
             a, _ = ops.conv_bias_query(desc)
-            assert a.id == DW
+            assert a.id == DW and routes([desc])[0].kernels[0].startswith("dwm_kernel")
             check_case(oracle, desc, seed=50 + i, tag="dw matrix %d" % i)
     # scales outside the range of the divide-free epilogue
     d = _abi.make_conv_desc("NCHW4", n, c, ih, iw, c, fh, fw, group=c, pad=pad, stride=stride, nonline="RELU", has_z=True,

@@ -1,6 +1,7 @@
 """Plain NCHW through packed inputs and the planar epilogue at its edges: channel counts on both sides of the packing switch,
 planes around the 64 and 128 pixels of a conversion tile, output planes that are no multiple of 4 (groups of four pixels
-that straddle two images), odd channel counts, group boundaries inside a channel tile, misaligned tensors."""
+that straddle two images), odd channel counts, group boundaries inside a channel tile, misaligned tensors.  Most square filters run
+in one launch without packing (test_gpu_nchw_patch.py); the sizes that do are here again with filters that are packed."""
 import numpy as np
 import pytest
 import torch
@@ -8,6 +9,7 @@ import torch
 from megengine_amd import _abi, lib, ops
 from tests import util
 from tests.gpu_util import check_case
+from tests.routes import routes
 
 pytestmark = pytest.mark.gpu
 
@@ -26,7 +28,14 @@ CASES = [
     (6, 40, 57, 45, 140, 3, 1, 1, 1),
     (2, 192, 9, 9, 128, 3, 1, 1, 2),
     (3, 64, 11, 11, 192, 5, 2, 1, 2),     # 96 channels per group: a tile of 64 ends inside one
+    (3, 3, 9, 7, 5, (3, 2), 1, 1, 1),
+    (2, 16, 8, 8, 33, (3, 2), (1, 0), 1, 1),
+    (2, 17, 7, 9, 31, (2, 3), 1, 2, 1),
+    (3, 40, 8, 8, 96, (1, 2), 0, 1, 1),
+    (40, 48, 13, 13, 66, (3, 1), (1, 0), 1, 1),
+    (6, 40, 57, 45, 140, (1, 3), (0, 1), 1, 1),
 ]
+ONE_LAUNCH = (1, 2, 3, 4, 7, 8)
 
 
 @pytest.mark.parametrize("i", range(len(CASES)))
@@ -35,6 +44,7 @@ def test_edges(oracle, i):
     fh, fw = f if isinstance(f, tuple) else (f, f)
     for nl, kw in (("RELU", dict(has_z=True)), ("IDENTITY", dict()), ("H_SWISH", dict(has_z=True, bias_mode=_abi.BIAS_NONE))):
         d = _abi.make_conv_desc("NCHW", n, ic, ih, iw, oc, fh, fw, pad=pad, stride=stride, group=group, nonline=nl, **kw, **S)
+        assert (routes([(d, NCHW, -1, True)])[0].kernels[0] == "nchw_prep_kernel") == (i not in ONE_LAUNCH)
         check_case(oracle, d, seed=30 + i, algo=NCHW, tag="nchw planar %d" % i)
 
 
@@ -42,6 +52,7 @@ def test_edges(oracle, i):
 @pytest.mark.parametrize("n,ic,oc", [(2, 12, 45), (2, 75, 70), (24, 40, 66)])   # packed by 4, by 32; pixels for the tiled kernel
 def test_filters_that_are_not_square(oracle, n, ic, oc, fh, fw):
     d = _abi.make_conv_desc("NCHW", n, ic, 21, 23, oc, fh, fw, pad=(fh // 2, fw // 2), stride=(1, 2), nonline="RELU", has_z=True, **S)
+    assert routes([(d, NCHW, -1, True)])[0].kernels[0] == "nchw_prep_kernel"
     check_case(oracle, d, seed=fh * fw + n, algo=NCHW, tag="nchw planar %dx%d" % (fh, fw))
 
 

@@ -7,6 +7,7 @@ import torch
 from megengine_amd import _abi, lib, ops
 from tests import util
 from tests.gpu_util import check_case, run_gpu, say, to_dev
+from tests.routes import routes
 
 pytestmark = pytest.mark.gpu
 
@@ -497,19 +498,27 @@ NCHW_MFMA_CASES = [
     dict(n=2, ic=20, ih=19, iw=23, oc=36, fh=5, fw=3, pad=(2, 1), stride=(2, 1)),
     dict(n=2, ic=64, ih=16, iw=16, oc=128, fh=3, pad=1, group=2),           # groups of whole 32-channel blocks
     dict(n=1, ic=100, ih=30, iw=30, oc=7, fh=3),
+    # the second to fourth, which run in one launch (conv_patch1.hip), again with filters that it does not take: packed by 4, whole blocks
+    # without the vector path, and with it
+    dict(n=16, ic=3, ih=57, iw=49, oc=5, fh=3, fw=5, pad=(1, 2)),
+    dict(n=3, ic=64, ih=14, iw=14, oc=128, fh=2, fw=1, pad=(1, 0)),
+    dict(n=2, ic=32, ih=32, iw=32, oc=64, fh=3, fw=5, pad=(1, 2), stride=2),
 ]
+NCHW_ONE_LAUNCH = (1, 2, 3)
 
 
 @pytest.mark.parametrize("i", range(len(NCHW_MFMA_CASES)))
 def test_plain_nchw_on_the_mfma_kernel(oracle, i):
-    """Format::NCHW through relayout -> NCHW32 MFMA kernel -> relayout in the caller's workspace, against the checker's
-    NCHW path, every activation, with and without a residual; the generic kernel must give the same tensor."""
+    """Format::NCHW packed into the caller's workspace and convolved by an MFMA kernel with a planar epilogue, or in one launch without
+    the packing, against the checker's NCHW path, every activation, with and without a residual; the generic kernel must give the
+    same tensor."""
     c = NCHW_MFMA_CASES[i]
     nchw = lib.algo_names().index("MI355_NCHW_RELAYOUT_MFMA_I8")
     for nl, has_z in (("RELU", True), ("IDENTITY", False), ("H_SWISH", True)):
         d = mk(dict(c, fmt="NCHW"), nonline=nl, has_z=has_z, **S)
         a, ws = ops.conv_bias_query(d)
         assert a.id == nchw and ws > 0, (i, a.id, ws)
+        assert (routes([d])[0].kernels[0] == "nchw_prep_kernel") == (i not in NCHW_ONE_LAUNCH)
         want = check_case(oracle, d, seed=1200 + i, algo=nchw, tag="nchw-mfma %d" % i)
         check_case(oracle, d, seed=1200 + i, algo=DIRECT, tag="nchw-direct %d" % i)
         assert want is not None

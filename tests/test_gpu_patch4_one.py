@@ -4,6 +4,7 @@ import pytest
 
 from megengine_amd import _abi, lib
 from tests.gpu_util import check_case
+from tests.routes import routes
 
 pytestmark = pytest.mark.gpu
 
@@ -31,4 +32,5 @@ def test_one_stage(oracle, i):
                                  dst_stride_n=do + 4, z_stride_n=do + 12 if "has_z" in kw else 0, **kw, **S)
         for d in (d0, d1):
             for t in [k for k, name in enumerate(lib.tile_names()) if name.startswith("patch4_")]:
+                assert routes([(d, 1, t, False)])[0].kernels[0].startswith("patch4_one_kernel<%d," % (1 if ic <= 32 else 2))
                 assert check_case(oracle, d, seed=60 + i, algo=1, tile=t, tag=lib.tile_names()[t]) is not None

@@ -10,6 +10,7 @@ import torch
 
 from megengine_amd import _abi, lib, ops
 from tests import util
+from tests.routes import routes
 
 pytestmark = pytest.mark.gpu
 
@@ -27,21 +28,27 @@ def _case(d, seed):
     return [None if x is None else torch.from_numpy(x).cuda() for x in (src, flt, bias, z)]
 
 
-def test_static_workspace_exec_matches_exec_two_calls_in_a_row():
+@pytest.mark.parametrize("fh,fw,packs", [(5, 3, True), (3, 3, False)])
+def test_static_workspace_exec_matches_exec_two_calls_in_a_row(fh, fw, packs):
     """Two calls in a row on the one array, the second with a smaller input (its tensors cover only the front of what
     the first call left behind), then the first again: each must equal mi355_convbias_s8_exec with a workspace of the
-    caller's, bit for bit, for the algorithm that needs the workspace (plain NCHW through relayout + MFMA)."""
+    caller's, bit for bit, for the algorithm that needs the workspace (plain NCHW, packed ahead of the MFMA kernel).  The smaller
+    layer is packed too, or one that runs in a single launch and touches no workspace."""
     nchw = lib.algo_names().index("MI355_NCHW_RELAYOUT_MFMA_I8")
     big = _abi.make_conv_desc("NCHW", 4, 24, 28, 28, 40, 3, pad=1, nonline="RELU", has_z=True, **S)
-    small = _abi.make_conv_desc("NCHW", 2, 20, 19, 23, 36, 3, pad=1, nonline="H_SWISH", has_z=True, **S)
+    small = _abi.make_conv_desc("NCHW", 2, 20, 19, 23, 36, fh, fw, pad=(fh // 2, fw // 2), nonline="H_SWISH", has_z=True, **S)
+    written = {id(big): True, id(small): packs}
+    assert [r.kernels[0] == "nchw_prep_kernel" for r in routes([(d, nchw, -1, True) for d in (big, small)])] == [True, packs]
     assert lib.lib().mi355_static_workspace_bytes() == 32 << 20
     plans = []
     for d, seed in ((big, 5), (small, 6)):
         algo, ws = ops.conv_bias_query(d, nchw)
         assert algo.id == nchw and 0 < ws <= lib.lib().mi355_static_workspace_bytes()
         t = _case(d, seed)
-        want = ops.conv_bias_exec(d, *t, algo=algo, workspace=torch.empty(ws, dtype=torch.uint8, device="cuda"))
+        room = torch.full((ws,), 113, dtype=torch.uint8, device="cuda")
+        want = ops.conv_bias_exec(d, *t, algo=algo, workspace=room)
         torch.cuda.synchronize()
+        assert bool((room != 113).any()) == written[id(d)]
         plans.append((d, algo, t, want))
     for d, algo, t, want in (plans[0], plans[1], plans[0]):
         got = torch.full_like(want, 77)
