@@ -806,7 +806,7 @@ static int exec_impl(void* stream, const mi355_conv_desc* d, const mi355_algo* a
             rc = launch_conv_igemm(hs, p, cfg, cu_count(), src, filter, bias, z, reinterpret_cast<int8_t*>(dst), preprocessed);
             break;
         case ALGO_DEPTHWISE:
-            rc = launch_conv_depthwise(hs, p, src, filter, bias, z, reinterpret_cast<int8_t*>(dst));
+            rc = launch_conv_depthwise(hs, p, cu_count(), src, filter, bias, z, reinterpret_cast<int8_t*>(dst));
             break;
         case ALGO_C4_MFMA:
             rc = launch_conv_c4(hs, p, cu_count(), src, filter, bias, z, reinterpret_cast<int8_t*>(dst));

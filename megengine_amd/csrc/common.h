@@ -67,9 +67,14 @@ int launch_igemm_preprocess(hipStream_t st, const ConvProblem& p, const int8_t* 
 
 bool depthwise_usable(const ConvProblem& p);
 bool dwm_usable(const ConvProblem& p);
+struct DwmBands {
+    int PW, PH, TH, bands;  // patch columns and rows of a band, its output rows, bands of a plane
+    int rpw, waves;         // patch rows of one copy instruction, waves of a workgroup
+};
+DwmBands dwm_bands(const ConvProblem& p);
 int launch_dwm(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                int8_t* dst);
-int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt,
+int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt,
                           const int32_t* bias, const int8_t* z, int8_t* dst);
 
 bool c4_usable(const ConvProblem& p);

@@ -550,7 +550,34 @@ bool depthwise_usable(const ConvProblem& p) {
     return true;
 }
 
-int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt,
+// 5x5 with its own padding: whether the matrix form (conv_dwm.hip) or dwf_kernel is ahead, by what each takes on a device of 256 CUs.
+// The prices, in us, are fitted to graph replays of both on 4800 layers of 4 to 1200 channels, planes of 4 x 4 to 128 x 128, batch 1 to
+// 128.  The matrix form: its launch, the chain of a workgroup -- copies of the patch, which a row of just over 64 columns takes two of,
+// and units of results --, one per round of workgroups over the CUs, and what a CU has to do in all.  dwf: its launch, and the waves of
+// one and two rows per thread.  Always the matrix form: 606 of 6000 layers more than 3 % slower than dwf (163 more than 10 %, up to
+// 1.30), most of them between one and two workgroups to a CU or with rows of 65 to 100 columns at stride 2.  By prices 52 of the 4800
+// (2, at most 1.16); on 1317 other layers 18 (1), where it was 185 (56), and 0.92 of dwf's time on average, 0.93 before.
+static bool dw5_matrix(const ConvProblem& p, int QW, int rows_per_thread, int cu_count) {
+    struct Price {
+        float launch, copy, unit, round, cu_copy, cu_unit, vec_launch, vec_rows, vec_wave, vec_round;
+    };
+    static const Price prices[2] = {{2.370f, 0.076f, 0.318f, 0.273f, 0.007f, 0.033f, 1.594f, 1.037f, 0.157f, 1.024f},
+                                    {2.745f, 0.061f, 0.000f, 0.257f, 0.005f, 0.049f, 1.943f, 0.850f, 0.248f, 1.021f}};
+    const Price& c = prices[p.d.stride_h - 1];
+    const DwmBands b = dwm_bands(p);
+    const int per_copy = b.waves * b.rpw, per_unit = b.waves * 32;
+    const int copies = (b.PH + per_copy - 1) / per_copy * ((b.PW + 63) / 64), units = (b.TH * QW + per_unit - 1) / per_unit;
+    const uint32_t planes = p.d.n * (p.d.ic / 4), cu = (uint32_t)cu_count, wgs = planes * (uint32_t)b.bands, R = (uint32_t)rows_per_thread;
+    const float share = (float)wgs / (float)cu, in_cu = share * (float)b.waves;
+    const uint64_t waves = ((uint64_t)planes * ((p.oh + R - 1) / R) * (uint32_t)QW + 63) / 64;
+    const float matrix = c.launch + c.copy * copies + c.unit * units + c.round * (float)((wgs + cu - 1) / cu) +
+                         in_cu * (c.cu_copy * copies + c.cu_unit * units);
+    const float vector = c.vec_launch + c.vec_rows * (float)R + c.vec_wave * (float)R * ((float)waves / (float)cu) +
+                         c.vec_round * (float)((waves + 4 * cu - 1) / (4 * cu));
+    return matrix <= vector;
+}
+
+int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt,
                           const int32_t* bias, const int8_t* z, int8_t* dst) {
     const mi355_conv_desc& d = p.d;
     DwArgs a;
@@ -568,15 +595,20 @@ int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, const int8_t* sr
     //   5x5 and 7x7 "same", against dwf_kernel: 560 channels, 5x5 at 30 x 55, batch 14: 14.3 / 20.1; 240, 5x5 stride 2 at 57 x 57,
     //     batch 16: 8.4 / 9.4; 136, 7x7 at 42 x 37, batch 7: 6.1 / 7.8; 68, 5x5 stride 2 at 24 x 10, batch 3: 3.6 / 4.3.  Its workgroups
     //     set themselves up for one plane each, so many small planes stay behind: 740, 5x5 stride 2 at 10 x 14, batch 16 (10 quads a
-    //     plane): 5.7 / 4.8; 604 at 14 x 78, batch 17 (70 quads): 10 / 8.2; from about 100 quads it is ahead at any number of planes.
+    //     plane): 5.7 / 4.8; 604 at 14 x 78, batch 17 (70 quads): 10 / 8.2; from about 100 quads 7x7 is ahead at any number of planes
+    //     (708 layers, 10 of them more than 3 % behind, the worst 1.13), 5x5 by the prices of dw5_matrix.
     //   other filters, against dw4_kernel: 4x4 at 35 x 38, 112 channels, batch 45: 8.8 / 29.9; 6x6 at 101 x 14, 256, batch 1: 4.2 / 12.8;
     //     2x2 at 71 x 26, 108, batch 63: 12.6 / 15.7.  At strides of 3 and 4 a filter of few taps leaves most of the patch unused: 7x1,
     //     stride 3, 448 at 44 x 82, batch 2: 6.3 / 5.6.
     const bool small_planes = (int64_t)d.n * a.CG >= 512 && (int64_t)a.OH * a.QW < 100;
+    // (output rows per thread of the vector forms, see below)
+    const int64_t rows = (int64_t)d.n * a.CG * a.OH * a.QW;
+    const bool few = rows <= (a.OH % 2 && a.OH <= 7 ? 262144 : 131072);
     const bool matrix = wide ? !small_planes : !(sq && d.fh == 3) && (d.stride_w <= 2 || d.fh * d.fw >= 9);
-    if (matrix && dwm_usable(p)) return launch_dwm(st, p, src, flt, bias, z, dst);
     const int64_t src_total = (int64_t)(d.n - 1) * p.src_sn + (int64_t)d.ic * d.ih * d.iw;
-    if (sq && (d.fh == 3 || (wide && src_total < ((int64_t)1 << 31)))) {
+    const bool dwf = wide && src_total < ((int64_t)1 << 31);
+    if (matrix && dwm_usable(p) && (!dwf || d.fh == 7 || dw5_matrix(p, a.QW, few ? 1 : 2, cu_count))) return launch_dwm(st, p, src, flt, bias, z, dst);
+    if (sq && (d.fh == 3 || dwf)) {
         // Output rows per thread.  Few work items: one, because a thread's own chain -- its rows' loads, products and stores -- is
         // all there is to wait for; at stride 2 always, where rows share little.  With enough threads to fill the device two
         // rows at stride 1 read a third less, and four a sixth less again once there are a million rows of four pixels.
@@ -584,8 +616,6 @@ int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, const int8_t* sr
         // 4.0 / 4.1 / 4.1, batch 64: 8.5 / 7.2 / 7.8; 144 at 56 x 56, batch 64: 19.9 / 15.4 / 14.4; stride 2, 192 at 28 x 28,
         // batch 64: 4.2 / 4.8, 96 at 112 x 112: 16.6 / 16.4.  Planes of few, odd rows leave strips of two half empty: 960 at
         // 7 x 7, batch 64 (215040): 4.6 / 5.1.
-        const int64_t rows = (int64_t)d.n * a.CG * a.OH * a.QW;
-        const bool few = rows <= (a.OH % 2 && a.OH <= 7 ? 262144 : 131072);
         const int R = few || (!wide && d.stride_h == 2) ? 1 : !wide && p.oh % 4 == 0 && rows >= 1000000 ? 4 : 2;
         Dw3Args b;
         b.src = src; b.flt = flt; b.bias = bias; b.z = z; b.dst = dst;

@@ -193,6 +193,23 @@ bool dwm_usable(const ConvProblem& p) {
 }
 
 // Bands: as much of the patch as 16 KiB hold, so that eight workgroups share a CU; fewer rows where that leaves CUs without one.
+DwmBands dwm_bands(const ConvProblem& p) {
+    const mi355_conv_desc& d = p.d;
+    const int QW = ((int)p.ow + 3) / 4, FH = d.fh, sh = d.stride_h;
+    DwmBands b;
+    b.PW = dwm_columns(p);
+    const int64_t most = (4096 / b.PW - FH) / sh + 1;
+    b.TH = most < 1 ? 1 : most < (int64_t)p.oh ? (int)most : (int)p.oh;
+    while (b.TH > 1 && b.TH * QW > 64 && (int64_t)d.n * (d.ic / 4) * ((p.oh + b.TH - 1) / b.TH) < 256) b.TH = (b.TH + 1) / 2;
+    b.bands = ((int)p.oh + b.TH - 1) / b.TH;
+    b.TH = ((int)p.oh + b.bands - 1) / b.bands;  // even bands
+    b.PH = (b.TH - 1) * sh + FH;
+    b.rpw = b.PW < 64 ? 64 / b.PW : 1;
+    const int units = (b.TH * QW + 15) / 16;
+    b.waves = units > 4 ? 4 : units > 2 ? 2 : 1;
+    return b;
+}
+
 int launch_dwm(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                int8_t* dst) {
     const mi355_conv_desc& d = p.d;
@@ -200,18 +217,12 @@ int launch_dwm(hipStream_t st, const ConvProblem& p, const int8_t* src, const in
     a.src = src; a.flt = flt; a.bias = bias; a.z = z; a.dst = dst;
     a.IH = d.ih; a.IW = d.iw; a.OH = p.oh; a.OW = p.ow; a.FH = d.fh; a.FW = d.fw; a.sh = d.stride_h; a.sw = d.stride_w;
     a.ph = d.pad_h; a.pw = d.pad_w;
-    a.NB = dwm_blocks(p); a.PW = dwm_columns(p); a.part = a.PW / 4 / a.sw;
+    const DwmBands b = dwm_bands(p);
+    a.NB = dwm_blocks(p); a.PW = b.PW; a.part = a.PW / 4 / a.sw;
     a.CG = d.ic / 4; a.taps = d.fh * d.fw; a.QW = ((int)p.ow + 3) / 4;
     a.has_bias = d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL;
-    const int64_t most = (4096 / a.PW - a.FH) / a.sh + 1;
-    a.TH = most < 1 ? 1 : most < (int64_t)p.oh ? (int)most : (int)p.oh;
-    while (a.TH > 1 && a.TH * a.QW > 64 && (int64_t)d.n * a.CG * ((p.oh + a.TH - 1) / a.TH) < 256) a.TH = (a.TH + 1) / 2;
-    a.bands = ((int)p.oh + a.TH - 1) / a.TH;
-    a.TH = ((int)p.oh + a.bands - 1) / a.bands;  // even bands
-    a.PH = (a.TH - 1) * a.sh + a.FH;
-    a.rpw = a.PW < 64 ? 64 / a.PW : 1;
-    const int units = (a.TH * a.QW + 15) / 16, steps = (a.FH * a.NB + 3) / 4;
-    a.waves = units > 4 ? 4 : units > 2 ? 2 : 1;
+    a.TH = b.TH; a.bands = b.bands; a.PH = b.PH; a.rpw = b.rpw; a.waves = b.waves;
+    const int steps = (a.FH * a.NB + 3) / 4;
     a.tab_w = a.NB * 4 + 3 * a.sw;
     a.tab = (((steps * 4 - 1) / a.NB + 1) * a.tab_w + 63) / 64 * 64;
     a.tab_at = a.PH * a.PW + a.NB * 4;  // the window of a row's last quad may end past its columns

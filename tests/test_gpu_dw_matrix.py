@@ -27,7 +27,10 @@ CASES = [
     (1, 4, 40, 33, 8, 4, 9, 1),              # padding wider than the filter
     (1, 8, 21, 26, 3, 3, 1, (3, 3)),
     (1, 8, 25, 40, 3, 5, 1, (4, 4)),
+    (1, 8, 29, 31, 5, 5, (1, 2), (1, 2)),    # the third and the seventh again, as the matrix form takes them
+    (1, 4, 3, 1000, 5, 5, (2, 3), 1),
 ]
+VECTOR = (2, 6)  # dwf_kernel is ahead there, at its price
 
 
 @pytest.mark.parametrize("i", range(len(CASES)))
@@ -41,7 +44,7 @@ def test_depthwise_matrix(oracle, i):
                                 dst_stride_n=do + 8, z_stride_n=do + 12 if "has_z" in kw else 0, **kw, **S)
         for desc in (d0, d):
             a, _ = ops.conv_bias_query(desc)
-            assert a.id == DW and routes([desc])[0].kernels[0].startswith("dwm_kernel")
+            assert a.id == DW and routes([desc])[0].kernels[0].startswith("dwf_kernel" if i in VECTOR else "dwm_kernel")
             check_case(oracle, desc, seed=50 + i, tag="dw matrix %d" % i)
     # scales outside the range of the divide-free epilogue
     d = _abi.make_conv_desc("NCHW4", n, c, ih, iw, c, fh, fw, group=c, pad=pad, stride=stride, nonline="RELU", has_z=True,

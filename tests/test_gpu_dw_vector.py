@@ -1,5 +1,5 @@
 """The vector forms of channel-wise convolution where the matrix form (test_gpu_dw_matrix.py) leaves layers to them: dwf_kernel for many
-small planes of 5x5 and 7x7, one and two output rows per thread, and dw4_kernel for wide strides of few taps, large windows and rows whose
+small planes of 5x5 and 7x7 and where its price is lower, one and two output rows per thread, and dw4_kernel for wide strides of few taps, large windows and rows whose
 patch does not fit.  Each case names the kernel that it is about."""
 import pytest
 
@@ -27,6 +27,8 @@ CASES = [
     (32, 264, 21, 13, 7, 7, 3, 1, "dwf_kernel<7, 1, 2>"),
     (32, 256, 45, 32, 7, 7, 3, 2, "dwf_kernel<7, 2, 2>"),
     (1, 8, 5, 1701, 5, 5, 2, 1, "dwf_kernel<5, 1, 1>"),        # no room for a row's patch
+    (7, 172, 18, 40, 5, 5, 2, 1, "dwf_kernel<5, 1, 1>"),       # by price: 301 workgroups of the matrix form on 256 CUs
+    (9, 48, 31, 143, 5, 5, 2, 2, "dwf_kernel<5, 2, 1>"),       # its patch is two copies wide
     (2, 12, 44, 41, 7, 1, (3, 0), 3, "dw4_kernel"),
     (2, 12, 23, 46, 2, 4, (1, 2), (1, 3), "dw4_kernel"),
     (2, 8, 31, 33, 5, 5, 2, 5, "dw4_kernel"),

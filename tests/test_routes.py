@@ -65,8 +65,8 @@ def test_plain_nchw_lines():
     assert _kernels([one(4, UNNAMED), one(5, UNNAMED), one(5, 0)]) == [("conv_direct_kernel",), k(1, 1, 1), ("conv_direct_kernel",)]
 
 
-def _dw(n, c, ih, iw, fh, fw, pad, stride):
-    return _abi.make_conv_desc("NCHW4", n, c, ih, iw, c, fh, fw, group=c, pad=pad, stride=stride, nonline="RELU", has_z=True, **S)
+def _dw(n, c, ih, iw, fh, fw, pad, stride, z=1):
+    return _abi.make_conv_desc("NCHW4", n, c, ih, iw, c, fh, fw, group=c, pad=pad, stride=stride, nonline="RELU", has_z=bool(z), **S)
 
 
 def test_channel_wise_lines():
@@ -76,7 +76,7 @@ def test_channel_wise_lines():
         (_dw(7, 292, 24, 16, 5, 5, 2, 1), "dwm_kernel<3, true>"), (_dw(8, 256, 24, 16, 5, 5, 2, 1), "dwf_kernel<5, 1, 1>"),
         (_dw(8, 256, 25, 16, 5, 5, 2, 1), "dwm_kernel<3, true>"), (_dw(8, 256, 50, 32, 7, 7, 3, 2), "dwm_kernel<7, true>"),
         (_dw(8, 256, 48, 32, 7, 7, 3, 2), "dwf_kernel<7, 2, 1>"), (_dw(32, 256, 24, 16, 5, 5, 2, 1), "dwf_kernel<5, 1, 2>"),
-        (_dw(1, 8, 5, 1632, 5, 5, 2, 1), "dwm_kernel<3, true>"), (_dw(1, 8, 5, 1633, 5, 5, 2, 1), "dwf_kernel<5, 1, 1>"),   # one row's patch
+        (_dw(1, 8, 7, 1162, 7, 7, 3, 1), "dwm_kernel<6, true>"), (_dw(1, 8, 7, 1163, 7, 7, 3, 1), "dwf_kernel<7, 1, 1>"),   # one row's patch
         # other filters: strides, taps, the window's blocks, one row's patch
         (_dw(1, 8, 24, 24, 7, 1, 0, 2), "dwm_kernel<4, true>"), (_dw(1, 8, 24, 24, 7, 1, 0, 3), "dw4_kernel"),
         (_dw(1, 8, 24, 24, 9, 1, 0, 3), "dwm_kernel<7, true>"), (_dw(1, 8, 24, 24, 5, 5, 2, 4), "dwm_kernel<7, true>"),
@@ -86,6 +86,48 @@ def test_channel_wise_lines():
     ]
     for got, (d, want) in zip(_kernels([d for d, _ in table]), table):
         assert got == (want,), (d.key(), got)
+
+
+# 5x5, pad 2: n, channels, ih, iw, stride, residual; us of dwf_kernel and of the matrix form, graph replays on 256 CUs.  Every ninth of the 125 (of
+# 1317 drawn) on which the matrix form is more than 5 % behind, and every fortieth of those on which it is more than 10 % ahead.
+CHANNEL_WISE = [
+    (4, 860, 85, 24, 2, 1, 6.3, 6.7),
+    (1, 704, 105, 64, 2, 1, 6.0, 6.6),
+    (10, 12, 33, 65, 1, 1, 4.0, 4.3),
+    (6, 100, 75, 85, 2, 1, 4.9, 5.9),
+    (5, 92, 55, 16, 2, 0, 3.9, 4.1),
+    (3, 156, 27, 99, 2, 1, 4.4, 4.7),
+    (9, 108, 41, 87, 2, 1, 4.7, 4.9),
+    (2, 132, 40, 71, 2, 1, 4.1, 4.8),
+    (12, 484, 84, 30, 2, 0, 8.7, 9.6),
+    (1, 340, 41, 69, 2, 1, 4.2, 5.0),
+    (1, 340, 105, 23, 1, 1, 4.4, 4.7),
+    (4, 72, 92, 21, 1, 0, 4.2, 4.6),
+    (6, 172, 33, 68, 2, 0, 4.2, 4.9),
+    (2, 388, 29, 77, 2, 0, 4.3, 4.6),
+    (9, 12, 11, 15, 1, 0, 3.5, 3.0),
+    (2, 12, 13, 58, 2, 1, 4.1, 3.7),
+    (62, 12, 16, 11, 1, 0, 3.7, 3.3),
+    (42, 96, 48, 107, 1, 1, 30.0, 22.9),
+    (8, 460, 11, 83, 1, 1, 8.2, 7.0),
+    (1, 60, 83, 12, 2, 0, 3.7, 3.2),
+    (15, 80, 36, 55, 1, 0, 7.1, 6.3),
+    (20, 664, 13, 103, 1, 0, 24.5, 15.0),
+    (7, 60, 15, 13, 2, 1, 4.2, 3.8),
+    (11, 48, 105, 86, 1, 0, 9.2, 7.3),
+    (1, 60, 7, 17, 2, 0, 3.8, 3.4),
+    (7, 68, 14, 28, 1, 0, 3.5, 3.1),
+]
+
+
+def test_channel_wise_5x5():
+    got = _kernels([_dw(n, c, ih, iw, 5, 5, 2, s, z) for n, c, ih, iw, s, z, _, _ in CHANNEL_WISE])
+    lost = []
+    for (k,), (*layer, dwf, dwm) in zip(got, CHANNEL_WISE):
+        assert k.startswith(("dwf_kernel<5", "dwm_kernel"))
+        lost.append((dwf if k.startswith("dwf") else dwm) / min(dwf, dwm) - 1)
+    # the prices leave 18 of the 1317 more than 3 % behind, at most 16 %
+    assert max(lost) <= 0.16 and sum(l > 0.03 for l in lost) <= 2, lost
 
 
 def test_one_stage_line():
