@@ -183,10 +183,11 @@ __global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
         const int c0 = (st * GS + g) * 16;
 #pragma unroll
         for (int k = 0; k < FI; ++k) {
-            // (a quad past the last channel, or whose bytes pass the end of the filter, is not loaded here, see store)
+            // (a quad past the last channel is not loaded; one whose bytes pass the end of the filter is loaded whole channels further
+            // left, and turned back in store)
             const int at = f_off[k] + st * GS * 16 * T;
-            const bool in = (f_off[k] >= 0) & (st * GS * 16 + f_quad * 4 < a.IC) & (at + 4 * T <= a.flt_bytes);
-            const int v0 = in ? at : SENT;
+            const bool in = (f_off[k] >= 0) & (st * GS * 16 + f_quad * 4 < a.IC);
+            const int v0 = in ? min(at, a.flt_bytes - 4 * T) : SENT;
 #pragma unroll
             for (int v = 0; v + 4 <= T; v += 4) {
                 const v4i y = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, v0 + 4 * v, 0, 0);
@@ -209,23 +210,17 @@ __global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
 #pragma unroll
         for (int k = 0; k < FI; ++k) {
             const int row = f_row + k * ROWS_PER_PASS, left = a.IC - (st * GS * 16 + f_quad * 4);  // channels from here on
-            uint32_t keep = left >= 4 ? 0xffffffffu : left > 0 ? (1u << (8 * left)) - 1 : 0u;
-            const int at = f_off[k] + st * GS * 16 * T;
-            if (f_off[k] < 0) keep = 0;
-            if (keep != 0 && at + 4 * T > a.flt_bytes) {  // the last quad of the last row
-#pragma unroll
-                for (int v = 0; v < T; ++v) {
-                    uint32_t w = 0;
-#pragma unroll
-                    for (int b = 0; b < 4; ++b)
-                        w |= (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rs_flt, 4 * v + b < left * T ? at + 4 * v + b : SENT, 0, 0) << (8 * b);
-                    xf[k][v] = w;
-                }
-            }
+            // Channels that exist, and the quads at the filter's end, which may be those of its last three rows: loaded one to three
+            // channels further left.  One selector does both.  (Loading such a quad byte by byte, 4 T loads of one lane, held up the last
+            // channel tile: 5x5 59 -> 63 at 79 x 22, batch 4: 13.3 us.)
+            const int over = f_off[k] + st * GS * 16 * T + 4 * T - a.flt_bytes;
+            const int turned = over <= 0 ? 0 : over <= T ? 1 : over <= 2 * T ? 2 : 3;
+            const uint32_t there = left >= 4 ? 0xffffffffu : left > 0 ? (1u << (8 * left)) - 1 : 0u;
+            const uint32_t keep = ((0x03020100u + 0x01010101u * (uint32_t)turned) & there) | (0x0c0c0c0cu & ~there);
             if (BM * QPR >= 256 || row < BM)
 #pragma unroll
                 for (int tap = 0; tap < T; ++tap)
-                    sw[(((f_quad >> 2) * T + tap) * BMP + row) * 4 + (f_quad & 3)] = p1_tap<T>(xf[k], tap) & keep;
+                    sw[(((f_quad >> 2) * T + tap) * BMP + row) * 4 + (f_quad & 3)] = __builtin_amdgcn_perm(0u, p1_tap<T>(xf[k], tap), keep);
         }
 #pragma unroll
         for (int k = 0; k < NPI; ++k) {

@@ -37,6 +37,11 @@ CASES = [
     (14, 13, 71, 73, 70, 1, 0, 2, (2, 1)),
     (14, 3, 57, 59, 190, 5, 2, 1, (2, 2)),
     (12, 5, 67, 65, 70, 5, 2, 2, (2, 1)),
+    (2, 1, 6, 5, 5, 5, 2, 1, (1, 1)),        # filters that end inside the quads of their last three rows, and of the last row alone
+    (1, 2, 5, 7, 2, 3, 1, 1, (1, 1)),
+    (1, 3, 6, 9, 33, 5, 2, 2, (1, 1)),
+    (1, 18, 9, 9, 65, 3, 1, 1, (1, 1)),
+    (1, 35, 9, 9, 34, 1, 0, 1, (1, 1)),
 ]
 
 
