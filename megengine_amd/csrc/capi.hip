@@ -797,7 +797,7 @@ static int exec_impl(void* stream, const mi355_conv_desc* d, const mi355_algo* a
             // over 6 channels, 101 x 7 pixels: 5.1 us / 4.6; 3x3 over 256, 6 x 6: 617 / 15).  Named by the caller it runs as itself.
             const bool planar = by_heuristic && d->format == MI355_FMT_NCHW && p.icpg * d->fh * d->fw >= 5 &&
                                 (reinterpret_cast<uintptr_t>(bias) & 3) == 0;
-            const int tile = planar ? patch1_pick(p, false) : -1;
+            const int tile = planar ? patch1_pick(p, false, cu_count()) : -1;
             rc = tile >= 0 ? launch_patch1(hs, p, tile, src, filter, bias, z, reinterpret_cast<int8_t*>(dst))
                            : launch_conv_direct(hs, p, src, filter, bias, z, dst);
             break;

@@ -89,7 +89,7 @@ size_t nchw_mfma_workspace_used(const ConvProblem& p);
 // plain NCHW in one launch without a workspace (conv_patch1.hip): the tile, or -1 where it cannot run or is not ahead
 bool patch1_usable(const ConvProblem& p);
 // (packed: the caller could run the packed path instead)
-int patch1_pick(const ConvProblem& p, bool packed);
+int patch1_pick(const ConvProblem& p, bool packed, int cu_count);
 int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                   int8_t* dst);
 int launch_conv_nchw_mfma(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt,

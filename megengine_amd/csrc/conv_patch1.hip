@@ -459,9 +459,8 @@ bool patch1_usable(const ConvProblem& p) {
 // ahead on filters of 1x1 and 3x3 (23 layers, this kernel over the packed path: 0.84 to 1.83, 1.19 on average; 3x3 6 -> 194 at 59 x 107,
 // batch 57: 51.4 / 28.1; 1x1 7 -> 197 at 89 x 27, batch 51: 19.6 / 13.9).  Not with a residual (1.00 on 10 layers), not where rows out
 // are whole quads (0.95 on 5), not with 25 taps (1.0 on 4), whose products outweigh the turning.
-int patch1_pick(const ConvProblem& p, bool packed) {
-    if (!patch1_usable(p)) return -1;
-    P1Args k;
+//   5x5 with two and more stages at strides of 1 and 2, against the packed path: by what each takes, see p1_behind_packed.
+static int p1_tile(const ConvProblem& p, bool packed, P1Args& k) {
     int lds;
     auto wgs = [&](int tile) { return p1_plan(p, tile, &k, &lds) ? (int64_t)k.tiles_n * k.tiles_m : (int64_t)-1; };
     const int64_t w0 = wgs(0);
@@ -477,6 +476,46 @@ int patch1_pick(const ConvProblem& p, bool packed) {
     }
     if (p.d.oc > 32 && wgs(2) >= 512) return 2;
     return wgs(1) > 0 ? 1 : 0;
+}
+
+// 5x5 in two and more stages: whether the packed path is ahead of this kernel on its tile, by prices on a device of 256 CUs in us and, of
+// reductions, us per stage or per 1024 packed bytes.  This kernel walks its stages one after the other, so workgroups that begin another
+// round over the device -- of one or two to a CU -- cost a whole chain more; the packed path splits few tiles' reductions and deals
+// many tiles out smoothly.  Fitted to graph replays of 2397 layers over 17 to 256 channels on both; of these 213 were more than 3 %
+// behind the packed path and 117 more than 10 % (5x5 209 -> 33 at 26 x 7, batch 38: 24.2 / 13.3; 183 -> 164 at 41 x 85, batch 5:
+// 56.4 / 36.8); with the prices 40 and 12.  On 591 others 70 and 44 before, 9 and 1 now, 0.70 and 0.69 of the packed path on average.
+static bool p1_behind_packed(const ConvProblem& p, int tile, const P1Args& k, int cu_count) {
+    struct One {
+        float launch, stage, round2_stage, round_stage, share;
+    };
+    static const One one[4] = {{2.907f, 0.716f, 0.178f, 0.457f, 0.981f},   // 32 x 128
+                               {3.431f, 0.046f, 1.065f, 0.460f, 1.673f},   // 32 x 256
+                               {5.295f, 0.710f, 0.615f, 1.079f, 2.326f},   // 64 x 256
+                               {2.954f, 0.303f, 1.051f, 0.647f, 1.806f}};  // 64 x 128
+    struct Packed {
+        float launch, k, round_k, share_k, share, strided_k, round2_k;
+    };
+    static const Packed packed[2] = {{5.747f, 1.533f, 0.000f, 3.430f, 0.000f, 1.973f, 0.000f},   // tiles of 64 x 128 for a quarter of the CUs
+                                     {7.846f, 0.155f, 1.474f, 0.277f, 1.204f, 2.086f, 1.357f}};
+    const uint32_t cu = (uint32_t)cu_count, wgs = (uint32_t)k.tiles_n * (uint32_t)k.tiles_m, r1 = (wgs + cu - 1) / cu;
+    const One& a = one[tile];
+    const float this_us = a.launch + (float)k.nstages * (a.stage + a.round2_stage * (float)((r1 + 1) / 2) + a.round_stage * (float)r1) +
+                          a.share * ((float)wgs / (float)cu);
+    const uint64_t px = (uint64_t)p.d.n * p.oh * p.ow, tiles = (px + 127) / 128 * ((p.d.oc + 63) / 64), rounds = (tiles + cu - 1) / cu;
+    const float share = (float)tiles / (float)cu, kb = (float)((p.d.ic + 31) / 32 * 32 * 25) / 1024.0f;
+    const Packed& b = packed[share > 0.25f];
+    const float packed_us = b.launch + b.share * share + kb * (b.k + b.round_k * (float)rounds + b.share_k * share + b.round2_k * (float)((rounds + 1) / 2) +
+                                                               (p.d.stride_h * p.d.stride_w > 1 ? b.strided_k * share : 0.0f));
+    return this_us > 0.97f * packed_us;
+}
+
+int patch1_pick(const ConvProblem& p, bool packed, int cu_count) {
+    if (!patch1_usable(p)) return -1;
+    P1Args k;
+    const int tile = p1_tile(p, packed, k);
+    if (tile < 0 || !packed || p.d.fh != 5 || p.d.ic <= 16 || p.d.stride_h > 2 || p.d.stride_w > 2) return tile;
+    int lds;
+    return p1_plan(p, tile, &k, &lds) && p1_behind_packed(p, tile, k, cu_count) ? -1 : tile;
 }
 
 int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,

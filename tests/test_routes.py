@@ -36,6 +36,55 @@ def test_plain_nchw_strides():
         assert (packed if r.launches == 2 else one) <= 1.05 * min(packed, one), layer
 
 
+def _lost(layers):
+    """what the way taken costs over the faster one"""
+    out = []
+    for r, (*_, packed, one) in zip(routes([_nchw(*layer[:8]) for layer in layers]), layers):
+        assert r.launches in (1, 2)
+        out.append((packed if r.launches == 2 else one) / min(packed, one) - 1)
+    return out
+
+
+# 5x5 over 17 and more channels, the same columns: of 2397 drawn layers every 16th that is more than 5 % behind in one launch and every 120th that
+# is more than 10 % ahead
+PLAIN_5X5 = [
+    (55, 131, 21, 50, 85, 5, 2, 1, 31.5, 36.2),
+    (26, 47, 34, 51, 252, 5, 2, 1, 22.8, 25.9),
+    (41, 49, 66, 14, 73, 5, 1, 1, 23.8, 25.2),
+    (12, 57, 80, 66, 51, 5, 1, 1, 18.6, 23.9),
+    (26, 66, 50, 10, 111, 5, 1, 1, 16.8, 17.8),
+    (28, 249, 67, 40, 37, 5, 1, 0, 62.9, 66.9),
+    (61, 82, 8, 38, 220, 5, 1, 0, 26.0, 31.3),
+    (30, 193, 12, 18, 169, 5, 2, 0, 20.6, 22.9),
+    (32, 98, 25, 9, 37, 5, 1, 1, 11.4, 13.9),
+    (52, 93, 11, 49, 243, 5, 2, 1, 20.9, 25.8),
+    (3, 211, 20, 72, 238, 5, 1, 0, 24.1, 27.4),
+    (23, 182, 28, 11, 52, 5, 1, 0, 15.1, 20.0),
+    (13, 122, 8, 62, 84, 5, 1, 0, 18.2, 15.0),
+    (12, 25, 14, 87, 132, 5, 1, 1, 15.8, 12.4),
+    (11, 124, 52, 11, 66, 5, 1, 0, 18.0, 13.1),
+    (20, 23, 50, 28, 24, 5, 1, 1, 11.6, 7.3),
+    (9, 69, 19, 82, 119, 5, 1, 0, 17.1, 13.5),
+    (51, 19, 29, 13, 8, 5, 1, 1, 11.6, 6.8),
+    (13, 198, 25, 48, 6, 5, 1, 1, 22.9, 19.3),
+    (2, 83, 25, 63, 143, 5, 1, 0, 15.9, 12.5),
+    (60, 26, 36, 11, 125, 5, 1, 1, 15.1, 12.2),
+    (27, 75, 7, 37, 94, 5, 1, 1, 17.9, 15.3),
+    (8, 50, 33, 102, 15, 5, 1, 0, 14.1, 10.4),
+    (24, 19, 96, 11, 6, 5, 1, 1, 9.9, 6.8),
+    (31, 156, 87, 103, 5, 5, 2, 0, 56.7, 27.5),
+    (1, 48, 81, 43, 171, 5, 1, 0, 12.9, 7.6),
+    (20, 58, 28, 26, 37, 5, 1, 0, 12.1, 10.3),
+    (51, 35, 12, 47, 4, 5, 1, 0, 12.3, 8.2),
+]
+
+
+def test_plain_nchw_5x5():
+    lost = _lost(PLAIN_5X5)
+    # always in one launch 12 of these 28 are more than 3 % behind, by up to 32 %
+    assert sum(l > 0.03 for l in lost) <= 3 and max(lost) <= 0.2, lost
+
+
 def _kernels(execs):
     return [r.kernels for r in routes(execs)]
 
@@ -43,7 +92,7 @@ def _kernels(execs):
 def test_plain_nchw_lines():
     """Both sides of every line of patch1_pick, with a workspace; planes out of 8 x 16 are one tile of 128 pixels, 32 channels out one of 32"""
     plane = lambda n, ic, oc, f, stride=1: _nchw(n, ic, 8 * stride, 16 * stride, oc, f, stride)  # noqa: E731
-    k = lambda mt, nt, taps: ("patch1_kernel<%d, %d, %d>" % (mt, nt, taps),)  # noqa: E731
+    k = lambda mt, nt, taps: ("patch1_kernel<3, 3, 3>" % (mt, nt, taps),)  # noqa: E731
     table = [
         (plane(63, 64, 32, 3), None), (plane(64, 64, 32, 3), k(1, 1, 9)),     # 64 workgroups,
         (plane(63, 14, 32, 3), None), (plane(63, 7, 32, 3), k(1, 1, 9)),      # or 2^24 multiply-adds
@@ -137,7 +186,7 @@ def test_one_stage_line():
     execs = [(_abi.make_conv_desc("NCHW4", 4, ic, 28, 28, 64, f, pad=f // 2, nonline="RELU", **S), 1, t, False)
              for ic, f in ((32, 3), (36, 3), (64, 3), (68, 3), (64, 5)) for t in tiles]
     want = []
-    for form in ("patch4_one_kernel<1, %d, %d>", "patch4_one_kernel<2, %d, %d>", "patch4_one_kernel<2, %d, %d>", "patch4_kernel<%d, %d, 9>",
-                 "patch4_kernel<%d, %d, 0>"):
+    for form in ("patch4_one_kernel<1, 3, 3>", "patch4_one_kernel<2, 3, 3>", "patch4_one_kernel<2, 3, 3>", "patch4_kernel<3, 3, 9>",
+                 "patch4_kernel<3, 3, 0>"):
         want += [(form % tile,) for tile in ((1, 1), (1, 2), (2, 2))]
     assert _kernels(execs) == want
