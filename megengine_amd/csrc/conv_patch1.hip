@@ -455,12 +455,16 @@ bool patch1_usable(const ConvProblem& p) {
 // 14 -> 19, 202800 pixels: 15.6 us against 18.5), and 64 x 256, which turns a patch for twice the channels, once those are two per
 // CU (3x3 8 -> 189, 61950 pixels: 15.6 against 18.9 and 20.1).  At strides a patch is several times its pixels: 64 x 128 (3x3 38 ->
 // 97, stride 2, 588 workgroups: 14.0 against 18.3).
-//   At strides every tile of 64 channels turns that patch again, so from three of them on, at 2000 workgroups and more, packing once is
-// ahead on filters of 1x1 and 3x3 (23 layers, this kernel over the packed path: 0.84 to 1.83, 1.19 on average; 3x3 6 -> 194 at 59 x 107,
-// batch 57: 51.4 / 28.1; 1x1 7 -> 197 at 89 x 27, batch 51: 19.6 / 13.9).  Not with a residual (1.00 on 10 layers), not where rows out
-// are whole quads (0.95 on 5), not with 25 taps (1.0 on 4), whose products outweigh the turning.
+//   At strides every tile of 64 channels turns that patch again, so from three of them on (tm) packing once gets ahead on filters of 1x1 and
+// 3x3 as their workgroups (w) grow.  Of 7315 layers at stride 2, this kernel over the packed path (two launches), us:
+//     w >= 4 per CU, tm >= 4: 1.14 on average without a residual (3x3 6 -> 193 at 69 x 65, batch 64: 34.7 / 23.2), with one only 3x3 with
+//       rows out that are not whole quads (1.04; 1x1 0.94, whole quads 0.84);
+//     w >= 1200, tm = 3: 1.03 without a residual, rows out that are not whole quads;
+//     another round of chains of three and more stages, w of 1 to 1.6 or 2 to 2.5 per CU, tm >= 3: 1.04 (1x1 219 -> 207 at 106 x 28, batch
+//       20, w = 640: 22.6 / 16.4).
+//   744 of the 7315 were more than 3 % behind packing in one launch and 485 more than 10 %; with these lines 235 and 108.
 //   5x5 with two and more stages at strides of 1 and 2, against the packed path: by what each takes, see p1_behind_packed.
-static int p1_tile(const ConvProblem& p, bool packed, P1Args& k) {
+static int p1_tile(const ConvProblem& p, bool packed, int cu_count, P1Args& k) {
     int lds;
     auto wgs = [&](int tile) { return p1_plan(p, tile, &k, &lds) ? (int64_t)k.tiles_n * k.tiles_m : (int64_t)-1; };
     const int64_t w0 = wgs(0);
@@ -471,8 +475,14 @@ static int p1_tile(const ConvProblem& p, bool packed, P1Args& k) {
     if (packed && w0 < 128 && k.nstages >= (T == 1 ? 4 : T == 9 ? 3 : 2)) return -1;
     if (w0 <= (T == 25 ? 256 : 400)) return 0;
     if (p.d.stride_h > 1 || p.d.stride_w > 1) {
-        if (packed && w0 >= 2000 && p.d.oc > 128 && T <= 9 && !p.d.has_z && p.ow % 4 != 0) return -1;
-        return p.d.oc > 32 && wgs(3) > 0 ? 3 : 0;
+        if (p.d.oc <= 32) return 0;
+        const int64_t w = wgs(3), cu = cu_count;
+        if (packed && p.d.oc > 128 && T <= 9) {
+            const bool ragged = p.ow % 4 != 0, z = p.d.has_z != 0;
+            if (p.d.oc > 192 ? w >= 4 * cu && (!z || (T == 9 && ragged)) : 256 * w >= 1200 * cu && !z && ragged) return -1;
+            if (k.nstages >= 3 && ((w > cu && 5 * w <= 8 * cu) || (w > 2 * cu && 2 * w <= 5 * cu))) return -1;
+        }
+        return w > 0 ? 3 : 0;
     }
     if (p.d.oc > 32 && wgs(2) >= 512) return 2;
     return wgs(1) > 0 ? 1 : 0;
@@ -512,7 +522,7 @@ static bool p1_behind_packed(const ConvProblem& p, int tile, const P1Args& k, in
 int patch1_pick(const ConvProblem& p, bool packed, int cu_count) {
     if (!patch1_usable(p)) return -1;
     P1Args k;
-    const int tile = p1_tile(p, packed, k);
+    const int tile = p1_tile(p, packed, cu_count, k);
     if (tile < 0 || !packed || p.d.fh != 5 || p.d.ic <= 16 || p.d.stride_h > 2 || p.d.stride_w > 2) return tile;
     int lds;
     return p1_plan(p, tile, &k, &lds) && p1_behind_packed(p, tile, k, cu_count) ? -1 : tile;

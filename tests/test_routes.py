@@ -6,43 +6,35 @@ from tests.routes import UNNAMED, routes
 S = dict(scale_bias=2e-4, scale_z=0.05, scale_dst=0.05)
 
 
-# n, ic, ih, iw, oc, f, stride, residual; us packed (two launches) and in one launch
+# n, ic, ih, iw, oc, f, stride, residual; us packed (two launches) and in one launch.  Of 7315 drawn layers at stride 2 every 70th that is more than
+# 5 % behind in one launch and every 110th over 128 channels out that is ahead
 PLAIN_NCHW = [
-    (44, 206, 29, 90, 254, 1, 2, 0, 28.8, 35.2),
-    (40, 5, 75, 49, 185, 3, 2, 0, 18.5, 20.6),
-    (51, 7, 89, 27, 197, 1, 2, 0, 13.9, 19.6),
-    (17, 15, 103, 91, 237, 1, 2, 0, 16.1, 19.2),
-    (55, 134, 105, 35, 200, 3, 2, 0, 54.8, 77.9),
-    (50, 4, 57, 93, 204, 3, 2, 0, 28.0, 34.5),
-    (57, 6, 59, 107, 194, 3, 2, 0, 28.1, 51.4),
-    (56, 17, 84, 85, 236, 1, 2, 0, 29.0, 44.4),
-    (25, 200, 41, 85, 182, 3, 2, 0, 38.9, 38.7),    # fewer workgroups
-    (57, 61, 90, 69, 243, 1, 2, 1, 51.0, 53.5),     # a residual
-    (51, 11, 75, 104, 234, 5, 2, 1, 65.9, 54.2),    # 25 taps
-    (52, 49, 63, 104, 163, 1, 2, 0, 34.0, 22.1),    # rows of whole quads
-    (6, 75, 61, 45, 150, 3, 1, 1, 16.4, 11.6),      # stride 1
+    (31, 99, 109, 88, 250, 3, 2, 0, 61.0, 74.4),
+    (64, 29, 106, 45, 227, 1, 2, 0, 23.2, 32.5),
+    (18, 81, 85, 62, 199, 1, 2, 0, 16.9, 18.4),
+    (64, 86, 41, 35, 249, 1, 2, 0, 16.2, 18.1),
+    (64, 73, 32, 74, 241, 1, 2, 0, 20.9, 24.2),
+    (22, 216, 77, 72, 208, 1, 2, 0, 25.6, 26.9),
+    (54, 82, 67, 52, 208, 1, 2, 1, 33.0, 38.3),
+    (37, 4, 90, 93, 133, 3, 2, 0, 21.1, 24.8),
+    (59, 11, 57, 32, 225, 1, 2, 0, 12.5, 14.7),
+    (68, 115, 28, 27, 105, 3, 2, 1, 17.8, 19.7),
+    (27, 18, 46, 111, 130, 3, 2, 0, 17.5, 13.3),
+    (35, 46, 29, 108, 139, 3, 2, 0, 20.6, 18.0),
+    (48, 4, 28, 104, 163, 3, 2, 0, 15.9, 12.8),
+    (32, 3, 38, 93, 180, 3, 2, 0, 12.7, 11.3),
+    (41, 28, 73, 42, 143, 3, 2, 0, 15.8, 13.3),
+    (33, 101, 65, 108, 243, 1, 2, 0, 31.1, 26.0),
+    (11, 36, 110, 94, 252, 3, 2, 0, 22.5, 19.1),
+    (34, 79, 96, 32, 140, 1, 2, 1, 18.0, 13.9),
+    (45, 5, 40, 23, 135, 1, 2, 1, 9.4, 7.2),
+    (21, 16, 44, 32, 223, 1, 2, 0, 8.4, 6.3),
+    (53, 4, 28, 20, 211, 1, 2, 0, 8.3, 6.8),
+    (46, 3, 20, 32, 205, 3, 2, 1, 9.9, 7.4),
+    (16, 45, 65, 66, 188, 1, 2, 0, 10.8, 9.6),
+    (37, 8, 49, 26, 186, 1, 2, 0, 9.9, 7.8),
+    (3, 7, 109, 96, 225, 3, 2, 0, 9.8, 6.5),
 ]
-
-
-def _nchw(n, ic, ih, iw, oc, f, stride=1, z=0, **kw):
-    return _abi.make_conv_desc("NCHW", n, ic, ih, iw, oc, f, pad=f // 2, stride=stride, nonline="RELU", has_z=bool(z), **dict(S, **kw))
-
-
-def test_plain_nchw_strides():
-    got = routes([_nchw(n, ic, ih, iw, oc, f, s, z) for n, ic, ih, iw, oc, f, s, z, _, _ in PLAIN_NCHW])
-    for r, layer in zip(got, PLAIN_NCHW):
-        packed, one = layer[-2:]
-        assert r.launches in (1, 2)
-        assert (packed if r.launches == 2 else one) <= 1.05 * min(packed, one), layer
-
-
-def _lost(layers):
-    """what the way taken costs over the faster one"""
-    out = []
-    for r, (*_, packed, one) in zip(routes([_nchw(*layer[:8]) for layer in layers]), layers):
-        assert r.launches in (1, 2)
-        out.append((packed if r.launches == 2 else one) / min(packed, one) - 1)
-    return out
 
 
 # 5x5 over 17 and more channels, the same columns: of 2397 drawn layers every 16th that is more than 5 % behind in one launch and every 120th that
@@ -79,6 +71,25 @@ PLAIN_5X5 = [
 ]
 
 
+def _nchw(n, ic, ih, iw, oc, f, stride=1, z=0, **kw):
+    return _abi.make_conv_desc("NCHW", n, ic, ih, iw, oc, f, pad=f // 2, stride=stride, nonline="RELU", has_z=bool(z), **dict(S, **kw))
+
+
+def _lost(layers):
+    """what the way taken costs over the faster one"""
+    out = []
+    for r, (*_, packed, one) in zip(routes([_nchw(*layer[:8]) for layer in layers]), layers):
+        assert r.launches in (1, 2)
+        out.append((packed if r.launches == 2 else one) / min(packed, one) - 1)
+    return out
+
+
+def test_plain_nchw_strides():
+    lost = _lost(PLAIN_NCHW)
+    # always in one launch 10 of these 25 are more than 3 % behind, by up to 40 %
+    assert sum(l > 0.03 for l in lost) <= 4 and max(lost) <= 0.2, lost
+
+
 def test_plain_nchw_5x5():
     lost = _lost(PLAIN_5X5)
     # always in one launch 12 of these 28 are more than 3 % behind, by up to 32 %
@@ -92,7 +103,7 @@ def _kernels(execs):
 def test_plain_nchw_lines():
     """Both sides of every line of patch1_pick, with a workspace; planes out of 8 x 16 are one tile of 128 pixels, 32 channels out one of 32"""
     plane = lambda n, ic, oc, f, stride=1: _nchw(n, ic, 8 * stride, 16 * stride, oc, f, stride)  # noqa: E731
-    k = lambda mt, nt, taps: ("patch1_kernel<3, 3, 3>" % (mt, nt, taps),)  # noqa: E731
+    k = lambda mt, nt, taps: ("patch1_kernel<%d, %d, %d>" % (mt, nt, taps),)  # noqa: E731
     table = [
         (plane(63, 64, 32, 3), None), (plane(64, 64, 32, 3), k(1, 1, 9)),     # 64 workgroups,
         (plane(63, 14, 32, 3), None), (plane(63, 7, 32, 3), k(1, 1, 9)),      # or 2^24 multiply-adds
@@ -186,7 +197,7 @@ def test_one_stage_line():
     execs = [(_abi.make_conv_desc("NCHW4", 4, ic, 28, 28, 64, f, pad=f // 2, nonline="RELU", **S), 1, t, False)
              for ic, f in ((32, 3), (36, 3), (64, 3), (68, 3), (64, 5)) for t in tiles]
     want = []
-    for form in ("patch4_one_kernel<1, 3, 3>", "patch4_one_kernel<2, 3, 3>", "patch4_one_kernel<2, 3, 3>", "patch4_kernel<3, 3, 9>",
-                 "patch4_kernel<3, 3, 0>"):
+    for form in ("patch4_one_kernel<1, %d, %d>", "patch4_one_kernel<2, %d, %d>", "patch4_one_kernel<2, %d, %d>", "patch4_kernel<%d, %d, 9>",
+                 "patch4_kernel<%d, %d, 0>"):
         want += [(form % tile,) for tile in ((1, 1), (1, 2), (2, 2))]
     assert _kernels(execs) == want
