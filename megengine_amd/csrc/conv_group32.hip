@@ -302,7 +302,10 @@ bool grp32_can_run(const IgemmArgs& a, int pin, int pout, int cfg) {
 // against 8.3 on 32 x 256 for 11 groups of 32 at 70 x 23, batch 15; the second-generation tile 16.2).  64 channels per group: 64 x
 // 128 from 500 on, where the patch is turned over half as often as 32 wide (7 groups, 15 x 25, batch 18, residual: 6.8 / 6.3), 64 x
 // 256 from 2400 on (19344: 63.1 / 57.6, the second-generation tile 87.4).  At stride 2 a patch is four times its pixels and never 256
-// wide; 64 x 128 from 250 on (11 groups of 64 at 41 x 105, batch 26: 39.7 / 32.1).
+// wide; 64 x 128 from 250 on (11 groups of 64 at 41 x 105, batch 26: 39.7 / 32.1).  Without a residual and into more than 64 channels
+// per group the second-generation tiles, whose 128 channels share the nine reads of a pixel, are ahead of large layers: over 64 channels
+// from 1200 on (224 layers, 1.09 of their time here on average; 11 groups, 64 -> 128 at 14 x 38, batch 45: 18.6 / 13.8), over 32 from 2000 on
+// if they fill the tiles of 128 to three quarters (100 layers, 1.06; others 0.97).  With a residual 0.92 (149 layers), at stride 1 0.7 to 1.0.
 //   Dense layers over 32 or 64 channels that are too large for the few-pixel tiles: 64 -> 64 at 49 x 49, batch 7: 6.4 / 4.7; 64 -> 96
 // at 61 x 23, batch 49, residual: 13.6 / 9.6.  The weight-resident tile keeps its range, from 2560 tiles of 64 x 128 on; and at stride
 // 2 with several channel tiles the staged tiles are ahead from 800 workgroups on (64 -> 128 at 56 x 56, batch 64: 11.1 / 10.0).
@@ -320,6 +323,8 @@ int grp32_pick(const IgemmArgs& a, int pin, int pout, bool will_preprocess) {
         const int64_t t64 = px * ((a.OC + 63) / 64);
         if (t64 >= (!will_preprocess || (s1 && a.OC % 64 != 0) ? 2560 : s1 && a.OC == 64 ? 1500 : 1200)) return -1;
         if (!s1 && a.OC > 64 && w0 >= 800) return -1;
+    } else if (!s1 && a.ocpg > 64 && !a.epi.has_z) {
+        if (a.kbytes == 576 ? w0 >= 1200 : w0 >= 2000 && (a.ocpg + 127) / 128 * 128 - a.ocpg <= 32) return -1;
     }
     int cfg;
     if (a.ocpg % 64 != 0) cfg = s1 && w0 >= 600 ? 1 : 0;
