@@ -599,12 +599,15 @@ int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, int cu_count, co
     //     (708 layers, 10 of them more than 3 % behind, the worst 1.13), 5x5 by the prices of dw5_matrix.
     //   other filters, against dw4_kernel: 4x4 at 35 x 38, 112 channels, batch 45: 8.8 / 29.9; 6x6 at 101 x 14, 256, batch 1: 4.2 / 12.8;
     //     2x2 at 71 x 26, 108, batch 63: 12.6 / 15.7.  At strides of 3 and 4 a filter of few taps leaves most of the patch unused: 7x1,
-    //     stride 3, 448 at 44 x 82, batch 2: 6.3 / 5.6.
+    //     stride 3, 448 at 44 x 82, batch 2: 6.3 / 5.6.  A 1x1, or two taps at stride 2, costs dw4 next to nothing beyond its bytes: from 40000
+    //     quads of output on it is ahead (248 of 1311 layers of one and two taps, 1.08 of its time in the matrix form on average, up to 1.5; 832
+    //     channels, 1x1 stride 2 at 76 x 80, batch 4: 8.6 / 5.9); below, the matrix form (0.88 on the other 1063).
     const bool small_planes = (int64_t)d.n * a.CG >= 512 && (int64_t)a.OH * a.QW < 100;
     // (output rows per thread of the vector forms, see below)
     const int64_t rows = (int64_t)d.n * a.CG * a.OH * a.QW;
     const bool few = rows <= (a.OH % 2 && a.OH <= 7 ? 262144 : 131072);
-    const bool matrix = wide ? !small_planes : !(sq && d.fh == 3) && (d.stride_w <= 2 || d.fh * d.fw >= 9);
+    const bool few_taps = rows > 40000 && (d.fh * d.fw == 1 || (d.fh * d.fw == 2 && d.stride_w > 1));
+    const bool matrix = wide ? !small_planes : !(sq && d.fh == 3) && !few_taps && (d.stride_w <= 2 || d.fh * d.fw >= 9);
     const int64_t src_total = (int64_t)(d.n - 1) * p.src_sn + (int64_t)d.ic * d.ih * d.iw;
     const bool dwf = wide && src_total < ((int64_t)1 << 31);
     if (matrix && dwm_usable(p) && (!dwf || d.fh == 7 || dw5_matrix(p, a.QW, few ? 1 : 2, cu_count))) return launch_dwm(st, p, src, flt, bias, z, dst);

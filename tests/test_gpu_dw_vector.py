@@ -37,6 +37,10 @@ CASES = [
     (1, 4, 5, 1703, 5, 5, (2, 1), 1, "dw4_kernel"),
     (2, 8, 140, 9, 5, 5, (0, 2), (70, 1), "dw4_kernel"),
     (1, 4, 1, 1, 11, 11, 5, 1, "dw4_kernel"),
+    (8, 100, 25, 37, 1, 1, 0, 1, "dw4_kernel"),                # one tap, two at stride 2: more than 40000 quads out
+    (10, 100, 49, 125, 2, 1, (1, 0), 2, "dw4_kernel"),
+    (10, 100, 51, 123, 1, 2, (0, 1), 2, "dw4_kernel"),
+    (8, 100, 25, 32, 1, 1, 0, 1, "dwm_kernel<1, true>"),       # exactly that many
 ]
 
 

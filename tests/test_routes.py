@@ -141,7 +141,8 @@ def test_channel_wise_lines():
         (_dw(1, 8, 24, 24, 7, 1, 0, 2), "dwm_kernel<4, true>"), (_dw(1, 8, 24, 24, 7, 1, 0, 3), "dw4_kernel"),
         (_dw(1, 8, 24, 24, 9, 1, 0, 3), "dwm_kernel<7, true>"), (_dw(1, 8, 24, 24, 5, 5, 2, 4), "dwm_kernel<7, true>"),
         (_dw(1, 8, 24, 24, 5, 5, 2, 5), "dw4_kernel"), (_dw(1, 8, 24, 24, 8, 8, 0, 1), "dwm_kernel<6, true>"),
-        (_dw(1, 8, 24, 24, 11, 11, 0, 1), "dw4_kernel"), (_dw(1, 8, 5, 1634, 5, 5, (2, 1), 1), "dwm_kernel<3, true>"),
+        (_dw(1, 8, 24, 24, 11, 11, 0, 1), "dw4_kernel"), (_dw(10, 400, 25, 32, 1, 1, 0, 1), "dw4_kernel"), (_dw(10, 400, 25, 32, 1, 2, (0, 1), 1), "dwm_kernel<1, true>"),
+        (_dw(8, 100, 25, 32, 1, 1, 0, 1), "dwm_kernel<1, true>"), (_dw(8, 100, 25, 36, 1, 1, 0, 1), "dw4_kernel"), (_dw(10, 100, 50, 126, 2, 1, (1, 0), 2), "dw4_kernel"), (_dw(1, 8, 5, 1634, 5, 5, (2, 1), 1), "dwm_kernel<3, true>"),
         (_dw(1, 8, 5, 1635, 5, 5, (2, 1), 1), "dw4_kernel"), (_dw(1, 8, 70, 9, 5, 5, 0, (65, 1)), "dw4_kernel"),
     ]
     for got, (d, want) in zip(_kernels([d for d, _ in table]), table):
@@ -188,6 +189,46 @@ def test_channel_wise_5x5():
         lost.append((dwf if k.startswith("dwf") else dwm) / min(dwf, dwm) - 1)
     # the prices leave 18 of the 1317 more than 3 % behind, at most 16 %
     assert max(lost) <= 0.16 and sum(l > 0.03 for l in lost) <= 2, lost
+
+
+# filters of one and two taps: n, channels, ih, iw, fh, fw, stride, residual; us of dw4_kernel and of the matrix form.  Of 1311 drawn layers every
+# 16th on which the matrix form is more than 5 % behind, and every 70th on which it is more than 10 % ahead
+FEW_TAPS = [
+    (17, 164, 80, 16, 1, 1, 2, 0, 4.1, 4.4),
+    (24, 736, 13, 74, 1, 1, 1, 0, 11.4, 13.8),
+    (30, 28, 105, 73, 1, 2, 1, 0, 8.3, 11.4),
+    (3, 780, 38, 48, 1, 1, 1, 0, 5.6, 7.1),
+    (41, 852, 24, 19, 1, 2, 1, 1, 16.7, 21.6),
+    (43, 28, 12, 12, 1, 1, 1, 0, 3.0, 3.2),
+    (7, 772, 12, 51, 1, 2, 2, 0, 4.1, 4.3),
+    (10, 80, 35, 38, 1, 1, 1, 0, 4.1, 4.4),
+    (13, 148, 34, 13, 1, 1, 2, 0, 3.1, 3.4),
+    (57, 880, 18, 24, 2, 1, 1, 1, 19.6, 26.8),
+    (6, 872, 88, 5, 2, 1, 2, 0, 3.9, 4.3),
+    (25, 12, 104, 67, 1, 1, 1, 1, 5.1, 6.8),
+    (17, 1036, 12, 36, 2, 1, 1, 0, 9.1, 10.9),
+    (54, 8, 80, 91, 2, 1, 2, 1, 4.9, 5.3),
+    (5, 48, 33, 11, 2, 1, 1, 1, 3.9, 3.2),
+    (4, 16, 11, 14, 1, 1, 1, 1, 3.8, 3.3),
+    (13, 296, 58, 10, 2, 1, 1, 1, 6.2, 5.5),
+    (4, 128, 12, 49, 1, 2, 1, 1, 4.1, 3.3),
+    (2, 60, 5, 10, 2, 1, 2, 1, 3.9, 3.0),
+    (3, 48, 8, 4, 2, 1, 1, 0, 3.7, 2.9),
+    (32, 36, 6, 37, 2, 1, 2, 1, 4.5, 3.7),
+    (2, 72, 75, 5, 1, 1, 1, 0, 3.6, 3.1),
+    (3, 20, 23, 5, 1, 2, 1, 1, 3.8, 3.1),
+    (3, 20, 22, 5, 1, 2, 2, 1, 3.4, 3.0),
+    (1, 16, 12, 15, 2, 1, 1, 0, 3.5, 2.9),
+]
+
+
+def test_channel_wise_few_taps():
+    got = _kernels([_dw(n, c, ih, iw, fh, fw, (fh // 2, fw // 2), s, z) for n, c, ih, iw, fh, fw, s, z, _, _ in FEW_TAPS])
+    lost = []
+    for (k,), (*_, dw4, dwm) in zip(got, FEW_TAPS):
+        assert k.startswith(("dw4_kernel", "dwm_kernel"))
+        lost.append((dw4 if k.startswith("dw4") else dwm) / min(dw4, dwm) - 1)
+    assert sum(l > 0.03 for l in lost) <= 6 and max(lost) <= 0.38, lost
 
 
 def test_one_stage_line():
