@@ -613,7 +613,7 @@ static bool igemm_plain_s32(const ConvProblem& p) {
 // eleven to nineteen to 1.9 % on average and are 1.13 times as fast as thresholds on tile counts: 3x3 288 -> 672 at 45 x 37, batch 10:
 // 48.8 -> 34.4 us; 5x5 32 -> 992 at 51 x 64, stride 2, batch 59: 70.8 -> 63.4; 1x1 320 -> 672 at 60 x 34, batch 49: 63.7 -> 47.8.
 // Without the four terms and the last tile it was 1.11, and 306 of the 2640 were more than 3 % slower than by thresholds (97 more than
-// 10 %); 79 are with them (9), at most 1.19.
+// 10 %); 79 are with them (9), at most 1.19.  Layers into 32 channels and fewer are not priced: they keep the 32 x 256 tile.
 static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool window, bool strided, bool has_z, int cu_count) {
     struct Price {
         int cfg, bm, bn;  // tile: 2^bm channels x 2^bn pixels

@@ -464,10 +464,16 @@ bool patch1_usable(const ConvProblem& p) {
 //       20, w = 640: 22.6 / 16.4).
 //   744 of the 7315 were more than 3 % behind packing in one launch and 485 more than 10 %; with these lines 235 and 108.
 //   5x5 with two and more stages at strides of 1 and 2, against the packed path: by what each takes, see p1_behind_packed.
-static int p1_tile(const ConvProblem& p, bool packed, int cu_count, P1Args& k) {
+// (k: the geometry of some tile; *chosen: the workgroups of the one that is returned)
+static int p1_tile(const ConvProblem& p, bool packed, int cu_count, P1Args& k, int64_t* chosen) {
     int lds;
     auto wgs = [&](int tile) { return p1_plan(p, tile, &k, &lds) ? (int64_t)k.tiles_n * k.tiles_m : (int64_t)-1; };
     const int64_t w0 = wgs(0);
+    *chosen = w0;
+    auto take = [&](int tile, int64_t w) {
+        *chosen = w;
+        return tile;
+    };
     const int T = (int)(p.d.fh * p.d.fw);
     if (w0 < 0) return -1;
     const uint64_t macs = (uint64_t)p.d.n * p.d.oc * p.oh * p.ow * p.icpg * p.d.fh * p.d.fw;
@@ -482,10 +488,12 @@ static int p1_tile(const ConvProblem& p, bool packed, int cu_count, P1Args& k) {
             if (p.d.oc > 192 ? w >= 4 * cu && (!z || (T == 9 && ragged)) : 256 * w >= 1200 * cu && !z && ragged) return -1;
             if (k.nstages >= 3 && ((w > cu && 5 * w <= 8 * cu) || (w > 2 * cu && 2 * w <= 5 * cu))) return -1;
         }
-        return w > 0 ? 3 : 0;
+        return w > 0 ? take(3, w) : 0;
     }
-    if (p.d.oc > 32 && wgs(2) >= 512) return 2;
-    return wgs(1) > 0 ? 1 : 0;
+    const int64_t w2 = p.d.oc > 32 ? wgs(2) : 0;
+    if (w2 >= 512) return take(2, w2);
+    const int64_t w1 = wgs(1);
+    return w1 > 0 ? take(1, w1) : 0;
 }
 
 // 5x5 in two and more stages: whether the packed path is ahead of this kernel on its tile, by prices on a device of 256 CUs in us and, of
@@ -494,7 +502,7 @@ static int p1_tile(const ConvProblem& p, bool packed, int cu_count, P1Args& k) {
 // many tiles out smoothly.  Fitted to graph replays of 2397 layers over 17 to 256 channels on both; of these 213 were more than 3 %
 // behind the packed path and 117 more than 10 % (5x5 209 -> 33 at 26 x 7, batch 38: 24.2 / 13.3; 183 -> 164 at 41 x 85, batch 5:
 // 56.4 / 36.8); with the prices 40 and 12.  On 591 others 70 and 44 before, 9 and 1 now, 0.70 and 0.69 of the packed path on average.
-static bool p1_behind_packed(const ConvProblem& p, int tile, const P1Args& k, int cu_count) {
+static bool p1_behind_packed(const ConvProblem& p, int tile, int64_t workgroups, int nstages, int cu_count) {
     struct One {
         float launch, stage, round2_stage, round_stage, share;
     };
@@ -507,9 +515,9 @@ static bool p1_behind_packed(const ConvProblem& p, int tile, const P1Args& k, in
     };
     static const Packed packed[2] = {{5.747f, 1.533f, 0.000f, 3.430f, 0.000f, 1.973f, 0.000f},   // tiles of 64 x 128 for a quarter of the CUs
                                      {7.846f, 0.155f, 1.474f, 0.277f, 1.204f, 2.086f, 1.357f}};
-    const uint32_t cu = (uint32_t)cu_count, wgs = (uint32_t)k.tiles_n * (uint32_t)k.tiles_m, r1 = (wgs + cu - 1) / cu;
+    const uint32_t cu = (uint32_t)cu_count, wgs = (uint32_t)workgroups, r1 = (wgs + cu - 1) / cu;
     const One& a = one[tile];
-    const float this_us = a.launch + (float)k.nstages * (a.stage + a.round2_stage * (float)((r1 + 1) / 2) + a.round_stage * (float)r1) +
+    const float this_us = a.launch + (float)nstages * (a.stage + a.round2_stage * (float)((r1 + 1) / 2) + a.round_stage * (float)r1) +
                           a.share * ((float)wgs / (float)cu);
     const uint64_t px = (uint64_t)p.d.n * p.oh * p.ow, tiles = (px + 127) / 128 * ((p.d.oc + 63) / 64), rounds = (tiles + cu - 1) / cu;
     const float share = (float)tiles / (float)cu, kb = (float)((p.d.ic + 31) / 32 * 32 * 25) / 1024.0f;
@@ -522,10 +530,10 @@ static bool p1_behind_packed(const ConvProblem& p, int tile, const P1Args& k, in
 int patch1_pick(const ConvProblem& p, bool packed, int cu_count) {
     if (!patch1_usable(p)) return -1;
     P1Args k;
-    const int tile = p1_tile(p, packed, cu_count, k);
+    int64_t wgs;
+    const int tile = p1_tile(p, packed, cu_count, k, &wgs);
     if (tile < 0 || !packed || p.d.fh != 5 || p.d.ic <= 16 || p.d.stride_h > 2 || p.d.stride_w > 2) return tile;
-    int lds;
-    return p1_plan(p, tile, &k, &lds) && p1_behind_packed(p, tile, k, cu_count) ? -1 : tile;
+    return p1_behind_packed(p, tile, wgs, k.nstages, cu_count) ? -1 : tile;
 }
 
 int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
