@@ -15,7 +15,7 @@
 //   * Two stages in LDS, the next one's loads in registers while the current one is multiplied, one barrier per stage.
 //   * Bound by LDS, as the 4-packed patch tiles are, and by the latency of a stage where tiles are few.
 // Filters of 1x1, 3x3 and 5x5; others go through the
-// workspace.  Graph replays: 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual: 17.3 us packed, 13.2 here (four waves of
+// workspace.  Graph replays: 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual: 16.6 us packed, 12.2 here (four waves of
 // 1200 vector instructions for 23 products each, a third of their time waiting for a stage's loads); more at patch1_pick.
 #include <atomic>
 
@@ -447,7 +447,7 @@ bool patch1_usable(const ConvProblem& p) {
 //   The packed path takes 6 to 9 us however few the tiles -- two launches, but its few-pixel kernel splits the reduction -- where
 // this kernel walks the stages one after the other at 0.9 us each (1.7 with 25 taps): up to half a workgroup per CU a long
 // reduction goes there (3x3 130 -> 44 at 12 x 12, five stages: 8.6 us here, 6.9 there; 48 -> 12, two: 5.0 / 6.4).  With more tiles
-// it is the other way round: 3x3 45 -> 12 at 22 x 22, batch 47: 5.9 / 11.5; 1x1 20 -> 149 at 96 x 78: 24.1 / 34.3; 5x5 46 -> 45,
+// it is the other way round: 3x3 45 -> 12 at 22 x 22, batch 47: 5.3 / 9.4; 1x1 20 -> 149 at 96 x 78: 24.1 / 34.3; 5x5 46 -> 45,
 // 168640 pixels: 25.4 / 41.4.  A caller without a workspace has no packed path (packed = false).
 //   Below 64 workgroups and from 2^24 multiply-adds on the packed path stays, 5 to 25 % behind on one or two stages: a workspace of
 // the size that it needs is written there, which the interface's tests hold (24 -> 40 at 28 x 28, batch 4, among them).
