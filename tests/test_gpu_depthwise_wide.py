@@ -1,5 +1,5 @@
 """Channel-wise 5x5 and 7x7 convolutions at widths around the blocks of four pixels, odd heights, images smaller than the filter,
-both strides, every activation with and without a residual, and other paddings and strides: on these few or large planes all of them
+both strides, every activation with and without a residual, and other paddings and strides: on these few or large planes all of them but one
 run the matrix form (test_gpu_dw_matrix.py); the vector forms have their cases in test_gpu_dw_vector.py.  3x3 layers with one,
 two and four output rows per thread."""
 import pytest
