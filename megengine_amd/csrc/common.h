@@ -146,9 +146,10 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t x, const FastDiv& f) {
 // Workgroup b runs on XCD b % 8, and each XCD has an L2 of its own.  Kernels that walk a tensor from front to back give every
 // XCD one contiguous eighth of it, so that an operator finds the bytes that the operator before it wrote in the L2 in front
 // of it (and not in another one's, behind the fabric): images of a batch stay with their XCD through a chain of operators.
-// xcd_block: the block of this workgroup when blocks are dealt out that way (a permutation of 0 .. gridDim.x - 1).
-__device__ __forceinline__ uint32_t xcd_block() {
-    const uint32_t x = blockIdx.x & 7, per = gridDim.x >> 3, rem = gridDim.x & 7;
+// (The number of workgroups is an argument of the kernels: gridDim is a hidden one, 66 bytes behind the others, see wire.h.)
+// xcd_block: the block of this workgroup when blocks are dealt out that way (a permutation of 0 .. grid - 1).
+__device__ __forceinline__ uint32_t xcd_block(uint32_t grid) {
+    const uint32_t x = blockIdx.x & 7, per = grid >> 3, rem = grid & 7;
     return x * per + (x < rem ? x : rem) + (blockIdx.x >> 3);
 }
 // xcd_run: the units of this thread (workgroups of 256) as a strided loop
@@ -157,11 +158,11 @@ struct XcdRun {
     T at, end, step;
 };
 template <class T>
-__device__ __forceinline__ XcdRun<T> xcd_run(T units) {
-    if (gridDim.x < 16) return {(T)blockIdx.x * 256 + threadIdx.x, units, (T)gridDim.x * 256};
+__device__ __forceinline__ XcdRun<T> xcd_run(T units, uint32_t grid) {
+    if (grid < 16) return {(T)blockIdx.x * 256 + threadIdx.x, units, (T)grid * 256};
     const T per = (units + 2047) / 2048 * 256, lo = (T)(blockIdx.x & 7) * per;
     const T hi = lo + per < units ? lo + per : units;
-    return {lo + (T)(blockIdx.x >> 3) * 256 + threadIdx.x, hi, (T)((gridDim.x + 7 - (blockIdx.x & 7)) >> 3) * 256};
+    return {lo + (T)(blockIdx.x >> 3) * 256 + threadIdx.x, hi, (T)((grid + 7 - (blockIdx.x & 7)) >> 3) * 256};
 }
 // whole rounds over the XCDs, so that no XCD lacks a workgroup for its eighth
 static inline uint64_t xcd_grid(uint64_t blocks) { return blocks < 16 ? blocks : (blocks + 7) & ~(uint64_t)7; }

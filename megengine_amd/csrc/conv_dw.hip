@@ -12,7 +12,10 @@
 // That form (dw4_kernel) serves every filter size / stride.  The 3x3, stride 1 or 2 case -- every
 // channel-wise layer of the MobileNet family -- has its own kernel, dw3x3_kernel, and so have 5x5 and 7x7 with "same"
 // padding, dwf_kernel, below.  Where the dot products bound them, the matrix cores take over (conv_dwm.hip).
+#include <tuple>
+
 #include "common.h"
+#include "wire.h"
 
 namespace mi355 {
 namespace {
@@ -109,6 +112,7 @@ __global__ __launch_bounds__(256) void dw4_kernel(DwArgs a) {
 //     multiplies three horizontally adjacent taps with a single v_dot4: 3 dot products per output
 //     instead of 9.
 // ---------------------------------------------------------------------------------------------
+template <class Div>
 struct Dw3Args {
     const int8_t* src;
     const int8_t* flt;
@@ -117,13 +121,80 @@ struct Dw3Args {
     int8_t* dst;
     int CG, IH, IW, OH, OW, QW, OHS;  // QW = pixel quads per output row, OHS = row strips per plane
     int ph, pw;
-    uint32_t items;
+    uint32_t items, grid;
     uint32_t src_bytes;  // whole source tensor if it is addressable with 31-bit offsets, else 0
     int64_t src_sn, dst_sn, z_sn;
     int has_bias;
-    FastDiv div_qw, div_ohs, div_cg;
+    Div div_qw, div_ohs, div_cg;
     EpiParams epi;
+
+    auto numbers() const { return std::tie(CG, IH, IW, OH, OW, QW, OHS, ph, pw, items, grid, src_bytes, src_sn, dst_sn, z_sn, has_bias); }
 };
+
+// The two forms of the kernels' argument (see wire.h)
+struct Dw3Wide {
+    Dw3Args<FastDiv> a;
+    // Every kernel argument is requested in one batch of scalar loads: left alone the compiler fetches them where they
+    // are first used, behind the early exit and the item decoding -- three dependent round trips to the argument
+    // segment before the first vector load of a kernel whose whole life is a few microseconds.
+    template <int R>
+    __device__ __forceinline__ Dw3Args<FastDiv> open() const {
+        asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.CG), "s"(a.IH), "s"(a.IW), "s"(a.OH),
+                     "s"(a.OW), "s"(a.QW), "s"(a.OHS), "s"(a.ph), "s"(a.pw), "s"(a.items), "s"(a.src_bytes), "s"(a.src_sn),
+                     "s"(a.dst_sn), "s"(a.z_sn), "s"(a.has_bias), "s"(a.grid));
+        asm volatile("" ::"s"(a.div_qw.m), "s"(a.div_qw.s1), "s"(a.div_qw.s2), "s"(a.div_ohs.m), "s"(a.div_ohs.s1),
+                     "s"(a.div_ohs.s2), "s"(a.div_cg.m), "s"(a.div_cg.s1), "s"(a.div_cg.s2), "s"(a.epi.fast), "s"(a.epi.lin),
+                     "s"(a.epi.has_z), "s"(a.epi.nonline), "s"(a.epi.lin_c), "s"(a.epi.lin_d), "s"(a.epi.lin_lo));
+        return a;
+    }
+};
+
+struct Dw3Wire {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    uint32_t items, in, out, window, flags;  // in, out: height | width << 16; window: padding | channel blocks << 16
+    EpiWire epi;
+
+    template <int R, class Div>
+    __host__ __device__ __forceinline__ void numbers(Dw3Args<Div>& k) const {
+        k.CG = wire_hi(window); k.ph = wire_byte(window, 0); k.pw = wire_byte(window, 1);
+        k.IH = wire_lo(in); k.IW = wire_hi(in); k.OH = wire_lo(out); k.OW = wire_hi(out);
+        k.QW = (k.OW + 3) / 4; k.OHS = (k.OH + R - 1) / R;
+        k.items = items; k.grid = (items + 63) / 64;
+        k.src_sn = (uint32_t)wire_mul(k.CG, k.IH, k.IW * 4);
+        k.dst_sn = (uint32_t)wire_mul(k.CG, k.OH, k.OW * 4);
+        k.z_sn = (flags >> 3 & 1) ? k.dst_sn : 0;
+        k.src_bytes = (flags >> 16) * (uint32_t)k.src_sn;  // (images)
+        k.has_bias = (int)(flags >> 8 & 1);
+    }
+    template <int R>
+    __device__ __forceinline__ Dw3Args<Quot> open() const {
+        asm volatile("" ::"s"(src), "s"(flt), "s"(bias), "s"(z), "s"(dst), "s"(items), "s"(in), "s"(out), "s"(window), "s"(flags), "s"(epi.f[0]),
+                     "s"(epi.f[1]), "s"(epi.f[2]), "s"(epi.f[3]));  // one batch of scalar loads
+        Dw3Args<Quot> k;
+        k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
+        numbers<R>(k);
+        k.div_qw = quot(k.QW); k.div_ohs = quot(k.OHS); k.div_cg = quot(k.CG);
+        k.epi = epi_open(epi, flags & 255);
+        return k;
+    }
+    // false: the problem has a number that does not fit
+    template <int R>
+    bool pack(const Dw3Args<FastDiv>& k, uint32_t n) {
+        src = k.src; flt = k.flt; bias = k.bias; z = k.z; dst = k.dst;
+        items = k.items; in = wire2(k.IH, k.IW); out = wire2(k.OH, k.OW);
+        window = wire4(k.ph, k.pw, 0, 0) | (uint32_t)k.CG << 16;
+        flags = epi_wire(k.epi, false, &epi) | (k.has_bias ? 1u << 8 : 0) | n << 16;
+        Dw3Args<FastDiv> o;
+        numbers<R>(o);
+        if (!k.epi.has_z) o.z_sn = k.z_sn;  // (nothing reads it)
+        return o.numbers() == k.numbers() && items < QUOT_MAX && n < 65536;
+    }
+};
+static_assert(sizeof(Dw3Wire) <= WIRE_BYTES, "a wire");
 
 __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
     return __builtin_amdgcn_perm(hi, lo, sel);
@@ -157,8 +228,8 @@ __device__ __forceinline__ void load_px4(const uint32_t* row, int c0, int IW, bo
     }
 }
 
-template <int R, int NL, bool HZ, bool FAST>
-__device__ __forceinline__ void dw3_store(const Dw3Args& a, const int (&acc)[R][4][4], int n, int cg, int oh0, int ow0) {
+template <int R, int NL, bool HZ, bool FAST, class Args>
+__device__ __forceinline__ void dw3_store(const Args& a, const int (&acc)[R][4][4], int n, int cg, int oh0, int ow0) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int oh = oh0 + r;
@@ -199,18 +270,10 @@ __device__ __forceinline__ void dw3_store(const Dw3Args& a, const int (&acc)[R][
 // fast form), 2: any other, chosen at run time.  BUF: input rows through bounds-checked buffer loads (tensors below
 // 2 GiB, padding at most 1); otherwise pointer loads.  The two common forms of the MobileNet family get kernels that
 // hold nothing else: a launch of a few microseconds should not have to fetch eight epilogues' worth of code.
-template <int S, int R, int EPI, bool BUF>
-__global__ __launch_bounds__(256) void dw3x3_kernel(Dw3Args a) {
-    // Every kernel argument is requested in one batch of scalar loads: left alone the compiler fetches them where they
-    // are first used, behind the early exit and the item decoding -- three dependent round trips to the argument
-    // segment before the first vector load of a kernel whose whole life is a few microseconds.
-    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.CG), "s"(a.IH), "s"(a.IW), "s"(a.OH),
-                 "s"(a.OW), "s"(a.QW), "s"(a.OHS), "s"(a.ph), "s"(a.pw), "s"(a.items), "s"(a.src_bytes), "s"(a.src_sn),
-                 "s"(a.dst_sn), "s"(a.z_sn), "s"(a.has_bias));
-    asm volatile("" ::"s"(a.div_qw.m), "s"(a.div_qw.s1), "s"(a.div_qw.s2), "s"(a.div_ohs.m), "s"(a.div_ohs.s1),
-                 "s"(a.div_ohs.s2), "s"(a.div_cg.m), "s"(a.div_cg.s1), "s"(a.div_cg.s2), "s"(a.epi.fast), "s"(a.epi.lin),
-                 "s"(a.epi.has_z), "s"(a.epi.nonline), "s"(a.epi.lin_c), "s"(a.epi.lin_d), "s"(a.epi.lin_lo));
-    const uint32_t item = xcd_block() * 64u + threadIdx.x;
+template <int S, int R, int EPI, bool BUF, class Form>
+__device__ __forceinline__ void dw3x3_run(const Form& form) {
+    const auto a = form.template open<R>();
+    const uint32_t item = xcd_block(a.grid) * 64u + threadIdx.x;
     if (item >= a.items) return;
     // item = ((n * CG + cg) * OHS + strip) * QW + quad
     const uint32_t i1 = fdiv(item, a.div_qw), q = item - i1 * a.QW;
@@ -401,16 +464,28 @@ __global__ __launch_bounds__(256) void dw3x3_kernel(Dw3Args a) {
     }
 }
 
-template <int S, int R>
-int launch_dw3(hipStream_t st, dim3 grid, dim3 block, const Dw3Args& b) {
+template <int S, int R, int EPI, bool BUF>
+__global__ __launch_bounds__(256) void dw3x3_kernel(Dw3Wire a) {
+    dw3x3_run<S, R, EPI, BUF>(a);
+}
+template <int S, int R, int EPI, bool BUF>
+__global__ __launch_bounds__(256) void dw3x3_kernel(Dw3Wide a) {
+    dw3x3_run<S, R, EPI, BUF>(a);
+}
+
+template <int S, int R, class Form>
+int launch_dw3_form(hipStream_t st, dim3 grid, dim3 block, const Dw3Args<FastDiv>& b, const Form& form) {
     const bool buf = b.src_bytes != 0 && b.pw <= 1;
     const int epi = !b.epi.fast ? 2 : b.epi.lin ? 0 : (!b.epi.has_z && b.epi.nonline == NL_RELU) ? 1 : 2;
-    if (buf) {
-        if (epi == 0) return launch_kernel((dw3x3_kernel<S, R, 0, true>), grid, block, 0, st, b);
-        if (epi == 1) return launch_kernel((dw3x3_kernel<S, R, 1, true>), grid, block, 0, st, b);
-        return launch_kernel((dw3x3_kernel<S, R, 2, true>), grid, block, 0, st, b);
-    }
-    return launch_kernel((dw3x3_kernel<S, R, 2, false>), grid, block, 0, st, b);
+    typedef void (*Kernel)(Form);
+    const Kernel kern = !buf ? (Kernel)dw3x3_kernel<S, R, 2, false> : epi == 0 ? (Kernel)dw3x3_kernel<S, R, 0, true> :
+                        epi == 1 ? (Kernel)dw3x3_kernel<S, R, 1, true> : (Kernel)dw3x3_kernel<S, R, 2, true>;
+    return launch_kernel(kern, grid, block, 0, st, form);
+}
+template <int S, int R>
+int launch_dw3(hipStream_t st, dim3 grid, dim3 block, const Dw3Args<FastDiv>& b, uint32_t n) {
+    Dw3Wire wire;
+    return wire.pack<R>(b, n) ? launch_dw3_form<S, R>(st, grid, block, b, wire) : launch_dw3_form<S, R>(st, grid, block, b, Dw3Wide{b});
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -425,12 +500,13 @@ int launch_dw3(hipStream_t st, dim3 grid, dim3 block, const Dw3Args& b) {
 // 240 channels, 5x5 stride 2 at 57 x 57, batch 16 (16 MB): 22.5 -> 8.6 us; 96 channels, stride 1 at 56 x 56: 36.7 -> 9.2 us.
 // (launch bounds of 256 although workgroups hold one wave: with 64 the compiler spends twice the registers on these kernels)
 // ---------------------------------------------------------------------------------------------
-template <int F, int S, int R>
-__global__ __launch_bounds__(256) void dwf_kernel(Dw3Args a) {
+template <int F, int S, int R, class Form>
+__device__ __forceinline__ void dwf_run(const Form& form) {
     constexpr int P = F / 2, ROWS = (R - 1) * S + F;
     constexpr int FIRST = 4 - P;                       // pixel of the loaded blocks at which output 0's window starts
     constexpr int NB = (FIRST + 3 * S + F + 3) / 4;    // blocks a thread loads per row
-    const uint32_t item = xcd_block() * 64u + threadIdx.x;
+    const auto a = form.template open<R>();
+    const uint32_t item = xcd_block(a.grid) * 64u + threadIdx.x;
     if (item >= a.items) return;
     const uint32_t i1 = fdiv(item, a.div_qw), q = item - i1 * a.QW;
     const uint32_t i2 = fdiv(i1, a.div_ohs), strip = i1 - i2 * a.OHS;
@@ -537,6 +613,22 @@ __global__ __launch_bounds__(256) void dwf_kernel(Dw3Args a) {
     }
 }
 
+template <int F, int S, int R>
+__global__ __launch_bounds__(256) void dwf_kernel(Dw3Wire a) {
+    dwf_run<F, S, R>(a);
+}
+template <int F, int S, int R>
+__global__ __launch_bounds__(256) void dwf_kernel(Dw3Wide a) {
+    dwf_run<F, S, R>(a);
+}
+
+template <int F, int S, int R>
+int launch_dwf(hipStream_t st, dim3 grid, dim3 block, const Dw3Args<FastDiv>& b, uint32_t n) {
+    Dw3Wire wire;
+    if (wire.pack<R>(b, n)) return launch_kernel((void (*)(Dw3Wire))dwf_kernel<F, S, R>, grid, block, 0, st, wire);
+    return launch_kernel((void (*)(Dw3Wide))dwf_kernel<F, S, R>, grid, block, 0, st, Dw3Wide{b});
+}
+
 }  // namespace
 
 bool depthwise_usable(const ConvProblem& p) {
@@ -620,7 +712,7 @@ int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, int cu_count, co
         // batch 64: 4.2 / 4.8, 96 at 112 x 112: 16.6 / 16.4.  Planes of few, odd rows leave strips of two half empty: 960 at
         // 7 x 7, batch 64 (215040): 4.6 / 5.1.
         const int R = few || (!wide && d.stride_h == 2) ? 1 : !wide && p.oh % 4 == 0 && rows >= 1000000 ? 4 : 2;
-        Dw3Args b;
+        Dw3Args<FastDiv> b;
         b.src = src; b.flt = flt; b.bias = bias; b.z = z; b.dst = dst;
         b.CG = a.CG; b.IH = a.IH; b.IW = a.IW; b.OH = a.OH; b.OW = a.OW; b.QW = a.QW; b.OHS = (a.OH + R - 1) / R;
         b.ph = a.ph; b.pw = a.pw;
@@ -632,16 +724,17 @@ int launch_conv_depthwise(hipStream_t st, const ConvProblem& p, int cu_count, co
             b.div_qw = make_fastdiv(b.QW); b.div_ohs = make_fastdiv(b.OHS); b.div_cg = make_fastdiv(b.CG);
             // workgroups of one wave: waves share nothing, and a layer of a few hundred of them spreads over as many CUs
             // (7 x 7 x 960, batch 1: 2.64 us against 2.97 with four waves; batch 64: 4.6 against 4.8)
-            const dim3 grid((unsigned)((items + 63) / 64)), block(64);
+            b.grid = (unsigned)((items + 63) / 64);
+            const dim3 grid(b.grid), block(64);
             if (wide) {
-                auto kern = d.fh == 5 ? (d.stride_h == 1 ? (R == 1 ? dwf_kernel<5, 1, 1> : dwf_kernel<5, 1, 2>)
-                                                          : (R == 1 ? dwf_kernel<5, 2, 1> : dwf_kernel<5, 2, 2>))
-                                      : (d.stride_h == 1 ? (R == 1 ? dwf_kernel<7, 1, 1> : dwf_kernel<7, 1, 2>)
-                                                          : (R == 1 ? dwf_kernel<7, 2, 1> : dwf_kernel<7, 2, 2>));
-                return launch_kernel(kern, grid, block, 0, st, b);
+                auto launch = d.fh == 5 ? (d.stride_h == 1 ? (R == 1 ? launch_dwf<5, 1, 1> : launch_dwf<5, 1, 2>)
+                                                            : (R == 1 ? launch_dwf<5, 2, 1> : launch_dwf<5, 2, 2>))
+                                        : (d.stride_h == 1 ? (R == 1 ? launch_dwf<7, 1, 1> : launch_dwf<7, 1, 2>)
+                                                            : (R == 1 ? launch_dwf<7, 2, 1> : launch_dwf<7, 2, 2>));
+                return launch(st, grid, block, b, d.n);
             }
-            if (d.stride_h == 1) return R == 4 ? launch_dw3<1, 4>(st, grid, block, b) : R == 2 ? launch_dw3<1, 2>(st, grid, block, b) : launch_dw3<1, 1>(st, grid, block, b);
-            return launch_dw3<2, 1>(st, grid, block, b);
+            if (d.stride_h == 1) return R == 4 ? launch_dw3<1, 4>(st, grid, block, b, d.n) : R == 2 ? launch_dw3<1, 2>(st, grid, block, b, d.n) : launch_dw3<1, 1>(st, grid, block, b, d.n);
+            return launch_dw3<2, 1>(st, grid, block, b, d.n);
         }
     }
     const int quads = a.OH * a.QW;

@@ -15,7 +15,10 @@
 // is zero there.  Bound by the vector instructions: the requantisation of 8 values per lane and iteration and the set-up of
 // a workgroup (350 instructions per wave), not by the matrix instructions (5x5 stride 2, 240 channels at 57 x 57, batch 16:
 // 8.4 us, of which the copy rate accounts for 3.2; the byte dot products took 9.4).
+#include <tuple>
+
 #include "lds_copy.h"
+#include "wire.h"
 
 namespace mi355 {
 namespace {
@@ -35,6 +38,8 @@ SmallDiv small_div(uint32_t d, uint32_t most) {  // most < 32768
 __device__ __forceinline__ int sdiv(int x, const SmallDiv& d) { return (int)(__umul24((uint32_t)x, d.m) >> d.s); }
 __device__ __forceinline__ int mad24(int a, int b, int c) { return (int)(__umul24((uint32_t)a, (uint32_t)b) + (uint32_t)c); }
 
+// (Div: of the divisions that a workgroup needs once)
+template <class Div, class Small>
 struct DwmArgs {
     const int8_t* src;
     const int8_t* flt;
@@ -47,26 +52,100 @@ struct DwmArgs {
     int part;            // blocks of a patch row that lie together
     int QW, tab_w, tab, tab_at;  // quads of an output row; columns of the filter table and its entries (whole runs of 64), and where it starts
     int CG, bands, taps, has_bias;
+    uint32_t grid;
     int64_t src_sn, dst_sn, z_sn;
-    FastDiv div_bands, div_cg, div_tab;
-    SmallDiv div_qw, div_pw, div_nb, div_part, div_sw;
+    Div div_bands, div_cg, div_tab;
+    SmallDiv div_qw;
+    Small div_pw, div_nb, div_part, div_sw;
     EpiParams epi;
+
+    auto numbers() const {
+        return std::tie(IH, IW, OH, OW, FH, FW, sh, sw, ph, pw, TH, PH, PW, NB, rpw, waves, part, QW, tab_w, tab, tab_at, CG, bands, taps, has_bias, grid,
+                        src_sn, dst_sn, z_sn, div_qw.m, div_qw.s);
+    }
+};
+__device__ __forceinline__ int sdiv(int x, const Quot& d) { return (int)fdiv((uint32_t)x, d); }
+
+// The two forms of the kernel's argument (see wire.h)
+struct DwmWide {
+    DwmArgs<FastDiv, SmallDiv> a;
+    __device__ __forceinline__ DwmArgs<FastDiv, SmallDiv> open() const {
+        asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.IH), "s"(a.IW), "s"(a.OH), "s"(a.OW), "s"(a.FH), "s"(a.FW),
+                     "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.TH), "s"(a.PH), "s"(a.PW), "s"(a.NB), "s"(a.rpw), "s"(a.waves), "s"(a.part),
+                     "s"(a.CG), "s"(a.bands), "s"(a.grid));
+        asm volatile("" ::"s"(a.taps), "s"(a.has_bias), "s"(a.src_sn), "s"(a.dst_sn), "s"(a.z_sn), "s"(a.QW), "s"(a.tab_w), "s"(a.tab), "s"(a.tab_at),
+                     "s"(a.div_bands.m), "s"(a.div_cg.m), "s"(a.div_tab.m), "s"(a.div_qw.m), "s"(a.div_pw.m), "s"(a.div_nb.m), "s"(a.epi.s_b),
+                     "s"(a.epi.lin_lo));
+        return a;
+    }
 };
 
-template <int STEPS, bool HZ>
-__global__ __launch_bounds__(256) void dwm_kernel(DwmArgs a) {
+struct DwmWire {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    // in, out: height | width << 16; window: its height, width, strides; pads: padding, rows per copy, waves; bands: output rows of a
+    // band | bands << 16; more: channel blocks | entries of the filter table << 16; qw: its SmallDiv; part: blocks of a row together
+    uint32_t grid, in, out, window, pads, bands, more, qw, part, flags;
+    EpiWire epi;
+
+    template <class Div, class Small>
+    __host__ __device__ __forceinline__ void numbers(DwmArgs<Div, Small>& k) const {
+        k.IH = wire_lo(in); k.IW = wire_hi(in); k.OH = wire_lo(out); k.OW = wire_hi(out);
+        k.FH = wire_byte(window, 0); k.FW = wire_byte(window, 1); k.sh = wire_byte(window, 2); k.sw = wire_byte(window, 3);
+        k.ph = wire_byte(pads, 0); k.pw = wire_byte(pads, 1); k.rpw = wire_byte(pads, 2); k.waves = wire_byte(pads, 3);
+        k.TH = wire_lo(bands); k.bands = wire_hi(bands);
+        k.CG = wire_lo(more); k.tab = wire_hi(more);
+        k.part = (int)part; k.PW = wire_mul(k.part, 4, k.sw);
+        k.PH = (k.TH - 1) * k.sh + k.FH;
+        k.NB = (3 * k.sw + k.FW + 3) / 4;
+        k.tab_w = k.NB * 4 + 3 * k.sw; k.tab_at = k.PH * k.PW + k.NB * 4;
+        k.QW = (k.OW + 3) / 4;
+        k.taps = k.FH * k.FW;
+        k.has_bias = (int)(flags >> 8 & 1);
+        k.grid = grid;
+        k.src_sn = (uint32_t)wire_mul(k.CG, k.IH, k.IW * 4); k.dst_sn = (uint32_t)wire_mul(k.CG, k.OH, k.OW * 4);
+        k.z_sn = (flags >> 3 & 1) ? k.dst_sn : 0;
+        k.div_qw.m = qw & 0xffffff; k.div_qw.s = qw >> 24;
+    }
+    __device__ __forceinline__ DwmArgs<Quot, Quot> open() const {
+        asm volatile("" ::"s"(src), "s"(flt), "s"(bias), "s"(z), "s"(dst), "s"(grid), "s"(in), "s"(out), "s"(window), "s"(pads), "s"(bands), "s"(more),
+                     "s"(qw), "s"(part), "s"(flags), "s"(epi.f[0]), "s"(epi.f[1]), "s"(epi.f[2]), "s"(epi.f[3]));  // one batch of scalar loads
+        DwmArgs<Quot, Quot> k;
+        k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
+        numbers(k);
+        k.div_bands = quot(k.bands); k.div_cg = quot(k.CG); k.div_tab = quot(k.tab_w);
+        k.div_pw = quot(k.PW); k.div_nb = quot(k.NB); k.div_part = quot(k.part); k.div_sw = quot(k.sw);
+        k.epi = epi_open(epi, flags & 255);
+        return k;
+    }
+    // false: the problem has a number that does not fit
+    bool pack(const DwmArgs<FastDiv, SmallDiv>& k) {
+        src = k.src; flt = k.flt; bias = k.bias; z = k.z; dst = k.dst;
+        grid = k.grid; in = wire2(k.IH, k.IW); out = wire2(k.OH, k.OW);
+        window = wire4(k.FH, k.FW, k.sh, k.sw); pads = wire4(k.ph, k.pw, k.rpw, k.waves);
+        bands = wire2(k.TH, k.bands); more = wire2(k.CG, k.tab);
+        qw = k.div_qw.m | k.div_qw.s << 24; part = (uint32_t)k.part;
+        flags = epi_wire(k.epi, false, &epi) | (k.has_bias ? 1u << 8 : 0);
+        DwmArgs<FastDiv, SmallDiv> o;
+        numbers(o);
+        if (!k.epi.has_z) o.z_sn = k.z_sn;  // (nothing reads it)
+        return o.numbers() == k.numbers() && grid < QUOT_MAX;
+    }
+};
+static_assert(sizeof(DwmWire) <= WIRE_BYTES, "a wire");
+
+template <int STEPS, bool HZ, class Form>
+__device__ __forceinline__ void dwm_run(const Form& form) {
     extern __shared__ __attribute__((aligned(16))) v4i lds_dwm[];  // patch, filter table
-    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.IH), "s"(a.IW), "s"(a.OH), "s"(a.OW), "s"(a.FH), "s"(a.FW),
-                 "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.TH), "s"(a.PH), "s"(a.PW), "s"(a.NB), "s"(a.rpw), "s"(a.waves), "s"(a.part),
-                 "s"(a.CG), "s"(a.bands));
-    asm volatile("" ::"s"(a.taps), "s"(a.has_bias), "s"(a.src_sn), "s"(a.dst_sn), "s"(a.z_sn), "s"(a.QW), "s"(a.tab_w), "s"(a.tab), "s"(a.tab_at),
-                 "s"(a.div_bands.m), "s"(a.div_cg.m), "s"(a.div_tab.m), "s"(a.div_qw.m), "s"(a.div_pw.m), "s"(a.div_nb.m), "s"(a.epi.s_b),
-                 "s"(a.epi.lin_lo));
+    const auto a = form.open();
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int l16 = lane & 15, kq = lane >> 4;
-    const uint32_t item = xcd_block();
-    const uint32_t i1 = fdiv(item, a.div_bands), band = item - i1 * a.bands;
-    const uint32_t n = fdiv(i1, a.div_cg), cg = i1 - n * a.CG;
+    const uint32_t item = xcd_block(a.grid);
+    const uint32_t i1 = fdiv_u(item, a.div_bands), band = item - i1 * a.bands;
+    const uint32_t n = fdiv_u(i1, a.div_cg), cg = i1 - n * a.CG;
     const int oh0 = (int)band * a.TH, th = a.OH - oh0 < a.TH ? a.OH - oh0 : a.TH;
     const int plane = a.IH * a.IW * 4, oplane = a.OH * a.OW * 4;
     const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)lds_dwm);
@@ -170,9 +249,26 @@ __global__ __launch_bounds__(256) void dwm_kernel(DwmArgs a) {
     }
 }
 
+template <int STEPS, bool HZ>
+__global__ __launch_bounds__(256) void dwm_kernel(DwmWire a) {
+    dwm_run<STEPS, HZ>(a);
+}
+template <int STEPS, bool HZ>
+__global__ __launch_bounds__(256) void dwm_kernel(DwmWide a) {
+    dwm_run<STEPS, HZ>(a);
+}
+
+template <int STEPS, class Form>
+int launch_form(hipStream_t st, dim3 grid, dim3 block, int lds, const Form& form, bool hz) {
+    typedef void (*Kernel)(Form);
+    return launch_kernel(hz ? (Kernel)dwm_kernel<STEPS, true> : (Kernel)dwm_kernel<STEPS, false>, grid, block, lds, st, form);
+}
 template <int STEPS>
-int launch_steps(hipStream_t st, dim3 grid, dim3 block, int lds, const DwmArgs& a, bool hz) {
-    return hz ? launch_kernel((dwm_kernel<STEPS, true>), grid, block, lds, st, a) : launch_kernel((dwm_kernel<STEPS, false>), grid, block, lds, st, a);
+int launch_steps(hipStream_t st, dim3 grid, dim3 block, int lds, const DwmArgs<FastDiv, SmallDiv>& a, bool hz) {
+    // Up to four workgroups per CU; beyond, opening the wire in each of them costs more than the launch gains (5x5, 1132 channels at 73 x 5,
+    // batch 28, 7924 workgroups, as graph replays: 21.3 us wide, 22.7 so)
+    DwmWire wire;
+    return a.grid <= 1024 && wire.pack(a) ? launch_form<STEPS>(st, grid, block, lds, wire, hz) : launch_form<STEPS>(st, grid, block, lds, DwmWide{a}, hz);
 }
 
 int dwm_blocks(const ConvProblem& p) { return (3 * p.d.stride_w + (int)p.d.fw + 3) / 4; }
@@ -213,7 +309,7 @@ DwmBands dwm_bands(const ConvProblem& p) {
 int launch_dwm(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                int8_t* dst) {
     const mi355_conv_desc& d = p.d;
-    DwmArgs a;
+    DwmArgs<FastDiv, SmallDiv> a;
     a.src = src; a.flt = flt; a.bias = bias; a.z = z; a.dst = dst;
     a.IH = d.ih; a.IW = d.iw; a.OH = p.oh; a.OW = p.ow; a.FH = d.fh; a.FW = d.fw; a.sh = d.stride_h; a.sw = d.stride_w;
     a.ph = d.pad_h; a.pw = d.pad_w;
@@ -233,6 +329,7 @@ int launch_dwm(hipStream_t st, const ConvProblem& p, const int8_t* src, const in
     a.epi = p.epi;
     const int64_t items = (int64_t)d.n * a.CG * a.bands;
     if (items > 0x7fffffff) return (int)hipErrorInvalidValue;
+    a.grid = (uint32_t)items;
     const int lds = (a.tab_at + a.tab) * 4;
     const dim3 grid((unsigned)items), block(64 * a.waves);
     switch (steps) {

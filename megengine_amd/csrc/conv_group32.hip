@@ -14,8 +14,10 @@
 // 8 groups of 32 at 46 x 28, batch 23, residual: 23.0 us on the second-generation tiles, 9.5 here (floor 6.3); more at grp32_pick.
 // A dense layer over 32 or 64 channels is one group.
 #include <atomic>
+#include <tuple>
 
 #include "igemm_shared.h"
+#include "wire.h"
 
 namespace mi355 {
 namespace {
@@ -23,6 +25,7 @@ namespace {
 constexpr int G32_BMP(int mt) { return mt * 32 + 1; }             // odd: consecutive pieces of a filter row land on other banks
 constexpr int G32_NPV(int kb) { return kb == 1 ? 10 : 6; }        // patch vectors per thread and channel block
 
+template <class Div>
 struct G32Args {
     const int8_t* src;
     const int8_t* flt;
@@ -34,12 +37,97 @@ struct G32Args {
     int src_sn, src_scb, src_sg, dst_sn, dst_scb, z_sn, has_bias;
     int NI, TH, TW, PWC, PXI, PX, PXP, pkn;   // images, rows, columns of a tile; patch columns, pixels per image, pixels, plane pitch
     int tiles_m, tiles_mg, tiles_n, tiles_img, tiles_w;  // channel tiles: of all groups, of one
-    FastDiv div_tiles_m, div_tiles_mg, div_tiles_img, div_tiles_w, div_tw, div_tile_px, div_pxi, div_pwc;
+    Div div_tiles_m, div_tiles_mg, div_tiles_img, div_tiles_w, div_tw, div_tile_px, div_pxi, div_pwc;
     EpiParams epi;
+
+    auto numbers() const {
+        return std::tie(src_bytes, flt_bytes, z_bytes, dst_bytes, IH, IW, OH, OW, sh, sw, ph, pw, N, OC, ocpg, flt_rstride, flt_kstride, src_sn, src_scb,
+                        src_sg, dst_sn, dst_scb, z_sn, has_bias, NI, TH, TW, PWC, PXI, PX, PXP, pkn, tiles_m, tiles_mg, tiles_n, tiles_img, tiles_w);
+    }
 };
 
-template <int MT, int NT, int NL, bool HZ>
-__device__ __forceinline__ void g32_epilogue(const G32Args& a, v16i (&acc)[MT][NT], const v4i (&zv)[NT][MT], const int (&d_px)[NT], int oc0, int oc_end) {
+constexpr int g32_pitch(int px) { return ((px + 3) & ~7) + 4; }  // 4 mod 8: the two halves of a pixel on different banks
+
+// The two forms of the kernel's argument (see wire.h)
+struct G32Wide {
+    G32Args<FastDiv> a;
+    // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
+    template <int KB, int MT>
+    __device__ __forceinline__ G32Args<FastDiv> open() const {
+        asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.z_bytes), "s"(a.IH),
+                     "s"(a.IW), "s"(a.OH), "s"(a.OW), "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.N), "s"(a.OC), "s"(a.ocpg), "s"(a.flt_rstride), "s"(a.flt_kstride));
+        asm volatile("" ::"s"(a.src_sn), "s"(a.src_scb), "s"(a.src_sg), "s"(a.dst_sn), "s"(a.z_sn), "s"(a.NI), "s"(a.TH), "s"(a.TW), "s"(a.PWC),
+                     "s"(a.PX), "s"(a.PXP), "s"(a.pkn), "s"(a.tiles_m), "s"(a.tiles_mg), "s"(a.tiles_n), "s"(a.tiles_img), "s"(a.tiles_w),
+                     "s"(a.div_pxi.m), "s"(a.div_pwc.m), "s"(a.div_tw.m), "s"(a.div_tile_px.m), "s"(a.epi.s_b), "s"(a.epi.lin_lo));
+        return a;
+    }
+};
+
+struct G32Wire {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    // in, out: height | width << 16; window: strides, padding; channels: out of a group | groups << 16; tile: images, rows, columns of
+    // one, ten bits each; tiles: of an image, down | across << 16
+    uint32_t images, in, out, window, channels, kstride, tile, tiles, all_tiles, flags;
+    EpiWire epi;
+
+    template <int KB, int MT, class Div>
+    __host__ __device__ __forceinline__ void numbers(G32Args<Div>& k) const {
+        k.N = (int)images;
+        k.IH = wire_lo(in); k.IW = wire_hi(in); k.OH = wire_lo(out); k.OW = wire_hi(out);
+        k.sh = wire_byte(window, 0); k.sw = wire_byte(window, 1); k.ph = wire_byte(window, 2); k.pw = wire_byte(window, 3);
+        k.ocpg = wire_lo(channels);
+        const int groups = wire_hi(channels);
+        k.OC = wire_mul(k.ocpg, groups);
+        k.src_scb = wire_mul(k.IH, k.IW, 32); k.src_sg = wire_mul(k.src_scb, KB); k.src_sn = wire_mul(k.src_sg, groups);
+        k.dst_scb = wire_mul(k.OH, k.OW, 32); k.dst_sn = wire_mul(k.OC / 32, k.dst_scb);
+        k.z_sn = (flags >> 3 & 1) ? k.dst_sn : 0;
+        k.src_bytes = images * (uint32_t)k.src_sn; k.dst_bytes = images * (uint32_t)k.dst_sn; k.z_bytes = images * (uint32_t)k.z_sn;
+        const bool pre = (flags >> 9 & 1) != 0;  // [32-byte chunk][channel] instead of rows
+        k.flt_kstride = (int)kstride; k.flt_rstride = pre ? 32 : KB * 288;
+        k.flt_bytes = pre ? KB * 9 * kstride : (uint32_t)k.OC * (KB * 288);
+        k.has_bias = (int)(flags >> 8 & 1);
+        k.NI = (int)(tile & 1023); k.TH = (int)(tile >> 10 & 1023); k.TW = (int)(tile >> 20 & 1023);
+        k.PWC = (k.TW - 1) * k.sw + 3;
+        k.PXI = ((k.TH - 1) * k.sh + 3) * k.PWC;
+        k.PX = k.NI * k.PXI; k.PXP = g32_pitch(k.PX); k.pkn = (2 * k.PX + 255) / 256;
+        k.tiles_mg = (k.ocpg + MT * 32 - 1) / (MT * 32); k.tiles_m = k.tiles_mg * groups;
+        k.tiles_w = wire_hi(tiles); k.tiles_img = wire_mul(wire_lo(tiles), k.tiles_w); k.tiles_n = (int)all_tiles;
+    }
+    template <int KB, int MT>
+    __device__ __forceinline__ G32Args<Quot> open() const {
+        asm volatile("" ::"s"(src), "s"(flt), "s"(bias), "s"(z), "s"(dst), "s"(images), "s"(in), "s"(out), "s"(window), "s"(channels), "s"(kstride),
+                     "s"(tile), "s"(tiles), "s"(all_tiles), "s"(flags), "s"(epi.f[0]), "s"(epi.f[1]), "s"(epi.f[2]), "s"(epi.f[3]));  // one batch of scalar loads
+        G32Args<Quot> k;
+        k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
+        numbers<KB, MT>(k);
+        k.div_tiles_m = quot(k.tiles_m); k.div_tiles_mg = quot(k.tiles_mg); k.div_tiles_img = quot(k.tiles_img); k.div_tiles_w = quot(k.tiles_w);
+        k.div_tw = quot(k.TW); k.div_tile_px = quot(k.TH * k.TW); k.div_pxi = quot(k.PXI); k.div_pwc = quot(k.PWC);
+        k.epi = epi_open(epi, flags & 255);
+        return k;
+    }
+    // false: the problem has a number that does not fit
+    template <int KB, int MT>
+    bool pack(const G32Args<FastDiv>& k, uint32_t groups) {
+        src = k.src; flt = k.flt; bias = k.bias; z = k.z; dst = k.dst;
+        images = (uint32_t)k.N; in = wire2(k.IH, k.IW); out = wire2(k.OH, k.OW); window = wire4(k.sh, k.sw, k.ph, k.pw);
+        channels = wire2(k.ocpg, groups); kstride = (uint32_t)k.flt_kstride;
+        tile = (uint32_t)k.NI | (uint32_t)k.TH << 10 | (uint32_t)k.TW << 20;
+        tiles = wire2(k.tiles_img / k.tiles_w, k.tiles_w); all_tiles = (uint32_t)k.tiles_n;
+        flags = epi_wire(k.epi, false, &epi) | (k.has_bias ? 1u << 8 : 0) | (k.flt_rstride != KB * 288 ? 1u << 9 : 0);
+        G32Args<FastDiv> o;
+        numbers<KB, MT>(o);
+        if (!k.epi.has_z) o.z_sn = k.z_sn;  // (nothing reads it)
+        return o.numbers() == k.numbers() && (int64_t)(k.tiles_n + 8) * k.tiles_m < QUOT_MAX;
+    }
+};
+static_assert(sizeof(G32Wire) <= WIRE_BYTES, "a wire");
+
+template <int MT, int NT, int NL, bool HZ, class Args>
+__device__ __forceinline__ void g32_epilogue(const Args& a, v16i (&acc)[MT][NT], const v4i (&zv)[NT][MT], const int (&d_px)[NT], int oc0, int oc_end) {
     const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes);
 #pragma unroll
     for (int j = 0; j < NT; ++j)
@@ -66,33 +154,28 @@ __device__ __forceinline__ void g32_epilogue(const G32Args& a, v16i (&acc)[MT][N
         }
 }
 
-template <int KB, int MT, int NT>
-__global__ __launch_bounds__(256, 2) void grp32_kernel(G32Args a) {
+template <int KB, int MT, int NT, class Form>
+__device__ __forceinline__ void grp32_run(const Form& form) {
     constexpr int BM = MT * 32, BMP = G32_BMP(MT), STEPS = 9 * KB, PIECES = 2 * STEPS, NPV = G32_NPV(KB);
     constexpr int NFV = (BM * PIECES + 255) / 256;
     constexpr int A_VECS = PIECES * BMP;
     extern __shared__ __attribute__((aligned(16))) v4i lds[];
-    // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
-    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.z_bytes), "s"(a.IH),
-                 "s"(a.IW), "s"(a.OH), "s"(a.OW), "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.N), "s"(a.OC), "s"(a.ocpg), "s"(a.flt_rstride), "s"(a.flt_kstride));
-    asm volatile("" ::"s"(a.src_sn), "s"(a.src_scb), "s"(a.src_sg), "s"(a.dst_sn), "s"(a.z_sn), "s"(a.NI), "s"(a.TH), "s"(a.TW), "s"(a.PWC),
-                 "s"(a.PX), "s"(a.PXP), "s"(a.pkn), "s"(a.tiles_m), "s"(a.tiles_mg), "s"(a.tiles_n), "s"(a.tiles_img), "s"(a.tiles_w),
-                 "s"(a.div_pxi.m), "s"(a.div_pwc.m), "s"(a.div_tw.m), "s"(a.div_tile_px.m), "s"(a.epi.s_b), "s"(a.epi.lin_lo));
+    const auto a = form.template open<KB, MT>();
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l32 = lane & 31, lh = lane >> 5;
 
     // tile: contiguous pixel tiles per XCD (workgroup b runs on XCD b % 8), the groups of a pixel tile side by side
     int tm, tn;
     {
         const int per = (a.tiles_n + 7) >> 3, x = blockIdx.x & 7, i = blockIdx.x >> 3;
-        const int r = (int)fdiv(i, a.div_tiles_m);
+        const int r = (int)fdiv_u(i, a.div_tiles_m);
         tm = i - r * a.tiles_m;
         tn = x * per + r;
         if (r >= per || tn >= a.tiles_n) return;
     }
-    const int ig = (int)fdiv(tn, a.div_tiles_img), ti = tn - ig * a.tiles_img;
-    const int th = (int)fdiv(ti, a.div_tiles_w), tw = ti - th * a.tiles_w;
+    const int ig = (int)fdiv_u(tn, a.div_tiles_img), ti = tn - ig * a.tiles_img;
+    const int th = (int)fdiv_u(ti, a.div_tiles_w), tw = ti - th * a.tiles_w;
     const int n0 = ig * a.NI, oh0 = th * a.TH, ow0 = tw * a.TW;
-    const int grp = (int)fdiv(tm, a.div_tiles_mg), oc0 = grp * a.ocpg + (tm - grp * a.tiles_mg) * BM, oc_end = (grp + 1) * a.ocpg;
+    const int grp = (int)fdiv_u(tm, a.div_tiles_mg), oc0 = grp * a.ocpg + (tm - grp * a.tiles_mg) * BM, oc_end = (grp + 1) * a.ocpg;
     const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes), rs_flt = make_rsrc(a.flt, a.flt_bytes);
     const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0), rs_z = make_rsrc(a.z, a.epi.has_z ? a.z_bytes : 0);
 
@@ -205,6 +288,15 @@ __global__ __launch_bounds__(256, 2) void grp32_kernel(G32Args a) {
 #undef MI355_G32
 }
 
+template <int KB, int MT, int NT>
+__global__ __launch_bounds__(256, 2) void grp32_kernel(G32Wire a) {
+    grp32_run<KB, MT, NT>(a);
+}
+template <int KB, int MT, int NT>
+__global__ __launch_bounds__(256, 2) void grp32_kernel(G32Wide a) {
+    grp32_run<KB, MT, NT>(a);
+}
+
 struct G32Cfg {
     int mt, nt;
     const char* name;
@@ -213,7 +305,7 @@ constexpr G32Cfg kG32[] = {{1, 1, "v2_patch_32x128"}, {1, 2, "v2_patch_32x256"},
 constexpr int kG32Count = sizeof(kG32) / sizeof(kG32[0]);
 
 // geometry of a tile; false where no patch fits
-bool g32_plan(const IgemmArgs& a, int cfg, G32Args* k, int* lds_bytes) {
+bool g32_plan(const IgemmArgs& a, int cfg, G32Args<FastDiv>* k, int* lds_bytes) {
     const int kb = a.kbytes / 288, mt = kG32[cfg].mt, bm = mt * 32, bn = kG32[cfg].nt * 128, max_px = G32_NPV(kb) * 128;
     int64_t best = -1;
     // equal columns, as wide as a tile or narrower (nothing is gained below 8), and as many rows, or whole images, as fit
@@ -250,7 +342,7 @@ bool g32_plan(const IgemmArgs& a, int cfg, G32Args* k, int* lds_bytes) {
         }
     }
     if (best < 0) return false;
-    k->PXP = ((k->PX + 3) & ~7) + 4;  // 4 mod 8: the two halves of a pixel on different banks
+    k->PXP = g32_pitch(k->PX);
     k->pkn = (2 * k->PX + 255) / 256;
     k->tiles_mg = (a.ocpg + bm - 1) / bm;
     k->tiles_m = k->tiles_mg * a.groups;
@@ -259,26 +351,35 @@ bool g32_plan(const IgemmArgs& a, int cfg, G32Args* k, int* lds_bytes) {
     return *lds_bytes <= 80 * 1024;
 }
 
-template <int KB, int MT, int NT>
-int launch_g32(hipStream_t st, const G32Args& k, int lds) {
-    auto kern = grp32_kernel<KB, MT, NT>;
+template <int KB, int MT, int NT, class Form>
+int launch_g32_form(hipStream_t st, const Form& form, unsigned grid, int lds) {
+    void (*const kern)(Form) = grp32_kernel<KB, MT, NT>;
     static std::atomic<int> max_lds_set{0};
     if (max_lds_set.load(std::memory_order_relaxed) == 0) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
         if (e != hipSuccess) return (int)e;
         max_lds_set.store(1, std::memory_order_relaxed);
     }
+    return launch_kernel(kern, dim3(grid), dim3(256), lds, st, form);
+}
+
+template <int KB, int MT, int NT>
+int launch_g32(hipStream_t st, const G32Args<FastDiv>& k, int groups, int lds) {
     const int64_t grid = (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
-    return launch_kernel(kern, dim3((unsigned)grid), dim3(256), lds, st, k);
+    G32Wire wire;
+    // Up to a workgroup per CU the launch is what a call costs.  Beyond, a workgroup's start is, which opening the wire makes longer (2 groups
+    // of 64 at 24 x 27, batch 17, residual, 384 workgroups, as graph replays: 4.42 us wide, 4.81 so).
+    if (grid <= 256 && wire.pack<KB, MT>(k, (uint32_t)groups)) return launch_g32_form<KB, MT, NT>(st, wire, (unsigned)grid, lds);
+    return launch_g32_form<KB, MT, NT>(st, G32Wide{k}, (unsigned)grid, lds);
 }
 
 template <int KB>
-int launch_g32_tile(hipStream_t st, const G32Args& k, int cfg, int lds) {
+int launch_g32_tile(hipStream_t st, const G32Args<FastDiv>& k, int cfg, int groups, int lds) {
     switch (cfg) {
-        case 0: return launch_g32<KB, 1, 1>(st, k, lds);
-        case 1: return launch_g32<KB, 1, 2>(st, k, lds);
-        case 2: return launch_g32<KB, 2, 1>(st, k, lds);
-        default: return launch_g32<KB, 2, 2>(st, k, lds);
+        case 0: return launch_g32<KB, 1, 1>(st, k, groups, lds);
+        case 1: return launch_g32<KB, 1, 2>(st, k, groups, lds);
+        case 2: return launch_g32<KB, 2, 1>(st, k, groups, lds);
+        default: return launch_g32<KB, 2, 2>(st, k, groups, lds);
     }
 }
 
@@ -291,7 +392,7 @@ bool grp32_can_run(const IgemmArgs& a, int pin, int pout, int cfg) {
     if (cfg < 0 || cfg >= kG32Count || pin != 32 || pout != 32 || a.general || a.FH != 3 || a.FW != 3 || a.ocpg % 32 != 0) return false;
     if (a.kbytes != 288 && a.kbytes != 576) return false;
     if (kG32[cfg].mt == 2 && a.ocpg == 32) return false;
-    G32Args k;
+    G32Args<FastDiv> k;
     int lds;
     return g32_plan(a, cfg, &k, &lds);
 }
@@ -334,7 +435,7 @@ int grp32_pick(const IgemmArgs& a, int pin, int pout, bool will_preprocess) {
 }
 
 int launch_grp32(hipStream_t st, const IgemmArgs& a, int cfg) {
-    G32Args k;
+    G32Args<FastDiv> k;
     int lds;
     if (!g32_plan(a, cfg, &k, &lds)) return (int)hipErrorInvalidConfiguration;
     k.src = a.src; k.flt = a.flt; k.bias = a.bias; k.z = a.z; k.dst = a.dst;
@@ -348,7 +449,7 @@ int launch_grp32(hipStream_t st, const IgemmArgs& a, int cfg) {
     k.div_tw = make_fastdiv(k.TW); k.div_tile_px = make_fastdiv(k.TH * k.TW);
     k.div_pxi = make_fastdiv(k.PXI); k.div_pwc = make_fastdiv(k.PWC);
     k.epi = a.epi;
-    return a.kbytes == 288 ? launch_g32_tile<1>(st, k, cfg, lds) : launch_g32_tile<2>(st, k, cfg, lds);
+    return a.kbytes == 288 ? launch_g32_tile<1>(st, k, cfg, a.groups, lds) : launch_g32_tile<2>(st, k, cfg, a.groups, lds);
 }
 
 }  // namespace mi355

@@ -22,13 +22,17 @@
 // (51 MB): 50 us with dot products, 17 here.  Small layers are a chain: with the filter staged beside the first band instead of
 // gathered dword by dword ahead of it, and the next operands read while results are requantised, 55 groups of 16 at 8 x 47,
 // stride 2, batch 4 went from 6.2 to 4.2 us, 5 groups of 16 at 33 x 100, stride 2, batch 64 from 9.8 to 8.4.
+#include <tuple>
+
 #include "igemm_shared.h"
+#include "wire.h"
 
 namespace mi355 {
 namespace {
 
 constexpr int GRP4_MAX_IC = 16;  // beyond, a group is worth a matrix tile of its own
 
+template <class Div>
 struct Grp4Args {
     const int8_t* src;
     const int* flt;
@@ -39,18 +43,79 @@ struct Grp4Args {
     int icb, ocpg, src_scb, dst_scb, has_bias;
     int64_t src_sn, dst_sn, z_sn;
     uint32_t items;
-    FastDiv div_ow;
+    Div div_ow, div_ocpg;
     EpiParams epi;
+
+    auto numbers() const {
+        return std::tie(IH, IW, OH, OW, FH, FW, sh, sw, ph, pw, icb, ocpg, src_scb, dst_scb, has_bias, src_sn, dst_sn, z_sn, items);
+    }
 };
 
+// The two forms of the kernel's argument (see wire.h)
+struct Grp4Wide {
+    Grp4Args<FastDiv> a;
+    template <int R>
+    __device__ __forceinline__ const Grp4Args<FastDiv>& open() const { return a; }
+};
+
+struct Grp4Wire {
+    const int8_t* src;
+    const int* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    // in, out: height | width << 16; window: its height, width, strides; pads: padding, channel blocks into a group; channels: out of a
+    // group | groups << 16
+    uint32_t in, out, window, pads, channels, flags;
+    EpiWire epi;
+
+    template <int R, class Div>
+    __host__ __device__ __forceinline__ void numbers(Grp4Args<Div>& k) const {
+        k.IH = wire_lo(in); k.IW = wire_hi(in); k.OH = wire_lo(out); k.OW = wire_hi(out);
+        k.FH = wire_byte(window, 0); k.FW = wire_byte(window, 1); k.sh = wire_byte(window, 2); k.sw = wire_byte(window, 3);
+        k.ph = wire_byte(pads, 0); k.pw = wire_byte(pads, 1); k.icb = wire_byte(pads, 2);
+        k.ocpg = wire_lo(channels);
+        k.src_scb = wire_mul(k.IH, k.IW, 4); k.dst_scb = wire_mul(k.OH, k.OW, 4);
+        k.src_sn = (uint32_t)wire_mul(wire_hi(channels), k.icb, k.src_scb);
+        k.dst_sn = (uint32_t)wire_mul(wire_hi(channels), k.ocpg / 4, k.dst_scb);
+        k.z_sn = (flags >> 3 & 1) ? k.dst_sn : 0;
+        k.items = (uint32_t)wire_mul((k.OH + R - 1) / R, k.OW);
+        k.has_bias = (int)(flags >> 8 & 1);
+    }
+    template <int R>
+    __device__ __forceinline__ Grp4Args<Quot> open() const {
+        // (no asm statement to batch the loads: behind one the filter's words are no scalar loads any more)
+        Grp4Args<Quot> k;
+        k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
+        numbers<R>(k);
+        k.div_ow = quot(k.OW); k.div_ocpg = quot(k.ocpg);
+        k.epi = epi_open(epi, flags & 255);
+        return k;
+    }
+    // false: the problem has a number that does not fit
+    template <int R>
+    bool pack(const Grp4Args<FastDiv>& k, uint32_t groups) {
+        src = k.src; flt = k.flt; bias = k.bias; z = k.z; dst = k.dst;
+        in = wire2(k.IH, k.IW); out = wire2(k.OH, k.OW);
+        window = wire4(k.FH, k.FW, k.sh, k.sw); pads = wire4(k.ph, k.pw, k.icb, 0); channels = wire2(k.ocpg, groups);
+        flags = epi_wire(k.epi, false, &epi) | (k.has_bias ? 1u << 8 : 0);
+        Grp4Args<FastDiv> o;
+        numbers<R>(o);
+        if (!k.epi.has_z) o.z_sn = k.z_sn;  // (nothing reads it)
+        return o.numbers() == k.numbers() && groups < 65536 && k.items < QUOT_MAX && (int64_t)groups * k.ocpg < QUOT_MAX;
+    }
+};
+static_assert(sizeof(Grp4Wire) <= WIRE_BYTES, "a wire");
+
 // OQ: output channel quads per thread; F = 3: 3x3 filter, stride ST, two output rows per thread; F = 0: any filter, one row
-template <int OQ, int F, int ST>
-__global__ __launch_bounds__(256) void grp4_kernel(Grp4Args a) {
+template <int OQ, int F, int ST, class Form>
+__device__ __forceinline__ void grp4_run(const Form& form) {
     constexpr int R = F == 3 ? 2 : 1;
+    const auto a = form.template open<R>();
     const uint32_t it = blockIdx.x * 256 + threadIdx.x;
     const bool live = it < a.items;
     const uint32_t ohs = fdiv(live ? it : 0, a.div_ow), ow = (live ? it : 0) - ohs * a.OW;
-    const int oh0 = (int)ohs * R, oc0 = blockIdx.y * OQ * 4, g = oc0 / a.ocpg;
+    const int oh0 = (int)ohs * R, oc0 = blockIdx.y * OQ * 4, g = (int)fdiv_u(oc0, a.div_ocpg);
     const int64_t n = blockIdx.z;
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.src + n * a.src_sn + (int64_t)g * a.icb * a.src_scb, (uint32_t)(a.icb * a.src_scb));
     const int ih0 = oh0 * a.sh - a.ph, iw0 = (int)ow * a.sw - a.pw;
@@ -116,8 +181,25 @@ __global__ __launch_bounds__(256) void grp4_kernel(Grp4Args a) {
         }
 }
 
+template <int OQ, int F, int ST>
+__global__ __launch_bounds__(256) void grp4_kernel(Grp4Wire a) {
+    grp4_run<OQ, F, ST>(a);
+}
+template <int OQ, int F, int ST>
+__global__ __launch_bounds__(256) void grp4_kernel(Grp4Wide a) {
+    grp4_run<OQ, F, ST>(a);
+}
+
+template <int OQ, int F, int ST>
+int launch_grp4_kernel(hipStream_t st, dim3 grid, const Grp4Args<FastDiv>& a, uint32_t groups) {
+    Grp4Wire wire;
+    if (wire.pack<F == 3 ? 2 : 1>(a, groups)) return launch_kernel((void (*)(Grp4Wire))grp4_kernel<OQ, F, ST>, grid, dim3(256), 0, st, wire);
+    return launch_kernel((void (*)(Grp4Wide))grp4_kernel<OQ, F, ST>, grid, dim3(256), 0, st, Grp4Wide{a});
+}
+
 constexpr int G16_PX = 1024;  // pixels of a staged band (16 KiB), four per thread
 
+template <class Div>
 struct G16Args {
     const int8_t* src;
     const int* flt;
@@ -129,24 +211,81 @@ struct G16Args {
     int log_icpg, src_scb, dst_scb, has_bias;
     int slabs, step;  // blocks of 16 channels; workgroups per slab
     int64_t src_sn, dst_sn, z_sn;
-    FastDiv div_pw, div_ow, div_bands;
+    Div div_pw, div_ow, div_bands;
     EpiParams epi;
+
+    auto numbers() const {
+        return std::tie(IH, IW, OH, OW, s, ph, pw, TH, PW, bands, items, log_icpg, src_scb, dst_scb, has_bias, slabs, step, src_sn, dst_sn, z_sn);
+    }
 };
 
-template <bool HZ>
-__global__ __launch_bounds__(256) void grp16_kernel(G16Args a) {
-    __shared__ __attribute__((aligned(16))) v4i sm[G16_PX], sf[144];
+struct G16Wide {
+    G16Args<FastDiv> a;
     // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
-    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.IH), "s"(a.IW), "s"(a.OH), "s"(a.OW), "s"(a.s), "s"(a.ph),
-                 "s"(a.pw), "s"(a.TH), "s"(a.PW), "s"(a.bands), "s"(a.items), "s"(a.log_icpg), "s"(a.src_scb), "s"(a.dst_scb), "s"(a.has_bias),
-                 "s"(a.slabs), "s"(a.src_sn), "s"(a.div_pw.m), "s"(a.div_bands.m), "s"(a.div_ow.m), "s"(a.epi.s_b), "s"(a.epi.lin_lo));
+    __device__ __forceinline__ G16Args<FastDiv> open() const {
+        asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.dst), "s"(a.IH), "s"(a.IW), "s"(a.OH), "s"(a.OW), "s"(a.s), "s"(a.ph),
+                     "s"(a.pw), "s"(a.TH), "s"(a.PW), "s"(a.bands), "s"(a.items), "s"(a.log_icpg), "s"(a.src_scb), "s"(a.dst_scb), "s"(a.has_bias),
+                     "s"(a.slabs), "s"(a.src_sn), "s"(a.div_pw.m), "s"(a.div_bands.m), "s"(a.div_ow.m), "s"(a.epi.s_b), "s"(a.epi.lin_lo));
+        return a;
+    }
+};
+
+struct G16Wire {
+    const int8_t* src;
+    const int* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    // in, out: height | width << 16; window: stride, padding, log of a group's channels; bands: output rows of one | slabs << 16
+    uint32_t N, in, out, window, bands, per_image, step, flags;
+    EpiWire epi;
+
+    template <class Div>
+    __host__ __device__ __forceinline__ void numbers(G16Args<Div>& k) const {
+        k.IH = wire_lo(in); k.IW = wire_hi(in); k.OH = wire_lo(out); k.OW = wire_hi(out);
+        k.s = wire_byte(window, 0); k.ph = wire_byte(window, 1); k.pw = wire_byte(window, 2); k.log_icpg = wire_byte(window, 3);
+        k.TH = wire_lo(bands); k.slabs = wire_hi(bands); k.PW = (k.OW - 1) * k.s + 3;
+        k.bands = (int)per_image; k.items = wire_mul((int)N, k.bands); k.step = (int)step;
+        k.src_scb = wire_mul(k.IH, k.IW, 4); k.dst_scb = wire_mul(k.OH, k.OW, 4);
+        k.src_sn = (uint32_t)wire_mul(k.slabs, 4, k.src_scb); k.dst_sn = (uint32_t)wire_mul(k.slabs, 4, k.dst_scb);
+        k.z_sn = (flags >> 3 & 1) ? k.dst_sn : 0;
+        k.has_bias = (int)(flags >> 8 & 1);
+    }
+    __device__ __forceinline__ G16Args<Quot> open() const {
+        asm volatile("" ::"s"(src), "s"(flt), "s"(bias), "s"(z), "s"(dst), "s"(N), "s"(in), "s"(out), "s"(window), "s"(bands), "s"(per_image), "s"(step),
+                     "s"(flags), "s"(epi.f[0]), "s"(epi.f[1]), "s"(epi.f[2]), "s"(epi.f[3]));  // one batch of scalar loads
+        G16Args<Quot> k;
+        k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
+        numbers(k);
+        k.div_pw = quot(k.PW); k.div_ow = quot(k.OW); k.div_bands = quot(k.bands);
+        k.epi = epi_open(epi, flags & 255);
+        return k;
+    }
+    // false: the problem has a number that does not fit
+    bool pack(const G16Args<FastDiv>& k, uint32_t n) {
+        src = k.src; flt = k.flt; bias = k.bias; z = k.z; dst = k.dst;
+        N = n; in = wire2(k.IH, k.IW); out = wire2(k.OH, k.OW); window = wire4(k.s, k.ph, k.pw, k.log_icpg);
+        bands = wire2(k.TH, k.slabs); per_image = (uint32_t)k.bands; step = (uint32_t)k.step;
+        flags = epi_wire(k.epi, false, &epi) | (k.has_bias ? 1u << 8 : 0);
+        G16Args<FastDiv> o;
+        numbers(o);
+        if (!k.epi.has_z) o.z_sn = k.z_sn;  // (nothing reads it)
+        return o.numbers() == k.numbers() && k.items < QUOT_MAX;
+    }
+};
+static_assert(sizeof(G16Wire) <= WIRE_BYTES, "a wire");
+
+template <bool HZ, class Form>
+__device__ __forceinline__ void grp16_run(const Form& form) {
+    __shared__ __attribute__((aligned(16))) v4i sm[G16_PX], sf[144];
+    const auto a = form.open();
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int l16 = lane & 15, kq = lane >> 4, slab = blockIdx.y;
     const int PH = (a.TH - 1) * a.s + 3, patch = PH * a.PW;
 
     v4i x[G16_PX / 256];
     auto fetch = [&](int item) __attribute__((always_inline)) {
-        const int n = (int)fdiv(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
+        const int n = (int)fdiv_u(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
         const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.src + n * a.src_sn + (int64_t)slab * 4 * a.src_scb, (uint32_t)a.src_scb * 4);
 #pragma unroll
         for (int k = 0; k < G16_PX / 256; ++k) {
@@ -190,7 +329,7 @@ __global__ __launch_bounds__(256) void grp16_kernel(G16Args a) {
     for (;;) {
         const int next = item + a.step;
         if (next < a.items) fetch(next);  // lands during the multiplies
-        const int n = (int)fdiv(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
+        const int n = (int)fdiv_u(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
         const int pixels = (a.OH - oh0 < a.TH ? a.OH - oh0 : a.TH) * a.OW;
         const int64_t at = (int64_t)(slab * 4 + kq) * a.dst_scb + (int64_t)oh0 * a.OW * 4;
         int8_t* dst = a.dst + n * a.dst_sn + at;
@@ -239,6 +378,21 @@ __global__ __launch_bounds__(256) void grp16_kernel(G16Args a) {
     }
 }
 
+template <bool HZ>
+__global__ __launch_bounds__(256) void grp16_kernel(G16Wire a) {
+    grp16_run<HZ>(a);
+}
+template <bool HZ>
+__global__ __launch_bounds__(256) void grp16_kernel(G16Wide a) {
+    grp16_run<HZ>(a);
+}
+
+template <class Form>
+int launch_g16_form(hipStream_t st, dim3 grid, const Form& form, bool hz) {
+    typedef void (*Kernel)(Form);
+    return launch_kernel(hz ? (Kernel)grp16_kernel<true> : (Kernel)grp16_kernel<false>, grid, dim3(256), 0, st, form);
+}
+
 // output rows of a band: the largest number whose input patch fits; 0: not even one row fits
 int g16_rows(const ConvProblem& p) {
     const int s = p.d.stride_h, pw = ((int)p.ow - 1) * s + 3;
@@ -256,7 +410,7 @@ bool g16_usable(const ConvProblem& p) {
 int launch_g16(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                int8_t* dst) {
     const mi355_conv_desc& d = p.d;
-    G16Args a;
+    G16Args<FastDiv> a;
     a.src = src; a.flt = reinterpret_cast<const int*>(flt); a.bias = bias; a.z = z; a.dst = dst;
     a.IH = d.ih; a.IW = d.iw; a.OH = p.oh; a.OW = p.ow; a.s = d.stride_h; a.ph = d.pad_h; a.pw = d.pad_w;
     const int slabs = d.oc / 16;
@@ -284,7 +438,8 @@ int launch_g16(hipStream_t st, const ConvProblem& p, const int8_t* src, const in
     if (per_slab > items) per_slab = items;
     a.slabs = slabs; a.step = (int)per_slab;
     const dim3 grid((unsigned)per_slab, slabs);
-    return d.has_z ? launch_kernel(grp16_kernel<true>, grid, dim3(256), 0, st, a) : launch_kernel(grp16_kernel<false>, grid, dim3(256), 0, st, a);
+    G16Wire wire;
+    return wire.pack(a, d.n) ? launch_g16_form(st, grid, wire, d.has_z) : launch_g16_form(st, grid, G16Wide{a}, d.has_z);
 }
 
 }  // namespace
@@ -328,7 +483,7 @@ int launch_grp4(hipStream_t st, const ConvProblem& p, const int8_t* src, const i
     const mi355_conv_desc& d = p.d;
     if (d.n == 0 || p.oh == 0 || p.ow == 0) return 0;
     if (g16_usable(p)) return launch_g16(st, p, src, flt, bias, z, dst);
-    Grp4Args a;
+    Grp4Args<FastDiv> a;
     a.src = src; a.flt = reinterpret_cast<const int*>(flt); a.bias = bias; a.z = z; a.dst = dst;
     a.IH = d.ih; a.IW = d.iw; a.OH = p.oh; a.OW = p.ow; a.FH = d.fh; a.FW = d.fw;
     a.sh = d.stride_h; a.sw = d.stride_w; a.ph = d.pad_h; a.pw = d.pad_w;
@@ -336,15 +491,15 @@ int launch_grp4(hipStream_t st, const ConvProblem& p, const int8_t* src, const i
     a.src_scb = d.ih * d.iw * 4; a.dst_scb = p.oh * p.ow * 4;
     a.has_bias = d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL;
     a.src_sn = p.src_sn; a.dst_sn = p.dst_sn; a.z_sn = p.z_sn;
-    a.div_ow = make_fastdiv(p.ow);
+    a.div_ow = make_fastdiv(p.ow); a.div_ocpg = make_fastdiv(p.ocpg);
     a.epi = p.epi;
     const bool f3 = d.fh == 3 && d.fw == 3 && d.stride_h == d.stride_w && d.stride_h <= 2;
     const bool wide = p.ocpg % 8 == 0;  // 8 channels per thread halve the loads per output
     a.items = (f3 ? (p.oh + 1) / 2 : p.oh) * p.ow;
     const dim3 grid((a.items + 255) / 256, d.oc / (wide ? 8 : 4), d.n);
-    if (f3 && d.stride_h == 1) return wide ? launch_kernel(grp4_kernel<2, 3, 1>, grid, dim3(256), 0, st, a) : launch_kernel(grp4_kernel<1, 3, 1>, grid, dim3(256), 0, st, a);
-    if (f3) return wide ? launch_kernel(grp4_kernel<2, 3, 2>, grid, dim3(256), 0, st, a) : launch_kernel(grp4_kernel<1, 3, 2>, grid, dim3(256), 0, st, a);
-    return wide ? launch_kernel(grp4_kernel<2, 0, 1>, grid, dim3(256), 0, st, a) : launch_kernel(grp4_kernel<1, 0, 1>, grid, dim3(256), 0, st, a);
+    if (f3 && d.stride_h == 1) return wide ? launch_grp4_kernel<2, 3, 1>(st, grid, a, d.group) : launch_grp4_kernel<1, 3, 1>(st, grid, a, d.group);
+    if (f3) return wide ? launch_grp4_kernel<2, 3, 2>(st, grid, a, d.group) : launch_grp4_kernel<1, 3, 2>(st, grid, a, d.group);
+    return wide ? launch_grp4_kernel<2, 0, 1>(st, grid, a, d.group) : launch_grp4_kernel<1, 0, 1>(st, grid, a, d.group);
 }
 
 }  // namespace mi355

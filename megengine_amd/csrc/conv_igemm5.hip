@@ -19,8 +19,10 @@
 // 4-packed inputs: a lane's 16 k-bytes are four dwords of its pixel, one per (channel block, tap) unit of the filter's own
 // order; a table in LDS says where each unit lies.
 #include <atomic>
+#include <tuple>
 
 #include "igemm_shared.h"
+#include "wire.h"
 
 namespace mi355 {
 namespace {
@@ -32,6 +34,7 @@ constexpr int ks_ahead(int s, int mt) { return s == 16 ? 6 : mt == 1 ? 8 : 4; }
 // per pass
 constexpr int ks_row(int s) { return s == 32 ? 34 : 20; }
 
+template <class Div>
 struct KsArgs {
     const int8_t* src;
     const int8_t* flt;
@@ -46,11 +49,93 @@ struct KsArgs {
     int flt_rstride, flt_kstride;
     int tiles_m, tiles_n, by_m;
     int FH, steps, per_wave, extra;  // steps of the reduction: per_wave for every wave, one more for the first `extra`
-    FastDiv div_tile;                // by tiles_n (by_m) or tiles_m
     int log_pout, has_bias, dst_s32;
-    FastDiv div_ohw, div_ow, div_t, div_fw;
+    Div div_tile;                    // by tiles_n (by_m) or tiles_m
+    Div div_ohw, div_ow, div_t, div_fw;
     EpiParams epi;
+
+    auto numbers() const {
+        return std::tie(src_bytes, flt_bytes, z_bytes, dst_bytes, IH, IW, OHW, OW, FW, T, sh, sw, ph, pw, OC, M, KC, entries, src_sn, src_scb,
+                        dst_sn, dst_scb, z_sn, flt_rstride, flt_kstride, tiles_m, tiles_n, by_m, FH, steps, per_wave, extra, log_pout, has_bias,
+                        dst_s32);
+    }
 };
+
+// The two forms of the kernel's argument (see wire.h)
+struct KsWide {
+    static constexpr bool WIRE = false;
+    KsArgs<FastDiv> a;
+    template <int PIN, int S, int MT, int W>
+    __device__ __forceinline__ KsArgs<FastDiv> open() const { return a; }
+};
+
+struct KsWire {
+    static constexpr bool WIRE = true;
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    uint32_t N, in, out, channels, window, flags, kstride;  // in, out: height | width << 16; channels: out | blocks in << 16
+    EpiWire epi;
+
+    template <int PIN, int S, int MT, int W, class Div>
+    __host__ __device__ __forceinline__ void numbers(KsArgs<Div>& k) const {
+        k.IH = wire_lo(in); k.IW = wire_hi(in);
+        k.OW = wire_hi(out); k.OHW = wire_mul(wire_lo(out), k.OW);
+        k.sh = wire_byte(window, 0); k.sw = wire_byte(window, 1); k.ph = wire_byte(window, 2); k.pw = wire_byte(window, 3);
+        k.FH = wire_byte(flags, 2); k.FW = wire_byte(flags, 3); k.T = k.FH * k.FW;
+        k.OC = wire_lo(channels);
+        k.M = wire_mul((int)N, k.OHW);
+        k.entries = wire_mul(wire_hi(channels), k.T);
+        k.KC = PIN == 32 ? k.entries : (k.entries + 7) / 8;
+        k.src_scb = wire_mul(k.IH, k.IW, PIN); k.src_sn = wire_mul(wire_hi(channels), k.src_scb);
+        k.log_pout = (int)(flags >> 8 & 7); k.has_bias = (int)(flags >> 11 & 1); k.dst_s32 = (int)(flags >> 12 & 1);
+        k.dst_scb = wire_mul(k.OHW, 1 << k.log_pout); k.dst_sn = wire_mul(k.OC, k.OHW);
+        k.z_sn = (flags >> 3 & 1) ? k.dst_sn : 0;
+        const uint32_t el = k.dst_s32 ? 4 : 1;
+        k.src_bytes = N * (uint32_t)k.src_sn; k.dst_bytes = N * (uint32_t)k.dst_sn * el; k.z_bytes = N * (uint32_t)k.z_sn * el;
+        const bool pre = (flags >> 13 & 1) != 0;  // [32-byte chunk][channel] instead of rows
+        k.flt_kstride = (int)kstride;
+        k.flt_rstride = pre ? 32 : wire_mul(k.entries, PIN);
+        k.flt_bytes = pre ? (uint32_t)k.KC * kstride : (uint32_t)k.OC * (uint32_t)k.flt_rstride;
+        k.tiles_m = (k.OC + MT * S - 1) / (MT * S);
+        k.tiles_n = (k.M + S - 1) / S;
+        k.by_m = k.tiles_m >= 8;
+        k.steps = S == 32 ? k.KC : (k.KC + 1) / 2;
+        k.per_wave = k.steps / W;
+        k.extra = k.steps % W;
+    }
+    template <int PIN, int S, int MT, int W>
+    __device__ __forceinline__ KsArgs<Quot> open() const {
+        asm volatile("" ::"s"(src), "s"(flt), "s"(bias), "s"(z), "s"(dst), "s"(N), "s"(in), "s"(out), "s"(channels), "s"(window), "s"(flags),
+                     "s"(kstride), "s"(epi.f[0]), "s"(epi.f[1]), "s"(epi.f[2]), "s"(epi.f[3]));  // one batch of scalar loads
+        KsArgs<Quot> k;
+        k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
+        numbers<PIN, S, MT, W>(k);
+        k.div_tile = quot(k.by_m ? k.tiles_n : k.tiles_m);
+        k.div_ohw = quot(k.OHW); k.div_ow = quot(k.OW);
+        k.div_t = quot(k.T); k.div_fw = quot(k.FW);
+        k.epi = epi_open(epi, flags & 255);
+        return k;
+    }
+    // false: the problem has a number that does not fit
+    template <int PIN, int S, int MT, int W>
+    bool pack(const KsArgs<FastDiv>& k, uint32_t n) {
+        src = k.src; flt = k.flt; bias = k.bias; z = k.z; dst = k.dst;
+        N = n; in = wire2(k.IH, k.IW); out = wire2(k.OW ? k.OHW / k.OW : 0, k.OW);
+        channels = wire2(k.OC, k.T ? k.entries / k.T : 0);
+        window = wire4(k.sh, k.sw, k.ph, k.pw);
+        kstride = (uint32_t)k.flt_kstride;
+        flags = epi_wire(k.epi, k.dst_s32, &epi) | (uint32_t)k.log_pout << 8 | (k.has_bias ? 1u << 11 : 0) | (k.dst_s32 ? 1u << 12 : 0) |
+                (k.flt_rstride != wire_mul(k.entries, PIN) ? 1u << 13 : 0) | wire4(0, 0, k.FH, k.FW);
+        KsArgs<FastDiv> o;
+        numbers<PIN, S, MT, W>(o);
+        if (!k.epi.has_z) o.z_sn = k.z_sn;  // (nothing reads it)
+        return o.numbers() == k.numbers() && k.M < QUOT_MAX && (int64_t)k.entries + 16 < QUOT_MAX && (int64_t)(k.tiles_m + 8) * (k.tiles_n + 8) < QUOT_MAX;
+    }
+};
+static_assert(sizeof(KsWire) <= WIRE_BYTES, "a wire");
 
 // S = 32: v_mfma_i32_32x32x32_i8, a step is one 32-byte k-chunk; S = 16: v_mfma_i32_16x16x64_i8, a step is two of them.
 // Lane l holds filter row (pixel) l % S and 16 bytes at 16 (l / S) of the step.
@@ -72,8 +157,8 @@ struct KsAcc<16> {
     __device__ __forceinline__ v4i quad(int) const { return v; }  // channels 4 (lane / 16) .. + 3
 };
 
-template <int PIN, int S, int MT, int W, bool PW>
-__global__ __launch_bounds__(W * 64) void ks_kernel(KsArgs a) {
+template <int PIN, int S, int MT, int W, bool PW, class Form>
+__device__ __forceinline__ void ks_run(const Form& form) {
     constexpr int ROWS = S / 4;           // channel quads of a block
     constexpr int PARTS = S == 32 ? 4 : 1;  // a block's quads over its pixels, 64 at a time
     constexpr int ROWP = ks_row(S), WP = MT * ROWS * ROWP;  // vectors per row, per wave
@@ -82,15 +167,18 @@ __global__ __launch_bounds__(W * 64) void ks_kernel(KsArgs a) {
     extern __shared__ __attribute__((aligned(16))) v4i red[];
     // Every argument on the way to the operands in one batch of scalar loads (left alone, the compiler asks for them where they
     // are first used, behind the early exit: a second round trip), and one word of each line that the epilogue reads.
-    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.OHW), "s"(a.OW), "s"(a.IW),
-                 "s"(a.IH), "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.OC), "s"(a.M), "s"(a.src_sn), "s"(a.src_scb),
-                 "s"(a.flt_rstride), "s"(a.flt_kstride), "s"(a.tiles_m), "s"(a.tiles_n), "s"(a.by_m), "s"(a.KC));
-    asm volatile("" ::"s"(a.steps), "s"(a.per_wave), "s"(a.extra), "s"(a.div_tile.m), "s"(a.div_tile.s1), "s"(a.div_tile.s2),
-                 "s"(a.div_ohw.m), "s"(a.div_ohw.s1), "s"(a.div_ohw.s2), "s"(a.div_ow.m), "s"(a.div_ow.s1), "s"(a.div_ow.s2),
-                 "s"(a.log_pout), "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo));
-    if (!PW)
-        asm volatile("" ::"s"(a.div_t.m), "s"(a.div_t.s1), "s"(a.div_t.s2), "s"(a.div_fw.m), "s"(a.div_fw.s1), "s"(a.div_fw.s2), "s"(a.T),
-                     "s"(a.FW), "s"(a.FH));
+    const auto a = form.template open<PIN, S, MT, W>();
+    if constexpr (!Form::WIRE) {
+        asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.z), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.OHW), "s"(a.OW), "s"(a.IW),
+                     "s"(a.IH), "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.OC), "s"(a.M), "s"(a.src_sn), "s"(a.src_scb),
+                     "s"(a.flt_rstride), "s"(a.flt_kstride), "s"(a.tiles_m), "s"(a.tiles_n), "s"(a.by_m), "s"(a.KC));
+        asm volatile("" ::"s"(a.steps), "s"(a.per_wave), "s"(a.extra), "s"(a.div_tile.m), "s"(a.div_tile.s1), "s"(a.div_tile.s2),
+                     "s"(a.div_ohw.m), "s"(a.div_ohw.s1), "s"(a.div_ohw.s2), "s"(a.div_ow.m), "s"(a.div_ow.s1), "s"(a.div_ow.s2),
+                     "s"(a.log_pout), "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo));
+        if (!PW)
+            asm volatile("" ::"s"(a.div_t.m), "s"(a.div_t.s1), "s"(a.div_t.s2), "s"(a.div_fw.m), "s"(a.div_fw.s1), "s"(a.div_fw.s2), "s"(a.T),
+                         "s"(a.FW), "s"(a.FH));
+    }
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int ls = lane & (S - 1), lk = lane / S;
 
@@ -100,12 +188,12 @@ __global__ __launch_bounds__(W * 64) void ks_kernel(KsArgs a) {
     {
         const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
         if (a.by_m) {
-            const int r = (int)fdiv(i, a.div_tile);
+            const int r = (int)fdiv_u(i, a.div_tile);
             tm = r * 8 + x;
             tn = i - r * a.tiles_n;
             if (tm >= a.tiles_m) return;
         } else {
-            const int per = (a.tiles_n + 7) >> 3, r = (int)fdiv(i, a.div_tile);
+            const int per = (a.tiles_n + 7) >> 3, r = (int)fdiv_u(i, a.div_tile);
             tm = i - r * a.tiles_m;
             tn = x * per + r;
             if (tn >= a.tiles_n) return;
@@ -150,9 +238,9 @@ __global__ __launch_bounds__(W * 64) void ks_kernel(KsArgs a) {
     // load cursor: step kc; for 32-packed inputs and one chunk per step its channel block and tap (wave-uniform)
     int kc = k0, cb = 0, fh = 0, fw = 0;
     if (PIN == 32 && !PW && S == 32) {
-        cb = (int)fdiv(k0, a.div_t);
+        cb = (int)fdiv_u(k0, a.div_t);
         const int tap = k0 - cb * a.T;
-        fh = (int)fdiv(tap, a.div_fw);
+        fh = (int)fdiv_u(tap, a.div_fw);
         fw = tap - fh * a.FW;
     }
     // Operands of the next step.  Past the wave's piece every lane is out of the buffers' range: zeros, no memory access
@@ -172,7 +260,9 @@ __global__ __launch_bounds__(W * 64) void ks_kernel(KsArgs a) {
             fb = __builtin_amdgcn_raw_buffer_load_b128(rs_src, in && half_in && pix != SENT ? pix + c : SENT, kc * CH * a.src_scb, 0);
         } else if (PIN == 32 && S == 32) {
             const bool ok = in && (unsigned)(ih0 + fh) < (unsigned)a.IH && (unsigned)(iw0 + fw) < (unsigned)a.IW;
-            fb = __builtin_amdgcn_raw_buffer_load_b128(rs_src, ok ? pix + (fh * a.IW + fw) * 32 : SENT, cb * a.src_scb, 0);
+            // (not the block's offset as the instruction's scalar one: where the compiler keeps the cursor in a vector register, that
+            // makes a loop of the load)
+            fb = __builtin_amdgcn_raw_buffer_load_b128(rs_src, ok ? pix + (fh * a.IW + fw) * 32 + cb * a.src_scb : SENT, 0, 0);
         } else if (PIN == 32) {
             const uint32_t c = kc * 2 + (lk >> 1), b = fdiv(c, a.div_t), tap = c - b * a.T, h = fdiv(tap, a.div_fw), w = tap - h * a.FW;
             const bool ok = in && half_in && (unsigned)(ih0 + (int)h) < (unsigned)a.IH && (unsigned)(iw0 + (int)w) < (unsigned)a.IW;
@@ -293,6 +383,15 @@ __global__ __launch_bounds__(W * 64) void ks_kernel(KsArgs a) {
     }
 }
 
+template <int PIN, int S, int MT, int W, bool PW>
+__global__ __launch_bounds__(W * 64) void ks_kernel(KsWire a) {
+    ks_run<PIN, S, MT, W, PW>(a);
+}
+template <int PIN, int S, int MT, int W, bool PW>
+__global__ __launch_bounds__(W * 64) void ks_kernel(KsWide a) {
+    ks_run<PIN, S, MT, W, PW>(a);
+}
+
 struct KsCfg {
     int pin, s, mt, waves;
     const char* name;
@@ -308,18 +407,25 @@ int ks_lds(const IgemmArgs& a, const KsCfg& c, bool pw) {
     return c.waves * c.mt * (c.s / 4) * ks_row(c.s) * 16 + (c.pin == 4 && !pw ? (a.KC + 1) * 8 * 8 : 0);
 }
 
-template <int PIN, int S, int MT, int W, bool PW>
-int launch_ks(hipStream_t st, const KsArgs& k, int lds) {
-    auto kern = ks_kernel<PIN, S, MT, W, PW>;
+template <int PIN, int S, int MT, int W, bool PW, class Form>
+int launch_ks_form(hipStream_t st, const Form& form, unsigned grid, int lds) {
+    void (*const kern)(Form) = ks_kernel<PIN, S, MT, W, PW>;
     static std::atomic<int> max_lds_set{0};
     if (lds > max_lds_set.load(std::memory_order_relaxed)) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return (int)e;
         max_lds_set.store(160 * 1024, std::memory_order_relaxed);
     }
+    return launch_kernel(kern, dim3(grid), dim3(W * 64), lds, st, form);
+}
+
+template <int PIN, int S, int MT, int W, bool PW>
+int launch_ks(hipStream_t st, const KsArgs<FastDiv>& k, uint32_t n, int lds) {
     const int64_t grid = k.by_m ? (int64_t)((k.tiles_m + 7) / 8) * k.tiles_n * 8 : (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
-    return launch_kernel(kern, dim3((unsigned)grid), dim3(W * 64), lds, st, k);
+    KsWire wire;
+    if (wire.pack<PIN, S, MT, W>(k, n)) return launch_ks_form<PIN, S, MT, W, PW>(st, wire, (unsigned)grid, lds);
+    return launch_ks_form<PIN, S, MT, W, PW>(st, KsWide{k}, (unsigned)grid, lds);
 }
 
 }  // namespace
@@ -382,7 +488,7 @@ bool igemm5_can_run(const IgemmArgs& a, int pin, int pout, int cfg) {
 int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg) {
     if (!igemm5_can_run(a, pin, pout, cfg)) return (int)hipErrorInvalidConfiguration;
     const KsCfg& c = kKs[cfg];
-    KsArgs k;
+    KsArgs<FastDiv> k;
     k.src = a.src; k.flt = a.flt; k.bias = a.bias; k.z = a.z; k.dst = a.dst;
     k.src_bytes = a.src_bytes; k.flt_bytes = a.flt_bytes; k.z_bytes = a.z_bytes; k.dst_bytes = a.dst_bytes;
     k.IH = a.IH; k.IW = a.IW; k.OHW = a.OHW; k.OW = a.OW; k.FW = a.FW; k.T = a.T;
@@ -410,8 +516,8 @@ int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg
     const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0;
     const int lds = ks_lds(a, c, pw);
 #define MI355_KS(PIN, S, MT) \
-    (pw ? c.waves == 8 ? launch_ks<PIN, S, MT, 8, true>(st, k, lds) : launch_ks<PIN, S, MT, 4, true>(st, k, lds) \
-        : c.waves == 8 ? launch_ks<PIN, S, MT, 8, false>(st, k, lds) : launch_ks<PIN, S, MT, 4, false>(st, k, lds))
+    (pw ? c.waves == 8 ? launch_ks<PIN, S, MT, 8, true>(st, k, a.NB, lds) : launch_ks<PIN, S, MT, 4, true>(st, k, a.NB, lds) \
+        : c.waves == 8 ? launch_ks<PIN, S, MT, 8, false>(st, k, a.NB, lds) : launch_ks<PIN, S, MT, 4, false>(st, k, a.NB, lds))
     if (pin == 32) {
         if (c.s == 16) return MI355_KS(32, 16, 1);
         return c.mt == 1 ? MI355_KS(32, 32, 1) : MI355_KS(32, 32, 2);

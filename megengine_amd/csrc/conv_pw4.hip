@@ -14,8 +14,12 @@
 //     kernels (igemm_shared.h).
 // Channel blocks past the last one, and filter bytes past the end of a row, meet zero activations.
 #include <string.h>
+
+#include <tuple>
 #include <type_traits>
+
 #include "igemm_shared.h"
+#include "wire.h"
 
 namespace mi355 {
 namespace {
@@ -30,19 +34,21 @@ __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70
 // How the waves of a streaming launch walk the pixel blocks: wave g of the launch (of its XCD's share of the launch) takes the
 // channel group g % n_ocg of the blocks g / n_ocg, + step, ...  With slabs the XCDs take one contiguous eighth of the blocks
 // each.  The divisions are the host's: a run-time integer division is 0.1 us on the way to the first load.
+template <class Div>
 struct PwWalk {
     int n_ocg, step, slabs;
-    FastDiv div_ocg;
+    Div div_ocg;
 };
-PwWalk make_walk(int64_t blocks, int n_ocg) {
-    PwWalk w;
+PwWalk<FastDiv> make_walk(int64_t blocks, int n_ocg) {
+    PwWalk<FastDiv> w;
     w.n_ocg = n_ocg;
     w.slabs = blocks % 8 == 0 && blocks / 8 * 4 % n_ocg == 0;
     w.step = (int)((w.slabs ? blocks / 8 : blocks) * 4 / n_ocg);
     w.div_ocg = make_fastdiv(n_ocg);
     return w;
 }
-__device__ __forceinline__ void pw_walk(const PwWalk& w, int n_pb, int wave, int* pb0, int* pb_hi, int* ocg) {
+template <class Div>
+__device__ __forceinline__ void pw_walk(const PwWalk<Div>& w, int n_pb, int wave, int* pb0, int* pb_hi, int* ocg) {
     int lo = 0, hi = n_pb, g = (int)blockIdx.x * 4 + wave;
     if (w.slabs) {
         const int xc = blockIdx.x & 7, per = n_pb >> 3, rem = n_pb & 7;
@@ -50,7 +56,7 @@ __device__ __forceinline__ void pw_walk(const PwWalk& w, int n_pb, int wave, int
         hi = lo + per + (xc < rem ? 1 : 0);
         g = (int)(blockIdx.x >> 3) * 4 + wave;
     }
-    const int q = (int)fdiv(g, w.div_ocg);
+    const int q = (int)fdiv_u(g, w.div_ocg);
     *ocg = g - q * w.n_ocg;
     *pb0 = lo + q;
     *pb_hi = hi;
@@ -130,6 +136,78 @@ __global__ __launch_bounds__(256) void pw4s_kernel(IgemmArgs a, int n_ocg, int n
     }
 }
 
+// The arguments of the kernels with four pixels per lane (groups of them, at stride 1)
+template <class Div>
+struct QuadArgs {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    uint32_t src_bytes, flt_bytes, z_bytes, dst_bytes;
+    int NB, OHW, OC, kbytes, has_bias;
+    int src_sn, src_scb, dst_sn, dst_scb, z_sn;
+    int groups;  // of four pixels in an image
+    Div div_g;
+    EpiParams epi;
+
+    auto numbers() const {
+        return std::tie(src_bytes, flt_bytes, z_bytes, dst_bytes, NB, OHW, OC, kbytes, has_bias, src_sn, src_scb, dst_sn, dst_scb, z_sn, groups);
+    }
+};
+QuadArgs<FastDiv> quad_args(const IgemmArgs& a) {
+    QuadArgs<FastDiv> k;
+    k.src = a.src; k.flt = a.flt; k.bias = a.bias; k.z = a.z; k.dst = a.dst;
+    k.src_bytes = a.src_bytes; k.flt_bytes = a.flt_bytes; k.z_bytes = a.z_bytes; k.dst_bytes = a.dst_bytes;
+    k.NB = a.NB; k.OHW = a.OHW; k.OC = a.OC; k.kbytes = a.kbytes; k.has_bias = a.has_bias;
+    k.src_sn = a.src_sn; k.src_scb = a.src_scb; k.dst_sn = a.dst_sn; k.dst_scb = a.dst_scb; k.z_sn = a.z_sn;
+    k.groups = (a.OHW + 3) / 4; k.div_g = make_fastdiv(k.groups);
+    k.epi = a.epi;
+    return k;
+}
+
+// What the wire forms of those kernels carry of it (see wire.h)
+struct QuadWire {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    uint32_t images, plane, channels, flags;  // channels: out | in << 16
+    EpiWire epi;
+
+    template <class Div>
+    __host__ __device__ __forceinline__ void numbers(QuadArgs<Div>& k) const {
+        k.NB = (int)images; k.OHW = (int)plane; k.OC = wire_lo(channels); k.kbytes = wire_hi(channels);
+        k.has_bias = (int)(flags >> 8 & 1);
+        k.src_scb = k.dst_scb = wire_mul(k.OHW, 4);
+        k.src_sn = wire_mul(k.kbytes, k.OHW); k.dst_sn = wire_mul(k.OC, k.OHW); k.z_sn = (flags >> 3 & 1) ? k.dst_sn : 0;
+        k.src_bytes = images * (uint32_t)k.src_sn; k.dst_bytes = images * (uint32_t)k.dst_sn; k.z_bytes = images * (uint32_t)k.z_sn;
+        k.flt_bytes = (uint32_t)k.OC * (uint32_t)k.kbytes;
+        k.groups = (k.OHW + 3) / 4;
+    }
+    __device__ __forceinline__ QuadArgs<Quot> open() const {
+        asm volatile("" ::"s"(src), "s"(flt), "s"(bias), "s"(z), "s"(dst), "s"(images), "s"(plane), "s"(channels), "s"(flags), "s"(epi.f[0]), "s"(epi.f[1]),
+                     "s"(epi.f[2]), "s"(epi.f[3]));  // one batch of scalar loads
+        QuadArgs<Quot> k;
+        k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
+        numbers(k);
+        k.div_g = quot(k.groups);
+        k.epi = epi_open(epi, flags & 255);
+        return k;
+    }
+    // false: the problem has a number that does not fit
+    bool pack(const QuadArgs<FastDiv>& k) {
+        src = k.src; flt = k.flt; bias = k.bias; z = k.z; dst = k.dst;
+        images = (uint32_t)k.NB; plane = (uint32_t)k.OHW; channels = wire2(k.OC, k.kbytes);
+        flags = epi_wire(k.epi, false, &epi) | (k.has_bias ? 1u << 8 : 0);
+        QuadArgs<FastDiv> o;
+        numbers(o);
+        if (!k.epi.has_z) o.z_sn = k.z_sn;  // (nothing reads it)
+        return o.numbers() == k.numbers() && (int64_t)k.NB * k.groups < QUOT_MAX;
+    }
+};
+
 // Stride 1, at most 64 input channels and many tiles: the same with four consecutive pixels per lane.  pw4s_kernel's cost is its memory instructions -- a dword per lane,
 // four loads and four stores for every 32 x 32 block, 256 bytes each -- and an NCHW4 plane is contiguous over its pixels.  The
 // 32 columns of an MFMA need not be 32 neighbouring pixels: column l of product j is pixel 4 l + j here, so that a lane's operands
@@ -137,17 +215,44 @@ __global__ __launch_bounds__(256) void pw4s_kernel(IgemmArgs a, int n_ocg, int n
 // block.  The last group of an image whose plane is no multiple of four holds 1 to 3 pixels: its surplus columns multiply
 // whatever follows (the descriptor answers zeros past the tensor) and are not stored.  Bound by the output stream and the
 // four vector instructions per output: 16 -> 96 at 112 x 112, batch 64, 18.9 us for 90 MB (4.8 TB/s) against 22.2.
-template <int MT, int KC, bool HZ>
-__global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, PwWalk w, int n_pb, int groups, FastDiv div_g) {
+struct Pw4qWide {
+    QuadArgs<FastDiv> a;
+    PwWalk<FastDiv> w;
+    __device__ __forceinline__ const QuadArgs<FastDiv>& open() const {
+        // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
+        asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.OHW), "s"(a.OC), "s"(a.NB),
+                     "s"(a.kbytes), "s"(a.src_sn), "s"(a.src_scb), "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(w.div_ocg.m),
+                     "s"(w.div_ocg.s1), "s"(w.div_ocg.s2), "s"(w.n_ocg), "s"(w.step), "s"(w.slabs), "s"(a.groups), "s"(a.div_g.m),
+                     "s"(a.div_g.s1), "s"(a.div_g.s2));
+        return a;
+    }
+    template <int MT>
+    __device__ __forceinline__ const PwWalk<FastDiv>& walk(int) const { return w; }
+};
+struct Pw4qWire : QuadWire {
+    uint32_t step;  // and whether it walks slabs, << 31
+    template <int MT>
+    __device__ __forceinline__ PwWalk<Quot> walk(int oc) const {
+        PwWalk<Quot> w;
+        w.n_ocg = (oc + MT * 32 - 1) / (MT * 32);
+        w.step = (int)(step & 0x7fffffff);
+        w.slabs = (int)(step >> 31);
+        w.div_ocg = quot(w.n_ocg);
+        return w;
+    }
+};
+static_assert(sizeof(Pw4qWire) <= WIRE_BYTES, "a wire");
+
+template <int MT, int KC, bool HZ, class Form>
+__device__ __forceinline__ void pw4q_run(const Form& form) {
     __shared__ __attribute__((aligned(16))) int sBias[4][MT * 32];
     const int t = threadIdx.x;
     const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
-    // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
-    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.OHW), "s"(a.OC), "s"(a.NB),
-                 "s"(a.kbytes), "s"(a.src_sn), "s"(a.src_scb), "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(w.div_ocg.m),
-                 "s"(w.div_ocg.s1), "s"(w.div_ocg.s2), "s"(w.n_ocg), "s"(w.step), "s"(w.slabs), "s"(n_pb), "s"(groups), "s"(div_g.m),
-                 "s"(div_g.s1), "s"(div_g.s2));
+    const auto a = form.open();
+    const auto w = form.template walk<MT>(a.OC);
+    const auto div_g = a.div_g;
+    const int groups = a.groups, n_pb = (a.NB * groups + 31) / 32;
     int pb0, pb_hi, ocg;
     pw_walk(w, n_pb, wave, &pb0, &pb_hi, &ocg);
     const int oc_w = ocg * MT * 32, step = w.step;
@@ -266,18 +371,35 @@ __global__ __launch_bounds__(256, 3) void pw4q_kernel(IgemmArgs a, PwWalk w, int
 // and, of pixels 4 (l % 16) .. + 3, the 16 k-bytes at 16 (l / 16)).  What bounds these layers is latency -- a few megabytes and a
 // few hundred products per CU -- so a wave asks for all (or four steps) of its operands at once, and the partial sums meet
 // in LDS once.
-template <int MT, int W>
-__global__ __launch_bounds__(W * 64, 2) void pw4k_kernel(IgemmArgs a, int tiles_m, int tiles_n, int groups, FastDiv div_g, FastDiv div_tm) {
+struct Pw4kWide {
+    QuadArgs<FastDiv> a;
+    FastDiv div_tm;  // by the channel tiles
+    __device__ __forceinline__ const QuadArgs<FastDiv>& open() const {
+        asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.z), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.z_bytes),
+                     "s"(a.OHW), "s"(a.OC), "s"(a.NB), "s"(a.kbytes), "s"(a.src_sn), "s"(a.src_scb), "s"(a.dst_scb), "s"(a.z_sn),
+                     "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(a.groups), "s"(a.div_g.m), "s"(a.div_g.s1),
+                     "s"(a.div_g.s2), "s"(div_tm.m), "s"(div_tm.s1), "s"(div_tm.s2));
+        return a;
+    }
+    __device__ __forceinline__ const FastDiv& by_tiles(int) const { return div_tm; }
+};
+struct Pw4kWire : QuadWire {
+    __device__ __forceinline__ Quot by_tiles(int tiles_m) const { return quot(tiles_m); }
+};
+static_assert(sizeof(Pw4kWire) <= WIRE_BYTES, "a wire");
+
+template <int MT, int W, class Form>
+__device__ __forceinline__ void pw4k_run(const Form& form) {
     constexpr int AHEAD = MT <= 2 ? 4 : 3;
     extern __shared__ __attribute__((aligned(16))) v4i part[];
-    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.z), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.z_bytes),
-                 "s"(a.OHW), "s"(a.OC), "s"(a.NB), "s"(a.kbytes), "s"(a.src_sn), "s"(a.src_scb), "s"(a.dst_scb), "s"(a.z_sn),
-                 "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(tiles_m), "s"(tiles_n), "s"(groups), "s"(div_g.m), "s"(div_g.s1),
-                 "s"(div_g.s2), "s"(div_tm.m), "s"(div_tm.s1), "s"(div_tm.s2));
+    const auto a = form.open();
+    const int groups = a.groups, tiles_m = (a.OC + MT * 16 - 1) / (MT * 16), tiles_n = (a.NB * groups + 15) / 16;
+    const auto div_g = a.div_g;
+    const auto div_tm = form.by_tiles(tiles_m);
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int ls = lane & 15, lk = lane >> 4;
     // workgroup b runs on XCD b % 8: each XCD takes a contiguous run of pixels with all their channels
-    const uint32_t at = blockIdx.x >> 3, r0 = fdiv(at, div_tm);
+    const uint32_t at = blockIdx.x >> 3, r0 = fdiv_u(at, div_tm);
     const int tm = (int)(at - r0 * tiles_m), tn = (int)(blockIdx.x & 7) * ((tiles_n + 7) >> 3) + (int)r0;
     if (tn >= tiles_n) return;
     const int oc0 = tm * MT * 16;
@@ -443,18 +565,88 @@ __global__ __launch_bounds__(W * 64, 2) void pw4k_kernel(IgemmArgs a, int tiles_
 // bottleneck block and its projection shortcut, whose cost is their output (and residual) stream.  A lane's B fragment
 // of k-step kc is one 16-byte load -- half of its pixel's 32-byte block kc; 32 consecutive pixels are one contiguous
 // kilobyte -- and the stores are the 16-byte stores of the tiled kernels.
-template <int MT, int KC, bool HZ>
-__global__ __launch_bounds__(256, 3) void pw32s_kernel(IgemmArgs a, PwWalk w, int n_pb,
-                                                       std::conditional_t<HZ, ResidualTable, NoResidualTable> tab) {
+struct Pw32sWide {
+    IgemmArgs a;
+    PwWalk<FastDiv> w;
+    __device__ __forceinline__ const IgemmArgs& open() const {
+        asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.z), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.z_bytes),
+                     "s"(a.OHW), "s"(a.OC), "s"(a.M), "s"(a.OW), "s"(a.IW), "s"(a.sh), "s"(a.sw), "s"(a.kbytes), "s"(a.src_sn), "s"(a.src_scb),
+                     "s"(a.dst_scb), "s"(a.z_sn), "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(w.div_ocg.m));
+        asm volatile("" ::"s"(a.div_ohw.m), "s"(a.div_ohw.s1), "s"(a.div_ohw.s2), "s"(a.div_ow.m), "s"(a.div_ow.s1), "s"(a.div_ow.s2),
+                     "s"(w.div_ocg.s1), "s"(w.div_ocg.s2), "s"(w.n_ocg), "s"(w.step), "s"(w.slabs));
+        return a;
+    }
+    template <int MT>
+    __device__ __forceinline__ const PwWalk<FastDiv>& walk(int) const { return w; }
+};
+struct Pw32sWire {
+    const int8_t* src;
+    const int8_t* flt;
+    const int32_t* bias;
+    const int8_t* z;
+    int8_t* dst;
+    // in: columns | rows << 16, out: columns | rows << 16; channels: out | in << 16; window: strides; m_*: multipliers of the divisions
+    uint32_t images, in, out, channels, window, step, m_ohw, m_ow, flags;
+    EpiWire epi;
+
+    __host__ __device__ __forceinline__ void numbers(IgemmArgs& k) const {
+        k.IW = wire_lo(in); k.OW = wire_lo(out); k.OHW = wire_mul(k.OW, wire_hi(out));
+        k.OC = wire_lo(channels); k.kbytes = wire_hi(channels);
+        k.sh = wire_lo(window); k.sw = wire_hi(window);
+        k.M = wire_mul((int)images, k.OHW);
+        k.src_scb = wire_mul(k.IW, wire_hi(in), 32); k.dst_scb = wire_mul(k.OHW, 32);
+        k.src_sn = wire_mul(k.kbytes / 32, k.src_scb); k.dst_sn = wire_mul(k.OC, k.OHW); k.z_sn = (flags >> 3 & 1) ? k.dst_sn : 0;
+        k.src_bytes = images * (uint32_t)k.src_sn; k.dst_bytes = images * (uint32_t)k.dst_sn; k.z_bytes = images * (uint32_t)k.z_sn;
+        k.flt_bytes = (uint32_t)k.OC * (uint32_t)k.kbytes;
+        k.has_bias = (int)(flags >> 8 & 1);
+    }
+    static auto compared(const IgemmArgs& k) {
+        return std::tie(k.IW, k.OW, k.OHW, k.OC, k.kbytes, k.sh, k.sw, k.M, k.src_scb, k.dst_scb, k.src_sn, k.dst_sn, k.z_sn, k.src_bytes, k.dst_bytes,
+                        k.z_bytes, k.flt_bytes, k.has_bias);
+    }
+    __device__ __forceinline__ IgemmArgs open() const {
+        asm volatile("" ::"s"(src), "s"(flt), "s"(bias), "s"(z), "s"(dst), "s"(images), "s"(in), "s"(out), "s"(channels), "s"(window), "s"(step), "s"(m_ohw),
+                     "s"(m_ow), "s"(flags), "s"(epi.f[0]), "s"(epi.f[1]), "s"(epi.f[2]), "s"(epi.f[3]));  // one batch of scalar loads
+        IgemmArgs k;
+        k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
+        numbers(k);
+        k.div_ohw = fastdiv_open(m_ohw, k.OHW); k.div_ow = fastdiv_open(m_ow, k.OW);
+        k.epi = epi_open(epi, flags & 255);
+        return k;
+    }
+    template <int MT>
+    __device__ __forceinline__ PwWalk<Quot> walk(int oc) const {
+        PwWalk<Quot> w;
+        w.n_ocg = (oc + MT * 32 - 1) / (MT * 32);
+        w.step = (int)step;
+        w.slabs = (int)(flags >> 9 & 1);
+        w.div_ocg = quot(w.n_ocg);
+        return w;
+    }
+    // false: the problem has a number that does not fit
+    bool pack(const IgemmArgs& k, const PwWalk<FastDiv>& w, int64_t blocks) {
+        if (k.OW <= 0 || k.IW <= 0) return false;
+        src = k.src; flt = k.flt; bias = k.bias; z = k.z; dst = k.dst;
+        images = (uint32_t)k.NB; in = wire2(k.IW, k.IH); out = wire2(k.OW, k.OHW / k.OW); channels = wire2(k.OC, k.kbytes); window = wire2(k.sh, k.sw);
+        step = (uint32_t)w.step; m_ohw = k.div_ohw.m; m_ow = k.div_ow.m;
+        flags = epi_wire(k.epi, false, &epi) | (k.has_bias ? 1u << 8 : 0) | (w.slabs ? 1u << 9 : 0);
+        IgemmArgs o;
+        numbers(o);
+        if (!k.epi.has_z) o.z_sn = k.z_sn;  // (nothing reads it)
+        return compared(o) == compared(k) && !k.epi.zlin && blocks * 4 < QUOT_MAX;
+    }
+};
+static_assert(sizeof(Pw32sWire) <= WIRE_BYTES, "a wire");
+
+template <int MT, int KC, bool HZ, class Form, class Table>
+__device__ __forceinline__ void pw32s_run(const Form& form, const Table& tab) {
     const int t = threadIdx.x;
     const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
 
-    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.z), "s"(a.src_bytes), "s"(a.flt_bytes), "s"(a.z_bytes),
-                 "s"(a.OHW), "s"(a.OC), "s"(a.M), "s"(a.OW), "s"(a.IW), "s"(a.sh), "s"(a.sw), "s"(a.kbytes), "s"(a.src_sn), "s"(a.src_scb),
-                 "s"(a.dst_scb), "s"(a.z_sn), "s"(a.has_bias), "s"(a.epi.s_b), "s"(a.epi.lin_lo), "s"(w.div_ocg.m));
-    asm volatile("" ::"s"(a.div_ohw.m), "s"(a.div_ohw.s1), "s"(a.div_ohw.s2), "s"(a.div_ow.m), "s"(a.div_ow.s1), "s"(a.div_ow.s2),
-                 "s"(w.div_ocg.s1), "s"(w.div_ocg.s2), "s"(w.n_ocg), "s"(w.step), "s"(w.slabs), "s"(n_pb));
+    const auto a = form.open();
+    const auto w = form.template walk<MT>(a.OC);
+    const int n_pb = (a.M + 31) / 32;
     // Pixel blocks by XCD, as the tiled kernels deal out their tiles: workgroup b runs on XCD b % 8 (round-robin
     // dispatch) and each XCD takes one contiguous eighth of the pixel blocks, so that this layer finds its inputs in the
     // L2 of the XCD that wrote them and leaves its outputs where the next layer's workgroups will look for them.
@@ -465,11 +657,12 @@ __global__ __launch_bounds__(256, 3) void pw32s_kernel(IgemmArgs a, PwWalk w, in
     const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes);
     const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, a.flt_bytes);
     const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
-    // residual table form: the 256 offsets from the kernel's last argument into LDS, once per workgroup (ahead of the first
+    // residual table form (the wide one only): the 256 offsets from the kernel's last argument into LDS, once per workgroup (ahead of the first
     // loads: behind them, with the barrier holding every wave until the slowest wave's loads are back, the stack is 3 us
     // slower)
-    __shared__ float zt[HZ ? 256 : 1];
-    if constexpr (HZ) {
+    constexpr bool TABLE = std::is_same<Table, ResidualTable>::value;
+    __shared__ float zt[TABLE ? 256 : 1];
+    if constexpr (TABLE) {
         if (a.epi.zlin) zt[t] = tab.v[t];
         __syncthreads();
     }
@@ -546,8 +739,8 @@ __global__ __launch_bounds__(256, 3) void pw32s_kernel(IgemmArgs a, PwWalk w, in
         }
     };
     using std::integral_constant;
-    if (HZ && a.epi.zlin) {
-        if constexpr (HZ) blocks(integral_constant<int, NL_ZLIN>{});
+    if (TABLE && a.epi.zlin) {
+        if constexpr (TABLE) blocks(integral_constant<int, NL_ZLIN>{});
     } else if (!HZ && a.epi.lin) {
         if constexpr (!HZ) blocks(integral_constant<int, NL_LIN>{});
     } else {
@@ -557,6 +750,31 @@ __global__ __launch_bounds__(256, 3) void pw32s_kernel(IgemmArgs a, PwWalk w, in
             default: blocks(integral_constant<int, NL_IDENTITY>{}); break;
         }
     }
+}
+
+template <int MT, int KC, bool HZ>
+__global__ __launch_bounds__(256, 3) void pw32s_kernel(Pw32sWide a, std::conditional_t<HZ, ResidualTable, NoResidualTable> tab) {
+    pw32s_run<MT, KC, HZ>(a, tab);
+}
+template <int MT, int KC, bool HZ>
+__global__ __launch_bounds__(256, 3) void pw32s_wire_kernel(Pw32sWire a) {
+    pw32s_run<MT, KC, HZ>(a, NoResidualTable{});
+}
+template <int MT, int KC, bool HZ>
+__global__ __launch_bounds__(256, 3) void pw4q_kernel(Pw4qWide a) {
+    pw4q_run<MT, KC, HZ>(a);
+}
+template <int MT, int KC, bool HZ>
+__global__ __launch_bounds__(256, 3) void pw4q_kernel(Pw4qWire a) {
+    pw4q_run<MT, KC, HZ>(a);
+}
+template <int MT, int W>
+__global__ __launch_bounds__(W * 64, 2) void pw4k_kernel(Pw4kWide a) {
+    pw4k_run<MT, W>(a);
+}
+template <int MT, int W>
+__global__ __launch_bounds__(W * 64, 2) void pw4k_kernel(Pw4kWire a) {
+    pw4k_run<MT, W>(a);
 }
 
 template <int MT, int KC>
@@ -571,12 +789,18 @@ int launch32_mt(hipStream_t st, const IgemmArgs& a, int cu_count) {
     blocks = (blocks + n_ocg - 1) / n_ocg * n_ocg;  // waves of one pixel block stay together; 4 * blocks % n_ocg == 0
     // large grids: a multiple of 8 n_ocg workgroups, which the kernel splits into one slab of pixel blocks per XCD
     if (blocks >= 16 * (int64_t)n_ocg) blocks = blocks / (8 * n_ocg) * (8 * n_ocg);
+    const dim3 grid((unsigned)blocks);
+    const PwWalk<FastDiv> walk = make_walk(blocks, n_ocg);
+    Pw32sWire wire;
+    if (wire.pack(a, walk, blocks)) {
+        return launch_kernel(a.epi.has_z ? pw32s_wire_kernel<MT, KC, true> : pw32s_wire_kernel<MT, KC, false>, grid, dim3(256), 0, st, wire);
+    }
     if (a.epi.has_z) {
         ResidualTable tab;
         if (a.epi.zlin) memcpy(tab.v, a.ztab, sizeof(tab.v)); else memset(tab.v, 0, sizeof(tab.v));
-        return launch_kernel((pw32s_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, make_walk(blocks, n_ocg), n_pb, tab);
+        return launch_kernel(pw32s_kernel<MT, KC, true>, grid, dim3(256), 0, st, Pw32sWide{a, walk}, tab);
     }
-    return launch_kernel((pw32s_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, make_walk(blocks, n_ocg), n_pb, NoResidualTable{});
+    return launch_kernel(pw32s_kernel<MT, KC, false>, grid, dim3(256), 0, st, Pw32sWide{a, walk}, NoResidualTable{});
 }
 
 template <int MT, int KC>
@@ -593,10 +817,17 @@ int launch_quad(hipStream_t st, const IgemmArgs& a, int cu_count) {
     // a multiple of the workgroups that deal out whole pixel blocks on every XCD (see the kernel)
     const int unit = 8 * (n_ocg % 4 == 0 ? n_ocg / 4 : n_ocg % 2 == 0 ? n_ocg / 2 : n_ocg);
     if (2 * blocks >= unit) blocks = (blocks + unit - 1) / unit * unit;
-    const FastDiv div_g = make_fastdiv(groups);
-    if (a.epi.has_z)
-        return launch_kernel((pw4q_kernel<MT, KC, true>), dim3((unsigned)blocks), dim3(256), 0, st, a, make_walk(blocks, n_ocg), n_pb, groups, div_g);
-    return launch_kernel((pw4q_kernel<MT, KC, false>), dim3((unsigned)blocks), dim3(256), 0, st, a, make_walk(blocks, n_ocg), n_pb, groups, div_g);
+    const dim3 grid((unsigned)blocks);
+    const PwWalk<FastDiv> walk = make_walk(blocks, n_ocg);
+    const QuadArgs<FastDiv> k = quad_args(a);
+    Pw4qWire wire;
+    if (wire.pack(k) && blocks * 4 < QUOT_MAX) {
+        wire.step = (uint32_t)walk.step | (walk.slabs ? 1u << 31 : 0u);
+        typedef void (*Kernel)(Pw4qWire);
+        return launch_kernel(a.epi.has_z ? (Kernel)pw4q_kernel<MT, KC, true> : (Kernel)pw4q_kernel<MT, KC, false>, grid, dim3(256), 0, st, wire);
+    }
+    typedef void (*Kernel)(Pw4qWide);
+    return launch_kernel(a.epi.has_z ? (Kernel)pw4q_kernel<MT, KC, true> : (Kernel)pw4q_kernel<MT, KC, false>, grid, dim3(256), 0, st, Pw4qWide{k, walk});
 }
 
 template <int MT, int W>
@@ -606,8 +837,11 @@ int launch_split(hipStream_t st, const IgemmArgs& a) {
     const int tiles_n = (int)(((int64_t)a.NB * groups + 15) / 16);
     const int64_t grid = (int64_t)((tiles_n + 7) / 8) * 8 * tiles_m;
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
-    return launch_kernel(pw4k_kernel<MT, W>, dim3((unsigned)grid), dim3(W * 64), W > 1 ? W * MT * 4096 : 0, st, a, tiles_m, tiles_n,
-                         groups, make_fastdiv(groups), make_fastdiv(tiles_m));
+    const QuadArgs<FastDiv> k = quad_args(a);
+    const int lds = W > 1 ? W * MT * 4096 : 0;
+    Pw4kWire wire;
+    if (wire.pack(k) && grid < QUOT_MAX) return launch_kernel((void (*)(Pw4kWire))pw4k_kernel<MT, W>, dim3((unsigned)grid), dim3(W * 64), lds, st, wire);
+    return launch_kernel((void (*)(Pw4kWide))pw4k_kernel<MT, W>, dim3((unsigned)grid), dim3(W * 64), lds, st, Pw4kWide{k, make_fastdiv(tiles_m)});
 }
 
 template <int MT, int KC>

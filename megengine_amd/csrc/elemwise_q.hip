@@ -90,7 +90,7 @@ struct EwArgs {
     float scale[3];
     float scale_dst, y_hi, y_lo;
     uint64_t blocks16, count;
-    uint32_t mode;
+    uint32_t mode, grid;
 };
 
 typedef int v4iu __attribute__((ext_vector_type(4), aligned(4)));  // QuantizedS8 tensors are 4-byte aligned
@@ -116,7 +116,7 @@ __device__ __forceinline__ int ew_one(const EwArgs& a, int v0, int v1, int v2, u
 
 template <int MODE, int ARITY, bool SRC32, bool DST32, bool FAST>
 __device__ __forceinline__ void ew_run(const EwArgs& a) {
-    const XcdRun<uint64_t> run = xcd_run<uint64_t>(a.blocks16);
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(a.blocks16, a.grid);
     for (uint64_t i = run.at; i < run.end; i += run.step) {
         v4i in[ARITY][SRC32 ? 4 : 1];
 #pragma unroll
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256) void elemwise_q_table_kernel(EwArgs a) {
     const int t = threadIdx.x;
     table[t] = (uint8_t)ew_one<-1, 1, false, false, false>(a, (int)(int8_t)t, 0, 0, a.mode);
     __syncthreads();
-    const XcdRun<uint64_t> run = xcd_run<uint64_t>(a.blocks16);
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(a.blocks16, a.grid);
     for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4i x = reinterpret_cast<const v4iu*>(a.src[0])[i];
         v4i o;
@@ -288,6 +288,7 @@ int launch_elemwise_q(hipStream_t st, const mi355_elemwise_desc& d, const void* 
     if (blocks > cap) blocks = cap;
     if (blocks == 0) blocks = 1;
     blocks = xcd_grid(blocks);
+    a.grid = (uint32_t)blocks;
     const bool src32 = d.src_dtype == MI355_DT_QS32, dst32 = d.dst_dtype == MI355_DT_QS32;
     if (d.arity == 1 && !src32 && !dst32) return launch_kernel(elemwise_q_table_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a);
     // the divide-free quotient: QuantizedS8 dst, a bounded result that stays far from overflow on the way to the clamp, a

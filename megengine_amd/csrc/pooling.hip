@@ -21,7 +21,7 @@ typedef short s2 __attribute__((ext_vector_type(2)));
 struct PoolArgs {
     const int8_t* src;
     int8_t* dst;
-    uint32_t units;  // output vectors
+    uint32_t units, grid;  // output vectors, workgroups
     int IH, IW, OH, OW, ph, pw, sh, sw, fh, fw;
     FastDiv div_ow, div_oh;
 };
@@ -101,7 +101,7 @@ template <int PACK, int VB, int MODE, int FH, int FW>
 __global__ __launch_bounds__(256) void pooling_static_kernel(PoolArgs a) {
     constexpr int UPP = PACK / VB;
     constexpr int W = VB / 4;
-    const XcdRun<uint32_t> run = xcd_run<uint32_t>(a.units);
+    const XcdRun<uint32_t> run = xcd_run<uint32_t>(a.units, a.grid);
     for (uint32_t u = run.at; u < run.end; u += run.step) {
         const uint32_t sub = UPP == 1 ? 0 : u % UPP, pix = UPP == 1 ? u : u / UPP;
         const uint32_t t = fdiv(pix, a.div_ow), ow = pix - t * a.OW;
@@ -177,7 +177,7 @@ template <int PACK, int VB, int MODE>
 __global__ __launch_bounds__(256) void pooling_kernel(PoolArgs a) {
     constexpr int UPP = PACK / VB;  // threads per pixel
     constexpr int W = VB >= 4 ? VB / 4 : 1;
-    const XcdRun<uint32_t> run = xcd_run<uint32_t>(a.units);
+    const XcdRun<uint32_t> run = xcd_run<uint32_t>(a.units, a.grid);
     for (uint32_t u = run.at; u < run.end; u += run.step) {
         const uint32_t sub = UPP == 1 ? 0 : u % UPP, pix = UPP == 1 ? u : u / UPP;
         const uint32_t t = fdiv(pix, a.div_ow), ow = pix - t * a.OW;
@@ -402,6 +402,7 @@ int launch_pooling(hipStream_t st, const mi355_pooling_desc& d, int pack, uint32
     const uint64_t cap = (uint64_t)cu_count * 64;
     if (blocks > cap) blocks = cap;
     blocks = xcd_grid(blocks);
+    a.grid = (uint32_t)blocks;
     if (pack == 32) return launch_mode<32, 16>(st, a, (int)d.mode, (unsigned)blocks);
     if (pack == 4) return launch_mode<4, 4>(st, a, (int)d.mode, (unsigned)blocks);
     return launch_mode<1, 1>(st, a, (int)d.mode, (unsigned)blocks);

@@ -11,8 +11,8 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(256) void requant_kernel(const int32_t* __restrict__ src, const int8_t* __restrict__ z,
-                                                      int8_t* __restrict__ dst, uint64_t quads, uint64_t count, EpiParams e) {
-    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads);
+                                                      int8_t* __restrict__ dst, uint64_t quads, uint64_t count, EpiParams e, uint32_t grid) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads, grid);
     for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4i a = reinterpret_cast<const v4i*>(src)[i];
         const uint32_t zw = e.has_z ? reinterpret_cast<const uint32_t*>(z)[i] : 0u;
@@ -27,8 +27,8 @@ __global__ __launch_bounds__(256) void requant_kernel(const int32_t* __restrict_
 
 // QuantizedS8 first operand: 16 elements per thread step (16 + 16 bytes in, 16 out; 2-3 bytes per element)
 __global__ __launch_bounds__(256) void requant8_kernel(const int8_t* __restrict__ src, const int8_t* __restrict__ z,
-                                                       int8_t* __restrict__ dst, uint64_t blocks16, uint64_t count, EpiParams e) {
-    const XcdRun<uint64_t> run = xcd_run<uint64_t>(blocks16);
+                                                       int8_t* __restrict__ dst, uint64_t blocks16, uint64_t count, EpiParams e, uint32_t grid) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(blocks16, grid);
     for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4i a = reinterpret_cast<const v4i*>(src)[i];
         v4i zv = {0, 0, 0, 0};
@@ -59,8 +59,8 @@ __device__ __forceinline__ int quantize_s8(float x, float scale) {
 }
 
 __global__ __launch_bounds__(256) void cvt_f32_s8_kernel(const float* __restrict__ src, int8_t* __restrict__ dst,
-                                                         uint64_t quads, uint64_t count, float scale) {
-    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads);
+                                                         uint64_t quads, uint64_t count, float scale, uint32_t grid) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads, grid);
     for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4f x = reinterpret_cast<const v4f*>(src)[i];
         reinterpret_cast<uint32_t*>(dst)[i] =
@@ -72,8 +72,8 @@ __global__ __launch_bounds__(256) void cvt_f32_s8_kernel(const float* __restrict
 
 // TypeCvt QuantizedS8 -> Float32: dequantize = float(x) * scale
 __global__ __launch_bounds__(256) void cvt_s8_f32_kernel(const int8_t* __restrict__ src, float* __restrict__ dst,
-                                                         uint64_t quads, uint64_t count, float scale) {
-    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads);
+                                                         uint64_t quads, uint64_t count, float scale, uint32_t grid) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads, grid);
     for (uint64_t i = run.at; i < run.end; i += run.step) {
         const int w = reinterpret_cast<const int*>(src)[i];
         v4f o;
@@ -99,14 +99,14 @@ unsigned stream_blocks(uint64_t steps, int cu_count) {
 
 int launch_cvt_f32_s8(hipStream_t st, float scale, const float* src, int8_t* dst, uint64_t count, int cu_count) {
     if (count == 0) return 0;
-    return launch_kernel(cvt_f32_s8_kernel, dim3(stream_blocks(count / 4, cu_count)), dim3(256), 0, st, src, dst, count / 4,
-                       count, scale);
+    const unsigned grid = stream_blocks(count / 4, cu_count);
+    return launch_kernel(cvt_f32_s8_kernel, dim3(grid), dim3(256), 0, st, src, dst, count / 4, count, scale, grid);
 }
 
 int launch_cvt_s8_f32(hipStream_t st, float scale, const int8_t* src, float* dst, uint64_t count, int cu_count) {
     if (count == 0) return 0;
-    return launch_kernel(cvt_s8_f32_kernel, dim3(stream_blocks(count / 4, cu_count)), dim3(256), 0, st, src, dst, count / 4,
-                       count, scale);
+    const unsigned grid = stream_blocks(count / 4, cu_count);
+    return launch_kernel(cvt_s8_f32_kernel, dim3(grid), dim3(256), 0, st, src, dst, count / 4, count, scale, grid);
 }
 
 int launch_requant8(hipStream_t st, const EpiParams& e, const int8_t* src, const int8_t* z, int8_t* dst, uint64_t count,
@@ -119,7 +119,7 @@ int launch_requant8(hipStream_t st, const EpiParams& e, const int8_t* src, const
     if (blocks > cap) blocks = cap;
     if (blocks == 0) blocks = 1;
     blocks = xcd_grid(blocks);
-    return launch_kernel(requant8_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, blocks16, count, e);
+    return launch_kernel(requant8_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, blocks16, count, e, (uint32_t)blocks);
 }
 
 int launch_requant(hipStream_t st, const EpiParams& e, const int32_t* src, const int8_t* z, int8_t* dst, uint64_t count,
@@ -132,7 +132,7 @@ int launch_requant(hipStream_t st, const EpiParams& e, const int32_t* src, const
     if (blocks > cap) blocks = cap;
     if (blocks == 0) blocks = 1;
     blocks = xcd_grid(blocks);
-    return launch_kernel(requant_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, quads, count, e);
+    return launch_kernel(requant_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, quads, count, e, (uint32_t)blocks);
 }
 
 // ---- streaming probe: what a launch that only moves bytes costs on this device ----------------------------------
