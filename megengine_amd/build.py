@@ -65,7 +65,7 @@ def build_native(verbose=False):
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
            *["-isystem" + p for p in cpp_extension.include_paths("cuda")], "-isystem" + sysconfig.get_paths()["include"],
            os.path.join(CSRC, "native.cpp"), "-o", NATIVE, "-L" + HERE, "-lmi355_convbias", *["-L" + p for p in libs],
-           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
