@@ -33,6 +33,11 @@ constexpr int ks_ahead(int s, int mt) { return s == 16 ? 6 : mt == 1 ? 8 : 4; }
 // reading them back -- a row by consecutive lanes, or all rows of a pixel by consecutive lanes -- then meet every bank once
 // per pass
 constexpr int ks_row(int s) { return s == 32 ? 34 : 20; }
+// vectors of a wave's share of LDS: its partial sums, and before them (TURN) a stage of the filter, 128 bytes of each row of the tile
+constexpr int ks_wave_vecs(int s, int mt, bool turn) {
+    const int sums = mt * (s / 4) * ks_row(s), stage = mt * s * 8;
+    return turn && stage > sums ? stage : sums;
+}
 
 template <class Div>
 struct KsArgs {
@@ -157,11 +162,15 @@ struct KsAcc<16> {
     __device__ __forceinline__ v4i quad(int) const { return v; }  // channels 4 (lane / 16) .. + 3
 };
 
-template <int PIN, int S, int MT, int W, bool PW, class Form>
+// TURN: long rows of a filter in the reference layout.  Loaded as operands, where neighbouring lanes hold different rows, 16 bytes per
+// lane take the address path 64 clocks instead of the 16 of a contiguous kilobyte, and that path is what the kernel is then bound by.
+// Here an instruction loads 128 bytes of each of eight rows, and LDS that only this wave uses turns them into operands (no barrier: a
+// wave's own LDS operations are in order).  A stage costs its LDS round trip, so short pieces do not take it: see ks_turns.
+template <int PIN, int S, int MT, int W, bool PW, bool TURN, class Form>
 __device__ __forceinline__ void ks_run(const Form& form) {
     constexpr int ROWS = S / 4;           // channel quads of a block
     constexpr int PARTS = S == 32 ? 4 : 1;  // a block's quads over its pixels, 64 at a time
-    constexpr int ROWP = ks_row(S), WP = MT * ROWS * ROWP;  // vectors per row, per wave
+    constexpr int ROWP = ks_row(S), WP = ks_wave_vecs(S, MT, TURN);  // vectors per row, per wave
     constexpr int CH = S == 32 ? 1 : 2;   // 32-byte chunks per step
     constexpr int AHEAD = ks_ahead(S, MT);
     extern __shared__ __attribute__((aligned(16))) v4i red[];
@@ -246,7 +255,7 @@ __device__ __forceinline__ void ks_run(const Form& form) {
     // Operands of the next step.  Past the wave's piece every lane is out of the buffers' range: zeros, no memory access
     // (an unconditional load keeps the number of loads in flight known to the compiler, and with it the waits short).
     // A 4-packed row may end inside its last chunk, so there the whole offset stands where the descriptor checks it.
-    auto load = [&](v4i (&fa)[MT], v4i& fb) __attribute__((always_inline)) {
+    auto load_filter = [&](v4i (&fa)[MT]) __attribute__((always_inline)) {
         const bool in = kc < k1;
         const int kf = kc * CH * a.flt_kstride;
         const bool half_in = S == 32 || kc * 2 + (lk >> 1) < a.KC;  // an odd number of chunks: no second one in the last step
@@ -255,6 +264,10 @@ __device__ __forceinline__ void ks_run(const Form& form) {
             const bool ok = in && half_in && arow[i] != SENT;
             fa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, ok ? arow[i] + kf : SENT, 0, 0);
         }
+    };
+    auto load_pixels = [&](v4i& fb) __attribute__((always_inline)) {
+        const bool in = kc < k1;
+        const bool half_in = S == 32 || kc * 2 + (lk >> 1) < a.KC;
         if (PIN == 32 && PW) {
             const int c = S == 32 ? 0 : (lk >> 1) * a.src_scb;
             fb = __builtin_amdgcn_raw_buffer_load_b128(rs_src, in && half_in && pix != SENT ? pix + c : SENT, kc * CH * a.src_scb, 0);
@@ -329,11 +342,71 @@ __device__ __forceinline__ void ks_run(const Form& form) {
         } else if (a.epi.has_z && !a.dst_s32) zw = __builtin_amdgcn_raw_buffer_load_b32(rs_z, z_off, 0, 0);
     };
 
-    {
+    if constexpr (TURN) {
+        // A stage is 128 bytes of every row: load j of a wave holds rows 8 j + lane / 8.  In LDS a row's 16-byte pieces change places
+        // by its number, so that neither the writes (a row by eight lanes) nor the reads (a piece of sixteen rows) meet on a bank.
+        constexpr int LOADS = MT * S / 8, STEPS = S == 32 ? 4 : 2, STEP_BYTES = 128 / STEPS;
+        v4i* mine = red + wave * WP;
+        int off[LOADS], at_w[LOADS], at_r[MT];
+#pragma unroll
+        for (int j = 0; j < LOADS; ++j) {
+            const int row = j * 8 + (lane >> 3), piece = lane & 7;
+            off[j] = oc0 + row < a.OC ? (oc0 + row) * a.flt_rstride + piece * 16 : SENT;
+            at_w[j] = row * 8 + (piece ^ ((row >> 1) & 7));
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i) at_r[i] = (i * S + ls) * 8;
+        const int turn = (ls >> 1) & 7;
+        v4i xf[2][LOADS], fb[2][STEPS];
+        int kf = k0, left = k1 - k0;
+        const int tail = a.flt_rstride - (lane & 7) * 16;  // bytes of the row from this lane's piece on
+        auto load_f = [&](int buf) __attribute__((always_inline)) {
+            // (nothing past the wave's piece of the reduction, whose last stage may be cut short, or past the row's end)
+            const bool in = kf * STEP_BYTES + (lane & 7) * 16 < k1 * STEP_BYTES && kf * STEP_BYTES < tail;
+#pragma unroll
+            for (int j = 0; j < LOADS; ++j) xf[buf][j] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, in && off[j] != SENT ? off[j] + kf * STEP_BYTES : SENT, 0, 0);
+            kf += STEPS;
+        };
+        auto load_p = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+            for (int b = 0; b < STEPS; ++b) load_pixels(fb[buf][b]);
+        };
+        auto stage = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < LOADS; ++j) mine[at_w[j]] = xf[buf][j];
+            load_f(buf);
+            v4i fa[STEPS][MT];
+#pragma unroll
+            for (int b = 0; b < STEPS; ++b)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) fa[b][i] = mine[at_r[i] + ((b * (8 / STEPS) + lk) ^ turn)];
+#pragma unroll
+            for (int b = 0; b < STEPS; ++b)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) acc[i].mfma(fa[b][i], fb[buf][b]);  // (steps past the piece: zeros)
+            load_p(buf);
+        };
+        if (left > 0) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                load_f(b);
+                load_p(b);
+            }
+        }
+        fetch(wave);
+        for (; left > 0; left -= 2 * STEPS) {
+            stage(0);
+            if (left <= STEPS) break;
+            stage(1);
+        }
+    } else {
         v4i fa[AHEAD][MT], fb[AHEAD];
         if (k0 < k1)  // (waves beyond the number of steps have nothing to add)
 #pragma unroll
-            for (int g = 0; g < AHEAD; ++g) load(fa[g], fb[g]);
+            for (int g = 0; g < AHEAD; ++g) {
+                load_filter(fa[g]);
+                load_pixels(fb[g]);
+            }
         fetch(wave);  // behind the first operands, so that bias and residual cost no round trip of their own
         auto multiply = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
@@ -344,7 +417,8 @@ __device__ __forceinline__ void ks_run(const Form& form) {
 #pragma unroll
             for (int g = 0; g < AHEAD; ++g) {
                 multiply(g);
-                load(fa[g], fb[g]);
+                load_filter(fa[g]);
+                load_pixels(fb[g]);
             }
         }
 #pragma unroll
@@ -385,11 +459,19 @@ __device__ __forceinline__ void ks_run(const Form& form) {
 
 template <int PIN, int S, int MT, int W, bool PW>
 __global__ __launch_bounds__(W * 64) void ks_kernel(KsWire a) {
-    ks_run<PIN, S, MT, W, PW>(a);
+    ks_run<PIN, S, MT, W, PW, false>(a);
 }
 template <int PIN, int S, int MT, int W, bool PW>
 __global__ __launch_bounds__(W * 64) void ks_kernel(KsWide a) {
-    ks_run<PIN, S, MT, W, PW>(a);
+    ks_run<PIN, S, MT, W, PW, false>(a);
+}
+template <int PIN, int S, int MT, int W, bool PW>
+__global__ __launch_bounds__(W * 64) void ks_turn_kernel(KsWire a) {
+    ks_run<PIN, S, MT, W, PW, true>(a);
+}
+template <int PIN, int S, int MT, int W, bool PW>
+__global__ __launch_bounds__(W * 64) void ks_turn_kernel(KsWide a) {
+    ks_run<PIN, S, MT, W, PW, true>(a);
 }
 
 struct KsCfg {
@@ -403,13 +485,25 @@ constexpr KsCfg kKs[] = {
         {4, 32, 1, 4, "ks4_32x32w4"},    {4, 32, 2, 8, "ks4_64x32w8"},    {4, 32, 2, 4, "ks4_64x32w4"}};
 constexpr int kKsCount = sizeof(kKs) / sizeof(kKs[0]);
 
+// Whether the filter goes through LDS (see ks_run): rows in the reference layout, and pieces of them from which on it pays.  Graph replays,
+// new / old by bytes of a row per wave, means over drawn layers: 64x32w8 256 to 383: 1.02 .. 1.07, 384 to 511: 0.93, 512 to 767: 0.86, from
+// 768 on 0.67 .. 0.84 (3x3 over 864 channels, 192 tiles: 14.5 -> 12.4 us); 16x16w4 256 to 511: 1.04 .. 1.14, 512 to 767: 0.99, from 768
+// on 0.89; 16x16w8 256 to 383: 1.07, 384 to 767: 0.93 .. 1.0, from 768 on 0.86.  The 32 x 32 tile of four waves has twice the
+// workgroups to a CU that cover its loads for each other: 1.16 to 1.31 with it at any length, and 4-packed rows 1.0 to 1.25.  Nor the
+// 64 x 32 tile with half of its rows missing (32 channels: 1.12 .. 1.19).
+constexpr bool ks_can_turn(int pin, int s, int mt, int waves) { return pin == 32 && (s == 16 || waves == 8); }
+bool ks_turns(const IgemmArgs& a, const KsCfg& c) {
+    return ks_can_turn(c.pin, c.s, c.mt, c.waves) && (c.mt == 1 || a.OC > 32) && a.flt_rstride == a.kbytes && a.kbytes >= (c.s == 32 ? 384 : 640) * c.waves;
+}
 int ks_lds(const IgemmArgs& a, const KsCfg& c, bool pw) {
-    return c.waves * c.mt * (c.s / 4) * ks_row(c.s) * 16 + (c.pin == 4 && !pw ? (a.KC + 1) * 8 * 8 : 0);
+    return c.waves * ks_wave_vecs(c.s, c.mt, ks_turns(a, c)) * 16 + (c.pin == 4 && !pw ? (a.KC + 1) * 8 * 8 : 0);
 }
 
-template <int PIN, int S, int MT, int W, bool PW, class Form>
+template <int PIN, int S, int MT, int W, bool PW, bool TURN, class Form>
 int launch_ks_form(hipStream_t st, const Form& form, unsigned grid, int lds) {
-    void (*const kern)(Form) = ks_kernel<PIN, S, MT, W, PW>;
+    void (*kern)(Form);
+    if constexpr (TURN) kern = ks_turn_kernel<PIN, S, MT, W, PW>;
+    else kern = ks_kernel<PIN, S, MT, W, PW>;
     static std::atomic<int> max_lds_set{0};
     if (lds > max_lds_set.load(std::memory_order_relaxed)) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -420,12 +514,14 @@ int launch_ks_form(hipStream_t st, const Form& form, unsigned grid, int lds) {
 }
 
 template <int PIN, int S, int MT, int W, bool PW>
-int launch_ks(hipStream_t st, const KsArgs<FastDiv>& k, uint32_t n, int lds) {
+int launch_ks(hipStream_t st, const KsArgs<FastDiv>& k, uint32_t n, int lds, bool turn) {
     const int64_t grid = k.by_m ? (int64_t)((k.tiles_m + 7) / 8) * k.tiles_n * 8 : (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
     KsWire wire;
-    if (wire.pack<PIN, S, MT, W>(k, n)) return launch_ks_form<PIN, S, MT, W, PW>(st, wire, (unsigned)grid, lds);
-    return launch_ks_form<PIN, S, MT, W, PW>(st, KsWide{k}, (unsigned)grid, lds);
+    const bool fits = wire.pack<PIN, S, MT, W>(k, n);
+    if constexpr (ks_can_turn(PIN, S, MT, W))
+        if (turn) return fits ? launch_ks_form<PIN, S, MT, W, PW, true>(st, wire, (unsigned)grid, lds) : launch_ks_form<PIN, S, MT, W, PW, true>(st, KsWide{k}, (unsigned)grid, lds);
+    return fits ? launch_ks_form<PIN, S, MT, W, PW, false>(st, wire, (unsigned)grid, lds) : launch_ks_form<PIN, S, MT, W, PW, false>(st, KsWide{k}, (unsigned)grid, lds);
 }
 
 }  // namespace
@@ -515,9 +611,10 @@ int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg
     k.epi = a.epi;
     const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0;
     const int lds = ks_lds(a, c, pw);
+    const bool turn = ks_turns(a, c);
 #define MI355_KS(PIN, S, MT) \
-    (pw ? c.waves == 8 ? launch_ks<PIN, S, MT, 8, true>(st, k, a.NB, lds) : launch_ks<PIN, S, MT, 4, true>(st, k, a.NB, lds) \
-        : c.waves == 8 ? launch_ks<PIN, S, MT, 8, false>(st, k, a.NB, lds) : launch_ks<PIN, S, MT, 4, false>(st, k, a.NB, lds))
+    (pw ? c.waves == 8 ? launch_ks<PIN, S, MT, 8, true>(st, k, a.NB, lds, turn) : launch_ks<PIN, S, MT, 4, true>(st, k, a.NB, lds, turn) \
+        : c.waves == 8 ? launch_ks<PIN, S, MT, 8, false>(st, k, a.NB, lds, turn) : launch_ks<PIN, S, MT, 4, false>(st, k, a.NB, lds, turn))
     if (pin == 32) {
         if (c.s == 16) return MI355_KS(32, 16, 1);
         return c.mt == 1 ? MI355_KS(32, 32, 1) : MI355_KS(32, 32, 2);
