@@ -599,45 +599,39 @@ static bool igemm_plain_s32(const ConvProblem& p) {
     return p.d.dst_dtype == MI355_DT_QS32 && p.d.bias_mode != MI355_BIAS_FULL;
 }
 
-// 32-packed dense layers with the filter in the reference layout.  What such a layer takes on a tile is a price per launch (a chain of
-// copies as long as the reduction), one per round of tiles over the device's CUs and one per tile and CU, each with a part that grows
-// with the reduction.  Four terms separate what those leave together:
+// Dense 32-packed layers.  What such a layer takes on a tile is a price per launch (a chain of copies as long as the reduction), one per
+// round of tiles over the device's CUs and one per tile and CU, each with a part that grows with the reduction.  Four terms separate
+// what those leave together:
 //   line_k: filter rows of whole 128-byte lines.  The second-generation tiles read a plain filter 32 bytes of every row at a time, all
 //     of them at the same place of a line then: 10 to 20 % longer than one channel block more or less (3x3 over 384 channels, stride 2,
 //     165 tiles of 64 x 64: 13.8 us; over 416, 168 of them: 12.2).  The first-generation tiles read whole rows and hardly have it.
 //   alone_k: no more tiles than CUs, so that no second workgroup covers a stage's copies.
 //   pair_k: a round of two workgroups to a CU, which the tiles with small rings go by.
 //   window: the table of offsets that a workgroup of a windowed layer begins with.
-// The prices, in us and us per 1024 reduction bytes, are fitted to graph replays on 256 CUs of 2640 layers of 32 to 2048 channels, 1x1 to
-// 5x5, stride 1 and 2, batch 1 to 64 (two halves of them predict each other as well as themselves).  The six tiles here hold the best of
-// eleven to nineteen to 1.9 % on average and are 1.13 times as fast as thresholds on tile counts: 3x3 288 -> 672 at 45 x 37, batch 10:
-// 48.8 -> 34.4 us; 5x5 32 -> 992 at 51 x 64, stride 2, batch 59: 70.8 -> 63.4; 1x1 320 -> 672 at 60 x 34, batch 49: 63.7 -> 47.8.
-// Without the four terms and the last tile it was 1.11, and 306 of the 2640 were more than 3 % slower than by thresholds (97 more than
-// 10 %); 79 are with them (9), at most 1.19.  Layers into 32 channels and fewer are not priced: they keep the 32 x 256 tile.
-static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool window, bool strided, bool has_z, int cu_count) {
-    struct Price {
-        int cfg, bm, bn;  // tile: 2^bm channels x 2^bn pixels
-        float launch, window, launch_k, round, round_k, pair_k, tile, tile_k, strided_k, z, line_k, alone_k;
-    };
-    const int dma = kNumCfgs, v2 = igemm_first_v2_cfg();
-    const Price prices[] = {
-            {dma + 18, 6, 7, 3.61f, 0.25f, 0.00f, 0.70f, 1.53f, 0.18f, 0.30f, 0.50f, 0.18f, 0.28f, 0.02f, 0.31f},  // dma64x128x128w8
-            {v2 + 10, 7, 8, 3.78f, 0.01f, 0.03f, 0.96f, 4.89f, 0.03f, 1.01f, 0.14f, 2.61f, 2.21f, 1.64f, 0.00f},   // v2_128x256x64r3w8
-            {v2 + 8, 6, 6, 3.44f, 0.22f, 0.32f, 0.47f, 1.62f, 0.01f, 0.00f, 0.00f, 0.36f, 0.19f, 0.39f, 0.00f},    // v2_64x64x128r4
-            {dma + 17, 7, 7, 3.30f, 0.21f, 0.00f, 0.84f, 1.64f, 1.83f, 0.50f, 0.79f, 0.38f, 0.79f, 0.00f, 0.09f},  // dma128x128x128r2w8
-            {v2 + 4, 6, 7, 3.46f, 0.64f, 0.04f, 0.32f, 2.30f, 0.18f, 0.21f, 0.00f, 0.48f, 0.55f, 0.60f, 0.31f},    // v2_64x128x64r4
-            {dma + 12, 6, 6, 3.37f, 0.53f, 0.00f, 0.69f, 0.23f, 1.41f, 0.00f, 0.41f, 0.11f, 0.19f, 0.00f, 0.21f},  // dma64x64x128r4
-    };
-    const float k = kbytes / 1024.0f;
-    const bool lines = kbytes % 128 == 0;
-    const uint32_t cu = cu_count;
+// The prices, in us and us per 1024 reduction bytes, are fitted (no term negative) to graph replays on 256 CUs of every tile here, and ten
+// to twenty more, on drawn layers of 32 to 2048 channels, 1x1 to 5x5, stride 1 and 2, batch 1 to 64: 9414 with the filter in the reference
+// layout, 5930 with it pre-processed, of which the layers of ResNet-50 for drawn batches and image sizes are half.  Two halves of them
+// predict each other as well as themselves.  Thresholds on tile counts, fitted to powers of two, were behind the best tile by 6.0 % (plain)
+// and 5.1 % (pre-processed) on average, the prices by 2.1 and 1.7; 3 and 6 % of the layers are more than 3 % slower with them, 0.8 and
+// 0.6 % more than 10 %, at most 1.27.  Into at most 32 channels, plain, which the 32 x 256 tile had whatever their number of pixels:
+// 1.22 times the best, now 1.01 (3x3 480 -> 32 at 8 x 29, batch 44: 35.0 -> 12.3 us).
+// The tiles that split the reduction over waves are priced where operand traffic does not bound them: up to `split_most` 64 x 32 tiles.
+struct TilePrice {
+    int cfg, bm, bn;  // tile: 2^bm channels x 2^bn pixels
+    float launch, window, launch_k, round, round_k, pair_k, tile, tile_k, strided_k, z, line_k, alone_k;
+};
+static int cheapest_tile(const TilePrice* prices, int count, const IgemmArgs& a, int cu_count) {
+    const float k = a.kbytes / 1024.0f;
+    const bool lines = a.kbytes % 128 == 0, window = a.T > 1, strided = a.sh * a.sw > 1;
+    const uint32_t cu = cu_count > 0 ? cu_count : 256;
     float best = 0;
     int cfg = -1;
-    for (const Price& c : prices) {
-        const uint32_t tiles = (uint32_t)((OC + (1 << c.bm) - 1) >> c.bm) * (uint32_t)((M + (1 << c.bn) - 1) >> c.bn);  // (OC * M < 2^31)
+    for (int i = 0; i < count; ++i) {
+        const TilePrice& c = prices[i];
+        const uint32_t tiles = (uint32_t)((a.OC + (1 << c.bm) - 1) >> c.bm) * (uint32_t)(((int64_t)a.M + (1 << c.bn) - 1) >> c.bn);  // (OC * M < 2^31)
         const uint32_t full = (tiles + cu - 1) / cu;
         const float rounds = (float)full, pairs = (float)((full + 1) / 2), share = (float)tiles / (float)cu;
-        const float tile = c.tile + k * (c.tile_k + (strided ? c.strided_k : 0) + (lines ? c.line_k : 0)) + (has_z ? c.z : 0);
+        const float tile = c.tile + k * (c.tile_k + (strided ? c.strided_k : 0) + (lines ? c.line_k : 0)) + (a.epi.has_z ? c.z : 0);
         const float us = c.launch + (window ? c.window : 0) + k * (c.launch_k + (full <= 1 ? c.alone_k : 0) + pairs * c.pair_k) +
                          rounds * (c.round + c.round_k * k) + share * tile;
         if (cfg < 0 || us < best) {
@@ -648,6 +642,68 @@ static int pick_plain_cfg(int64_t M, int OC, int kbytes, bool window, bool strid
     return cfg;
 }
 
+// 64 x 32 tiles: the unit in which few output pixels are counted
+static int64_t split_tiles(const IgemmArgs& a) { return (int64_t)((a.OC + 63) / 64) * (((int64_t)a.M + 31) / 32); }
+constexpr int64_t kSplitFew = 256;
+
+// `split_only`: among the tiles that split the reduction over waves
+static int pick_by_price(const IgemmArgs& a, bool pre, bool split_only, int cu_count) {
+    static const int dma = kNumCfgs, v2 = igemm_first_v2_cfg(), ks = igemm_first_ks_cfg();
+    constexpr int SPLIT = 5;  // of each list: the tiles that split the reduction
+    static const TilePrice plain_prices[] = {
+        {ks + 1, 4, 4, 3.28f, 0.00f, 0.24f, 0.16f, 0.22f, 0.00f, 0.13f, 0.08f, 0.09f, 0.00f, 0.00f, 0.14f},    // v2_ks_16x16w4
+        {ks + 0, 4, 4, 3.34f, 0.09f, 0.12f, 0.30f, 0.26f, 0.00f, 0.23f, 0.05f, 0.11f, 0.02f, 0.01f, 0.00f},    // v2_ks_16x16w8
+        {ks + 3, 5, 5, 3.53f, 0.00f, 0.10f, 0.10f, 0.71f, 0.03f, 0.14f, 0.19f, 0.36f, 0.03f, 0.34f, 0.00f},    // v2_ks_32x32w4
+        {ks + 2, 5, 5, 3.59f, 0.09f, 0.06f, 0.27f, 0.73f, 0.00f, 0.38f, 0.15f, 0.24f, 0.00f, 0.05f, 0.00f},    // v2_ks_32x32w8
+        {ks + 4, 6, 5, 3.79f, 0.00f, 0.33f, 0.11f, 0.94f, 0.00f, 0.42f, 0.22f, 0.33f, 0.07f, 0.13f, 0.00f},    // v2_ks_64x32w8
+        {v2 + 8, 6, 6, 3.94f, 0.32f, 0.43f, 0.19f, 1.44f, 0.02f, 0.42f, 0.00f, 0.34f, 0.21f, 0.43f, 0.00f},    // v2_64x64x128r4
+        {v2 + 4, 6, 7, 4.13f, 0.40f, 0.24f, 0.00f, 1.90f, 0.64f, 0.69f, 0.06f, 0.69f, 0.46f, 0.31f, 0.27f},    // v2_64x128x64r4
+        {v2 + 10, 7, 8, 4.77f, 0.00f, 0.00f, 0.00f, 4.88f, 0.18f, 2.18f, 0.86f, 2.34f, 1.57f, 0.60f, 0.28f},   // v2_128x256x64r3w8
+        {dma + 12, 6, 6, 4.20f, 0.24f, 0.00f, 0.27f, 0.41f, 1.49f, 0.49f, 0.19f, 0.13f, 0.14f, 0.00f, 0.09f},  // dma64x64x128r4
+        {dma + 18, 6, 7, 4.29f, 0.17f, 0.00f, 0.26f, 1.73f, 0.14f, 0.91f, 0.31f, 0.23f, 0.21f, 0.00f, 0.25f},  // dma64x128x128w8
+        {dma + 17, 7, 7, 4.12f, 0.00f, 0.00f, 0.26f, 1.63f, 1.87f, 1.17f, 0.85f, 0.33f, 0.58f, 0.00f, 0.42f},  // dma128x128x128r2w8
+        {dma + 6, 6, 6, 3.70f, 0.00f, 1.25f, 0.36f, 0.30f, 0.00f, 0.19f, 0.88f, 0.18f, 0.12f, 0.00f, 0.87f},   // dma64x64x128r2
+    };
+    static const TilePrice pre_prices[] = {
+        {ks + 1, 4, 4, 3.33f, 0.00f, 0.10f, 0.11f, 0.18f, 0.05f, 0.17f, 0.02f, 0.11f, 0.02f, 0.00f, 0.05f},    // v2_ks_16x16w4
+        {ks + 0, 4, 4, 3.38f, 0.00f, 0.05f, 0.25f, 0.22f, 0.00f, 0.26f, 0.00f, 0.13f, 0.01f, 0.00f, 0.00f},    // v2_ks_16x16w8
+        {ks + 3, 5, 5, 3.34f, 0.28f, 0.21f, 0.20f, 0.33f, 0.07f, 0.22f, 0.14f, 0.19f, 0.00f, 0.03f, 0.00f},    // v2_ks_32x32w4
+        {ks + 2, 5, 5, 3.31f, 0.18f, 0.09f, 0.52f, 0.33f, 0.11f, 0.34f, 0.13f, 0.21f, 0.02f, 0.04f, 0.00f},    // v2_ks_32x32w8
+        {ks + 4, 6, 5, 3.60f, 0.10f, 0.13f, 0.25f, 0.62f, 0.00f, 0.33f, 0.09f, 0.37f, 0.14f, 0.07f, 0.00f},    // v2_ks_64x32w8
+        {v2 + 8, 6, 6, 3.90f, 0.39f, 0.17f, 0.15f, 0.72f, 0.56f, 0.47f, 0.24f, 0.25f, 0.19f, 0.00f, 0.22f},    // v2_64x64x128r4
+        {v2 + 4, 6, 7, 4.11f, 0.63f, 0.37f, 0.00f, 1.00f, 0.64f, 0.77f, 0.69f, 0.56f, 0.41f, 0.03f, 0.46f},    // v2_64x128x64r4
+        {v2 + 12, 7, 7, 4.54f, 0.18f, 0.00f, 0.00f, 2.99f, 0.00f, 1.10f, 0.60f, 0.36f, 1.32f, 0.12f, 0.01f},   // v2_128x128x64r4w8
+        {v2 + 10, 7, 8, 5.15f, 0.00f, 0.00f, 0.00f, 4.31f, 0.00f, 1.90f, 1.58f, 1.04f, 1.72f, 0.20f, 0.76f},   // v2_128x256x64r3w8
+        {dma + 6, 6, 6, 3.56f, 0.05f, 1.44f, 0.24f, 0.17f, 0.00f, 0.20f, 1.04f, 0.22f, 0.08f, 0.00f, 0.67f},   // dma64x64x128r2
+        {dma + 1, 6, 6, 3.82f, 0.46f, 0.19f, 0.18f, 0.82f, 0.31f, 0.35f, 0.36f, 0.19f, 0.04f, 0.00f, 0.57f},   // dma64x64x128
+        {dma + 18, 6, 7, 3.99f, 0.32f, 0.00f, 0.34f, 1.84f, 0.00f, 0.72f, 0.38f, 0.28f, 0.02f, 0.00f, 0.30f},  // dma64x128x128w8
+        {dma + 17, 7, 7, 4.15f, 0.00f, 0.00f, 0.26f, 1.79f, 1.17f, 0.87f, 1.32f, 0.34f, 0.67f, 0.00f, 0.76f},  // dma128x128x128r2w8
+        {dma + 14, 7, 7, 4.37f, 0.28f, 0.02f, 0.03f, 2.67f, 0.56f, 0.99f, 0.86f, 0.49f, 0.61f, 0.00f, 0.46f},  // dma128x128x64w8
+        {v2 + 9, 8, 7, 4.97f, 0.00f, 0.00f, 0.00f, 3.79f, 0.00f, 1.23f, 2.10f, 0.61f, 2.20f, 0.00f, 1.12f},    // v2_256x128x64r3w8
+        {v2 + 11, 8, 8, 5.20f, 0.00f, 0.00f, 0.92f, 8.74f, 0.00f, 2.58f, 2.42f, 1.32f, 4.53f, 0.00f, 0.00f},   // v2_256x256x64r3w8
+    };
+    const TilePrice* const prices = pre ? pre_prices : plain_prices;
+    int count = pre ? sizeof(pre_prices) / sizeof(TilePrice) : sizeof(plain_prices) / sizeof(TilePrice);
+    const int64_t cu = cu_count > 0 ? cu_count : 256, t128 = (int64_t)((a.OC + 127) / 128) * (((int64_t)a.M + 127) / 128);
+    if (pre && t128 < 4 * cu) count -= 2;  // tiles of 256 channels: only where every CU has several (fitted there alone)
+    if (split_only) return cheapest_tile(prices, SPLIT, a, cu_count);
+    const int64_t split_most = pre ? 400 : kSplitFew;
+    const bool split = split_tiles(a) <= split_most || a.OC <= 32;
+    return split ? cheapest_tile(prices, count, a, cu_count) : cheapest_tile(prices + SPLIT, count - SPLIT, a, cu_count);
+}
+
+// the tile for few output pixels, or -1 where there are too many
+static int pick_split(const IgemmArgs& a, const ConvProblem& p, bool pre, int cu_count) {
+    const int first = igemm_first_ks_cfg();
+    if (p.pin != 32) {
+        const int ks = igemm5_pick(a, p.pin, p.pout);
+        return ks >= 0 ? first + ks : -1;
+    }
+    if (split_tiles(a) > kSplitFew) return -1;
+    const int cfg = pick_by_price(a, pre, true, cu_count);
+    return igemm5_can_run(a, p.pin, p.pout, cfg - first) ? cfg : -1;
+}
+
 static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_preprocess) {
     const mi355_conv_desc& d = p.d;
     if (p.pout == 1) {
@@ -656,8 +712,8 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         if (d.group == 1 && inner_planar(p)) {
             IgemmArgs a;
             igemm_fill_args(p, a);
-            const int ks = igemm5_pick(a, p.pin, p.pout);
-            if (ks >= 0) return igemm_first_ks_cfg() + ks;
+            const int ks = pick_split(a, p, will_preprocess, cu_count);
+            if (ks >= 0) return ks;
         }
         if (p.pin == 32)
             return igemm_first_v2_cfg() + (p.ocpg <= 64 || 2 * t128 < 3 * (int64_t)(cu_count > 0 ? cu_count : 256) ? 3 : 0);
@@ -670,8 +726,8 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         igemm_fill_args(p, a);
         // NCHW4 pointwise at stride 1: four pixels per lane, at any number of pixels
         if (pw4_quad_pick(a, p.pin, p.pout)) return pw4s_usable(a) ? kNumCfgs + igemm_dma_num_cfgs() - 1 : igemm_pw4_split_cfg();
-        const int ks = igemm5_pick(a, p.pin, p.pout);
-        if (ks >= 0) return igemm_first_ks_cfg() + ks;
+        const int ks = pick_split(a, p, will_preprocess, cu_count);
+        if (ks >= 0) return ks;
         const int p4 = patch4_pick(a, p.pin, p.pout);
         if (p4 >= 0) return igemm_first_p4_cfg() + p4;
         const int g32 = igemm_needs_general(p) ? -1 : grp32_pick(a, p.pin, p.pout, will_preprocess);
@@ -717,47 +773,27 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         const int s = igemm_pw32s_cfg();
         if ((d.ic <= 64 || igemm_takes_table(p)) && igemm_resolve_cfg(p, s) == s) return s;
     }
-    if (will_preprocess && p.pin == 32 && p.pout == 32 && d.group == 1 && !igemm_needs_general(p)) {
-        // The caller re-tiles the filter for the chosen algorithm (weight pre-processing): the second-generation tiles
-        // then copy whole kilobytes for both operands.  Every tile was forced on every ResNet-50 shape in turn and timed
-        // as whole-stack replays of one captured graph, against the unchanged stack in the same process.
-        enum { V128x128x64r4 = 0, V128x128x128r3 = 2, V64x128x128r3 = 3, V64x128x64r4 = 4, V64x64x128r3 = 7, V64x64x128r4 = 8, V128x256x64w8 = 10, V256x256x64w8 = 11 };
-        enum { V3_128x128x256r3 = 6 };
-        const int v2 = igemm_first_v2_cfg();
-        const int cu = cu_count > 0 ? cu_count : 256;
-        const int64_t M = (int64_t)d.n * p.oh * p.ow;
-        const int64_t t128 = ((d.oc + 127) / 128) * ((M + 127) / 128);
-        const int kb = (int)(p.icpg * d.fh * d.fw);
-        const bool pw = d.fh == 1 && d.fw == 1 && d.pad_h == 0 && d.pad_w == 0;
-        // Large convolutions (six and more 128 x 128 tiles per CU, long reductions), with or without a residual: the
-        // 8-wave tiles of 256 rows or columns, which read a residual in the epilogue instead of staging it in LDS
-        // (1.8 / 2.2 / 2.1 Pop/s against 1.5 / 1.9 / 1.9 on the first-generation tiles for 3x3 256->256 at 64x64, 3x3
-        // stride 2 512->1024 at 32x32 and 5x5 128->128 at 80x80, batch 128, residual + H_SWISH).
-        if (t128 >= 6 * (int64_t)cu && kb >= 1024 && d.oc > 64) return v2 + (d.oc >= 256 ? V256x256x64w8 : V128x256x64w8);
-        if (!d.has_z) {
-            // the layers without a residual; the others stay on the first-generation tiles below, where the residual
-            // costs no LDS
-            if (d.oc <= 64) return v2 + V64x128x64r4;
-            if (t128 >= cu) return v2 + V128x128x64r4;
-            // a handful of tiles (small batches): the smallest tile puts the most CUs to work (3x3 256->256 at 14x14,
-            // batch 1 and 8: 7.4 / 7.6 us against 8.9 / 9.1 on 64 x 128 tiles)
-            const int64_t t64 = (int64_t)((d.oc + 63) / 64) * ((M + 127) / 128);
-            if (2 * t64 < cu) return v2 + V64x64x128r3;
-            const bool s1 = d.stride_h == 1 && d.stride_w == 1;
-            // 3x3 over 256 channels at stride 1 with one 128 x 128 tile for most CUs: the patch-staged tile, whose stage of
-            // eight k-chunks halves both the bytes through the CU's copy path and the stage boundaries (-1.4 us per
-            // launch against the tile below on 256 -> 256 at 14 x 14, batch 64; falls back when the patch does not fit)
-            if (d.fh == 3 && d.fw == 3 && s1 && kb >= 2304 && kb < 4608 && 2 * t128 >= cu) return igemm_first_v3_cfg() + V3_128x128x256r3;
-            // long reductions with a 128 x 128 tile for more than half of the CUs: that tile, with half the operand bytes per
-            // MAC of the 64 x 64 one (2048 -> 512 at 7 x 7, batch 128: 8.9 against 12.6 us; 3x3 512 -> 512: 17 against 24.6)
-            if (kb >= 2048 && 2 * t128 > cu && (pw || s1 || kb >= 4608)) return v2 + V128x128x128r3;
-            // pointwise: more pixels than channels per tile; with few tiles and a very long reduction the small tile with
-            // the deepest ring
-            if (pw) return v2 + (kb >= 2048 ? V64x64x128r4 : V64x128x128r3);
-            if (kb >= 4608) return v2 + V64x64x128r4;
-            if (s1) return v2 + V64x128x128r3;
-            // few tiles, strided 3x3 over at most 256 channels: the first-generation tiles below
+    if (p.pin == 32 && d.group == 1 && !igemm_needs_general(p)) {
+        IgemmArgs a;
+        igemm_fill_args(p, a);
+        if (will_preprocess && p.pout == 32 && !d.has_z && d.oc > 64 && d.stride_h == 1 && d.stride_w == 1) {
+            // Three places where the prices of a pre-processed filter cannot tell what timing every tile does
+            const int v2 = igemm_first_v2_cfg(), cu = cu_count > 0 ? cu_count : 256;
+            enum { V64x128x128r3 = 3, V64x64x128r4 = 8, V3_128x128x256r3 = 6 };
+            const int64_t t128 = (int64_t)((d.oc + 127) / 128) * (((int64_t)a.M + 127) / 128);
+            const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0, one_round = 2 * t128 >= cu && t128 < cu;
+            // 3x3 over 256 channels with one 128 x 128 tile for most CUs: the patch-staged tile, whose stage of eight k-chunks
+            // halves both the bytes through the CU's copy path and the stage boundaries (41 layers: 1.005 times the best tile,
+            // by price 1.03; falls back when the patch does not fit)
+            if (d.fh == 3 && d.fw == 3 && a.kbytes >= 2304 && a.kbytes < 4608 && one_round) return igemm_first_v3_cfg() + V3_128x128x256r3;
+            // pointwise over 1024 to 2047 channels, the same number of tiles: more pixels than channels per tile (inside a network,
+            // where weights are cold; by itself, warm, it is 1.07 times the 8-wave 128 x 128 tile)
+            if (pw && a.kbytes >= 1024 && a.kbytes < 2048 && one_round) return v2 + V64x128x128r3;
+            // windows over 4608 bytes and more with few tiles, but too many to split the reduction: the smallest tile with the deepest
+            // ring (3x3 over 512 channels, 200 to 490 of them: 0.97 .. 1.0 times the 64 x 128 tile of eight waves)
+            if (a.T > 1 && a.kbytes >= 4608 && split_tiles(a) > 400 && 2 * t128 < cu) return v2 + V64x64x128r4;
         }
+        return pick_by_price(a, will_preprocess, false, cu_count);
     }
     const int64_t M = (int64_t)d.n * p.oh * p.ow;
     const int OC = d.oc;
@@ -792,39 +828,8 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
     if (OC <= 32) {
         // 32 x 256 tiles waste no matrix rows, but need enough pixels to fill the chip (measured on the 4-packed
         // 1x1 projections of MobileNetV2)
-        if (p.pin == 32 || tiles(4) >= 2 * cu_count) return 4;
+        if (tiles(4) >= 2 * cu_count) return 4;
         return tiles(0) >= cu_count ? 0 : 3;
-    }
-    if (p.pin == 32) {
-        // 32-packed inputs: LDS-direct tiles (ids after the register-staged ones).  t128 = number of 128x128 tiles.
-        // A plain filter over 256 bytes and more, or with a window, goes by prices.  What is left to the lines below reads the
-        // reference layout too: callers that pre-process the filter, for layers with a residual (which costs these tiles no LDS;
-        // chosen from a sweep of every tile over the ResNet-50 and large-convolution shapes inside their networks, where weights
-        // are cold), for strided windows on few tiles, and for 4-packed outputs; and pointwise layers over at most 224 channels.
-        enum {
-            D128x128x64 = kNumCfgs + 0, D64x64x128 = kNumCfgs + 1, D128x128x128r2 = kNumCfgs + 7, D64x64x64r4 = kNumCfgs + 10,
-            D128x64x128r2 = kNumCfgs + 11, D64x128x128r2 = kNumCfgs + 13, D128x128x64w8 = kNumCfgs + 14,
-            D128x64x128w8 = kNumCfgs + 15, D256x128x64w8 = kNumCfgs + 16, D128x128x128r2w8 = kNumCfgs + 17,
-            D64x64x128r2 = kNumCfgs + 6, D64x128x128w8 = kNumCfgs + 18, D64x64x128r4 = kNumCfgs + 12
-        };
-        if (!will_preprocess && (d.fh * d.fw > 1 || kbytes >= 256)) return pick_plain_cfg(M, OC, kbytes, d.fh * d.fw > 1, d.stride_h * d.stride_w > 1, d.has_z != 0, cu_count);
-        if (OC <= 64) return kbytes <= 64 ? D128x128x64w8 : kbytes <= 256 ? D64x64x128r2 : D64x128x128r2;
-        const int64_t t128 = tiles(0);
-        // layers with a residual and a short reduction (the expanding 1x1 of a bottleneck block) are bound by their
-        // epilogue: three 8-wave workgroups per CU at every size (whole-stack graph replays, each tile in turn)
-        if (d.has_z && t128 >= cu_count && (kbytes <= 128 || (kbytes <= 512 && t128 < 2 * cu_count))) return D128x128x64w8;
-        if (t128 >= 4 * cu_count)
-            return kbytes >= 1024 ? (OC >= 256 ? D256x128x64w8 : D128x128x128r2) : (kbytes <= 128 ? D128x128x64w8 : D128x128x128r2w8);
-        if (t128 >= 2 * cu_count) return D128x64x128r2;
-        if (2 * t128 >= 3 * cu_count) return kbytes >= 512 ? D128x128x128r2w8 : D128x128x64;
-        // few tiles, long reductions: the deeper ring hides the cold first touch of every weight byte; the longest
-        // ones (strided 3x3 over 256 channels) run best with more pixels than channels per tile
-        if (kbytes >= 2304 && tiles(6) >= cu_count) return D64x128x128w8;
-        if (tiles(7) >= cu_count) return D128x64x128w8;
-        // fewer tiles than CUs: the longest reductions take the deepest ring, those of 2048 to 4607 bytes with a 64 x 128 tile for
-        // three CUs of four the 8-wave tile with more pixels than channels
-        if (kbytes >= 4608) return D64x64x128r4;
-        return kbytes >= 2048 && 4 * tiles(6) >= 3 * cu_count ? D64x128x128w8 : D64x64x128;
     }
     if (OC <= 64) return tiles(1) >= cu_count ? 1 : 3;
     // 4-packed windowed layers that are not on the patch tiles: the gather of their operands bounds them, which a 128 x 128 tile

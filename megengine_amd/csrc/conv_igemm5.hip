@@ -529,12 +529,10 @@ int launch_ks(hipStream_t st, const KsArgs<FastDiv>& k, uint32_t n, int lds, boo
 int igemm5_num_cfgs() { return kKsCount; }
 const char* igemm5_cfg_name(int cfg) { return kKs[cfg].name; }
 
-// The tile for a problem, or -1 where the staged tiles are the better ones.  The line between them is the number of
-// workgroups a tile would make: up to about one per CU this kernel hides what the staged tiles wait for, beyond that its
-// operand traffic costs more.  Drawn from the ResNet-50 and MobileNetV2 layers at batch 1 to 64 (sizes 128 to 263), each on
-// every tile: the choice is within 2 % of the best tile over each network's layers.  At batch 1 its layers sum to 178 us
-// instead of 255 (3x3 over 512 channels at 7 x 7: 11.0 -> 4.2 us; over 256 at 14 x 14: 7.2 -> 3.4; 1024 -> 256 at 14 x 14:
-// 4.3 -> 3.0), the pointwise layers of MobileNetV2 to 115 instead of 140.
+// The tile for a 4-packed problem, or -1 where the staged tiles are the better ones (32-packed ones go by prices, conv_igemm.hip).  The
+// line between them is the number of workgroups a tile would make: up to about one per CU this kernel hides what the staged tiles wait
+// for, beyond that its operand traffic costs more.  (At batch 1 the layers of ResNet-50 sum to 178 us instead of 255 with these tiles, 3x3
+// over 512 channels at 7 x 7: 11.0 -> 4.2 us; over 256 at 14 x 14: 7.2 -> 3.4; the pointwise layers of MobileNetV2 to 115 instead of 140.)
 static int ks_id(int pin, int s, int mt, int waves) {
     for (int i = 0; i < kKsCount; ++i)
         if (kKs[i].pin == pin && kKs[i].s == s && kKs[i].mt == mt && kKs[i].waves == waves) return i;
@@ -542,17 +540,12 @@ static int ks_id(int pin, int s, int mt, int waves) {
 }
 int igemm5_pick(const IgemmArgs& a, int pin, int pout) {
     auto tiles = [&](int bm, int bn) { return (int64_t)((a.OC + bm - 1) / bm) * ((a.M + bn - 1) / bn); };
+    if (pin != 4) return -1;
     const int64_t g16 = tiles(16, 16), g32 = tiles(32, 32), g64 = tiles(64, 32);
     const int K = a.kbytes;
     const bool window = a.T > 1;
     int id = -1;
-    if (pin == 32) {
-        if (K >= 512 && g16 <= 256) id = ks_id(32, 16, 1, K >= 2048 ? 8 : 4);
-        else if (K >= 512 && window && g16 <= 600) id = ks_id(32, 16, 1, 4);
-        else if (g32 <= 256 && (K < 1024 || g16 <= 600)) id = ks_id(32, 32, 1, K >= 2048 && !window ? 8 : 4);
-        else if (g32 <= 200 && window && K >= 1024) id = ks_id(32, 32, 1, 4);
-        else if (g64 <= 256) id = ks_id(32, 32, 2, K >= 512 || K <= 128 ? 8 : 4);
-    } else if (window) {
+    if (window) {
         // Against the 4-packed patch tiles: they pay a fixed price per 32 input channels, this kernel one per pixel and tap.
         // Graph replays of every tile, us, ks against patch: 128 -> 128 at 28 x 28, batch 1 (g16 = 392): 5.4 / 5.9, batch 4:
         // 6.8 / 6.0; 232 -> 72 at 40 x 16, stride 2, batch 12: 8.9 / 10.8; 5x5 64 -> 64 at 32 x 32, batch 8: 8.0 / 8.9;

@@ -539,7 +539,7 @@ int launch_grp4(hipStream_t st, const ConvProblem& p, const int8_t* src, const i
 int igemm5_num_cfgs();
 const char* igemm5_cfg_name(int cfg);
 bool igemm5_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
-int igemm5_pick(const IgemmArgs& a, int pin, int pout);  // the tile for few output pixels, -1 where there are too many
+int igemm5_pick(const IgemmArgs& a, int pin, int pout);  // the 4-packed tile for few output pixels, -1 where there are too many
 int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg);
 
 // windowed layers on 4-packed tensors: the input patch of a tile turned to 16 channels per pixel in LDS (conv_patch4.hip)

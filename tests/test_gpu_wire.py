@@ -26,7 +26,7 @@ def _desc(fmt, n, ic, h, w, oc, f, gap=None, **kw):
 
 # kernel, format, (n, ic, h, w, oc, f) and the rest: edges of tiles and odd sizes, every family that has a wire
 CASES = [
-    ("ks_kernel<32, 32, 1, 4, true>", "NCHW32", (2, 64, 11, 13, 96, 1), dict(nonline="RELU")),
+    ("ks_kernel<32, 16, 1, 4, true>", "NCHW32", (2, 64, 11, 13, 96, 1), dict(nonline="RELU")),
     ("ks_kernel<32, 16, 1, 4, false>", "NCHW32", (3, 96, 9, 7, 96, 3), dict(nonline="H_SWISH", stride=2)),
     ("ks_kernel<32, 32, 2, 8, false>", "NCHW32", (2, 64, 21, 19, 352, 5), dict()),
     ("ks_kernel<4, 16, 1, 8, false>", "NCHW4", (2, 132, 9, 11, 36, 3), dict(nonline="RELU")),
