@@ -57,9 +57,10 @@ int igemm_pick_cfg(const ConvProblem& p, int cu_count, bool will_preprocess = fa
 // the tile the launch code takes in its place (another kernel generation for this packing, a tile that has the general
 // epilogue, a ring that fits the LDS).  A choice of the heuristic is replaced silently; a tile the caller forced is not.
 int igemm_resolve_cfg(const ConvProblem& p, int tile_cfg);
-// flt_preprocessed: flt points to the artefact of launch_igemm_preprocess (only tiles with igemm_preprocessed_bytes > 0)
+// flt_preprocessed: flt points to the artefact of launch_igemm_preprocess (only tiles with igemm_preprocessed_bytes > 0), or to one
+// with flt_rows rows to a chunk, the channels without their padding to whole blocks
 int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int tile_cfg, int cu_count, const int8_t* src,
-                      const int8_t* flt, const int32_t* bias, const int8_t* z, int8_t* dst, bool flt_preprocessed = false);
+                      const int8_t* flt, const int32_t* bias, const int8_t* z, int8_t* dst, bool flt_preprocessed = false, int flt_rows = 0);
 // weight pre-processing: bytes of the re-tiled filter for this problem and tile (0: the tile reads the reference
 // layout only), and the pass that writes it
 size_t igemm_preprocessed_bytes(const ConvProblem& p, int tile_cfg);

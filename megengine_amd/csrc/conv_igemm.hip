@@ -699,7 +699,10 @@ static int pick_split(const IgemmArgs& a, const ConvProblem& p, bool pre, int cu
         const int ks = igemm5_pick(a, p.pin, p.pout);
         return ks >= 0 ? first + ks : -1;
     }
-    if (split_tiles(a) > kSplitFew) return -1;
+    // A planar destination has but one other tile, 64 x 128, until 128 x 128 ones fill the device: the line is further out there (1760 drawn
+    // plain NCHW layers, every seventh on these tiles or at the line: none slower than with thresholds on 16 x 16 and 32 x 32 tiles by
+    // more than 4 %; at 256 for all, layers into 4 to 15 channels with 260 to 300 of these tiles were 1.4 to 1.8 times as long).
+    if (split_tiles(a) > (p.pout != 1 ? kSplitFew : a.OC <= 32 ? 800 : 400)) return -1;
     const int cfg = pick_by_price(a, pre, true, cu_count);
     return igemm5_can_run(a, p.pin, p.pout, cfg - first) ? cfg : -1;
 }
@@ -1007,7 +1010,7 @@ int igemm_resolve_cfg(const ConvProblem& p, int cfg) {
 }
 
 int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_count, const int8_t* src,
-                      const int8_t* flt, const int32_t* bias, const int8_t* z, int8_t* dst, bool flt_preprocessed) {
+                      const int8_t* flt, const int32_t* bias, const int8_t* z, int8_t* dst, bool flt_preprocessed, int flt_rows) {
     if (igemm_group_by_launch(p)) {
         if (flt_preprocessed) return (int)hipErrorInvalidValue;
         if (cfg == igemm_grp4_cfg() && grp4_usable(p)) return launch_grp4(st, p, src, flt, bias, z, dst);
@@ -1032,10 +1035,10 @@ int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_coun
     if (cfg < 0) return (int)hipErrorInvalidValue;
     if (flt_preprocessed) {
         if (igemm_preprocessed_bytes(p, cfg) == 0) return (int)hipErrorInvalidValue;
-        const int ocp = (a.OC + 31) / 32 * 32;
+        const int rows = flt_rows ? flt_rows : (a.OC + 31) / 32 * 32;
         a.flt_rstride = 32;
-        a.flt_kstride = ocp * 32;
-        a.flt_bytes = (uint32_t)igemm_preprocessed_bytes(p, cfg);
+        a.flt_kstride = rows * 32;
+        a.flt_bytes = (uint32_t)a.KC * (uint32_t)a.flt_kstride;
     }
     if (p.pout == 1) {
         if (p.d.bias_mode == MI355_BIAS_NONE) a.bias = nullptr;  // the planar epilogue tests the pointer

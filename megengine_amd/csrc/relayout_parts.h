@@ -61,8 +61,9 @@ static inline SmallPlanes make_small_planes(uint32_t n, uint32_t c, uint32_t hw,
     g.cb = make_fastdiv(g.CB);
     return g;
 }
+// `images` (not zero): not image by image, but [channel block][pixel][image][pack channels], the order of a pre-processed filter
 __device__ __forceinline__ void small_planes_quad(const int8_t* __restrict__ src, uint32_t* __restrict__ dst, const SmallPlanes& g,
-                                                  uint32_t it) {
+                                                  uint32_t it, uint32_t images = 0) {
     if (it >= g.items) return;
     const uint32_t k = it & ((1u << g.log_quads) - 1), t = it >> g.log_quads;
     const uint32_t b = fdiv(t, g.hw), px = t - b * g.HW;
@@ -72,7 +73,7 @@ __device__ __forceinline__ void small_planes_quad(const int8_t* __restrict__ src
 #pragma unroll
     for (uint32_t q = 0; q < 4; ++q)
         if (c0 + q < g.C) w |= (uint32_t)(uint8_t)s[(int64_t)q * g.HW] << (8 * q);
-    dst[it] = w;
+    dst[images ? (((((b - n * g.CB) * g.HW + px) * images + n) << g.log_quads) + k) : it] = w;
 }
 
 }  // namespace
