@@ -685,7 +685,8 @@ static int pick_by_price(const IgemmArgs& a, bool pre, bool split_only, int cu_c
     const TilePrice* const prices = pre ? pre_prices : plain_prices;
     int count = pre ? sizeof(pre_prices) / sizeof(TilePrice) : sizeof(plain_prices) / sizeof(TilePrice);
     const int64_t cu = cu_count > 0 ? cu_count : 256, t128 = (int64_t)((a.OC + 127) / 128) * (((int64_t)a.M + 127) / 128);
-    if (pre && t128 < 4 * cu) count -= 2;  // tiles of 256 channels: only where every CU has several (fitted there alone)
+    // tiles of 256 channels: where every CU has several and they are not bound by bytes (fitted there; below, 1.08 times the best of 38 layers)
+    if (pre && (t128 < 4 * cu || a.kbytes < 512)) count -= 2;
     if (split_only) return cheapest_tile(prices, SPLIT, a, cu_count);
     const int64_t split_most = pre ? 400 : kSplitFew;
     const bool split = split_tiles(a) <= split_most || a.OC <= 32;
@@ -773,8 +774,14 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         // 128 -> 512 at 28 x 28: 14.6 against 16.1)
         // Over at most 64 channels the streaming kernel wins without a table too (64 -> 256 at 56 x 56 with the
         // multi-step form, inside the ResNet-50 stack: -4 us per step against the tiled kernel, alternating bench runs).
+        // Without a table, us of the streaming kernel against the 64 x 64 tile with 64 bytes to a stage (both filter layouts): over 64
+        // channels 1.06 .. 1.11 to 5 million outputs, beyond 0.95 and 0.81 (64 -> 256 at 56 x 56, batch 1: 4.8 / 4.2; at 24 x 38, batch
+        // 12: 6.1 / 5.2); over 32 it is ahead everywhere; over 96 against the best of all: 1.0 to 2 million, 0.97 to 10, then 0.84.
         const int s = igemm_pw32s_cfg();
-        if ((d.ic <= 64 || igemm_takes_table(p)) && igemm_resolve_cfg(p, s) == s) return s;
+        const int64_t outputs = (int64_t)d.n * p.oh * p.ow * d.oc;
+        const bool table = igemm_takes_table(p);
+        if (!table && d.ic == 64 && d.oc > 32 && outputs < 5000000) return kNumCfgs + 10;  // dma64x64x64r4
+        if ((table || d.ic <= 64 || (d.ic <= 96 && outputs >= 2000000)) && igemm_resolve_cfg(p, s) == s) return s;
     }
     if (p.pin == 32 && d.group == 1 && !igemm_needs_general(p)) {
         IgemmArgs a;
