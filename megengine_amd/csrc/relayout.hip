@@ -114,56 +114,78 @@ __global__ __launch_bounds__(256) void relayout_generic_kernel(RelayoutArgs a) {
 // (the memory pipe takes them at full rate as long as a wave's run is contiguous).  The last 16 pixels of a plane start
 // at HW - 16, so they overlap the run before them and both write the same bytes: no tail code, every lane does the same.
 //
-// NCHW -> NCHW4 (C any: missing channels are zero), HW >= 16.  Thread: 4 channels x 16 pixels.
-// grid.x covers CB * ceil(HW / 16) work items per image, grid.y = N.  3 x 224 x 224, batch 64 (the image of a first
-// layer): 53 us one byte per thread, 8.4 here.
+// NCHW -> NCHW4 (C any: missing channels are zero), HW >= 4.  A step is 4 pixels of 4 channels: a wave loads 256 consecutive bytes of
+// each channel and stores one contiguous kilobyte.  (With 16 pixels to a thread the loads are four times as wide, but a store covers a
+// quarter of 64 lines, and small images leave the chip idle.)  A thread takes STEPS of them, 64 steps apart, whose loads are in flight
+// together.  The last step of a plane ends with it: its first pixels are written twice, with the same bytes.
+// grid.x covers CB * ceil(HW / 4) steps per image, grid.y = N.  3 x 224 x 224 (the image of a first layer), against
+// 16 pixels to a thread: batch 1 2.55 -> 2.29 us, 16 3.36 -> 2.70, 64 7.50 -> 4.48; 256 x 64 x 64, batch 32: 16.6 -> 11.2 (6 TB/s).
+template <int STEPS>
 __global__ __launch_bounds__(256) void nchw_to_nchw4_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
-                                                            uint32_t C, uint32_t HW, uint32_t items, FastDiv pq) {
-    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
-    if (it >= items) return;
-    const uint32_t cg = fdiv(it, pq), pb = it - cg * pq.d;
-    const uint32_t px = pb * 16 + 16 <= HW ? pb * 16 : HW - 16;
+                                                            uint32_t C, uint32_t HW, uint32_t steps, FastDiv pq) {
+    const uint32_t first = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * STEPS) + (threadIdx.x & 63);
     const uint32_t CB = (C + 3) / 4;
-    const int8_t* s = src + ((int64_t)blockIdx.y * C + cg * 4) * HW + px;
-    const uint32_t have = C - cg * 4;
-    u32x4 r[4];
+    const int8_t* image = src + (int64_t)blockIdx.y * C * HW;
+    int8_t* out = dst + (int64_t)blockIdx.y * CB * HW * 4;
+    uint32_t r[STEPS][4];
+    int64_t at[STEPS];
 #pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-        r[k] = u32x4{0, 0, 0, 0};
-        if (k < have) r[k] = load16u(s + (int64_t)k * HW);
+    for (int i = 0; i < STEPS; ++i) {
+        const uint32_t it = first + i * 64 < steps ? first + i * 64 : steps - 1;
+        const uint32_t cg = fdiv(it, pq), pb = it - cg * pq.d;
+        const uint32_t px = pb * 4 + 4 <= HW ? pb * 4 : HW - 4;
+        const int8_t* s = image + (int64_t)cg * 4 * HW + px;
+        const uint32_t have = C - cg * 4;
+        at[i] = ((int64_t)cg * HW + px) * 4;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            r[i][k] = 0;
+            if (k < have) r[i][k] = load4u(s + (int64_t)k * HW);
+        }
     }
-    int8_t* d = dst + (((int64_t)blockIdx.y * CB + cg) * HW + px) * 4;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int i = 0; i < STEPS; ++i) {
+        if (first + i * 64 >= steps) return;
         uint32_t c0, c1, c2, c3;
-        transpose4x4(r[0][j], r[1][j], r[2][j], r[3][j], c0, c1, c2, c3);
-        store16u(d + j * 16, u32x4{c0, c1, c2, c3});
+        transpose4x4(r[i][0], r[i][1], r[i][2], r[i][3], c0, c1, c2, c3);
+        store16u(out + at[i], u32x4{c0, c1, c2, c3});
     }
 }
 
-// NCHW4 -> NCHW (the first C channels), HW >= 16.
+// NCHW4 -> NCHW (the first C channels), HW >= 4: the same steps the other way round.  Against 16 pixels to a thread: 64 x 56 x 56, batch 64
+// 5.13 -> 4.48 us, batch 1 2.37 -> 2.31, the largest the same (256 x 64 x 64, batch 32: 10.8 and 10.9).
+template <int STEPS>
 __global__ __launch_bounds__(256) void nchw4_to_nchw_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
-                                                            uint32_t C, uint32_t HW, uint32_t items, FastDiv pq) {
-    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
-    if (it >= items) return;
-    const uint32_t cg = fdiv(it, pq), pb = it - cg * pq.d;
-    const uint32_t px = pb * 16 + 16 <= HW ? pb * 16 : HW - 16;
+                                                            uint32_t C, uint32_t HW, uint32_t steps, FastDiv pq) {
+    const uint32_t first = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * STEPS) + (threadIdx.x & 63);
     const uint32_t CB = (C + 3) / 4;
-    const int8_t* s = src + (((int64_t)blockIdx.y * CB + cg) * HW + px) * 4;
-    u32x4 o[4];
+    const int8_t* image = src + (int64_t)blockIdx.y * CB * HW * 4;
+    int8_t* out = dst + (int64_t)blockIdx.y * C * HW;
+    u32x4 v[STEPS];
+    uint32_t group[STEPS], pixel[STEPS];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const u32x4 v = load16u(s + j * 16);  // 4 pixels x 4 channels
-        uint32_t c0, c1, c2, c3;
-        transpose4x4(v[0], v[1], v[2], v[3], c0, c1, c2, c3);
-        o[0][j] = c0; o[1][j] = c1; o[2][j] = c2; o[3][j] = c3;
+    for (int i = 0; i < STEPS; ++i) {
+        const uint32_t it = first + i * 64 < steps ? first + i * 64 : steps - 1;
+        const uint32_t cg = fdiv(it, pq), pb = it - cg * pq.d;
+        group[i] = cg;
+        pixel[i] = pb * 4 + 4 <= HW ? pb * 4 : HW - 4;
+        v[i] = load16u(image + ((int64_t)cg * HW + pixel[i]) * 4);  // 4 pixels x 4 channels
     }
-    int8_t* d = dst + ((int64_t)blockIdx.y * C + cg * 4) * HW + px;
-    const uint32_t have = C - cg * 4;
 #pragma unroll
-    for (uint32_t k = 0; k < 4; ++k)
-        if (k < have) store16u(d + (int64_t)k * HW, o[k]);
+    for (int i = 0; i < STEPS; ++i) {
+        if (first + i * 64 >= steps) return;
+        uint32_t o[4];
+        transpose4x4(v[i][0], v[i][1], v[i][2], v[i][3], o[0], o[1], o[2], o[3]);
+        int8_t* d = out + (int64_t)group[i] * 4 * HW + pixel[i];
+        const uint32_t have = C - group[i] * 4;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            if (k < have) store4u(d + (int64_t)k * HW, o[k]);
+    }
 }
+
+// 4 steps to a thread where that leaves four workgroups and more for every CU; below, a launch is its latency and threads are what it lacks
+static bool four_steps(uint64_t steps, uint32_t N) { return steps * N >= 4ull * 256 * 4 * 256; }
 
 // NCHW4 <-> NCHW32: dwords change places.  Two threads per pixel of a 32-channel block, each moves 16 channels: on the
 // NCHW32 side a wave covers one contiguous kilobyte, on the other side two runs of 128 bytes per access.
@@ -303,10 +325,13 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
             case MI355_RL_NCHW_NCHW4_IC_SMALL:
             case MI355_RL_NCHW_NCHW32: {
                 const uint32_t C = d.shape[1], CB = oshape[1];
-                const uint32_t pq = (HW + 15) / 16;
-                if (oshape[4] == 4 && HW >= 16 && numbered((uint64_t)CB * pq)) {
-                    const uint32_t items = CB * pq;
-                    return launch_kernel(nchw_to_nchw4_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, items,
+                const uint32_t pq = (HW + 3) / 4;
+                if (oshape[4] == 4 && HW >= 16 && numbered((uint64_t)CB * pq + 1024)) {
+                    const uint32_t steps = CB * pq;
+                    if (four_steps(steps, N))
+                        return launch_kernel(nchw_to_nchw4_kernel<4>, dim3((steps + 1023) / 1024, N), dim3(256), 0, st, s8, d8, C, HW,
+                                             steps, make_fastdiv(pq));
+                    return launch_kernel(nchw_to_nchw4_kernel<1>, dim3((steps + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, steps,
                                          make_fastdiv(pq));
                 }
                 // planes of a quarter of the LDS tile and more: below, most of a tile's threads would find no pixel
@@ -318,9 +343,12 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
                                      reinterpret_cast<uint32_t*>(dst), g);
             }
             case MI355_RL_NCHW4_NCHW:
-                if (HW >= 16 && numbered((uint64_t)d.shape[1] * ((HW + 15) / 16))) {
-                    const uint32_t C = oshape[1], pq = (HW + 15) / 16, items = d.shape[1] * pq;
-                    return launch_kernel(nchw4_to_nchw_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, items,
+                if (HW >= 16 && numbered((uint64_t)d.shape[1] * ((HW + 3) / 4) + 1024)) {
+                    const uint32_t C = oshape[1], pq = (HW + 3) / 4, steps = d.shape[1] * pq;
+                    if (four_steps(steps, N))
+                        return launch_kernel(nchw4_to_nchw_kernel<4>, dim3((steps + 1023) / 1024, N), dim3(256), 0, st, s8, d8, C, HW,
+                                             steps, make_fastdiv(pq));
+                    return launch_kernel(nchw4_to_nchw_kernel<1>, dim3((steps + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, steps,
                                          make_fastdiv(pq));
                 }
                 break;

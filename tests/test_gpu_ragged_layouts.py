@@ -73,3 +73,18 @@ def test_large_tensors(shape):
         for lo in range(n):
             assert torch.equal(z[lo].view(c // 32, h * w, 8, 4).permute(0, 2, 1, 3).reshape(c // 4, h, w, 4), y[lo]), lo
         assert torch.equal(ops.relayout_exec(ops.relayout_desc(_abi.RL_NCHW32_NCHW4, tuple(z.shape)), z), y)
+
+
+@pytest.mark.parametrize("n,c,h,w", [(9, 5, 1031, 481), (9, 3, 1031, 481), (4096, 4, 33, 31), (2, 12, 3, 700001), (1, 4, 2048, 2047), (1, 4, 2048, 2048)])
+def test_nchw4_with_several_steps_to_a_thread(n, c, h, w):
+    """Both sides of the line (2^22 pixels of a channel block in all), last steps that overlap and threads with a part of their
+    steps.  A layout conversion moves bytes, so torch's own copies are the reference."""
+    x = torch.randint(-128, 128, (n, c, h, w), dtype=torch.int8, device="cuda")
+    blocks = (c + 3) // 4
+    want = torch.zeros((n, blocks * 4, h, w), dtype=torch.int8, device="cuda")
+    want[:, :c] = x
+    want = want.view(n, blocks, 4, h, w)
+    y = ops.relayout_exec(ops.relayout_desc(_abi.RL_NCHW_NCHW4_IC_SMALL if c < 4 else _abi.RL_NCHW_NCHW4, (n, c, h, w)), x)
+    assert torch.equal(y, want.permute(0, 1, 3, 4, 2))
+    back = ops.relayout_exec(ops.relayout_desc(_abi.RL_NCHW4_NCHW, tuple(y.shape)), y)
+    assert torch.equal(back, want.reshape(n, blocks * 4, h, w))
