@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256) void pooling_kernel(PoolArgs a) {
 // at batch 64).  Sixteen lanes share a window, lane k takes taps k, k + 16, ..., and a butterfly adds the partial sums up:
 // in each of its first steps a lane hands half of its channels to its partner and keeps the other half, so 16 channels
 // cost 15 exchanges and every lane ends with one channel, whose byte it writes.
-// 7 x 7 x 2048: 5.5 us at batch 1, 7.4 us at batch 64.
+// 7 x 7 x 2048 in NCHW4: 2.6 us at batch 1, 5.0 us at batch 64.
 constexpr int POOL_LANES = 16;
 template <int PACK, int VB, int MODE>
 __global__ __launch_bounds__(256) void pooling_split_kernel(PoolArgs a, FastDiv div_fw) {
@@ -336,6 +336,126 @@ __global__ __launch_bounds__(256) void pooling_split_kernel(PoolArgs a, FastDiv 
     a.dst[((size_t)pix * UPP + sub) * VB + mine] = (int8_t)r;
 }
 
+// The same with a wave or several to a window.  Four channels to a lane: the 32 channels of an NCHW32 pixel are eight lanes, so a wave
+// loads eight taps, 256 bytes, at a time (NCHW4: 64 taps) and eight such loads are in flight.  A lane sums its four channels with one
+// byte dot product each (taps outside the window or the image are zeros), and the shares of a wave are added up in registers, 32 lanes
+// apart, 16, 8 and so on: in the first two exchanges a lane gives half of its channels for the other half of its partner's, so that it
+// ends with one channel to divide and to write.  Short code matters as much as the few exchanges: in a network it comes cold from
+// memory.  Several waves meet in LDS.  Against the kernel above:
+// NCHW32, 7 x 7 over 2048 channels: batch 1 5.1 -> 2.5 us, batch 64 6.9 -> 3.9; 4 x 4 at 32 x 32 over 256, batch 16: 10.5 -> 5.7; 28 x 28
+// over 512, batch 1: 11.4 -> 3.6; 56 x 56 over 256, batch 64: 48.7 -> 12.7.  NCHW4, 56 x 56 over 256, batch 1: 18.8 -> 3.2.
+template <int PACK, int MODE, int WAVES>
+__global__ __launch_bounds__(WAVES == 1 ? 256 : WAVES * 64) void pooling_wave_kernel(PoolArgs a, FastDiv div_fw) {
+    constexpr int UPP = PACK / 4, SHARES = 64 / UPP, STEP = WAVES * 8 * SHARES;
+    __shared__ int part[WAVES][WAVES == 1 ? 1 : PACK];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t pix = WAVES == 1 ? blockIdx.x * 4 + wave : blockIdx.x;
+    if (pix >= a.units / (PACK == 32 ? 2 : 1)) return;  // (all of a wave; of a workgroup where its waves meet)
+    const uint32_t lane = threadIdx.x & 63, sub = lane % UPP, share = lane / UPP;
+    const uint32_t t = fdiv(pix, a.div_ow), ow = pix - t * a.OW;
+    const uint32_t plane = fdiv(t, a.div_oh), oh = t - plane * a.OH;
+    const int ih0 = (int)oh * a.sh - a.ph, iw0 = (int)ow * a.sw - a.pw;
+    const int8_t* base = a.src + (size_t)plane * a.IH * a.IW * PACK;
+    const uint32_t taps = (uint32_t)(a.fh * a.fw);
+    Max4 most;
+    most.init();
+    int sum[4] = {0, 0, 0, 0};
+    for (uint32_t k0 = WAVES == 1 ? 0 : wave * (8 * SHARES); k0 < taps; k0 += STEP) {
+        uint32_t x[8];
+        bool ok[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t k = k0 + j * SHARES + share;
+            const uint32_t fh = fdiv(k, div_fw), fw = k - fh * a.fw;
+            const int ih = ih0 + (int)fh, iw = iw0 + (int)fw;
+            ok[j] = k < taps && (unsigned)ih < (unsigned)a.IH && (unsigned)iw < (unsigned)a.IW;
+            x[j] = *reinterpret_cast<const uint32_t*>(base + ((ok[j] ? (uint32_t)(ih * a.IW + iw) * PACK : 0u) + sub * 4));
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (MODE == POOL_MAX) {
+                most.feed(ok[j] ? x[j] : 0x80808080u);
+            } else {
+                const int w = ok[j] ? (int)x[j] : 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sum[q] = __builtin_amdgcn_sdot4(w, 1 << (8 * q), sum[q], false);
+            }
+        }
+    }
+    int8_t* out = a.dst + (size_t)pix * PACK;
+    if (MODE == POOL_MAX) {
+        uint32_t m[2] = {most.odd, most.even};
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const auto h = __builtin_amdgcn_permlane32_swap(m[q], m[q], false, false);
+            m[q] = pk_max_i16(h[0], h[1]);
+            const auto r = __builtin_amdgcn_permlane16_swap(m[q], m[q], false, false);
+            m[q] = pk_max_i16(r[0], r[1]);
+            // rotations of a row of 16 lanes
+            m[q] = pk_max_i16(m[q], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m[q], 0x128, 0xf, 0xf, false));
+            if (UPP == 1) {
+                m[q] = pk_max_i16(m[q], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m[q], 0x124, 0xf, 0xf, false));
+                m[q] = pk_max_i16(m[q], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m[q], 0x122, 0xf, 0xf, false));
+                m[q] = pk_max_i16(m[q], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m[q], 0x121, 0xf, 0xf, false));
+            }
+        }
+        if (WAVES > 1) {
+            if (share == 0) {
+                part[wave][2 * sub] = (int)m[0];
+                part[wave][2 * sub + 1] = (int)m[1];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < WAVES; ++i) {
+                m[0] = pk_max_i16(m[0], (uint32_t)part[i][2 * sub]);
+                m[1] = pk_max_i16(m[1], (uint32_t)part[i][2 * sub + 1]);
+            }
+        }
+        most.odd = m[0];
+        most.even = m[1];
+        if ((WAVES == 1 || wave == 0) && share == 0) reinterpret_cast<uint32_t*>(out)[sub] = most.get();
+        return;
+    }
+    const auto h0 = __builtin_amdgcn_permlane32_swap((uint32_t)sum[0], (uint32_t)sum[2], false, false);
+    const auto h1 = __builtin_amdgcn_permlane32_swap((uint32_t)sum[1], (uint32_t)sum[3], false, false);
+    const auto r = __builtin_amdgcn_permlane16_swap(h0[0] + h0[1], h1[0] + h1[1], false, false);
+    int s = (int)(r[0] + r[1]);
+    s += __builtin_amdgcn_update_dpp(0, s, 0x128, 0xf, 0xf, false);
+    if (UPP == 1) {
+        s += __builtin_amdgcn_update_dpp(0, s, 0x124, 0xf, 0xf, false);
+        s += __builtin_amdgcn_update_dpp(0, s, 0x122, 0xf, 0xf, false);
+        s += __builtin_amdgcn_update_dpp(0, s, 0x121, 0xf, 0xf, false);
+    }
+    const uint32_t channel = sub * 4 + (lane >> 5) * 2 + (lane >> 4 & 1);
+    const bool first = (lane & 15) < UPP;  // one of the lanes that hold a channel
+    if (WAVES > 1) {
+        if (first) part[wave][channel] = s;
+        __syncthreads();
+        s = 0;
+#pragma unroll
+        for (int i = 0; i < WAVES; ++i) s += part[i][channel];
+    }
+    if (!first || (WAVES > 1 && wave != 0)) return;
+    float count = (float)taps;
+    if (MODE == POOL_AVG_EXCL) {
+        const int h_lo = ih0 < 0 ? 0 : ih0, h_hi = ih0 + a.fh > a.IH ? a.IH : ih0 + a.fh;
+        const int w_lo = iw0 < 0 ? 0 : iw0, w_hi = iw0 + a.fw > a.IW ? a.IW : iw0 + a.fw;
+        count = (float)((h_hi > h_lo ? h_hi - h_lo : 0) * (w_hi > w_lo ? w_hi - w_lo : 0));
+    }
+    out[channel] = (int8_t)(int)roundf((float)s / count);
+}
+
+template <int PACK, int WAVES>
+int launch_wave(hipStream_t st, const PoolArgs& a, int mode, FastDiv dfw) {
+    const uint32_t pixels = a.units / (PACK == 32 ? 2 : 1);
+    const dim3 grid(WAVES == 1 ? (pixels + 3) / 4 : pixels), block(WAVES == 1 ? 256 : WAVES * 64);
+    switch (mode) {
+        case POOL_MAX: return launch_kernel((pooling_wave_kernel<PACK, POOL_MAX, WAVES>), grid, block, 0, st, a, dfw);
+        case POOL_AVG: return launch_kernel((pooling_wave_kernel<PACK, POOL_AVG, WAVES>), grid, block, 0, st, a, dfw);
+        default: return launch_kernel((pooling_wave_kernel<PACK, POOL_AVG_EXCL, WAVES>), grid, block, 0, st, a, dfw);
+    }
+}
+
 template <int PACK, int VB, int FH, int FW>
 int launch_static(hipStream_t st, const PoolArgs& a, int mode, unsigned blocks) {
     switch (mode) {
@@ -363,6 +483,23 @@ generic:
         const uint32_t threads = a.units * POOL_LANES;
         const dim3 grid((threads + 255) / 256);
         const FastDiv dfw = make_fastdiv((uint32_t)a.fw);
+        if constexpr (PACK > 1) {
+            const uint32_t taps = (uint32_t)(a.fh * a.fw), pixels = a.units / (PACK == 32 ? 2 : 1);
+            if ((uint64_t)a.IH * (uint64_t)a.IW * PACK < (1ull << 31)) {  // (32-bit offsets in a plane)
+                // NCHW32: always.  One wave where it has a window's taps in flight at once, or where the windows alone fill the chip and
+                // are not long (2048 windows of 81 taps 3.8 us with one wave, 4.1 with four; of 400 9.1 and 8.1)
+                if (PACK == 32) {
+                    if (taps <= 64 || (pixels > 1024 && taps <= 256)) return launch_wave<PACK, 1>(st, a, mode, dfw);
+                    return taps <= 512 ? launch_wave<PACK, 4>(st, a, mode, dfw) : launch_wave<PACK, 16>(st, a, mode, dfw);
+                }
+                // NCHW4: where sixteen lanes to a window leave the chip idle (512 windows of 81 taps 2.6 us, 2.9 with sixteen lanes; 2048
+                // of 784 4.0 and 6.8; but 8192 of 576 10.4 and 6.8, 8192 of 196 5.4 and 4.4)
+                if (pixels <= 1024 ? taps > 64 : pixels <= 4096 && taps > 512) {
+                    if (taps <= 512) return launch_wave<PACK, 1>(st, a, mode, dfw);
+                    return taps <= 4096 ? launch_wave<PACK, 4>(st, a, mode, dfw) : launch_wave<PACK, 16>(st, a, mode, dfw);
+                }
+            }
+        }
         switch (mode) {
             case POOL_MAX: return launch_kernel(pooling_split_kernel<PACK, VB, POOL_MAX>, grid, dim3(256), 0, st, a, dfw);
             case POOL_AVG: return launch_kernel(pooling_split_kernel<PACK, VB, POOL_AVG>, grid, dim3(256), 0, st, a, dfw);

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from megengine_amd import _abi, ops
+from megengine_amd import synth as util
 from megengine_amd.lib import Mi355Error
 from tests.gpu_util import say
 
@@ -124,3 +125,27 @@ def test_errors():
     d = _abi.make_pooling_desc("MAX", "NCHW32", 1, 32, 4, 4, 2)
     with pytest.raises(Mi355Error, match="alignment"):
         ops.pooling_exec(d, buf[4:4 + 512].view(1, 1, 4, 4, 32))
+
+
+@pytest.mark.parametrize("window,pad,size", [((8, 8), 0, (8, 8)), ((5, 13), (2, 6), (7, 13)), ((16, 32), 0, (16, 33)),
+                                             ((19, 27), (9, 3), (19, 25)), ((64, 64), 0, (64, 64)), ((17, 241), (0, 1), (18, 241))])
+@pytest.mark.parametrize("fmt,c", [("NCHW4", 12), ("NCHW32", 96)])
+@pytest.mark.parametrize("mode", ["MAX", "AVERAGE", "AVERAGE_COUNT_EXCLUDE_PADDING"])
+def test_windows_shared_by_waves(oracle, mode, fmt, c, window, pad, size):
+    """64, 65, 512, 513, 4096 and 4097 taps: both sides of every number of waves to a window, with windows that leave the image."""
+    d = _abi.make_pooling_desc(mode, fmt, 3, c, size[0], size[1], window, 1, pad)
+    shape = _abi.packed_shape(d.format, 3, c, *size)
+    for x in (util.uniform_int(window[1], shape, -128, 127, np.int8), np.full(shape, -128, np.int8), np.full(shape, 127, np.int8)):
+        got = ops.pooling_exec(d, torch.from_numpy(x).cuda())
+        torch.cuda.synchronize()
+        assert np.array_equal(got.cpu().numpy(), oracle.pooling(d, x))
+
+
+@pytest.mark.parametrize("window,size", [((9, 9), 9), ((16, 16), 16), ((17, 17), 17)])
+def test_many_windows_shared_by_waves(oracle, window, size):
+    """More than 1024 windows of an NCHW32 tensor: up to 256 taps a wave to a window, four above."""
+    d = _abi.make_pooling_desc("AVERAGE", "NCHW32", 33, 1024, size, size, window, 1, 0)
+    x = util.uniform_int(size, _abi.packed_shape(d.format, 33, 1024, size, size), -128, 127, np.int8)
+    got = ops.pooling_exec(d, torch.from_numpy(x).cuda())
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), oracle.pooling(d, x))
