@@ -149,3 +149,21 @@ def test_many_windows_shared_by_waves(oracle, window, size):
     got = ops.pooling_exec(d, torch.from_numpy(x).cuda())
     torch.cuda.synchronize()
     assert np.array_equal(got.cpu().numpy(), oracle.pooling(d, x))
+
+
+@pytest.mark.parametrize("n,c,h,w,pad_h", [(1, 4, 1, 4, 1), (3, 12, 2, 8, 1), (2, 8, 7, 4, 2), (2, 20, 15, 36, 0), (3, 64, 56, 12, 1),
+                                           (2, 12, 5, 5, 1), (3, 4, 6, 6, 2), (2, 8, 3, 7, 1), (1, 8, 9, 9, 0), (2, 4, 4, 3, 1),
+                                           (2, 16, 31, 131, 1), (33, 64, 112, 112, 1), (9, 64, 97, 97, 1)])
+@pytest.mark.parametrize("fmt", ["NCHW4", "NCHW44"])
+def test_max_of_three_at_stride_two_by_pairs(oracle, fmt, n, c, h, w, pad_h):
+    """Every remainder of the width over the vector of four columns, one below it, windows that leave the image on every side, ties,
+    and a tensor that is aligned to 4 bytes only."""
+    d = _abi.make_pooling_desc("MAX", fmt, n, c, h, w, 3, 2, (pad_h, 1))
+    shape = _abi.packed_shape(d.format, n, c, h, w)
+    for lo, hi in ((-128, 127), (-128, -126), (-1, 1)):
+        x = util.uniform_int(h * w - lo, shape, lo, hi, np.int8)
+        want = oracle.pooling(d, x)
+        assert np.array_equal(ops.pooling_exec(d, torch.from_numpy(x).cuda()).cpu().numpy(), want)
+    buf = torch.zeros(x.size + 4, dtype=torch.int8, device="cuda")
+    buf[4:] = torch.from_numpy(x).cuda().flatten()
+    assert np.array_equal(ops.pooling_exec(d, buf[4:].view(shape)).cpu().numpy(), want)
