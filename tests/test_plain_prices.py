@@ -1,5 +1,5 @@
 """The tile for a dense 32-packed layer whose filter is in the reference layout (no GPU).  The layers are every fifteenth of the 306 (of
-2640 timed) on which prices by launches, rounds and tiles alone, without the terms that pick_plain_cfg explains, chose a tile more
+2640 timed) on which prices by launches, rounds and tiles alone, without the terms that TilePrice explains, chose a tile more
 than 3 % behind thresholds on tile counts: 1.08 times the best of the six tiles below on average, up to 1.21."""
 import math
 
