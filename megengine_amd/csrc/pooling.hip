@@ -227,10 +227,9 @@ __global__ __launch_bounds__(256) void pooling_max3s2_kernel(PoolArgs a) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) m[q].feed((uint32_t)x[fh][q]);
             }
-            if (up) {
+            if (up) {  // (at most 3: the last pair begins inside the row)
                 if (up & 1) { m[0] = m[1]; m[1] = m[2]; m[2] = m[3]; }
                 if (up & 2) { m[0] = m[2]; m[1] = m[3]; m[2] = m[3]; }
-                if (up & 4) { m[0] = m[3]; m[1] = m[3]; m[2] = m[3]; }
             }
             first.join(m[0]);
             first.join(m[1]);
