@@ -10,9 +10,11 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
+// These two take the number of workgroups from gridDim: as an argument, as the conversions below have it, the chain of int32 convolution,
+// requantisation, gate, activation, add, pool and dequantisation (256 x 28 x 28, batch 32) was 37.8 us instead of 36.75.
 __global__ __launch_bounds__(256) void requant_kernel(const int32_t* __restrict__ src, const int8_t* __restrict__ z,
-                                                      int8_t* __restrict__ dst, uint64_t quads, uint64_t count, EpiParams e, uint32_t grid) {
-    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads, grid);
+                                                      int8_t* __restrict__ dst, uint64_t quads, uint64_t count, EpiParams e) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads, gridDim.x);
     for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4i a = reinterpret_cast<const v4i*>(src)[i];
         const uint32_t zw = e.has_z ? reinterpret_cast<const uint32_t*>(z)[i] : 0u;
@@ -27,8 +29,8 @@ __global__ __launch_bounds__(256) void requant_kernel(const int32_t* __restrict_
 
 // QuantizedS8 first operand: 16 elements per thread step (16 + 16 bytes in, 16 out; 2-3 bytes per element)
 __global__ __launch_bounds__(256) void requant8_kernel(const int8_t* __restrict__ src, const int8_t* __restrict__ z,
-                                                       int8_t* __restrict__ dst, uint64_t blocks16, uint64_t count, EpiParams e, uint32_t grid) {
-    const XcdRun<uint64_t> run = xcd_run<uint64_t>(blocks16, grid);
+                                                       int8_t* __restrict__ dst, uint64_t blocks16, uint64_t count, EpiParams e) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t>(blocks16, gridDim.x);
     for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4i a = reinterpret_cast<const v4i*>(src)[i];
         v4i zv = {0, 0, 0, 0};
@@ -119,7 +121,7 @@ int launch_requant8(hipStream_t st, const EpiParams& e, const int8_t* src, const
     if (blocks > cap) blocks = cap;
     if (blocks == 0) blocks = 1;
     blocks = xcd_grid(blocks);
-    return launch_kernel(requant8_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, blocks16, count, e, (uint32_t)blocks);
+    return launch_kernel(requant8_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, blocks16, count, e);
 }
 
 int launch_requant(hipStream_t st, const EpiParams& e, const int32_t* src, const int8_t* z, int8_t* dst, uint64_t count,
@@ -132,7 +134,7 @@ int launch_requant(hipStream_t st, const EpiParams& e, const int32_t* src, const
     if (blocks > cap) blocks = cap;
     if (blocks == 0) blocks = 1;
     blocks = xcd_grid(blocks);
-    return launch_kernel(requant_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, quads, count, e, (uint32_t)blocks);
+    return launch_kernel(requant_kernel, dim3((unsigned)blocks), dim3(256), 0, st, src, z, dst, quads, count, e);
 }
 
 // ---- streaming probe: what a launch that only moves bytes costs on this device ----------------------------------
