@@ -164,8 +164,8 @@ struct KsAcc<16> {
 
 // TURN: long rows of a filter in the reference layout.  Loaded as operands, where neighbouring lanes hold different rows, 16 bytes per
 // lane take the address path 64 clocks instead of the 16 of a contiguous kilobyte, and that path is what the kernel is then bound by.
-// Here an instruction loads 128 bytes of each of eight rows, and LDS that only this wave uses turns them into operands (no barrier: a
-// wave's own LDS operations are in order).  A stage costs its LDS round trip, so short pieces do not take it: see ks_turns.
+// Here an instruction loads 128 bytes of each of eight rows, and LDS that only this wave uses turns them into operands (no barrier, but
+// see lds_between_lanes).  A stage costs its LDS round trip, so short pieces do not take it: see ks_turns.
 template <int PIN, int S, int MT, int W, bool PW, bool TURN, class Form>
 __device__ __forceinline__ void ks_run(const Form& form) {
     constexpr int ROWS = S / 4;           // channel quads of a block
@@ -374,12 +374,14 @@ __device__ __forceinline__ void ks_run(const Form& form) {
         auto stage = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < LOADS; ++j) mine[at_w[j]] = xf[buf][j];
+            lds_between_lanes();
             load_f(buf);
             v4i fa[STEPS][MT];
 #pragma unroll
             for (int b = 0; b < STEPS; ++b)
 #pragma unroll
                 for (int i = 0; i < MT; ++i) fa[b][i] = mine[at_r[i] + ((b * (8 / STEPS) + lk) ^ turn)];
+            lds_between_lanes();  // (the next stage, and the sums behind the last, overwrite what is read here)
 #pragma unroll
             for (int b = 0; b < STEPS; ++b)
 #pragma unroll

@@ -295,7 +295,7 @@ __device__ __forceinline__ void pw4q_run(const Form& form) {
 #pragma unroll
     for (int i = 0; i < MT * 32; i += 64)
         if (i + lane < MT * 32) bias_w[i + lane] = bias_v[i / 64];
-    __builtin_amdgcn_wave_barrier();
+    lds_between_lanes();
     wait_loads();
     const int tail = a.OHW & 3;
     auto blocks = [&](auto nl) __attribute__((always_inline)) {

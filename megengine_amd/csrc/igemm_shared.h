@@ -8,6 +8,15 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// Between LDS accesses by which lanes of one wave hand data to each other, on LDS that no other wave uses.  The hardware keeps a wave's
+// LDS operations in order; for the compiler the store of one lane and the load of another are addresses that differ, and it may swap
+// them wherever it can tell.  No instruction comes of this.
+__device__ __forceinline__ void lds_between_lanes() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 constexpr int IG_THREADS = 256;
 constexpr int IG_MAX_ENTRIES = 4096;  // k-unit table capacity (entries of 8 bytes: 32 KiB of LDS when full)
 
