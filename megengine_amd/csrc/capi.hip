@@ -1251,7 +1251,7 @@ int mi355_relayout_exec(void* stream, const mi355_relayout_desc* d, const void* 
     if (!src || !dst) return fail(MI355_ERR_BAD_ARG, "null tensor pointer");
     // the byte-transposing kernels use 16-byte vectors; misaligned tensors take the generic kernel
     const bool fast = aligned16(src) && aligned16(dst);
-    int rc = launch_relayout(reinterpret_cast<hipStream_t>(stream), *d, oshape, ondim, src, dst, fast);
+    int rc = launch_relayout(reinterpret_cast<hipStream_t>(stream), *d, oshape, ondim, src, dst, fast, cu_count());
     if (rc) return fail(MI355_ERR_LAUNCH, "relayout: %s", hipGetErrorString((hipError_t)rc));
     return MI355_OK;
 }

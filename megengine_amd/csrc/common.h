@@ -113,7 +113,7 @@ int launch_pooling(hipStream_t st, const mi355_pooling_desc& d, int pack, uint32
                    int8_t* dst, int cu_count);
 
 int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t* oshape, uint32_t ondim,
-                    const void* src, void* dst, bool allow_fast);
+                    const void* src, void* dst, bool allow_fast, int cu_count);
 
 static inline uint32_t conv_out_size(uint32_t i, uint32_t f, uint32_t dil, uint32_t s, uint32_t p) {
     uint32_t df = (f - 1) * dil + 1;

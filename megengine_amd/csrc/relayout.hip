@@ -114,10 +114,10 @@ __global__ __launch_bounds__(256) void relayout_generic_kernel(RelayoutArgs a) {
 // (the memory pipe takes them at full rate as long as a wave's run is contiguous).  The last 16 pixels of a plane start
 // at HW - 16, so they overlap the run before them and both write the same bytes: no tail code, every lane does the same.
 //
-// NCHW -> NCHW4 (C any: missing channels are zero), HW >= 4.  A step is 4 pixels of 4 channels: a wave loads 256 consecutive bytes of
+// NCHW -> NCHW4 (C any: missing channels are zero), HW >= 4 (the dispatch sends planes from 16 pixels on).  A step is 4 pixels of 4 channels: a wave loads 256 consecutive bytes of
 // each channel and stores one contiguous kilobyte.  (With 16 pixels to a thread the loads are four times as wide, but a store covers a
 // quarter of 64 lines, and small images leave the chip idle.)  A thread takes STEPS of them, 64 steps apart, whose loads are in flight
-// together.  The last step of a plane ends with it: its first pixels are written twice, with the same bytes.
+// together (see four_steps).  The last step of a plane ends with it: its first pixels are written twice, with the same bytes.
 // grid.x covers CB * ceil(HW / 4) steps per image, grid.y = N.  3 x 224 x 224 (the image of a first layer), against
 // 16 pixels to a thread: batch 1 2.55 -> 2.29 us, 16 3.36 -> 2.70, 64 7.50 -> 4.48; 256 x 64 x 64, batch 32: 16.6 -> 11.2 (6 TB/s).
 template <int STEPS>
@@ -152,40 +152,65 @@ __global__ __launch_bounds__(256) void nchw_to_nchw4_kernel(const int8_t* __rest
     }
 }
 
-// NCHW4 -> NCHW (the first C channels), HW >= 4: the same steps the other way round.  Against 16 pixels to a thread: 64 x 56 x 56, batch 64
-// 5.13 -> 4.48 us, batch 1 2.37 -> 2.31, the largest the same (256 x 64 x 64, batch 32: 10.8 and 10.9).
-template <int STEPS>
-__global__ __launch_bounds__(256) void nchw4_to_nchw_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
-                                                            uint32_t C, uint32_t HW, uint32_t steps, FastDiv pq) {
-    const uint32_t first = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * STEPS) + (threadIdx.x & 63);
-    const uint32_t CB = (C + 3) / 4;
-    const int8_t* image = src + (int64_t)blockIdx.y * CB * HW * 4;
-    int8_t* out = dst + (int64_t)blockIdx.y * C * HW;
-    u32x4 v[STEPS];
-    uint32_t group[STEPS], pixel[STEPS];
-#pragma unroll
-    for (int i = 0; i < STEPS; ++i) {
-        const uint32_t it = first + i * 64 < steps ? first + i * 64 : steps - 1;
-        const uint32_t cg = fdiv(it, pq), pb = it - cg * pq.d;
-        group[i] = cg;
-        pixel[i] = pb * 4 + 4 <= HW ? pb * 4 : HW - 4;
-        v[i] = load16u(image + ((int64_t)cg * HW + pixel[i]) * 4);  // 4 pixels x 4 channels
-    }
-#pragma unroll
-    for (int i = 0; i < STEPS; ++i) {
-        if (first + i * 64 >= steps) return;
-        uint32_t o[4];
-        transpose4x4(v[i][0], v[i][1], v[i][2], v[i][3], o[0], o[1], o[2], o[3]);
-        int8_t* d = out + (int64_t)group[i] * 4 * HW + pixel[i];
-        const uint32_t have = C - group[i] * 4;
-#pragma unroll
-        for (uint32_t k = 0; k < 4; ++k)
-            if (k < have) store4u(d + (int64_t)k * HW, o[k]);
-    }
+// 4 steps to a thread: from four workgroups for every CU to thirty-two, where few lanes of an image's last workgroup lack a step.  Against one
+// step, by the share of lanes that have one: two workgroups to an image and more 0.94 .. 0.98 of the time from 0.88 on, 1.05 to 1.4 below;
+// one workgroup 0.84 .. 0.94 from 0.69 on, 1.0 to 2.2 below (2873 images of 364 steps 1.3); beyond thirty-two 1.02 and more.
+static bool four_steps(uint64_t steps, uint32_t N, int cu) {
+    const uint64_t all = steps * N, few = 4096ull * cu, lanes = (steps + 1023) / 1024 * 1024;
+    return all >= few && all < 8 * few && (steps <= 1024 ? steps >= 704 : steps * 8 >= lanes * 7);
 }
 
-// 4 steps to a thread where that leaves four workgroups and more for every CU; below, a launch is its latency and threads are what it lacks
-static bool four_steps(uint64_t steps, uint32_t N) { return steps * N >= 4ull * 256 * 4 * 256; }
+// NCHW4 -> NCHW (the first C channels), HW >= 4: the same steps the other way round, one to a thread (four are 1.0 to 1.25 times as long).
+__global__ __launch_bounds__(256) void nchw4_to_nchw_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
+                                                            uint32_t C, uint32_t HW, uint32_t steps, FastDiv pq) {
+    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
+    if (it >= steps) return;
+    const uint32_t cg = fdiv(it, pq), pb = it - cg * pq.d;
+    const uint32_t px = pb * 4 + 4 <= HW ? pb * 4 : HW - 4;
+    const uint32_t CB = (C + 3) / 4;
+    const u32x4 v = load16u(src + (((int64_t)blockIdx.y * CB + cg) * HW + px) * 4);  // 4 pixels x 4 channels
+    uint32_t o[4];
+    transpose4x4(v[0], v[1], v[2], v[3], o[0], o[1], o[2], o[3]);
+    int8_t* d = dst + ((int64_t)blockIdx.y * C + cg * 4) * HW + px;
+    const uint32_t have = C - cg * 4;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        if (k < have) store4u(d + (int64_t)k * HW, o[k]);
+}
+
+// The same with 16 pixels to a thread, HW >= 16: a quarter of the workgroups, whose dispatch is what many small images cost.
+__global__ __launch_bounds__(256) void nchw4_to_nchw16_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
+                                                              uint32_t C, uint32_t HW, uint32_t items, FastDiv pq) {
+    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
+    if (it >= items) return;
+    const uint32_t cg = fdiv(it, pq), pb = it - cg * pq.d;
+    const uint32_t px = pb * 16 + 16 <= HW ? pb * 16 : HW - 16;
+    const uint32_t CB = (C + 3) / 4;
+    const int8_t* s = src + (((int64_t)blockIdx.y * CB + cg) * HW + px) * 4;
+    u32x4 o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const u32x4 v = load16u(s + j * 16);  // 4 pixels x 4 channels
+        uint32_t c0, c1, c2, c3;
+        transpose4x4(v[0], v[1], v[2], v[3], c0, c1, c2, c3);
+        o[0][j] = c0; o[1][j] = c1; o[2][j] = c2; o[3][j] = c3;
+    }
+    int8_t* d = dst + ((int64_t)blockIdx.y * C + cg * 4) * HW + px;
+    const uint32_t have = C - cg * 4;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        if (k < have) store16u(d + (int64_t)k * HW, o[k]);
+}
+
+// Which of the two.  16 pixels: where an image is one workgroup of those and more of the others, if there are two for every CU (4 pixels take
+// 1.02 to 1.2 times as long, 770 images of 280 steps 1.3); where it is three workgroups and more, from four of the others for every CU on
+// (1.0 to 1.07); where it is two, if those are nearly full and there are sixteen (1.02 to 1.07).  Elsewhere 4 pixels: of two workgroups the
+// second half empty 0.76 to 0.96, small tensors 0.95 to 1.0.
+static bool sixteen_pixels(uint64_t steps, uint64_t items, uint32_t N, int cu) {
+    const uint64_t all = steps * N;
+    if (items <= 256) return steps > 256 && all >= 512ull * cu;
+    return items <= 512 ? items >= 448 && all >= 4096ull * cu : all >= 1024ull * cu;
+}
 
 // NCHW4 <-> NCHW32: dwords change places.  Two threads per pixel of a 32-channel block, each moves 16 channels: on the
 // NCHW32 side a wave covers one contiguous kilobyte, on the other side two runs of 128 bytes per access.
@@ -303,8 +328,9 @@ __global__ __launch_bounds__(256) void nchw32_to_nchw_kernel(const int8_t* __res
 }  // namespace
 
 int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t* oshape, uint32_t ondim,
-                    const void* src, void* dst, bool allow_fast) {
+                    const void* src, void* dst, bool allow_fast, int cu_count) {
     int64_t total = 1;
+    if (cu_count <= 0) cu_count = 256;
     for (uint32_t i = 0; i < ondim; ++i) total *= oshape[i];
     if (total == 0) return 0;
     const bool requant = d.elem_bytes == 1 && d.scale_src != d.scale_dst;
@@ -328,7 +354,7 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
                 const uint32_t pq = (HW + 3) / 4;
                 if (oshape[4] == 4 && HW >= 16 && numbered((uint64_t)CB * pq + 1024)) {
                     const uint32_t steps = CB * pq;
-                    if (four_steps(steps, N))
+                    if (four_steps(steps, N, cu_count))
                         return launch_kernel(nchw_to_nchw4_kernel<4>, dim3((steps + 1023) / 1024, N), dim3(256), 0, st, s8, d8, C, HW,
                                              steps, make_fastdiv(pq));
                     return launch_kernel(nchw_to_nchw4_kernel<1>, dim3((steps + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, steps,
@@ -343,12 +369,13 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
                                      reinterpret_cast<uint32_t*>(dst), g);
             }
             case MI355_RL_NCHW4_NCHW:
-                if (HW >= 16 && numbered((uint64_t)d.shape[1] * ((HW + 3) / 4) + 1024)) {
+                if (HW >= 16 && numbered((uint64_t)d.shape[1] * ((HW + 3) / 4) + 256)) {
                     const uint32_t C = oshape[1], pq = (HW + 3) / 4, steps = d.shape[1] * pq;
-                    if (four_steps(steps, N))
-                        return launch_kernel(nchw4_to_nchw_kernel<4>, dim3((steps + 1023) / 1024, N), dim3(256), 0, st, s8, d8, C, HW,
-                                             steps, make_fastdiv(pq));
-                    return launch_kernel(nchw4_to_nchw_kernel<1>, dim3((steps + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, steps,
+                    const uint32_t p16 = (HW + 15) / 16, items = d.shape[1] * p16;
+                    if (sixteen_pixels(steps, items, N, cu_count))
+                        return launch_kernel(nchw4_to_nchw16_kernel, dim3((items + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, items,
+                                             make_fastdiv(p16));
+                    return launch_kernel(nchw4_to_nchw_kernel, dim3((steps + 255) / 256, N), dim3(256), 0, st, s8, d8, C, HW, steps,
                                          make_fastdiv(pq));
                 }
                 break;

@@ -27,7 +27,6 @@ typedef uint32_t u32u __attribute__((aligned(1)));
 
 __device__ __forceinline__ u32x4 load16u(const int8_t* p) { return *reinterpret_cast<const u32x4u*>(p); }
 __device__ __forceinline__ void store16u(int8_t* p, u32x4 v) { *reinterpret_cast<u32x4u*>(p) = v; }
-typedef uint32_t u32u __attribute__((aligned(1)));
 __device__ __forceinline__ uint32_t load4u(const int8_t* p) { return *reinterpret_cast<const u32u*>(p); }
 __device__ __forceinline__ void store4u(int8_t* p, uint32_t v) { *reinterpret_cast<u32u*>(p) = v; }
 

@@ -2,6 +2,7 @@
 // One exec per line of the input: the descriptor's bytes in hexadecimal, an algorithm (a number: by that name; -1: the heuristic's
 // choice, named; -2: none, exec chooses for itself), its tile (-1: the query's), and whether there is a workspace.  One line of the
 // output for each: the number of launches, dynamic LDS and threads of the last one, and the kernels, separated by tabs.
+// A descriptor of a layout conversion or of a pooling, told apart by its size, is executed as such.
 #include <cxxabi.h>
 #include <hip/hip_runtime.h>
 #include <stdio.h>
@@ -56,27 +57,39 @@ int main() {
     snprintf(format, sizeof(format), "%%%zus %%d %%d %%d", sizeof(hex) - 1);
     int algo, tile, room;
     while (scanf(format, hex, &algo, &tile, &room) == 4) {
-        mi355_conv_desc d;
-        unsigned char* bytes = reinterpret_cast<unsigned char*>(&d);
+        unsigned char bytes[sizeof(mi355_conv_desc)];
+        const size_t size = strlen(hex) / 2;
         unsigned b;
-        if (strlen(hex) != 2 * sizeof(d)) {
-            printf("a descriptor of %zu characters\n", strlen(hex));
-            return 1;
-        }
-        for (size_t i = 0; i < sizeof(d); ++i) {
+        for (size_t i = 0; i < size; ++i) {
             if (sscanf(hex + 2 * i, "%2x", &b) != 1) return 1;
             bytes[i] = (unsigned char)b;
         }
-        mi355_algo a;
-        size_t ws = 0;
         int8_t* const t = reinterpret_cast<int8_t*>(0x1000000);  // device addresses that nothing on the host reads
         g_launches = 0;
         g_names.clear();
-        int st = mi355_convbias_s8_query(&d, algo < 0 ? MI355_ALGO_HEURISTIC : algo, &a, &ws);
-        if (tile >= 0) a.tile_cfg = tile;
-        if (!st)
-            st = mi355_convbias_s8_exec(nullptr, &d, algo == -2 ? nullptr : &a, t, t, reinterpret_cast<int32_t*>(t), d.has_z ? t : nullptr, t,
-                                        room ? t : nullptr, room ? ws : 0);
+        int st;
+        if (size == sizeof(mi355_conv_desc)) {
+            mi355_conv_desc d;
+            memcpy(&d, bytes, size);
+            mi355_algo a;
+            size_t ws = 0;
+            st = mi355_convbias_s8_query(&d, algo < 0 ? MI355_ALGO_HEURISTIC : algo, &a, &ws);
+            if (tile >= 0) a.tile_cfg = tile;
+            if (!st)
+                st = mi355_convbias_s8_exec(nullptr, &d, algo == -2 ? nullptr : &a, t, t, reinterpret_cast<int32_t*>(t), d.has_z ? t : nullptr,
+                                            t, room ? t : nullptr, room ? ws : 0);
+        } else if (size == sizeof(mi355_relayout_desc)) {
+            mi355_relayout_desc d;
+            memcpy(&d, bytes, size);
+            st = mi355_relayout_exec(nullptr, &d, t, t);
+        } else if (size == sizeof(mi355_pooling_desc)) {
+            mi355_pooling_desc d;
+            memcpy(&d, bytes, size);
+            st = mi355_pooling_s8_exec(nullptr, &d, t, t);
+        } else {
+            printf("a descriptor of %zu bytes\n", size);
+            return 1;
+        }
         if (st) {
             printf("status %d: %s\n", st, mi355_last_error());
             return 1;
