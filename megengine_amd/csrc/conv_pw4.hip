@@ -840,7 +840,8 @@ int launch_split(hipStream_t st, const IgemmArgs& a) {
     const QuadArgs<FastDiv> k = quad_args(a);
     const int lds = W > 1 ? W * MT * 4096 : 0;
     Pw4kWire wire;
-    if (wire.pack(k) && grid < QUOT_MAX) return launch_kernel((void (*)(Pw4kWire))pw4k_kernel<MT, W>, dim3((unsigned)grid), dim3(W * 64), lds, st, wire);
+    // (Up to eight workgroups per CU.  Graph replays, wire / wide: to 2047 workgroups 0.99 to 1.005, from 2048 on 1.01 to 1.04.)
+    if (grid < 2048 && wire.pack(k)) return launch_kernel((void (*)(Pw4kWire))pw4k_kernel<MT, W>, dim3((unsigned)grid), dim3(W * 64), lds, st, wire);
     return launch_kernel((void (*)(Pw4kWide))pw4k_kernel<MT, W>, dim3((unsigned)grid), dim3(W * 64), lds, st, Pw4kWide{k, make_fastdiv(tiles_m)});
 }
 

@@ -65,12 +65,11 @@ def test_which_form():
         if kernel.startswith("patch4"):
             continue
         forms = _forms(descs)
-        if not kernel.startswith("grp32_kernel<2"):  # (more workgroups than its line)
-            assert forms[0].endswith("Wire"), (kernel, forms)
-            wires.append(kernel)
+        assert forms[0].endswith("Wire"), (kernel, forms)
+        wires.append(kernel)
         assert all(f.endswith("Wide") for f in forms[1:]), (kernel, forms)
         wides.append(kernel)
-    assert len(wires) >= 12 and len(wides) >= 14
+    assert len(wires) == len(wides) == len(CASES) - 1
 
 
 def test_numbers_that_do_not_fit():
@@ -78,6 +77,9 @@ def test_numbers_that_do_not_fit():
         return _abi.make_conv_desc("NCHW4", n, c, h, w, c, 3, group=c, pad=1, **S)
 
     assert _forms([dw(1, 4, 1, 65535), dw(1, 4, 1, 65536), dw(1, 4, 65535, 1), dw(1, 4, 65536, 1)]) == ["Dw3Wire", "Dw3Wide"] * 2
+    # (such sides of the other families are the generic kernel's, so that gaps between images are what they meet: above)
+    wide = [_desc("NCHW32", 1, 64, 1, 65535, 64, 1), _desc("NCHW4", 1, 12, 3, 65535, 12, 3, group=3), _desc("NCHW32", 1, 64, 3, 65535, 64, 3, group=2)]
+    assert all(r.kernels == ("conv_direct_kernel",) for r in routes.routes(wide))
     # work items (four columns of four rows here) that the wire's divisions are exact for: fewer than 2^21
     assert _forms([dw(1, 4 * 127, 4 * 128, 4 * 128), dw(1, 4 * 128, 4 * 128, 4 * 128)]) == ["Dw3Wire", "Dw3Wide"]
 
@@ -92,3 +94,33 @@ def test_both_forms(i):
         for has_z in (True, False):
             if gap != "z" or has_z:
                 check_case(oracle, _desc(fmt, *shape, has_z=has_z, gap=gap, **kw), seed=i + 5, tag="%s gap %s" % (kernel, gap))
+
+
+# The sizes where opening the wire in every workgroup begins to cost more than the launch gains: kernel, format, the layer on the wire's
+# side of the line and the one beyond, options
+SIZE_LINES = [
+    ("grp4_kernel<1, 3, 1>", "NCHW4", (28, 36, 7, 9, 36, 3), (29, 36, 7, 9, 36, 3), dict(group=9)),                   # 252, 261 workgroups
+    ("grp4_kernel<2, 3, 2>", "NCHW4", (42, 24, 56, 56, 24, 3), (43, 24, 56, 56, 24, 3), dict(group=3, stride=2)),     # 252, 258
+    ("ks_kernel<32, 32, 1, 4, false>", "NCHW32", (1, 96, 64, 128, 32, 3), (1, 96, 65, 128, 32, 3), dict()),           # 256, 264
+    ("pw4k_kernel<4, 1>", "NCHW4", (145, 72, 29, 31, 36, 1), (146, 72, 29, 31, 36, 1), dict()),                       # 2040, 2056
+    ("grp32_kernel<2, 1, 1>", "NCHW32", (20, 128, 29, 30, 192, 3), (21, 128, 29, 30, 192, 3), dict(group=2, stride=2)),   # 240, 288
+]
+
+
+def test_which_form_by_the_size_of_a_launch():
+    for kernel, fmt, small, large, kw in SIZE_LINES:
+        descs = [_desc(fmt, *small, **kw), _desc(fmt, *large, **kw)]
+        assert [r.kernels[-1] for r in routes.routes(descs)] == [kernel] * 2
+        small, large = _forms(descs)
+        assert small.endswith("Wire") and large.endswith("Wide"), (kernel, small, large)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("i", range(len(SIZE_LINES)))
+def test_both_sides_of_a_size(i):
+    from oracle import oracle
+    from tests.gpu_util import check_case
+    kernel, fmt, small, large, kw = SIZE_LINES[i]
+    for shape in (small, large):
+        for has_z in (True, False):
+            check_case(oracle, _desc(fmt, *shape, has_z=has_z, nonline="RELU", **kw), seed=i + 31, tag=kernel)
