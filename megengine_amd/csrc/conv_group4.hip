@@ -193,10 +193,10 @@ __global__ __launch_bounds__(256) void grp4_kernel(Grp4Wide a) {
 template <int OQ, int F, int ST>
 int launch_grp4_kernel(hipStream_t st, dim3 grid, const Grp4Args<FastDiv>& a, uint32_t groups) {
     Grp4Wire wire;
-    // Up to a workgroup per CU the launch is what a call costs; beyond, opening the wire in every workgroup is.  Graph replays, wire / wide by
-    // workgroups: to 255 1.01 .. 1.02 (0.05 us of kernels of 3, where the launch gains 0.6), 256 to 1023 1.02 .. 1.04, beyond 1.04 .. 1.06 (9
-    // groups of 4 at 57 x 61, batch 20, 1260 workgroups: 4.43 us wide, 4.70 so).
-    if ((uint64_t)grid.x * grid.y * grid.z <= 256 && wire.pack<F == 3 ? 2 : 1>(a, groups))
+    // Up to two workgroups per CU the launch is what a call costs; beyond, opening the wire in every workgroup is.  Graph replays, wire / wide by
+    // workgroups: to 255 1.01 .. 1.02 (0.05 us of kernels of 3, where a launch that is waited for gains 0.6), to 511 1.02 .. 1.04 (0.1 of 3.9),
+    // to 1023 1.02 .. 1.03 (of 5), beyond 1.04 .. 1.06 (9 groups of 4 at 57 x 61, batch 20, 1260 workgroups: 4.43 us wide, 4.70 so).
+    if ((uint64_t)grid.x * grid.y * grid.z <= 512 && wire.pack<F == 3 ? 2 : 1>(a, groups))
         return launch_kernel((void (*)(Grp4Wire))grp4_kernel<OQ, F, ST>, grid, dim3(256), 0, st, wire);
     return launch_kernel((void (*)(Grp4Wide))grp4_kernel<OQ, F, ST>, grid, dim3(256), 0, st, Grp4Wide{a});
 }

@@ -520,10 +520,11 @@ int launch_ks(hipStream_t st, const KsArgs<FastDiv>& k, uint32_t n, int lds, boo
     const int64_t grid = k.by_m ? (int64_t)((k.tiles_m + 7) / 8) * k.tiles_n * 8 : (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
     KsWire wire;
-    // 32 x 32 tiles up to a workgroup per CU: beyond, opening the wire costs more than the launch gains.  Graph replays, wire / wide, 32 x 32:
-    // to 256 workgroups 1.01 (0.04 us of 3 to 4, where the launch gains 0.6), to 512 1.015 .. 1.03, beyond 1.035 .. 1.045 (3x3 160 -> 32 at 90 x
-    // 15, batch 12, 512 workgroups: 5.16 us wide, 5.73 so).  The others at any number: 16 x 16 0.98 .. 1.0, 64 x 32 1.0 .. 1.01.
-    const bool fits = (S != 32 || MT != 1 || grid <= 256) && wire.pack<PIN, S, MT, W>(k, n);
+    // Windowed 32 x 32 tiles up to two workgroups per CU: beyond, opening the wire costs more than the launch gains.  Graph replays, wire /
+    // wide: to 256 workgroups 1.01 (0.04 us of 4, where a launch that is waited for gains 0.6), to 512 1.02, beyond 1.035 .. 1.04 (0.27 us of 6
+    // to 11; 3x3 160 -> 32 at 90 x 15, batch 12, 512 workgroups: 5.16 us wide, 5.73 so).  Pointwise ones take 3 to 4 us at any number, and one
+    // image of ResNet-50 0.8 % longer with them wide from 256 on.  The others: 16 x 16 0.98 .. 1.0, 64 x 32 1.0 .. 1.01.
+    const bool fits = (PW || S != 32 || MT != 1 || grid <= 512) && wire.pack<PIN, S, MT, W>(k, n);
     if constexpr (ks_can_turn(PIN, S, MT, W))
         if (turn) return fits ? launch_ks_form<PIN, S, MT, W, PW, true>(st, wire, (unsigned)grid, lds) : launch_ks_form<PIN, S, MT, W, PW, true>(st, KsWide{k}, (unsigned)grid, lds);
     return fits ? launch_ks_form<PIN, S, MT, W, PW, false>(st, wire, (unsigned)grid, lds) : launch_ks_form<PIN, S, MT, W, PW, false>(st, KsWide{k}, (unsigned)grid, lds);

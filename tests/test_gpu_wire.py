@@ -99,9 +99,9 @@ def test_both_forms(i):
 # The sizes where opening the wire in every workgroup begins to cost more than the launch gains: kernel, format, the layer on the wire's
 # side of the line and the one beyond, options
 SIZE_LINES = [
-    ("grp4_kernel<1, 3, 1>", "NCHW4", (28, 36, 7, 9, 36, 3), (29, 36, 7, 9, 36, 3), dict(group=9)),                   # 252, 261 workgroups
-    ("grp4_kernel<2, 3, 2>", "NCHW4", (42, 24, 56, 56, 24, 3), (43, 24, 56, 56, 24, 3), dict(group=3, stride=2)),     # 252, 258
-    ("ks_kernel<32, 32, 1, 4, false>", "NCHW32", (1, 96, 64, 128, 32, 3), (1, 96, 65, 128, 32, 3), dict()),           # 256, 264
+    ("grp4_kernel<1, 3, 1>", "NCHW4", (56, 36, 7, 9, 36, 3), (57, 36, 7, 9, 36, 3), dict(group=9)),                   # 504, 513 workgroups
+    ("grp4_kernel<2, 3, 2>", "NCHW4", (85, 24, 56, 56, 24, 3), (86, 24, 56, 56, 24, 3), dict(group=3, stride=2)),     # 510, 516
+    ("ks_kernel<32, 32, 1, 4, false>", "NCHW32", (1, 96, 128, 128, 32, 3), (1, 96, 129, 128, 32, 3), dict()),         # 512, 520
     ("pw4k_kernel<4, 1>", "NCHW4", (145, 72, 29, 31, 36, 1), (146, 72, 29, 31, 36, 1), dict()),                       # 2040, 2056
     ("grp32_kernel<2, 1, 1>", "NCHW32", (20, 128, 29, 30, 192, 3), (21, 128, 29, 30, 192, 3), dict(group=2, stride=2)),   # 240, 288
 ]
