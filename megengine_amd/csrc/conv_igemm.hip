@@ -600,8 +600,11 @@ static bool igemm_plain_s32(const ConvProblem& p) {
 }
 
 // Dense 32-packed layers.  What such a layer takes on a tile is a price per launch (a chain of copies as long as the reduction), one per
-// round of tiles over the device's CUs and one per tile and CU, each with a part that grows with the reduction.  Four terms separate
-// what those leave together:
+// round of tiles over the device's CUs and one per tile and CU, each with a part that grows with the reduction.  What separates what
+// those leave together:
+//   the tiles that split the reduction over waves are dealt out to eight XCDs by rows or columns of tiles, and are counted by the XCD that
+//     has the most (3x3 768 -> 448 at 13 x 14, batch 3, residual: 14 rows of 32 x 32 tiles, two for six of the XCDs, 10.6 us, where the seven
+//     rows of 64 x 32 take 7.6).  That changes 3 % of the choices, to 0.89 (plain) and 0.92 (pre-processed) of their time on average.
 //   line_k: filter rows of whole 128-byte lines.  The second-generation tiles read a plain filter 32 bytes of every row at a time, all
 //     of them at the same place of a line then: 10 to 20 % longer than one channel block more or less (3x3 over 384 channels, stride 2,
 //     165 tiles of 64 x 64: 13.8 us; over 416, 168 of them: 12.2).  The first-generation tiles read whole rows and hardly have it.
@@ -612,8 +615,13 @@ static bool igemm_plain_s32(const ConvProblem& p) {
 // to twenty more, on drawn layers of 32 to 2048 channels, 1x1 to 5x5, stride 1 and 2, batch 1 to 64: 9414 with the filter in the reference
 // layout, 5930 with it pre-processed, of which the layers of ResNet-50 for drawn batches and image sizes are half.  Two halves of them
 // predict each other as well as themselves.  Thresholds on tile counts, fitted to powers of two, were behind the best tile by 6.0 % (plain)
-// and 5.1 % (pre-processed) on average, the prices by 2.1 and 1.7; 3 and 6 % of the layers are more than 3 % slower with them, 0.8 and
-// 0.6 % more than 10 %, at most 1.27.  Into at most 32 channels, plain, which the 32 x 256 tile had whatever their number of pixels:
+// and 5.1 % (pre-processed) on average, the prices by 2.1 and 1.7.  On 26000 other layers, by graph replays again, they are 3.4 % behind,
+// ahead of the thresholds by 3.8 and 3.5 %, and of the layers 4.0 and 7.7 % are more than 3 % slower than by thresholds, 0.9 and 1.9 % more than
+// 10 %, at most 1.28.  Most of the latter are pointwise layers over 500 and more channels without a residual, where the second-generation
+// tiles of 64 x 128 and 128 x 128 with a pre-processed filter are 1.05 to 1.17 times as fast as the choice -- by themselves, their operands warm.
+// With prices for those tiles too 0.3 % were more than 10 % slower, but ResNet-50 took 0.5 to 2 % longer at each of eleven batches and sizes
+// between 1 x 224 and 64 x 224: inside a network, whose weights come from memory, the first-generation tiles are ahead.  Into at most 32 channels,
+// plain, which the 32 x 256 tile had whatever their number of pixels:
 // 1.22 times the best, now 1.01 (3x3 480 -> 32 at 8 x 29, batch 44: 35.0 -> 12.3 us).
 // The tiles that split the reduction over waves are priced where operand traffic does not bound them: up to `split_most` 64 x 32 tiles.
 struct TilePrice {
@@ -624,11 +632,13 @@ static int cheapest_tile(const TilePrice* prices, int count, const IgemmArgs& a,
     const float k = a.kbytes / 1024.0f;
     const bool lines = a.kbytes % 128 == 0, window = a.T > 1, strided = a.sh * a.sw > 1;
     const uint32_t cu = cu_count > 0 ? cu_count : 256;
+    const int first_ks = igemm_first_ks_cfg();
     float best = 0;
     int cfg = -1;
     for (int i = 0; i < count; ++i) {
         const TilePrice& c = prices[i];
-        const uint32_t tiles = (uint32_t)((a.OC + (1 << c.bm) - 1) >> c.bm) * (uint32_t)(((int64_t)a.M + (1 << c.bn) - 1) >> c.bn);  // (OC * M < 2^31)
+        const uint32_t tm = (uint32_t)((a.OC + (1 << c.bm) - 1) >> c.bm), tn = (uint32_t)(((int64_t)a.M + (1 << c.bn) - 1) >> c.bn);
+        const uint32_t tiles = c.cfg >= first_ks ? (uint32_t)igemm5_workgroups(tm, tn) : tm * tn;  // (OC * M < 2^31)
         const uint32_t full = (tiles + cu - 1) / cu;
         const float rounds = (float)full, pairs = (float)((full + 1) / 2), share = (float)tiles / (float)cu;
         const float tile = c.tile + k * (c.tile_k + (strided ? c.strided_k : 0) + (lines ? c.line_k : 0)) + (a.epi.has_z ? c.z : 0);
@@ -780,27 +790,28 @@ static int pick_cfg_by_shape(const ConvProblem& p, int cu_count, bool will_prepr
         const int s = igemm_pw32s_cfg();
         const int64_t outputs = (int64_t)d.n * p.oh * p.ow * d.oc;
         const bool table = igemm_takes_table(p);
-        if (!table && d.ic == 64 && d.oc > 32 && outputs < 5000000) return kNumCfgs + 10;  // dma64x64x64r4
+        if (!table && d.ic == 64 && outputs < 5000000) return kNumCfgs + 10;  // dma64x64x64r4
         if ((table || d.ic <= 64 || (d.ic <= 96 && outputs >= 2000000)) && igemm_resolve_cfg(p, s) == s) return s;
     }
     if (p.pin == 32 && d.group == 1 && !igemm_needs_general(p)) {
         IgemmArgs a;
         igemm_fill_args(p, a);
         if (will_preprocess && p.pout == 32 && !d.has_z && d.oc > 64 && d.stride_h == 1 && d.stride_w == 1) {
-            // Three places where the prices of a pre-processed filter cannot tell what timing every tile does
+            // Three kinds of layers for which timing networks, whose weights are cold, says something else than the prices, which were fitted
+            // to layers by themselves, their operands warm (ResNet-50 at batch 64, which has all three, alternating with and without each)
             const int v2 = igemm_first_v2_cfg(), cu = cu_count > 0 ? cu_count : 256;
             enum { V64x128x128r3 = 3, V64x64x128r4 = 8, V3_128x128x256r3 = 6 };
             const int64_t t128 = (int64_t)((d.oc + 127) / 128) * (((int64_t)a.M + 127) / 128);
             const bool pw = a.T == 1 && a.ph == 0 && a.pw == 0, one_round = 2 * t128 >= cu && t128 < cu;
             // 3x3 over 256 channels with one 128 x 128 tile for most CUs: the patch-staged tile, whose stage of eight k-chunks
-            // halves both the bytes through the CU's copy path and the stage boundaries (41 layers: 1.005 times the best tile,
-            // by price 1.03; falls back when the patch does not fit)
+            // halves both the bytes through the CU's copy path and the stage boundaries (722 us with it, 730 by price; falls back when the
+            // patch does not fit)
             if (d.fh == 3 && d.fw == 3 && a.kbytes >= 2304 && a.kbytes < 4608 && one_round) return igemm_first_v3_cfg() + V3_128x128x256r3;
-            // pointwise over 1024 to 2047 channels, the same number of tiles: more pixels than channels per tile (inside a network,
-            // where weights are cold; by itself, warm, it is 1.07 times the 8-wave 128 x 128 tile)
+            // pointwise over 1024 to 2047 channels, the same number of tiles: more pixels than channels per tile (723 us, 725 by price; by
+            // itself, warm, 1.07 times the 8-wave 128 x 128 tile)
             if (pw && a.kbytes >= 1024 && a.kbytes < 2048 && one_round) return v2 + V64x128x128r3;
             // windows over 4608 bytes and more with few tiles, but too many to split the reduction: the smallest tile with the deepest
-            // ring (3x3 over 512 channels, 200 to 490 of them: 0.97 .. 1.0 times the 64 x 128 tile of eight waves)
+            // ring (722 us, 726 by price)
             if (a.T > 1 && a.kbytes >= 4608 && split_tiles(a) > 400 && 2 * t128 < cu) return v2 + V64x64x128r4;
         }
         return pick_by_price(a, will_preprocess, false, cu_count);

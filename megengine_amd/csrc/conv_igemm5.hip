@@ -517,7 +517,7 @@ int launch_ks_form(hipStream_t st, const Form& form, unsigned grid, int lds) {
 
 template <int PIN, int S, int MT, int W, bool PW>
 int launch_ks(hipStream_t st, const KsArgs<FastDiv>& k, uint32_t n, int lds, bool turn) {
-    const int64_t grid = k.by_m ? (int64_t)((k.tiles_m + 7) / 8) * k.tiles_n * 8 : (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
+    const int64_t grid = igemm5_workgroups(k.tiles_m, k.tiles_n);
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
     KsWire wire;
     // Windowed 32 x 32 tiles up to two workgroups per CU: beyond, opening the wire costs more than the launch gains.  Graph replays, wire /

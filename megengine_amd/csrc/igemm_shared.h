@@ -548,6 +548,9 @@ int launch_grp4(hipStream_t st, const ConvProblem& p, const int8_t* src, const i
 int igemm5_num_cfgs();
 const char* igemm5_cfg_name(int cfg);
 bool igemm5_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
+// Workgroups of a launch of tm x tn tiles: eight XCDs (workgroup b runs on XCD b % 8) take rows of tiles each, or where those are few,
+// columns, and all are as many as those of the XCD that has the most.
+static inline int64_t igemm5_workgroups(int64_t tm, int64_t tn) { return 8 * (tm >= 8 ? (tm + 7) / 8 * tn : (tn + 7) / 8 * tm); }
 int igemm5_pick(const IgemmArgs& a, int pin, int pout);  // the 4-packed tile for few output pixels, -1 where there are too many
 int launch_igemm5(hipStream_t st, const IgemmArgs& a, int pin, int pout, int cfg);
 

@@ -99,3 +99,25 @@ def test_against_the_generic_kernel():
             used.add(lib.tile_names()[a.tile_cfg])
             assert torch.equal(out, want), (it, list(d.key()), lib.tile_names()[a.tile_cfg])
     assert len(used) >= 8, used
+
+
+# n, ic, h, w, oc, f, stride, residual, pre-processed; us (graph replays on 256 CUs) on the tile that the busiest XCD has least of, and on
+# the one that fewer tiles in all spoke for
+BUSIEST_XCD = [
+    (3, 416, 10, 22, 576, 3, 1, 0, 0, "v2_ks_32x32w4", 9.2, "v2_ks_64x32w8", 16.7),
+    (5, 512, 25, 9, 160, 3, 2, 1, 0, "v2_ks_16x16w4", 6.2, "v2_ks_16x16w8", 8.9),
+    (10, 448, 12, 17, 576, 3, 2, 0, 0, "v2_ks_32x32w8", 11.9, "v2_ks_64x32w8", 16.6),
+    (2, 256, 10, 78, 160, 5, 1, 0, 0, "v2_ks_64x32w8", 11.5, "v2_ks_32x32w8", 15.2),
+    (4, 864, 11, 18, 160, 5, 1, 1, 1, "v2_ks_32x32w8", 15.8, "v2_ks_16x16w8", 24.3),
+    (9, 288, 13, 22, 288, 5, 2, 0, 1, "v2_ks_64x32w8", 9.5, "v2_ks_32x32w8", 13.2),
+    (4, 352, 16, 10, 288, 3, 1, 0, 1, "v2_ks_64x32w8", 5.2, "v2_ks_32x32w4", 6.7),
+    (3, 416, 42, 20, 608, 5, 2, 0, 1, "v2_ks_32x32w4", 17.5, "v2_ks_64x32w8", 22.0),
+]
+
+
+def test_tiles_are_counted_by_the_busiest_xcd():
+    names = lib.tile_names()
+    for n, ic, h, w, oc, f, s, z, pre, best, us, other, other_us in BUSIEST_XCD:
+        d = _abi.make_conv_desc("NCHW32", n, ic, h, w, oc, f, pad=f // 2, stride=s, nonline="RELU", has_z=bool(z), **S)
+        a, _ = ops.conv_bias_query(d, _abi.ALGO_HEURISTIC_PREPROCESS if pre else _abi.ALGO_HEURISTIC)
+        assert us < 0.8 * other_us and names[a.tile_cfg] == best, (n, ic, oc, names[a.tile_cfg])
