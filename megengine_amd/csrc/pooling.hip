@@ -330,7 +330,9 @@ __global__ __launch_bounds__(256) void pooling_kernel(PoolArgs a) {
 // at batch 64).  Sixteen lanes share a window, lane k takes taps k, k + 16, ..., and a butterfly adds the partial sums up:
 // in each of its first steps a lane hands half of its channels to its partner and keeps the other half, so 16 channels
 // cost 15 exchanges and every lane ends with one channel, whose byte it writes.
-// 7 x 7 x 2048 in NCHW4: 2.6 us at batch 1, 5.0 us at batch 64.
+// 7 x 7 x 2048 in NCHW4: 2.6 us at batch 1, 5.0 us at batch 64.  The next kernel has taken over where it is ahead; what is left here are
+// windows of an NCHW4 tensor that are short or many (launch_mode has the lines), and planes of 2 GiB and more in either layout, whose
+// offsets that kernel does not hold.
 constexpr int POOL_LANES = 16;
 template <int PACK, int VB, int MODE>
 __global__ __launch_bounds__(256) void pooling_split_kernel(PoolArgs a, FastDiv div_fw) {

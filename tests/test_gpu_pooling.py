@@ -167,3 +167,23 @@ def test_max_of_three_at_stride_two_by_pairs(oracle, fmt, n, c, h, w, pad_h):
     buf = torch.zeros(x.size + 4, dtype=torch.int8, device="cuda")
     buf[4:] = torch.from_numpy(x).cuda().flatten()
     assert np.array_equal(ops.pooling_exec(d, buf[4:].view(shape)).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("fmt,c,h,w", [("NCHW32", 32, 8192, 8200), ("NCHW4", 4, 23200, 23200)])
+def test_large_windows_of_planes_beyond_two_gib(fmt, c, h, w):
+    """Byte offsets inside a plane that 32 bits do not hold: windows at its beginning, across the 2^31st byte and at its end.  (Sums and maxima
+    of bytes are exact, so torch's own are the reference.)"""
+    pack, stride = 32 if fmt == "NCHW32" else 4, (h - 20) // 4
+    d = _abi.make_pooling_desc("MAX", fmt, 1, c, h, w, (20, 24), (stride, w - 24), 0)
+    x = torch.randint(-128, 120, (1, 1, h, w, pack), dtype=torch.int8, device="cuda")
+    assert x.numel() > 2 ** 31
+    rows = range(0, h - 19, stride)
+    windows = torch.stack([x[0, 0, r:r + 20, q:q + 24].reshape(480, pack) for r in rows for q in (0, w - 24)]).int()
+    for mode in ("MAX", "AVERAGE"):
+        d.mode = _abi.POOL_NAMES[mode]
+        got = ops.pooling_exec(d, x).view(-1, pack).int()
+        total = windows.sum(1)
+        want = windows.amax(1) if mode == "MAX" else total.sign() * ((total.abs() + 240) // 480)  # (ties away from zero)
+        assert got.shape == want.shape and torch.equal(got, want), mode
+    del x
+    torch.cuda.empty_cache()
