@@ -10,8 +10,11 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-// These two take the number of workgroups from gridDim: as an argument, as the conversions below have it, the chain of int32 convolution,
-// requantisation, gate, activation, add, pool and dequantisation (256 x 28 x 28, batch 32) was 37.8 us instead of 36.75.
+// These two take the number of workgroups from gridDim and not, as the conversions below, as an argument.  That costs a single short call
+// 0.1 us (4096 values: 3.43 us as an argument, 3.58 so) and gains where the device is behind: the chain of int32 convolution, requantisation,
+// gate, activation, add, pool and dequantisation over 256 x 28 x 28 takes 36.7 us instead of 37.7 at batch 32, 68.2 instead of 68.9 at 64;
+// chains of short calls (24 to 29 us) differ by less than their runs.  Traced, the kernels themselves take the same time either way, so what
+// the chain gains lies between its launches; why is not known.
 __global__ __launch_bounds__(256) void requant_kernel(const int32_t* __restrict__ src, const int8_t* __restrict__ z,
                                                       int8_t* __restrict__ dst, uint64_t quads, uint64_t count, EpiParams e) {
     const XcdRun<uint64_t> run = xcd_run<uint64_t>(quads, gridDim.x);
