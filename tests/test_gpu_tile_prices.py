@@ -51,7 +51,7 @@ def test_near_the_best():
         assert a.id == 1 and lib.tile_usable(d, a.tile_cfg)
         if names[a.tile_cfg] not in near.split():
             miss.append((n, ic, h, w, oc, f, s, z, pre, names[a.tile_cfg], near))
-    # over all layers timed the pick is 2 % behind the best on average, more than 6 % on one in ten
+    # over 26000 other layers the pick is 3.4 % behind the best on average, more than 10 % on 13 in a hundred
     assert len(miss) <= len(LAYERS) // 6, miss
 
 
