@@ -251,7 +251,7 @@ def main():
                higher_is_better=True, scaling="weak", vs_baseline=None, dtype="s8",
                data="synthetic",
                config=dict(arithmetic="s8 x s8 products accumulated in s32 (exact), requantised to s8 through f32 as the reference does",
-                           workload="BASELINE configs[2]: ResNet-50 v1.5 int8 conv stack, batch 64, 224x224, "
+                           workload="ResNet-50 v1.5 int8 conv stack, batch 64, 224x224, "
                                     "NCHW4 stem + NCHW32, fused residual z + RELU, random per-tensor scales",
                            batch=batch, layers=nl, launch=launch_mode, graph=graph_note,
                            **(dict(forced_tiles=forced) if forced else {}),
