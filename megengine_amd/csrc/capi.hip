@@ -798,7 +798,7 @@ static int exec_impl(void* stream, const mi355_conv_desc* d, const mi355_algo* a
             const bool planar = by_heuristic && d->format == MI355_FMT_NCHW && p.icpg * d->fh * d->fw >= 5 &&
                                 (reinterpret_cast<uintptr_t>(bias) & 3) == 0;
             const int tile = planar ? patch1_pick(p, false, cu_count()) : -1;
-            rc = tile >= 0 ? launch_patch1(hs, p, tile, src, filter, bias, z, reinterpret_cast<int8_t*>(dst))
+            rc = tile >= 0 ? launch_patch1(hs, p, tile, cu_count(), src, filter, bias, z, reinterpret_cast<int8_t*>(dst))
                            : launch_conv_direct(hs, p, src, filter, bias, z, dst);
             break;
         }

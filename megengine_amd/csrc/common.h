@@ -91,7 +91,7 @@ size_t nchw_mfma_workspace_used(const ConvProblem& p);
 bool patch1_usable(const ConvProblem& p);
 // (packed: the caller could run the packed path instead)
 int patch1_pick(const ConvProblem& p, bool packed, int cu_count);
-int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, int cu_count, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                   int8_t* dst);
 int launch_conv_nchw_mfma(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt,
                           const int32_t* bias, const int8_t* z, int8_t* dst, void* workspace);

@@ -137,7 +137,7 @@ int launch_conv_nchw_mfma(hipStream_t st, const ConvProblem& p, int cu_count, co
     const mi355_conv_desc& d = p.d;
     if ((uint64_t)d.n * d.oc * p.oh * p.ow == 0) return 0;
     const int tile = patch1_pick(p, true, cu_count);  // no packing where the kernel that reads the planes is ahead
-    if (tile >= 0) return launch_patch1(st, p, tile, src, flt, bias, z, dst);
+    if (tile >= 0) return launch_patch1(st, p, tile, cu_count, src, flt, bias, z, dst);
     int8_t* ws = reinterpret_cast<int8_t*>(workspace);
     const uint32_t HW = d.ih * d.iw;
     PrepArgs a;

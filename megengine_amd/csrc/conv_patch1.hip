@@ -12,11 +12,13 @@
 //     eight lanes meet eight different bank groups.
 //   * The filter's rows are [channel][tap] bytes: a thread takes four channels of a row, 4 T contiguous bytes, and T times three
 //     v_perm with constant selectors make the T dwords (four channels of one tap) that an operand is made of.
+//   * A tile is rows and columns, or a run of pixels in the order of memory (p1_run says where), whose rows end wherever they do.
 //   * Two stages in LDS, the next one's loads in registers while the current one is multiplied, one barrier per stage.
 //   * Bound by LDS, as the 4-packed patch tiles are, and by the latency of a stage where tiles are few.
 // Filters of 1x1, 3x3 and 5x5; others go through the
-// workspace.  Graph replays: 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual: 16.6 us packed, 12.2 here (four waves of
+// workspace.  Graph replays: 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual: 16.6 us packed, 11.3 here (four waves of
 // 1200 vector instructions for 23 products each, a third of their time waiting for a stage's loads); more at patch1_pick.
+#include <algorithm>
 #include <atomic>
 
 #include "igemm_shared.h"
@@ -41,8 +43,9 @@ struct P1Args {
     int IC, IH, IW, IHW, OC, OH, OW, OHW, N, sh, sw, ph, pw;
     int src_sn, dst_sn, z_sn, kbytes, flt_bytes, has_bias, nstages;
     uint32_t src_bytes, dst_bytes, z_bytes;
-    int NI, TH, TW, PWC, PXI, PX, PXQ;  // images, rows, columns of a tile; patch columns (a multiple of 4), pixels per image, pixels, quads
+    int NI, TH, TW, tile_px, PWC, PXI, PX, PXQ;  // images, rows, columns of a tile; its pixels of an image; patch columns (a multiple of 4), pixels per image, pixels, quads
     int tiles_m, tiles_n, tiles_img, tiles_w;
+    int run;  // not zero: a tile is that many pixels in the order of memory (TW = OW), zero: TH rows of TW columns
     FastDiv div_tiles_m, div_tiles_img, div_tiles_w, div_tw, div_tile_px, div_pqi, div_pqw;
     EpiParams epi;
 };
@@ -58,26 +61,31 @@ __device__ __forceinline__ uint32_t p1_tap(const uint32_t (&x)[T], int tap) {
     return lo | hi;
 }
 
+// where a tile begins: image, row and column out; skip: columns of the first row that are the tile's before
+struct P1Tile {
+    int n0, oh0, ow0, skip;
+};
+
 // where four neighbouring lanes put (and find the residual of) their four columns: offset of channel ch = 4 lh + l32 % 4 of the
-// first eight channels, and the columns from there to the row's end (0: nothing)
+// first eight channels, and the columns from there to the end of the row, or of the image for a run (0: nothing)
 struct P1Out {
     int d0, z0, cols;
 };
-__device__ __forceinline__ P1Out p1_out(const P1Args& a, int p, int n0, int oh0, int ow0, int ch) {
-    const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)(a.TH * a.TW), oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
-    const bool in = ((int)im < a.NI) & (n0 + (int)im < a.N) & (oh0 + (int)oh < a.OH);
-    const int px = (oh0 + (int)oh) * a.OW + ow0 + (int)ow + ch * a.OHW;
-    return {(n0 + (int)im) * a.dst_sn + px, (n0 + (int)im) * a.z_sn + px, in ? a.OW - (ow0 + (int)ow) : 0};
+__device__ __forceinline__ P1Out p1_out(const P1Args& a, const P1Tile& o, int p, int ch) {
+    const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)a.tile_px + o.skip, oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
+    const bool in = ((int)im < a.NI) & (o.n0 + (int)im < a.N) & (o.oh0 + (int)oh < a.OH);
+    const int at = (o.oh0 + (int)oh) * a.OW + o.ow0 + (int)ow, px = at + ch * a.OHW;
+    return {(o.n0 + (int)im) * a.dst_sn + px, (o.n0 + (int)im) * a.z_sn + px, in ? a.run ? a.OHW - at : a.OW - (o.ow0 + (int)ow) : 0};
 }
 
 template <int MT, int NT, int NL, bool HZ>
-__device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT], const uint32_t (&zq)[NT][MT][4], int n0, int oh0, int ow0, int oc0,
+__device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT], const uint32_t (&zq)[NT][MT][4], const P1Tile& o, int oc0,
                                             int wave, int l32, int lh) {
     const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes), rs_z = make_rsrc(a.z, HZ ? a.z_bytes : 0);
     const int lane4 = l32 & 3, ch = 4 * lh + lane4;  // after the exchange a lane holds four columns of channel ch of every eight
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const P1Out w = p1_out(a, (wave * NT + j) * 32 + (l32 & ~3), n0, oh0, ow0, ch);
+        const P1Out w = p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), ch);
         const int d0 = w.d0, z0 = w.z0, cols = w.cols;
         const bool part = (cols > 0) & (cols < 4), split = __builtin_amdgcn_ballot_w64(part) != 0;
 #pragma unroll
@@ -97,12 +105,12 @@ __device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT]
                     zw = quad_transpose(zw, lane4);
                 }
                 const v16i& c = acc[i][j];
-                const uint32_t o = quad_transpose(requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], zw, a.epi), lane4);
-                __builtin_amdgcn_raw_buffer_store_b32((int)o, rs_dst, (ok & (cols >= 4)) ? d0 : SENT, at, 0);
+                const uint32_t y = quad_transpose(requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], zw, a.epi), lane4);
+                __builtin_amdgcn_raw_buffer_store_b32((int)y, rs_dst, (ok & (cols >= 4)) ? d0 : SENT, at, 0);
                 if (split) {
 #pragma unroll
                     for (int k = 0; k < 3; ++k)
-                        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(o >> (8 * k)), rs_dst, (ok & part & (k < cols)) ? d0 + k : SENT, at, 0);
+                        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(y >> (8 * k)), rs_dst, (ok & part & (k < cols)) ? d0 + k : SENT, at, 0);
                 }
             }
     }
@@ -122,7 +130,7 @@ __global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
     // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
     asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.IC), "s"(a.IH), "s"(a.IW), "s"(a.IHW), "s"(a.OC), "s"(a.N),
                  "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.src_sn), "s"(a.kbytes), "s"(a.flt_bytes), "s"(a.has_bias), "s"(a.nstages),
-                 "s"(a.NI), "s"(a.TH), "s"(a.TW), "s"(a.PWC), "s"(a.PX), "s"(a.PXQ), "s"(a.tiles_m));
+                 "s"(a.NI), "s"(a.TH), "s"(a.TW), "s"(a.tile_px), "s"(a.run), "s"(a.PWC), "s"(a.PX), "s"(a.PXQ), "s"(a.tiles_m));
     asm volatile("" ::"s"(a.tiles_n), "s"(a.tiles_img), "s"(a.tiles_w), "s"(a.div_tiles_m.m), "s"(a.div_tiles_img.m), "s"(a.div_tiles_w.m),
                  "s"(a.div_pqi.m), "s"(a.div_pqi.s2), "s"(a.div_pqw.m), "s"(a.div_pqw.s2), "s"(a.div_tile_px.m), "s"(a.div_tw.m), "s"(a.epi.s_b),
                  "s"(a.epi.lin_lo));
@@ -139,8 +147,10 @@ __global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
         if (r >= per || tn >= a.tiles_n) return;
     }
     const int ig = (int)fdiv(tn, a.div_tiles_img), ti = tn - ig * a.tiles_img;
-    const int th = (int)fdiv(ti, a.div_tiles_w), tw = ti - th * a.tiles_w;
-    const int n0 = ig * a.NI, oh0 = th * a.TH, ow0 = tw * a.TW, oc0 = tm * BM;
+    const bool is_run = a.run != 0;
+    const int at = is_run ? ti * a.run : ti, th = (int)fdiv(at, a.div_tiles_w), tw = at - th * a.tiles_w;  // (a run: row and column)
+    const int n0 = ig * a.NI, oc0 = tm * BM, oh0 = is_run ? th : th * a.TH, ow0 = is_run ? 0 : tw * a.TW;
+    const P1Tile o{n0, oh0, ow0, is_run ? tw : 0};
     const int iw_lo = (ow0 * a.sw - a.pw) & ~3;  // the patch starts at a column that is a multiple of four: a quad that starts
                                                  // inside a row starts at one of its columns
 
@@ -228,14 +238,14 @@ __global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
             if (p_lds[k] >= 0)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    v4i o;
+                    v4i turned;
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
                         const uint32_t lo = __builtin_amdgcn_perm(xp[k][4 * c + 1], xp[k][4 * c], p_sel[k][j]);
                         const uint32_t hi = __builtin_amdgcn_perm(xp[k][4 * c + 3], xp[k][4 * c + 2], p_sel[k][j]);
-                        o[c] = (int)(lo | hi << 16);
+                        turned[c] = (int)(lo | hi << 16);
                     }
-                    s[p_lds[k] + ((j + turn) & 3)] = o;
+                    s[p_lds[k] + ((j + turn) & 3)] = turned;
                 }
         }
     };
@@ -252,8 +262,8 @@ __global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         const uint32_t p = (wave * NT + j) * 32 + l32;
-        const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)(a.TH * a.TW), oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
-        b_px[j] = (int)im < a.NI ? (int)(im * a.PXI + oh * a.sh * a.PWC) + ((int)ow + ow0) * a.sw - a.pw - iw_lo : 0;
+        const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)a.tile_px + o.skip, oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
+        b_px[j] = (((int)im < a.NI) & ((int)oh < a.TH)) ? (int)(im * a.PXI + oh * a.sh * a.PWC) + ((int)ow + ow0) * a.sw - a.pw - iw_lo : 0;
     }
     int offs[STEPS];
 #pragma unroll
@@ -271,7 +281,7 @@ __global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
     if constexpr (ZPRE)
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const P1Out w = p1_out(a, (wave * NT + j) * 32 + (l32 & ~3), n0, oh0, ow0, 4 * lh + (l32 & 3));
+        const P1Out w = p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), 4 * lh + (l32 & 3));
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -328,7 +338,7 @@ __global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
         __syncthreads();
     }
 
-#define MI355_P1(NL, HZ) p1_epilogue<MT, NT, NL, HZ>(a, acc, zq, n0, oh0, ow0, oc0, wave, l32, lh)
+#define MI355_P1(NL, HZ) p1_epilogue<MT, NT, NL, HZ>(a, acc, zq, o, oc0, wave, l32, lh)
     if (a.epi.lin) {
         MI355_P1(NL_LIN, false);
     } else if (a.epi.has_z) {
@@ -390,6 +400,8 @@ bool p1_plan(const ConvProblem& p, int tile, P1Args* k, int* lds_bytes) {
                 k->NI = NI; k->TH = TH; k->TW = TW; k->PWC = PWC; k->PXI = PXI; k->PX = PXQ * 4; k->PXQ = PXQ;
                 k->tiles_w = cols;
                 k->tiles_img = cols * ((OH + TH - 1) / TH);
+                k->tile_px = TH * TW;
+                k->run = 0;
                 if (tiles > 0x3fffffff) return false;
                 k->tiles_n = (int)tiles;
             }
@@ -401,6 +413,44 @@ bool p1_plan(const ConvProblem& p, int tile, P1Args* k, int* lds_bytes) {
     const int E = GS * T, EP = (E + 1) & ~1;
     *lds_bytes = 2 * (EP * p1_bmp(mt) + GS * k->PX) * 16;
     return *lds_bytes <= 150 * 1024;
+}
+
+// The same tile as a run of pixels in the order of memory where that is ahead of the rows and columns of p1_plan.
+// Rows that end inside a group of four columns cost rows-and-columns tiles a group of single bytes in each row, six more memory
+// instructions for four outputs of every channel, and columns of the tile that hold nothing; a run has one such group at an image's end.
+// Its patch is all columns of the rows that it touches.  231 drawn layers with such rows, graph replays: 0.97 of the time since
+// this rule takes runs for some (3x3 121 -> 251 at 45 x 10, batch 54: 29.2 -> 18.6 us; 3x3 75 -> 150 at 61 x 45, batch 6, residual: 12.4 -> 11.3).
+// Not where a run's patch asks more of a thread or leaves fewer workgroups to a CU (3x3 at stride 2, 202 -> 106 at 60 x 91, batch 14: 24.5 ->
+// 37.4), nor, where every workgroup has a CU for itself, for a patch that takes longer to turn (5x5 5 -> 180 at 14 x 43, batch 2: 4.8 -> 6.4).
+void p1_run(const ConvProblem& p, int tile, int cu_count, P1Args* k, int* lds_bytes) {
+    const mi355_conv_desc& d = p.d;
+    const int T = (int)(d.fh * d.fw), F = (int)d.fw, GS = p1_gs(T), TPG = 256 / GS, bm = kP1Tiles[tile][0] * 32, bn = kP1Tiles[tile][1] * 128;
+    const int OH = (int)p.oh, OW = (int)p.ow, sh = (int)d.stride_h, sw = (int)d.stride_w;
+    if (OW % 4 == 0 || (int64_t)OH * OW > 0x3fffff00) return;
+    const int ohw4 = (OH * OW + 3) & ~3;
+    int NI = ohw4 < bn ? bn / ohw4 : 1, run = ohw4, runs = 1;
+    if (NI == 1) {
+        runs = (ohw4 + bn - 1) / bn;
+        run = ((ohw4 + runs - 1) / runs + 3) & ~3;
+        runs = (ohw4 + run - 1) / run;
+    }
+    const int64_t pwc = ((int64_t)(OW - 1) * sw + F + 3 + 3) & ~3;
+    if (pwc > 0xffff) return;
+    const int PWC = (int)pwc, TH = std::min((run + OW - 2) / OW + 1, OH);
+    const int64_t pxi = (int64_t)((TH - 1) * sh + F) * PWC, pxq = NI * pxi / 4;
+    const int threads_had = (k->PXQ + TPG - 1) / TPG;  // quads of a thread
+    if (pxq > (int64_t)threads_had * TPG) return;
+    const int64_t tiles = ((int64_t)d.n + NI - 1) / NI * runs;
+    const int lds = *lds_bytes + 2 * GS * ((int)pxq * 4 - k->PX) * 16;
+    if (tiles > k->tiles_n || lds > 150 * 1024 || std::min(3, 160 * 1024 / lds) < std::min(3, 160 * 1024 / *lds_bytes)) return;
+    if (tiles * pxq * 5 > (int64_t)k->tiles_n * k->PXQ * 8) return;
+    if (tiles * ((d.oc + bm - 1) / bm) <= cu_count && pxq * 10 > (int64_t)k->PXQ * 13) return;
+    k->NI = NI; k->TH = TH; k->TW = OW; k->PWC = PWC; k->PXI = (int)pxi; k->PX = (int)pxq * 4; k->PXQ = (int)pxq;
+    k->tiles_w = OW;  // (what a run's first pixel is divided by)
+    k->tiles_img = runs;
+    k->tile_px = k->run = run;
+    k->tiles_n = (int)tiles;
+    *lds_bytes = lds;
 }
 
 template <int MT, int NT, int T>
@@ -536,12 +586,13 @@ int patch1_pick(const ConvProblem& p, bool packed, int cu_count) {
     return p1_behind_packed(p, tile, wgs, k.nstages, cu_count) ? -1 : tile;
 }
 
-int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, int cu_count, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                   int8_t* dst) {
     const mi355_conv_desc& d = p.d;
     P1Args k;
     int lds;
     if (!p1_plan(p, tile, &k, &lds)) return (int)hipErrorInvalidConfiguration;
+    p1_run(p, tile, cu_count, &k, &lds);
     k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
     k.IC = d.ic; k.IH = d.ih; k.IW = d.iw; k.IHW = d.ih * d.iw;
     k.OC = d.oc; k.OH = p.oh; k.OW = p.ow; k.OHW = p.oh * p.ow; k.N = d.n;
@@ -554,7 +605,7 @@ int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, const int8_t* 
     k.flt_bytes = k.kbytes * d.oc;
     k.has_bias = d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL;
     k.div_tiles_m = make_fastdiv(k.tiles_m); k.div_tiles_img = make_fastdiv(k.tiles_img); k.div_tiles_w = make_fastdiv(k.tiles_w);
-    k.div_tw = make_fastdiv(k.TW); k.div_tile_px = make_fastdiv(k.TH * k.TW);
+    k.div_tw = make_fastdiv(k.TW); k.div_tile_px = make_fastdiv(k.tile_px);
     k.div_pqi = make_fastdiv(k.PXI >> 2); k.div_pqw = make_fastdiv(k.PWC >> 2);
     k.epi = p.epi;
     const int T = (int)(d.fh * d.fw);
