@@ -248,6 +248,21 @@ __global__ __launch_bounds__(256) void nchw_to_packed_small_kernel(const int8_t*
 constexpr int RL_TP = 512;           // pixels per tile
 constexpr int RL_ROW = RL_TP + 8;    // padded channel row (bytes): 16 rows = 8320 = 32*256 + 128
 
+// Where 16-byte unit u of a wave's 128 pixels (two units each) lies in LDS: lanes that write units 8 apart and lanes that read consecutive ones
+// meet different banks.
+__device__ __forceinline__ uint32_t rl_slot(uint32_t u) { return u ^ ((u >> 3 & 3) << 1); }
+
+// Whole lines: from two workgroups to a CU on, if their tiles are three quarters full, and half full from four on.  Bound by bytes there:
+// 256 x 64 x 64 at batch 128 46.0 -> 41.3 us (5.8 -> 6.5 TB/s), 64 x 112 x 112 at batch 64 19.7 -> 17.0; 220 drawn conversions 0.84 .. 0.97 of the
+// time on this side of the line, 1.03 .. 1.08 with fewer workgroups, where the second meeting in LDS is one more step of a chain, and 1.06 on
+// emptier tiles (512 x 14 x 14 at batch 128: 9.5 / 10.1).
+static bool whole_lines(uint64_t workgroups, uint64_t tiles_of_plane, uint32_t HW, int cu) {
+    const uint64_t room = tiles_of_plane * RL_TP;
+    return workgroups >= 4 * (uint64_t)cu ? 2ull * HW >= room : workgroups >= 2 * (uint64_t)cu && 4ull * HW >= 3 * room;
+}
+
+// LINES: stores of whole lines, see below
+template <bool LINES>
 __global__ __launch_bounds__(256) void nchw_to_nchw32_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
                                                              uint32_t C, uint32_t CB, uint32_t HW) {
     __shared__ __attribute__((aligned(16))) int8_t sm[32 * RL_ROW];
@@ -279,11 +294,29 @@ __global__ __launch_bounds__(256) void nchw_to_nchw32_kernel(const int8_t* __res
         transpose4x4(rows[4 * q], rows[4 * q + 1], rows[4 * q + 2], rows[4 * q + 3], c0, c1, c2, c3);
         out[0][q] = c0; out[1][q] = c1; out[2][q] = c2; out[3][q] = c3;
     }
-    const uint32_t px = p0 + pq * 4;
+    if constexpr (!LINES) {
+        const uint32_t px = p0 + pq * 4;
+        int8_t* d = dst + ((n * CB + cb) * HW + px) * 32 + half * 16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (px + i < HW) *reinterpret_cast<u32x4*>(d + i * 32) = out[i];
+        return;
+    }
+    // A wave's 128 pixels are four contiguous kilobytes of dst: turned once more in LDS, so that a store writes one of them and not 32 bytes of
+    // every 128 of all four.
+    __syncthreads();
+    u32x4* mine = reinterpret_cast<u32x4*>(sm) + (t >> 6) * 256;
+    const uint32_t lane = t & 63;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) mine[rl_slot((lane >> 1) * 8 + i * 2 + half)] = out[i];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t px = p0 + (t >> 6) * 128 + (lane >> 1);
     int8_t* d = dst + ((n * CB + cb) * HW + px) * 32 + half * 16;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (px + i < HW) *reinterpret_cast<u32x4*>(d + i * 32) = out[i];
+    for (uint32_t i = 0; i < 4; ++i)
+        if (px + i * 32 < HW) *reinterpret_cast<u32x4*>(d + i * 1024) = mine[rl_slot(i * 64 + lane)];
 }
 
 __global__ __launch_bounds__(256) void nchw32_to_nchw_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
@@ -361,8 +394,11 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
                                          make_fastdiv(pq));
                 }
                 // planes of a quarter of the LDS tile and more: below, most of a tile's threads would find no pixel
-                if (oshape[4] == 32 && HW >= RL_TP / 4 && numbered((uint64_t)CB * ptiles * 256))
-                    return launch_kernel(nchw_to_nchw32_kernel, dim3(CB * ptiles, N), dim3(256), 0, st, s8, d8, C, CB, HW);
+                if (oshape[4] == 32 && HW >= RL_TP / 4 && numbered((uint64_t)CB * ptiles * 256)) {
+                    if (whole_lines((uint64_t)N * CB * ptiles, ptiles, HW, cu_count))
+                        return launch_kernel(nchw_to_nchw32_kernel<true>, dim3(CB * ptiles, N), dim3(256), 0, st, s8, d8, C, CB, HW);
+                    return launch_kernel(nchw_to_nchw32_kernel<false>, dim3(CB * ptiles, N), dim3(256), 0, st, s8, d8, C, CB, HW);
+                }
                 if (!numbered((uint64_t)total / 4)) break;
                 const SmallPlanes g = make_small_planes(N, C, HW, oshape[4]);
                 return launch_kernel(nchw_to_packed_small_kernel, dim3((g.items + 255) / 256), dim3(256), 0, st, s8,
