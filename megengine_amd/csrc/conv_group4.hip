@@ -17,12 +17,14 @@
 // a lane of v_mfma_i32_16x16x64_i8 holds, so a step is four taps and 3x3 is three steps, zeros of the block diagonal
 // included a third of the time of the dot products.  A workgroup stages a band of input rows in LDS as [pixel][16
 // channels] (NCHW4 keeps them in four planes), so every operand is one conflict-free ds_read_b128; the filter stays in
-// twelve registers; the next band is in flight while this one is multiplied.
-// 32 groups of 4 at 56 x 56, batch 16 (13 MB): 165 us as 32 launches, 9.8 with dot products, 6.6 here; 32 groups of 16
-// (51 MB): 50 us with dot products, 17 here.  Small layers are a chain: with the filter staged beside the first band instead of
+// twelve registers.  A workgroup is one band, with no band in flight behind it: the sixteen registers of a second band's pixels cost a
+// fifth workgroup on the CU, which hides more (six fit now, three with them).
+// 32 groups of 4 at 56 x 56, batch 16 (13 MB): 165 us as 32 launches, 9.8 with dot products, 5.8 here; 32 groups of 16
+// (51 MB): 50 us with dot products, 17 here; 47 groups of 16 at 78 x 8, batch 60: 20.7 with bands in a row, 16.8 one to a workgroup.  Small layers are a chain: with the filter staged beside the first band instead of
 // gathered dword by dword ahead of it, and the next operands read while results are requantised, 55 groups of 16 at 8 x 47,
 // stride 2, batch 4 went from 6.2 to 4.2 us, 5 groups of 16 at 33 x 100, stride 2, batch 64 from 9.8 to 8.4.
 #include <tuple>
+#include <type_traits>
 
 #include "igemm_shared.h"
 #include "wire.h"
@@ -201,6 +203,7 @@ int launch_grp4_kernel(hipStream_t st, dim3 grid, const Grp4Args<FastDiv>& a, ui
     return launch_kernel((void (*)(Grp4Wide))grp4_kernel<OQ, F, ST>, grid, dim3(256), 0, st, Grp4Wide{a});
 }
 
+constexpr int64_t G16_BANDS = 1 << 24;  // bands of a batch (256 times as many threads in a grid's first dimension)
 constexpr int G16_PX = 1024;  // pixels of a staged band (16 KiB), four per thread
 
 template <class Div>
@@ -213,13 +216,13 @@ struct G16Args {
     int IH, IW, OH, OW, s, ph, pw;
     int TH, PW, bands, items;  // output rows of a band, padded input columns, bands per image, bands of the batch
     int log_icpg, src_scb, dst_scb, has_bias;
-    int slabs, step;  // blocks of 16 channels; workgroups per slab
+    int slabs;  // blocks of 16 channels
     int64_t src_sn, dst_sn, z_sn;
     Div div_pw, div_ow, div_bands;
     EpiParams epi;
 
     auto numbers() const {
-        return std::tie(IH, IW, OH, OW, s, ph, pw, TH, PW, bands, items, log_icpg, src_scb, dst_scb, has_bias, slabs, step, src_sn, dst_sn, z_sn);
+        return std::tie(IH, IW, OH, OW, s, ph, pw, TH, PW, bands, items, log_icpg, src_scb, dst_scb, has_bias, slabs, src_sn, dst_sn, z_sn);
     }
 };
 
@@ -241,7 +244,7 @@ struct G16Wire {
     const int8_t* z;
     int8_t* dst;
     // in, out: height | width << 16; window: stride, padding, log of a group's channels; bands: output rows of one | slabs << 16
-    uint32_t N, in, out, window, bands, per_image, step, flags;
+    uint32_t N, in, out, window, bands, per_image, flags;
     EpiWire epi;
 
     template <class Div>
@@ -249,14 +252,14 @@ struct G16Wire {
         k.IH = wire_lo(in); k.IW = wire_hi(in); k.OH = wire_lo(out); k.OW = wire_hi(out);
         k.s = wire_byte(window, 0); k.ph = wire_byte(window, 1); k.pw = wire_byte(window, 2); k.log_icpg = wire_byte(window, 3);
         k.TH = wire_lo(bands); k.slabs = wire_hi(bands); k.PW = (k.OW - 1) * k.s + 3;
-        k.bands = (int)per_image; k.items = wire_mul((int)N, k.bands); k.step = (int)step;
+        k.bands = (int)per_image; k.items = wire_mul((int)N, k.bands);
         k.src_scb = wire_mul(k.IH, k.IW, 4); k.dst_scb = wire_mul(k.OH, k.OW, 4);
         k.src_sn = (uint32_t)wire_mul(k.slabs, 4, k.src_scb); k.dst_sn = (uint32_t)wire_mul(k.slabs, 4, k.dst_scb);
         k.z_sn = (flags >> 3 & 1) ? k.dst_sn : 0;
         k.has_bias = (int)(flags >> 8 & 1);
     }
     __device__ __forceinline__ G16Args<Quot> open() const {
-        asm volatile("" ::"s"(src), "s"(flt), "s"(bias), "s"(z), "s"(dst), "s"(N), "s"(in), "s"(out), "s"(window), "s"(bands), "s"(per_image), "s"(step),
+        asm volatile("" ::"s"(src), "s"(flt), "s"(bias), "s"(z), "s"(dst), "s"(N), "s"(in), "s"(out), "s"(window), "s"(bands), "s"(per_image),
                      "s"(flags), "s"(epi.f[0]), "s"(epi.f[1]), "s"(epi.f[2]), "s"(epi.f[3]));  // one batch of scalar loads
         G16Args<Quot> k;
         k.src = src; k.flt = flt; k.bias = bias; k.z = z; k.dst = dst;
@@ -269,7 +272,7 @@ struct G16Wire {
     bool pack(const G16Args<FastDiv>& k, uint32_t n) {
         src = k.src; flt = k.flt; bias = k.bias; z = k.z; dst = k.dst;
         N = n; in = wire2(k.IH, k.IW); out = wire2(k.OH, k.OW); window = wire4(k.s, k.ph, k.pw, k.log_icpg);
-        bands = wire2(k.TH, k.slabs); per_image = (uint32_t)k.bands; step = (uint32_t)k.step;
+        bands = wire2(k.TH, k.slabs); per_image = (uint32_t)k.bands;
         flags = epi_wire(k.epi, false, &epi) | (k.has_bias ? 1u << 8 : 0);
         G16Args<FastDiv> o;
         numbers(o);
@@ -279,6 +282,66 @@ struct G16Wire {
 };
 static_assert(sizeof(G16Wire) <= WIRE_BYTES, "a wire");
 
+constexpr int G16_ANY = -1;  // the requantisation form is chosen where it is used
+
+struct G16Lane {
+    int ow[2], at[2];  // of the lane's two pixels of a band's first step: column out, byte of the staged band
+    int OW, step, wrap, cols, last;  // (uniform) columns out; 128 pixels on: bytes, bytes where the row ends, columns; the last pixel's byte
+    int tap[3];        // byte of the lane's tap of each matrix step, relative to the pixel
+    int out, p;        // byte of the first pixel in the planes of the slab; the pixel
+};
+
+// The pixels of one staged band, two units of 16 per wave and step; the operands and the residual of the next step are read while this
+// one is requantised.
+template <int NL, bool HZ>
+__device__ __forceinline__ void grp16_band(const EpiParams& epi, const G16Lane& l, const v4i* sm, const v4i (&fa)[3], v4i bv,
+                                           __amdgpu_buffer_rsrc_t rs_dst, __amdgpu_buffer_rsrc_t rs_z, int base, int pixels, int first) {
+    v4i fb[2][3];
+    uint32_t zn[2] = {0, 0};
+    int ow[2] = {l.ow[0], l.ow[1]}, at[2] = {l.at[0], l.at[1]};
+    const char* band = reinterpret_cast<const char*>(sm);
+    auto operands = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int here = at[k] < l.last ? at[k] : l.last;  // (past the band: any pixel of it)
+#pragma unroll
+            for (int st = 0; st < 3; ++st) fb[k][st] = *reinterpret_cast<const v4i*>(band + here + l.tap[st]);
+            ow[k] += l.cols;
+            at[k] += l.step;
+            const bool over = ow[k] >= l.OW;
+            ow[k] -= over ? l.OW : 0;
+            at[k] += over ? l.wrap : 0;
+        }
+    };
+    auto residual = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            zn[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, l.p + u + k * 16 < pixels ? l.out + k * 64 : SENT, base + u * 4, 0);
+    };
+    if (HZ) residual(0);
+    operands();
+    for (int u = 0; first + u < pixels; u += 128) {
+        uint32_t zw[2] = {zn[0], zn[1]};
+        v4i acc[2] = {bv, bv};
+#pragma unroll
+        for (int st = 0; st < 3; ++st)
+#pragma unroll
+            for (int k = 0; k < 2; ++k) acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[st], fb[k][st], acc[k], 0, 0, 0);
+        operands();
+        if (HZ) residual(u + 128);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (NL == G16_ANY) {
+            requant8(acc[0], acc[1], zw, epi);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) zw[k] = requant4_fast<NL, HZ>(acc[k][0], acc[k][1], acc[k][2], acc[k][3], zw[k], epi);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            __builtin_amdgcn_raw_buffer_store_b32((int)zw[k], rs_dst, l.p + u + k * 16 < pixels ? l.out + k * 64 : SENT, base + u * 4, 0);
+    }
+}
+
 template <bool HZ, class Form>
 __device__ __forceinline__ void grp16_run(const Form& form) {
     __shared__ __attribute__((aligned(16))) v4i sm[G16_PX], sf[144];
@@ -287,9 +350,16 @@ __device__ __forceinline__ void grp16_run(const Form& form) {
     const int l16 = lane & 15, kq = lane >> 4, slab = blockIdx.y;
     const int PH = (a.TH - 1) * a.s + 3, patch = PH * a.PW;
 
-    v4i x[G16_PX / 256];
-    auto fetch = [&](int item) __attribute__((always_inline)) {
-        const int n = (int)fdiv_u(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
+    // The slab's filter is one contiguous piece, at most 2304 bytes: 16 bytes per thread into LDS, ahead of the band's pixels, and
+    // from there each lane takes its dwords.  (Taken from memory, 48 gathers of 64 scattered dwords per workgroup cost more of the
+    // vector-memory path than everything else.)
+    const int icb = 1 << (a.log_icpg - 2), f_vecs = 36 * icb;
+    const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, (uint32_t)(a.slabs * f_vecs) * 16);
+    const v4i f_vec = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, t < f_vecs ? (slab * f_vecs + t) * 16 : SENT, 0, 0);
+    const v4i bv = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(a.bias, a.has_bias ? a.slabs * 64 : 0), (slab * 16 + kq * 4) * 4, 0, 0);
+    const int item = blockIdx.x, n = (int)fdiv_u(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
+    {
+        v4i x[G16_PX / 256];
         const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.src + n * a.src_sn + (int64_t)slab * 4 * a.src_scb, (uint32_t)a.src_scb * 4);
 #pragma unroll
         for (int k = 0; k < G16_PX / 256; ++k) {
@@ -300,20 +370,10 @@ __device__ __forceinline__ void grp16_run(const Form& form) {
 #pragma unroll
             for (int b = 0; b < 4; ++b) x[k][b] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, off, b * a.src_scb, 0);
         }
-    };
-
-    // The slab's filter is one contiguous piece, at most 2304 bytes: 16 bytes per thread into LDS, ahead of the band's pixels, and
-    // from there each lane takes its dwords.  (Taken from memory, 48 gathers of 64 scattered dwords per workgroup cost more of the
-    // vector-memory path than everything else.)
-    const int icb = 1 << (a.log_icpg - 2), f_vecs = 36 * icb;
-    const __amdgpu_buffer_rsrc_t rs_flt = make_rsrc(a.flt, (uint32_t)(a.slabs * f_vecs) * 16);
-    const v4i f_vec = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, t < f_vecs ? (slab * f_vecs + t) * 16 : SENT, 0, 0);
-    const v4i bv = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(a.bias, a.has_bias ? a.slabs * 64 : 0), (slab * 16 + kq * 4) * 4, 0, 0);
-    int item = blockIdx.x;
-    fetch(item);
-    if (t < f_vecs) sf[t] = f_vec;
+        if (t < f_vecs) sf[t] = f_vec;
 #pragma unroll
-    for (int k = 0; k < G16_PX / 256; ++k) sm[t + k * 256] = x[k];
+        for (int k = 0; k < G16_PX / 256; ++k) sm[t + k * 256] = x[k];
+    }
     __syncthreads();
     // filter rows: lane = output channel, 16 bytes of tap 4 step + kq = its 16 input channels, zero outside its group
     v4i fa[3];
@@ -330,64 +390,51 @@ __device__ __forceinline__ void grp16_run(const Form& form) {
             fa[st][b] = in ? w : 0;
         }
     }
-    for (;;) {
-        const int next = item + a.step;
-        if (next < a.items) fetch(next);  // lands during the multiplies
-        const int n = (int)fdiv_u(item, a.div_bands), oh0 = (item - n * a.bands) * a.TH;
-        const int pixels = (a.OH - oh0 < a.TH ? a.OH - oh0 : a.TH) * a.OW;
-        const int64_t at = (int64_t)(slab * 4 + kq) * a.dst_scb + (int64_t)oh0 * a.OW * 4;
-        int8_t* dst = a.dst + n * a.dst_sn + at;
-        const int8_t* z = a.z + n * a.z_sn + at;
-        // two units of 16 pixels at a time; the operands of the next two are read while these are requantised
-        v4i fb[2][3];
-        auto operands = [&](int u) __attribute__((always_inline)) {
+    // Where a lane's two pixels of a step lie: column out and byte of the staged band.  Every band begins with the same, and 128 pixels
+    // further on is a sum and a wrap (a division per pixel and step, with its quarter-rate multiplications, was a third of the loop's
+    // vector instructions).
+    const uint32_t rows128 = fdiv_u(128, a.div_ow);
+    const int cols128 = 128 - (int)rows128 * a.OW;
+    G16Lane l;
+    l.step = ((int)rows128 * a.PW + cols128) * a.s * 16;
+    l.wrap = (a.PW - a.OW) * a.s * 16;
+    l.cols = cols128;
+    l.OW = a.OW;
+    l.last = (((a.TH - 1) * a.PW + a.OW - 1) * a.s) * 16;
 #pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const int p = u + k * 16 + l16, pp = p < pixels ? p : 0;
-                const int oh = (int)fdiv(pp, a.div_ow), ow = pp - oh * a.OW;
-                const v4i* px = sm + (oh * a.PW + ow) * a.s;
-#pragma unroll
-                for (int st = 0; st < 3; ++st) fb[k][st] = px[tap_off[st]];
-            }
-        };
-        operands(wave * 32);
-        for (int u = wave * 32; u < pixels; u += 128) {
-            uint32_t zw[2] = {0, 0};
-            v4i acc[2] = {bv, bv};
-            if (HZ)
-#pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const int p = u + k * 16 + l16;
-                    zw[k] = *reinterpret_cast<const uint32_t*>(z + (p < pixels ? p : 0) * 4);
-                }
-#pragma unroll
-            for (int st = 0; st < 3; ++st)
-#pragma unroll
-                for (int k = 0; k < 2; ++k) acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[st], fb[k][st], acc[k], 0, 0, 0);
-            operands(u + 128);
-            __builtin_amdgcn_sched_barrier(0);
-            requant8(acc[0], acc[1], zw, a.epi);
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const int p = u + k * 16 + l16;
-                if (p < pixels) *reinterpret_cast<uint32_t*>(dst + p * 4) = zw[k];
-            }
-        }
-        if (next >= a.items) break;
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < G16_PX / 256; ++k) sm[t + k * 256] = x[k];
-        __syncthreads();
-        item = next;
+    for (int k = 0; k < 2; ++k) {
+        const int p = wave * 32 + k * 16 + l16, oh = (int)fdiv(p, a.div_ow);
+        l.ow[k] = p - oh * a.OW;
+        l.at[k] = (oh * a.PW + l.ow[k]) * a.s * 16;
     }
+#pragma unroll
+    for (int st = 0; st < 3; ++st) l.tap[st] = tap_off[st] * 16;
+    l.out = kq * a.dst_scb + (wave * 32 + l16) * 4;
+    l.p = wave * 32 + l16;
+    const int pixels = (a.OH - oh0 < a.TH ? a.OH - oh0 : a.TH) * a.OW;
+    const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst + n * a.dst_sn + (int64_t)slab * 4 * a.dst_scb, (uint32_t)a.dst_scb * 4);
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z + (HZ ? n * a.z_sn + (int64_t)slab * 4 * a.dst_scb : 0), HZ ? (uint32_t)a.dst_scb * 4 : 0);
+#define MI355_BAND(NL) grp16_band<NL, HZ>(a.epi, l, sm, fa, bv, rs_dst, rs_z, oh0 * a.OW * 4, pixels, wave * 32)
+    // one loop per requantisation form: with the choice inside it a step was a dozen branches longer and the kernel held 116 registers
+    if (HZ) {
+        if (!a.epi.fast) MI355_BAND(G16_ANY);
+        else if (a.epi.nonline == NL_RELU) MI355_BAND(NL_RELU);
+        else if (a.epi.nonline == NL_H_SWISH) MI355_BAND(NL_H_SWISH);
+        else MI355_BAND(NL_IDENTITY);
+    } else {
+        if (a.epi.lin) MI355_BAND(NL_LIN);
+        else if (a.epi.fast && a.epi.nonline == NL_H_SWISH) MI355_BAND(NL_H_SWISH);
+        else MI355_BAND(G16_ANY);
+    }
+#undef MI355_BAND
 }
 
 template <bool HZ>
-__global__ __launch_bounds__(256) void grp16_kernel(G16Wire a) {
+__global__ __launch_bounds__(256, 6) void grp16_kernel(G16Wire a) {
     grp16_run<HZ>(a);
 }
 template <bool HZ>
-__global__ __launch_bounds__(256) void grp16_kernel(G16Wide a) {
+__global__ __launch_bounds__(256, 6) void grp16_kernel(G16Wide a) {
     grp16_run<HZ>(a);
 }
 
@@ -404,44 +451,55 @@ int g16_rows(const ConvProblem& p) {
     return rows < 3 ? 0 : (rows - 3) / s + 1;
 }
 
+// Output rows of a band, one band to a workgroup: equal bands (oh = 87 in rows of 44, not 76 and 11), as many as cost least.  A workgroup
+// takes 0.29 us of its CU and 0.06 per step of 128 pixels, beside 0.09 per step of its own chain and 0.12 of memory; W: workgroups of the
+// busiest CU, w: on average.  Fitted to graph replays of every band of 160 drawn layers: 0.3 % behind the best band on average, 6 % at most,
+// where fewer rows until there were 240 or 512 workgroups was 5.4 % behind (8 groups of 16 at 46 x 30, batch 42: 6.91 -> 5.69 us).
+int g16_band_rows(const ConvProblem& p, int cu_count) {
+    const int rows = g16_rows(p), oh = (int)p.oh, ow = (int)p.ow, cu = cu_count > 0 ? cu_count : 256;
+    int best = 0;
+    float least = 0.f;
+    for (int bands = (oh + rows - 1) / rows;;) {
+        const int th = (oh + bands - 1) / bands, steps = (th * ow + 127) / 128;
+        const int64_t items = (int64_t)p.d.n * ((oh + th - 1) / th), wgs = items * (p.d.oc / 16);
+        const float W = (float)((wgs + cu - 1) / cu), w = (float)wgs / (float)cu;
+        const float cost = (float)steps * (0.091f + 0.117f * w + 0.059f * W) + 0.287f * W;
+        if (best == 0 || (cost < least && items < G16_BANDS)) {
+            best = th;
+            least = cost;
+        }
+        if (th == 1 || steps == 1) return best;
+        bands = (oh + th - 2) / (th - 1);  // the next smaller band
+    }
+}
+
 bool g16_usable(const ConvProblem& p) {
     const mi355_conv_desc& d = p.d;
     return d.fh == 3 && d.fw == 3 && d.stride_h == d.stride_w && d.stride_h <= 2 && p.icpg == p.ocpg &&
            (p.icpg == 4 || p.icpg == 8 || p.icpg == 16) && d.oc % 16 == 0 && p.ow < G16_PX && g16_rows(p) > 0 &&
-           (int64_t)d.ih * d.iw * 16 < (1ll << 31);
+           (int64_t)d.ih * d.iw * 16 < (1ll << 31) && (int64_t)p.oh * p.ow * 16 < (1ll << 31) &&
+           (int64_t)d.n * ((p.oh + g16_rows(p) - 1) / g16_rows(p)) < G16_BANDS;
 }
 
-int launch_g16(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+int launch_g16(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                int8_t* dst) {
     const mi355_conv_desc& d = p.d;
     G16Args<FastDiv> a;
     a.src = src; a.flt = reinterpret_cast<const int*>(flt); a.bias = bias; a.z = z; a.dst = dst;
     a.IH = d.ih; a.IW = d.iw; a.OH = p.oh; a.OW = p.ow; a.s = d.stride_h; a.ph = d.pad_h; a.pw = d.pad_w;
     const int slabs = d.oc / 16;
-    a.TH = g16_rows(p);
-    if (a.TH > (int)p.oh) a.TH = p.oh;
-    // Fewer rows per band while that leaves CUs without one, or with one long one: a workgroup's fixed part is worth about 200
-    // pixels (8 groups of 16 at 11 x 10, batch 30, 240 workgroups: 4.3 us, 5.0 with twice as many; 6 groups of 16 at 20 x 70, batch
-    // 18, H_SWISH and a residual: 7.8 with bands of 420 pixels, 6.9 with 210).
-    while (a.TH > 1) {
-        const int64_t wgs = (int64_t)slabs * d.n * ((p.oh + a.TH - 1) / a.TH);
-        if (wgs >= (a.TH * (int)p.ow > 400 ? 512 : 240)) break;
-        a.TH = (a.TH + 1) / 2;
-    }
+    a.TH = g16_band_rows(p, cu_count);
     a.PW = ((int)p.ow - 1) * a.s + 3;
     a.bands = ((int)p.oh + a.TH - 1) / a.TH;
     const int64_t items = (int64_t)d.n * a.bands;
-    if (items > 0x3fffffff) return (int)hipErrorInvalidValue;
     a.items = (int)items;
     a.log_icpg = p.icpg == 4 ? 2 : p.icpg == 8 ? 3 : 4; a.src_scb = d.ih * d.iw * 4; a.dst_scb = p.oh * p.ow * 4;
     a.has_bias = d.bias_mode == MI355_BIAS_BROADCAST_CHANNEL;
     a.src_sn = p.src_sn; a.dst_sn = p.dst_sn; a.z_sn = p.z_sn;
     a.div_pw = make_fastdiv(a.PW); a.div_ow = make_fastdiv(p.ow); a.div_bands = make_fastdiv(a.bands);
     a.epi = p.epi;
-    int64_t per_slab = (2048 + slabs - 1) / slabs;  // eight workgroups per CU over all slabs
-    if (per_slab > items) per_slab = items;
-    a.slabs = slabs; a.step = (int)per_slab;
-    const dim3 grid((unsigned)per_slab, slabs);
+    a.slabs = slabs;
+    const dim3 grid((unsigned)items, slabs);
     G16Wire wire;
     return wire.pack(a, d.n) ? launch_g16_form(st, grid, wire, d.has_z) : launch_g16_form(st, grid, G16Wide{a}, d.has_z);
 }
@@ -482,11 +540,11 @@ bool grp4_usable(const ConvProblem& p) {
            d.n <= 65535 && d.oc / 4 <= 65535 && (uint64_t)p.oh * p.ow < (1u << 28);
 }
 
-int launch_grp4(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+int launch_grp4(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                 int8_t* dst) {
     const mi355_conv_desc& d = p.d;
     if (d.n == 0 || p.oh == 0 || p.ow == 0) return 0;
-    if (g16_usable(p)) return launch_g16(st, p, src, flt, bias, z, dst);
+    if (g16_usable(p)) return launch_g16(st, p, cu_count, src, flt, bias, z, dst);
     Grp4Args<FastDiv> a;
     a.src = src; a.flt = reinterpret_cast<const int*>(flt); a.bias = bias; a.z = z; a.dst = dst;
     a.IH = d.ih; a.IW = d.iw; a.OH = p.oh; a.OW = p.ow; a.FH = d.fh; a.FW = d.fw;

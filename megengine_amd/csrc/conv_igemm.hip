@@ -1031,7 +1031,7 @@ int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_coun
                       const int8_t* flt, const int32_t* bias, const int8_t* z, int8_t* dst, bool flt_preprocessed, int flt_rows) {
     if (igemm_group_by_launch(p)) {
         if (flt_preprocessed) return (int)hipErrorInvalidValue;
-        if (cfg == igemm_grp4_cfg() && grp4_usable(p)) return launch_grp4(st, p, src, flt, bias, z, dst);
+        if (cfg == igemm_grp4_cfg() && grp4_usable(p)) return launch_grp4(st, p, cu_count, src, flt, bias, z, dst);
         const ConvProblem q = igemm_group_view(p);
         const mi355_conv_desc& d = p.d;
         const int64_t src_g = (int64_t)p.icpg * d.ih * d.iw, dst_g = (int64_t)p.ocpg * p.oh * p.ow;

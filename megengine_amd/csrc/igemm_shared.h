@@ -540,7 +540,7 @@ int launch_igemm4(hipStream_t st, IgemmArgs& a, int pin, int pout, int cfg, int 
 // NCHW4 group convolutions with few channels per group in one launch (conv_group4.hip, tile "grp4_dot4")
 bool grp4_usable(const ConvProblem& p);
 bool grp4_pick(const ConvProblem& p);  // whether it is ahead of one dense launch per group
-int launch_grp4(hipStream_t st, const ConvProblem& p, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
+int launch_grp4(hipStream_t st, const ConvProblem& p, int cu_count, const int8_t* src, const int8_t* flt, const int32_t* bias, const int8_t* z,
                 int8_t* dst);
 
 // few output pixels: the reduction split over the waves of a workgroup, operands straight into registers
