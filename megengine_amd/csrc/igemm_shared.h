@@ -110,7 +110,7 @@ __device__ __forceinline__ void requant8(v4i x, v4i y, uint32_t (&w)[2], const E
         w[1] = F(y[0], y[1], y[2], y[3], w[1], e);     \
     } while (0)
     if (e.lin) MI355_BOTH((requant4_fast<NL_LIN, false>));
-    else if (e.nonline == NL_RELU && !e.has_z) MI355_BOTH((requant4_fast<NL_RELU, false>));
+    else if (e.fast && e.nonline == NL_RELU && !e.has_z) MI355_BOTH((requant4_fast<NL_RELU, false>));
     else MI355_BOTH(requant4);
 #undef MI355_BOTH
 }

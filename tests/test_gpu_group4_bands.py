@@ -22,7 +22,7 @@ CASES = [
 SCALES = [
     dict(scale_bias=1.3e-3, scale_z=0.05, scale_dst=0.0271),   # a linear form for IDENTITY and RELU without a residual
     dict(scale_bias=2e-4, scale_z=0.05, scale_dst=0.05),       # none: the quotient form
-    dict(scale_bias=2e-4, scale_z=0.05, scale_dst=1e-39),      # not even that: the literal chain
+    dict(scale_bias=1e-20, scale_z=3e-19, scale_dst=1e-18),    # not even that: the literal chain
 ]
 
 
