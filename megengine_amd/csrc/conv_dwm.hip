@@ -223,38 +223,47 @@ __device__ __forceinline__ void dwm_run(const Form& form) {
     for (int st = 0; st < STEPS; ++st)
 #pragma unroll
         for (int p = 0; p < 4; ++p) fa[st][p] = reinterpret_cast<const int*>(lds_dwm)[woff[st] + p] & mask;
-    for (int u = wave * 32; u < quads; u += step) {
-        v4i fb[2][STEPS];
-        uint32_t zw[2] = {zn[0], zn[1]};
-        int d[2];
+    // One loop per requantisation form: chosen inside it the form was a dozen branches per step (5x5, 60 channels at 76 x 22, batch 21, with a
+    // residual: 6.99 -> 5.81 us; 240 channels at 57 x 57, stride 2, batch 16, H_SWISH: 7.41 -> 6.67).  Without branches the compiler reads a
+    // step's operands further ahead, so registers are bounded to five waves per SIMD, as before (unbounded: 544 channels at 95 x 100, stride 2,
+    // batch 22: 45.9 -> 52.0 us).  Longer windows would spill then and keep the choice inside.
+    auto multiply = [&](auto form_of) __attribute__((always_inline)) {
+        constexpr int NL = decltype(form_of)::value;
+        for (int u = wave * 32; u < quads; u += step) {
+            v4i fb[2][STEPS];
+            uint32_t zw[2] = {zn[0], zn[1]};
+            int d[2];
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
+            for (int k = 0; k < 2; ++k) {
 #pragma unroll
-            for (int st = 0; st < STEPS; ++st) fb[k][st] = lds_dwm[un[k].src + boff[st]];
-            d[k] = un[k].dst;
+                for (int st = 0; st < STEPS; ++st) fb[k][st] = lds_dwm[un[k].src + boff[st]];
+                d[k] = un[k].dst;
+            }
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                un[k] = unit(u + step + k * 16);
+                if (HZ) zn[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, un[k].dst, 0, 0);
+            }
+            v4i acc[2] = {bv, bv};
+#pragma unroll
+            for (int st = 0; st < STEPS; ++st)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[st], fb[k][st], acc[k], 0, 0, 0);
+            requant8_as<NL, HZ>(acc[0], acc[1], zw, a.epi);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) __builtin_amdgcn_raw_buffer_store_b32(zw[k], rs_dst, d[k], 0, 0);
         }
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            un[k] = unit(u + step + k * 16);
-            if (HZ) zn[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, un[k].dst, 0, 0);
-        }
-        v4i acc[2] = {bv, bv};
-#pragma unroll
-        for (int st = 0; st < STEPS; ++st)
-#pragma unroll
-            for (int k = 0; k < 2; ++k) acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[st], fb[k][st], acc[k], 0, 0, 0);
-        requant8(acc[0], acc[1], zw, a.epi);
-#pragma unroll
-        for (int k = 0; k < 2; ++k) __builtin_amdgcn_raw_buffer_store_b32(zw[k], rs_dst, d[k], 0, 0);
-    }
+    };
+    if constexpr (STEPS <= 4) with_requant_form<HZ>(a.epi, multiply);
+    else multiply(std::integral_constant<int, NL_ANY>());
 }
 
 template <int STEPS, bool HZ>
-__global__ __launch_bounds__(256) void dwm_kernel(DwmWire a) {
+__global__ __launch_bounds__(256, 5) void dwm_kernel(DwmWire a) {
     dwm_run<STEPS, HZ>(a);
 }
 template <int STEPS, bool HZ>
-__global__ __launch_bounds__(256) void dwm_kernel(DwmWide a) {
+__global__ __launch_bounds__(256, 5) void dwm_kernel(DwmWide a) {
     dwm_run<STEPS, HZ>(a);
 }
 

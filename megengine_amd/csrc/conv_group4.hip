@@ -24,7 +24,6 @@
 // gathered dword by dword ahead of it, and the next operands read while results are requantised, 55 groups of 16 at 8 x 47,
 // stride 2, batch 4 went from 6.2 to 4.2 us, 5 groups of 16 at 33 x 100, stride 2, batch 64 from 9.8 to 8.4.
 #include <tuple>
-#include <type_traits>
 
 #include "igemm_shared.h"
 #include "wire.h"
@@ -282,8 +281,6 @@ struct G16Wire {
 };
 static_assert(sizeof(G16Wire) <= WIRE_BYTES, "a wire");
 
-constexpr int G16_ANY = -1;  // the requantisation form is chosen where it is used
-
 struct G16Lane {
     int ow[2], at[2];  // of the lane's two pixels of a band's first step: column out, byte of the staged band
     int OW, step, wrap, cols, last;  // (uniform) columns out; 128 pixels on: bytes, bytes where the row ends, columns; the last pixel's byte
@@ -330,12 +327,7 @@ __device__ __forceinline__ void grp16_band(const EpiParams& epi, const G16Lane& 
         operands();
         if (HZ) residual(u + 128);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (NL == G16_ANY) {
-            requant8(acc[0], acc[1], zw, epi);
-        } else {
-#pragma unroll
-            for (int k = 0; k < 2; ++k) zw[k] = requant4_fast<NL, HZ>(acc[k][0], acc[k][1], acc[k][2], acc[k][3], zw[k], epi);
-        }
+        requant8_as<NL, HZ>(acc[0], acc[1], zw, epi);
 #pragma unroll
         for (int k = 0; k < 2; ++k)
             __builtin_amdgcn_raw_buffer_store_b32((int)zw[k], rs_dst, l.p + u + k * 16 < pixels ? l.out + k * 64 : SENT, base + u * 4, 0);
@@ -414,19 +406,10 @@ __device__ __forceinline__ void grp16_run(const Form& form) {
     const int pixels = (a.OH - oh0 < a.TH ? a.OH - oh0 : a.TH) * a.OW;
     const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst + n * a.dst_sn + (int64_t)slab * 4 * a.dst_scb, (uint32_t)a.dst_scb * 4);
     const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z + (HZ ? n * a.z_sn + (int64_t)slab * 4 * a.dst_scb : 0), HZ ? (uint32_t)a.dst_scb * 4 : 0);
-#define MI355_BAND(NL) grp16_band<NL, HZ>(a.epi, l, sm, fa, bv, rs_dst, rs_z, oh0 * a.OW * 4, pixels, wave * 32)
     // one loop per requantisation form: with the choice inside it a step was a dozen branches longer and the kernel held 116 registers
-    if (HZ) {
-        if (!a.epi.fast) MI355_BAND(G16_ANY);
-        else if (a.epi.nonline == NL_RELU) MI355_BAND(NL_RELU);
-        else if (a.epi.nonline == NL_H_SWISH) MI355_BAND(NL_H_SWISH);
-        else MI355_BAND(NL_IDENTITY);
-    } else {
-        if (a.epi.lin) MI355_BAND(NL_LIN);
-        else if (a.epi.fast && a.epi.nonline == NL_H_SWISH) MI355_BAND(NL_H_SWISH);
-        else MI355_BAND(G16_ANY);
-    }
-#undef MI355_BAND
+    with_requant_form<HZ>(a.epi, [&](auto form_of) __attribute__((always_inline)) {
+        grp16_band<decltype(form_of)::value, HZ>(a.epi, l, sm, fa, bv, rs_dst, rs_z, oh0 * a.OW * 4, pixels, wave * 32);
+    });
 }
 
 template <bool HZ>

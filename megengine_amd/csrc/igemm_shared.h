@@ -1,5 +1,7 @@
 // Declarations shared by the implicit-GEMM kernels (register-staged and LDS-direct variants).
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace mi355 {
@@ -113,6 +115,32 @@ __device__ __forceinline__ void requant8(v4i x, v4i y, uint32_t (&w)[2], const E
     else if (e.fast && e.nonline == NL_RELU && !e.has_z) MI355_BOTH((requant4_fast<NL_RELU, false>));
     else MI355_BOTH(requant4);
 #undef MI355_BOTH
+}
+
+// For loops that requantise in every step: the form chosen once, ahead of the loop.  f is called with an integral_constant, the NL of
+// requant8_as; NL_ANY stands for the forms that are rare (the literal chain; IDENTITY and RELU without a residual and without a linear form).
+constexpr int NL_ANY = -1;
+template <bool HZ, class F>
+__device__ __forceinline__ void with_requant_form(const EpiParams& e, F f) {
+    if (HZ) {
+        if (!e.fast) f(std::integral_constant<int, NL_ANY>());
+        else if (e.nonline == NL_RELU) f(std::integral_constant<int, NL_RELU>());
+        else if (e.nonline == NL_H_SWISH) f(std::integral_constant<int, NL_H_SWISH>());
+        else f(std::integral_constant<int, NL_IDENTITY>());
+    } else {
+        if (e.lin) f(std::integral_constant<int, NL_LIN>());
+        else if (e.fast && e.nonline == NL_H_SWISH) f(std::integral_constant<int, NL_H_SWISH>());
+        else f(std::integral_constant<int, NL_ANY>());
+    }
+}
+template <int NL, bool HZ>
+__device__ __forceinline__ void requant8_as(v4i x, v4i y, uint32_t (&w)[2], const EpiParams& e) {
+    if constexpr (NL == NL_ANY) {
+        requant8(x, y, w, e);
+    } else {
+        w[0] = requant4_fast<NL, HZ>(x[0], x[1], x[2], x[3], w[0], e);
+        w[1] = requant4_fast<NL, HZ>(y[0], y[1], y[2], y[3], w[1], e);
+    }
 }
 
 // Residual (z) of one wave tile in the order the epilogue consumes it: POUT = 32: one 16-byte vector per 32x32 block
