@@ -1081,7 +1081,7 @@ int launch_conv_igemm(hipStream_t st, const ConvProblem& p, int cfg, int cu_coun
     }
     if (cfg >= igemm_first_g32_cfg()) return launch_grp32(st, a, cfg - igemm_first_g32_cfg());
     if (cfg == igemm_pw4_split_cfg()) return launch_pw4_split(st, a);
-    if (cfg >= igemm_first_p4_cfg()) return launch_patch4(st, a, cfg - igemm_first_p4_cfg());
+    if (cfg >= igemm_first_p4_cfg()) return launch_patch4(st, a, cfg - igemm_first_p4_cfg(), cu_count > 0 ? cu_count : 256);
     if (cfg >= igemm_first_ks_cfg()) return launch_igemm5(st, a, p.pin, p.pout, cfg - igemm_first_ks_cfg());
     if (cfg == igemm_pw32s_cfg()) return launch_pw32s(st, a, cu_count);
     if (cfg >= igemm_first_v4_cfg()) return launch_igemm4(st, a, p.pin, p.pout, cfg - igemm_first_v4_cfg(), cu_count);

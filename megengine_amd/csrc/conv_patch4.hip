@@ -19,12 +19,16 @@
 //     costs a third of the occupancy.  Loads two stages ahead, tried, cost more occupancy than they hid (7.5 us against 6.9 at
 //     56 x 56 below); reading one step's operands ahead instead of two, or computing a descriptor per channel block instead of
 //     a scalar offset (157 scalar instructions per stage instead of 64), cost up to a quarter of the time.
+//   * Where there is a workgroup to a CU or fewer, it has two groups of four waves that take every other stage each (p4_split_lds).
 //   * 3x3 over at most 64 channels has a kernel of its own with one stage (patch4_one_kernel), ahead at every size and tile: 64 -> 64 at
 //     56 x 56, batch 16: 7.5 -> 7.0 us; 28 -> 20 at 29 x 28, stride 2, batch 34: 4.6 -> 3.9; 48 -> 148 at 97 x 107, batch 7: 20.7 -> 14.3;
 //     56 -> 480 at 82 x 94, batch 10: 50 -> 41; 30 drawn layers on each tile: 1.05 to 1.25 times as fast.
 // Graph replays of the layer, here and below: 3x3 64 -> 64 at 56 x 56, batch 16: 12.4 -> 6.9 us, batch 64: 31.7 -> 17.0; 256 ->
 // 256 at 14 x 14, batch 16: 15.5 -> 8.3; 32 -> 32 at 112 x 112, batch 64: 52 -> 26.8; 5x5 100 -> 132 at 33 x 35, batch 20: 50 -> 22.5.
+// 5x5 has its thirteen steps compiled in as nine taps have: in the general form's loop the compiler reads a step's operands next to the product that
+// waits for them (80 -> 228 at 15 x 52, batch 30: 28.3 -> 22.6 us; 220 -> 88 at 65 x 102, batch 9: 82 -> 68).
 #include <atomic>
+#include <algorithm>
 
 #include "igemm_shared.h"
 
@@ -55,16 +59,17 @@ struct P4Args {
     EpiParams epi;
 };
 
-template <int MT, int NT, int NL, bool HZ>
+// QN: quads of channels of each block of 32 that are in acc (all four of the sixteen sums, or the first two)
+template <int MT, int NT, int QN, int NL, bool HZ>
 __device__ __forceinline__ void p4_epilogue(const P4Args& a, v16i (&acc)[MT][NT], int oc0, const int (&d_px)[NT], const int (&z_px)[NT], int lh) {
-    uint32_t zw[NT][MT][4];
+    uint32_t zw[NT][MT][QN];
     if (HZ) {
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
+                for (int q = 0; q < QN; ++q) {
                     const int oc4 = oc0 + i * 32 + 8 * q + 4 * lh;
                     zw[j][i][q] = d_px[j] >= 0 && oc4 < a.OC ? *reinterpret_cast<const uint32_t*>(a.z + z_px[j] + (int64_t)(oc4 >> 2) * a.dst_scb) : 0u;
                 }
@@ -74,7 +79,7 @@ __device__ __forceinline__ void p4_epilogue(const P4Args& a, v16i (&acc)[MT][NT]
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
+            for (int q = 0; q < QN; ++q) {
                 const int oc4 = oc0 + i * 32 + 8 * q + 4 * lh;
                 const v16i& c = acc[i][j];
                 const uint32_t o = requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], HZ ? zw[j][i][q] : 0u, a.epi);
@@ -82,9 +87,9 @@ __device__ __forceinline__ void p4_epilogue(const P4Args& a, v16i (&acc)[MT][NT]
             }
 }
 
-template <int MT, int NT>
+template <int MT, int NT, int QN = 4>
 __device__ __forceinline__ void p4_finish(const P4Args& a, v16i (&acc)[MT][NT], int oc0, const int (&d_px)[NT], const int (&z_px)[NT], int lh) {
-#define MI355_P4(NL, HZ) p4_epilogue<MT, NT, NL, HZ>(a, acc, oc0, d_px, z_px, lh)
+#define MI355_P4(NL, HZ) p4_epilogue<MT, NT, QN, NL, HZ>(a, acc, oc0, d_px, z_px, lh)
     if (a.epi.lin) {
         MI355_P4(NL_LIN, false);
     } else if (a.epi.has_z) {
@@ -103,216 +108,27 @@ __device__ __forceinline__ void p4_finish(const P4Args& a, v16i (&acc)[MT][NT], 
 #undef MI355_P4
 }
 
-// STEPS: MFMA steps of a stage when known (9: nine taps, two channel groups), 0: from the arguments
-template <int MT, int NT, int STEPS>
-__global__ __launch_bounds__(256, 2) void patch4_kernel(P4Args a) {
-    constexpr int BM = MT * 32, KAN = (BM + 13) / 14;
-    // vectors from one entry to the next: the rows its passes store, made odd so that the stores of a row spread over the banks
-    const int kan = STEPS ? KAN : a.kan, rpi = STEPS ? 14 : a.rpi, BMP = (kan * rpi) | 1;
-    extern __shared__ __attribute__((aligned(16))) v4i lds[];
-    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l32 = lane & 31, lh = lane >> 5;
-    const int E = a.GS * a.T, EP = (E + 1) & ~1;              // entries of a stage, of a whole number of steps
-    const int a_vecs = EP * BMP, stage_vecs = a_vecs + a.GS * a.PX;
-
-    // tile: contiguous pixel tiles per XCD (workgroup b runs on XCD b % 8), channel tiles of a pixel tile side by side
-    int tm, tn;
-    {
-        const int per = (a.tiles_n + 7) >> 3, x = blockIdx.x & 7, i = blockIdx.x >> 3;
-        const int r = (int)fdiv(i, a.div_tiles_m);
-        tm = i - r * a.tiles_m;
-        tn = x * per + r;
-        if (r >= per || tn >= a.tiles_n) return;
-    }
-    const int ig = (int)fdiv(tn, a.div_tiles_img), ti = tn - ig * a.tiles_img;
-    const int th = (int)fdiv(ti, a.div_tiles_w), tw = ti - th * a.tiles_w;
-    const int n0 = ig * a.NI, oh0 = th * a.TH, ow0 = tw * a.TW, oc0 = tm * BM;
-
-    // patch pixels of this thread: source offset of the first channel block, SENT outside the image
-    int p_off[P4_NPK];
-#pragma unroll
-    for (int k = 0; k < P4_NPK; ++k) {
-        if (k >= a.pkn) break;
-        const uint32_t px = t + k * 256, im = fdiv(px, a.div_pxi), r = px - im * a.PXI, pr = fdiv(r, a.div_pwc), pc = r - pr * a.PWC;
-        const int ih = oh0 * a.sh - a.ph + (int)pr, iw = ow0 * a.sw - a.pw + (int)pc, n = n0 + (int)im;
-        const bool ok = (int)px < a.PX && n < a.N && (unsigned)ih < (unsigned)a.IH && (unsigned)iw < (unsigned)a.IW;
-        p_off[k] = ok ? n * a.src_sn + (ih * a.IW + iw) * 4 : SENT;
-    }
-    // filter vectors of this thread: the same 16 bytes of every rpi-th row; dword d of a row is tap d % T of channel block
-    // d / T (rows past the last channel lie past the end of the buffer: zero)
-    const int T = STEPS ? 9 : a.T, vr = STEPS ? 18 : a.vr;
-    const int f_row = STEPS ? t / 18 : (int)fdiv(t, a.div_vr), f_first = (t - f_row * vr) * 4;
-    int f_off[P4_NKA];
-#pragma unroll
-    for (int k = 0; k < P4_NKA; ++k) {
-        if (k >= kan) break;
-        f_off[k] = f_row < rpi ? (oc0 + f_row + k * rpi) * a.kbytes + f_first * 4 : SENT;
-    }
-    const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes), rs_flt = make_rsrc(a.flt, a.flt_bytes);
-    v4i xp[P4_NPK], xf[P4_NKA];
-    const int row_words = a.icb * T, GS = STEPS ? 2 : a.GS;
-    // The patch's channel blocks are a scalar offset: those past the last one are the last one's again (they meet zero filter
-    // bytes), so that the scalar offset never leads out of the image.  The filter's stage is part of the lane's offset, which
-    // the descriptor's bounds check covers.
-    const uint32_t last_cb = (uint32_t)(a.icb - 1) * a.src_scb;
-    auto fetch = [&](int st) __attribute__((always_inline)) {
-        const int cb0 = st * GS * 4, left = row_words - cb0 * T;  // filter words left in a row
-        const int fo = cb0 * T * 4;
-#pragma unroll
-        for (int k = 0; k < P4_NKA; ++k) {
-            if (k >= kan) break;
-            xf[k] = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, f_off[k] + fo, 0, 0);
-        }
-        int so[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) so[i] = (int)min((uint32_t)(cb0 + i) * a.src_scb, last_cb);
-#pragma unroll
-        for (int k = 0; k < P4_NPK; ++k) {
-            if (k >= a.pkn) break;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) xp[k][i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_src, p_off[k], so[i], 0);
-            if (k < P4_NPK / 2 && GS == 2) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) xp[P4_NPK / 2 + k][i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_src, p_off[k], so[4 + i], 0);
-            }
-        }
-        if (left < vr * 4) {  // the last stage, incomplete: words past the row's end are the next row's
-#pragma unroll
-            for (int k = 0; k < P4_NKA; ++k)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) xf[k][i] = f_first + i < left ? xf[k][i] : 0;
-        }
-    };
-    fetch(0);
-
-    int f_lds[4];
-    {
-        uint32_t cb = STEPS ? f_first / 9 : fdiv(f_first, a.div_t), tap = f_first - cb * T;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            f_lds[i] = (int)((((cb >> 2) * T + tap) * BMP + f_row) * 4 + (cb & 3));
-            if (++tap == (uint32_t)T) {
-                tap = 0;
-                ++cb;
-            }
-        }
-    }
-    auto store = [&](int buf) __attribute__((always_inline)) {
-        v4i* s = lds + buf * stage_vecs;
-        int* sw = reinterpret_cast<int*>(s);
-        if (f_row < rpi) {
-#pragma unroll
-            for (int k = 0; k < P4_NKA; ++k) {
-                if (k >= kan) break;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) sw[f_lds[i] + k * rpi * 4] = xf[k][i];
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < P4_NPK; ++k) {
-            if (k >= a.pkn) break;
-            if (t + k * 256 < a.PX) {
-                s[a_vecs + t + k * 256] = xp[k];
-                if (k < P4_NPK / 2 && GS == 2) s[a_vecs + a.PX + t + k * 256] = xp[P4_NPK / 2 + k];
-            }
-        }
-    };
-
-    // B operands: patch vector of each of this lane's pixels, and of each entry relative to it
-    int b_px[NT], d_px[NT], z_px[NT];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const uint32_t p = (wave * NT + j) * 32 + l32;
-        const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)(a.TH * a.TW), oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
-        const bool ok = (int)im < a.NI && n0 + (int)im < a.N && oh0 + (int)oh < a.OH && ow0 + (int)ow < a.OW;
-        b_px[j] = (int)im < a.NI ? (int)(im * a.PXI + oh * a.sh * a.PWC + ow * a.sw) : 0;
-        const int at = ((oh0 + (int)oh) * a.OW + ow0 + (int)ow) * 4;
-        d_px[j] = ok ? (n0 + (int)im) * a.dst_sn + at : -1;
-        z_px[j] = (n0 + (int)im) * a.z_sn + at;
-    }
-    int* tab = reinterpret_cast<int*>(lds + 2 * stage_vecs);
-    for (int e = t; e < EP; e += 256) {
-        const int g = (int)fdiv(e, a.div_t), tap = e - g * a.T, fh = tap / a.FW, fw = tap - fh * a.FW;
-        tab[e] = e < E ? a_vecs + g * a.PX + fh * a.PWC + fw : a_vecs;
-    }
-    // the filter entry that fills up an odd number stays zero
-    if (EP != E && t < 2 * BM) lds[(t / BM) * stage_vecs + E * BMP + t % BM] = v4i{0, 0, 0, 0};
-    v16i acc[MT][NT];
-    {
-        const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            v16i b;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const v4i v = __builtin_amdgcn_raw_buffer_load_b128(rs_bias, (oc0 + i * 32 + 8 * q + 4 * lh) * 4, 0, 0);
-                b[4 * q] = v[0]; b[4 * q + 1] = v[1]; b[4 * q + 2] = v[2]; b[4 * q + 3] = v[3];
-            }
-#pragma unroll
-            for (int j = 0; j < NT; ++j) acc[i][j] = b;
-        }
-    }
-    store(0);
-    __syncthreads();
-    const int steps = EP / 2;
-    int offs[STEPS ? STEPS : 1];
-    if constexpr (STEPS != 0) {
-#pragma unroll
-        for (int k = 0; k < STEPS; ++k) offs[k] = tab[2 * k + lh];
-    }
-    for (int st = 0; st < a.nstages; ++st) {
-        if (st + 1 < a.nstages) fetch(st + 1);
-        const v4i* s = lds + (st & 1) * stage_vecs;
-        const v4i* pa = s + lh * BMP + l32;
-        auto load = [&](int k, int off, v4i (&fa)[MT], v4i (&fb)[NT]) __attribute__((always_inline)) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i) fa[i] = pa[k * 2 * BMP + i * 32];
-#pragma unroll
-            for (int j = 0; j < NT; ++j) fb[j] = s[off + b_px[j]];
-        };
-        auto mult = [&](const v4i (&fa)[MT], const v4i (&fb)[NT]) __attribute__((always_inline)) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        };
-        if constexpr (STEPS != 0) {
-            constexpr int AHEAD = 2;  // steps whose operands are read ahead
-            v4i fa[AHEAD + 1][MT], fb[AHEAD + 1][NT];
-#pragma unroll
-            for (int k = 0; k < AHEAD; ++k) load(k, offs[k], fa[k], fb[k]);
-#pragma unroll
-            for (int k = 0; k < STEPS; ++k) {
-                if (k + AHEAD < STEPS) load(k + AHEAD, offs[k + AHEAD], fa[(k + AHEAD) % (AHEAD + 1)], fb[(k + AHEAD) % (AHEAD + 1)]);
-                __builtin_amdgcn_sched_barrier(0);
-                mult(fa[k % (AHEAD + 1)], fb[k % (AHEAD + 1)]);
-            }
-        } else {
-            // two steps' operands, and the table entries of the two after them, are read ahead (past the last step: its own)
-            v4i fa[3][MT], fb[3][NT];
-            const int last = steps - 1;
-            load(0, tab[lh], fa[0], fb[0]);
-            load(min(1, last), tab[2 * min(1, last) + lh], fa[1], fb[1]);
-            int o0 = tab[2 * min(2, last) + lh], o1 = tab[2 * min(3, last) + lh], o2 = tab[2 * min(4, last) + lh];
-            for (int k = 0; k < steps; k += 3) {
-                load(min(k + 2, last), o0, fa[2], fb[2]);
-                o0 = tab[2 * min(k + 5, last) + lh];
-                mult(fa[0], fb[0]);
-                if (k + 1 >= steps) break;
-                load(min(k + 3, last), o1, fa[0], fb[0]);
-                o1 = tab[2 * min(k + 6, last) + lh];
-                mult(fa[1], fb[1]);
-                if (k + 2 >= steps) break;
-                load(min(k + 4, last), o2, fa[1], fb[1]);
-                o2 = tab[2 * min(k + 7, last) + lh];
-                mult(fa[2], fb[2]);
-            }
-        }
-        if (st + 1 < a.nstages) store((st + 1) & 1);
-        __syncthreads();
-    }
-
-    p4_finish(a, acc, oc0, d_px, z_px, lh);
-}
+// the kernel, by groups of waves and taps of a stage
+namespace one {
+constexpr int KS = 1;
+constexpr bool TAPS25 = false;
+#include "patch4_kernel.h"
+}  // namespace one
+namespace two {
+constexpr int KS = 2;
+constexpr bool TAPS25 = false;
+#include "patch4_kernel.h"
+}  // namespace two
+namespace one25 {
+constexpr int KS = 1;
+constexpr bool TAPS25 = true;
+#include "patch4_kernel.h"
+}  // namespace one25
+namespace two25 {
+constexpr int KS = 2;
+constexpr bool TAPS25 = true;
+#include "patch4_kernel.h"
+}  // namespace two25
 
 // 3x3 over at most 32 KB channels: the whole reduction in one stage.  All of a workgroup's loads are in flight at once and one barrier
 // stands between them and the products, where the kernel above waits for a stage's latency per 32 channels.  LDS: [step][half of 32
@@ -509,6 +325,16 @@ bool p4_plan(const IgemmArgs& a, int cfg, bool one, P4Args* k, int* lds_bytes) {
     return *lds_bytes <= 160 * 1024;
 }
 
+// LDS of the form with two groups of waves, or 0 where one is better.  Where every workgroup has a CU to itself a layer is its chain of stages,
+// each as long as its loads and its way through LDS, and two groups halve it (us, graph replays, one group / two): 5x5 356 -> 24 at 76 x 108, stride
+// 2, batch 9, 23 stages: 40.8 / 29.5; 3x3 424 -> 220 at 12 x 10, batch 60, 14: 17.2 / 14.0; 72 -> 28 at 24 x 33, batch 8, three: 5.0 / 4.6.  104 drawn
+// layers with no more workgroups to an XCD than it has CUs: 0.70 to 0.98.  With one more the second form has two to a CU, which its LDS seldom
+// allows: 76 such layers 0.86 to 1.36, all but two behind.
+int p4_split_lds(const P4Args& k, int lds, int cu_count) {
+    const int tab = ((k.GS * k.T + 1) & ~1) * 4, both = std::max(2 * (lds - tab) + tab, 16 * 1024);  // (16 KiB: the sums that the groups exchange)
+    return k.nstages >= 2 && (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m <= cu_count / 8 && both <= 160 * 1024 ? both : 0;
+}
+
 template <int KB, int MT, int NT>
 int launch_one(hipStream_t st, const P4Args& k, int lds) {
     auto kern = patch4_one_kernel<KB, MT, NT>;
@@ -522,21 +348,33 @@ int launch_one(hipStream_t st, const P4Args& k, int lds) {
     return launch_kernel(kern, dim3((unsigned)grid), dim3(256), lds, st, k);
 }
 
-template <int MT, int NT>
-int launch_p4(hipStream_t st, const P4Args& k, int lds) {
-    // two groups of nine taps, and not one group of eighteen (3x6, 2x9, ...): the stage has as many entries, the filter rows
-    // and the patch of the two differ
-    auto kern = k.GS == 2 && k.T == 9 ? patch4_kernel<MT, NT, 9> : patch4_kernel<MT, NT, 0>;
+typedef void (*P4Kernel)(P4Args);
+template <P4Kernel kern>
+int launch_form(hipStream_t st, const P4Args& k, int threads, int lds) {
     static std::atomic<int> max_lds_set{0};
     if (max_lds_set.load(std::memory_order_relaxed) == 0) {
-        for (auto f : {patch4_kernel<MT, NT, 9>, patch4_kernel<MT, NT, 0>}) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            if (e != hipSuccess) return (int)e;
-        }
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return (int)e;
         max_lds_set.store(1, std::memory_order_relaxed);
     }
     const int64_t grid = (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
-    return launch_kernel(kern, dim3((unsigned)grid), dim3(256), lds, st, k);
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(threads), lds, st, k);
+}
+
+template <int MT, int NT>
+int launch_p4(hipStream_t st, const P4Args& k, int lds, int lds2 = 0) {
+    // two groups of nine taps, and not one group of eighteen (3x6, 2x9, ...): the stage has as many entries, the filter rows
+    // and the patch of the two differ
+    const bool nine = k.GS == 2 && k.T == 9, five = k.GS == 1 && k.T == 25;
+    if constexpr (MT * NT == 1) {
+        if (lds2)
+            return nine   ? launch_form<two::patch4_kernel<1, 1, 9>>(st, k, 512, lds2)
+                   : five ? launch_form<two25::patch4_kernel<1, 1, 0>>(st, k, 512, lds2)
+                          : launch_form<two::patch4_kernel<1, 1, 0>>(st, k, 512, lds2);
+    }
+    return nine   ? launch_form<one::patch4_kernel<MT, NT, 9>>(st, k, 256, lds)
+           : five ? launch_form<one25::patch4_kernel<MT, NT, 0>>(st, k, 256, lds)
+                  : launch_form<one::patch4_kernel<MT, NT, 0>>(st, k, 256, lds);
 }
 
 }  // namespace
@@ -581,7 +419,7 @@ int patch4_pick(const IgemmArgs& a, int pin, int pout) {
     return wgs(1) >= 300 ? 1 : 0;
 }
 
-int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg) {
+int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg, int cu_count) {
     P4Args k;
     int lds;
     const bool one = p4_plan(a, cfg, true, &k, &lds);
@@ -601,7 +439,7 @@ int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg) {
     if (one && k.GS == 2) return cfg == 0 ? launch_one<1, 1, 1>(st, k, lds) : cfg == 1 ? launch_one<1, 1, 2>(st, k, lds) : launch_one<1, 2, 2>(st, k, lds);
     if (one) return cfg == 0 ? launch_one<2, 1, 1>(st, k, lds) : cfg == 1 ? launch_one<2, 1, 2>(st, k, lds) : launch_one<2, 2, 2>(st, k, lds);
     switch (cfg) {
-        case 0: return launch_p4<1, 1>(st, k, lds);
+        case 0: return launch_p4<1, 1>(st, k, lds, p4_split_lds(k, lds, cu_count));
         case 1: return launch_p4<1, 2>(st, k, lds);
         default: return launch_p4<2, 2>(st, k, lds);
     }

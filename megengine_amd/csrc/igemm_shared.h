@@ -588,7 +588,7 @@ const char* patch4_cfg_name(int cfg);
 bool patch4_can_run(const IgemmArgs& a, int pin, int pout, int cfg);
 bool patch4_one_stage(const IgemmArgs& a, int pin, int pout);
 int patch4_pick(const IgemmArgs& a, int pin, int pout);  // its tile for this problem, -1 where another kernel is ahead
-int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg);
+int launch_patch4(hipStream_t st, const IgemmArgs& a, int cfg, int cu_count);
 
 // 3x3 over 32 or 64 channels per group, 32-packed, the whole reduction in one stage (conv_group32.hip, tiles "v2_patch_*")
 int grp32_num_cfgs();
