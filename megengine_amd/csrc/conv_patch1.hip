@@ -78,8 +78,9 @@ __device__ __forceinline__ P1Out p1_out(const P1Args& a, const P1Tile& o, int p,
     return {(o.n0 + (int)im) * a.dst_sn + px, (o.n0 + (int)im) * a.z_sn + px, in ? a.run ? a.OHW - at : a.OW - (o.ow0 + (int)ow) : 0};
 }
 
-template <int MT, int NT, int NL, bool HZ>
-__device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT], const uint32_t (&zq)[NT][MT][4], const P1Tile& o, int oc0,
+// QN: eights of channels of each block of 32 that are in acc (all four, or two)
+template <int MT, int NT, int QN, int NL, bool HZ>
+__device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT], const uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0,
                                             int wave, int l32, int lh) {
     const __amdgpu_buffer_rsrc_t rs_dst = make_rsrc(a.dst, a.dst_bytes), rs_z = make_rsrc(a.z, HZ ? a.z_bytes : 0);
     const int lane4 = l32 & 3, ch = 4 * lh + lane4;  // after the exchange a lane holds four columns of channel ch of every eight
@@ -91,7 +92,7 @@ __device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT]
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
+            for (int q = 0; q < QN; ++q) {
                 const int oc8 = oc0 + i * 32 + 8 * q, at = oc8 * a.OHW;  // wave-uniform
                 const bool ok = oc8 + ch < a.OC;
                 uint32_t zw = 0;
@@ -116,246 +117,14 @@ __device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT]
     }
 }
 
-template <int MT, int NT, int T>
-__global__ __launch_bounds__(256, 2) void patch1_kernel(P1Args a) {
-    constexpr int NPI = P1_NPI;
-    constexpr bool ZPRE = MT * NT <= 2;  // the residual is asked for ahead of the products (the largest tile has no registers for it)
-    constexpr int BM = MT * 32, GS = p1_gs(T), F = p1_f(T), E = GS * T, EP = (E + 1) & ~1, STEPS = EP / 2, BMP = p1_bmp(MT);
-    constexpr int TPG = 256 / GS;                          // threads per channel group of the patch
-    constexpr int QPR = 4 * GS;                            // channel quads of a filter row and stage
-    constexpr int FI = (BM * QPR + 255) / 256;             // filter items per thread and stage
-    constexpr int A_VECS = EP * BMP;
-    extern __shared__ __attribute__((aligned(16))) v4i lds[];
-    __shared__ __attribute__((aligned(16))) int sBias[BM];
-    // everything up to the first operands in one batch of scalar loads, and a word of each line that the epilogue reads
-    asm volatile("" ::"s"(a.src), "s"(a.flt), "s"(a.bias), "s"(a.dst), "s"(a.IC), "s"(a.IH), "s"(a.IW), "s"(a.IHW), "s"(a.OC), "s"(a.N),
-                 "s"(a.sh), "s"(a.sw), "s"(a.ph), "s"(a.pw), "s"(a.src_sn), "s"(a.kbytes), "s"(a.flt_bytes), "s"(a.has_bias), "s"(a.nstages),
-                 "s"(a.NI), "s"(a.TH), "s"(a.TW), "s"(a.tile_px), "s"(a.run), "s"(a.PWC), "s"(a.PX), "s"(a.PXQ), "s"(a.tiles_m));
-    asm volatile("" ::"s"(a.tiles_n), "s"(a.tiles_img), "s"(a.tiles_w), "s"(a.div_tiles_m.m), "s"(a.div_tiles_img.m), "s"(a.div_tiles_w.m),
-                 "s"(a.div_pqi.m), "s"(a.div_pqi.s2), "s"(a.div_pqw.m), "s"(a.div_pqw.s2), "s"(a.div_tile_px.m), "s"(a.div_tw.m), "s"(a.epi.s_b),
-                 "s"(a.epi.lin_lo));
-    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l32 = lane & 31, lh = lane >> 5;
-    const int stage_vecs = A_VECS + GS * a.PX;
-
-    // tile: contiguous pixel tiles per XCD (workgroup b runs on XCD b % 8), channel tiles of a pixel tile side by side
-    int tm, tn;
-    {
-        const int per = (a.tiles_n + 7) >> 3, x = blockIdx.x & 7, i = blockIdx.x >> 3;
-        const int r = (int)fdiv(i, a.div_tiles_m);
-        tm = i - r * a.tiles_m;
-        tn = x * per + r;
-        if (r >= per || tn >= a.tiles_n) return;
-    }
-    const int ig = (int)fdiv(tn, a.div_tiles_img), ti = tn - ig * a.tiles_img;
-    const bool is_run = a.run != 0;
-    const int at = is_run ? ti * a.run : ti, th = (int)fdiv(at, a.div_tiles_w), tw = at - th * a.tiles_w;  // (a run: row and column)
-    const int n0 = ig * a.NI, oc0 = tm * BM, oh0 = is_run ? th : th * a.TH, ow0 = is_run ? 0 : tw * a.TW;
-    const P1Tile o{n0, oh0, ow0, is_run ? tw : 0};
-    const int iw_lo = (ow0 * a.sw - a.pw) & ~3;  // the patch starts at a column that is a multiple of four: a quad that starts
-                                                 // inside a row starts at one of its columns
-
-    // Patch quads of this thread.  Waves of a group of TPG threads share a channel group, so a channel's plane is a scalar base.
-    const int g = GS == 1 ? 0 : wave / (TPG / 64), tg = t & (TPG - 1);
-    uint32_t p_sel[NPI][4];
-    int p_off[NPI], p_lds[NPI];
-    const int turn = (tg >> 1) & 3;
-#pragma unroll
-    for (int k = 0; k < NPI; ++k) {
-        const uint32_t pq = tg + k * TPG, im = fdiv(pq, a.div_pqi), r = pq - im * (uint32_t)(a.PXI >> 2);
-        const uint32_t pr = fdiv(r, a.div_pqw), pc = (r - pr * (uint32_t)(a.PWC >> 2)) * 4;
-        const int ih = oh0 * a.sh - a.ph + (int)pr, iw = iw_lo + (int)pc, n = n0 + (int)im;
-        const bool ok = ((int)pq < a.PXQ) & (n < a.N) & ((unsigned)ih < (unsigned)a.IH) & ((unsigned)iw < (unsigned)a.IW);
-        const int back = iw + 4 > a.IW ? iw + 4 - a.IW : 0;  // the row ends inside the quad: loaded `back` columns further left
-        p_off[k] = ok ? n * a.src_sn + ih * a.IW + iw - back : SENT;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int p = ((j + turn) & 3) + back;  // byte of the loaded dword that is this pixel
-            p_sel[k][j] = ok && p < 4 ? 0x00000400u | (uint32_t)(p | p << 8) : 0x0c0cu;
-            p_sel[k][j] |= 0x0c0c0000u;
-        }
-        p_lds[k] = (int)pq < a.PXQ ? A_VECS + g * a.PX + (int)pq * 4 : -1;
-    }
-    // filter items of this thread: four channels of a row
-    const int f_quad = t & (QPR - 1), f_row = t / QPR;
-    constexpr int ROWS_PER_PASS = 256 / QPR;
-    int f_off[FI];
-#pragma unroll
-    for (int k = 0; k < FI; ++k) {
-        const int row = f_row + k * ROWS_PER_PASS;
-        f_off[k] = row < BM && oc0 + row < a.OC ? (oc0 + row) * a.kbytes + f_quad * 4 * T : -1;
-    }
-
-    const __amdgpu_buffer_rsrc_t rs_src = make_rsrc(a.src, a.src_bytes), rs_flt = make_rsrc(a.flt, (uint32_t)a.flt_bytes);
-    const __amdgpu_buffer_rsrc_t rs_bias = make_rsrc(a.bias, a.has_bias ? a.OC * 4 : 0);
-    uint32_t xp[NPI][16], xf[FI][T];
-    const bool two = a.PXQ > TPG;  // a second quad per thread
-    auto fetch = [&](int st) __attribute__((always_inline)) {
-        const int c0 = (st * GS + g) * 16;
-#pragma unroll
-        for (int k = 0; k < FI; ++k) {
-            // (a quad past the last channel is not loaded; one whose bytes pass the end of the filter is loaded whole channels further
-            // left, and turned back in store)
-            const int at = f_off[k] + st * GS * 16 * T;
-            const bool in = (f_off[k] >= 0) & (st * GS * 16 + f_quad * 4 < a.IC);
-            const int v0 = in ? min(at, a.flt_bytes - 4 * T) : SENT;
-#pragma unroll
-            for (int v = 0; v + 4 <= T; v += 4) {
-                const v4i y = __builtin_amdgcn_raw_buffer_load_b128(rs_flt, v0 + 4 * v, 0, 0);
-                xf[k][v] = y[0]; xf[k][v + 1] = y[1]; xf[k][v + 2] = y[2]; xf[k][v + 3] = y[3];
-            }
-            if constexpr (T % 4 != 0) xf[k][T - 1] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_flt, v0 + 4 * (T - 1), 0, 0);
-        }
-        // (channels past the last one meet zero filter bytes; the scalar offset never leads out of the image)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            xp[0][i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_src, p_off[0], min(c0 + i, a.IC - 1) * a.IHW, 0);
-        if (two)
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                xp[NPI - 1][i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_src, p_off[NPI - 1], min(c0 + i, a.IC - 1) * a.IHW, 0);
-    };
-    auto store = [&](int st) __attribute__((always_inline)) {
-        v4i* s = lds + (st & 1) * stage_vecs;
-        uint32_t* sw = reinterpret_cast<uint32_t*>(s);
-#pragma unroll
-        for (int k = 0; k < FI; ++k) {
-            const int row = f_row + k * ROWS_PER_PASS, left = a.IC - (st * GS * 16 + f_quad * 4);  // channels from here on
-            // Channels that exist, and the quads at the filter's end, which may be those of its last three rows: loaded one to three
-            // channels further left.  One selector does both.  (Loading such a quad byte by byte, 4 T loads of one lane, held up the last
-            // channel tile: 5x5 59 -> 63 at 79 x 22, batch 4: 13.3 us.)
-            const int over = f_off[k] + st * GS * 16 * T + 4 * T - a.flt_bytes;
-            const int turned = over <= 0 ? 0 : over <= T ? 1 : over <= 2 * T ? 2 : 3;
-            const uint32_t there = left >= 4 ? 0xffffffffu : left > 0 ? (1u << (8 * left)) - 1 : 0u;
-            const uint32_t keep = ((0x03020100u + 0x01010101u * (uint32_t)turned) & there) | (0x0c0c0c0cu & ~there);
-            if (BM * QPR >= 256 || row < BM)
-#pragma unroll
-                for (int tap = 0; tap < T; ++tap)
-                    sw[(((f_quad >> 2) * T + tap) * BMP + row) * 4 + (f_quad & 3)] = __builtin_amdgcn_perm(0u, p1_tap<T>(xf[k], tap), keep);
-        }
-#pragma unroll
-        for (int k = 0; k < NPI; ++k) {
-            if (k == 1 && !two) break;
-            if (p_lds[k] >= 0)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    v4i turned;
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const uint32_t lo = __builtin_amdgcn_perm(xp[k][4 * c + 1], xp[k][4 * c], p_sel[k][j]);
-                        const uint32_t hi = __builtin_amdgcn_perm(xp[k][4 * c + 3], xp[k][4 * c + 2], p_sel[k][j]);
-                        turned[c] = (int)(lo | hi << 16);
-                    }
-                    s[p_lds[k] + ((j + turn) & 3)] = turned;
-                }
-        }
-    };
-    const int bias_v = __builtin_amdgcn_raw_buffer_load_b32(rs_bias, (oc0 + (t & (BM - 1))) * 4, 0, 0);
-    fetch(0);
-
-    // the filter entry that fills up an odd number stays zero, and the bias
-    if (EP != E)
-        for (int u = t; u < 2 * BM; u += 256) lds[(u / BM) * stage_vecs + E * BMP + u % BM] = v4i{0, 0, 0, 0};
-    if (t < BM) sBias[t] = bias_v;
-
-    // B operands: patch vector of each of this lane's pixels, and of each step's entry relative to it
-    int b_px[NT];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const uint32_t p = (wave * NT + j) * 32 + l32;
-        const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)a.tile_px + o.skip, oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
-        b_px[j] = (((int)im < a.NI) & ((int)oh < a.TH)) ? (int)(im * a.PXI + oh * a.sh * a.PWC) + ((int)ow + ow0) * a.sw - a.pw - iw_lo : 0;
-    }
-    int offs[STEPS];
-#pragma unroll
-    for (int k = 0; k < STEPS; ++k) {
-        const int e0 = 2 * k, e1 = 2 * k + 1 < E ? 2 * k + 1 : 0;  // (the filling entry multiplies any vector by zero)
-        const int o0 = (e0 / T) * a.PX + ((e0 % T) / F) * a.PWC + (e0 % T) % F, o1 = (e1 / T) * a.PX + ((e1 % T) / F) * a.PWC + (e1 % T) % F;
-        offs[k] = A_VECS + (lh ? o1 : o0);
-    }
-    store(0);
-    __builtin_amdgcn_s_waitcnt(P1_VMCNT0);  // (the compiler knows: a stage's products do not wait for the next stage's loads)
-    if (a.nstages > 1) fetch(1);
-    // the residual of whole groups of four columns (a launch without one: a descriptor of no bytes)
-    uint32_t zq[NT][MT][4];
-    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.epi.has_z ? a.z_bytes : 0);
-    if constexpr (ZPRE)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const P1Out w = p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), 4 * lh + (l32 & 3));
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int oc8 = oc0 + i * 32 + 8 * q;
-                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(
-                        rs_z, ((oc8 + 4 * lh + (l32 & 3) < a.OC) & (w.cols >= 4)) ? w.z0 : SENT, oc8 * a.OHW, 0);
-            }
-    }
-    __syncthreads();
-    v16i acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const v4i b = *reinterpret_cast<const v4i*>(sBias + i * 32 + 8 * q + 4 * lh);
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                acc[i][j][4 * q] = b[0]; acc[i][j][4 * q + 1] = b[1]; acc[i][j][4 * q + 2] = b[2]; acc[i][j][4 * q + 3] = b[3];
-            }
-        }
-    const int groups = (a.IC + 15) >> 4;
-    auto products = [&](int st) __attribute__((always_inline)) {
-        const v4i* s = lds + (st & 1) * stage_vecs;
-        const v4i* pa = s + lh * BMP + l32;
-        auto load = [&](int k, v4i (&fa)[MT], v4i (&fb)[NT]) __attribute__((always_inline)) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i) fa[i] = pa[k * 2 * BMP + i * 32];
-#pragma unroll
-            for (int j = 0; j < NT; ++j) fb[j] = s[offs[k] + b_px[j]];
-        };
-        constexpr int AHEAD = 2;  // steps whose operands are read ahead
-        v4i fa[AHEAD + 1][MT], fb[AHEAD + 1][NT];
-#pragma unroll
-        for (int k = 0; k < AHEAD && k < STEPS; ++k) load(k, fa[k], fb[k]);
-#pragma unroll
-        for (int k = 0; k < STEPS; ++k) {
-            // (an incomplete last stage: nothing of the groups past the last one; wave-uniform)
-            if (k > 0 && (2 * k) % T < 2 && st * GS + (2 * k) / T >= groups) break;
-            if (k + AHEAD < STEPS) load(k + AHEAD, fa[(k + AHEAD) % (AHEAD + 1)], fb[(k + AHEAD) % (AHEAD + 1)]);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[k % (AHEAD + 1)][i], fb[k % (AHEAD + 1)][j], acc[i][j], 0, 0, 0);
-        }
-    };
-    for (int st = 0;; ++st) {
-        products(st);
-        if (st + 1 >= a.nstages) break;
-        store(st + 1);
-        if (st + 2 < a.nstages) fetch(st + 2);
-        __syncthreads();
-    }
-
-#define MI355_P1(NL, HZ) p1_epilogue<MT, NT, NL, HZ>(a, acc, zq, o, oc0, wave, l32, lh)
-    if (a.epi.lin) {
-        MI355_P1(NL_LIN, false);
-    } else if (a.epi.has_z) {
-        switch (a.epi.nonline) {
-            case NL_RELU: MI355_P1(NL_RELU, true); break;
-            case NL_H_SWISH: MI355_P1(NL_H_SWISH, true); break;
-            default: MI355_P1(NL_IDENTITY, true); break;
-        }
-    } else {
-        switch (a.epi.nonline) {
-            case NL_RELU: MI355_P1(NL_RELU, false); break;
-            case NL_H_SWISH: MI355_P1(NL_H_SWISH, false); break;
-            default: MI355_P1(NL_IDENTITY, false); break;
-        }
-    }
-#undef MI355_P1
-}
+namespace one {
+constexpr int KS = 1;
+#include "patch1_kernel.h"
+}  // namespace one
+namespace two {
+constexpr int KS = 2;
+#include "patch1_kernel.h"
+}  // namespace two
 
 constexpr int kP1Tiles[][2] = {{1, 1}, {1, 2}, {2, 2}, {2, 1}};  // 32 x 128, 32 x 256, 64 x 256, 64 x 128
 
@@ -453,9 +222,9 @@ void p1_run(const ConvProblem& p, int tile, int cu_count, P1Args* k, int* lds_by
     *lds_bytes = lds;
 }
 
-template <int MT, int NT, int T>
-int launch_p1(hipStream_t st, const P1Args& k, int lds) {
-    auto kern = patch1_kernel<MT, NT, T>;
+typedef void (*P1Kernel)(P1Args);
+template <P1Kernel kern>
+int launch_p1(hipStream_t st, const P1Args& k, int threads, int lds) {
     static std::atomic<int> max_lds_set{0};
     if (max_lds_set.load(std::memory_order_relaxed) == 0) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024);
@@ -463,16 +232,28 @@ int launch_p1(hipStream_t st, const P1Args& k, int lds) {
         max_lds_set.store(1, std::memory_order_relaxed);
     }
     const int64_t grid = (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m * 8;
-    return launch_kernel(kern, dim3((unsigned)grid), dim3(256), lds, st, k);
+    return launch_kernel(kern, dim3((unsigned)grid), dim3(threads), lds, st, k);
+}
+
+// LDS of the form with two groups of waves, or 0 where one is better.  Where every workgroup has a CU to itself a layer is its chain of stages, and
+// two groups halve it (us, graph replays of one group / two): 5x5, 129 workgroups, 27.0 / 20.6; 3x3, 88 workgroups, eight stages, 13.6 / 11.0;
+// 1x1 230 -> 16 at 17 x 105, batch 14, four stages, 7.6 / 6.6.  Not two stages (68 layers: 0.987 on average, up to 1.034), nor more than one workgroup to a CU, where
+// registers and LDS keep the second one out: 1.04 to 1.4 times as long on 12 of 13 such layers.
+int p1_split_lds(const P1Args& k, int lds, int cu_count) {
+    const int both = std::max(2 * lds, 16 * 1024);  // (16 KiB: the sums that the groups exchange)
+    return k.nstages >= 3 && (int64_t)((k.tiles_n + 7) / 8) * k.tiles_m <= cu_count / 8 && both <= 150 * 1024 ? both : 0;
 }
 
 template <int T>
-int launch_p1_tile(hipStream_t st, const P1Args& k, int tile, int lds) {
+int launch_p1_tile(hipStream_t st, const P1Args& k, int tile, int lds, int cu_count) {
     switch (tile) {
-        case 0: return launch_p1<1, 1, T>(st, k, lds);
-        case 1: return launch_p1<1, 2, T>(st, k, lds);
-        case 2: return launch_p1<2, 2, T>(st, k, lds);
-        default: return launch_p1<2, 1, T>(st, k, lds);
+        case 0: {
+            const int lds2 = p1_split_lds(k, lds, cu_count);
+            return lds2 ? launch_p1<two::patch1_kernel<1, 1, T>>(st, k, 512, lds2) : launch_p1<one::patch1_kernel<1, 1, T>>(st, k, 256, lds);
+        }
+        case 1: return launch_p1<one::patch1_kernel<1, 2, T>>(st, k, 256, lds);
+        case 2: return launch_p1<one::patch1_kernel<2, 2, T>>(st, k, 256, lds);
+        default: return launch_p1<one::patch1_kernel<2, 1, T>>(st, k, 256, lds);
     }
 }
 
@@ -609,7 +390,7 @@ int launch_patch1(hipStream_t st, const ConvProblem& p, int tile, int cu_count, 
     k.div_pqi = make_fastdiv(k.PXI >> 2); k.div_pqw = make_fastdiv(k.PWC >> 2);
     k.epi = p.epi;
     const int T = (int)(d.fh * d.fw);
-    return T == 1 ? launch_p1_tile<1>(st, k, tile, lds) : T == 9 ? launch_p1_tile<9>(st, k, tile, lds) : launch_p1_tile<25>(st, k, tile, lds);
+    return T == 1 ? launch_p1_tile<1>(st, k, tile, lds, cu_count) : T == 9 ? launch_p1_tile<9>(st, k, tile, lds, cu_count) : launch_p1_tile<25>(st, k, tile, lds, cu_count);
 }
 
 }  // namespace mi355

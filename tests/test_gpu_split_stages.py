@@ -23,6 +23,11 @@ CASES = [
     ("NCHW4", 2, 64, 11, 13, 36, 5, 2, 1, 512),
     ("NCHW4", 1, 52, 14, 40, 24, (1, 25), (0, 12), 1, 512),   # 25 taps in a row
     ("NCHW4", 40, 20, 21, 22, 40, 5, 2, 1, 256),     # 25 taps, one group of waves
+    ("NCHW", 1, 75, 13, 11, 35, 3, 1, 1, 512),       # three stages, the last one with eleven channels
+    ("NCHW", 1, 130, 16, 17, 20, 1, 0, 1, 512),      # three stages of 64
+    ("NCHW", 1, 33, 12, 19, 70, 5, 2, 2, 512),
+    ("NCHW", 1, 150, 15, 14, 20, 3, 1, 2, 512),
+    ("NCHW", 3, 40, 9, 7, 33, 3, 1, 1, 256),         # two stages
 ]
 
 
