@@ -78,6 +78,24 @@ __device__ __forceinline__ P1Out p1_out(const P1Args& a, const P1Tile& o, int p,
     return {(o.n0 + (int)im) * a.dst_sn + px, (o.n0 + (int)im) * a.z_sn + px, in ? a.run ? a.OHW - at : a.OW - (o.ow0 + (int)ow) : 0};
 }
 
+// the residual of whole groups of four columns: that of a wave's outputs, in flight at once
+template <int MT, int NT, int QN>
+__device__ __forceinline__ void p1_residual(const P1Args& a, uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0, int wave, int l32, int lh) {
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.z_bytes);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const P1Out w = p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), 4 * lh + (l32 & 3));
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < QN; ++q) {
+                const int oc8 = oc0 + i * 32 + 8 * q;
+                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(
+                        rs_z, ((oc8 + 4 * lh + (l32 & 3) < a.OC) & (w.cols >= 4)) ? w.z0 : SENT, oc8 * a.OHW, 0);
+            }
+    }
+}
+
 // QN: eights of channels of each block of 32 that are in acc (all four, or two)
 template <int MT, int NT, int QN, int NL, bool HZ>
 __device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT], const uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0,
@@ -97,7 +115,7 @@ __device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT]
                 const bool ok = oc8 + ch < a.OC;
                 uint32_t zw = 0;
                 if (HZ) {
-                    zw = MT * NT <= 2 ? zq[j][i][q] : (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, (ok & (cols >= 4)) ? z0 : SENT, at, 0);
+                    zw = zq[j][i][q];
                     if (split) {
 #pragma unroll
                         for (int k = 0; k < 3; ++k)

@@ -244,6 +244,10 @@ __global__ __launch_bounds__(256 * KS, 2) void patch1_kernel(P1Args a) {
         for (int i = 0; i < 8; ++i) c[i] = (kg ? c[8 + i] : c[i]) + y[(i >> 2) * 256][i & 3];
     }
 
+    // (the largest tile has registers for it once the products are done: all of it at once, where each dword used to be waited for behind the
+    // store before it; 3x3 7 -> 210 at 63 x 84, batch 42: 75.4 -> 59.1 us)
+    if constexpr (!ZPRE)
+        if (a.epi.has_z) p1_residual<MT, NT, QN>(a, zq, o, oc0, wave, l32, lh);
 #define MI355_P1(NL, HZ) p1_epilogue<MT, NT, QN, NL, HZ>(a, acc, zq, o, oc0 + kg * 16, wave, l32, lh)
     if (a.epi.lin) {
         MI355_P1(NL_LIN, false);
