@@ -246,7 +246,8 @@ __global__ __launch_bounds__(256) void nchw_to_packed_small_kernel(const int8_t*
 // apart); global accesses on both sides are 16-byte vectors over contiguous runs, unaligned ones on the plain side when
 // the image has an odd size.  C any: missing channels are zero on the way in and dropped on the way out.
 constexpr int RL_TP = 512;           // pixels per tile
-constexpr int RL_ROW = RL_TP + 8;    // padded channel row (bytes): 16 rows = 8320 = 32*256 + 128
+constexpr int RL_WAVE = 128;         // of a tile that is one wave (see RlWave)
+constexpr int rl_row(int tp) { return tp + 8; }  // padded channel row (bytes): 16 rows = 8320 = 32*256 + 128, or 2176 = 8*256 + 128
 
 // Where 16-byte unit u of a wave's 128 pixels (two units each) lies in LDS: lanes that write units 8 apart and lanes that read consecutive ones
 // meet different banks.
@@ -262,19 +263,20 @@ static bool whole_lines(uint64_t workgroups, uint64_t tiles_of_plane, uint32_t H
 }
 
 // LINES: stores of whole lines, see below
-template <bool LINES>
-__global__ __launch_bounds__(256) void nchw_to_nchw32_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
-                                                             uint32_t C, uint32_t CB, uint32_t HW) {
+template <bool LINES, int TP>
+__device__ __forceinline__ void nchw_to_nchw32(const int8_t* __restrict__ src, int8_t* __restrict__ dst, uint32_t C, uint32_t CB, uint32_t HW) {
+    constexpr int RL_ROW = rl_row(TP);
+    constexpr uint32_t VECS = TP / 16;  // of a row; a pass of the workgroup (TP / 2 threads) takes eight rows
     __shared__ __attribute__((aligned(16))) int8_t sm[32 * RL_ROW];
     const uint32_t t = threadIdx.x;
-    const uint32_t ptiles = (HW + RL_TP - 1) / RL_TP;
+    const uint32_t ptiles = (HW + TP - 1) / TP;
     const uint32_t cb = blockIdx.x / ptiles, pt = blockIdx.x % ptiles;
-    const uint32_t p0 = pt * RL_TP;
+    const uint32_t p0 = pt * TP;
     const int64_t n = blockIdx.y;
-    // load: 32 rows x 32 vectors; thread t -> vector (t % 32), rows t/32 + 8*i
+    // load: 32 rows of VECS vectors; thread t -> vector t % VECS, rows t / VECS + 8 i
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        uint32_t row = t / 32 + 8 * i, v = t % 32;
+        uint32_t row = t / VECS + 8 * i, v = t % VECS;
         uint32_t px = p0 + v * 16;
         u32x4 x = {0, 0, 0, 0};
         if (px < HW && cb * 32 + row < C) x = load16_tail(src + (n * C + cb * 32 + row) * HW + px, HW - px);
@@ -319,13 +321,15 @@ __global__ __launch_bounds__(256) void nchw_to_nchw32_kernel(const int8_t* __res
         if (px + i * 32 < HW) *reinterpret_cast<u32x4*>(d + i * 1024) = mine[rl_slot(i * 64 + lane)];
 }
 
-__global__ __launch_bounds__(256) void nchw32_to_nchw_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst,
-                                                             uint32_t C, uint32_t CB, uint32_t HW) {
+template <int TP>
+__device__ __forceinline__ void nchw32_to_nchw(const int8_t* __restrict__ src, int8_t* __restrict__ dst, uint32_t C, uint32_t CB, uint32_t HW) {
+    constexpr int RL_ROW = rl_row(TP);
+    constexpr uint32_t VECS = TP / 16;
     __shared__ __attribute__((aligned(16))) int8_t sm[32 * RL_ROW];
     const uint32_t t = threadIdx.x;
-    const uint32_t ptiles = (HW + RL_TP - 1) / RL_TP;
+    const uint32_t ptiles = (HW + TP - 1) / TP;
     const uint32_t cb = blockIdx.x / ptiles, pt = blockIdx.x % ptiles;
-    const uint32_t p0 = pt * RL_TP;
+    const uint32_t p0 = pt * TP;
     const int64_t n = blockIdx.y;
     const uint32_t pq = t >> 1, half = t & 1;
     const uint32_t px = p0 + pq * 4;
@@ -349,13 +353,39 @@ __global__ __launch_bounds__(256) void nchw32_to_nchw_kernel(const int8_t* __res
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        uint32_t row = t / 32 + 8 * i, v = t % 32;
+        uint32_t row = t / VECS + 8 * i, v = t % VECS;
         uint32_t p = p0 + v * 16;
         if (p < HW && cb * 32 + row < C) {
             u32x4 x = *reinterpret_cast<const u32x4*>(sm + row * RL_ROW + v * 16);
             store16_tail(dst + (n * C + cb * 32 + row) * HW + p, x, HW - p);
         }
     }
+}
+
+template <bool LINES>
+__global__ __launch_bounds__(256) void nchw_to_nchw32_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst, uint32_t C, uint32_t CB,
+                                                             uint32_t HW) {
+    nchw_to_nchw32<LINES, RL_TP>(src, dst, C, CB, HW);
+}
+__global__ __launch_bounds__(256) void nchw32_to_nchw_kernel(const int8_t* __restrict__ src, int8_t* __restrict__ dst, uint32_t C, uint32_t CB,
+                                                             uint32_t HW) {
+    nchw32_to_nchw<RL_TP>(src, dst, C, CB, HW);
+}
+
+// The form with tiles of one wave, four times as many: where workgroups of the other are few, into NCHW32 up to three for four CUs (130 drawn
+// conversions 0.91 of the time on average, beyond, to 384, 0.97 .. 1.04; 128 x 54 x 33 at batch 2 3.96 -> 3.47 us), back up to one for two (93 drawn ones
+// 0.94, beyond 0.99 .. 1.05; 128 x 27 x 22 at batch 2 3.05 -> 2.88).  From 400 on it loses to shorter runs of a plane: 1.02 .. 1.4.
+struct RlWave {
+    const int8_t* src;
+    int8_t* dst;
+    uint32_t C, CB, HW;
+};
+template <bool LINES>
+__global__ __launch_bounds__(64) void nchw_to_nchw32_kernel(RlWave a) {
+    nchw_to_nchw32<LINES, RL_WAVE>(a.src, a.dst, a.C, a.CB, a.HW);
+}
+__global__ __launch_bounds__(64) void nchw32_to_nchw_kernel(RlWave a) {
+    nchw32_to_nchw<RL_WAVE>(a.src, a.dst, a.C, a.CB, a.HW);
 }
 
 }  // namespace
@@ -395,9 +425,12 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
                 }
                 // planes of a quarter of the LDS tile and more: below, most of a tile's threads would find no pixel
                 if (oshape[4] == 32 && HW >= RL_TP / 4 && numbered((uint64_t)CB * ptiles * 256)) {
-                    if (whole_lines((uint64_t)N * CB * ptiles, ptiles, HW, cu_count))
-                        return launch_kernel(nchw_to_nchw32_kernel<true>, dim3(CB * ptiles, N), dim3(256), 0, st, s8, d8, C, CB, HW);
-                    return launch_kernel(nchw_to_nchw32_kernel<false>, dim3(CB * ptiles, N), dim3(256), 0, st, s8, d8, C, CB, HW);
+                    typedef void (*Tile)(const int8_t*, int8_t*, uint32_t, uint32_t, uint32_t);
+                    if (4ull * N * CB * ptiles <= 3ull * cu_count)
+                        return launch_kernel((void (*)(RlWave))nchw_to_nchw32_kernel<false>, dim3(CB * ((HW + RL_WAVE - 1) / RL_WAVE), N), dim3(64), 0, st,
+                                             RlWave{s8, d8, C, CB, HW});
+                    const Tile tile = whole_lines((uint64_t)N * CB * ptiles, ptiles, HW, cu_count) ? (Tile)nchw_to_nchw32_kernel<true> : (Tile)nchw_to_nchw32_kernel<false>;
+                    return launch_kernel(tile, dim3(CB * ptiles, N), dim3(256), 0, st, s8, d8, C, CB, HW);
                 }
                 if (!numbered((uint64_t)total / 4)) break;
                 const SmallPlanes g = make_small_planes(N, C, HW, oshape[4]);
@@ -417,8 +450,11 @@ int launch_relayout(hipStream_t st, const mi355_relayout_desc& d, const uint32_t
                 break;
             case MI355_RL_NCHW32_NCHW:
                 if (!numbered((uint64_t)d.shape[1] * ptiles * 256)) break;
-                return launch_kernel(nchw32_to_nchw_kernel, dim3(d.shape[1] * ptiles, N), dim3(256), 0, st, s8, d8, oshape[1],
-                                     d.shape[1], HW);
+                if (2ull * N * d.shape[1] * ptiles <= (uint64_t)cu_count)
+                    return launch_kernel((void (*)(RlWave))nchw32_to_nchw_kernel, dim3(d.shape[1] * ((HW + RL_WAVE - 1) / RL_WAVE), N), dim3(64), 0, st,
+                                         RlWave{s8, d8, oshape[1], d.shape[1], HW});
+                return launch_kernel((void (*)(const int8_t*, int8_t*, uint32_t, uint32_t, uint32_t))nchw32_to_nchw_kernel, dim3(d.shape[1] * ptiles, N),
+                                     dim3(256), 0, st, s8, d8, oshape[1], d.shape[1], HW);
             case MI355_RL_NCHW4_NCHW32:
             case MI355_RL_NCHW32_NCHW4: {
                 if (!numbered((uint64_t)total / 16)) break;
