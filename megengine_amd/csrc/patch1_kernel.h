@@ -165,20 +165,19 @@ __global__ __launch_bounds__(256 * KS, 2) void patch1_kernel(P1Args a) {
     store(kg, 0);
     __builtin_amdgcn_s_waitcnt(P1_VMCNT0);  // (the compiler knows: a stage's products do not wait for the next stage's loads)
     if (kg + KS < a.nstages) fetch(kg + KS);
-    // the residual of whole groups of four columns (a launch without one: a descriptor of no bytes)
+    // the residual (a launch without one: a descriptor of no bytes)
     uint32_t zq[NT][MT][QN];
     const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.epi.has_z ? a.z_bytes : 0);
     if constexpr (ZPRE)
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const P1Out w = p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), 4 * lh + (l32 & 3));
+        const P1Residual z = p1_residual_at(a, p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), 4 * lh + (l32 & 3)));
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int q = 0; q < QN; ++q) {
                 const int oc8 = oc0 + kg * 16 + i * 32 + 8 * q;
-                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(
-                        rs_z, ((oc8 + 4 * lh + (l32 & 3) < a.OC) & (w.cols >= 4)) ? w.z0 : SENT, oc8 * a.OHW, 0);
+                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, z.off, oc8 < a.OC ? oc8 * a.OHW : 0, 0);
             }
     }
     __syncthreads();
@@ -246,8 +245,11 @@ __global__ __launch_bounds__(256 * KS, 2) void patch1_kernel(P1Args a) {
 
     // (the largest tile has registers for it once the products are done: all of it at once, where each dword used to be waited for behind the
     // store before it; 3x3 7 -> 210 at 63 x 84, batch 42: 75.4 -> 59.1 us)
-    if constexpr (!ZPRE)
-        if (a.epi.has_z) p1_residual<MT, NT, QN>(a, zq, o, oc0, wave, l32, lh);
+    if constexpr (ZPRE) {
+        if (a.epi.has_z && a.OHW < 4) p1_residual_bytes<MT, NT, QN>(a, zq, o, oc0 + kg * 16, wave, l32, lh);
+    } else if (a.epi.has_z) {
+        p1_residual<MT, NT, QN>(a, zq, o, oc0, wave, l32, lh);
+    }
 #define MI355_P1(NL, HZ) p1_epilogue<MT, NT, QN, NL, HZ>(a, acc, zq, o, oc0 + kg * 16, wave, l32, lh)
     if (a.epi.lin) {
         MI355_P1(NL_LIN, false);
