@@ -4,11 +4,18 @@
 // 16 bytes in (+ 4), 4 bytes out per thread step; bound by HBM (5-6 bytes per element) and by the ~10 VALU operations
 // per element of the bit-exact requantisation.
 #include "common.h"
+#include "igemm_shared.h"
 
 namespace mi355 {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+
+template <int NL, bool HZ>
+__device__ __forceinline__ uint32_t requant4_form(v4i a, uint32_t zw, const EpiParams& e) {
+    if constexpr (NL == NL_ANY) return requant4(a[0], a[1], a[2], a[3], zw, e);
+    else return requant4_fast<NL, HZ>(a[0], a[1], a[2], a[3], zw, e);
+}
 
 // These two take the number of workgroups from gridDim and not, as the conversions below, as an argument.  That costs a single short call
 // 0.1 us (4096 values: 3.43 us as an argument, 3.58 so) and gains where the device is behind: the chain of int32 convolution, requantisation,
@@ -30,22 +37,69 @@ __global__ __launch_bounds__(256) void requant_kernel(const int32_t* __restrict_
     }
 }
 
-// QuantizedS8 first operand: 16 elements per thread step (16 + 16 bytes in, 16 out; 2-3 bytes per element)
-__global__ __launch_bounds__(256) void requant8_kernel(const int8_t* __restrict__ src, const int8_t* __restrict__ z,
-                                                       int8_t* __restrict__ dst, uint64_t blocks16, uint64_t count, EpiParams e) {
+// Four quads of a thread in flight and one form of the requantisation for the loop, where every workgroup is resident and has one step
+// (requant_wide).  Bound by bytes and the latency of a wave's first loads: 6.4 million values with a residual, 39 MB, 6.00 -> 5.33 us.
+constexpr int RQ_U = 4;
+template <int NL, bool HZ>
+__device__ __forceinline__ void requant_wide_run(const int32_t* __restrict__ src, const int8_t* __restrict__ z, int8_t* __restrict__ dst,
+                                                 uint64_t quads, const EpiParams& e) {
+    const XcdRun<uint64_t> run = xcd_run<uint64_t, 256 * RQ_U>(quads, gridDim.x);
+    for (uint64_t i = run.at; i < run.end; i += run.step) {
+        if (i + 256 * (RQ_U - 1) < run.end) {
+            v4i a[RQ_U];
+            uint32_t zw[RQ_U];
+#pragma unroll
+            for (int u = 0; u < RQ_U; ++u) {
+                a[u] = reinterpret_cast<const v4i*>(src)[i + 256 * u];
+                zw[u] = HZ ? reinterpret_cast<const uint32_t*>(z)[i + 256 * u] : 0u;
+            }
+#pragma unroll
+            for (int u = 0; u < RQ_U; ++u) reinterpret_cast<uint32_t*>(dst)[i + 256 * u] = requant4_form<NL, HZ>(a[u], zw[u], e);
+        } else {
+            for (uint64_t k = i; k < run.end; k += 256)
+                reinterpret_cast<uint32_t*>(dst)[k] =
+                        requant4_form<NL, HZ>(reinterpret_cast<const v4i*>(src)[k], HZ ? reinterpret_cast<const uint32_t*>(z)[k] : 0u, e);
+        }
+    }
+}
+__global__ __launch_bounds__(256) void requant_wide_kernel(const int32_t* __restrict__ src, const int8_t* __restrict__ z, int8_t* __restrict__ dst,
+                                                           uint64_t quads, uint64_t count, EpiParams e) {
+    if (e.has_z)
+        with_requant_form<true>(e, [&](auto nl) { requant_wide_run<decltype(nl)::value, true>(src, z, dst, quads, e); });
+    else
+        with_requant_form<false>(e, [&](auto nl) { requant_wide_run<decltype(nl)::value, false>(src, z, dst, quads, e); });
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        for (uint64_t j = quads * 4; j < count; ++j)
+            dst[j] = (int8_t)requant_s8_exact(src[j], e.has_z != 0, e.has_z ? (int)z[j] : 0, e);
+    }
+}
+
+// QuantizedS8 first operand: 16 elements per thread step (16 + 16 bytes in, 16 out; 2-3 bytes per element), in a loop of its own for every
+// form: the form chosen for each dword, four times a step, took the vector instructions of four apart.  42 registers, still eight
+// waves to a SIMD; of 36 drawn sizes up to 46 million values 0.91 of the time (0.85 to 0.99).
+template <int NL, bool HZ>
+__device__ __forceinline__ void requant8_run(const int8_t* __restrict__ src, const int8_t* __restrict__ z, int8_t* __restrict__ dst, uint64_t blocks16,
+                                             const EpiParams& e) {
     const XcdRun<uint64_t> run = xcd_run<uint64_t>(blocks16, gridDim.x);
     for (uint64_t i = run.at; i < run.end; i += run.step) {
         const v4i a = reinterpret_cast<const v4i*>(src)[i];
         v4i zv = {0, 0, 0, 0};
-        if (e.has_z) zv = reinterpret_cast<const v4i*>(z)[i];
+        if (HZ) zv = reinterpret_cast<const v4i*>(z)[i];
         v4i o;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int w = a[q];
-            o[q] = (int)requant4((w << 24) >> 24, (w << 16) >> 24, (w << 8) >> 24, w >> 24, (uint32_t)zv[q], e);
+            o[q] = (int)requant4_form<NL, HZ>(v4i{(w << 24) >> 24, (w << 16) >> 24, (w << 8) >> 24, w >> 24}, (uint32_t)zv[q], e);
         }
         reinterpret_cast<v4i*>(dst)[i] = o;
     }
+}
+__global__ __launch_bounds__(256) void requant8_kernel(const int8_t* __restrict__ src, const int8_t* __restrict__ z,
+                                                       int8_t* __restrict__ dst, uint64_t blocks16, uint64_t count, EpiParams e) {
+    if (e.has_z)
+        with_requant_form<true>(e, [&](auto nl) { requant8_run<decltype(nl)::value, true>(src, z, dst, blocks16, e); });
+    else
+        with_requant_form<false>(e, [&](auto nl) { requant8_run<decltype(nl)::value, false>(src, z, dst, blocks16, e); });
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         for (uint64_t j = blocks16 * 16; j < count; ++j)
             dst[j] = (int8_t)requant_s8_exact((int)src[j], e.has_z != 0, e.has_z ? (int)z[j] : 0, e);
@@ -92,6 +146,11 @@ __global__ __launch_bounds__(256) void cvt_s8_f32_kernel(const int8_t* __restric
         for (uint64_t j = quads * 4; j < count; ++j) dst[j] = (float)src[j] * scale;
 }
 
+// tiles of 4096 values: at least two to a CU, and all of them resident (eight to a CU): 0.89 to 0.99 of requant_kernel's time there, 0.94 on average.
+// With fewer the loads of a CU are too few either way and quads of their own start sooner (1.1 million values, residual: 2.9 / 3.2 us); with
+// more the tiles run in uneven rounds (8.7 million: 9.9 / 10.4; 12.3 million: 10.7 / 11.3), and from 20 million on both are bound by bytes.
+bool requant_wide(uint64_t tiles, int cu_count) { return tiles >= 2 * (uint64_t)cu_count && tiles <= 8 * (uint64_t)cu_count; }
+
 unsigned stream_blocks(uint64_t steps, int cu_count) {
     if (cu_count <= 0) cu_count = 256;
     uint64_t blocks = (steps + 255) / 256;
@@ -132,6 +191,9 @@ int launch_requant(hipStream_t st, const EpiParams& e, const int32_t* src, const
     if (count == 0) return 0;
     const uint64_t quads = count / 4;
     if (cu_count <= 0) cu_count = 256;
+    const uint64_t tiles = (quads + 256 * RQ_U - 1) / (256 * RQ_U);
+    if (requant_wide(tiles, cu_count))
+        return launch_kernel(requant_wide_kernel, dim3((unsigned)xcd_grid(tiles)), dim3(256), 0, st, src, z, dst, quads, count, e);
     uint64_t blocks = (quads + 255) / 256;
     const uint64_t cap = (uint64_t)cu_count * 16;
     if (blocks > cap) blocks = cap;
