@@ -65,13 +65,19 @@ __device__ __forceinline__ uint32_t p1_tap(const uint32_t (&x)[T], int tap) {
 struct P1Tile {
     int n0, oh0, ow0, skip;
 };
+__host__ __device__ __forceinline__ P1Tile p1_tile_at(const P1Args& a, int tn) {
+    const int ig = (int)fdiv(tn, a.div_tiles_img), ti = tn - ig * a.tiles_img;
+    const bool is_run = a.run != 0;
+    const int at = is_run ? ti * a.run : ti, th = (int)fdiv(at, a.div_tiles_w), tw = at - th * a.tiles_w;  // (a run: row and column)
+    return {ig * a.NI, is_run ? th : th * a.TH, is_run ? 0 : tw * a.TW, is_run ? tw : 0};
+}
 
 // where four neighbouring lanes put (and find the residual of) their four columns: offset of channel ch = 4 lh + l32 % 4 of the
 // first eight channels, and the columns from there to the end of the row, or of the image for a run (0: nothing)
 struct P1Out {
     int d0, z0, cols;
 };
-__device__ __forceinline__ P1Out p1_out(const P1Args& a, const P1Tile& o, int p, int ch) {
+__host__ __device__ __forceinline__ P1Out p1_out(const P1Args& a, const P1Tile& o, int p, int ch) {
     const uint32_t im = fdiv(p, a.div_tile_px), r = p - im * (uint32_t)a.tile_px + o.skip, oh = fdiv(r, a.div_tw), ow = r - oh * a.TW;
     const bool in = ((int)im < a.NI) & (o.n0 + (int)im < a.N) & (o.oh0 + (int)oh < a.OH);
     const int at = (o.oh0 + (int)oh) * a.OW + o.ow0 + (int)ow, px = at + ch * a.OHW;
@@ -85,45 +91,58 @@ __device__ __forceinline__ P1Out p1_out(const P1Args& a, const P1Tile& o, int p,
 struct P1Residual {
     int off, turn;
 };
-__device__ __forceinline__ P1Residual p1_residual_at(const P1Args& a, const P1Out& w) {
+__host__ __device__ __forceinline__ P1Residual p1_residual_at(const P1Args& a, const P1Out& w) {
     const int at = w.cols >= 4 ? w.z0 : max(w.z0 + w.cols - 4, 0);
     const bool in = (w.cols > 0) & (a.OHW >= 4);
     return {in ? at : SENT, in ? (w.z0 - at) * 8 : 0};
 }
+// The two offsets of an access to channel oc8 + ch at offset `at` of the first eight channels, by the rule at SENT: a lane without a
+// channel passes SENT, and a scalar offset leads to a channel that exists.
+struct P1Access {
+    int lane, scalar;
+};
+__host__ __device__ __forceinline__ P1Access p1_access(const P1Args& a, int at, int oc8, int ch) {
+    int left = a.OC - oc8;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm("" : "+s"(left));  // (or the masks of a whole tile are made at once and kept, and scalar registers spill)
+#endif
+    return {ch < left ? at : SENT, left > 0 ? oc8 * a.OHW : 0};
+}
 template <int MT, int NT, int QN>
 __device__ __forceinline__ void p1_residual_bytes(const P1Args& a, uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0, int wave, int l32, int lh) {
     const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.z_bytes);
+    const int ch = 4 * lh + (l32 & 3);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const P1Out w = p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), 4 * lh + (l32 & 3));
+        const P1Out w = p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), ch);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int q = 0; q < QN; ++q) {
-                const int oc8 = oc0 + i * 32 + 8 * q;
-                const int at = oc8 < a.OC ? oc8 * a.OHW : 0;
                 zq[j][i][q] = 0;
 #pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    zq[j][i][q] |= (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rs_z, k < w.cols ? w.z0 + k : SENT, at, 0) << (8 * k);
+                for (int k = 0; k < 3; ++k) {
+                    const P1Access at = p1_access(a, k < w.cols ? w.z0 + k : SENT, oc0 + i * 32 + 8 * q, ch);
+                    zq[j][i][q] |= (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rs_z, at.lane, at.scalar, 0) << (8 * k);
+                }
             }
     }
 }
 
-// the residual of a wave's outputs, in flight at once (channels past the last one load what nothing uses; their lane masks, kept until the stores,
-// had 110 scalar registers of the largest tile spilled; the scalar offset never leads out of the tensor)
+// the residual of a wave's outputs, in flight at once (a launch without one: a descriptor of no bytes)
 template <int MT, int NT, int QN>
 __device__ __forceinline__ void p1_residual(const P1Args& a, uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0, int wave, int l32, int lh) {
-    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.z_bytes);
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.epi.has_z ? a.z_bytes : 0);
+    const int ch = 4 * lh + (l32 & 3);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const P1Residual z = p1_residual_at(a, p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), 4 * lh + (l32 & 3)));
+        const P1Residual z = p1_residual_at(a, p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), ch));
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int q = 0; q < QN; ++q) {
-                const int oc8 = oc0 + i * 32 + 8 * q;
-                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, z.off, oc8 < a.OC ? oc8 * a.OHW : 0, 0);
+                const P1Access at = p1_access(a, z.off, oc0 + i * 32 + 8 * q, ch);
+                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, at.lane, at.scalar, 0);
             }
     }
 }
@@ -145,10 +164,7 @@ __device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT]
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int q = 0; q < QN; ++q) {
-                const int oc8 = oc0 + i * 32 + 8 * q, at = oc8 * a.OHW;  // wave-uniform
-                int left = a.OC - oc8;
-                asm("" : "+s"(left));  // (or the masks of all sixteen are made ahead of the forms, and scalar registers spill)
-                const bool ok = ch < left;
+                const int oc8 = oc0 + i * 32 + 8 * q;  // wave-uniform
                 uint32_t zw = 0;
                 if (HZ) {
                     zw = zq[j][i][q] >> turn;
@@ -156,10 +172,12 @@ __device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT]
                 }
                 const v16i& c = acc[i][j];
                 const uint32_t y = quad_transpose(requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], zw, a.epi), lane4);
-                __builtin_amdgcn_raw_buffer_store_b32((int)y, rs_dst, ok ? four : SENT, at, 0);
+                const P1Access to = p1_access(a, four, oc8, ch);
+                __builtin_amdgcn_raw_buffer_store_b32((int)y, rs_dst, to.lane, to.scalar, 0);
                 if (split) {
-                    __builtin_amdgcn_raw_buffer_store_b16((uint16_t)y, rs_dst, ok ? two : SENT, at, 0);
-                    __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(cols == 3 ? y >> 16 : y), rs_dst, ok ? one : SENT, at, 0);
+                    const P1Access to2 = p1_access(a, two, oc8, ch), to1 = p1_access(a, one, oc8, ch);
+                    __builtin_amdgcn_raw_buffer_store_b16((uint16_t)y, rs_dst, to2.lane, to2.scalar, 0);
+                    __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(cols == 3 ? y >> 16 : y), rs_dst, to1.lane, to1.scalar, 0);
                 }
             }
     }

@@ -102,7 +102,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint3
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
 
-constexpr int SENT = (int)0x80000000;  // byte offset that is out of range for every buffer (< 2 GiB)
+// Byte offset that is out of range for every buffer (< 2 GiB).  It belongs into the lane's offset: LLVM declares the scalar offset of the buffer
+// builtins as left out of the range check, the instruction set manuals take it off the descriptor's size, and code here relies on neither.  So
+// a lane passes SENT wherever its two offsets together lead out of the tensor, what becomes of a loaded value notwithstanding.
+// (tests/host/reach.cpp walks such offsets.)
+constexpr int SENT = (int)0x80000000;
 
 // both dwords through one choice of the requantisation form; the results replace the residual words
 __device__ __forceinline__ void requant8(v4i x, v4i y, uint32_t (&w)[2], const EpiParams& e) {

@@ -36,11 +36,8 @@ __global__ __launch_bounds__(256 * KS, 2) void patch1_kernel(P1Args a) {
         tn = x * per + r;
         if (r >= per || tn >= a.tiles_n) return;
     }
-    const int ig = (int)fdiv(tn, a.div_tiles_img), ti = tn - ig * a.tiles_img;
-    const bool is_run = a.run != 0;
-    const int at = is_run ? ti * a.run : ti, th = (int)fdiv(at, a.div_tiles_w), tw = at - th * a.tiles_w;  // (a run: row and column)
-    const int n0 = ig * a.NI, oc0 = tm * BM, oh0 = is_run ? th : th * a.TH, ow0 = is_run ? 0 : tw * a.TW;
-    const P1Tile o{n0, oh0, ow0, is_run ? tw : 0};
+    const P1Tile o = p1_tile_at(a, tn);
+    const int n0 = o.n0, oc0 = tm * BM, oh0 = o.oh0, ow0 = o.ow0;
     const int iw_lo = (ow0 * a.sw - a.pw) & ~3;  // the patch starts at a column that is a multiple of four: a quad that starts
                                                  // inside a row starts at one of its columns
 
@@ -165,21 +162,8 @@ __global__ __launch_bounds__(256 * KS, 2) void patch1_kernel(P1Args a) {
     store(kg, 0);
     __builtin_amdgcn_s_waitcnt(P1_VMCNT0);  // (the compiler knows: a stage's products do not wait for the next stage's loads)
     if (kg + KS < a.nstages) fetch(kg + KS);
-    // the residual (a launch without one: a descriptor of no bytes)
     uint32_t zq[NT][MT][QN];
-    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.epi.has_z ? a.z_bytes : 0);
-    if constexpr (ZPRE)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const P1Residual z = p1_residual_at(a, p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), 4 * lh + (l32 & 3)));
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int q = 0; q < QN; ++q) {
-                const int oc8 = oc0 + kg * 16 + i * 32 + 8 * q;
-                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, z.off, oc8 < a.OC ? oc8 * a.OHW : 0, 0);
-            }
-    }
+    if constexpr (ZPRE) p1_residual<MT, NT, QN>(a, zq, o, oc0 + kg * 16, wave, l32, lh);
     __syncthreads();
     v16i acc[MT][NT];
 #pragma unroll

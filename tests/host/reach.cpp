@@ -1,0 +1,119 @@
+// Where the residual loads and the stores of plain NCHW layers in one launch lead (no GPU).  conv_patch1.hip is compiled into this program, a
+// launch is noted with its arguments, and the offsets of every lane of every wave are made by the kernel's own functions.  By the rule at SENT
+// (igemm_shared.h) a lane either passes SENT or stays inside the tensor with its scalar offset added, and the scalar offset alone does too.
+// One descriptor per line of the input, in hexadecimal; one line of the output for each: the tile (blocks of 32 channels, of 128 pixels), the accesses
+// that were looked at, and those that break the rule.
+#include <cxxabi.h>
+#include <hip/hip_runtime.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <map>
+#include <string>
+
+#include "../../megengine_amd/csrc/common.h"
+namespace mi355 {
+__host__ static inline uint32_t fdiv(uint32_t x, const FastDiv& f) {
+    const uint32_t t = (uint32_t)((uint64_t)x * f.m >> 32);
+    return (t + ((x - t) >> f.s1)) >> f.s2;
+}
+}  // namespace mi355
+#pragma GCC visibility push(hidden)  // (the library's launch code runs, not this copy of it)
+#include "../../megengine_amd/csrc/conv_patch1.hip"
+#pragma GCC visibility pop
+
+namespace mi355 {
+static int g_mt, g_nt;  // of the last launch
+static P1Args g_args;
+static long g_seen, g_broken;
+
+// `size` bytes at the two offsets, in a tensor of `bytes`
+static void look(const P1Access& at, int size, uint32_t bytes) {
+    ++g_seen;
+    const bool scalar_in = at.scalar >= 0 && (uint32_t)at.scalar <= bytes;
+    const bool lane_in = at.lane == SENT || (at.lane >= 0 && (int64_t)at.lane + at.scalar + size <= bytes);
+    if (!scalar_in || !lane_in) ++g_broken;
+}
+
+static void walk(const P1Args& a) {
+    for (int tm = 0; tm < a.tiles_m; ++tm)
+        for (int tn = 0; tn < a.tiles_n; ++tn) {
+            const P1Tile o = p1_tile_at(a, tn);
+            for (int px = 0; px < 128 * g_nt; px += 4)
+                for (int ch = 0; ch < 8; ++ch) {
+                    const P1Out w = p1_out(a, o, px, ch);
+                    const P1Residual z = p1_residual_at(a, w);
+                    for (int oc8 = tm * g_mt * 32; oc8 < (tm + 1) * g_mt * 32; oc8 += 8) {
+                        if (a.epi.has_z) {
+                            look(p1_access(a, z.off, oc8, ch), 4, a.z_bytes);
+                            if (a.OHW < 4)
+                                for (int k = 0; k < 3; ++k) look(p1_access(a, k < w.cols ? w.z0 + k : SENT, oc8, ch), 1, a.z_bytes);
+                        }
+                        look(p1_access(a, w.cols > 0 ? w.d0 : SENT, oc8, ch), w.cols < 4 ? w.cols : 4, a.dst_bytes);
+                    }
+                }
+        }
+}
+
+static std::map<const void*, std::string>& kernels() {  // (filled ahead of this file's constructors)
+    static std::map<const void*, std::string> m;
+    return m;
+}
+}  // namespace mi355
+
+extern "C" {
+char __hip_fatbin[16];  // (compiled for the host alone: no kernels to register)
+void** __hipRegisterFatBinary(const void*) {
+    static void* handle;
+    return &handle;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) {
+    int st;
+    char* s = abi::__cxa_demangle(name, nullptr, nullptr, &st);
+    mi355::kernels()[host] = s ? s : name;
+    free(s);
+}
+hipError_t hipGetDevice(int* d) {
+    *d = 0;
+    return hipSuccess;
+}
+hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
+    memset(p, 0, sizeof(*p));
+    p->multiProcessorCount = 256;
+    return hipSuccess;
+}
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
+    const std::string& name = mi355::kernels()[f];
+    const size_t at = name.find("patch1_kernel<");
+    if (at == std::string::npos || sscanf(name.c_str() + at, "patch1_kernel<%d, %d", &mi355::g_mt, &mi355::g_nt) != 2) return hipErrorInvalidValue;
+    memcpy(&mi355::g_args, args[0], sizeof(mi355::g_args));
+    return hipSuccess;
+}
+}
+
+int main() {
+    static char hex[2 * sizeof(mi355_conv_desc) + 2];
+    char format[32];
+    snprintf(format, sizeof(format), "%%%zus", sizeof(hex) - 1);
+    while (scanf(format, hex) == 1) {
+        mi355_conv_desc d;
+        unsigned b;
+        for (size_t i = 0; i < sizeof(d); ++i) {
+            if (sscanf(hex + 2 * i, "%2x", &b) != 1) return 1;
+            reinterpret_cast<unsigned char*>(&d)[i] = (unsigned char)b;
+        }
+        int8_t* const t = reinterpret_cast<int8_t*>(0x1000000);  // device addresses that nothing on the host reads
+        const int st = mi355_convbias_s8_exec(nullptr, &d, nullptr, t, t, reinterpret_cast<int32_t*>(t), d.has_z ? t : nullptr, t, nullptr, 0);
+        if (st) {
+            printf("status %d: %s\n", st, mi355_last_error());
+            return 1;
+        }
+        mi355::g_seen = mi355::g_broken = 0;
+        mi355::walk(mi355::g_args);
+        printf("%d %d %ld %ld\n", mi355::g_mt, mi355::g_nt, mi355::g_seen, mi355::g_broken);
+    }
+    return 0;
+}

@@ -1,0 +1,49 @@
+"""Plain NCHW in one launch: no lane of a residual load or a store leads out of its tensor, by the kernel's own offsets
+(tests/host/reach.cpp, no GPU).  Channels that eight and 32 do not divide, in the last image above all; every tile; runs and rows that end inside a group of four; planes that hold no dword; images apart."""
+import os
+import subprocess
+
+import pytest
+
+from megengine_amd import _abi
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+EXE = os.path.join(HERE, "host", "reach")
+
+CASES = [
+    # n, ic, ih, iw, oc, f, pad, stride; blocks of 32 channels and of 128 pixels of the tile
+    (6, 75, 61, 45, 150, 3, 1, 1, (1, 2)),
+    (1, 8, 9, 9, 1, 5, 0, 1, (1, 1)),
+    (2, 5, 8, 11, 33, 3, 1, 1, (1, 1)),
+    (3, 40, 20, 17, 70, 5, 2, 1, (1, 1)),         # two groups of waves
+    (70, 4, 5, 5, 41, 5, 0, 1, (1, 1)),           # planes of one byte
+    (7000, 4, 5, 6, 35, 5, 0, 1, (1, 2)),         # of two, on a tile of 256 pixels
+    (5000, 4, 3, 8, 69, 3, 0, 5, (2, 1)),         # at a stride
+    (70, 20, 45, 37, 27, 3, 1, 1, (1, 2)),
+    (64, 8, 31, 63, 189, 3, 1, 1, (2, 2)),
+    (64, 8, 41, 43, 70, 1, 0, 1, (2, 2)),
+    (64, 16, 61, 61, 100, 3, 1, 2, (2, 1)),
+]
+
+
+def _desc(c, z, gap):
+    n, ic, ih, iw, oc, f, pad, stride, _ = c
+    d = _abi.make_conv_desc("NCHW", n, ic, ih, iw, oc, f, pad=pad, stride=stride, nonline="RELU", has_z=z, scale_bias=2e-4, scale_z=0.05, scale_dst=0.05)
+    if gap:
+        out = oc * _abi.out_size(ih, f, 1, stride, pad) * _abi.out_size(iw, f, 1, stride, pad)
+        d.dst_stride_n, d.z_stride_n = out + 40, out + 24
+    return d
+
+
+@pytest.mark.parametrize("gap", [False, True])
+@pytest.mark.parametrize("z", [False, True])
+def test_no_lane_leads_out(z, gap):
+    subprocess.check_call(["make", "-C", os.path.dirname(EXE), "-s", EXE])
+    descs = [_desc(c, z, gap) for c in CASES]
+    lines = "".join(bytes(d).hex() + "\n" for d in descs)
+    r = subprocess.run([EXE], input=lines, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+    got = [tuple(int(v) for v in line.split()) for line in r.stdout.splitlines()]
+    assert [g[:2] for g in got] == [c[-1] for c in CASES]
+    assert all(g[2] > 0 for g in got)
+    assert [g[3] for g in got] == [0] * len(descs)
