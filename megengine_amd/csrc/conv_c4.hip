@@ -92,9 +92,11 @@ struct C4Out {
     bool full;   // all 64 channels of the tile exist
 };
 
-// scalar offset of quad (i, q): batch stride * n + plane of channel oc0 + 32 * i + 8 * q (the lane half adds 4 channels)
-__device__ __forceinline__ int c4_soff(const C4Out& o, int nbase, int i, int q) {
-    return nbase + ((o.oc0 + 32 * i + 8 * q) >> 2) * o.plane4;
+// scalar offset of quad (i, q): batch stride * n + plane of channel oc0 + 32 * i + 8 * q (the lane half adds 4 channels);
+// quads past the last channel, whose lanes pass SENT: of the image
+__device__ __forceinline__ int c4_soff(const C4Out& o, int OC, int nbase, int i, int q) {
+    const int oc = o.oc0 + 32 * i + 8 * q;
+    return nbase + (o.full || oc < OC ? (oc >> 2) * o.plane4 : 0);
 }
 
 // per-lane offset of quad (i, q) in a channel tile that reaches past OC
@@ -113,7 +115,7 @@ __device__ __forceinline__ void c4_epilogue(const C4Args& a, const v16i (&acc)[2
         for (int q = 0; q < 4; ++q) {
             const v16i& c = acc[i];
             const uint32_t o = requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], zr[i][q], a.epi);
-            __builtin_amdgcn_raw_buffer_store_b32(o, rs_dst, c4_voff(out, a.OC, lh, i, q), c4_soff(out, nbase, i, q), 0);
+            __builtin_amdgcn_raw_buffer_store_b32(o, rs_dst, c4_voff(out, a.OC, lh, i, q), c4_soff(out, a.OC, nbase, i, q), 0);
         }
 }
 
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(C4_THREADS, FHT ? 3 : 2) void c4_kernel(C4Args a) {
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    zr[i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, c4_voff(out, a.OC, lh, i, q), c4_soff(out, zbase, i, q), 0);
+                    zr[i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, c4_voff(out, a.OC, lh, i, q), c4_soff(out, a.OC, zbase, i, q), 0);
         }
 
         v16i acc[2];

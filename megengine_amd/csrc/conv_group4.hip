@@ -288,6 +288,15 @@ struct G16Lane {
     int out, p;        // byte of the first pixel in the planes of the slab; the pixel
 };
 
+// The two offsets of unit k of step u, pixels from p = l.p + u + 16 k on, in the four planes of a slab.  first: the wave's first pixel.  (Past the
+// wave's last step nothing is loaded, and the scalar offset would lead out of planes of few pixels: by the rule at SENT it is zero there.)
+struct G16Access {
+    int lane, scalar;
+};
+__host__ __device__ __forceinline__ G16Access g16_access(const G16Lane& l, int k, int u, int first, int pixels, int base) {
+    return {l.p + u + k * 16 < pixels ? l.out + k * 64 : SENT, first + u < pixels ? base + u * 4 : 0};
+}
+
 // The pixels of one staged band, two units of 16 per wave and step; the operands and the residual of the next step are read while this
 // one is requantised.
 template <int NL, bool HZ>
@@ -312,8 +321,10 @@ __device__ __forceinline__ void grp16_band(const EpiParams& epi, const G16Lane& 
     };
     auto residual = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
-            zn[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, l.p + u + k * 16 < pixels ? l.out + k * 64 : SENT, base + u * 4, 0);
+        for (int k = 0; k < 2; ++k) {
+            const G16Access at = g16_access(l, k, u, first, pixels, base);
+            zn[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, at.lane, at.scalar, 0);
+        }
     };
     if (HZ) residual(0);
     operands();
@@ -329,8 +340,10 @@ __device__ __forceinline__ void grp16_band(const EpiParams& epi, const G16Lane& 
         __builtin_amdgcn_sched_barrier(0);
         requant8_as<NL, HZ>(acc[0], acc[1], zw, epi);
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
-            __builtin_amdgcn_raw_buffer_store_b32((int)zw[k], rs_dst, l.p + u + k * 16 < pixels ? l.out + k * 64 : SENT, base + u * 4, 0);
+        for (int k = 0; k < 2; ++k) {
+            const G16Access to = g16_access(l, k, u, first, pixels, base);
+            __builtin_amdgcn_raw_buffer_store_b32((int)zw[k], rs_dst, to.lane, to.scalar, 0);
+        }
     }
 }
 

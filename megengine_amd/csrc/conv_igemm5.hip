@@ -270,7 +270,7 @@ __device__ __forceinline__ void ks_run(const Form& form) {
         const bool half_in = S == 32 || kc * 2 + (lk >> 1) < a.KC;
         if (PIN == 32 && PW) {
             const int c = S == 32 ? 0 : (lk >> 1) * a.src_scb;
-            fb = __builtin_amdgcn_raw_buffer_load_b128(rs_src, in && half_in && pix != SENT ? pix + c : SENT, kc * CH * a.src_scb, 0);
+            fb = __builtin_amdgcn_raw_buffer_load_b128(rs_src, in && half_in && pix != SENT ? pix + c : SENT, (in ? kc : 0) * CH * a.src_scb, 0);
         } else if (PIN == 32 && S == 32) {
             const bool ok = in && (unsigned)(ih0 + fh) < (unsigned)a.IH && (unsigned)(iw0 + fw) < (unsigned)a.IW;
             // (not the block's offset as the instruction's scalar one: where the compiler keeps the cursor in a vector register, that

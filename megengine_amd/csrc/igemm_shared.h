@@ -104,7 +104,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint3
 
 // Byte offset that is out of range for every buffer (< 2 GiB).  It belongs into the lane's offset: LLVM declares the scalar offset of the buffer
 // builtins as left out of the range check, the instruction set manuals take it off the descriptor's size, and code here relies on neither.  So
-// a lane passes SENT wherever its two offsets together lead out of the tensor, what becomes of a loaded value notwithstanding.
+// a lane passes SENT wherever its two offsets together lead out of the tensor, what becomes of a loaded value notwithstanding, and the scalar
+// offset does not lead out by itself where all lanes pass SENT either.
 // (tests/host/reach.cpp walks such offsets.)
 constexpr int SENT = (int)0x80000000;
 

@@ -1,8 +1,9 @@
-// Where the residual loads and the stores of plain NCHW layers in one launch lead (no GPU).  conv_patch1.hip is compiled into this program, a
-// launch is noted with its arguments, and the offsets of every lane of every wave are made by the kernel's own functions.  By the rule at SENT
-// (igemm_shared.h) a lane either passes SENT or stays inside the tensor with its scalar offset added, and the scalar offset alone does too.
-// One descriptor per line of the input, in hexadecimal; one line of the output for each: the tile (blocks of 32 channels, of 128 pixels), the accesses
-// that were looked at, and those that break the rule.
+// Where the residual loads and the stores of plain NCHW layers in one launch and of grouped layers on the matrix cores lead (no GPU).
+// conv_patch1.hip and conv_group4.hip are compiled into this program, a launch is noted with its arguments, and the offsets of every lane of
+// every wave are made by the kernel's own functions.  By the rule at SENT (igemm_shared.h) a lane either passes SENT or stays inside the tensor
+// with its scalar offset added, and the scalar offset alone does too.
+// One descriptor per line of the input, in hexadecimal; one line of the output for each: the tile (blocks of 32 channels, of 128 pixels; 0 0 for
+// grouped layers), the accesses that were looked at, and those that break the rule.
 #include <cxxabi.h>
 #include <hip/hip_runtime.h>
 #include <stdio.h>
@@ -21,15 +22,18 @@ __host__ static inline uint32_t fdiv(uint32_t x, const FastDiv& f) {
 }  // namespace mi355
 #pragma GCC visibility push(hidden)  // (the library's launch code runs, not this copy of it)
 #include "../../megengine_amd/csrc/conv_patch1.hip"
+#include "../../megengine_amd/csrc/conv_group4.hip"
 #pragma GCC visibility pop
 
 namespace mi355 {
 static int g_mt, g_nt;  // of the last launch
 static P1Args g_args;
+static G16Args<FastDiv> g_grouped;
 static long g_seen, g_broken;
 
 // `size` bytes at the two offsets, in a tensor of `bytes`
-static void look(const P1Access& at, int size, uint32_t bytes) {
+template <class Access>
+static void look(const Access& at, int size, uint32_t bytes) {
     ++g_seen;
     const bool scalar_in = at.scalar >= 0 && (uint32_t)at.scalar <= bytes;
     const bool lane_in = at.lane == SENT || (at.lane >= 0 && (int64_t)at.lane + at.scalar + size <= bytes);
@@ -54,6 +58,26 @@ static void walk(const P1Args& a) {
                     }
                 }
         }
+}
+
+static void walk(const G16Args<FastDiv>& a) {
+    const uint32_t bytes = (uint32_t)a.dst_scb * 4;
+    for (int band = 0; band < a.bands; ++band) {
+        const int oh0 = band * a.TH, pixels = (a.OH - oh0 < a.TH ? a.OH - oh0 : a.TH) * a.OW, base = oh0 * a.OW * 4;
+        for (int t = 0; t < 256; ++t) {
+            G16Lane l;
+            l.p = (t >> 6) * 32 + (t & 15);
+            l.out = (t >> 4 & 3) * a.dst_scb + l.p * 4;
+            const int first = (t >> 6) * 32;
+            for (int k = 0; k < 2; ++k) {
+                if (a.epi.has_z) look(g16_access(l, k, 0, first, pixels, base), 4, bytes);
+                for (int u = 0; first + u < pixels; u += 128) {
+                    if (a.epi.has_z) look(g16_access(l, k, u + 128, first, pixels, base), 4, bytes);
+                    look(g16_access(l, k, u, first, pixels, base), 4, bytes);
+                }
+            }
+        }
+    }
 }
 
 static std::map<const void*, std::string>& kernels() {  // (filled ahead of this file's constructors)
@@ -87,6 +111,16 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
     const std::string& name = mi355::kernels()[f];
+    mi355::g_mt = mi355::g_nt = 0;
+    if (name.find("grp16_kernel<") != std::string::npos) {
+        if (name.find("G16Wide") != std::string::npos) {
+            mi355::g_grouped = static_cast<mi355::G16Wide*>(args[0])->a;
+        } else {
+            static_cast<mi355::G16Wire*>(args[0])->numbers(mi355::g_grouped);
+            mi355::g_grouped.epi.has_z = static_cast<mi355::G16Wire*>(args[0])->flags >> 3 & 1;
+        }
+        return hipSuccess;
+    }
     const size_t at = name.find("patch1_kernel<");
     if (at == std::string::npos || sscanf(name.c_str() + at, "patch1_kernel<%d, %d", &mi355::g_mt, &mi355::g_nt) != 2) return hipErrorInvalidValue;
     memcpy(&mi355::g_args, args[0], sizeof(mi355::g_args));
@@ -112,7 +146,7 @@ int main() {
             return 1;
         }
         mi355::g_seen = mi355::g_broken = 0;
-        mi355::walk(mi355::g_args);
+        mi355::g_mt ? mi355::walk(mi355::g_args) : mi355::walk(mi355::g_grouped);
         printf("%d %d %ld %ld\n", mi355::g_mt, mi355::g_nt, mi355::g_seen, mi355::g_broken);
     }
     return 0;

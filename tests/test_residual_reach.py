@@ -1,5 +1,6 @@
-"""Plain NCHW in one launch: no lane of a residual load or a store leads out of its tensor, by the kernel's own offsets
-(tests/host/reach.cpp, no GPU).  Channels that eight and 32 do not divide, in the last image above all; every tile; runs and rows that end inside a group of four; planes that hold no dword; images apart."""
+"""Plain NCHW in one launch and grouped layers on the matrix cores: no lane of a residual load or a store leads out of its tensor, by the kernels'
+own offsets (tests/host/reach.cpp, no GPU).  Plain: channels that eight and 32 do not divide, in the last image above all; every tile; runs and
+rows that end inside a group of four; planes that hold no dword; images apart.  Grouped: planes of fewer pixels than a step, bands."""
 import os
 import subprocess
 
@@ -24,6 +25,10 @@ CASES = [
     (64, 8, 41, 43, 70, 1, 0, 1, (2, 2)),
     (64, 16, 61, 61, 100, 3, 1, 2, (2, 1)),
 ]
+GROUPED = [
+    # n, groups, channels of one, ih, iw, pad, stride
+    (2, 4, 4, 3, 3, 0, 1), (1, 2, 8, 5, 5, 1, 1), (3, 2, 16, 7, 5, 1, 2), (1, 4, 4, 8, 16, 1, 1), (64, 8, 16, 46, 30, 1, 1), (40, 22, 8, 87, 13, 1, 1),
+]
 
 
 def _desc(c, z, gap):
@@ -35,15 +40,24 @@ def _desc(c, z, gap):
     return d
 
 
+def _grouped(c, z, gap):
+    n, g, per, ih, iw, pad, stride = c
+    d = _abi.make_conv_desc("NCHW4", n, g * per, ih, iw, g * per, 3, pad=pad, stride=stride, group=g, nonline="RELU", has_z=z, scale_bias=2e-4,
+                            scale_z=0.05, scale_dst=0.05)
+    if gap:   # the kernel's wide argument
+        d.dst_stride_n = g * per * _abi.out_size(ih, 3, 1, stride, pad) * _abi.out_size(iw, 3, 1, stride, pad) + 64
+    return d
+
+
 @pytest.mark.parametrize("gap", [False, True])
 @pytest.mark.parametrize("z", [False, True])
 def test_no_lane_leads_out(z, gap):
     subprocess.check_call(["make", "-C", os.path.dirname(EXE), "-s", EXE])
-    descs = [_desc(c, z, gap) for c in CASES]
+    descs = [_desc(c, z, gap) for c in CASES] + [_grouped(c, z, gap) for c in GROUPED]
     lines = "".join(bytes(d).hex() + "\n" for d in descs)
     r = subprocess.run([EXE], input=lines, capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
     got = [tuple(int(v) for v in line.split()) for line in r.stdout.splitlines()]
-    assert [g[:2] for g in got] == [c[-1] for c in CASES]
+    assert [g[:2] for g in got] == [c[-1] for c in CASES] + [(0, 0)] * len(GROUPED)
     assert all(g[2] > 0 for g in got)
     assert [g[3] for g in got] == [0] * len(descs)
