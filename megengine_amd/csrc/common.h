@@ -158,12 +158,12 @@ template <class T>
 struct XcdRun {
     T at, end, step;
 };
-template <class T, int STEP = 256>
+template <class T>
 __device__ __forceinline__ XcdRun<T> xcd_run(T units, uint32_t grid) {
-    if (grid < 16) return {(T)blockIdx.x * STEP + threadIdx.x, units, (T)grid * STEP};
-    const T per = (units + 8 * STEP - 1) / (8 * STEP) * STEP, lo = (T)(blockIdx.x & 7) * per;
+    if (grid < 16) return {(T)blockIdx.x * 256 + threadIdx.x, units, (T)grid * 256};
+    const T per = (units + 2047) / 2048 * 256, lo = (T)(blockIdx.x & 7) * per;
     const T hi = lo + per < units ? lo + per : units;
-    return {lo + (T)(blockIdx.x >> 3) * STEP + threadIdx.x, hi, (T)((grid + 7 - (blockIdx.x & 7)) >> 3) * STEP};
+    return {lo + (T)(blockIdx.x >> 3) * 256 + threadIdx.x, hi, (T)((grid + 7 - (blockIdx.x & 7)) >> 3) * 256};
 }
 // whole rounds over the XCDs, so that no XCD lacks a workgroup for its eighth
 static inline uint64_t xcd_grid(uint64_t blocks) { return blocks < 16 ? blocks : (blocks + 7) & ~(uint64_t)7; }

@@ -37,46 +37,11 @@ __global__ __launch_bounds__(256) void requant_kernel(const int32_t* __restrict_
     }
 }
 
-// Four quads of a thread in flight and one form of the requantisation for the loop, where every workgroup is resident and has one step
-// (requant_wide).  Bound by bytes and the latency of a wave's first loads: 6.4 million values with a residual, 39 MB, 6.00 -> 5.33 us.
-constexpr int RQ_U = 4;
-template <int NL, bool HZ>
-__device__ __forceinline__ void requant_wide_run(const int32_t* __restrict__ src, const int8_t* __restrict__ z, int8_t* __restrict__ dst,
-                                                 uint64_t quads, const EpiParams& e) {
-    const XcdRun<uint64_t> run = xcd_run<uint64_t, 256 * RQ_U>(quads, gridDim.x);
-    for (uint64_t i = run.at; i < run.end; i += run.step) {
-        if (i + 256 * (RQ_U - 1) < run.end) {
-            v4i a[RQ_U];
-            uint32_t zw[RQ_U];
-#pragma unroll
-            for (int u = 0; u < RQ_U; ++u) {
-                a[u] = reinterpret_cast<const v4i*>(src)[i + 256 * u];
-                zw[u] = HZ ? reinterpret_cast<const uint32_t*>(z)[i + 256 * u] : 0u;
-            }
-#pragma unroll
-            for (int u = 0; u < RQ_U; ++u) reinterpret_cast<uint32_t*>(dst)[i + 256 * u] = requant4_form<NL, HZ>(a[u], zw[u], e);
-        } else {
-            for (uint64_t k = i; k < run.end; k += 256)
-                reinterpret_cast<uint32_t*>(dst)[k] =
-                        requant4_form<NL, HZ>(reinterpret_cast<const v4i*>(src)[k], HZ ? reinterpret_cast<const uint32_t*>(z)[k] : 0u, e);
-        }
-    }
-}
-__global__ __launch_bounds__(256) void requant_wide_kernel(const int32_t* __restrict__ src, const int8_t* __restrict__ z, int8_t* __restrict__ dst,
-                                                           uint64_t quads, uint64_t count, EpiParams e) {
-    if (e.has_z)
-        with_requant_form<true>(e, [&](auto nl) { requant_wide_run<decltype(nl)::value, true>(src, z, dst, quads, e); });
-    else
-        with_requant_form<false>(e, [&](auto nl) { requant_wide_run<decltype(nl)::value, false>(src, z, dst, quads, e); });
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        for (uint64_t j = quads * 4; j < count; ++j)
-            dst[j] = (int8_t)requant_s8_exact(src[j], e.has_z != 0, e.has_z ? (int)z[j] : 0, e);
-    }
-}
-
 // QuantizedS8 first operand: 16 elements per thread step (16 + 16 bytes in, 16 out; 2-3 bytes per element), in a loop of its own for every
 // form: the form chosen for each dword, four times a step, took the vector instructions of four apart.  42 registers, still eight
-// waves to a SIMD; of 36 drawn sizes up to 46 million values 0.91 of the time (0.85 to 0.99).
+// waves to a SIMD.  36 drawn sizes up to 46 million values, replays of this kernel alone: 0.91 of the time (0.85 to 0.99).  In chains of
+// convolution, requantisation, gate, activation, add, pool and dequantisation, where it is one of seven kernels, 30 drawn sizes: 0.990 (0.967
+// to 1.022) as graph replays, 0.995 call by call.
 template <int NL, bool HZ>
 __device__ __forceinline__ void requant8_run(const int8_t* __restrict__ src, const int8_t* __restrict__ z, int8_t* __restrict__ dst, uint64_t blocks16,
                                              const EpiParams& e) {
@@ -146,11 +111,6 @@ __global__ __launch_bounds__(256) void cvt_s8_f32_kernel(const int8_t* __restric
         for (uint64_t j = quads * 4; j < count; ++j) dst[j] = (float)src[j] * scale;
 }
 
-// tiles of 4096 values: at least two to a CU, and all of them resident (eight to a CU): 0.89 to 0.99 of requant_kernel's time there, 0.94 on average.
-// With fewer the loads of a CU are too few either way and quads of their own start sooner (1.1 million values, residual: 2.9 / 3.2 us); with
-// more the tiles run in uneven rounds (8.7 million: 9.9 / 10.4; 12.3 million: 10.7 / 11.3), and from 20 million on both are bound by bytes.
-bool requant_wide(uint64_t tiles, int cu_count) { return tiles >= 2 * (uint64_t)cu_count && tiles <= 8 * (uint64_t)cu_count; }
-
 unsigned stream_blocks(uint64_t steps, int cu_count) {
     if (cu_count <= 0) cu_count = 256;
     uint64_t blocks = (steps + 255) / 256;
@@ -191,9 +151,6 @@ int launch_requant(hipStream_t st, const EpiParams& e, const int32_t* src, const
     if (count == 0) return 0;
     const uint64_t quads = count / 4;
     if (cu_count <= 0) cu_count = 256;
-    const uint64_t tiles = (quads + 256 * RQ_U - 1) / (256 * RQ_U);
-    if (requant_wide(tiles, cu_count))
-        return launch_kernel(requant_wide_kernel, dim3((unsigned)xcd_grid(tiles)), dim3(256), 0, st, src, z, dst, quads, count, e);
     uint64_t blocks = (quads + 255) / 256;
     const uint64_t cap = (uint64_t)cu_count * 16;
     if (blocks > cap) blocks = cap;

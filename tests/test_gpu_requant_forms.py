@@ -1,5 +1,5 @@
-"""Stand-alone requantisation where a thread has four quads in flight: both ends of the sizes that take it, parts of a tile, counts that four does
-not divide; and every form of the arithmetic, the literal chain included, for int32 and int8 operands.  Against the oracle."""
+"""Stand-alone requantisation around whole rounds of 4096 values to a CU, and counts that four does not divide; every form of the arithmetic, the
+literal chain included, for int32 and int8 operands, of which the latter has a loop per form.  Against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -9,7 +9,7 @@ from tests.test_gpu_requant import run_case
 
 pytestmark = pytest.mark.gpu
 
-TILE = 4096   # values of a workgroup's step
+TILE = 4096
 
 
 @pytest.mark.parametrize("tiles,more", [(2, -TILE), (2, -TILE + 4), (2, 0), (2, 3), (2, 4), (5, 1023 * 4 + 1), (8, -5), (8, 0), (8, 4)])
