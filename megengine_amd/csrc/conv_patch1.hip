@@ -96,17 +96,19 @@ __host__ __device__ __forceinline__ P1Residual p1_residual_at(const P1Args& a, c
     const bool in = (w.cols > 0) & (a.OHW >= 4);
     return {in ? at : SENT, in ? (w.z0 - at) * 8 : 0};
 }
-// The two offsets of an access to channel oc8 + ch at offset `at` of the first eight channels, by the rule at SENT: a lane without a
-// channel passes SENT, and a scalar offset leads to a channel that exists.
+// What an access to channel oc8 + ch passes beside its offset of the first eight channels, by the rule at SENT: SENT, to be or'ed to that offset, in
+// a lane without a channel, and a scalar offset that does not lead out of the tensor.  (One minimum and no selection: with the scalar offset
+// chosen and a mask for each store, 200 drawn layers without a residual took 1.006 of the time.)
 struct P1Access {
     int lane, scalar;
 };
-__host__ __device__ __forceinline__ P1Access p1_access(const P1Args& a, int at, int oc8, int ch) {
-    int left = a.OC - oc8;
+__host__ __device__ __forceinline__ P1Access p1_access(const P1Args& a, int oc8, int ch) {
+    const int oc = min(oc8, a.OC);
+    int left = a.OC - oc;
 #ifdef __HIP_DEVICE_COMPILE__
     asm("" : "+s"(left));  // (or the masks of a whole tile are made at once and kept, and scalar registers spill)
 #endif
-    return {ch < left ? at : SENT, left > 0 ? oc8 * a.OHW : 0};
+    return {ch < left ? 0 : SENT, oc * a.OHW};
 }
 template <int MT, int NT, int QN>
 __device__ __forceinline__ void p1_residual_bytes(const P1Args& a, uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0, int wave, int l32, int lh) {
@@ -119,32 +121,39 @@ __device__ __forceinline__ void p1_residual_bytes(const P1Args& a, uint32_t (&zq
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int q = 0; q < QN; ++q) {
+                const P1Access at = p1_access(a, oc0 + i * 32 + 8 * q, ch);
                 zq[j][i][q] = 0;
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
-                    const P1Access at = p1_access(a, k < w.cols ? w.z0 + k : SENT, oc0 + i * 32 + 8 * q, ch);
-                    zq[j][i][q] |= (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rs_z, at.lane, at.scalar, 0) << (8 * k);
+                    const int off = k < w.cols ? w.z0 + k : SENT;
+                    zq[j][i][q] |= (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rs_z, at.lane | off, at.scalar, 0) << (8 * k);
                 }
             }
     }
 }
 
-// the residual of a wave's outputs, in flight at once (a launch without one: a descriptor of no bytes)
+// the residual of a wave's outputs, in flight at once; ch: the lane's channel of eight
 template <int MT, int NT, int QN>
-__device__ __forceinline__ void p1_residual(const P1Args& a, uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0, int wave, int l32, int lh) {
-    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.epi.has_z ? a.z_bytes : 0);
-    const int ch = 4 * lh + (l32 & 3);
+__device__ __forceinline__ void p1_residual(const P1Args& a, uint32_t (&zq)[NT][MT][QN], const P1Residual (&z)[NT], int oc0, int ch) {
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.z_bytes);
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const P1Residual z = p1_residual_at(a, p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), ch));
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int q = 0; q < QN; ++q) {
-                const P1Access at = p1_access(a, z.off, oc0 + i * 32 + 8 * q, ch);
-                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, at.lane, at.scalar, 0);
+                const P1Access at = p1_access(a, oc0 + i * 32 + 8 * q, ch);
+                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, at.lane | z[j].off, at.scalar, 0);
             }
-    }
+}
+// the same for the largest tile, where it is asked for behind the products
+template <int MT, int NT, int QN>
+__device__ __forceinline__ void p1_residual_late(const P1Args& a, uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0, int wave, int l32, int lh) {
+    const int ch = 4 * lh + (l32 & 3);
+    P1Residual z[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) z[j] = p1_residual_at(a, p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), ch));
+    p1_residual<MT, NT, QN>(a, zq, z, oc0, ch);
 }
 
 // QN: eights of channels of each block of 32 that are in acc (all four, or two)
@@ -172,12 +181,11 @@ __device__ __forceinline__ void p1_epilogue(const P1Args& a, v16i (&acc)[MT][NT]
                 }
                 const v16i& c = acc[i][j];
                 const uint32_t y = quad_transpose(requant4_fast<NL, HZ>(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3], zw, a.epi), lane4);
-                const P1Access to = p1_access(a, four, oc8, ch);
-                __builtin_amdgcn_raw_buffer_store_b32((int)y, rs_dst, to.lane, to.scalar, 0);
+                const P1Access to = p1_access(a, oc8, ch);
+                __builtin_amdgcn_raw_buffer_store_b32((int)y, rs_dst, to.lane | four, to.scalar, 0);
                 if (split) {
-                    const P1Access to2 = p1_access(a, two, oc8, ch), to1 = p1_access(a, one, oc8, ch);
-                    __builtin_amdgcn_raw_buffer_store_b16((uint16_t)y, rs_dst, to2.lane, to2.scalar, 0);
-                    __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(cols == 3 ? y >> 16 : y), rs_dst, to1.lane, to1.scalar, 0);
+                    __builtin_amdgcn_raw_buffer_store_b16((uint16_t)y, rs_dst, to.lane | two, to.scalar, 0);
+                    __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(cols == 3 ? y >> 16 : y), rs_dst, to.lane | one, to.scalar, 0);
                 }
             }
     }

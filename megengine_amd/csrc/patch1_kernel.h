@@ -159,11 +159,21 @@ __global__ __launch_bounds__(256 * KS, 2) void patch1_kernel(P1Args a) {
         const int o0 = (e0 / T) * a.PX + ((e0 % T) / F) * a.PWC + (e0 % T) % F, o1 = (e1 / T) * a.PX + ((e1 % T) / F) * a.PWC + (e1 % T) % F;
         offs[k] = A_VECS + (lh ? o1 : o0);
     }
+    // Where the residual lies is worked out while the first operands are on their way, and its loads stand ahead of the next stage's, which are
+    // waited for first.  (Both inside the branch, behind those: 300 drawn layers with a residual 1.025 of the time.  Without the branch sixteen loads
+    // of no bytes: 300 without a residual 1.01 to 1.03.)
+    P1Residual z_at[NT];
+    if constexpr (ZPRE)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            z_at[j] = p1_residual_at(a, p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), 4 * lh + (l32 & 3)));
+            asm volatile("" : "+v"(z_at[j].off));
+        }
     store(kg, 0);
     __builtin_amdgcn_s_waitcnt(P1_VMCNT0);  // (the compiler knows: a stage's products do not wait for the next stage's loads)
-    if (kg + KS < a.nstages) fetch(kg + KS);
     uint32_t zq[NT][MT][QN];
-    if constexpr (ZPRE) p1_residual<MT, NT, QN>(a, zq, o, oc0 + kg * 16, wave, l32, lh);
+    if (ZPRE && a.epi.has_z) p1_residual<MT, NT, QN>(a, zq, z_at, oc0 + kg * 16, 4 * lh + (l32 & 3));
+    if (kg + KS < a.nstages) fetch(kg + KS);
     __syncthreads();
     v16i acc[MT][NT];
 #pragma unroll
@@ -232,7 +242,7 @@ __global__ __launch_bounds__(256 * KS, 2) void patch1_kernel(P1Args a) {
     if constexpr (ZPRE) {
         if (a.epi.has_z && a.OHW < 4) p1_residual_bytes<MT, NT, QN>(a, zq, o, oc0 + kg * 16, wave, l32, lh);
     } else if (a.epi.has_z) {
-        p1_residual<MT, NT, QN>(a, zq, o, oc0, wave, l32, lh);
+        p1_residual_late<MT, NT, QN>(a, zq, o, oc0, wave, l32, lh);
     }
 #define MI355_P1(NL, HZ) p1_epilogue<MT, NT, QN, NL, HZ>(a, acc, zq, o, oc0 + kg * 16, wave, l32, lh)
     if (a.epi.lin) {

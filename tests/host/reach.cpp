@@ -32,11 +32,10 @@ static G16Args<FastDiv> g_grouped;
 static long g_seen, g_broken;
 
 // `size` bytes at the two offsets, in a tensor of `bytes`
-template <class Access>
-static void look(const Access& at, int size, uint32_t bytes) {
+static void look(int lane, int scalar, int size, uint32_t bytes) {
     ++g_seen;
-    const bool scalar_in = at.scalar >= 0 && (uint32_t)at.scalar <= bytes;
-    const bool lane_in = at.lane == SENT || (at.lane >= 0 && (int64_t)at.lane + at.scalar + size <= bytes);
+    const bool scalar_in = scalar >= 0 && (uint32_t)scalar <= bytes;
+    const bool lane_in = lane < 0 || (int64_t)lane + scalar + size <= bytes;  // (SENT, whatever is or'ed to it)
     if (!scalar_in || !lane_in) ++g_broken;
 }
 
@@ -49,17 +48,19 @@ static void walk(const P1Args& a) {
                     const P1Out w = p1_out(a, o, px, ch);
                     const P1Residual z = p1_residual_at(a, w);
                     for (int oc8 = tm * g_mt * 32; oc8 < (tm + 1) * g_mt * 32; oc8 += 8) {
+                        const P1Access at = p1_access(a, oc8, ch);
                         if (a.epi.has_z) {
-                            look(p1_access(a, z.off, oc8, ch), 4, a.z_bytes);
+                            look(at.lane | z.off, at.scalar, 4, a.z_bytes);
                             if (a.OHW < 4)
-                                for (int k = 0; k < 3; ++k) look(p1_access(a, k < w.cols ? w.z0 + k : SENT, oc8, ch), 1, a.z_bytes);
+                                for (int k = 0; k < 3; ++k) look(at.lane | (k < w.cols ? w.z0 + k : SENT), at.scalar, 1, a.z_bytes);
                         }
-                        look(p1_access(a, w.cols > 0 ? w.d0 : SENT, oc8, ch), w.cols < 4 ? w.cols : 4, a.dst_bytes);
+                        look(at.lane | (w.cols > 0 ? w.d0 : SENT), at.scalar, w.cols < 4 ? w.cols : 4, a.dst_bytes);
                     }
                 }
         }
 }
 
+static void look(const G16Access& at, uint32_t bytes) { look(at.lane, at.scalar, 4, bytes); }
 static void walk(const G16Args<FastDiv>& a) {
     const uint32_t bytes = (uint32_t)a.dst_scb * 4;
     for (int band = 0; band < a.bands; ++band) {
@@ -70,10 +71,10 @@ static void walk(const G16Args<FastDiv>& a) {
             l.out = (t >> 4 & 3) * a.dst_scb + l.p * 4;
             const int first = (t >> 6) * 32;
             for (int k = 0; k < 2; ++k) {
-                if (a.epi.has_z) look(g16_access(l, k, 0, first, pixels, base), 4, bytes);
+                if (a.epi.has_z) look(g16_access(l, k, 0, first, pixels, base), bytes);
                 for (int u = 0; first + u < pixels; u += 128) {
-                    if (a.epi.has_z) look(g16_access(l, k, u + 128, first, pixels, base), 4, bytes);
-                    look(g16_access(l, k, u, first, pixels, base), 4, bytes);
+                    if (a.epi.has_z) look(g16_access(l, k, u + 128, first, pixels, base), bytes);
+                    look(g16_access(l, k, u, first, pixels, base), bytes);
                 }
             }
         }
