@@ -87,7 +87,8 @@ __host__ __device__ __forceinline__ P1Out p1_out(const P1Args& a, const P1Tile& 
 // Where a lane loads the residual of its four columns, and how far it turns the dword: a group that the row's end cuts short is loaded as the
 // dword that ends there, or begins with the plane, and not byte by byte, three loads to be waited for behind the store before them.  Of 300
 // drawn layers those with a residual take 0.944 of the time, the others the same (1x1 27 -> 37 at 83 x 93, stride 2, batch 14: 7.40 -> 6.02 us;
-// 3x3 11 -> 41 at 70 x 13, stride 2, batch 10: 5.43 -> 4.58).  (Planes of fewer than four bytes hold no dword: p1_residual_bytes.)
+// 3x3 11 -> 41 at 70 x 13, stride 2, batch 10: 5.43 -> 4.58).  (Planes of fewer than four bytes hold no dword: p1_residual_across on the largest tile,
+// which has many, p1_residual_bytes on the others.)
 struct P1Residual {
     int off, turn;
 };
@@ -109,6 +110,12 @@ __host__ __device__ __forceinline__ P1Access p1_access(const P1Args& a, int oc8,
     asm("" : "+s"(left));  // (or the masks of a whole tile are made at once and kept, and scalar registers spill)
 #endif
     return {ch < left ? 0 : SENT, oc * a.OHW};
+}
+// The residual in planes of fewer than four bytes, which hold no dword, in a tensor that does: the dword that ends with the group or begins with
+// the tensor, by the whole offset, which the lane's part does not tell.
+__host__ __device__ __forceinline__ P1Residual p1_residual_across(const P1Out& w, const P1Access& at) {
+    const int off = w.z0 + at.scalar, start = max(off + w.cols - 4, 0);
+    return {w.cols > 0 ? at.lane | start : SENT, (off - start) * 8 & 31};
 }
 template <int MT, int NT, int QN>
 __device__ __forceinline__ void p1_residual_bytes(const P1Args& a, uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0, int wave, int l32, int lh) {
@@ -146,14 +153,29 @@ __device__ __forceinline__ void p1_residual(const P1Args& a, uint32_t (&zq)[NT][
                 zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, at.lane | z[j].off, at.scalar, 0);
             }
 }
-// the same for the largest tile, where it is asked for behind the products
+// The same for the largest tile, where it is asked for behind the products.  (Planes of fewer than four bytes: 8192 images of 64 channels, 3 x 4
+// -> 256, 3x3, take 66 us by single bytes, 80 on the smaller tiles, 52 so.)
 template <int MT, int NT, int QN>
 __device__ __forceinline__ void p1_residual_late(const P1Args& a, uint32_t (&zq)[NT][MT][QN], const P1Tile& o, int oc0, int wave, int l32, int lh) {
     const int ch = 4 * lh + (l32 & 3);
+    P1Out w[NT];
     P1Residual z[NT];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) z[j] = p1_residual_at(a, p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), ch));
-    p1_residual<MT, NT, QN>(a, zq, z, oc0, ch);
+    for (int j = 0; j < NT; ++j) {
+        w[j] = p1_out(a, o, (wave * NT + j) * 32 + (l32 & ~3), ch);
+        z[j] = p1_residual_at(a, w[j]);
+    }
+    if (a.OHW >= 4) return p1_residual<MT, NT, QN>(a, zq, z, oc0, ch);
+    const __amdgpu_buffer_rsrc_t rs_z = make_rsrc(a.z, a.z_bytes);
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < QN; ++q) {
+                const P1Residual at = p1_residual_across(w[j], p1_access(a, oc0 + i * 32 + 8 * q, ch));
+                zq[j][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_z, at.off, 0, 0) >> at.turn;
+            }
 }
 
 // QN: eights of channels of each block of 32 that are in acc (all four, or two)
@@ -395,7 +417,7 @@ static int p1_tile(const ConvProblem& p, bool packed, int cu_count, P1Args& k, i
         }
         return w > 0 ? take(3, w) : 0;
     }
-    const int64_t w2 = p.d.oc > 32 && (!p.d.has_z || p.oh * p.ow >= 4) ? wgs(2) : 0;  // (its form has no loads of single residual bytes: spills)
+    const int64_t w2 = p.d.oc > 32 ? wgs(2) : 0;
     if (w2 >= 512) return take(2, w2);
     const int64_t w1 = wgs(1);
     return w1 > 0 ? take(1, w1) : 0;

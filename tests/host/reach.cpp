@@ -51,7 +51,8 @@ static void walk(const P1Args& a) {
                         const P1Access at = p1_access(a, oc8, ch);
                         if (a.epi.has_z) {
                             look(at.lane | z.off, at.scalar, 4, a.z_bytes);
-                            if (a.OHW < 4)
+                            if (a.OHW < 4 && g_mt * g_nt > 2) look(p1_residual_across(w, at).off, 0, 4, a.z_bytes);
+                            if (a.OHW < 4 && g_mt * g_nt <= 2)
                                 for (int k = 0; k < 3; ++k) look(at.lane | (k < w.cols ? w.z0 + k : SENT), at.scalar, 1, a.z_bytes);
                         }
                         look(at.lane | (w.cols > 0 ? w.d0 : SENT), at.scalar, w.cols < 4 ? w.cols : 4, a.dst_bytes);

@@ -1,6 +1,6 @@
 """Plain NCHW in one launch where rows end inside a group of four columns: the residual of such a group is the dword that ends there, from the first
 byte of the tensor on, and its outputs are stored as two bytes and one.  Images of one to seven columns, whose first group has fewer than four bytes
-before it; planes that hold no dword; one channel and nine; the largest tile.  Against the oracle, and over the residual."""
+before it; planes that hold no dword; one channel and nine; every tile.  Against the oracle, and over the residual."""
 import numpy as np
 import pytest
 import torch
@@ -10,18 +10,27 @@ from tests import util
 from tests.routes import UNNAMED, routes
 
 S = dict(scale_bias=2e-4, scale_z=0.05, scale_dst=0.05)
-# n, ic, oh, ow, oc
-CASES = [(1, 4, 2, w, oc) for w in range(1, 8) for oc in (2, 9)] + [(1, 8, 1, 5, 1), (1, 8, 4, 1, 1), (1, 8, 1, 3, 1), (70, 4, 1, 1, 40), (5, 4, 1, 2, 65), (3, 4, 3, 1, 9), (3, 5, 3, 2, 33), (2, 5, 9, 37, 40), (9, 3, 41, 43, 70)]
+# n, ic, oh, ow, oc, stride; blocks of 32 channels and of 128 pixels of the tile; ahead of them the filter and the threads of a workgroup
+CASES = [(1, 4, 2, w, oc, 1, (1, 1)) for w in range(1, 8) for oc in (2, 9)] + [
+    (1, 8, 1, 5, 1, 1, (1, 1)), (1, 8, 4, 1, 1, 1, (1, 1)), (1, 8, 1, 3, 1, 1, (1, 1)), (70, 4, 1, 1, 40, 1, (1, 1)), (5, 4, 1, 2, 65, 1, (1, 1)),
+    (3, 4, 3, 1, 9, 1, (1, 1)), (3, 5, 3, 2, 33, 1, (1, 1)), (2, 5, 9, 37, 40, 1, (1, 1)), (9, 3, 41, 43, 70, 1, (1, 2)),
+    (70, 3, 41, 43, 37, 1, (2, 2)), (64, 4, 30, 43, 70, 1, (2, 2)),                                   # the largest tile
+    (7000, 4, 1, 2, 35, 1, (1, 2)), (9000, 3, 3, 1, 33, 1, (1, 2)),                                   # single residual bytes on 32 x 256
+    (5000, 4, 1, 2, 69, 2, (2, 1)), (5000, 3, 1, 3, 70, 2, (2, 1)), (60, 3, 23, 41, 70, 2, (2, 1)),   # and on 64 x 128; its dwords
+    (16400, 3, 1, 2, 70, 1, (2, 2)), (16400, 3, 1, 1, 65, 1, (2, 2)), (11000, 3, 3, 1, 66, 1, (2, 2)),   # the largest, dwords across planes
+]
+CASES = [(5, 256) + c for c in CASES] + [(3, 512, 20, 70, 1, 2, 33, 1, (1, 1)), (3, 512, 2, 70, 1, 3, 19, 1, (1, 1)), (3, 512, 3, 75, 9, 7, 20, 1, (1, 1))]   # two groups
 
 
 def _desc(c, nl, has_z):
-    n, ic, oh, ow, oc = c
-    return _abi.make_conv_desc("NCHW", n, ic, oh + 4, ow + 4, oc, 5, nonline=nl, has_z=has_z, **S)
+    f, _, n, ic, oh, ow, oc, stride, _ = c
+    return _abi.make_conv_desc("NCHW", n, ic, (oh - 1) * stride + f, (ow - 1) * stride + f, oc, f, stride=stride, nonline=nl, has_z=has_z, **S)
 
 
 def test_route():
     got = routes([(_desc(c, "RELU", True), UNNAMED, -1, False) for c in CASES])
-    assert all(r.kernels[0].startswith("patch1_kernel") for r in got)
+    assert [r.kernels for r in got] == [("patch1_kernel<%d, %d, %d>" % (c[-1] + (c[0] ** 2,)),) for c in CASES]
+    assert [r.threads for r in got] == [c[1] for c in CASES]
 
 
 @pytest.mark.gpu

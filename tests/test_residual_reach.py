@@ -20,6 +20,7 @@ CASES = [
     (70, 4, 5, 5, 41, 5, 0, 1, (1, 1)),           # planes of one byte
     (7000, 4, 5, 6, 35, 5, 0, 1, (1, 2)),         # of two, on a tile of 256 pixels
     (5000, 4, 3, 8, 69, 3, 0, 5, (2, 1)),         # at a stride
+    (16400, 3, 5, 6, 70, 5, 0, 1, (2, 2)),        # on the largest
     (70, 20, 45, 37, 27, 3, 1, 1, (1, 2)),
     (64, 8, 31, 63, 189, 3, 1, 1, (2, 2)),
     (64, 8, 41, 43, 70, 1, 0, 1, (2, 2)),
