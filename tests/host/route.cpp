@@ -1,7 +1,8 @@
 // Which kernels an exec launches (no GPU: the runtime's calls that would need one are answered here, and a launch is only noted).
 // One exec per line of the input: the descriptor's bytes in hexadecimal, an algorithm (a number: by that name; -1: the heuristic's
 // choice, named; -2: none, exec chooses for itself), its tile (-1: the query's), and whether there is a workspace.  One line of the
-// output for each: the number of launches, dynamic LDS and threads of the last one, and the kernels, separated by tabs.
+// output for each: the number of launches, dynamic LDS, threads, and workgroups in the first dimension of the last one, and the kernels, separated by
+// tabs.
 // A descriptor of a layout conversion or of a pooling, told apart by its size, is executed as such.
 #include <cxxabi.h>
 #include <hip/hip_runtime.h>
@@ -20,7 +21,7 @@ static std::map<const void*, std::string>& kernels() {  // (filled by the librar
 }
 static std::string g_names;
 static int g_launches;
-static unsigned g_lds, g_threads;
+static unsigned g_lds, g_threads, g_grid;
 extern "C" {
 void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) {
     int st;
@@ -42,10 +43,11 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int
     *n = 2;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3 block, void**, size_t lds, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t lds, hipStream_t) {
     ++g_launches;
     g_lds = (unsigned)lds;
     g_threads = block.x;
+    g_grid = grid.x;
     g_names += "\t" + (kernels().count(f) ? kernels()[f] : "?");
     return hipSuccess;
 }
@@ -94,7 +96,7 @@ int main() {
             printf("status %d: %s\n", st, mi355_last_error());
             return 1;
         }
-        printf("%d %u %u%s\n", g_launches, g_lds, g_threads, g_names.c_str());
+        printf("%d %u %u %u%s\n", g_launches, g_lds, g_threads, g_grid, g_names.c_str());
     }
     return 0;
 }

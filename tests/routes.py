@@ -1,5 +1,6 @@
 """The kernels that an exec launches, through tests/host/route.cpp (no GPU)."""
 import collections
+import functools
 import os
 import re
 import subprocess
@@ -7,7 +8,7 @@ import subprocess
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 EXE = os.path.join(ROOT, "tests", "host", "route")
 HEURISTIC, UNNAMED = -1, -2
-Route = collections.namedtuple("Route", "launches lds threads kernels")
+Route = collections.namedtuple("Route", "launches lds threads grid kernels")
 
 
 def _short(name):
@@ -15,10 +16,14 @@ def _short(name):
     return re.match(r"(?:void )?(?:\w+::)*(\w+(?:<[^()]*>)?)\(", name.replace("(anonymous namespace)::", "")).group(1)
 
 
+@functools.lru_cache(None)
+def _build():
+    subprocess.check_call(["make", "-C", os.path.dirname(EXE), "-s", EXE])
+
+
 def routes(execs):
     """execs: descriptors, or (descriptor, algorithm, tile, workspace) -> a Route for each"""
-    if not os.path.exists(EXE):
-        subprocess.check_call(["make", "-C", os.path.dirname(EXE), "-s", EXE])
+    _build()
     lines = ["%s %d %d %d\n" % ((bytes(e[0]).hex(),) + tuple(int(v) for v in e[1:])) for e in
              (e if isinstance(e, tuple) else (e, HEURISTIC, -1, True) for e in execs)]
     r = subprocess.run([EXE], input="".join(lines), capture_output=True, text=True, timeout=120)
