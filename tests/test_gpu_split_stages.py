@@ -1,6 +1,8 @@
 """Windowed layers whose stages two groups of waves share (conv_patch4.hip, conv_patch1.hip, tiles of 32 x 128): odd and even numbers of stages, an
-incomplete last one, either side of the number of workgroups where it begins, both requantisation halves with and without a residual.  Against
-the oracle; which form runs, by the workgroup's threads."""
+incomplete last one, either side of the number of workgroups where it begins, every requantisation form of either half of a block with and without
+a residual.  Against the oracle; which form runs, by the workgroup's threads."""
+import itertools
+
 import numpy as np
 import pytest
 import torch
@@ -9,7 +11,10 @@ from megengine_amd import _abi, lib, ops
 from tests import util
 from tests.routes import UNNAMED, routes
 
-S = dict(scale_bias=2e-4, scale_z=0.05, scale_dst=0.05)
+SCALES = [
+    dict(scale_bias=2e-4, scale_z=0.05, scale_dst=0.05),       # the quotient form
+    dict(scale_bias=1.3e-3, scale_z=0.05, scale_dst=0.0271),   # a linear form for IDENTITY and RELU without a residual
+]
 IGEMM = 1
 CASES = [
     # format, n, ic, ih, iw, oc, f, pad, stride, threads of a workgroup
@@ -28,13 +33,17 @@ CASES = [
     ("NCHW", 1, 33, 12, 19, 70, 5, 2, 2, 512),
     ("NCHW", 1, 150, 15, 14, 20, 3, 1, 2, 512),
     ("NCHW", 3, 40, 9, 7, 33, 3, 1, 1, 256),         # two stages
+    ("NCHW", 64, 75, 16, 16, 33, 3, 1, 1, 512),      # 32 workgroups to an XCD
+    ("NCHW", 65, 75, 16, 16, 33, 3, 1, 1, 256),      # 34
+    ("NCHW", 64, 130, 16, 16, 33, 1, 0, 1, 512),
+    ("NCHW", 65, 130, 16, 16, 33, 1, 0, 1, 256),
 ]
 
 
-def _desc(c, nl, z):
+def _desc(c, nl, z, scales=SCALES[0]):
     fmt, n, ic, ih, iw, oc, f, pad, stride, _ = c
     f = f if isinstance(f, tuple) else (f, f)
-    return _abi.make_conv_desc(fmt, n, ic, ih, iw, oc, *f, pad=pad, stride=stride, nonline=nl, has_z=z, **S)
+    return _abi.make_conv_desc(fmt, n, ic, ih, iw, oc, *f, pad=pad, stride=stride, nonline=nl, has_z=z, **scales)
 
 
 def _exec(c, d):
@@ -51,8 +60,8 @@ def test_which_form():
 @pytest.mark.parametrize("i", range(len(CASES)))
 def test_split(oracle, i):
     c = CASES[i]
-    for nl, has_z in (("RELU", True), ("IDENTITY", False), ("H_SWISH", True)):
-        d = _desc(c, nl, has_z)
+    for scales, nl, has_z in itertools.product(SCALES, ("IDENTITY", "RELU", "H_SWISH"), (False, True)):
+        d = _desc(c, nl, has_z, scales)
         src, flt, bias, z = util.make_tensors(d, seed=500 + i)
         want = oracle.conv_bias(d, src, flt, bias, z)
         dev = [None if x is None else torch.from_numpy(x).cuda() for x in (src, flt, bias, z)]
@@ -61,6 +70,6 @@ def test_split(oracle, i):
         if c[0] == "NCHW4":
             a = ops.conv_bias_query(d, algo)[0]
             a.tile_cfg = tile
-        assert np.array_equal(ops.conv_bias_exec(d, *dev, algo=a).cpu().numpy(), want), (c, nl)
+        assert np.array_equal(ops.conv_bias_exec(d, *dev, algo=a).cpu().numpy(), want), (c, nl, has_z, scales)
         if has_z:   # the output over its residual
-            assert np.array_equal(ops.conv_bias_exec(d, *dev, dev[3], algo=a).cpu().numpy(), want), (c, nl)
+            assert np.array_equal(ops.conv_bias_exec(d, *dev, dev[3], algo=a).cpu().numpy(), want), (c, nl, has_z, scales)
