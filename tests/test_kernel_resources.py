@@ -113,3 +113,23 @@ def test_streaming_pointwise_kernels_keep_accumulators_in_vgprs(resources):
         assert r["agprs"] == 0 and r["scratch"] == 0, (name, r)
         assert r["lds"] <= (1024 if ", true>" in name else 16), (name, r)
         assert r["occupancy"] >= 3, (name, r)
+
+
+def test_grouped_and_channel_wise_kernels_keep_their_budget(resources):
+    """grp16_kernel is one band to a workgroup because six workgroups fit on a CU (six waves per SIMD: 80 registers, all of them taken with a
+    residual), and dwm_kernel is bounded to five waves per SIMD; a spill would be reloaded in every step of their loops."""
+    for name, r in kernels(resources, r"grp16_kernel<").items():
+        assert r["scratch"] == 0 and r["vgprs"] <= 80 and r["occupancy"] >= 6, (name, r)
+    for name, r in kernels(resources, r"dwm_kernel<[1-8], ").items():
+        assert r["scratch"] == 0 and r["occupancy"] >= 5, (name, r)
+
+
+@pytest.mark.parametrize("tile,occupancy", [("1, 1", 3), ("1, 2", 2), ("2, 2", 2), ("2, 1", 2)])
+def test_windowed_kernels_do_not_spill(resources, tile, occupancy):
+    """patch4_kernel and patch1_kernel in all their forms: their loops have a barrier per stage, and a spill on either side of it is a round trip
+    that nothing hides.  The smallest tile, which also runs as two groups of waves, keeps a third workgroup on a CU."""
+    for name, r in kernels(resources, r"patch1_kernel<%s, \d+>" % tile).items():
+        assert r["scratch"] == 0 and r["occupancy"] >= occupancy, (name, r)
+    if tile != "2, 1":
+        for name, r in kernels(resources, r"patch4_kernel<%s, \d+>" % tile).items():
+            assert r["scratch"] == 0 and r["occupancy"] >= (4 if tile == "1, 1" else 3 if tile == "1, 2" else 2), (name, r)
