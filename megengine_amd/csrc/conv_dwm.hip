@@ -225,8 +225,9 @@ __device__ __forceinline__ void dwm_run(const Form& form) {
         for (int p = 0; p < 4; ++p) fa[st][p] = reinterpret_cast<const int*>(lds_dwm)[woff[st] + p] & mask;
     // One loop per requantisation form: chosen inside it the form was a dozen branches per step (5x5, 60 channels at 76 x 22, batch 21, with a
     // residual: 6.99 -> 5.81 us; 240 channels at 57 x 57, stride 2, batch 16, H_SWISH: 7.41 -> 6.67).  Without branches the compiler reads a
-    // step's operands further ahead, so registers are bounded to five waves per SIMD, as before (unbounded: 544 channels at 95 x 100, stride 2,
-    // batch 22: 45.9 -> 52.0 us).  Longer windows would spill then and keep the choice inside.
+    // step's operands further ahead: four steps take 73 to 95 registers, five and six waves per SIMD, where they took 49 to 70, five to eight, with
+    // the choice inside.  They are bounded to five (unbounded: 544 channels at 95 x 100, stride 2, batch 22: 45.9 -> 52.0 us).  Longer windows would
+    // spill then and keep the choice inside.
     auto multiply = [&](auto form_of) __attribute__((always_inline)) {
         constexpr int NL = decltype(form_of)::value;
         for (int u = wave * 32; u < quads; u += step) {

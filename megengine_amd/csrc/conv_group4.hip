@@ -17,10 +17,11 @@
 // a lane of v_mfma_i32_16x16x64_i8 holds, so a step is four taps and 3x3 is three steps, zeros of the block diagonal
 // included a third of the time of the dot products.  A workgroup stages a band of input rows in LDS as [pixel][16
 // channels] (NCHW4 keeps them in four planes), so every operand is one conflict-free ds_read_b128; the filter stays in
-// twelve registers.  A workgroup is one band, with no band in flight behind it: the sixteen registers of a second band's pixels cost a
-// fifth workgroup on the CU, which hides more (six fit now, three with them).
-// 32 groups of 4 at 56 x 56, batch 16 (13 MB): 165 us as 32 launches, 9.8 with dot products, 5.8 here; 32 groups of 16
-// (51 MB): 50 us with dot products, 17 here; 47 groups of 16 at 78 x 8, batch 60: 20.7 with bands in a row, 16.8 one to a workgroup.  Small layers are a chain: with the filter staged beside the first band instead of
+// twelve registers.  A workgroup is one band, with no band in flight behind it: other workgroups on the CU hide more than a second band's pixels
+// in sixteen registers did (six of 77 to 80 registers fit, four of 100 to 104 with those).
+// 32 groups of 4 at 56 x 56, batch 16 (13 MB): 165 us as 32 launches, 9.8 with dot products, 5.9 here; 32 groups of 16
+// (51 MB): 50 us with dot products, 17 here; 47 groups of 16 at 78 x 8, batch 60: 20.7 with bands in a row,
+// 16.8 one to a workgroup.  Small layers are a chain: with the filter staged beside the first band instead of
 // gathered dword by dword ahead of it, and the next operands read while results are requantised, 55 groups of 16 at 8 x 47,
 // stride 2, batch 4 went from 6.2 to 4.2 us, 5 groups of 16 at 33 x 100, stride 2, batch 64 from 9.8 to 8.4.
 #include <tuple>

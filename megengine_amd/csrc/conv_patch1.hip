@@ -16,8 +16,8 @@
 //   * Two stages in LDS, the next one's loads in registers while the current one is multiplied, one barrier per stage.
 //   * Bound by LDS, as the 4-packed patch tiles are, and by the latency of a stage where tiles are few.
 // Filters of 1x1, 3x3 and 5x5; others go through the
-// workspace.  Graph replays: 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual: 16.6 us packed, 11.3 here (four waves of
-// 1200 vector instructions for 23 products each, a third of their time waiting for a stage's loads); more at patch1_pick.
+// workspace.  Graph replays: 75 -> 150 channels, 3x3 at 61 x 45, batch 6, with a residual: 16.6 us packed, 11.1 here (four waves of
+// 1200 vector instructions for 23 products each, a third of their time waiting for a stage's loads); more at p1_tile.
 #include <algorithm>
 #include <atomic>
 
@@ -281,10 +281,11 @@ bool p1_plan(const ConvProblem& p, int tile, P1Args* k, int* lds_bytes) {
 }
 
 // The same tile as a run of pixels in the order of memory where that is ahead of the rows and columns of p1_plan.
-// Rows that end inside a group of four columns cost rows-and-columns tiles a group of single bytes in each row, six more memory
-// instructions for four outputs of every channel, and columns of the tile that hold nothing; a run has one such group at an image's end.
-// Its patch is all columns of the rows that it touches.  231 drawn layers with such rows, graph replays: 0.97 of the time since
-// this rule takes runs for some (3x3 121 -> 251 at 45 x 10, batch 54: 29.2 -> 18.6 us; 3x3 75 -> 150 at 61 x 45, batch 6, residual: 12.4 -> 11.3).
+// Rows that end inside a group of four columns cost rows-and-columns tiles a group of its own in each row, two more stores for its outputs of
+// every channel (six more memory instructions, all of single bytes, when this rule was made), and columns of the tile that hold nothing; a run has
+// one such group at an image's end.  Its patch is all columns of the rows that it touches.  231 drawn layers with such rows, graph replays:
+// 0.97 of the time since this rule takes runs for some (3x3 121 -> 251 at 45 x 10, batch 54: 29.2 -> 18.6 us; 3x3 75 -> 150 at 61 x 45, batch 6,
+// residual: 12.4 -> 11.3).  What a run needs to know costs layers with rows of whole groups up to 3 % of a launch of 4 us.
 // Not where a run's patch asks more of a thread or leaves fewer workgroups to a CU (3x3 at stride 2, 202 -> 106 at 60 x 91, batch 14: 24.5 ->
 // 37.4), nor, where every workgroup has a CU for itself, for a patch that takes longer to turn (5x5 5 -> 180 at 14 x 43, batch 2: 4.8 -> 6.4).
 void p1_run(const ConvProblem& p, int tile, int cu_count, P1Args* k, int* lds_bytes) {
@@ -376,6 +377,9 @@ bool patch1_usable(const ConvProblem& p) {
 // reduction goes there (3x3 130 -> 44 at 12 x 12, five stages: 8.6 us here, 6.9 there; 48 -> 12, two: 5.0 / 6.4).  With more tiles
 // it is the other way round: 3x3 45 -> 12 at 22 x 22, batch 47: 5.3 / 9.4; 1x1 20 -> 149 at 96 x 78: 24.1 / 34.3; 5x5 46 -> 45,
 // 168640 pixels: 25.4 / 41.4.  A caller without a workspace has no packed path (packed = false).
+//   (These figures are of one group of waves.  With two, p1_split_lds, the lines for few tiles and long chains still lie right: of 240 drawn layers that go to the
+// packed path and that two groups would share here, one launch is ahead on 27, and takes 1.04 of the packed path's time on average with 1x1,
+// 1.19 with 3x3, 1.41 with 5x5.)
 //   Below 64 workgroups and from 2^24 multiply-adds on the packed path stays, 5 to 25 % behind on one or two stages: a workspace of
 // the size that it needs is written there, which the interface's tests hold (24 -> 40 at 28 x 28, batch 4, among them).
 //   Tiles: the smallest up to 400 workgroups of it (5x5: 256), where a stage's latency is all there is; beyond that 32 x 256 (3x3
@@ -426,7 +430,7 @@ static int p1_tile(const ConvProblem& p, bool packed, int cu_count, P1Args& k, i
 // 5x5 in two and more stages: whether the packed path is ahead of this kernel on its tile, by prices on a device of 256 CUs in us and, of
 // reductions, us per stage or per 1024 packed bytes.  This kernel walks its stages one after the other, so workgroups that begin another
 // round over the device -- of one or two to a CU -- cost a whole chain more; the packed path splits few tiles' reductions and deals
-// many tiles out smoothly.  Fitted to graph replays of 2397 layers over 17 to 256 channels on both; of these 213 were more than 3 %
+// many tiles out smoothly.  (Prices of one group of waves and of tiles of rows and columns: two groups and runs take less than this says.)  Fitted to graph replays of 2397 layers over 17 to 256 channels on both; of these 213 were more than 3 %
 // behind the packed path and 117 more than 10 % (5x5 209 -> 33 at 26 x 7, batch 38: 24.2 / 13.3; 183 -> 164 at 41 x 85, batch 5:
 // 56.4 / 36.8); with the prices 40 and 12.  On 591 others 70 and 44 before, 9 and 1 now, 0.70 and 0.69 of the packed path on average.
 static bool p1_behind_packed(const ConvProblem& p, int tile, int64_t workgroups, int nstages, int cu_count) {

@@ -238,7 +238,7 @@ __global__ __launch_bounds__(256 * KS, 2) void patch1_kernel(P1Args a) {
     }
 
     // (the largest tile has registers for it once the products are done: all of it at once, where each dword used to be waited for behind the
-    // store before it; 3x3 7 -> 210 at 63 x 84, batch 42: 75.4 -> 59.1 us)
+    // store before it; 3x3 7 -> 210 at 63 x 84, batch 42: 75.4 -> 61.2 us)
     if constexpr (ZPRE) {
         if (a.epi.has_z && a.OHW < 4) p1_residual_bytes<MT, NT, QN>(a, zq, o, oc0 + kg * 16, wave, l32, lh);
     } else if (a.epi.has_z) {
